@@ -42,6 +42,8 @@ SIGNATURES = {
     "cg_scan_lengths_static": (_INT, [_P, _I64, _P, _P]),
     "cg_tables_to_counts": (_INT, [_P, _INT, _I64, _I64, _P, _P, _P, _P, _P]),
     "cg_pack_counts": (_INT, [_P, _INT, _I64, _I64, _P, _P, _P, _P]),
+    "cg_wire_meta": (_INT, [_P, _P, _I64, _I64, _P, _P, _P, _I64, _P, _P]),
+    "cg_lengths_to_u16": (_INT, [_P, _I64, _P, _P, _P]),
     "cg_counts_to_tables": (_INT, [_P, _I64, _INT, _I64, _I64, _P, _P, _P, _P, _P, _P]),
     "cg_decode_kv": (_INT, [_P, _INT, _P, _INT, _P, _P, _I64, _P, _P, _I64, _I64, _I64, _I64, _I64, _INT,
                             _P, _INT, _I64, _I64, _I64, _I64, _P]),

@@ -627,13 +627,34 @@ int cg_tables_to_counts(const int16_t *cdf, int max_bins, int64_t ngroups, int64
 int cg_pack_counts(const uint8_t *counts, int max_bins, int64_t ngroups, int64_t C, const int32_t *nsym,
                    const int64_t *starts, uint8_t *out, void *stream)
 {
-    if (!counts || !nsym || !starts || !out) return fail(CG_ERR_ARG, "pack_counts: null pointer");
+    if (!counts || !nsym || !out) return fail(CG_ERR_ARG, "pack_counts: null pointer");
     if (int rc = check_lp(max_bins + 1, "pack_counts")) return rc;
     if (ngroups <= 0 || C <= 0 || ngroups > 65535) return fail(CG_ERR_ARG, "pack_counts: bad group or channel count");
     const dim3 grid((unsigned)ceil_div(C, kWireThreads), (unsigned)ngroups);
     pack_counts_kernel<<<grid, dim3(kWireThreads), 0, static_cast<hipStream_t>(stream)>>>(counts, max_bins + 1, C, nsym,
                                                                                          starts, out);
     return check_launch("pack_counts");
+}
+
+int cg_wire_meta(const int32_t *status, const int64_t *offsets, int64_t per_sub, int64_t nbounds, const int32_t *wide,
+                 const int32_t *inexact, const int32_t *nsym, int64_t ngroups, int64_t *out, void *stream)
+{
+    if (!status || !offsets || !out || (ngroups > 0 && !nsym)) return fail(CG_ERR_ARG, "wire_meta: null pointer");
+    if (per_sub <= 0 || nbounds <= 0 || ngroups < 0) return fail(CG_ERR_ARG, "wire_meta: bad count");
+    wire_meta_kernel<<<dim3(1), dim3(kWireThreads), 0, static_cast<hipStream_t>(stream)>>>(status, offsets, per_sub, nbounds, wide,
+                                                                                           inexact, nsym, ngroups, out);
+    return check_launch("wire_meta");
+}
+
+int cg_lengths_to_u16(const int32_t *lengths, int64_t n, uint16_t *out, int32_t *wide, void *stream)
+{
+    if (!lengths || !out || !wide) return fail(CG_ERR_ARG, "lengths_to_u16: null pointer");
+    const int64_t nblocks = ceil_div(n, kWireThreads);
+    if (n <= 0 || nblocks > INT_MAX) return fail(CG_ERR_ARG, "lengths_to_u16: bad count");
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    clear_ints_kernel<<<dim3(1), dim3(kWireThreads), 0, s>>>(wide, 1, nullptr);
+    lengths_to_u16_kernel<<<dim3((unsigned)nblocks), dim3(kWireThreads), 0, s>>>(lengths, n, out, wide);
+    return check_launch("lengths_to_u16");
 }
 
 int cg_counts_to_tables(const uint8_t *data, int64_t data_bytes, int max_bins, int64_t ngroups, int64_t C,

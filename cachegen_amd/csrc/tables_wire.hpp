@@ -20,6 +20,34 @@ __global__ void clear_ints_kernel(int32_t *a, int64_t na, int32_t *b)
     if (i == 0 && b) *b = 0;
 }
 
+// What the host has to know of an encoded tensor before it can lay blobs out, stored straight into
+// host memory (pinned: the host reads it once the event behind this launch is through, without a
+// copy of its own): out = [status, wide, inexact, payload offset at each of nbounds sub-chunk
+// boundaries, nsym[0 .. ngroups)].  One block; a few hundred values.
+__global__ __launch_bounds__(kWireThreads) void wire_meta_kernel(
+    const int32_t *__restrict__ status, const int64_t *__restrict__ offsets, int64_t per_sub, int64_t nbounds,
+    const int32_t *__restrict__ wide, const int32_t *__restrict__ inexact, const int32_t *__restrict__ nsym, int64_t ngroups, int64_t *out)
+{
+    if (threadIdx.x == 0) {
+        out[0] = *status;
+        out[1] = wide ? *wide : 0;
+        out[2] = inexact ? *inexact : 0;
+    }
+    for (int64_t i = threadIdx.x; i < nbounds; i += kWireThreads) out[3 + i] = offsets[i * per_sub];
+    for (int64_t i = threadIdx.x; i < ngroups; i += kWireThreads) out[3 + nbounds + i] = nsym[i];
+}
+
+// Stream lengths as 16-bit words; *wide (zero before the launch) is set where one does not fit.
+__global__ __launch_bounds__(kWireThreads) void lengths_to_u16_kernel(
+    const int32_t *__restrict__ lengths, int64_t n, uint16_t *__restrict__ out, int32_t *wide)
+{
+    const int64_t i = (int64_t)blockIdx.x * kWireThreads + threadIdx.x;
+    if (i >= n) return;
+    const int32_t v = lengths[i];
+    out[i] = (uint16_t)v;
+    if (v < 0 || v > 0xFFFF) atomicOr(wide, 1);
+}
+
 // One thread per (group, channel).  counts: uint8 [ngroups, C, lp - 1], clamped to 255;
 // nsym[g]: one more than the largest symbol that occurs in group g (at least 1);
 // inexact: set to 1 if some table is not what the formula gives for any histogram.
@@ -58,17 +86,28 @@ __global__ __launch_bounds__(kWireThreads) void tables_to_counts_kernel(
     if ((threadIdx.x & 63) == 0) atomicMax(nsym + g, last);
 }
 
-// Ragged form: group g's channels in turn, nsym[g] counts each, from byte starts[g] on.
+// Ragged form: group g's channels in turn, nsym[g] counts each, from byte starts[g] on.  starts ==
+// null: the groups follow one another, and every block adds up the symbol counts before its group's
+// (the host does not have to see them first).
 __global__ __launch_bounds__(kWireThreads) void pack_counts_kernel(
     const uint8_t *__restrict__ counts, int lp, int64_t C, const int32_t *__restrict__ nsym,
     const int64_t *__restrict__ starts, uint8_t *__restrict__ out)
 {
     const int64_t g = blockIdx.y;
     const int64_t ch = (int64_t)blockIdx.x * kWireThreads + threadIdx.x;
+    __shared__ int32_t before;
+    if (!starts) {
+        if (threadIdx.x == 0) before = 0;
+        __syncthreads();
+        int32_t mine = 0;                                           // at most 65535 groups of 128 symbols
+        for (int64_t i = threadIdx.x; i < g; i += kWireThreads) mine += nsym[i];
+        if (mine) atomicAdd(&before, mine);
+        __syncthreads();
+    }
     if (ch >= C) return;
     const int k = nsym[g];
     const uint8_t *src = counts + (g * C + ch) * (lp - 1);
-    uint8_t *dst = out + starts[g] + ch * k;
+    uint8_t *dst = out + (starts ? starts[g] : (int64_t)before * C) + ch * k;
     for (int j = 0; j < k; ++j) dst[j] = src[j];
 }
 

@@ -70,6 +70,8 @@ class CacheGenSerializer(Serializer):
         self.fmt = metadata.fmt
         self.key_bins = self.make_key_bins(self.cachegen_config)
         self.value_bins = self.make_value_bins(self.cachegen_config)
+        # table size: known from the configuration, so that no call has to ask the device for it
+        self.max_bins = int(max(CGBasics.make_key_bins(self.cachegen_config).max(), CGBasics.make_value_bins(self.cachegen_config).max()))
 
     def make_key_bins(self, config: CacheGenConfig) -> torch.Tensor:
         return CGBasics.make_key_bins(config).cuda()
@@ -85,7 +87,7 @@ class CacheGenSerializer(Serializer):
             tensor = tensor.permute(0, 1, 3, 2, 4)
         ntokens = tensor.shape[2]
         if self.wire_format != "pickle":
-            enc = codec.encode_kv(tensor.cuda(), self.key_bins, self.value_bins, chunk_tokens=ntokens)
+            enc = codec.encode_kv(tensor.cuda(), self.key_bins, self.value_bins, chunk_tokens=ntokens, max_bins=self.max_bins)
             return wire.pack_chunks(enc, per_chunk=False, compact=self.wire_format == "compact")[0]
         output = encode_function(tensor.cuda(), self.cachegen_config, self.key_bins,
                                  self.value_bins, ntokens)
@@ -98,7 +100,7 @@ class CacheGenSerializer(Serializer):
         if self.fmt == "huggingface":
             tensor = tensor.permute(0, 1, 3, 2, 4)
         num_heads, head_size = tensor.shape[-2:]
-        enc = codec.encode_kv(tensor.cuda(), self.key_bins, self.value_bins, chunk_tokens=chunk_size)
+        enc = codec.encode_kv(tensor.cuda(), self.key_bins, self.value_bins, chunk_tokens=chunk_size, max_bins=self.max_bins)
         if self.wire_format != "pickle":
             return wire.pack_chunks(enc, compact=self.wire_format == "compact")
         enc.check()

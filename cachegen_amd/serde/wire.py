@@ -272,16 +272,18 @@ def _stream():
 
 
 def _device_counts_launch(cdf, tokens):
-    """First half of the device form of tables_to_counts + pack_counts for cdf int16
-    [nchunks, 2L, C, Lp]: launches the conversion and returns (dense counts uint8 [G, C, Lp-1],
-    nsym int32 [G], inexact int32 [1]), all still on the device and not waited for."""
+    """Device form of tables_to_counts for cdf int16 [nchunks, 2L, C, Lp]: launches the conversion
+    and returns (dense counts uint8 [G, C, Lp-1], nsym int32 [G], inexact int32 [1]), all still on
+    the device and not waited for.  tokens: per chunk; all but the last are the same."""
     import torch
     from .. import _lib
     nchunks, rows, C, lp = cdf.shape
     G = nchunks * rows
     dev = cdf.device
     cdf = cdf.contiguous()
-    tok = torch.tensor([t for t in tokens for _ in range(rows)], dtype=torch.int32).to(dev, non_blocking=True)
+    tok = torch.full((G,), tokens[0], dtype=torch.int32, device=dev)
+    if tokens[-1] != tokens[0]:
+        tok[G - rows:].fill_(tokens[-1])
     dense = torch.empty((G, C, lp - 1), dtype=torch.uint8, device=dev)
     nsym = torch.empty(G, dtype=torch.int32, device=dev)
     inexact = torch.empty(1, dtype=torch.int32, device=dev)
@@ -289,37 +291,6 @@ def _device_counts_launch(cdf, tokens):
         _lib.check(_lib.lib().cg_tables_to_counts(cdf.data_ptr(), lp - 1, G, C, tok.data_ptr(), dense.data_ptr(),
                                                   nsym.data_ptr(), inexact.data_ptr(), _stream()))
     return dense, nsym, inexact
-
-
-def _device_counts_finish(dense, nsym, ks):
-    """Second half: ks is nsym read back on the host; returns the ragged count bytes uint8 on
-    the device."""
-    import torch
-    from .. import _lib
-    G, C, nb = dense.shape
-    dev = dense.device
-    starts, total = [], 0
-    for k in ks:
-        starts.append(total)
-        total += C * k
-    data = torch.empty(total, dtype=torch.uint8, device=dev)
-    d_starts = torch.tensor(starts, dtype=torch.int64).to(dev, non_blocking=True)
-    with torch.cuda.device(dev):
-        _lib.check(_lib.lib().cg_pack_counts(dense.data_ptr(), nb, G, C, nsym.data_ptr(), d_starts.data_ptr(),
-                                             data.data_ptr(), _stream()))
-    return data
-
-
-def _device_counts(cdf, tokens):
-    """Device form of tables_to_counts + pack_counts for cdf int16 [nchunks, 2L, C, Lp]:
-    (nsym list per (chunk, row), ragged count bytes uint8 on the device) or None if some table is
-    not the table of a histogram."""
-    import torch
-    dense, nsym, inexact = _device_counts_launch(cdf, tokens)
-    host = torch.cat([nsym, inexact]).tolist()
-    if host[-1]:
-        return None
-    return host[:-1], _device_counts_finish(dense, nsym, host[:-1])
 
 
 def _raise_if_invalid_counts(invalid):
@@ -355,13 +326,24 @@ def _device_tables(nsym_host, nsym_dev, data, C, lp, tokens, defer=False):
     return cdf
 
 
+# Bytes of blobs that leave the GPU in one go: while the host copies one piece into its blobs, the
+# next is on the bus.  Blobs of one 256-token chunk (6 MB) are a piece each.
+_PIECE_BYTES = 4 << 20
+
+
 def pack_chunks(enc, first_chunk: int = 0, num_chunks: Optional[int] = None, per_chunk: bool = True,
                 compact: bool = False) -> List[bytes]:
     """Blobs for chunks [first_chunk, first_chunk + num_chunks) of an `EncodedKV`: one blob per
     chunk (what one `to_bytes` call of the reference covers) or, with per_chunk=False, a single
-    blob holding all of them; compact: version 2.  All blobs are assembled in one device buffer
-    and leave the GPU in one copy into pinned host memory."""
+    blob holding all of them; compact: version 2.
+
+    The blob's sections leave the encoder's own tensors for pinned memory as they are and are put
+    together on the host, where the blob has to be written anyway: no second copy of them on the
+    device.  The host waits for the device once for the sizes (status, payload offsets, symbol
+    counts, stored into pinned memory by one kernel) while the tables, whose size it knows, are
+    already on the bus, and then for each piece of about _PIECE_BYTES."""
     import torch
+    from .. import _lib, hostmem
     nch = enc.num_chunks
     if num_chunks is None:
         num_chunks = nch - first_chunk
@@ -369,90 +351,142 @@ def pack_chunks(enc, first_chunk: int = 0, num_chunks: Optional[int] = None, per
         raise ValueError("chunk range outside the encoded tensor")
     L, H, D, S, T = enc.num_layers, enc.num_heads, enc.head_size, enc.chunk_tokens, enc.num_tokens
     C = H * D
+    rows = 2 * L
     spc = enc.subchunks_per_chunk
     bf16 = enc.maxima.dtype == torch.bfloat16
-    groups = [(c, c + 1) for c in range(first_chunk, first_chunk + num_chunks)] if per_chunk \
-        else [(first_chunk, first_chunk + num_chunks)]
-    all_tokens = chunk_token_counts(T, S)
-    c0, c1 = first_chunk, first_chunk + num_chunks
-
-    # everything the host has to know before it can lay the blobs out, read back at once:
-    # status word, payload offset at every sub-chunk boundary, smallest and largest stream
-    # length, and (compact) the symbol count of every table plus the flag that says whether
-    # all tables are tables of histograms
+    c_first, c_last = first_chunk, first_chunk + num_chunks
+    g_first, g_last = c_first * spc, min(c_last * spc, enc.lengths.shape[0])
+    tokens = chunk_token_counts(T, S)[c_first:c_last]
     dev = enc.payload.device
-    nsub = enc.lengths.shape[0]
-    idx = torch.arange(0, nsub + 1, device=dev) * (2 * L * C)
-    want_counts = compact and S <= MAX_STREAM_BYTES
-    parts = [enc.status.to(torch.int64).reshape(1), enc.offsets[idx]]
-    if compact:
-        parts += [enc.lengths.min().to(torch.int64).reshape(1), enc.lengths.max().to(torch.int64).reshape(1)]
-    if want_counts:
-        dense, nsym_dev, inexact = _device_counts_launch(enc.cdf[c0:c1], all_tokens[c0:c1])
-        parts += [inexact.to(torch.int64), nsym_dev.to(torch.int64)]
-    meta = torch.cat(parts).tolist()
-    enc.raise_for_status(meta[0])
-    bounds = meta[1:nsub + 2]
-    rest = meta[nsub + 2:]
+    lib = _lib.lib()
 
-    version, flags, lengths_src = VERSION, 0, enc.lengths
-    packed = None                       # (nsym [nch, 2L], data, byte offset of every (chunk, row) in data)
-    if compact:
-        version = VERSION_COMPACT
-        lo, hi = rest[0], rest[1]
-        if want_counts and not rest[2]:
-            ks = rest[3:]                                        # nsym per (chunk, row)
-            data = _device_counts_finish(dense, nsym_dev, ks)    # ragged count bytes
-            starts = [0]
-            for k in range(c1 - c0):
-                starts.append(starts[-1] + C * sum(ks[k * 2 * L:(k + 1) * 2 * L]))
-            nsym = nsym_dev.to(torch.uint8).view(c1 - c0, 2 * L)
-            packed = (nsym, data, starts)
-            flags |= FLAG_COUNT_TABLES
-        if lo >= 0 and hi <= 0xFFFF:
-            lengths_src = enc.lengths.to(torch.int16)         # bit pattern of the uint16 value
-            flags |= FLAG_LENGTHS_U16
+    def fetch(src):
+        """The bytes of a contiguous device tensor on their way into pinned memory."""
+        flat = src.reshape(-1).view(torch.uint8)
+        host = torch.empty(flat.numel(), dtype=torch.uint8, pin_memory=True)
+        host.copy_(flat, non_blocking=True)
+        return host
 
-    plans, total = [], 0
-    for c0, c1 in groups:
-        t0, t1 = c0 * S, min(c1 * S, T)
-        g0, g1 = c0 * spc, min(c1 * spc, enc.lengths.shape[0])
-        nbytes = bounds[g1] - bounds[g0]
-        table_tokens = min(S, t1 - t0)          # a short last chunk is a blob of its own length
-        tables_bytes = None
-        if packed is not None:
-            k0, k1 = c0 - first_chunk, c1 - first_chunk
-            tables_bytes = (k1 - k0) * 2 * L + packed[2][k1] - packed[2][k0]
-        geo = geometry(L, t1 - t0, H, D, table_tokens, enc.max_bins, nbytes, tables_bytes,
-                       lengths_src.element_size())
-        head = write_header(L, t1 - t0, H, D, table_tokens, enc.max_bins, enc.delta_group, g1 - g0, nbytes, bf16,
-                            version, flags, tables_bytes or 0)
-        plans.append((total, geo, head, (c0, c1, t0, t1, g0, g1)))
-        total += geo["total"][0]
-    stage = torch.zeros(total, dtype=torch.uint8, device=dev)
-    heads = torch.frombuffer(bytearray(b"".join(p[2] for p in plans)), dtype=torch.uint8).to(dev)
+    def mark():
+        event = torch.cuda.Event()
+        event.record()
+        return event
 
-    def place(base, span, src):
-        off, size = span
-        if size:
-            stage[base + off:base + off + size].view(src.dtype).view(src.shape).copy_(src)
-    for i, (base, geo, head, (c0, c1, t0, t1, g0, g1)) in enumerate(plans):
-        stage[base:base + HEADER_BYTES] = heads[i * HEADER_BYTES:(i + 1) * HEADER_BYTES]
-        if packed is None:
-            place(base, geo["cdf"], enc.cdf[c0:c1])
-        else:
-            k0, k1 = c0 - first_chunk, c1 - first_chunk
-            off, size = geo["cdf"]
-            head_bytes = (k1 - k0) * 2 * L
-            place(base, (off, head_bytes), packed[0][k0:k1])
-            place(base, (off + head_bytes, size - head_bytes), packed[1][packed[2][k0]:packed[2][k1]])
-        place(base, geo["maxima"], enc.maxima[:, :, t0:t1])
-        place(base, geo["lengths"], lengths_src[g0:g1])
-        place(base, geo["payload"], enc.payload[bounds[g0]:bounds[g1]])
-    host = torch.empty(total, dtype=torch.uint8, pin_memory=True)
-    host.copy_(stage, non_blocking=False)
-    raw = host.numpy()
-    return [raw[base:base + geo["total"][0]].tobytes() for base, geo, _, _ in plans]
+    with torch.cuda.device(dev):
+        stream = _stream()
+        cdf = enc.cdf[c_first:c_last]
+        lengths = enc.lengths[g_first:g_last]
+        wide = inexact = nsym = dense = None
+        if compact:
+            lengths16 = torch.empty(lengths.shape, dtype=torch.int16, device=dev)
+            wide = torch.empty(1, dtype=torch.int32, device=dev)
+            _lib.check(lib.cg_lengths_to_u16(lengths.data_ptr(), lengths.numel(), lengths16.data_ptr(), wide.data_ptr(), stream))
+            if S <= MAX_STREAM_BYTES:
+                dense, nsym, inexact = _device_counts_launch(cdf, tokens)
+        nbounds, ngroups = g_last - g_first + 1, 0 if nsym is None else nsym.numel()
+        meta = torch.empty(3 + nbounds + ngroups, dtype=torch.int64, pin_memory=True)
+
+        def ptr(t):
+            return None if t is None else t.data_ptr()
+        _lib.check(lib.cg_wire_meta(enc.status.data_ptr(), enc.offsets[g_first * rows * C:].data_ptr(), rows * C, nbounds,
+                                    ptr(wide), ptr(inexact), ptr(nsym), ngroups, meta.data_ptr(), stream))
+        sizes_known = mark()
+
+        # blobs by pieces: (first blob, last blob) covering about _PIECE_BYTES of tables and lengths
+        groups = [(c, c + 1) for c in range(c_first, c_last)] if per_chunk else [(c_first, c_last)]
+        chunk_bytes = max(1, cdf[0].numel() * cdf.element_size() + min(spc, lengths.shape[0]) * rows * C * 4)
+        step = max(1, _PIECE_BYTES // chunk_bytes) if per_chunk else 1
+        pieces = [(i, min(i + step, len(groups))) for i in range(0, len(groups), step)]
+
+        def subs(c):
+            return min(c * spc, g_last) - g_first
+
+        tables_src, lengths_src = cdf, lengths
+        early = {}                                       # the first piece's tables and lengths, sizes not needed
+        if dense is not None:
+            # ragged count bytes; their places follow from nsym, which is on the device
+            tables_src = torch.empty(dense.numel(), dtype=torch.uint8, device=dev)
+            _lib.check(lib.cg_pack_counts(dense.data_ptr(), dense.shape[2], ngroups, C, nsym.data_ptr(), None,
+                                          tables_src.data_ptr(), stream))
+        elif not compact:
+            a, b = groups[0][0], groups[pieces[0][1] - 1][1]
+            early = {"tables": fetch(cdf[a - c_first:b - c_first]), "lengths": fetch(lengths[subs(a):subs(b)])}
+        maxima = fetch(enc.maxima).numpy().view(np.uint16).reshape(rows, T)
+
+        sizes_known.synchronize()
+        meta = meta.tolist()
+        enc.raise_for_status(meta[0])
+        bounds = meta[3:3 + nbounds]
+        version, flags = VERSION, 0
+        starts = None                                    # byte offset of every chunk's counts in tables_src
+        if compact:
+            version = VERSION_COMPACT
+            if dense is not None:
+                if meta[2]:
+                    tables_src = cdf                     # not the tables of histograms: stored as they are
+                else:
+                    ks = np.asarray(meta[3 + nbounds:], dtype=np.uint8)
+                    starts = [0] + np.cumsum(ks.reshape(-1, rows).sum(axis=1, dtype=np.int64) * C).tolist()
+                    flags |= FLAG_COUNT_TABLES
+            if not meta[1]:
+                lengths_src = lengths16                  # bit pattern of the uint16 value
+                flags |= FLAG_LENGTHS_U16
+
+        def table_range(a, b):
+            if starts is not None:
+                return tables_src[starts[a - c_first]:starts[b - c_first]]
+            return tables_src[a - c_first:b - c_first]
+
+        def queue(piece):
+            a, b = groups[piece[0]][0], groups[piece[1] - 1][1]
+            p0, p1 = bounds[subs(a)], bounds[subs(b)]
+            tables = early.pop("tables", None)
+            lens = early.pop("lengths", None)
+            host = {"tables": fetch(table_range(a, b)) if tables is None else tables,
+                    "lengths": fetch(lengths_src[subs(a):subs(b)]) if lens is None else lens,
+                    "payload": fetch(enc.payload[p0:p1]) if p1 > p0 else None}
+            return host, mark()
+
+        blobs = []
+        queued = queue(pieces[0])
+        for k, piece in enumerate(pieces):
+            (host, arrived), queued = queued, queue(pieces[k + 1]) if k + 1 < len(pieces) else None
+            at = {"tables": 0, "lengths": 0, "payload": 0}
+            made = []
+            for a, b in groups[piece[0]:piece[1]]:       # everything but the big sections, while these arrive
+                t0, t1 = a * S, min(b * S, T)
+                nbytes = bounds[subs(b)] - bounds[subs(a)]
+                tables_bytes = None if starts is None else (b - a) * rows + starts[b - c_first] - starts[a - c_first]
+                table_tokens = min(S, t1 - t0)           # a short last chunk is a blob of its own length
+                geo = geometry(L, t1 - t0, H, D, table_tokens, enc.max_bins, nbytes, tables_bytes, lengths_src.element_size())
+                head = write_header(L, t1 - t0, H, D, table_tokens, enc.max_bins, enc.delta_group, subs(b) - subs(a), nbytes,
+                                    bf16, version, flags, tables_bytes or 0)
+                blob, into = hostmem.new_bytes(geo["total"][0])
+                parts = [(0, head)]
+                if starts is not None:
+                    parts.append((HEADER_BYTES, ks[(a - c_first) * rows:(b - c_first) * rows].tobytes()))
+                made.append((blob, into, geo, parts, t0, t1))
+            arrived.synchronize()
+            for blob, into, geo, parts, t0, t1 in made:
+                raw = into.numpy()
+                end = 0
+                for off, head in parts:
+                    raw[off:off + len(head)] = np.frombuffer(head, dtype=np.uint8)
+                    end = off + len(head)
+                for name, section in (("tables", "cdf"), ("maxima", "maxima"), ("lengths", "lengths"), ("payload", "payload")):
+                    off, size = geo[section]
+                    start = max(off, end)
+                    raw[end:start] = 0                   # the gap before the section
+                    n = off + size - start               # count tables: the symbol counts are there already
+                    if name == "maxima":
+                        np.copyto(raw[start:start + n].view(np.uint16).reshape(rows, t1 - t0), maxima[:, t0:t1])
+                    elif n:
+                        into[start:start + n].copy_(host[name][at[name]:at[name] + n])
+                        at[name] += n
+                    end = off + size
+                raw[end:] = 0
+                blobs.append(blob)
+    return blobs
 
 
 def unpack_to_device(blob, device, defer_checks=False):

@@ -259,7 +259,8 @@ int cg_tables_to_counts(const int16_t *cdf, int max_bins, int64_t ngroups, int64
                         const int32_t *tokens, uint8_t *counts, int32_t *nsym, int32_t *inexact,
                         void *stream);
 
-/* Ragged form of `counts`: out[starts[g] + ch*nsym[g] + j] = counts[g, ch, j], j < nsym[g]. */
+/* Ragged form of `counts`: out[starts[g] + ch*nsym[g] + j] = counts[g, ch, j], j < nsym[g].
+ * starts may be null: the groups then follow one another (starts[g] = C * sum of nsym[0..g)). */
 int cg_pack_counts(const uint8_t *counts, int max_bins, int64_t ngroups, int64_t C,
                    const int32_t *nsym, const int64_t *starts, uint8_t *out, void *stream);
 
@@ -271,6 +272,17 @@ int cg_pack_counts(const uint8_t *counts, int max_bins, int64_t ngroups, int64_t
 int cg_counts_to_tables(const uint8_t *data, int64_t data_bytes, int max_bins, int64_t ngroups, int64_t C,
                         const int32_t *tokens, const uint8_t *nsym, const int64_t *starts, int16_t *cdf,
                         int32_t *invalid, void *stream);
+
+/* What a host that lays out containers has to read back of an encoded tensor, in one piece:
+ * out[0] = *status, out[1] = *wide (0 if null), out[2] = *inexact (0 if null), out[3 + i] =
+ * offsets[i * per_sub] for i < nbounds, out[3 + nbounds + g] = nsym[g] for g < ngroups.
+ * out  int64, device or pinned host memory (then no copy is needed: wait for the stream) */
+int cg_wire_meta(const int32_t *status, const int64_t *offsets, int64_t per_sub, int64_t nbounds,
+                 const int32_t *wide, const int32_t *inexact, const int32_t *nsym, int64_t ngroups,
+                 int64_t *out, void *stream);
+
+/* out[i] = lengths[i] as 16 bits; *wide (device int32, written) = 1 if some length does not fit. */
+int cg_lengths_to_u16(const int32_t *lengths, int64_t n, uint16_t *out, int32_t *wide, void *stream);
 
 #ifdef __cplusplus
 }
