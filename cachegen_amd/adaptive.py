@@ -98,44 +98,42 @@ def merge(configs: Sequence[int], blobs: Sequence[Dict[int, bytes]], chunk_size:
     T' = chunk_size * (length // chunk_size), in `out_dtype` (default: the dtype of `orig_kv`, else
     bfloat16 for "vllm" and float16 for "huggingface" as the deserializer gives); every chunk is
     decoded in place into its token range."""
-    from . import codec
-    from .serde import wire
+    from .serde import incoming
     nwhole = length // chunk_size
     if nwhole == 0:
         raise ValueError("context shorter than one chunk")
-    out = None
+    dev = orig_kv.device if orig_kv is not None and orig_kv.is_cuda else torch.device("cuda")
     tdim = 2 if fmt == "vllm" else 3
-    bins_cache = {}
+    bins, items, recomputed = {}, [], []
     for chunk_id in range(nwhole):
         level = configs[chunk_id]
-        t0, t1 = chunk_id * chunk_size, (chunk_id + 1) * chunk_size
         if level == 0:
             if orig_kv is None:
                 raise ValueError(f"chunk {chunk_id} is to be recomputed but no original cache was given")
-            piece = orig_kv.narrow(tdim, t0, chunk_size)
-            if out is None:
-                shape = list(orig_kv.shape)
-                shape[tdim] = nwhole * chunk_size
-                out = torch.empty(shape, dtype=out_dtype or orig_kv.dtype, device=orig_kv.device)
-            out.narrow(tdim, t0, chunk_size).copy_(piece)
+            recomputed.append(chunk_id)
             continue
-        blob = blobs[chunk_id][level]
-        dev = orig_kv.device if orig_kv is not None and orig_kv.is_cuda else torch.device("cuda")
-        h, cdf, maxima, lengths, payload = wire.unpack_to_device(blob, dev)
-        if h["num_tokens"] != chunk_size:
-            raise ValueError(f"chunk {chunk_id} holds {h['num_tokens']} tokens, expected {chunk_size}")
-        if out is None:
-            L, H, D = h["num_layers"], h["num_heads"], h["head_size"]
-            shape = (L, 2, nwhole * chunk_size, H, D) if fmt == "vllm" else (L, 2, H, nwhole * chunk_size, D)
-            dtype = out_dtype or (orig_kv.dtype if orig_kv is not None
-                                  else (torch.bfloat16 if fmt == "vllm" else torch.float16))
-            out = torch.empty(shape, dtype=dtype, device=dev)
-        if level not in bins_cache:
-            bins_cache[level] = level_bins(level, model_name)
-        kb, vb = bins_cache[level]
-        codec.decode_kv(cdf, maxima, codec.scan_lengths(lengths), payload, kb, vb, h["num_layers"],
-                        chunk_size, h["num_heads"], h["head_size"], h["chunk_tokens"], fmt=fmt,
-                        out=out.narrow(tdim, t0, chunk_size), delta_group=h["delta_group"])
+        container = incoming.Container.flat(blobs[chunk_id][level])
+        if container.num_tokens != chunk_size:
+            raise ValueError(f"chunk {chunk_id} holds {container.num_tokens} tokens, expected {chunk_size}")
+        if level not in bins:
+            bins[level] = level_bins(level, model_name)
+            if container.num_layers != bins[level][0].numel():
+                raise RuntimeError(f"bins vectors must have one entry per layer ({container.num_layers})")
+        items.append((container, *bins[level], chunk_id * chunk_size))
+    if items:
+        c = items[0][0]
+        L, H, D = c.num_layers, c.num_heads, c.head_size
+        shape = [L, 2, nwhole * chunk_size, H, D] if fmt == "vllm" else [L, 2, H, nwhole * chunk_size, D]
+    else:
+        shape = list(orig_kv.shape)
+        shape[tdim] = nwhole * chunk_size
+    dtype = out_dtype or (orig_kv.dtype if orig_kv is not None else (torch.bfloat16 if fmt == "vllm" else torch.float16))
+    out = torch.empty(shape, dtype=dtype, device=dev if items else orig_kv.device)
+    for chunk_id in recomputed:
+        t0 = chunk_id * chunk_size
+        out.narrow(tdim, t0, chunk_size).copy_(orig_kv.narrow(tdim, t0, chunk_size))
+    if items:
+        incoming.decode(items, out, fmt)
     return out
 
 

@@ -245,6 +245,17 @@ def decode_kv(cdf, maxima, offsets, payload, key_bins, value_bins, num_layers, n
     return out
 
 
+def decode_listed(subs_ptr, nsub, max_bins, num_layers, num_heads, head_size, delta_group, out, fmt):
+    """cg_decode_listed: nsub sub-chunks described by entries in device memory (serde/incoming.py
+    writes them), all with tables of max_bins + 1 entries, into token ranges of `out`."""
+    (L, _, H, D), (ol, okv, ot, oh) = _kv_strides(out, fmt)
+    if (L, H, D) != (num_layers, num_heads, head_size) or out.dtype not in _DT:
+        raise RuntimeError("output tensor does not match the encoded geometry")
+    with torch.cuda.device(out.device):
+        _lib.check(_lib.lib().cg_decode_listed(subs_ptr, nsub, max_bins, L, H, D, int(delta_group), out.data_ptr(),
+                                               _DT[out.dtype], ol, okv, ot, oh, _stream()))
+
+
 def decode_encoded(enc: EncodedKV, key_bins, value_bins, fmt="vllm", out_dtype=None, out=None):
     return decode_kv(enc.cdf, enc.maxima, enc.offsets, enc.payload, key_bins, value_bins,
                      enc.num_layers, enc.num_tokens, enc.num_heads, enc.head_size,

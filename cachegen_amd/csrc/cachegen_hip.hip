@@ -561,53 +561,60 @@ int cg_decode_kv(const int16_t *cdf, int max_bins, const void *maxima, int max_d
     if (!cdf || !maxima || !offsets || !key_bins || !value_bins || !out || !payload)
         return fail(CG_ERR_ARG, "decode_kv: null pointer");
     if (int rc = check_dt(max_dt, "decode_kv")) return rc;
-    if (int rc = check_dt(out_dt, "decode_kv")) return rc;
     if (L <= 0 || T <= 0 || H <= 0 || D <= 0 || chunk_tokens <= 0) return fail(CG_ERR_ARG, "decode_kv: empty input");
     if (int rc = check_lp(max_bins + 1, "decode_kv")) return rc;
     if (delta_group < 0 || delta_group > kSub) return fail(CG_ERR_ARG, "decode_kv: delta_group must be in [0, %d]", kSub);
     const int64_t C = H * D, rows = 2 * L;
-    if (D > INT_MAX) return fail(CG_ERR_ARG, "decode_kv: head size too large");
-    // the kernel stores through a buffer descriptor per block: a channel's byte offset plus a
-    // token row's byte offset inside one stream's token range must fit 32 bits
-    if (ot < 0 || oh < 0 || ((H - 1) * oh + (D - 1) + (int64_t)(kSub - 1) * ot) * 2 + 2 > 0xFFFFFFFFll)
-        return fail(CG_ERR_ARG, "decode_kv: negative output strides, or %d token rows of one layer's keys or values "
-                                "span 4 GiB or more", kSub);
-    const int64_t nsub = cg_num_subchunks(T, chunk_tokens);
-    // two wavefronts per block: a block's slot is held until its slowest wavefront is through
-    // its 256 symbols, and smaller blocks leave fewer finished wavefronts waiting for that
-    // (one wavefront per block loses more to the per-block set-up than it gains)
-    int block = pick_block(C, max_bins + 1);
-    if (block > 128) block = 128;
     DecodeArgs a;
     memset(&a, 0, sizeof(a));
+    if (int rc = set_output(a, "decode_kv", out, out_dt, H, D, ol, okv, ot, oh)) return rc;
     a.cdf = reinterpret_cast<const uint16_t *>(cdf);
     a.lp = max_bins + 1;
     if (int rc = set_byte_window(a, payload, payload_bytes, "decode_kv")) return rc;
     a.offsets = offsets;
-    a.out_kv = static_cast<uint16_t *>(out);
-    a.ol = ol;
-    a.okv = okv;
-    a.ot = ot;
-    a.oh = oh;
     a.L = L;
-    a.D = (int32_t)D;
     a.maxima = static_cast<const uint16_t *>(maxima);
     a.max_dt = max_dt;
     a.delta_group = delta_group;
     a.key_bins = key_bins;
     a.value_bins = value_bins;
+    const int block = decode_kv_block(C, a.lp);
     int64_t nblocks;
-    if (int rc = make_grid(rows, C, T, chunk_tokens, nsub, block, a.sg, nblocks)) return rc;
-    const size_t shmem = decode_shmem(a.lp, block);
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    const dim3 grid = stream_grid(a.sg, nblocks);
-    // the blocks that are resident together at the launch's end (32 wavefronts per compute unit
-    // where registers and LDS allow it, which they do for tables of up to 33 entries)
-    const int64_t resident = (int64_t)compute_units() * (2048 / block);
-    a.last_round_first = (uint32_t)(nblocks > resident ? nblocks - resident : 0);
-    if (out_dt == CG_DT_BF16) CG_DISPATCH_BS(block, (launch_decode_kv_log2<BS, OUT_BF16>(a, grid, shmem, s)));
-    else CG_DISPATCH_BS(block, (launch_decode_kv_log2<BS, OUT_F16>(a, grid, shmem, s)));
-    return check_launch("decode_kv");
+    if (int rc = make_grid(rows, C, T, chunk_tokens, cg_num_subchunks(T, chunk_tokens), block, a.sg, nblocks)) return rc;
+    return launch_decode_kv<SRC_OFFSETS>(a, nblocks, block, out_dt, static_cast<hipStream_t>(stream));
+}
+
+int cg_decode_listed(const CgListedSub *subs, int64_t nsub, int max_bins, int64_t L, int64_t H, int64_t D,
+                     int delta_group, void *out, int out_dt, int64_t ol, int64_t okv, int64_t ot, int64_t oh, void *stream)
+{
+    if (!subs || !out) return fail(CG_ERR_ARG, "decode_listed: null pointer");
+    if (L <= 0 || H <= 0 || D <= 0 || nsub <= 0) return fail(CG_ERR_ARG, "decode_listed: empty input");
+    if (int rc = check_lp(max_bins + 1, "decode_listed")) return rc;
+    if (delta_group < 0 || delta_group > kSub) return fail(CG_ERR_ARG, "decode_listed: delta_group must be in [0, %d]", kSub);
+    const int64_t C = H * D, rows = 2 * L;
+    DecodeArgs a;
+    memset(&a, 0, sizeof(a));
+    if (int rc = set_output(a, "decode_listed", out, out_dt, H, D, ol, okv, ot, oh)) return rc;
+    a.lp = max_bins + 1;
+    a.L = L;
+    a.delta_group = delta_group;
+    a.listed = subs;
+    const int block = decode_kv_block(C, a.lp);
+    int64_t nblocks;
+    // the entries hold the token geometry; the grid only needs its size
+    if (int rc = make_grid(rows, C, nsub, 1, nsub, block, a.sg, nblocks)) return rc;
+    return launch_decode_kv<SRC_LISTED>(a, nblocks, block, out_dt, static_cast<hipStream_t>(stream));
+}
+
+int cg_host_tile_starts(const void *lengths, int itemsize, int64_t nsub, int64_t rows, int64_t C,
+                        uint32_t *tile_starts, int64_t *sub_bytes)
+{
+    if (!lengths || !tile_starts || !sub_bytes) return fail(CG_ERR_ARG, "host_tile_starts: null pointer");
+    if (nsub <= 0 || rows <= 0 || C <= 0 || rows > (1 << 24) / C || (itemsize != 2 && itemsize != 4))
+        return fail(CG_ERR_ARG, "host_tile_starts: bad shape");
+    const bool fine = itemsize == 2 ? host_tile_starts(static_cast<const uint16_t *>(lengths), nsub, rows, C, tile_starts, sub_bytes)
+                                    : host_tile_starts(static_cast<const int32_t *>(lengths), nsub, rows, C, tile_starts, sub_bytes);
+    return fine ? CG_OK : fail(CG_ERR_ARG, "host_tile_starts: negative length");
 }
 
 int cg_tables_to_counts(const int16_t *cdf, int max_bins, int64_t ngroups, int64_t C, const int32_t *tokens,

@@ -116,7 +116,7 @@ struct BitReader {
     }
 };
 
-enum { SRC_OFFSETS = 0, SRC_PREFIX = 1, SRC_PADDED = 2 };
+enum { SRC_OFFSETS = 0, SRC_PREFIX = 1, SRC_PADDED = 2, SRC_LISTED = 3 };
 enum { OUT_SYMBOLS = 0, OUT_F16 = 1, OUT_BF16 = 2 };
 
 struct DecodeArgs {
@@ -142,6 +142,7 @@ struct DecodeArgs {
     // blocks from this one on (in launch order) start when no block is left to take a finished
     // one's place: see decode_lane
     uint32_t last_round_first;
+    const CgListedSub *listed;  // SRC_LISTED: one entry per sub-chunk of the launch (blockIdx.z)
     StreamGrid sg;
 };
 
@@ -372,7 +373,22 @@ __global__ __launch_bounds__(BS) void decode_streams_kernel(DecodeArgs a)
     extern __shared__ uint32_t smem[];
     constexpr int kRow = DecodeLayout<BS, OUT>::kRow;
     const int tid = threadIdx.x;
-    const StreamId id = locate<BS>(a.sg);
+    StreamId id;
+    // SRC_LISTED: the sub-chunks of a launch come from several containers, each with its own tables,
+    // maxima, lengths, payload and levels; a block reads its sub-chunk's entry (the same for all of
+    // its lanes: scalar loads)
+    CgListedSub d;
+    if (SRC == SRC_LISTED) {
+        d = a.listed[blockIdx.z];
+        id.row = blockIdx.y;
+        id.sub = id.chunk = 0;
+        id.t0 = d.t_out;
+        id.n = d.n;
+        id.ch = (int64_t)blockIdx.x * BS + threadIdx.x;
+        id.active = id.ch < a.sg.nc;
+    } else {
+        id = locate<BS>(a.sg);
+    }
     const int lp = LOG2 >= 0 ? (1 << LOG2) + 1 : a.lp;
     char *rows = reinterpret_cast<char *>(smem);
     float *rowmax = reinterpret_cast<float *>(rows + lp * kRow);     // one per token of the sub-chunk
@@ -382,7 +398,8 @@ __global__ __launch_bounds__(BS) void decode_streams_kernel(DecodeArgs a)
         // lanes of a wavefront read neighbouring tables, so each cache line is fetched once.
         // Entry 0 of a table is 0 by construction (cal_cdf.cu:29-49 counts into hist[sym+1]);
         // it is stored as 0 whatever the input holds so that the walk back always ends.
-        const uint16_t *mine = a.cdf + ((id.chunk * a.sg.rows + id.row) * a.sg.nc + id.ch) * lp;
+        const uint16_t *tables = SRC == SRC_LISTED ? reinterpret_cast<const uint16_t *>(d.cdf) : a.cdf;
+        const uint16_t *mine = tables + ((id.chunk * a.sg.rows + id.row) * a.sg.nc + id.ch) * lp;
         char *column = rows + 2 * tid;
         if (id.active) {
             *reinterpret_cast<uint16_t *>(column) = 0;
@@ -416,15 +433,18 @@ __global__ __launch_bounds__(BS) void decode_streams_kernel(DecodeArgs a)
     if (OUT != OUT_SYMBOLS) {
         kvi = id.row >= a.L ? 1 : 0;             // 2L rows: keys, then values
         l = id.row - kvi * a.L;
-        const float bins = (kvi ? a.value_bins : a.key_bins)[l];
+        const float *const levels = SRC == SRC_LISTED ? (kvi ? d.value_bins : d.key_bins) : (kvi ? a.value_bins : a.key_bins);
+        const float bins = levels[l];
         const float cq = floorf(bins * 0.5f) - 1.0f;
         nsym = (cq >= 0.0f && cq < 32768.0f) ? 2 * (int)cq + 1 : lp;
         for (int i = tid; i < lp; i += BS)
             *reinterpret_cast<float *>(rows + i * kRow + DecodeLayout<BS, OUT>::kQuot) =
                 __fdiv_rn(__fsub_rn((float)i, cq), cq);
-        const uint16_t *mx = a.maxima + id.row * a.sg.g.T + id.t0;
+        const uint16_t *mx = SRC == SRC_LISTED ? static_cast<const uint16_t *>(d.maxima) + id.row * d.maxima_pitch
+                                               : a.maxima + id.row * a.sg.g.T + id.t0;
+        const int max_dt = SRC == SRC_LISTED ? d.max_dt : a.max_dt;
         for (int i = tid; i < id.n; i += BS) {
-            const float m = a.max_dt == CG_DT_BF16 ? load16f<CG_DT_BF16>(mx[i]) : load16f<CG_DT_F16>(mx[i]);
+            const float m = max_dt == CG_DT_BF16 ? load16f<CG_DT_BF16>(mx[i]) : load16f<CG_DT_F16>(mx[i]);
             // also rows whose scale overflowed in the quantizer: they hold the table's last symbol
             special |= (__float_as_uint(m) & 0x7FFFFFFFu) >= 0x7F800000u || scale_overflows(cq, m);
             rowmax[i] = m;
@@ -434,7 +454,21 @@ __global__ __launch_bounds__(BS) void decode_streams_kernel(DecodeArgs a)
 
     const int64_t stream = (id.sub * a.sg.rows + id.row) * a.sg.nc + id.ch;
     int64_t begin = INT64_MAX;
-    if (id.active) {
+    if (SRC == SRC_LISTED) {
+        // the wavefront's 64 streams follow one another from where the host's sums put the first
+        // (see CgListedSub); a stream occupies at most 256 bytes, whatever its length field says
+        int len = 0;
+        if (id.active) len = d.lengths_u16 ? (int)static_cast<const uint16_t *>(d.lengths)[stream] : static_cast<const int32_t *>(d.lengths)[stream];
+        len = len < 0 ? 0 : (len > kStreamCap ? kStreamCap : len);
+        int incl = len;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int up = __shfl_up(incl, o, 64);
+            if ((tid & 63) >= o) incl += up;
+        }
+        const int64_t tile = id.row * ((a.sg.nc + 63) >> 6) + (id.ch >> 6);
+        begin = d.first + (int64_t)d.tile_starts[id.active ? tile : 0] + (incl - len);
+    } else if (id.active) {
         if (SRC == SRC_OFFSETS) begin = a.offsets[stream];
         else if (SRC == SRC_PREFIX) begin = stream ? a.offsets[stream - 1] : 0;
         else begin = id.row * a.p0 + id.ch * a.p1;
@@ -449,7 +483,8 @@ __global__ __launch_bounds__(BS) void decode_streams_kernel(DecodeArgs a)
     if (!id.active) return;
 
     DecodeLane s;
-    s.off = s.rd.start(a.bytes, a.last_word, begin + a.bytes_skew, lowest + a.bytes_skew);
+    if (SRC == SRC_LISTED) s.off = s.rd.start(d.bytes, d.last_word, begin, lowest);
+    else s.off = s.rd.start(a.bytes, a.last_word, begin + a.bytes_skew, lowest + a.bytes_skew);
     s.low = 0;
     s.span = 0;                        // span modulo 2^32: 0 is the full range (see RangeEncoder)
     s.colp = (lds_char *)(rows + 2 * tid);

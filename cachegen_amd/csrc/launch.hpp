@@ -429,10 +429,88 @@ int launch_decode_symbols(const DecodeArgs &a, int64_t nblocks, int block, hipSt
     return check_launch("decode");
 }
 
-template <int BS, int OUT>
-void launch_decode_kv_log2(const DecodeArgs &a, dim3 grid, size_t shmem, hipStream_t stream)
+// Dequantised output (SRC_OFFSETS, SRC_LISTED): blocks of at most 128 lanes.
+template <int SRC>
+int launch_decode_kv(DecodeArgs &a, int64_t nblocks, int block, int out_dt, hipStream_t stream)
 {
-    launch_decode_log2<BS, SRC_OFFSETS, OUT>(a, grid, shmem, stream);
+    const size_t shmem = decode_shmem(a.lp, block);
+    const dim3 grid = stream_grid(a.sg, nblocks);
+    // the blocks that are resident together at the launch's end (32 wavefronts per compute unit
+    // where registers and LDS allow it, which they do for tables of up to 33 entries)
+    const int64_t resident = (int64_t)compute_units() * (2048 / block);
+    a.last_round_first = (uint32_t)(nblocks > resident ? nblocks - resident : 0);
+    if (block == 128) {
+        if (out_dt == CG_DT_BF16) launch_decode_log2<128, SRC, OUT_BF16>(a, grid, shmem, stream);
+        else launch_decode_log2<128, SRC, OUT_F16>(a, grid, shmem, stream);
+    } else {
+        if (out_dt == CG_DT_BF16) launch_decode_log2<64, SRC, OUT_BF16>(a, grid, shmem, stream);
+        else launch_decode_log2<64, SRC, OUT_F16>(a, grid, shmem, stream);
+    }
+    return check_launch("decode_kv");
+}
+
+// What the dequantising decoder's output has to satisfy, and its part of the arguments.
+int set_output(DecodeArgs &a, const char *what, void *out, int out_dt, int64_t H, int64_t D, int64_t ol, int64_t okv, int64_t ot, int64_t oh)
+{
+    if (int rc = check_dt(out_dt, what)) return rc;
+    if (D > INT_MAX) return fail(CG_ERR_ARG, "%s: head size too large", what);
+    // the kernel stores through a buffer descriptor per block: a channel's byte offset plus a
+    // token row's byte offset inside one stream's token range must fit 32 bits
+    if (ot < 0 || oh < 0 || ((H - 1) * oh + (D - 1) + (int64_t)(kSub - 1) * ot) * 2 + 2 > 0xFFFFFFFFll)
+        return fail(CG_ERR_ARG, "%s: negative output strides, or %d token rows of one layer's keys or values "
+                                "span 4 GiB or more", what, kSub);
+    a.out_kv = static_cast<uint16_t *>(out);
+    a.ol = ol;
+    a.okv = okv;
+    a.ot = ot;
+    a.oh = oh;
+    a.D = (int32_t)D;
+    return CG_OK;
+}
+
+// two wavefronts per block: a block's slot is held until its slowest wavefront is through
+// its 256 symbols, and smaller blocks leave fewer finished wavefronts waiting for that
+// (one wavefront per block loses more to the per-block set-up than it gains)
+int decode_kv_block(int64_t C, int lp)
+{
+    const int block = pick_block(C, lp);
+    return block > 128 ? 128 : block;
+}
+
+// Bytes that streams occupy before every 64th stream of a row, from their lengths in host memory:
+// lengths are min'ed with a stream's capacity; false if one is negative.
+template <typename T>
+bool host_tile_starts(const T *lengths, int64_t nsub, int64_t rows, int64_t C, uint32_t *starts, int64_t *sub_bytes)
+{
+    const int64_t tiles = ceil_div(C, 64);
+    int32_t lowest = 0;
+    for (int64_t s = 0; s < nsub; ++s) {
+        uint32_t run = 0;                       // at most 256 bytes of at most 2^24 streams: checked by the caller
+        for (int64_t r = 0; r < rows; ++r, lengths += C)
+            for (int64_t t = 0; t < tiles; ++t) {
+                *starts++ = run;
+                const int64_t n = C - t * 64 < 64 ? C - t * 64 : 64;
+                const T *p = lengths + t * 64;
+                int32_t sum = 0, low = 0;
+                if (n == 64) {
+                    for (int i = 0; i < 64; ++i) {          // a fixed count: vector instructions
+                        const int32_t v = p[i];
+                        sum += v < kStreamCap ? v : kStreamCap;
+                        low = v < low ? v : low;
+                    }
+                } else {
+                    for (int i = 0; i < n; ++i) {
+                        const int32_t v = p[i];
+                        sum += v < kStreamCap ? v : kStreamCap;
+                        low = v < low ? v : low;
+                    }
+                }
+                run += (uint32_t)sum;
+                lowest = low < lowest ? low : lowest;
+            }
+        sub_bytes[s] = run;
+    }
+    return lowest >= 0;
 }
 
 }  // namespace

@@ -7,7 +7,7 @@ import torch
 from .. import codec, torchac_hip
 from ..config import LMCacheEngineConfig, LMCacheEngineMetadata
 from . import cachegen_basics as CGBasics
-from . import wire
+from . import incoming, wire
 from .cachegen_basics import CacheGenConfig, CacheGenGPUBytestream, CacheGenGPUEncoderOutput
 from .serde import Deserializer
 
@@ -102,17 +102,35 @@ class CacheGenDeserializer(Deserializer):
                                encoder_output.head_size, chunk_tokens=ntokens, fmt=self.fmt, out=out)
 
     def _from_flat(self, bs, out=None) -> torch.Tensor:
-        # the container's own consistency (stream lengths against the payload size) is checked on
-        # the host inside unpack_to_device; the decode is queued before anything waits for the device
-        h, cdf, maxima, lengths, payload = wire.unpack_to_device(bs, self.key_bins.device, defer_checks=True)
-        if h["num_layers"] != self.key_bins.numel():
+        container = incoming.Container.flat(bs)
+        L, T, H, D = container.num_layers, container.num_tokens, container.num_heads, container.head_size
+        self._check_layers(container)
+        if out is None:
+            shape = (L, 2, T, H, D) if self.fmt == "vllm" else (L, 2, H, T, D)
+            out = torch.empty(shape, dtype=torch.bfloat16 if self.fmt == "vllm" else torch.float16, device=self.key_bins.device)
+        elif out.shape[2 if self.fmt == "vllm" else 3] != T:
+            raise RuntimeError("output tensor does not match the encoded geometry")
+        return incoming.decode([(container, self.key_bins, self.value_bins, 0)], out, self.fmt)
+
+    def _check_layers(self, container):
+        if container.num_layers != self.key_bins.numel():
             raise ValueError("blob has %d layers, this deserializer's model %d"
-                             % (h["num_layers"], self.key_bins.numel()))
-        # a stream occupies min(length, 256) bytes of the payload (wire.py checks the same sum)
-        offsets = codec.scan_lengths(lengths.clamp(max=wire.MAX_STREAM_BYTES))
-        result = codec.decode_kv(cdf, maxima, offsets, payload, self.key_bins, self.value_bins,
-                                 h["num_layers"], h["num_tokens"], h["num_heads"], h["head_size"],
-                                 chunk_tokens=h["chunk_tokens"], fmt=self.fmt, delta_group=h["delta_group"],
-                                 out=out)
-        h["check"]()
-        return result
+                             % (container.num_layers, self.key_bins.numel()))
+
+    def from_bytes_concat(self, blobs: List[bytes]):
+        """The tensors of several blobs of the flat container side by side along the token
+        dimension, in one tensor that they are decoded into by one launch; None if a blob is of
+        another container (not in the reference, whose callers concatenate the decoded chunks)."""
+        if not all(wire.is_flat(bs) for bs in blobs):
+            return None
+        items, tokens = [], 0
+        for bs in blobs:
+            container = incoming.Container.flat(bs)
+            self._check_layers(container)
+            items.append((container, self.key_bins, self.value_bins, tokens))
+            tokens += container.num_tokens
+        first = items[0][0]
+        L, H, D = first.num_layers, first.num_heads, first.head_size
+        shape = (L, 2, tokens, H, D) if self.fmt == "vllm" else (L, 2, H, tokens, D)
+        out = torch.empty(shape, dtype=torch.bfloat16 if self.fmt == "vllm" else torch.float16, device=self.key_bins.device)
+        return incoming.decode(items, out, self.fmt)

@@ -126,6 +126,21 @@ def read_header(blob) -> dict:
                 lengths_u16=bool(flags & FLAG_LENGTHS_U16), version=version, geometry=geo)
 
 
+def table_symbol_counts(blob, h) -> np.ndarray:
+    """Version 2 with count tables: the symbols stored per (chunk, row), uint8 [nchunks * 2L], checked
+    against the table length and the size of the section."""
+    groups = h["geometry"]["nchunks"][0] * 2 * h["num_layers"]
+    off, size = h["geometry"]["cdf"]
+    if size < groups:
+        raise ValueError("wire container: table section does not match its symbol counts")
+    nsym = np.frombuffer(blob, dtype=np.uint8, count=groups, offset=off)
+    if int(nsym.min()) < 1 or int(nsym.max()) > h["max_bins"]:
+        raise ValueError("wire container: symbol count outside the table")
+    if groups + int(nsym.sum(dtype=np.int64)) * h["num_heads"] * h["head_size"] != size:
+        raise ValueError("wire container: table section does not match its symbol counts")
+    return nsym
+
+
 # --------------------------------------------------------------------------- #
 # tables <-> histogram counts (numpy: the definition; the device code below mirrors it)
 # --------------------------------------------------------------------------- #
@@ -293,16 +308,10 @@ def _device_counts_launch(cdf, tokens):
     return dense, nsym, inexact
 
 
-def _raise_if_invalid_counts(invalid):
-    if int(invalid.item()):
-        raise ValueError("wire container: histogram counts do not add up to the chunk's tokens")
-
-
-def _device_tables(nsym_host, nsym_dev, data, C, lp, tokens, defer=False):
+def _device_tables(nsym_host, nsym_dev, data, C, lp, tokens):
     """Device form of unpack_counts + counts_to_tables -> cdf int16 [nchunks, 2L, C, Lp].
     nsym_host: numpy uint8 [nchunks, 2L] (read from the blob on the host), nsym_dev the same bytes
-    on the device.  defer: do not wait for the kernel's verdict on the counts; returns
-    (cdf, check) where check() waits and raises."""
+    on the device."""
     import torch
     from .. import _lib
     nchunks, rows = nsym_host.shape
@@ -320,9 +329,8 @@ def _device_tables(nsym_host, nsym_dev, data, C, lp, tokens, defer=False):
         _lib.check(_lib.lib().cg_counts_to_tables(data.data_ptr(), data.numel(), lp - 1, G, C, tok.data_ptr(),
                                                   nsym_dev.data_ptr(), small.data_ptr(), cdf.data_ptr(),
                                                   invalid.data_ptr(), _stream()))
-    if defer:
-        return cdf, (lambda: _raise_if_invalid_counts(invalid))
-    _raise_if_invalid_counts(invalid)
+    if int(invalid.item()):
+        raise ValueError("wire container: histogram counts do not add up to the chunk's tokens")
     return cdf
 
 
@@ -489,20 +497,20 @@ def pack_chunks(enc, first_chunk: int = 0, num_chunks: Optional[int] = None, per
     return blobs
 
 
-def unpack_to_device(blob, device, defer_checks=False):
+def unpack_to_device(blob, device):
     """-> (header dict, cdf, maxima, lengths, payload) on the device, which the blob reached in a
     single copy from pinned host memory: views of that buffer where the stored form is the
     tensor itself, rebuilt tensors where it is not (version 2).  The stream lengths are checked
-    against the payload size on the host.  defer_checks: nothing here waits for the device; the
-    header dict then holds "check", to be called once the caller has queued its own work: it
-    waits for the device and raises what the device-side checks found."""
+    against the payload size on the host.  (The deserializer and the engine decode blobs without
+    these tensors: incoming.py.)"""
     import torch
     h = read_header(blob)
     geo = h["geometry"]
     L, T, C = h["num_layers"], h["num_tokens"], h["num_heads"] * h["head_size"]
     lp, nchunks = h["max_bins"] + 1, geo["nchunks"][0]
+    from .. import hostmem
     host = torch.empty(len(blob), dtype=torch.uint8, pin_memory=True)
-    host.numpy()[:] = np.frombuffer(blob, dtype=np.uint8)
+    host.copy_(hostmem.view(blob))
     buf = host.to(device, non_blocking=False)      # waits: the pinned buffer is free for the next call at once
     # the lengths are in the blob: their sum is checked here, without asking the device
     off, size = geo["lengths"]
@@ -512,23 +520,14 @@ def unpack_to_device(blob, device, defer_checks=False):
     if int(np.minimum(host_lengths, MAX_STREAM_BYTES).sum(dtype=np.int64)) != h["payload_bytes"] \
             or (host_lengths.size and int(host_lengths.min()) < 0):
         raise ValueError("wire container: payload size is not the sum of the stream lengths")
-    h["check"] = lambda: None
-
     def section(name, dtype, shape):
         off, size = geo[name]
         return buf[off:off + size].view(dtype).view(shape)
     if h["count_tables"]:
+        nsym_host = table_symbol_counts(blob, h).reshape(nchunks, 2 * L)
         raw = section("cdf", torch.uint8, (-1,))
-        if raw.numel() < nchunks * 2 * L:
-            raise ValueError("wire container: table section does not match its symbol counts")
-        off = geo["cdf"][0]
-        nsym_host = np.frombuffer(blob, dtype=np.uint8, count=nchunks * 2 * L, offset=off).reshape(nchunks, 2 * L)
-        if int(nsym_host.min()) < 1 or int(nsym_host.max()) > lp - 1:
-            raise ValueError("wire container: symbol count outside the table")
         cdf = _device_tables(nsym_host, raw[:nchunks * 2 * L], raw[nchunks * 2 * L:], C, lp,
-                             chunk_token_counts(T, h["chunk_tokens"]), defer=defer_checks)
-        if defer_checks:
-            cdf, h["check"] = cdf
+                             chunk_token_counts(T, h["chunk_tokens"]))
     else:
         cdf = section("cdf", torch.int16, (nchunks, 2 * L, C, lp))
     maxima = section("maxima", torch.bfloat16 if h["bf16_maxima"] else torch.float16, (2, L, T))

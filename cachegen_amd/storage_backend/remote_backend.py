@@ -3,7 +3,7 @@
 
 With a CacheGen serde the whole-tensor forms do what the codec is built for: `put_chunks`
 encodes every chunk of a KV cache in one pass over the tensor, and `get_chunks_concat` decodes
-every chunk it finds straight into its token range of one output tensor."""
+every chunk it finds straight into its token range of one output tensor, all of them in one launch."""
 import logging
 import queue
 import threading
@@ -129,18 +129,11 @@ class LMCRemoteBackend(LMCBackendInterface):
         if not blobs:
             return None
         tdim = 2 if fmt == "vllm" else 3
-        shapes = [self.deserializer.chunk_shape(bs) if hasattr(self.deserializer, "chunk_shape") else None
-                  for bs in blobs]
-        if any(s is None for s in shapes):
-            return torch.cat([self.deserializer.from_bytes(bs) for bs in blobs], dim=tdim)
-        shape = list(shapes[0])
-        shape[tdim] = sum(s[tdim] for s in shapes)
-        out = torch.empty(shape, dtype=torch.bfloat16 if fmt == "vllm" else torch.float16, device="cuda")
-        t0 = 0
-        for bs, s in zip(blobs, shapes):
-            self.deserializer.from_bytes_into(bs, out.narrow(tdim, t0, s[tdim]))
-            t0 += s[tdim]
-        return out
+        if hasattr(self.deserializer, "from_bytes_concat"):
+            out = self.deserializer.from_bytes_concat(blobs)
+            if out is not None:
+                return out
+        return torch.cat([self.deserializer.from_bytes(bs) for bs in blobs], dim=tdim)
 
     # ---- shutdown ----------------------------------------------------------------------
     def flush(self) -> None:

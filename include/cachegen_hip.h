@@ -243,6 +243,42 @@ int cg_decode_kv(const int16_t *cdf, int max_bins, const void *maxima, int max_d
                  void *out, int out_dt, int64_t ol, int64_t okv, int64_t ot, int64_t oh,
                  void *stream);
 
+/* cg_decode_kv for chunks that lie in several places, each with tables, maxima, lengths, payload
+ * and quantization levels of its own, decoded by one launch into token ranges of one tensor: the
+ * containers a store hands back, without bringing their sections together first.  One entry per
+ * sub-chunk; every pointer is a device pointer.  No counterpart in the reference, which decodes
+ * chunk by chunk and concatenates (cache_engine.py:229-293). */
+typedef struct CgListedSub {
+    const int16_t *cdf;             /* [2L, C, max_bins+1]: tables of the sub-chunk's chunk */
+    const void *maxima;             /* 16-bit: row r's maximum of the sub-chunk's token i at r*maxima_pitch + i */
+    const void *lengths;            /* [2L, C] int32, or uint16 (lengths_u16): bytes of every stream */
+    const uint8_t *bytes;           /* 4-byte aligned; the payload's words are loaded from here ... */
+    int64_t last_word;              /* ... up to the word at this byte offset */
+    int64_t first;                  /* byte offset from `bytes` of the sub-chunk's first stream */
+    const uint32_t *tile_starts;    /* [2L, ceil(C/64)]: bytes from the first stream to stream (row, 64*i) */
+    const float *key_bins, *value_bins;     /* float32 [L] each */
+    int64_t t_out;                  /* the sub-chunk's first token in the output tensor */
+    int32_t n;                      /* its tokens, 1..256 */
+    int32_t maxima_pitch;
+    int32_t max_dt;                 /* CG_DT_* of the maxima */
+    int32_t lengths_u16;
+} CgListedSub;
+
+/* subs: device array of nsub entries; the same max_bins, geometry and delta_group for all of them.
+ * The output arguments and limits are those of cg_decode_kv. */
+int cg_decode_listed(const CgListedSub *subs, int64_t nsub, int max_bins, int64_t L, int64_t H, int64_t D,
+                     int delta_group, void *out, int out_dt, int64_t ol, int64_t okv, int64_t ot, int64_t oh,
+                     void *stream);
+
+/* HOST memory, no GPU work: the running sums of stream lengths that cg_decode_listed starts from.
+ * lengths      [nsub, rows, C] int32, or uint16 (itemsize 2)
+ * tile_starts  uint32 [nsub, rows, ceil(C/64)], written: bytes of the sub-chunk's streams before
+ *              stream (row, 64*i), a stream counting min(length, 256) bytes
+ * sub_bytes    int64 [nsub], written: bytes of every sub-chunk
+ * CG_ERR_ARG if a length is negative. */
+int cg_host_tile_starts(const void *lengths, int itemsize, int64_t nsub, int64_t rows, int64_t C,
+                        uint32_t *tile_starts, int64_t *sub_bytes);
+
 /* ---------------------------------------------------------------------------
  * Tables as histogram counts, for containers that store the counts (no counterpart in
  * the reference, whose container pickles the tables; the relation inverted here is
