@@ -65,7 +65,28 @@ class LMCacheEngine:
     @staticmethod
     def _tuple_kv_to_blob(kv_tensors: KVCache) -> torch.Tensor:
         """Nested tuple -> one tensor with two leading dimensions (layer, key|value)."""
-        return torch.stack([torch.stack(pair, dim=0) for pair in kv_tensors], dim=0)
+        flat = [t for pair in kv_tensors for t in pair]
+        return torch.stack(flat, dim=0).view(len(kv_tensors), 2, *flat[0].shape)
+
+    @staticmethod
+    def _tuple_kv_as_view(kv_tensors: KVCache) -> Optional[torch.Tensor]:
+        """The same tensor without a copy where the tuple's tensors lie at even distances in one
+        storage (a cache that was allocated, or retrieved, in one piece); None where they do not."""
+        first = kv_tensors[0][0]
+        storage = first.untyped_storage().data_ptr()
+        offsets = []
+        for pair in kv_tensors:
+            for t in pair:
+                if t.shape != first.shape or t.stride() != first.stride() or t.dtype != first.dtype \
+                        or t.untyped_storage().data_ptr() != storage:
+                    return None
+                offsets.append(t.storage_offset())
+        to_value = offsets[1] - offsets[0]
+        to_layer = offsets[2] - offsets[0] if len(kv_tensors) > 1 else 2 * to_value
+        if to_value < 0 or to_layer < 0 or any(offsets[2 * l + j] != offsets[0] + l * to_layer + j * to_value
+                                               for l in range(len(kv_tensors)) for j in (0, 1)):
+            return None
+        return first.as_strided((len(kv_tensors), 2, *first.shape), (to_layer, to_value, *first.stride()))
 
     @staticmethod
     def _blob_to_tuple_kv(blob: torch.Tensor) -> KVCache:
@@ -90,7 +111,11 @@ class LMCacheEngine:
             keys.append(None if skip_existing and self.engine_.contains(key) else key)
         n_chunks = 0
         if any(key is not None for key in keys):
-            blob = self._tuple_kv_to_blob(kv_tensors).to(self.device)
+            # a store that copies or encodes what it is given reads the caller's memory in place
+            blob = self._tuple_kv_as_view(kv_tensors) if self.engine_.reads_in_place else None
+            if blob is None:
+                blob = self._tuple_kv_to_blob(kv_tensors)
+            blob = blob.to(self.device)
             n_chunks = self.engine_.put_chunks(keys, blob, self.chunk_size, fmt, blocking=blocking)
         logger.info("Stored/updated %d chunks, total time %.2fs", n_chunks, time.perf_counter() - start)
 

@@ -8,6 +8,10 @@ from ..utils import CacheEngineKey
 
 
 class LMCBackendInterface(metaclass=abc.ABCMeta):
+    # put_chunks has copied or encoded its tensor when it returns, whatever the tensor's strides:
+    # the caller may hand over a view of its own memory
+    reads_in_place = False
+
     @abc.abstractmethod
     def put(self, key: CacheEngineKey, kv_chunk: torch.Tensor, blocking: bool = True) -> None:
         """Store one chunk: a tensor [L, 2, ...] without a batch dimension."""

@@ -13,6 +13,8 @@ logger = logging.getLogger("cachegen_amd")
 
 
 class LMCLocalBackend(LMCBackendInterface):
+    reads_in_place = True
+
     def __init__(self, config: LMCacheEngineConfig):
         self.chunk_size = config.chunk_size
         self.config = config

@@ -28,6 +28,7 @@ class LMCRemoteBackend(LMCBackendInterface):
         self.existing_keys = set()
         self.connection = CreateConnector(config.remote_url)
         self.serializer, self.deserializer = CreateSerde(config.remote_serde, config, metadata)
+        self.reads_in_place = hasattr(self.serializer, "to_bytes_chunks")
         self.put_queue = queue.Queue()          # (key, chunk) or (key, None, blob bytes) for the worker
         self.put_thread = threading.Thread(target=self.put_worker, daemon=True)
         self.put_thread.start()

@@ -327,3 +327,32 @@ def test_gpu_compressing_store_equals_the_serializer_round_trip(fmt, serde, bloc
         else:
             assert torch.equal(d.from_bytes(stored), d.from_bytes(alone))
     engine.close()
+
+
+def test_store_reads_caches_of_any_layout():
+    """A cache whose tensors lie at even distances in one storage is read as a view, any other is
+    stacked first; what is stored does not alias the caller's memory either way."""
+    T, H, D, L = 9, 2, 4, 3
+    whole = torch.randn(L, 2, T, H, D)
+    token_major = torch.randn(T, L, 2, H, D).permute(1, 2, 0, 3, 4)
+    irregular = torch.randn(2 * L + 1, T, H, D)
+    order = [0, 1, 2, 4, 5, 6]
+    caches = {"whole": tuple((l[0], l[1]) for l in whole), "token_major": tuple((l[0], l[1]) for l in token_major),
+              "reversed": tuple((l[1], l[0]) for l in whole),
+              "separate": tuple((l[0].clone(), l[1].clone()) for l in whole),
+              "irregular": tuple((irregular[order[2 * l]], irregular[order[2 * l + 1]]) for l in range(L))}
+    viewed = {k: LMCacheEngine._tuple_kv_as_view(kv) is not None for k, kv in caches.items()}
+    assert viewed == {"whole": True, "token_major": True, "reversed": False, "separate": False, "irregular": False}
+    for kv in caches.values():
+        engine = LMCacheEngine(backend_config("cpu", chunk_size=4), dumb_metadata())
+        tokens = generate_tokens(T, "cpu")
+        want = tuple((k.clone(), v.clone()) for k, v in kv)
+        engine.store(tokens, kv)
+        got, n = engine.retrive(tokens, device="cpu")
+        assert n == T
+        check_kv_cache_equal(want, got, T, "vllm")
+        if kv is caches["whole"]:
+            whole.zero_()
+            again, _ = engine.retrive(tokens, device="cpu")
+            check_kv_cache_equal(want, again, T, "vllm")
+            whole.copy_(torch.stack([torch.stack(p) for p in want]))
