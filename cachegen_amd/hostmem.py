@@ -21,14 +21,32 @@ with warnings.catch_warnings():
     torch.frombuffer(b"\0", dtype=torch.uint8)
 
 
+_libc = ctypes.CDLL(None)
+_libc.madvise.argtypes = [ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int]
+_MADV_HUGEPAGE = 14
+_HUGE_PAGE = 2 << 20
+
+
 def view(buffer) -> torch.Tensor:
     """uint8 tensor over the bytes of any buffer (no copy; not to be written unless the caller owns
     the buffer)."""
     return torch.frombuffer(buffer, dtype=torch.uint8)
 
 
+def uninitialized(n: int) -> bytes:
+    """Bytes object of n bytes with undefined contents (one that is never touched takes no memory)."""
+    return _new(None, n)
+
+
 def new_bytes(n: int):
     """(bytes object of n > 0 bytes with undefined contents, uint8 tensor over them): to be filled
-    through the tensor before anybody else sees the object."""
+    through the tensor before anybody else sees the object.  Memory that is fresh from the system is
+    asked for in huge pages: a page fault per 4 KB costs more than the copy (a 14 MB blob made
+    and dropped again: 0.81 ms in small pages, 0.50 in huge ones; 6 MB: 0.37 and 0.31)."""
     b = _new(None, n)
-    return b, view(b)
+    t = view(b)
+    if n >= 2 * _HUGE_PAGE:
+        at = t.data_ptr()
+        first, last = -(-at // _HUGE_PAGE) * _HUGE_PAGE, (at + n) // _HUGE_PAGE * _HUGE_PAGE
+        _libc.madvise(first, last - first, _MADV_HUGEPAGE)
+    return b, t

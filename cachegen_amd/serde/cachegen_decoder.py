@@ -7,7 +7,7 @@ import torch
 from .. import codec, torchac_hip
 from ..config import LMCacheEngineConfig, LMCacheEngineMetadata
 from . import cachegen_basics as CGBasics
-from . import incoming, wire
+from . import incoming, pickled, wire
 from .cachegen_basics import CacheGenConfig, CacheGenGPUBytestream, CacheGenGPUEncoderOutput
 from .serde import Deserializer
 
@@ -82,7 +82,13 @@ class CacheGenDeserializer(Deserializer):
 
     def _decode(self, bs, out):
         if wire.is_flat(bs):
-            return self._from_flat(bs, out)
+            return self._from_container(incoming.Container.flat(bs), out)
+        container = pickled.container(bs)
+        if container is not None:
+            try:
+                return self._from_container(container, out)
+            except incoming.LengthsError:
+                pass                             # lengths that are not the stored streams': decoded as they say, below
         encoder_output = CacheGenGPUEncoderOutput.from_bytes(bs)
         cdf = encoder_output.cdf.cuda()
         max_k = encoder_output.max_tensors_key.cuda()
@@ -101,8 +107,7 @@ class CacheGenDeserializer(Deserializer):
                                self.value_bins, nlayers, ntokens, encoder_output.num_heads,
                                encoder_output.head_size, chunk_tokens=ntokens, fmt=self.fmt, out=out)
 
-    def _from_flat(self, bs, out=None) -> torch.Tensor:
-        container = incoming.Container.flat(bs)
+    def _from_container(self, container, out=None) -> torch.Tensor:
         L, T, H, D = container.num_layers, container.num_tokens, container.num_heads, container.head_size
         self._check_layers(container)
         if out is None:
@@ -118,14 +123,14 @@ class CacheGenDeserializer(Deserializer):
                              % (container.num_layers, self.key_bins.numel()))
 
     def from_bytes_concat(self, blobs: List[bytes]):
-        """The tensors of several blobs of the flat container side by side along the token
-        dimension, in one tensor that they are decoded into by one launch; None if a blob is of
-        another container (not in the reference, whose callers concatenate the decoded chunks)."""
-        if not all(wire.is_flat(bs) for bs in blobs):
-            return None
+        """The tensors of several blobs side by side along the token dimension, in one tensor that
+        they are decoded into by one launch; None if that takes the blobs one by one (not in the
+        reference, whose callers concatenate the decoded chunks)."""
         items, tokens = [], 0
         for bs in blobs:
-            container = incoming.Container.flat(bs)
+            container = incoming.Container.flat(bs) if wire.is_flat(bs) else pickled.container(bs)
+            if container is None:
+                return None
             self._check_layers(container)
             items.append((container, self.key_bins, self.value_bins, tokens))
             tokens += container.num_tokens
@@ -133,4 +138,7 @@ class CacheGenDeserializer(Deserializer):
         L, H, D = first.num_layers, first.num_heads, first.head_size
         shape = (L, 2, tokens, H, D) if self.fmt == "vllm" else (L, 2, H, tokens, D)
         out = torch.empty(shape, dtype=torch.bfloat16 if self.fmt == "vllm" else torch.float16, device=self.key_bins.device)
-        return incoming.decode(items, out, self.fmt)
+        try:
+            return incoming.decode(items, out, self.fmt)
+        except incoming.LengthsError:
+            return None

@@ -5,7 +5,7 @@ import torch
 from .. import codec, torchac_hip
 from ..config import LMCacheEngineConfig, LMCacheEngineMetadata
 from . import cachegen_basics as CGBasics
-from . import wire
+from . import pickled, wire
 from .cachegen_basics import CacheGenConfig, CacheGenGPUBytestream, CacheGenGPUEncoderOutput
 from .serde import Serializer
 
@@ -89,9 +89,15 @@ class CacheGenSerializer(Serializer):
         if self.wire_format != "pickle":
             enc = codec.encode_kv(tensor.cuda(), self.key_bins, self.value_bins, chunk_tokens=ntokens, max_bins=self.max_bins)
             return wire.pack_chunks(enc, per_chunk=False, compact=self.wire_format == "compact")[0]
-        output = encode_function(tensor.cuda(), self.cachegen_config, self.key_bins,
-                                 self.value_bins, ntokens)
-        return output.to_bytes()
+        enc = codec.encode_kv(tensor.cuda(), self.key_bins, self.value_bins, chunk_tokens=ntokens, max_bins=self.max_bins)
+        return self._pickled(enc)[0]
+
+    def _pickled(self, enc):
+        if pickled.can_write(enc):
+            return pickled.pack_chunks(enc)
+        enc.check()
+        bounds = enc.sub_boundaries()
+        return [_chunk_output(enc, i, bounds, enc.num_heads, enc.head_size).to_bytes() for i in range(enc.num_chunks)]
 
     def to_bytes_chunks(self, tensor: torch.Tensor, chunk_size: int):
         """One blob per `chunk_size` tokens of `tensor` (same layouts as `to_bytes`), each equal
@@ -99,10 +105,7 @@ class CacheGenSerializer(Serializer):
         tensor (not in the reference, whose callers loop over `to_bytes`)."""
         if self.fmt == "huggingface":
             tensor = tensor.permute(0, 1, 3, 2, 4)
-        num_heads, head_size = tensor.shape[-2:]
         enc = codec.encode_kv(tensor.cuda(), self.key_bins, self.value_bins, chunk_tokens=chunk_size, max_bins=self.max_bins)
         if self.wire_format != "pickle":
             return wire.pack_chunks(enc, compact=self.wire_format == "compact")
-        enc.check()
-        bounds = enc.sub_boundaries()
-        return [_chunk_output(enc, i, bounds, num_heads, head_size).to_bytes() for i in range(enc.num_chunks)]
+        return self._pickled(enc)

@@ -29,6 +29,10 @@ def _up(n, a=_ALIGN):
     return (n + a - 1) // a * a
 
 
+class LengthsError(ValueError):
+    """A container's stream lengths do not fit its payload."""
+
+
 class Container:
     """One container in host memory: its geometry, and where its sections lie in an area of `size`
     bytes that `pieces` ((offset, uint8 host tensor), in order) fill."""
@@ -39,7 +43,7 @@ class Container:
         self.bf16_maxima, self.lengths_u16 = bf16_maxima, lengths_u16
         self.pieces, self.size = [], 0
         self.tables = self.maxima = self.lengths = self.payload = self.payload_bytes = 0     # offsets in the area
-        self.length_arrays = []          # (host address, sub-chunks) of the stream lengths
+        self.length_arrays = []          # (host tensor, sub-chunks) of the stream lengths
         self.symbols = None              # count tables: stored symbols per (chunk, row), uint8 on the host
 
     @classmethod
@@ -53,10 +57,17 @@ class Container:
         c.pieces, c.size = [(0, whole)], whole.numel()
         c.tables, c.maxima, c.lengths, c.payload = (geo[k][0] for k in ("cdf", "maxima", "lengths", "payload"))
         c.payload_bytes = h["payload_bytes"]
-        c.length_arrays = [(whole.data_ptr() + c.lengths, h["nsub"])]
+        c.length_arrays = [(whole[c.lengths:], h["nsub"])]
         if h["count_tables"]:
             c.symbols = wire.table_symbol_counts(blob, h)
         return c
+
+    def add(self, host, align=64):
+        """Appends a section's bytes to the area; returns their offset."""
+        at = _up(self.size, align)
+        self.pieces.append((at, host))
+        self.size = at + host.numel()
+        return at
 
     def tile_starts(self, into: np.ndarray, sub_bytes: np.ndarray) -> None:
         """Fills the running sums (uint32, see CgListedSub) and the bytes of every sub-chunk;
@@ -64,14 +75,14 @@ class Container:
         rows, C = 2 * self.num_layers, self.num_heads * self.head_size
         per_sub = rows * -(-C // 64)
         at = 0
-        for address, nsub in self.length_arrays:
-            rc = _lib.lib().cg_host_tile_starts(address, 2 if self.lengths_u16 else 4, nsub, rows, C,
+        for lengths, nsub in self.length_arrays:
+            rc = _lib.lib().cg_host_tile_starts(lengths.data_ptr(), 2 if self.lengths_u16 else 4, nsub, rows, C,
                                                 into[at * per_sub:].ctypes.data, sub_bytes[at:].ctypes.data)
             if rc != _lib.CG_OK:
-                raise ValueError("wire container: payload size is not the sum of the stream lengths")
+                raise LengthsError("wire container: payload size is not the sum of the stream lengths")
             at += nsub
         if int(sub_bytes.sum()) != self.payload_bytes:
-            raise ValueError("wire container: payload size is not the sum of the stream lengths")
+            raise LengthsError("wire container: payload size is not the sum of the stream lengths")
 
 
 def _upload(pieces, total, index_at, write_index, device):

@@ -1,0 +1,289 @@
+"""The reference's pickle container without its copies.
+
+The container is a pickle of `CacheGenGPUEncoderOutput` (cachegen_basics.py:110-131 in the
+reference): a few hundred bytes of structure around one torch-saved storage per tensor.  Pickling
+the tensors reads every one back from the GPU by itself, and copies its bytes into a stream, into a
+bytes object and into the pickle; unpickling does the same in reverse.  Here the structure goes
+through the pickle module with stand-ins for the tensors, and the storages' bytes go straight
+between the blob and pinned memory: the same pickle, with one copy of the bytes.
+
+What a torch-saved storage looks like is taken from torch itself once (`_storage_template`); a
+storage that looks different is left to the plain unpickler."""
+import collections
+import ctypes
+import io
+import pickle
+import re
+import struct
+
+import numpy as np
+import torch
+
+from .. import hostmem
+from . import wire
+from .cachegen_basics import CacheGenGPUBytestream, CacheGenGPUEncoderOutput, _ContainerUnpickler
+from .incoming import Container
+
+_STORAGE_NAMES = {torch.uint8: "Byte", torch.int16: "Short", torch.int32: "Int", torch.float16: "Half", torch.bfloat16: "BFloat16"}
+_DTYPES = {name.encode(): dtype for dtype, name in _STORAGE_NAMES.items()}
+_LARGE = 1 << 16            # bytes objects of this size and more pass through a pickler's file uncopied
+_as_string = ctypes.pythonapi.PyBytes_AsString
+_as_string.restype = ctypes.c_void_p
+_as_string.argtypes = [ctypes.py_object]
+
+
+def _text(s: bytes) -> bytes:
+    return b"X" + struct.pack("<I", len(s)) + s
+
+
+def _storage_template():
+    """(what precedes, what lies between) the parts of a torch-saved storage that vary: its type,
+    key, location and size; None if torch writes something this module does not know."""
+    taken = []
+
+    class Spy(pickle.Unpickler):
+        def find_class(self, module, name):
+            if (module, name) == ("torch.storage", "_load_from_bytes"):
+                return lambda b: taken.append(b)
+            return lambda *a: None
+    Spy(io.BytesIO(pickle.dumps(torch.zeros(3, dtype=torch.uint8), protocol=4))).load()
+    saved = taken[0] if taken else b""
+    m = re.fullmatch(rb"(?s)(.*\nByte)(Storage\nq\x01)X....(\d+)(q\x02)X\x03\0\0\0cpu(q\x03)K\x03(Ntq\x04Q\..*)X....(\d+)(q\x01a\.)\x03\0{10}", saved)
+    if not m or m.group(3) != m.group(7):
+        return None
+    return m.group(1)[:-len("Byte")], m.group(2), m.group(4), m.group(5), m.group(6), m.group(8)
+
+
+_TEMPLATE = _storage_template()
+_PREFIX = None
+if _TEMPLATE is not None:
+    _head, _a, _b, _c, _d, _e = (re.escape(t) for t in _TEMPLATE)
+    _PREFIX = re.compile(rb"(?s)" + _head + rb"(\w{3,8})" + _a + rb"X....\d{1,20}" + _b + rb"X....[a-z]{1,8}(?::\d{1,3})?" + _c
+                         + rb"(?:K.|M..|J....|\x8a[\x04-\x08].{4,8}?)" + _d + rb"X....\d{1,20}" + _e + rb"(.{8})")
+
+
+def _storage_prefix(dtype, location: bytes, numel: int, key: bytes) -> bytes:
+    head, a, b, c, d, e = _TEMPLATE
+    size = pickle.dumps(numel, protocol=2)[2:-1]            # the number's opcode, without the frame around it
+    return (head + _STORAGE_NAMES[dtype].encode() + a + _text(key) + b + _text(location) + c + size + d + _text(key) + e
+            + struct.pack("<q", numel))
+
+
+class _Reduced:
+    """Pickles as the given call."""
+
+    def __init__(self, fn, args):
+        self._as = (fn, args)
+
+    def __reduce__(self):
+        return self._as
+
+
+class _Pieces:
+    """File of a pickler: keeps what is written, large bytes objects as they are."""
+
+    def __init__(self):
+        self.pieces = []
+
+    def write(self, b):
+        self.pieces.append(b if type(b) is bytes else bytes(b))
+
+
+class _Writer:
+    """One blob: tensors are added as host memory, `finish` writes the blob."""
+
+    def __init__(self, location: str):
+        self.location = location.encode()
+        self.large = {}              # id of a stand-in bytes object -> (object, prefix, host tensor)
+        self.count = 0
+
+    def tensor(self, host, dtype, shape):
+        """Stand-in for a contiguous device tensor of this type and shape whose bytes are `host`
+        (uint8 tensor); the bytes are read in `finish`."""
+        numel = int(np.prod(shape, dtype=np.int64))
+        self.count += 1
+        prefix = _storage_prefix(dtype, self.location, numel, b"%d" % self.count)
+        n = len(prefix) + host.numel()
+        if n >= _LARGE:
+            saved = hostmem.uninitialized(n)             # never touched: only its size counts
+            self.large[id(saved)] = (saved, prefix, host)
+        else:
+            saved = prefix + host.numpy().tobytes()
+        stride, acc = [], 1
+        for s in reversed(shape):
+            stride.append(acc)
+            acc *= s
+        storage = _Reduced(torch.storage._load_from_bytes, (saved,))
+        return _Reduced(torch._utils._rebuild_tensor_v2, (storage, 0, tuple(shape), tuple(reversed(stride)), False,
+                                                          collections.OrderedDict()))
+
+    def finish(self, output: CacheGenGPUEncoderOutput) -> bytes:
+        f = _Pieces()
+        pickle.dump(output, f, protocol=4)
+        blob, into = hostmem.new_bytes(sum(len(p) for p in f.pieces))
+        raw, at, seen = into.numpy(), 0, 0
+        for p in f.pieces:
+            big = self.large.get(id(p))
+            if big is None:
+                raw[at:at + len(p)] = np.frombuffer(p, dtype=np.uint8)
+            else:
+                _, prefix, host = big
+                seen += 1
+                raw[at:at + len(prefix)] = np.frombuffer(prefix, dtype=np.uint8)
+                into[at + len(prefix):at + len(p)].copy_(host)
+            at += len(p)
+        if seen != len(self.large):
+            raise RuntimeError("pickle: a stand-in was copied instead of passed through")
+        return blob
+
+
+def can_write(enc) -> bool:
+    return _TEMPLATE is not None and enc.max_bins > 0
+
+
+def pack_chunks(enc):
+    """One pickle blob per chunk of an `EncodedKV`, each what pickling the chunk's
+    `CacheGenGPUEncoderOutput` gives."""
+    L, H, D = enc.num_layers, enc.num_heads, enc.head_size
+    rows, C = 2 * L, H * D
+    blobs = []
+    for part in wire.bring_to_host(enc, 0, enc.num_chunks):
+        w = _Writer(str(enc.payload.device))
+        T = part.t1 - part.t0
+        maxima = torch.from_numpy(np.ascontiguousarray(part.maxima).view(np.uint8).reshape(-1))
+        half = maxima.numel() // 2
+        chunks, at = [], 0
+        per_sub = rows * C * 4
+        for g, nbytes in enumerate(part.sub_bytes):
+            chunks.append(CacheGenGPUBytestream(
+                bytestream=w.tensor(part.payload[at:at + nbytes], torch.uint8, (nbytes,)),
+                bytestream_lengths=w.tensor(part.lengths[g * per_sub:(g + 1) * per_sub], torch.int32, (rows, C)),
+                ntokens=min(wire.MAX_STREAM_BYTES, T - g * wire.MAX_STREAM_BYTES)))
+            at += nbytes
+        out = CacheGenGPUEncoderOutput(
+            chunks, w.tensor(part.tables, torch.int16, (rows, C, enc.max_bins + 1)),
+            max_tensors_key=w.tensor(maxima[:half], enc.maxima.dtype, (L, T, 1)),
+            max_tensors_value=w.tensor(maxima[half:], enc.maxima.dtype, (L, T, 1)), num_heads=H, head_size=D)
+        blobs.append(w.finish(out))
+    return blobs
+
+
+# ---- reading -------------------------------------------------------------------------------
+class _NotPlain(Exception):
+    """The blob is not laid out the way this module reads: the plain unpickler takes it."""
+
+
+class _Source:
+    """File of an unpickler over a blob: large bytes objects are not filled but remembered by
+    their address, with their place in the blob."""
+
+    def __init__(self, blob):
+        self.mv, self.pos, self.skipped = memoryview(blob), 0, {}
+
+    def read(self, n=-1):
+        b = self.mv[self.pos:] if n < 0 else self.mv[self.pos:self.pos + n]
+        self.pos += len(b)
+        return bytes(b)
+
+    def readline(self):
+        raise _NotPlain("text opcodes")
+
+    def readinto(self, buf):
+        n = min(len(buf), len(self.mv) - self.pos)
+        if n >= _LARGE:
+            self.skipped[np.frombuffer(buf, dtype=np.uint8).ctypes.data] = (self.pos, n)
+        else:
+            buf[:n] = self.mv[self.pos:self.pos + n]
+        self.pos += n
+        return n
+
+
+class _Tensor:
+    """A tensor of the container: its bytes in host memory."""
+
+    def __init__(self, dtype, host, shape):
+        self.dtype, self.host, self.shape = dtype, host, shape
+
+
+class _Reader(_ContainerUnpickler):
+    """Admits what `_ContainerUnpickler` admits, with tensors left where their bytes are."""
+
+    def __init__(self, source, whole):
+        super().__init__(source)
+        self._source, self._whole = source, whole
+
+    def _storage(self, b):
+        place = self._source.skipped.pop(_as_string(b), None) if type(b) is bytes else None
+        if place is None:
+            head, data = b[:4096], hostmem.view(b)
+        else:
+            data = self._whole[place[0]:place[0] + place[1]]
+            head = data[:4096].numpy().tobytes()
+        m = _PREFIX.match(head)
+        if not m or m.group(1) not in _DTYPES:
+            raise _NotPlain("storage")
+        dtype, numel = _DTYPES[m.group(1)], struct.unpack("<q", m.group(2))[0]
+        data = data[m.end():]
+        if data.numel() != numel * dtype.itemsize:
+            raise _NotPlain("storage size")
+        return dtype, data
+
+    def _tensor(self, storage, offset, shape, stride, *rest):
+        dtype, data = storage
+        acc = 1
+        for s, st in zip(reversed(shape), reversed(stride)):
+            if s != 1 and st != acc:
+                raise _NotPlain("strides")
+            acc *= s
+        size = dtype.itemsize
+        if offset < 0 or (offset + acc) * size > data.numel():
+            raise _NotPlain("tensor outside its storage")
+        return _Tensor(dtype, data[offset * size:(offset + acc) * size], tuple(shape))
+
+    def find_class(self, module, name):
+        if (module, name) == ("torch._utils", "_rebuild_tensor_v2"):
+            return self._tensor
+        if (module, name) == ("torch.storage", "_load_from_bytes"):
+            return self._storage
+        return super().find_class(module, name)
+
+
+def container(blob):
+    """The pickle container as an `incoming.Container`, or None where the blob is not laid out as
+    this module (or the reference on the same torch) writes it."""
+    if _PREFIX is None:
+        return None
+    whole = hostmem.view(blob)
+    try:
+        out = _Reader(_Source(blob), whole).load()
+        cdf, k, v = out.cdf, out.max_tensors_key, out.max_tensors_value
+        rows, C, lp = cdf.shape
+        L, T = k.shape[:2]
+        chunks = out.data_chunks
+        maxima_types = (torch.float16, torch.bfloat16)
+        fine = (rows == 2 * L and lp >= 2 and cdf.dtype is torch.int16 and out.num_heads * out.head_size == C and T > 0
+                and k.dtype in maxima_types and v.dtype is k.dtype and v.shape[:2] == (L, T)
+                and k.host.numel() == v.host.numel() == 2 * L * T and len(chunks) == -(-T // wire.MAX_STREAM_BYTES))
+        for g, c in enumerate(chunks if fine else ()):
+            fine = (fine and c.bytestream.dtype is torch.uint8 and c.bytestream_lengths.dtype is torch.int32
+                    and c.bytestream_lengths.shape == (rows, C)
+                    and c.ntokens == min(wire.MAX_STREAM_BYTES, T - g * wire.MAX_STREAM_BYTES))
+    except (_NotPlain, AttributeError, TypeError, ValueError, KeyError):
+        return None
+    if not fine:
+        return None
+    c = Container(L, T, out.num_heads, out.head_size, T, lp - 1, 0, k.dtype is torch.bfloat16, False)
+    c.tables = c.add(cdf.host)
+    c.maxima = c.add(k.host)
+    c.add(v.host, align=1)
+    for i, chunk in enumerate(chunks):
+        at = c.add(chunk.bytestream_lengths.host, align=64 if i == 0 else 1)
+        if i == 0:
+            c.lengths = at
+        c.length_arrays.append((chunk.bytestream_lengths.host, 1))
+    for i, chunk in enumerate(chunks):
+        at = c.add(chunk.bytestream.host, align=64 if i == 0 else 1)
+        if i == 0:
+            c.payload = at
+        c.payload_bytes += chunk.bytestream.host.numel()
+    return c

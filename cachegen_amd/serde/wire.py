@@ -339,29 +339,28 @@ def _device_tables(nsym_host, nsym_dev, data, C, lp, tokens):
 _PIECE_BYTES = 4 << 20
 
 
-def pack_chunks(enc, first_chunk: int = 0, num_chunks: Optional[int] = None, per_chunk: bool = True,
-                compact: bool = False) -> List[bytes]:
-    """Blobs for chunks [first_chunk, first_chunk + num_chunks) of an `EncodedKV`: one blob per
-    chunk (what one `to_bytes` call of the reference covers) or, with per_chunk=False, a single
-    blob holding all of them; compact: version 2.
+class HostPart:
+    """Chunks [first, last) of an encoded tensor in (pinned) host memory, one blob's worth: uint8
+    tensors `tables`, `lengths`, `payload` as they lie on the device, `maxima` (uint16 numpy view
+    [2L, tokens]), `sub_bytes` (payload bytes per sub-chunk), tokens [t0, t1).  `symbols`: stored
+    symbols per (chunk, row) where `tables` holds histogram counts, else None; `lengths_itemsize` 2
+    or 4."""
 
-    The blob's sections leave the encoder's own tensors for pinned memory as they are and are put
-    together on the host, where the blob has to be written anyway: no second copy of them on the
+
+def bring_to_host(enc, first_chunk, num_chunks, per_chunk=True, compact=False):
+    """Yields a HostPart per chunk (or one for all of them) once its bytes have arrived.
+
+    The sections leave the encoder's own tensors for pinned memory as they are; blobs are put
+    together on the host, where they have to be written anyway: no second copy of them on the
     device.  The host waits for the device once for the sizes (status, payload offsets, symbol
     counts, stored into pinned memory by one kernel) while the tables, whose size it knows, are
     already on the bus, and then for each piece of about _PIECE_BYTES."""
     import torch
-    from .. import _lib, hostmem
-    nch = enc.num_chunks
-    if num_chunks is None:
-        num_chunks = nch - first_chunk
-    if first_chunk < 0 or num_chunks <= 0 or first_chunk + num_chunks > nch:
-        raise ValueError("chunk range outside the encoded tensor")
+    from .. import _lib
     L, H, D, S, T = enc.num_layers, enc.num_heads, enc.head_size, enc.chunk_tokens, enc.num_tokens
     C = H * D
     rows = 2 * L
     spc = enc.subchunks_per_chunk
-    bf16 = enc.maxima.dtype == torch.bfloat16
     c_first, c_last = first_chunk, first_chunk + num_chunks
     g_first, g_last = c_first * spc, min(c_last * spc, enc.lengths.shape[0])
     tokens = chunk_token_counts(T, S)[c_first:c_last]
@@ -380,6 +379,12 @@ def pack_chunks(enc, first_chunk: int = 0, num_chunks: Optional[int] = None, per
         event.record()
         return event
 
+    def subs(c):
+        return min(c * spc, g_last) - g_first
+
+    # blobs by pieces: (first blob, last blob) covering about _PIECE_BYTES of tables and lengths
+    groups = [(c, c + 1) for c in range(c_first, c_last)] if per_chunk else [(c_first, c_last)]
+    early = {}                                           # the first piece's tables and lengths: sizes not needed
     with torch.cuda.device(dev):
         stream = _stream()
         cdf = enc.cdf[c_first:c_last]
@@ -399,18 +404,10 @@ def pack_chunks(enc, first_chunk: int = 0, num_chunks: Optional[int] = None, per
         _lib.check(lib.cg_wire_meta(enc.status.data_ptr(), enc.offsets[g_first * rows * C:].data_ptr(), rows * C, nbounds,
                                     ptr(wide), ptr(inexact), ptr(nsym), ngroups, meta.data_ptr(), stream))
         sizes_known = mark()
-
-        # blobs by pieces: (first blob, last blob) covering about _PIECE_BYTES of tables and lengths
-        groups = [(c, c + 1) for c in range(c_first, c_last)] if per_chunk else [(c_first, c_last)]
         chunk_bytes = max(1, cdf[0].numel() * cdf.element_size() + min(spc, lengths.shape[0]) * rows * C * 4)
         step = max(1, _PIECE_BYTES // chunk_bytes) if per_chunk else 1
         pieces = [(i, min(i + step, len(groups))) for i in range(0, len(groups), step)]
-
-        def subs(c):
-            return min(c * spc, g_last) - g_first
-
         tables_src, lengths_src = cdf, lengths
-        early = {}                                       # the first piece's tables and lengths, sizes not needed
         if dense is not None:
             # ragged count bytes; their places follow from nsym, which is on the device
             tables_src = torch.empty(dense.numel(), dtype=torch.uint8, device=dev)
@@ -419,81 +416,104 @@ def pack_chunks(enc, first_chunk: int = 0, num_chunks: Optional[int] = None, per
         elif not compact:
             a, b = groups[0][0], groups[pieces[0][1] - 1][1]
             early = {"tables": fetch(cdf[a - c_first:b - c_first]), "lengths": fetch(lengths[subs(a):subs(b)])}
-        maxima = fetch(enc.maxima).numpy().view(np.uint16).reshape(rows, T)
+        maxima = fetch(enc.maxima)
 
-        sizes_known.synchronize()
-        meta = meta.tolist()
-        enc.raise_for_status(meta[0])
-        bounds = meta[3:3 + nbounds]
-        version, flags = VERSION, 0
-        starts = None                                    # byte offset of every chunk's counts in tables_src
-        if compact:
-            version = VERSION_COMPACT
-            if dense is not None:
-                if meta[2]:
-                    tables_src = cdf                     # not the tables of histograms: stored as they are
-                else:
-                    ks = np.asarray(meta[3 + nbounds:], dtype=np.uint8)
-                    starts = [0] + np.cumsum(ks.reshape(-1, rows).sum(axis=1, dtype=np.int64) * C).tolist()
-                    flags |= FLAG_COUNT_TABLES
-            if not meta[1]:
-                lengths_src = lengths16                  # bit pattern of the uint16 value
-                flags |= FLAG_LENGTHS_U16
+    sizes_known.synchronize()
+    meta = meta.tolist()
+    enc.raise_for_status(meta[0])
+    bounds = meta[3:3 + nbounds]
+    symbols = starts = None                              # starts: byte offset of every chunk's counts in tables_src
+    if compact:
+        if dense is not None:
+            if meta[2]:
+                tables_src = cdf                         # not the tables of histograms: stored as they are
+            else:
+                symbols = np.asarray(meta[3 + nbounds:], dtype=np.uint8)
+                starts = [0] + np.cumsum(symbols.reshape(-1, rows).sum(axis=1, dtype=np.int64) * C).tolist()
+        if not meta[1]:
+            lengths_src = lengths16                      # bit pattern of the uint16 value
 
-        def table_range(a, b):
-            if starts is not None:
-                return tables_src[starts[a - c_first]:starts[b - c_first]]
-            return tables_src[a - c_first:b - c_first]
+    def table_range(a, b):
+        if starts is not None:
+            return tables_src[starts[a - c_first]:starts[b - c_first]]
+        return tables_src[a - c_first:b - c_first]
 
-        def queue(piece):
-            a, b = groups[piece[0]][0], groups[piece[1] - 1][1]
-            p0, p1 = bounds[subs(a)], bounds[subs(b)]
+    def queue(piece):
+        a, b = groups[piece[0]][0], groups[piece[1] - 1][1]
+        p0, p1 = bounds[subs(a)], bounds[subs(b)]
+        with torch.cuda.device(dev):
             tables = early.pop("tables", None)
             lens = early.pop("lengths", None)
-            host = {"tables": fetch(table_range(a, b)) if tables is None else tables,
-                    "lengths": fetch(lengths_src[subs(a):subs(b)]) if lens is None else lens,
-                    "payload": fetch(enc.payload[p0:p1]) if p1 > p0 else None}
-            return host, mark()
+            return (fetch(table_range(a, b)) if tables is None else tables,
+                    fetch(lengths_src[subs(a):subs(b)]) if lens is None else lens,
+                    fetch(enc.payload[p0:p1])), mark()
 
-        blobs = []
-        queued = queue(pieces[0])
-        for k, piece in enumerate(pieces):
-            (host, arrived), queued = queued, queue(pieces[k + 1]) if k + 1 < len(pieces) else None
-            at = {"tables": 0, "lengths": 0, "payload": 0}
-            made = []
-            for a, b in groups[piece[0]:piece[1]]:       # everything but the big sections, while these arrive
-                t0, t1 = a * S, min(b * S, T)
-                nbytes = bounds[subs(b)] - bounds[subs(a)]
-                tables_bytes = None if starts is None else (b - a) * rows + starts[b - c_first] - starts[a - c_first]
-                table_tokens = min(S, t1 - t0)           # a short last chunk is a blob of its own length
-                geo = geometry(L, t1 - t0, H, D, table_tokens, enc.max_bins, nbytes, tables_bytes, lengths_src.element_size())
-                head = write_header(L, t1 - t0, H, D, table_tokens, enc.max_bins, enc.delta_group, subs(b) - subs(a), nbytes,
-                                    bf16, version, flags, tables_bytes or 0)
-                blob, into = hostmem.new_bytes(geo["total"][0])
-                parts = [(0, head)]
-                if starts is not None:
-                    parts.append((HEADER_BYTES, ks[(a - c_first) * rows:(b - c_first) * rows].tobytes()))
-                made.append((blob, into, geo, parts, t0, t1))
-            arrived.synchronize()
-            for blob, into, geo, parts, t0, t1 in made:
-                raw = into.numpy()
-                end = 0
-                for off, head in parts:
-                    raw[off:off + len(head)] = np.frombuffer(head, dtype=np.uint8)
-                    end = off + len(head)
-                for name, section in (("tables", "cdf"), ("maxima", "maxima"), ("lengths", "lengths"), ("payload", "payload")):
-                    off, size = geo[section]
-                    start = max(off, end)
-                    raw[end:start] = 0                   # the gap before the section
-                    n = off + size - start               # count tables: the symbol counts are there already
-                    if name == "maxima":
-                        np.copyto(raw[start:start + n].view(np.uint16).reshape(rows, t1 - t0), maxima[:, t0:t1])
-                    elif n:
-                        into[start:start + n].copy_(host[name][at[name]:at[name] + n])
-                        at[name] += n
-                    end = off + size
-                raw[end:] = 0
-                blobs.append(blob)
+    itemsize = lengths_src.element_size()
+    queued = queue(pieces[0])
+    for k, piece in enumerate(pieces):
+        ((tables, lens, payload), arrived), queued = queued, queue(pieces[k + 1]) if k + 1 < len(pieces) else None
+        arrived.synchronize()
+        at = [0, 0, 0]
+        for a, b in groups[piece[0]:piece[1]]:
+            part = HostPart()
+            part.first, part.last = a, b
+            part.t0, part.t1 = a * S, min(b * S, T)
+            part.sub_bytes = [bounds[g + 1] - bounds[g] for g in range(subs(a), subs(b))]
+            n = [(starts[b - c_first] - starts[a - c_first]) if starts is not None else (b - a) * cdf[0].numel() * 2,
+                 len(part.sub_bytes) * rows * C * itemsize, sum(part.sub_bytes)]
+            part.tables, part.lengths, part.payload = (t[i:i + j] for t, i, j in zip((tables, lens, payload), at, n))
+            at = [i + j for i, j in zip(at, n)]
+            part.maxima = maxima.numpy().view(np.uint16).reshape(rows, T)[:, part.t0:part.t1]
+            part.symbols = None if symbols is None else symbols[(a - c_first) * rows:(b - c_first) * rows]
+            part.lengths_itemsize = itemsize
+            yield part
+
+
+def pack_chunks(enc, first_chunk: int = 0, num_chunks: Optional[int] = None, per_chunk: bool = True,
+                compact: bool = False) -> List[bytes]:
+    """Blobs for chunks [first_chunk, first_chunk + num_chunks) of an `EncodedKV`: one blob per
+    chunk (what one `to_bytes` call of the reference covers) or, with per_chunk=False, a single
+    blob holding all of them; compact: version 2."""
+    import torch
+    from .. import hostmem
+    nch = enc.num_chunks
+    if num_chunks is None:
+        num_chunks = nch - first_chunk
+    if first_chunk < 0 or num_chunks <= 0 or first_chunk + num_chunks > nch:
+        raise ValueError("chunk range outside the encoded tensor")
+    L, H, D = enc.num_layers, enc.num_heads, enc.head_size
+    bf16 = enc.maxima.dtype == torch.bfloat16
+    blobs = []
+    for part in bring_to_host(enc, first_chunk, num_chunks, per_chunk, compact):
+        T = part.t1 - part.t0
+        nbytes = part.payload.numel()
+        flags, tables_bytes = 0, None
+        if part.symbols is not None:
+            flags |= FLAG_COUNT_TABLES
+            tables_bytes = part.symbols.size + part.tables.numel()
+        if part.lengths_itemsize == 2:
+            flags |= FLAG_LENGTHS_U16
+        table_tokens = min(enc.chunk_tokens, T)          # a short last chunk is a blob of its own length
+        geo = geometry(L, T, H, D, table_tokens, enc.max_bins, nbytes, tables_bytes, part.lengths_itemsize)
+        head = write_header(L, T, H, D, table_tokens, enc.max_bins, enc.delta_group, len(part.sub_bytes), nbytes, bf16,
+                            VERSION_COMPACT if compact else VERSION, flags, tables_bytes or 0)
+        if part.symbols is not None:
+            head += part.symbols.tobytes()
+        blob, into = hostmem.new_bytes(geo["total"][0])
+        raw = into.numpy()
+        end = len(head)
+        raw[:end] = np.frombuffer(head, dtype=np.uint8)
+        for section, src in (("cdf", part.tables), ("maxima", part.maxima), ("lengths", part.lengths), ("payload", part.payload)):
+            off, size = geo[section]
+            start = max(off, end)                        # count tables: the symbol counts are there already
+            raw[end:start] = 0                           # the gap before the section
+            end = off + size
+            if section == "maxima":
+                np.copyto(raw[start:end].view(np.uint16).reshape(2 * L, T), src)
+            else:
+                into[start:end].copy_(src)
+        raw[end:] = 0
+        blobs.append(blob)
     return blobs
 
 
