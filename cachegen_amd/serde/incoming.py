@@ -87,17 +87,16 @@ class Container:
 
 def _upload(pieces, total, index_at, write_index, device):
     """Device buffer of `total` bytes holding the pieces ((offset, host tensor), in order) and, from
-    index_at on, what write_index(uint8 tensor in pinned memory) puts there; write_index runs while
-    the pieces before it are on the bus."""
+    index_at on, what write_index(device address, uint8 tensor in pinned memory) puts there;
+    write_index runs while the pieces before it are on the bus."""
     buf = torch.empty(total, dtype=torch.uint8, device=device)
-    step = total if total <= _WHOLE_BYTES else _PIECE_BYTES
+    step = index_at if index_at <= _WHOLE_BYTES else _PIECE_BYTES
     k = 0
     for p0 in range(0, index_at, step):
         p1 = min(p0 + step, index_at)
-        last = p1 == index_at
         # pinned blocks come from and go back to torch's pool, which reuses one only when the copy
         # out of it is through
-        host = torch.empty((total if last else p1) - p0, dtype=torch.uint8, pin_memory=True)
+        host = torch.empty(p1 - p0, dtype=torch.uint8, pin_memory=True)
         while k < len(pieces) and pieces[k][0] < p1:
             off, src = pieces[k]
             a, b = max(off, p0), min(off + src.numel(), p1)
@@ -105,9 +104,10 @@ def _upload(pieces, total, index_at, write_index, device):
             if off + src.numel() > p1:
                 break
             k += 1
-        if last:
-            write_index(buf.data_ptr(), host[index_at - p0:])
-        buf[p0:p0 + host.numel()].copy_(host, non_blocking=True)
+        buf[p0:p1].copy_(host, non_blocking=True)
+    host = torch.empty(total - index_at, dtype=torch.uint8, pin_memory=True)
+    write_index(buf.data_ptr(), host)
+    buf[index_at:].copy_(host, non_blocking=True)
     return buf
 
 

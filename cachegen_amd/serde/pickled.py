@@ -10,7 +10,6 @@ between the blob and pinned memory: the same pickle, with one copy of the bytes.
 What a torch-saved storage looks like is taken from torch itself once (`_storage_template`); a
 storage that looks different is left to the plain unpickler."""
 import collections
-import ctypes
 import io
 import pickle
 import re
@@ -26,10 +25,10 @@ from .incoming import Container
 
 _STORAGE_NAMES = {torch.uint8: "Byte", torch.int16: "Short", torch.int32: "Int", torch.float16: "Half", torch.bfloat16: "BFloat16"}
 _DTYPES = {name.encode(): dtype for dtype, name in _STORAGE_NAMES.items()}
-_LARGE = 1 << 16            # bytes objects of this size and more pass through a pickler's file uncopied
-_as_string = ctypes.pythonapi.PyBytes_AsString
-_as_string.restype = ctypes.c_void_p
-_as_string.argtypes = [ctypes.py_object]
+# A pickler hands bytes objects of this size and more to its file as they are, after a piece that
+# ends with their opcode and length, and puts no frame around them.
+_LARGE = 1 << 16
+_LARGE_HEADER = b"B" + struct.pack("<I", _LARGE)
 
 
 def _text(s: bytes) -> bytes:
@@ -94,7 +93,7 @@ class _Writer:
 
     def __init__(self, location: str):
         self.location = location.encode()
-        self.large = {}              # id of a stand-in bytes object -> (object, prefix, host tensor)
+        self.large = {}              # id of a stand-in bytes object of _LARGE bytes -> (object, prefix, host tensor)
         self.count = 0
 
     def tensor(self, host, dtype, shape):
@@ -105,7 +104,7 @@ class _Writer:
         prefix = _storage_prefix(dtype, self.location, numel, b"%d" % self.count)
         n = len(prefix) + host.numel()
         if n >= _LARGE:
-            saved = hostmem.uninitialized(n)             # never touched: only its size counts
+            saved = bytes(_LARGE)
             self.large[id(saved)] = (saved, prefix, host)
         else:
             saved = prefix + host.numpy().tobytes()
@@ -120,20 +119,31 @@ class _Writer:
     def finish(self, output: CacheGenGPUEncoderOutput) -> bytes:
         f = _Pieces()
         pickle.dump(output, f, protocol=4)
-        blob, into = hostmem.new_bytes(sum(len(p) for p in f.pieces))
-        raw, at, seen = into.numpy(), 0, 0
+        parts, seen = [], 0                              # small bytes objects and host tensors
         for p in f.pieces:
             big = self.large.get(id(p))
             if big is None:
-                raw[at:at + len(p)] = np.frombuffer(p, dtype=np.uint8)
-            else:
-                _, prefix, host = big
-                seen += 1
-                raw[at:at + len(prefix)] = np.frombuffer(prefix, dtype=np.uint8)
-                into[at + len(prefix):at + len(p)].copy_(host)
-            at += len(p)
+                parts.append(p)
+                continue
+            _, prefix, host = big
+            seen += 1
+            if not parts[-1].endswith(_LARGE_HEADER):
+                raise RuntimeError("pickle: a stand-in without its header")
+            n = len(prefix) + host.numel()               # the stand-in's length becomes the storage's
+            header = b"B" + struct.pack("<I", n) if n < 1 << 32 else b"\x8e" + struct.pack("<Q", n)
+            parts[-1] = parts[-1][:-len(_LARGE_HEADER)] + header + prefix
+            parts.append(host)
         if seen != len(self.large):
             raise RuntimeError("pickle: a stand-in was copied instead of passed through")
+        blob, into = hostmem.new_bytes(sum(len(p) if type(p) is bytes else p.numel() for p in parts))
+        raw, at = into.numpy(), 0
+        for p in parts:
+            if type(p) is bytes:
+                raw[at:at + len(p)] = np.frombuffer(p, dtype=np.uint8)
+                at += len(p)
+            else:
+                into[at:at + p.numel()].copy_(p)
+                at += p.numel()
         return blob
 
 
@@ -148,6 +158,7 @@ def pack_chunks(enc):
     rows, C = 2 * L, H * D
     blobs = []
     for part in wire.bring_to_host(enc, 0, enc.num_chunks):
+        part.arrive()
         w = _Writer(str(enc.payload.device))
         T = part.t1 - part.t0
         maxima = torch.from_numpy(np.ascontiguousarray(part.maxima).view(np.uint8).reshape(-1))
@@ -173,29 +184,40 @@ class _NotPlain(Exception):
     """The blob is not laid out the way this module reads: the plain unpickler takes it."""
 
 
-class _Source:
-    """File of an unpickler over a blob: large bytes objects are not filled but remembered by
-    their address, with their place in the blob."""
+_TOKEN = b"\xffstorage"
+# opcodes without an argument that may stand between frames (a frame of fewer than four bytes has no
+# header): memoize, tuple of one to three, reduce, append(s), build, setitem(s), stop
+_BARE = frozenset(b"\x94\x85\x86\x87Rabsuet.")
 
-    def __init__(self, blob):
-        self.mv, self.pos, self.skipped = memoryview(blob), 0, {}
 
-    def read(self, n=-1):
-        b = self.mv[self.pos:] if n < 0 else self.mv[self.pos:self.pos + n]
-        self.pos += len(b)
-        return bytes(b)
-
-    def readline(self):
-        raise _NotPlain("text opcodes")
-
-    def readinto(self, buf):
-        n = min(len(buf), len(self.mv) - self.pos)
-        if n >= _LARGE:
-            self.skipped[np.frombuffer(buf, dtype=np.uint8).ctypes.data] = (self.pos, n)
+def _condense(blob):
+    """(the pickle with every large bytes object replaced by a token, [(start, length) of these in
+    the blob])."""
+    mv = memoryview(blob)
+    if len(mv) < 4 or bytes(mv[:2]) != b"\x80\x04":
+        raise _NotPlain("protocol")
+    out, large, pos, end = [b"\x80\x04"], [], 2, len(mv)
+    while pos < end:
+        op = mv[pos]
+        if op == 0x95:                                   # frame
+            n = 9 + struct.unpack_from("<Q", mv, pos + 1)[0]
+            out.append(bytes(mv[pos:pos + n]))
+            pos += n
+        elif op == 0x42 or op == 0x8E:                   # bytes, 32- or 64-bit length
+            head = 5 if op == 0x42 else 9
+            n = struct.unpack_from("<I" if op == 0x42 else "<Q", mv, pos + 1)[0]
+            token = _TOKEN + struct.pack("<I", len(large))
+            out.append(b"C" + bytes([len(token)]) + token)
+            large.append((pos + head, n))
+            pos += head + n
+        elif op in _BARE:
+            out.append(bytes([op]))
+            pos += 1
         else:
-            buf[:n] = self.mv[self.pos:self.pos + n]
-        self.pos += n
-        return n
+            raise _NotPlain("opcode between frames")
+    if pos != end:
+        raise _NotPlain("truncated")
+    return b"".join(out), large
 
 
 class _Tensor:
@@ -208,17 +230,17 @@ class _Tensor:
 class _Reader(_ContainerUnpickler):
     """Admits what `_ContainerUnpickler` admits, with tensors left where their bytes are."""
 
-    def __init__(self, source, whole):
-        super().__init__(source)
-        self._source, self._whole = source, whole
+    def __init__(self, condensed, large, whole):
+        super().__init__(io.BytesIO(condensed))
+        self._large, self._whole = large, whole
 
     def _storage(self, b):
-        place = self._source.skipped.pop(_as_string(b), None) if type(b) is bytes else None
-        if place is None:
-            head, data = b[:4096], hostmem.view(b)
-        else:
-            data = self._whole[place[0]:place[0] + place[1]]
+        if type(b) is bytes and b.startswith(_TOKEN):
+            start, n = self._large[struct.unpack_from("<I", b, len(_TOKEN))[0]]
+            data = self._whole[start:start + n]
             head = data[:4096].numpy().tobytes()
+        else:
+            head, data = b[:4096], hostmem.view(b)
         m = _PREFIX.match(head)
         if not m or m.group(1) not in _DTYPES:
             raise _NotPlain("storage")
@@ -255,7 +277,7 @@ def container(blob):
         return None
     whole = hostmem.view(blob)
     try:
-        out = _Reader(_Source(blob), whole).load()
+        out = _Reader(*_condense(blob), whole).load()
         cdf, k, v = out.cdf, out.max_tensors_key, out.max_tensors_value
         rows, C, lp = cdf.shape
         L, T = k.shape[:2]
@@ -268,7 +290,7 @@ def container(blob):
             fine = (fine and c.bytestream.dtype is torch.uint8 and c.bytestream_lengths.dtype is torch.int32
                     and c.bytestream_lengths.shape == (rows, C)
                     and c.ntokens == min(wire.MAX_STREAM_BYTES, T - g * wire.MAX_STREAM_BYTES))
-    except (_NotPlain, AttributeError, TypeError, ValueError, KeyError):
+    except (_NotPlain, AttributeError, TypeError, ValueError, KeyError, IndexError, struct.error):
         return None
     if not fine:
         return None

@@ -335,20 +335,35 @@ def _device_tables(nsym_host, nsym_dev, data, C, lp, tokens):
 
 
 # Bytes of blobs that leave the GPU in one go: while the host copies one piece into its blobs, the
-# next is on the bus.  Blobs of one 256-token chunk (6 MB) are a piece each.
+# next is on the bus.  Blobs of one 256-token chunk (6 MB) are a piece each; where that is all
+# there is, the tables are cut in slices so that their copy overlaps with the rest's transfer (each
+# transfer costs about 10 us by itself).
 _PIECE_BYTES = 4 << 20
+_SLICE_BYTES = 2 << 20
 
 
 class HostPart:
-    """Chunks [first, last) of an encoded tensor in (pinned) host memory, one blob's worth: uint8
-    tensors `tables`, `lengths`, `payload` as they lie on the device, `maxima` (uint16 numpy view
-    [2L, tokens]), `sub_bytes` (payload bytes per sub-chunk), tokens [t0, t1).  `symbols`: stored
-    symbols per (chunk, row) where `tables` holds histogram counts, else None; `lengths_itemsize` 2
-    or 4."""
+    """Chunks [first, last) of an encoded tensor on their way to (pinned) host memory, one blob's
+    worth: uint8 tensors `tables`, `lengths`, `payload` as they lie on the device, `maxima` (uint16
+    numpy view [2L, tokens]), `sub_bytes` (payload bytes per sub-chunk), tokens [t0, t1).  `symbols`:
+    stored symbols per (chunk, row) where `tables` holds histogram counts, else None;
+    `lengths_itemsize` 2 or 4.  Sizes are known from the start; bytes are there after `arrive`."""
+
+    def table_slices(self):
+        """(start, end) slices of `tables`, each there when it is yielded."""
+        at = 0
+        for end, event in self.slices:
+            event.synchronize()
+            yield at, end
+            at = end
+
+    def arrive(self):
+        """Waits for everything."""
+        self.arrived.synchronize()
 
 
 def bring_to_host(enc, first_chunk, num_chunks, per_chunk=True, compact=False):
-    """Yields a HostPart per chunk (or one for all of them) once its bytes have arrived.
+    """Yields a HostPart per chunk (or one for all of them) once its sizes are known.
 
     The sections leave the encoder's own tensors for pinned memory as they are; blobs are put
     together on the host, where they have to be written anyway: no second copy of them on the
@@ -378,6 +393,21 @@ def bring_to_host(enc, first_chunk, num_chunks, per_chunk=True, compact=False):
         event = torch.cuda.Event()
         event.record()
         return event
+
+    def fetch_tables(src):
+        """(pinned tables, [(end, event)]): in slices where nothing else would overlap with them."""
+        flat = src.reshape(-1).view(torch.uint8)
+        n = flat.numel()
+        if len(pieces) > 1 or n < 2 * _SLICE_BYTES:
+            return fetch(src), [(n, mark())]
+        host = torch.empty(n, dtype=torch.uint8, pin_memory=True)
+        ends = [n * (i + 1) // (n // _SLICE_BYTES) for i in range(n // _SLICE_BYTES)]
+        slices = []
+        for i, end in enumerate(ends):
+            at = ends[i - 1] if i else 0
+            host[at:end].copy_(flat[at:end], non_blocking=True)
+            slices.append((end, mark()))
+        return host, slices
 
     def subs(c):
         return min(c * spc, g_last) - g_first
@@ -415,7 +445,7 @@ def bring_to_host(enc, first_chunk, num_chunks, per_chunk=True, compact=False):
                                           tables_src.data_ptr(), stream))
         elif not compact:
             a, b = groups[0][0], groups[pieces[0][1] - 1][1]
-            early = {"tables": fetch(cdf[a - c_first:b - c_first]), "lengths": fetch(lengths[subs(a):subs(b)])}
+            early = {"tables": fetch_tables(cdf[a - c_first:b - c_first]), "lengths": fetch(lengths[subs(a):subs(b)])}
         maxima = fetch(enc.maxima)
 
     sizes_known.synchronize()
@@ -444,15 +474,14 @@ def bring_to_host(enc, first_chunk, num_chunks, per_chunk=True, compact=False):
         with torch.cuda.device(dev):
             tables = early.pop("tables", None)
             lens = early.pop("lengths", None)
-            return (fetch(table_range(a, b)) if tables is None else tables,
+            return (fetch_tables(table_range(a, b)) if tables is None else tables,
                     fetch(lengths_src[subs(a):subs(b)]) if lens is None else lens,
                     fetch(enc.payload[p0:p1])), mark()
 
     itemsize = lengths_src.element_size()
     queued = queue(pieces[0])
     for k, piece in enumerate(pieces):
-        ((tables, lens, payload), arrived), queued = queued, queue(pieces[k + 1]) if k + 1 < len(pieces) else None
-        arrived.synchronize()
+        (((tables, slices), lens, payload), arrived), queued = queued, queue(pieces[k + 1]) if k + 1 < len(pieces) else None
         at = [0, 0, 0]
         for a, b in groups[piece[0]:piece[1]]:
             part = HostPart()
@@ -466,6 +495,9 @@ def bring_to_host(enc, first_chunk, num_chunks, per_chunk=True, compact=False):
             part.maxima = maxima.numpy().view(np.uint16).reshape(rows, T)[:, part.t0:part.t1]
             part.symbols = None if symbols is None else symbols[(a - c_first) * rows:(b - c_first) * rows]
             part.lengths_itemsize = itemsize
+            part.arrived = arrived
+            # several blobs in a piece: all of the piece's tables, there with its last slice
+            part.slices = slices if piece[1] - piece[0] == 1 else [(n[0], slices[-1][1])]
             yield part
 
 
@@ -508,7 +540,11 @@ def pack_chunks(enc, first_chunk: int = 0, num_chunks: Optional[int] = None, per
             start = max(off, end)                        # count tables: the symbol counts are there already
             raw[end:start] = 0                           # the gap before the section
             end = off + size
-            if section == "maxima":
+            if section == "cdf":
+                for a, b in part.table_slices():
+                    into[start + a:start + b].copy_(src[a:b])
+                part.arrive()
+            elif section == "maxima":
                 np.copyto(raw[start:end].view(np.uint16).reshape(2 * L, T), src)
             else:
                 into[start:end].copy_(src)
