@@ -19,8 +19,16 @@ MAX_TOKENS_PER_STREAM = 256
 _DT = {torch.float16: _lib.DT_F16, torch.bfloat16: _lib.DT_BF16}
 
 
-def _stream():
-    return torch.cuda.current_stream().cuda_stream
+def _stream(device):
+    """Handle of the current stream of `device`."""
+    return torch._C._cuda_getCurrentRawStream(device.index)
+
+
+def _largest(key_bins, value_bins):
+    """The larger of two bins vectors' largest values: one read of the device for both."""
+    if key_bins.device == value_bins.device:
+        return int(float(torch.maximum(key_bins, value_bins).max()))
+    return int(max(float(key_bins.max()), float(value_bins.max())))
 
 
 def _kv_strides(t, fmt):
@@ -129,7 +137,7 @@ def encode_kv(kv, key_bins, value_bins, chunk_tokens=None, fmt="vllm", max_bins=
     C = H * D
     S = int(chunk_tokens) if chunk_tokens else T
     if max_bins is None:
-        max_bins = int(max(float(key_bins.max()), float(value_bins.max())))
+        max_bins = _largest(key_bins, value_bins)
     dev = kv.device
     lib = _lib.lib()
     nchunks = int(lib.cg_num_chunks(T, S))
@@ -172,7 +180,7 @@ def encode_kv(kv, key_bins, value_bins, chunk_tokens=None, fmt="vllm", max_bins=
                 key_bins.data_ptr(), value_bins.data_ptr(), max_bins, S, int(delta_group),
                 out.cdf.data_ptr(), out.maxima.data_ptr(), out.lengths.data_ptr(), out.offsets.data_ptr(),
                 out.payload.data_ptr(), out.payload.numel(), out.status.data_ptr(),
-                workspace.data_ptr(), workspace.numel(), _stream())
+                workspace.data_ptr(), workspace.numel(), _stream(dev))
         if _test_flags is None:
             _lib.check(lib.cg_encode_kv(*args))
         else:
@@ -189,8 +197,23 @@ def scan_lengths(lengths):
     scratch = torch.empty(int(lib.cg_scan_workspace(n)), dtype=torch.uint8, device=flat.device)
     with torch.cuda.device(flat.device):
         _lib.check(lib.cg_scan_lengths(flat.data_ptr(), n, offsets.data_ptr(), scratch.data_ptr(),
-                                       scratch.numel(), _stream()))
+                                       scratch.numel(), _stream(flat.device)))
     return offsets
+
+
+def collect_streams(padded, offsets):
+    """uint8 streams of a padded buffer [nl, nc, cap], back to back; offsets: scan_lengths of their
+    lengths."""
+    nl, nc, cap = padded.shape
+    total = int(offsets[-1].item())
+    out = torch.empty(total, dtype=torch.uint8, device=padded.device)
+    if total:
+        if padded.stride(2) != 1:
+            padded = padded.contiguous()
+        with torch.cuda.device(padded.device):
+            _lib.check(_lib.lib().cg_collect_bytes(padded.data_ptr(), cap, padded.stride(0), padded.stride(1), offsets.data_ptr(),
+                                                   nl, nc, out.data_ptr(), total, _stream(padded.device)))
+    return out
 
 
 def decode_kv(cdf, maxima, offsets, payload, key_bins, value_bins, num_layers, num_tokens,
@@ -241,7 +264,7 @@ def decode_kv(cdf, maxima, offsets, payload, key_bins, value_bins, num_layers, n
             cdf.data_ptr(), cdf.shape[-1] - 1, maxima.data_ptr(), _DT[maxima.dtype],
             offsets.data_ptr(), payload.data_ptr(), payload.numel(),
             key_bins.data_ptr(), value_bins.data_ptr(), L, T, H, D, int(chunk_tokens), int(delta_group),
-            out.data_ptr(), _DT[out.dtype], ol, okv, ot, oh, _stream()))
+            out.data_ptr(), _DT[out.dtype], ol, okv, ot, oh, _stream(dev)))
     return out
 
 
@@ -253,7 +276,7 @@ def decode_listed(subs_ptr, nsub, max_bins, num_layers, num_heads, head_size, de
         raise RuntimeError("output tensor does not match the encoded geometry")
     with torch.cuda.device(out.device):
         _lib.check(_lib.lib().cg_decode_listed(subs_ptr, nsub, max_bins, L, H, D, int(delta_group), out.data_ptr(),
-                                               _DT[out.dtype], ol, okv, ot, oh, _stream()))
+                                               _DT[out.dtype], ol, okv, ot, oh, _stream(out.device)))
 
 
 def decode_encoded(enc: EncodedKV, key_bins, value_bins, fmt="vllm", out_dtype=None, out=None):
@@ -274,7 +297,7 @@ def quantize_kv(kv, key_bins, value_bins, fmt="vllm"):
     with torch.cuda.device(dev):
         _lib.check(_lib.lib().cg_quantize_kv(
             kv.data_ptr(), _DT[kv.dtype], L, T, H, D, sl, skv, st, sh,
-            key_bins.data_ptr(), value_bins.data_ptr(), sym.data_ptr(), maxima.data_ptr(), _stream()))
+            key_bins.data_ptr(), value_bins.data_ptr(), sym.data_ptr(), maxima.data_ptr(), _stream(dev)))
     return sym, maxima
 
 
@@ -309,7 +332,7 @@ def encode_kv_levels(kv, levels, chunk_tokens=None, fmt="vllm", workspace=None, 
             raise RuntimeError("bins vectors must have one entry per layer (%d)" % L)
         bins.append((kb.to(device=dev, dtype=torch.float32).contiguous(), vb.to(device=dev, dtype=torch.float32).contiguous()))
     if max_bins is None:
-        max_bins = [int(max(float(kb.max()), float(vb.max()))) for kb, vb in levels]
+        max_bins = [_largest(kb, vb) for kb, vb in levels]
     if len(max_bins) != n:
         raise RuntimeError("max_bins must have one entry per level")
     nchunks = int(lib.cg_num_chunks(T, S))
@@ -354,5 +377,5 @@ def encode_kv_levels(kv, levels, chunk_tokens=None, fmt="vllm", workspace=None, 
             ptrs(ctypes.c_void_p, [e.offsets.data_ptr() for e in out]),
             ptrs(ctypes.c_void_p, [e.payload.data_ptr() for e in out]),
             ptrs(ctypes.c_int64, [e.payload.numel() for e in out]),
-            out[0].status.data_ptr(), workspace.data_ptr(), workspace.numel(), _stream()))
+            out[0].status.data_ptr(), workspace.data_ptr(), workspace.numel(), _stream(dev)))
     return out

@@ -213,6 +213,18 @@ int cg_quantize_kv(const void *kv, int kv_dt, int64_t L, int64_t T, int64_t H, i
                            static_cast<hipStream_t>(stream));
 }
 
+int cg_collect_bytes(const uint8_t *padded, int64_t cap, int64_t p0, int64_t p1, const int64_t *offsets, int64_t nl, int64_t nc,
+                     uint8_t *out, int64_t out_bytes, void *stream)
+{
+    if (!padded || !offsets || !out) return fail(CG_ERR_ARG, "collect_bytes: null pointer");
+    if (nl <= 0 || nc <= 0 || cap <= 0 || out_bytes <= 0) return fail(CG_ERR_ARG, "collect_bytes: empty input");
+    const int64_t nblocks = ceil_div(nl * nc, 4 * kCollectPerWave);
+    if (nblocks > INT_MAX) return fail(CG_ERR_ARG, "collect_bytes: too many streams");
+    collect_bytes_kernel<<<dim3((unsigned)nblocks), dim3(256), 0, static_cast<hipStream_t>(stream)>>>(padded, cap, p0, p1, offsets, nc,
+                                                                                                     nl * nc, out, out_bytes);
+    return check_launch("collect_bytes");
+}
+
 size_t cg_scan_workspace(int64_t n) { return align_up((size_t)(ceil_div(n > 0 ? n : 1, kScanTile) + 1) * sizeof(int64_t), 256); }
 
 int cg_scan_lengths(const int32_t *lengths, int64_t n, int64_t *offsets, void *scratch,
@@ -389,6 +401,10 @@ int code_and_compact(const LevelOut &o, const uint32_t *sym4, const uint8_t *sym
         compact_streams_kernel<true><<<dim3((unsigned)cblocks), dim3(256), 0, s>>>(
             w.scratch, kStreamCap, o.offsets, o.lengths, nullptr, w.nstreams, o.payload, o.payload_cap, skew, o.status,
             w.group_sums, w.tile_sums);
+    } else if (fused_scan && w.ntiles <= kDirectTiles) {
+        compact_streams_kernel<true><<<dim3((unsigned)cblocks), dim3(256), 0, s>>>(
+            w.scratch, kStreamCap, o.offsets, o.lengths, nullptr, w.nstreams, o.payload, o.payload_cap, skew, o.status,
+            nullptr, w.tile_sums);
     } else if (fused_scan) {
         if (int rc = launch_scan(w.tile_sums, cblocks, INT_MAX, w.tile_base, w.tile_scan_scratch, s)) return rc;
         compact_streams_kernel<true><<<dim3((unsigned)cblocks), dim3(256), 0, s>>>(

@@ -528,11 +528,11 @@ __global__ __launch_bounds__(BS) void encode_streams_kernel(EncodeArgs a)
 #pragma unroll
                 for (int j = 0; j < 8; ++j) nxt[j] = (i0 + 8 + j < id.n) ? sp[(int64_t)(i0 + 8 + j) * a.s1] : 0u;
 #pragma unroll
-                for (int j = 0; j < 8; j += 2) {
-                    if (i0 + j < id.n) enc.template put_symbol<SENTINEL, true>(cur[j]);
-                    if (i0 + j + 1 < id.n) enc.template put_symbol<SENTINEL, false>(cur[j + 1]);
-                    enc.end_group();
+                for (int j = 0; j < 8; ++j) {
+                    if (j == 0) enc.template put_symbol<SENTINEL, true>(cur[j]);
+                    else if (i0 + j < id.n) enc.template put_symbol<SENTINEL, false>(cur[j]);
                 }
+                enc.end_group();
             }
         }
     };

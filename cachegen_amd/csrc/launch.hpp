@@ -92,9 +92,17 @@ int launch_cdf(const uint8_t *sym, const uint32_t *sym4, int64_t nsub, int64_t r
     if (nblocks <= 0 || nblocks > INT_MAX) return fail(CG_ERR_ARG, "calculate_cdf: grid out of range");
     const size_t shmem = sym4 ? (size_t)(max_bins + 1) * (block + 2) * sizeof(uint16_t)
                               : (size_t)(max_bins + 1) * (block + 1) * sizeof(uint32_t);     // TableStride
-    const dim3 grid((unsigned)nblocks), blk(block);
-    if (sym4) CG_DISPATCH_BS(block, (calculate_cdf_kernel<BS, true><<<grid, blk, shmem, stream>>>(a)));
-    else CG_DISPATCH_BS(block, (calculate_cdf_kernel<BS, false><<<grid, blk, shmem, stream>>>(a)));
+    // four blocks of 256 lanes per compute unit hide the loads of one another; below that the
+    // block's own slices do (see the kernel)
+    const bool sliced = nblocks * block < 1024 * 256;
+    const dim3 grid((unsigned)nblocks), blk(sliced ? block * 4 : block);
+    if (sliced) {
+        if (sym4) CG_DISPATCH_BS(block, (calculate_cdf_kernel<BS, true, 4><<<grid, blk, shmem, stream>>>(a)));
+        else CG_DISPATCH_BS(block, (calculate_cdf_kernel<BS, false, 4><<<grid, blk, shmem, stream>>>(a)));
+    } else {
+        if (sym4) CG_DISPATCH_BS(block, (calculate_cdf_kernel<BS, true, 1><<<grid, blk, shmem, stream>>>(a)));
+        else CG_DISPATCH_BS(block, (calculate_cdf_kernel<BS, false, 1><<<grid, blk, shmem, stream>>>(a)));
+    }
     return check_launch("calculate_cdf");
 }
 

@@ -194,9 +194,12 @@ constexpr int kCompactTile = 16384;
 
 // SCAN: the offsets are not known yet; `offsets` is written here from the streams' lengths and
 // the exclusive running sum of the tiles' byte counts, instead of being read.  That sum comes
-// from tile_base (a scan launch made it), or, group_sums != null, is added up here: the sums of
-// the groups of kTileGroup tiles before this block's group (at most kMaxTileGroups, left by the
-// coder) and the counts of the tiles before this one in its group.
+// from tile_base (a scan launch made it), or is added up here: from the sums of the groups of
+// kTileGroup tiles before this block's group (at most kMaxTileGroups, left by the coder) and the
+// counts of the tiles before this one in its group (group_sums != null), or from the counts of all
+// tiles before this one (neither: calls of at most kDirectTiles tiles, where that is a few loads per
+// thread and saves the scan launch, 5 us and its gap).
+constexpr int kDirectTiles = 1024;
 template <bool SCAN>
 __global__ __launch_bounds__(256) void compact_streams_kernel(
     const uint8_t *__restrict__ slots, int32_t cap, int64_t *__restrict__ offsets,
@@ -217,7 +220,17 @@ __global__ __launch_bounds__(256) void compact_streams_kernel(
             mine = mine < 0 ? 0 : (mine > cap ? cap : mine);
         }
         int32_t total32;
-        if (group_sums) {
+        if (!group_sums && !tile_base) {
+            int32_t part = 0;
+#pragma unroll
+            for (int i = 0; i < kDirectTiles / 256; ++i) {
+                const int t = tid + i * 256;
+                if (t < (int)blockIdx.x) part += tile_sums[t];
+            }
+            int32_t sum;
+            block_exclusive_scan_256(part, reinterpret_cast<int32_t *>(buf), sum);
+            o0 = sum;
+        } else if (group_sums) {
             const int g = (int)(blockIdx.x / kTileGroup), r = (int)(blockIdx.x % kTileGroup);
             int32_t part = tid < g ? group_sums[tid] : 0;
             if (tid < r) part += tile_sums[(int64_t)g * kTileGroup + tid];
@@ -296,6 +309,30 @@ __global__ __launch_bounds__(256) void compact_streams_kernel(
             }
         }
         __syncthreads();
+    }
+}
+
+// collect_bytes for streams in a padded buffer (encoder.py:209-222): stream g = row * nc + channel
+// goes to out[offsets[g] ...].  A wavefront copies four streams, a byte per lane: the streams are
+// some tens of bytes long and begin anywhere.
+constexpr int kCollectPerWave = 4;
+
+__global__ __launch_bounds__(256) void collect_bytes_kernel(
+    const uint8_t *__restrict__ padded, int64_t cap, int64_t p0, int64_t p1, const int64_t *__restrict__ offsets,
+    int64_t nc, int64_t nstreams, uint8_t *__restrict__ out, int64_t out_bytes)
+{
+    const int lane = threadIdx.x & 63;
+    const int64_t first = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * kCollectPerWave;
+#pragma unroll
+    for (int i = 0; i < kCollectPerWave; ++i) {
+        const int64_t g = first + i;
+        if (g >= nstreams) return;
+        const int64_t at = offsets[g];
+        int64_t n = offsets[g + 1] - at;
+        n = n < cap ? n : cap;
+        if (at < 0 || at + n > out_bytes) continue;          // never write past the caller's buffer
+        const uint8_t *src = padded + g / nc * p0 + g % nc * p1;
+        for (int64_t j = lane; j < n; j += 64) out[at + j] = src[j];
     }
 }
 

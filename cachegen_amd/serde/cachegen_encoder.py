@@ -21,11 +21,8 @@ def torch_quant_vectorized(bins: torch.Tensor, input_groups: torch.Tensor):
 
 def collect_bytes(output_buffer: torch.Tensor, output_lengths: torch.Tensor) -> torch.Tensor:
     """cachegen_encoder.py:209-222: the streams of a padded buffer, back to back."""
-    cap = output_buffer.shape[-1]
     offsets = codec.scan_lengths(output_lengths)
-    idx = torch.arange(int(offsets[-1].item()), device=output_buffer.device)
-    stream = torch.searchsorted(offsets[1:], idx, right=True)
-    return output_buffer.reshape(-1, cap)[stream, idx - offsets[stream]]
+    return codec.collect_streams(output_buffer, offsets)
 
 
 def encode_ntokens(cdf_int, encode_input, output_buffer, output_lengths) -> torch.Tensor:

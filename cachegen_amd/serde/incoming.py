@@ -227,7 +227,7 @@ def decode(items, out, fmt):
             invalid = torch.empty(1, dtype=torch.int32, device=device)
             _lib.check(_lib.lib().cg_counts_to_tables(
                 buf.data_ptr(), index_at, key[0], G, C, base + at + _up(8 * G), base + at + _up(8 * G) + _up(4 * G), base + at,
-                tables.data_ptr(), invalid.data_ptr(), codec._stream()))
+                tables.data_ptr(), invalid.data_ptr(), codec._stream(buf.device)))
             verdict = torch.empty(1, dtype=torch.int32, pin_memory=True)
             verdict.copy_(invalid, non_blocking=True)
             verdicts.append(verdict)

@@ -281,17 +281,12 @@ def unpack_host(blob):
 # --------------------------------------------------------------------------- #
 # device form: one staging buffer, one copy over PCIe per direction
 # --------------------------------------------------------------------------- #
-def _stream():
-    import torch
-    return torch.cuda.current_stream().cuda_stream
-
-
 def _device_counts_launch(cdf, tokens):
     """Device form of tables_to_counts for cdf int16 [nchunks, 2L, C, Lp]: launches the conversion
     and returns (dense counts uint8 [G, C, Lp-1], nsym int32 [G], inexact int32 [1]), all still on
     the device and not waited for.  tokens: per chunk; all but the last are the same."""
     import torch
-    from .. import _lib
+    from .. import _lib, codec
     nchunks, rows, C, lp = cdf.shape
     G = nchunks * rows
     dev = cdf.device
@@ -304,7 +299,7 @@ def _device_counts_launch(cdf, tokens):
     inexact = torch.empty(1, dtype=torch.int32, device=dev)
     with torch.cuda.device(dev):
         _lib.check(_lib.lib().cg_tables_to_counts(cdf.data_ptr(), lp - 1, G, C, tok.data_ptr(), dense.data_ptr(),
-                                                  nsym.data_ptr(), inexact.data_ptr(), _stream()))
+                                                  nsym.data_ptr(), inexact.data_ptr(), codec._stream(dev)))
     return dense, nsym, inexact
 
 
@@ -313,7 +308,7 @@ def _device_tables(nsym_host, nsym_dev, data, C, lp, tokens):
     nsym_host: numpy uint8 [nchunks, 2L] (read from the blob on the host), nsym_dev the same bytes
     on the device."""
     import torch
-    from .. import _lib
+    from .. import _lib, codec
     nchunks, rows = nsym_host.shape
     G = nchunks * rows
     dev = data.device
@@ -328,7 +323,7 @@ def _device_tables(nsym_host, nsym_dev, data, C, lp, tokens):
     with torch.cuda.device(dev):
         _lib.check(_lib.lib().cg_counts_to_tables(data.data_ptr(), data.numel(), lp - 1, G, C, tok.data_ptr(),
                                                   nsym_dev.data_ptr(), small.data_ptr(), cdf.data_ptr(),
-                                                  invalid.data_ptr(), _stream()))
+                                                  invalid.data_ptr(), codec._stream(dev)))
     if int(invalid.item()):
         raise ValueError("wire container: histogram counts do not add up to the chunk's tokens")
     return cdf
@@ -371,7 +366,7 @@ def bring_to_host(enc, first_chunk, num_chunks, per_chunk=True, compact=False):
     counts, stored into pinned memory by one kernel) while the tables, whose size it knows, are
     already on the bus, and then for each piece of about _PIECE_BYTES."""
     import torch
-    from .. import _lib
+    from .. import _lib, codec
     L, H, D, S, T = enc.num_layers, enc.num_heads, enc.head_size, enc.chunk_tokens, enc.num_tokens
     C = H * D
     rows = 2 * L
@@ -416,7 +411,7 @@ def bring_to_host(enc, first_chunk, num_chunks, per_chunk=True, compact=False):
     groups = [(c, c + 1) for c in range(c_first, c_last)] if per_chunk else [(c_first, c_last)]
     early = {}                                           # the first piece's tables and lengths: sizes not needed
     with torch.cuda.device(dev):
-        stream = _stream()
+        stream = codec._stream(dev)
         cdf = enc.cdf[c_first:c_last]
         lengths = enc.lengths[g_first:g_last]
         wide = inexact = nsym = dense = None

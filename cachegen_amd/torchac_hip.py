@@ -14,8 +14,8 @@ MAX_TOKENS_PER_STREAM = 256
 MAX_BINS_SUPPORTED = 128
 
 
-def _stream():
-    return torch.cuda.current_stream().cuda_stream
+def _stream(device):
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
 def _require(cond, msg):
@@ -31,13 +31,14 @@ def calculate_cdf(input, max_bins):
     _require(input.dim() == 3 and input.dtype in (torch.int8, torch.uint8),
              "Input must be an int8 tensor of shape [nlayers, ntokens, nchannels]")
     nl, nt, nc = input.shape
-    out = torch.zeros((nl, nc, max_bins + 1), dtype=torch.int16, device=input.device)
+    shape = (nl, nc, max_bins + 1)
     if nl == 0 or nt == 0 or nc == 0:
-        return out
+        return torch.zeros(shape, dtype=torch.int16, device=input.device)
+    out = torch.empty(shape, dtype=torch.int16, device=input.device)          # the kernel writes every entry
     s = input.stride()
     with torch.cuda.device(input.device):
         _lib.check(_lib.lib().cg_calculate_cdf(input.data_ptr(), nl, nt, nc, s[0], s[1], s[2],
-                                               int(max_bins), out.data_ptr(), _stream()))
+                                               int(max_bins), out.data_ptr(), _stream(input.device)))
     return out
 
 
@@ -69,7 +70,7 @@ def encode_fast_new(cdf, input_sym, output_buffer, output_lengths):
         _lib.check(_lib.lib().cg_encode_fast_new(
             cdf.data_ptr(), cdf.shape[2], input_sym.data_ptr(), nl, nt, nc, s[0], s[1], s[2],
             output_buffer.data_ptr(), output_buffer.shape[2], o[0], o[1],
-            output_lengths.data_ptr(), _stream()))
+            output_lengths.data_ptr(), _stream(cdf.device)))
 
 
 def _check_decode(cdf, lengths, output):
@@ -105,7 +106,7 @@ def decode_fast_new(cdf, bytestreams, lengths, output):
     with torch.cuda.device(cdf.device):
         _lib.check(_lib.lib().cg_decode_fast_new(
             cdf.data_ptr(), cdf.shape[2], bytestreams.data_ptr(), bytestreams.shape[2], p[0], p[1],
-            lengths.data_ptr(), nl, nt, nc, output.data_ptr(), o[0], o[1], o[2], _stream()))
+            lengths.data_ptr(), nl, nt, nc, output.data_ptr(), o[0], o[1], o[2], _stream(cdf.device)))
 
 
 def decode_fast_prefsum(cdf, bytestreams, lengths_prefsum, output):
@@ -126,4 +127,4 @@ def decode_fast_prefsum(cdf, bytestreams, lengths_prefsum, output):
     with torch.cuda.device(cdf.device):
         _lib.check(_lib.lib().cg_decode_fast_prefsum(
             cdf.data_ptr(), cdf.shape[2], bytestreams.data_ptr(), bytestreams.numel(),
-            lengths_prefsum.data_ptr(), nl, nt, nc, output.data_ptr(), o[0], o[1], o[2], _stream()))
+            lengths_prefsum.data_ptr(), nl, nt, nc, output.data_ptr(), o[0], o[1], o[2], _stream(cdf.device)))

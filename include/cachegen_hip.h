@@ -206,6 +206,13 @@ int cg_encode_kv_levels(const void *kv, int kv_dt, int64_t L, int64_t T, int64_t
                         int64_t *const *offsets, uint8_t *const *payload, const int64_t *payload_cap,
                         int32_t *status, void *workspace, size_t workspace_bytes, void *stream);
 
+/* collect_bytes (encoder.py:209-222): the streams of a padded buffer, back to back.
+ * padded   device uint8 [nl, nc, cap], strides (p0, p1, 1)
+ * offsets  device int64 [nl*nc + 1]: exclusive running sum of the lengths (cg_scan_lengths)
+ * out      device uint8 [out_bytes], written; nothing is written past it */
+int cg_collect_bytes(const uint8_t *padded, int64_t cap, int64_t p0, int64_t p1, const int64_t *offsets,
+                     int64_t nl, int64_t nc, uint8_t *out, int64_t out_bytes, void *stream);
+
 /* Exclusive running sum of stream lengths: offsets[0] = 0, offsets[i+1] =
  * offsets[i] + lengths[i] (the inclusive sums of decoder.py:70 are offsets[1:]).
  * scratch: device, cg_scan_workspace(n) bytes. */
