@@ -641,8 +641,8 @@ int cg_tables_to_counts(const int16_t *cdf, int max_bins, int64_t ngroups, int64
     if (ngroups <= 0 || C <= 0 || ngroups > 65535) return fail(CG_ERR_ARG, "tables_to_counts: bad group or channel count");
     hipStream_t s = static_cast<hipStream_t>(stream);
     clear_ints_kernel<<<dim3((unsigned)ceil_div(ngroups, kWireThreads)), dim3(kWireThreads), 0, s>>>(nsym, ngroups, inexact);
-    const dim3 grid((unsigned)ceil_div(C, kWireThreads), (unsigned)ngroups);
-    tables_to_counts_kernel<<<grid, dim3(kWireThreads), 0, s>>>(reinterpret_cast<const uint16_t *>(cdf), max_bins + 1, C,
+    const dim3 grid((unsigned)ceil_div(C, kTableChannels), (unsigned)ngroups);
+    tables_to_counts_kernel<<<grid, dim3(kTableChannels), 0, s>>>(reinterpret_cast<const uint16_t *>(cdf), max_bins + 1, C,
                                                                tokens, counts, nsym, inexact);
     return check_launch("tables_to_counts");
 }
@@ -653,8 +653,8 @@ int cg_pack_counts(const uint8_t *counts, int max_bins, int64_t ngroups, int64_t
     if (!counts || !nsym || !out) return fail(CG_ERR_ARG, "pack_counts: null pointer");
     if (int rc = check_lp(max_bins + 1, "pack_counts")) return rc;
     if (ngroups <= 0 || C <= 0 || ngroups > 65535) return fail(CG_ERR_ARG, "pack_counts: bad group or channel count");
-    const dim3 grid((unsigned)ceil_div(C, kWireThreads), (unsigned)ngroups);
-    pack_counts_kernel<<<grid, dim3(kWireThreads), 0, static_cast<hipStream_t>(stream)>>>(counts, max_bins + 1, C, nsym,
+    const dim3 grid((unsigned)ceil_div(C, kTableChannels), (unsigned)ngroups);
+    pack_counts_kernel<<<grid, dim3(kTableChannels), 0, static_cast<hipStream_t>(stream)>>>(counts, max_bins + 1, C, nsym,
                                                                                          starts, out);
     return check_launch("pack_counts");
 }
@@ -686,14 +686,17 @@ int cg_counts_to_tables(const uint8_t *data, int64_t data_bytes, int max_bins, i
 {
     if (!data || !tokens || !nsym || !starts || !cdf || !invalid) return fail(CG_ERR_ARG, "counts_to_tables: null pointer");
     if (int rc = check_lp(max_bins + 1, "counts_to_tables")) return rc;
-    if (ngroups <= 0 || C <= 0 || ngroups > 65535 || data_bytes < 0)
+    if (ngroups <= 0 || C <= 0 || data_bytes < 0)
         return fail(CG_ERR_ARG, "counts_to_tables: bad group or channel count");
     hipStream_t s = static_cast<hipStream_t>(stream);
     clear_ints_kernel<<<dim3(1), dim3(kWireThreads), 0, s>>>(invalid, 1, nullptr);
-    const dim3 grid((unsigned)ceil_div(C, kWireThreads), (unsigned)ngroups);
-    counts_to_tables_kernel<<<grid, dim3(kWireThreads), 0, s>>>(data, data_bytes, max_bins + 1, C, tokens, nsym, starts,
-                                                               reinterpret_cast<uint16_t *>(cdf), invalid);
-    return check_launch("counts_to_tables");
+    for (int64_t g = 0; g < ngroups; g += 65535) {                   // a grid's limit in y
+        const dim3 grid((unsigned)ceil_div(C, kTableChannels), (unsigned)(ngroups - g < 65535 ? ngroups - g : 65535));
+        counts_to_tables_kernel<<<grid, dim3(kTableChannels), 0, s>>>(data, data_bytes, max_bins + 1, C, tokens + g, nsym + g, starts + g,
+                                                                     reinterpret_cast<uint16_t *>(cdf) + g * C * (max_bins + 1), invalid);
+        if (int rc = check_launch("counts_to_tables")) return rc;
+    }
+    return CG_OK;
 }
 
 }  // extern "C"
