@@ -42,6 +42,8 @@ SIGNATURES = {
     "cg_scan_lengths": (_INT, [_P, _I64, _P, _P, _SZ, _P]),
     "cg_scan_lengths_static": (_INT, [_P, _I64, _P, _P]),
     "cg_decode_listed": (_INT, [_P, _I64, _INT, _I64, _I64, _I64, _INT, _P, _INT, _I64, _I64, _I64, _I64, _P]),
+    "cg_host_list": (_INT, [_P, _INT, _P, _P, _I64, _I64, _P, _I64, _P, _P]),
+    "cg_rebuild_tables": (_INT, [_P, _I64, _INT, _I64, _I64, _P, _P, _P, _P, _P, _P]),
     "cg_host_tile_starts": (_INT, [_P, _INT, _I64, _I64, _I64, _P, _P]),
     "cg_tables_to_counts": (_INT, [_P, _INT, _I64, _I64, _P, _P, _P, _P, _P]),
     "cg_pack_counts": (_INT, [_P, _INT, _I64, _I64, _P, _P, _P, _P]),

@@ -633,6 +633,52 @@ int cg_host_tile_starts(const void *lengths, int itemsize, int64_t nsub, int64_t
     return fine ? CG_OK : fail(CG_ERR_ARG, "host_tile_starts: negative length");
 }
 
+int cg_host_list(const CgHostContainer *items, int n, const void *const *lengths, const int64_t *array_subs,
+                 int64_t L, int64_t C, uint32_t *tile_starts, int64_t starts_at, CgListedSub *subs, int *bad)
+{
+    if (!items || !lengths || !array_subs || !tile_starts || !subs || !bad) return fail(CG_ERR_ARG, "host_list: null pointer");
+    if (n <= 0 || L <= 0 || C <= 0 || 2 * L > (1 << 24) / C) return fail(CG_ERR_ARG, "host_list: bad shape");
+    const int64_t rows = 2 * L, tiles = ceil_div(C, 64);
+    int64_t sum;
+    for (int i = 0; i < n; ++i) {
+        const CgHostContainer &c = items[i];
+        *bad = i;
+        if (c.tokens <= 0 || c.chunk_tokens <= 0 || c.payload_bytes <= 0) return fail(CG_ERR_ARG, "host_list: empty container");
+        const int64_t nsub = cg_num_subchunks(c.tokens, c.chunk_tokens), nsc = ceil_div(c.chunk_tokens, kSub);
+        const int64_t skew = c.payload & 3;
+        int64_t first = skew, g = 0;
+        for (int k = 0; k < c.narrays; ++k, ++lengths, ++array_subs) {
+            const int size = c.lengths_u16 ? 2 : 4;
+            const char *p = static_cast<const char *>(*lengths);
+            for (int64_t j = 0; j < *array_subs; ++j, ++g, ++subs, p += rows * C * size, tile_starts += rows * tiles, starts_at += rows * tiles * 4) {
+                if (g >= nsub) return fail(CG_ERR_ARG, "host_list: more lengths than sub-chunks");
+                if (int rc = cg_host_tile_starts(p, size, 1, rows, C, tile_starts, &sum)) return rc;
+                const int64_t chunk = g / nsc, t0 = chunk * c.chunk_tokens + (g - chunk * nsc) * kSub;
+                int64_t end = (chunk + 1) * c.chunk_tokens;
+                if (end > c.tokens) end = c.tokens;
+                subs->cdf = reinterpret_cast<const int16_t *>(c.tables + chunk * rows * C * (c.max_bins + 1) * 2);
+                subs->maxima = reinterpret_cast<const void *>(c.maxima + t0 * 2);
+                subs->lengths = reinterpret_cast<const void *>(c.lengths + g * rows * C * size);
+                subs->bytes = reinterpret_cast<const uint8_t *>(c.payload - skew);
+                subs->last_word = (skew + c.payload_bytes - 1) & ~3ll;
+                subs->first = first;
+                subs->tile_starts = reinterpret_cast<const uint32_t *>(starts_at);
+                subs->key_bins = reinterpret_cast<const float *>(c.key_bins);
+                subs->value_bins = reinterpret_cast<const float *>(c.value_bins);
+                subs->t_out = c.t_out + t0;
+                subs->n = (int32_t)(end - t0 < kSub ? end - t0 : kSub);
+                subs->maxima_pitch = (int32_t)c.tokens;
+                subs->max_dt = c.max_dt;
+                subs->lengths_u16 = c.lengths_u16;
+                first += sum;
+            }
+        }
+        if (g != nsub || first - skew != c.payload_bytes)
+            return fail(CG_ERR_ARG, "host_list: lengths do not add up to the payload");
+    }
+    return CG_OK;
+}
+
 int cg_tables_to_counts(const int16_t *cdf, int max_bins, int64_t ngroups, int64_t C, const int32_t *tokens,
                         uint8_t *counts, int32_t *nsym, int32_t *inexact, void *stream)
 {
@@ -684,12 +730,20 @@ int cg_counts_to_tables(const uint8_t *data, int64_t data_bytes, int max_bins, i
                         const int32_t *tokens, const uint8_t *nsym, const int64_t *starts, int16_t *cdf,
                         int32_t *invalid, void *stream)
 {
+    if (!invalid) return fail(CG_ERR_ARG, "counts_to_tables: null pointer");
+    clear_ints_kernel<<<dim3(1), dim3(kWireThreads), 0, static_cast<hipStream_t>(stream)>>>(invalid, 1, nullptr);
+    return cg_rebuild_tables(data, data_bytes, max_bins, ngroups, C, tokens, nsym, starts, cdf, invalid, stream);
+}
+
+int cg_rebuild_tables(const uint8_t *data, int64_t data_bytes, int max_bins, int64_t ngroups, int64_t C,
+                      const int32_t *tokens, const uint8_t *nsym, const int64_t *starts, int16_t *cdf,
+                      int32_t *invalid, void *stream)
+{
     if (!data || !tokens || !nsym || !starts || !cdf || !invalid) return fail(CG_ERR_ARG, "counts_to_tables: null pointer");
     if (int rc = check_lp(max_bins + 1, "counts_to_tables")) return rc;
     if (ngroups <= 0 || C <= 0 || data_bytes < 0)
         return fail(CG_ERR_ARG, "counts_to_tables: bad group or channel count");
     hipStream_t s = static_cast<hipStream_t>(stream);
-    clear_ints_kernel<<<dim3(1), dim3(kWireThreads), 0, s>>>(invalid, 1, nullptr);
     for (int64_t g = 0; g < ngroups; g += 65535) {                   // a grid's limit in y
         const dim3 grid((unsigned)ceil_div(C, kTableChannels), (unsigned)(ngroups - g < 65535 ? ngroups - g : 65535));
         counts_to_tables_kernel<<<grid, dim3(kTableChannels), 0, s>>>(data, data_bytes, max_bins + 1, C, tokens + g, nsym + g, starts + g,

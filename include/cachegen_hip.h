@@ -277,6 +277,28 @@ int cg_decode_listed(const CgListedSub *subs, int64_t nsub, int max_bins, int64_
                      int delta_group, void *out, int out_dt, int64_t ol, int64_t okv, int64_t ot, int64_t oh,
                      void *stream);
 
+/* HOST memory, no GPU work: the entries of cg_decode_listed and the running sums they point to, for
+ * containers whose sections are (or will be) in device memory. */
+typedef struct CgHostContainer {
+    int64_t tables, maxima, lengths, payload;       /* device addresses of the sections: [nchunks, 2L, C, max_bins+1],
+                                                       [2, L, T], [nsub, 2L, C], bytes back to back */
+    int64_t payload_bytes;
+    int64_t key_bins, value_bins;                   /* device addresses, float32 [L] each */
+    int64_t t_out;                                  /* first token in the output tensor */
+    int64_t tokens, chunk_tokens;
+    int32_t max_bins, max_dt, lengths_u16;
+    int32_t narrays;                                /* host arrays that hold the lengths, consecutive sub-chunks each */
+} CgHostContainer;
+
+/* lengths      HOST array of the containers' length arrays (narrays each, one after the other), array_subs
+ *              the sub-chunks of each
+ * tile_starts  HOST uint32, written; starts_at: its device address (see CgListedSub)
+ * subs         HOST, written: one entry per sub-chunk, containers in order
+ * bad          written: the number of the first container whose lengths are negative or do not add
+ *              up to its payload (CG_ERR_ARG then) */
+int cg_host_list(const CgHostContainer *items, int n, const void *const *lengths, const int64_t *array_subs,
+                 int64_t L, int64_t C, uint32_t *tile_starts, int64_t starts_at, CgListedSub *subs, int *bad);
+
 /* HOST memory, no GPU work: the running sums of stream lengths that cg_decode_listed starts from.
  * lengths      [nsub, rows, C] int32, or uint16 (itemsize 2)
  * tile_starts  uint32 [nsub, rows, ceil(C/64)], written: bytes of the sub-chunk's streams before
@@ -315,6 +337,12 @@ int cg_pack_counts(const uint8_t *counts, int max_bins, int64_t ngroups, int64_t
 int cg_counts_to_tables(const uint8_t *data, int64_t data_bytes, int max_bins, int64_t ngroups, int64_t C,
                         const int32_t *tokens, const uint8_t *nsym, const int64_t *starts, int16_t *cdf,
                         int32_t *invalid, void *stream);
+
+/* The same for groups that lie in several containers (starts: byte offsets from `data`), with the verdict
+ * stored to *invalid (device or pinned host memory, zero before the call) only where it is bad. */
+int cg_rebuild_tables(const uint8_t *data, int64_t data_bytes, int max_bins, int64_t ngroups, int64_t C,
+                      const int32_t *tokens, const uint8_t *nsym, const int64_t *starts, int16_t *cdf,
+                      int32_t *invalid, void *stream);
 
 /* What a host that lays out containers has to read back of an encoded tensor, in one piece:
  * out[0] = *status, out[1] = *wide (0 if null), out[2] = *inexact (0 if null), out[3 + i] =
