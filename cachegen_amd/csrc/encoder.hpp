@@ -204,9 +204,8 @@ struct RangeEncoder {
             : "vcc");
     }
 
-    // the same, then the step count of the interval [low, low + width - 1]: n1 = clz(low ^ high)
-    // E1/E2 steps and the E3 run below them, the leading zeros of (~low | high) once the first
-    // differing bit is shifted out
+    // the same, then the step count of the interval [low, low + width - 1], as step_count() has it
+    // (common.hpp), four instructions after the window's add
     __device__ __forceinline__ int add_and_count(uint32_t add, uint32_t width)
     {
         int n;
@@ -216,13 +215,11 @@ struct RangeEncoder {
         uint64_t carry;
         asm("v_add_co_u32 v56, vcc, v56, %4\n\t"
             "v_addc_co_u32 v57, %2, 0, v57, vcc\n\t"
-            "v_add3_u32 %1, %5, v56, -1\n\t"
-            "v_xor_b32 %0, %1, v56\n\t"
-            "v_bitop3_b32 %1, %1, v56, %1 bitop3:0xf3\n\t"
-            "v_ffbh_u32 %0, %0\n\t"
-            "v_add_lshl_u32 %1, %1, %1, %0\n\t"
-            "v_ffbh_u32 %1, %1\n\t"
-            "v_add_u32 %0, %0, %1"
+            "v_add_u32 %0, -1, %5\n\t"
+            "v_add_u32 %1, %0, v56\n\t"
+            "v_bitop3_b32 %1, %1, v56, %0 bitop3:0x82\n\t"
+            "v_lshl_or_b32 %1, %1, 1, %0\n\t"
+            "v_ffbh_u32 %0, %1"
             : "=&v"(n), "=&v"(t), "=&s"(carry), "+{v[56:57]}"(tail)
             : "v"(add), "v"(width)
             : "vcc");

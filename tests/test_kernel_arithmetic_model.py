@@ -233,3 +233,71 @@ def test_word_schedule_does_not_change_the_stream(group):
         cdf = random_table(rng, nsym, rng.choice([1, 8]))
         syms = [rng.randrange(nsym) for _ in range(rng.choice([5, 64, 300]))]
         assert model_encode(cdf, syms, group) == pycoder.encode(cdf, syms)[0]
+
+
+def step_count(low, high, d, bits=32):
+    """common.hpp: step_count(), for a window of `bits` bits."""
+    mask = (1 << bits) - 1
+    return bits - ((((d & ~(low ^ high)) << 1) | d) & mask).bit_length()
+
+
+def serial_steps(low, high, bits):
+    """E1, E2 and E3 steps one at a time (enc_new.cu:275-305)."""
+    half, quarter, mask = 1 << (bits - 1), 1 << (bits - 2), (1 << bits) - 1
+    n = 0
+    while True:
+        if high < half or low >= half:
+            low, high = (low << 1) & mask, ((high << 1) | 1) & mask
+        elif low >= quarter and high < half + quarter:
+            low, high = (low << 1) & mask & ~half, ((high << 1) | 1 | half) & mask
+        else:
+            return n
+        n += 1
+
+
+@pytest.mark.parametrize("bits", [4, 7, 8])
+def test_step_count_for_every_interval_of_a_small_window(bits):
+    half, mask = 1 << (bits - 1), (1 << bits) - 1
+    for low in range(mask):
+        for high in range(low + 1, mask + 1):
+            want = serial_steps(low, high, bits)
+            for flip in (0, half):                         # bit 31 may hold a stale 1 in both
+                assert step_count(low ^ flip, high ^ flip, high - low, bits) == want
+
+
+def test_step_count_of_the_whole_window():
+    rng = random.Random(5)
+    for _ in range(20000):
+        low, high = sorted(rng.getrandbits(32) >> rng.randrange(31) for _ in range(2))
+        if rng.random() < 0.5:                             # around the middle: runs of E3 steps
+            low, high = 0x7FFFFFFF - (low >> 1), 0x80000000 + (high >> 1)
+        if low < high:
+            assert step_count(low, high, high - low) == serial_steps(low, high, 32)
+
+
+def test_low_and_span_shifted_as_one_word():
+    """decode_symbol moves {low, width} by one 64-bit shift: a width that becomes 2^32 leaves a 1 in
+    low, which the full range's own branch clears before low is used again."""
+    rng = random.Random(11)
+    tables = [[0, 32768, 65534, 65535], [0, 16384, 32768, 49152, 65535], [0, 1, 32768, 65535]]
+    tables += [random_table(rng, rng.choice([3, 15, 31]), 3) for _ in range(10)]
+    full = 0
+    for cdf in tables:
+        state = true = (0, 0)
+        for _ in range(400):
+            s = rng.randrange(len(cdf) - 1)
+            low, span = state
+            if span == 0:
+                full += 1
+                low = 0
+            t_lo, width = bound(cdf, s, span)
+            low = (low + t_lo) & M32
+            n = step_count(low, (low + width - 1) & M32, (width - 1) & M32)
+            packed = ((low << 32 | width) << n) & (1 << 64) - 1
+            state = packed >> 32, packed & M32
+            t_lo, width = bound(cdf, s, true[1])
+            low = (true[0] + t_lo) & M32
+            assert n == sum(shift_count(low, (low + width - 1) & M32))
+            true = (low << n) & M32, (width << n) & M32
+            assert state[1] == true[1] and (state[1] == 0 or (state[0] - true[0]) & (M32 >> 1) == 0)
+    assert full > 20
