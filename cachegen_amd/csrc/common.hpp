@@ -107,7 +107,9 @@ __device__ __forceinline__ uint32_t store16f(float f)
 // that they do not differ at, moved up by one, puts the leading bit at t + 1.  Bits below t cannot
 // pass t that way, and at t = 31 low and high always differ.  One ffbh on a chain of four
 // instructions, where clz(low ^ high) and the run of E3 steps below it took two on a chain of six:
-// the coders issue 21.4 -> 19.4 (encode) and 42.7 -> 39.7 (decode) vector instructions a symbol.
+// the coding loops have 17 instead of 19 (encoder) and 35 instead of 38 (decoder, rows of at most
+// 16 levels) vector instructions a symbol; decode of 32 layers x 8192 tokens x 1024 channels
+// 534 -> 512 us, encode of 80 layers x 32768 tokens x 1024 channels 6.53 -> 6.28 ms.
 __device__ __forceinline__ int step_count(uint32_t low, uint32_t high, uint32_t d)
 {
     return __builtin_clz(((d & ~(low ^ high)) << 1) | d);

@@ -197,7 +197,7 @@ __host__ __device__ constexpr int first_probe(int log2, int skip) { return log2 
 // (its upper bound 2^16 is substituted, dec_new.cu:278) and values may be NaN.
 template <int BS, int LOG2, int OUT, int SKIP, bool SAFE>
 __device__ __forceinline__ void decode_symbol(const DecodeArgs &a, DecodeLane &s, int lp, int nsteps,
-                                              float rm, int i, bool last_symbol)
+                                              float rm, int i)
 {
     constexpr int kRow = DecodeLayout<BS, OUT>::kRow;
     constexpr int kStep1 = first_probe(LOG2, SKIP), kStep2 = kStep1 >> 1;
@@ -300,7 +300,6 @@ __device__ __forceinline__ void decode_symbol(const DecodeArgs &a, DecodeLane &s
         else bits = float_to_f16_bits(v);
         __builtin_amdgcn_raw_buffer_store_b16((short)bits, s.orsrc, (int)s.ovoff, (int)((uint32_t)i * (uint32_t)a.ot * 2u), 0);
     }
-    if (last_symbol) return;                    // no update after the last symbol
     s.low += t_lo;
     s.off = rel;
     const uint32_t d = width - 1u;
@@ -342,7 +341,8 @@ __device__ __forceinline__ void decode_lane(const DecodeArgs &a, DecodeLane &s, 
     // the window is topped up at the head of every group of kGroup symbols and, inside a
     // group, only when a symbol has left it short of bits
     constexpr int kGroup = kSymbolsPerTopUp;
-    for (int i0 = 0; i0 < n; i0 += kGroup, rmp += kGroup) {
+    int i0 = 0;
+    for (; i0 + kGroup <= n; i0 += kGroup, rmp += kGroup) {
         if (last_round && (i0 & 63) == 0) {             // uniform over the wavefront
             const int left = (n - i0) >> 6;
             if (left >= 3) __builtin_amdgcn_s_setprio(3);
@@ -350,18 +350,22 @@ __device__ __forceinline__ void decode_lane(const DecodeArgs &a, DecodeLane &s, 
             else if (left == 1) __builtin_amdgcn_s_setprio(1);
             else __builtin_amdgcn_s_setprio(0);
         }
-        // the maxima of the group's token rows (the array is padded to a whole group)
+        // the maxima of the group's token rows
         float rm[kGroup];
 #pragma unroll
         for (int j = 0; j < kGroup; ++j) rm[j] = OUT != OUT_SYMBOLS ? rmp[j] : 0.0f;
 #pragma unroll
         for (int j = 0; j < kGroup; ++j) {
-            const int i = i0 + j;
-            if (i >= n) break;
             if (j == 0) s.rd.top_up();
             else if (__builtin_expect(s.rd.short_of_bits, 0)) s.rd.top_up();
-            decode_symbol<BS, LOG2, OUT, SKIP, SAFE>(a, s, lp, nsteps, rm[j], i, i == n - 1);
+            decode_symbol<BS, LOG2, OUT, SKIP, SAFE>(a, s, lp, nsteps, rm[j], i0 + j);
         }
+    }
+    // what is left of a sub-chunk whose tokens are no multiple of the group
+#pragma unroll 1
+    for (; i0 < n; ++i0, ++rmp) {
+        s.rd.top_up();
+        decode_symbol<BS, LOG2, OUT, SKIP, SAFE>(a, s, lp, nsteps, OUT != OUT_SYMBOLS ? *rmp : 0.0f, i0);
     }
 }
 

@@ -381,22 +381,14 @@ __global__ __launch_bounds__(BS) void encode_streams_kernel(EncodeArgs a)
     bool sentinel = true;
     int mode = kBytes;
     uint32_t half_shift = 0;
-    if (PACKED && a.key_bins) {
+    float cq = 0.0f;
+    const bool levels_known = PACKED && a.key_bins;
+    if (levels_known) {
         const int64_t kvi = id.row >= a.L ? 1 : 0, l = id.row - kvi * a.L;       // 2L rows: keys, then values
-        const float cq = floorf((kvi ? a.value_bins : a.key_bins)[l] * 0.5f) - 1.0f;
+        cq = floorf((kvi ? a.value_bins : a.key_bins)[l] * 0.5f) - 1.0f;
         sentinel = !(cq >= 0.0f && 2.0f * cq + 1.0f <= (float)(lp - 2));
-        if (a.maxima) {
-            int saturates = 0;
-            // every token row of the sub-chunk, whatever the block size
-            for (int i = tid; i < id.n; i += BS) {
-                const uint32_t bits = a.maxima[id.row * a.sg.g.T + id.t0 + i];
-                const float m = a.max_dt == CG_DT_BF16 ? load16f<CG_DT_BF16>(bits) : load16f<CG_DT_F16>(bits);
-                saturates |= scale_overflows(cq, m);
-            }
-            if (__syncthreads_or(saturates)) sentinel = true;       // the last symbol does occur
-        }
         if (a.nibbles && narrow_alphabet(cq, lp)) {
-            mode = sentinel ? kNibblesEscaped : kNibbles;
+            mode = kNibbles;
             if (id.active) symbols_voff = (uint32_t)(id.ch >> 1) * 4u;
             half_shift = (uint32_t)(id.ch & 1) * 16u;
         }
@@ -413,6 +405,18 @@ __global__ __launch_bounds__(BS) void encode_streams_kernel(EncodeArgs a)
             words[w] = __builtin_amdgcn_raw_buffer_load_b32(symbols_rsrc, (int)symbols_voff,
                                                             (int)((uint32_t)(h * 32 + w) * row_bytes), 0);
     };
+
+    if (levels_known && a.maxima) {
+        int saturates = 0;
+        // every token row of the sub-chunk, whatever the block size
+        for (int i = tid; i < id.n; i += BS) {
+            const uint32_t bits = a.maxima[id.row * a.sg.g.T + id.t0 + i];
+            const float m = a.max_dt == CG_DT_BF16 ? load16f<CG_DT_BF16>(bits) : load16f<CG_DT_F16>(bits);
+            saturates |= scale_overflows(cq, m);
+        }
+        if (__syncthreads_or(saturates)) sentinel = true;       // the last symbol does occur
+    }
+    if (mode == kNibbles && sentinel) mode = kNibblesEscaped;
 
     if (FUSE_CDF) {
         for (int i = 0; i < lp; ++i) col[i * TableStride<BS>::k16] = 0;
@@ -450,12 +454,16 @@ __global__ __launch_bounds__(BS) void encode_streams_kernel(EncodeArgs a)
             normalize_column16<BS>(col, lp, lp - 1, (uint32_t)id.n);
             write_column16<BS>(col, cdf_block + (int64_t)tid * lp, lp);
         }
-    } else {
-        // packed symbols: every lane copies its own table (the transposed copy costs a division
-        // and a dozen instructions an entry; this one costs the coder under one a symbol)
-        if (!PACKED) stage_tables16<BS>(tab, cdf_block, lp, ch0, a.sg.nc);
-        else if (id.active) stage_column16_stride<TableStride<BS>::k16>(col, cdf_block + (int64_t)tid * lp, lp);
+    } else if (!PACKED) {
+        stage_tables16<BS>(tab, cdf_block, lp, ch0, a.sg.nc);
         __syncthreads();
+    } else if (id.active) {
+        // Packed symbols: every lane copies its own table (the transposed copy costs a division and a
+        // dozen instructions an entry; this one costs the coder under one a symbol).  A lane reads
+        // its own column only and LDS serves a wavefront's accesses in order: no barrier, but the
+        // compiler must not move the coder's reads up.
+        stage_column16_stride<TableStride<BS>::k16>(col, cdf_block + (int64_t)tid * lp, lp);
+        asm volatile("" ::: "memory");
     }
     if (!id.active) return;
 
@@ -488,31 +496,39 @@ __global__ __launch_bounds__(BS) void encode_streams_kernel(EncodeArgs a)
         constexpr bool CLAMP = MODE == kBytes && SENTINEL;
         const uint32_t smax = (uint32_t)(lp - 2);
         if (PACKED) {
-            for (int h = 0; h * 32 < nwords; ++h) {
+            const int full = (id.n >> 3) * 2;              // words of full groups
+            for (int h = 0; h == 0 || h * 32 < full; ++h) {
                 load_half(h);
                 // uniform; kept in a scalar register so that the loop test is scalar too
-                const int wn = __builtin_amdgcn_readfirstlane(nwords - h * 32 < 32 ? nwords - h * 32 : 32);
-                // two words = eight symbols between two visits of the store code (wn is even
-                // except in a sub-chunk's last, partial run of words)
+                const int wn = __builtin_amdgcn_readfirstlane(full - h * 32 < 32 ? full - h * 32 : 32);
+                // two words = eight symbols between two visits of the store code, and no test per
+                // symbol of whether there is one
 #pragma unroll 1
                 for (int w = 0; w < wn; w += 2) {
                     const uint32_t v = MODE == kBytes ? words[w] : words[w] >> half_shift;
-                    const int t = (h * 32 + w) * 4;            // first token of the word
-                    if (t + 0 < id.n) enc.template put_symbol<SENTINEL, true, CLAMP>(packed_symbol<MODE>(v, 0, smax));
-                    if (t + 1 < id.n) enc.template put_symbol<SENTINEL, false, CLAMP>(packed_symbol<MODE>(v, 1, smax));
-                    if (t + 2 < id.n) enc.template put_symbol<SENTINEL, false, CLAMP>(packed_symbol<MODE>(v, 2, smax));
-                    if (t + 3 < id.n) enc.template put_symbol<SENTINEL, false, CLAMP>(packed_symbol<MODE>(v, 3, smax));
-                    if (t + 4 < id.n) {
-                        // w + 1 <= 31: wn <= 32
-                        const uint32_t u = MODE == kBytes ? words[w + 1] : words[w + 1] >> half_shift;
-                        enc.template put_symbol<SENTINEL, false, CLAMP>(packed_symbol<MODE>(u, 0, smax));
-                        if (t + 5 < id.n) enc.template put_symbol<SENTINEL, false, CLAMP>(packed_symbol<MODE>(u, 1, smax));
-                        if (t + 6 < id.n) enc.template put_symbol<SENTINEL, false, CLAMP>(packed_symbol<MODE>(u, 2, smax));
-                        if (t + 7 < id.n) enc.template put_symbol<SENTINEL, false, CLAMP>(packed_symbol<MODE>(u, 3, smax));
-                    }
+                    enc.template put_symbol<SENTINEL, true, CLAMP>(packed_symbol<MODE>(v, 0, smax));
+                    enc.template put_symbol<SENTINEL, false, CLAMP>(packed_symbol<MODE>(v, 1, smax));
+                    enc.template put_symbol<SENTINEL, false, CLAMP>(packed_symbol<MODE>(v, 2, smax));
+                    enc.template put_symbol<SENTINEL, false, CLAMP>(packed_symbol<MODE>(v, 3, smax));
+                    // fetched only here: there is no register to hold it earlier
+                    int w1 = w + 1;
+                    asm volatile("" : "+s"(w1));
+                    const uint32_t u = MODE == kBytes ? words[w1] : words[w1] >> half_shift;
+                    enc.template put_symbol<SENTINEL, false, CLAMP>(packed_symbol<MODE>(u, 0, smax));
+                    enc.template put_symbol<SENTINEL, false, CLAMP>(packed_symbol<MODE>(u, 1, smax));
+                    enc.template put_symbol<SENTINEL, false, CLAMP>(packed_symbol<MODE>(u, 2, smax));
+                    enc.template put_symbol<SENTINEL, false, CLAMP>(packed_symbol<MODE>(u, 3, smax));
                     enc.end_group();
                 }
             }
+            // the fewer than eight symbols behind the last full group, loaded again one at a time
+            // (keeping the registers indexed up to here costs the kernel its eighth wavefront)
+#pragma unroll 1
+            for (int t = full * 4; t < id.n; ++t) {
+                const uint32_t x = __builtin_amdgcn_raw_buffer_load_b32(symbols_rsrc, (int)symbols_voff, (int)((uint32_t)(t >> 2) * row_bytes), 0);
+                enc.template put_symbol<SENTINEL, false, CLAMP>(packed_symbol<MODE>(MODE == kBytes ? x : x >> half_shift, t & 3, smax));
+            }
+            enc.end_group();
         } else {
             const uint8_t *sp = a.sym + id.row * a.s0 + id.t0 * a.s1 + id.ch * a.s2;
             uint32_t nxt[8];

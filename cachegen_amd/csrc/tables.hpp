@@ -129,20 +129,23 @@ __device__ __forceinline__ void stage_tables16(uint16_t *tab, const uint16_t *cd
 }
 
 // Copy one lane's own table (lp consecutive 16-bit entries at `mine`) into its LDS column
-// col[e * kS]: loads and LDS writes on immediate offsets, sixteen loads in flight; the lanes of a
-// wavefront read neighbouring tables, so every cache line is fetched once.
+// col[e * kS]: loads and LDS writes on immediate offsets.  Whole batches carry no test per entry, so
+// that the compiler joins a batch's loads into two of 128 bits: the lanes of a wavefront read places
+// lp entries apart, and every load instruction costs the memory pipeline a visit to each of them (33
+// 16-bit loads a lane took it longer than the data takes to arrive).
 template <int kS>
 __device__ __forceinline__ void stage_column16_stride(uint16_t *col, const uint16_t *mine, int lp)
 {
     constexpr int kBatch = 16;
-    for (int e0 = 0; e0 < lp; e0 += kBatch) {
+    int e0 = 0;
+    for (; e0 + kBatch <= lp; e0 += kBatch) {
         uint16_t v[kBatch];
 #pragma unroll
-        for (int j = 0; j < kBatch; ++j) v[j] = e0 + j < lp ? mine[e0 + j] : (uint16_t)0;
+        for (int j = 0; j < kBatch; ++j) v[j] = mine[e0 + j];
 #pragma unroll
-        for (int j = 0; j < kBatch; ++j)
-            if (e0 + j < lp) col[(e0 + j) * kS] = v[j];
+        for (int j = 0; j < kBatch; ++j) col[(e0 + j) * kS] = v[j];
     }
+    for (; e0 < lp; ++e0) col[e0 * kS] = mine[e0];
 }
 
 // Write one lane's own table, col[e * kS], e in [0, lp), to its lp consecutive 16-bit entries
