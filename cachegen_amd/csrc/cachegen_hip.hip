@@ -159,7 +159,8 @@ int cg_decode_fast_new(const int16_t *cdf, int lp, const uint8_t *padded, int64_
     if (nl <= 0 || nc <= 0 || nt <= 0) return fail(CG_ERR_ARG, "decode: empty input");
     if (nt > kSub) return fail(CG_ERR_ARG, "Number of tokens should be less than or equal to %d", kSub);
     if (cap <= 0 || cap > INT_MAX) return fail(CG_ERR_ARG, "decode: bad padded buffer length");
-    const int block = pick_block(nc, lp);
+    const bool few = few_wavefronts(nl, nc, 1, lp);
+    const int block = few ? 64 : pick_block(nc, lp);
     DecodeArgs a;
     memset(&a, 0, sizeof(a));
     a.cdf = reinterpret_cast<const uint16_t *>(cdf);
@@ -174,7 +175,7 @@ int cg_decode_fast_new(const int16_t *cdf, int lp, const uint8_t *padded, int64_
     a.last_round_first = 0xFFFFFFFFu;     // one sub-chunk: a single round of blocks
     int64_t nblocks;
     if (int rc = make_grid(nl, nc, nt, nt, 1, block, a.sg, nblocks)) return rc;
-    return launch_decode_symbols<SRC_PADDED>(a, nblocks, block, static_cast<hipStream_t>(stream));
+    return launch_decode_symbols<SRC_PADDED>(a, nblocks, block, few, static_cast<hipStream_t>(stream));
 }
 
 int cg_decode_fast_prefsum(const int16_t *cdf, int lp, const uint8_t *bytes, int64_t nbytes,
@@ -185,7 +186,8 @@ int cg_decode_fast_prefsum(const int16_t *cdf, int lp, const uint8_t *bytes, int
     if (int rc = check_lp(lp, "decode")) return rc;
     if (nl <= 0 || nc <= 0 || nt <= 0) return fail(CG_ERR_ARG, "decode: empty input");
     if (nt > kSub) return fail(CG_ERR_ARG, "Number of tokens should be less than or equal to %d", kSub);
-    const int block = pick_block(nc, lp);
+    const bool few = few_wavefronts(nl, nc, 1, lp);
+    const int block = few ? 64 : pick_block(nc, lp);
     DecodeArgs a;
     memset(&a, 0, sizeof(a));
     a.cdf = reinterpret_cast<const uint16_t *>(cdf);
@@ -199,7 +201,7 @@ int cg_decode_fast_prefsum(const int16_t *cdf, int lp, const uint8_t *bytes, int
     a.last_round_first = 0xFFFFFFFFu;     // one sub-chunk: a single round of blocks
     int64_t nblocks;
     if (int rc = make_grid(nl, nc, nt, nt, 1, block, a.sg, nblocks)) return rc;
-    return launch_decode_symbols<SRC_PREFIX>(a, nblocks, block, static_cast<hipStream_t>(stream));
+    return launch_decode_symbols<SRC_PREFIX>(a, nblocks, block, few, static_cast<hipStream_t>(stream));
 }
 
 int cg_quantize_kv(const void *kv, int kv_dt, int64_t L, int64_t T, int64_t H, int64_t D, int64_t sl,
@@ -594,10 +596,11 @@ int cg_decode_kv(const int16_t *cdf, int max_bins, const void *maxima, int max_d
     a.delta_group = delta_group;
     a.key_bins = key_bins;
     a.value_bins = value_bins;
-    const int block = decode_kv_block(C, a.lp);
+    const bool few = few_wavefronts(rows, C, cg_num_subchunks(T, chunk_tokens), a.lp);
+    const int block = few ? 64 : decode_kv_block(C, a.lp);
     int64_t nblocks;
     if (int rc = make_grid(rows, C, T, chunk_tokens, cg_num_subchunks(T, chunk_tokens), block, a.sg, nblocks)) return rc;
-    return launch_decode_kv<SRC_OFFSETS>(a, nblocks, block, out_dt, static_cast<hipStream_t>(stream));
+    return launch_decode_kv<SRC_OFFSETS>(a, nblocks, block, few, out_dt, static_cast<hipStream_t>(stream));
 }
 
 int cg_decode_listed(const CgListedSub *subs, int64_t nsub, int max_bins, int64_t L, int64_t H, int64_t D,
@@ -615,11 +618,12 @@ int cg_decode_listed(const CgListedSub *subs, int64_t nsub, int max_bins, int64_
     a.L = L;
     a.delta_group = delta_group;
     a.listed = subs;
-    const int block = decode_kv_block(C, a.lp);
+    const bool few = few_wavefronts(rows, C, nsub, a.lp);
+    const int block = few ? 64 : decode_kv_block(C, a.lp);
     int64_t nblocks;
     // the entries hold the token geometry; the grid only needs its size
     if (int rc = make_grid(rows, C, nsub, 1, nsub, block, a.sg, nblocks)) return rc;
-    return launch_decode_kv<SRC_LISTED>(a, nblocks, block, out_dt, static_cast<hipStream_t>(stream));
+    return launch_decode_kv<SRC_LISTED>(a, nblocks, block, few, out_dt, static_cast<hipStream_t>(stream));
 }
 
 int cg_host_tile_starts(const void *lengths, int itemsize, int64_t nsub, int64_t rows, int64_t C,

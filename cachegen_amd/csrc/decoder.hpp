@@ -176,6 +176,7 @@ struct DecodeLane {
     // the entries the first two probes of the unrolled search look at (one for the first, one
     // of two for the second), read once per stream: two LDS round trips less per symbol
     uint32_t probe1, probe2_lo, probe2_hi;
+    uint32_t held[16];         // FEW: every fourth entry of the part of the table that is searched (entry 0 unused)
     // the decoded symbol's two table entries, each shifted left by 16: only ever written by
     // loads into the upper half, so that the lower halves stay zero
     uint32_t bound_lo, bound_hi;
@@ -192,10 +193,24 @@ struct DecodeLane {
 // Distance of the unrolled search's first probe from entry 0, in entries.
 __host__ __device__ constexpr int first_probe(int log2, int skip) { return log2 >= 2 ? ((1 << log2) >> 1) >> skip : 0; }
 
+// A launch of few wavefronts (FEW) is as long as one stream's dependent chain: a SIMD with one to
+// three wavefronts has issue slots to spare, and an LDS round trip costs a lane some 120 cycles per
+// search step.  There the search holds every fourth entry in registers, halving them by selects
+// until four candidates are left, reads those and the next one in ONE round trip and picks both
+// bounds from them; a symbol's quotient and output follow after the interval's update, off the chain.
+// More instructions (about 50 instead of 35 to 39), so from four wavefronts a SIMD on the plain search
+// is faster (few_wavefronts in launch.hpp).  One chunk of 256 tokens x 1024 channels x 32 layers, one
+// wavefront a SIMD: tables of 32 symbols 93 -> 72 us, of 16 82 -> 68, of 64 107 -> 83 (the shorter step
+// count included).
+template <int LOG2, int SKIP>
+struct FewSearch {
+    static constexpr int kHeld = LOG2 - SKIP >= 3 ? (1 << (LOG2 - SKIP - 2)) : 0;   // four candidates per held entry
+};
+
 // One symbol.  SKIP: how many of the search's first probes are left out because the row's
 // alphabet fits the lower 2^(LOG2-SKIP) entries.  SAFE: the last table entry may be decoded
 // (its upper bound 2^16 is substituted, dec_new.cu:278) and values may be NaN.
-template <int BS, int LOG2, int OUT, int SKIP, bool SAFE>
+template <int BS, int LOG2, int OUT, int SKIP, bool SAFE, bool FEW>
 __device__ __forceinline__ void decode_symbol(const DecodeArgs &a, DecodeLane &s, int lp, int nsteps,
                                               float rm, int i)
 {
@@ -209,20 +224,48 @@ __device__ __forceinline__ void decode_symbol(const DecodeArgs &a, DecodeLane &s
     const uint32_t sh = s.span >> 16, sl = s.span & 0xFFFFu;
     if (LOG2 >= 2) {
         // largest m with T(m) <= off, probed with the lower bound sh * c <= T(c), which can
-        // only overshoot; the first two probes compare entries held in registers
-        const bool up1 = mul24(sh, s.probe1) <= s.off;
-        p = up1 ? p + kStep1 * kRow : p;
-        if (kStep2 >= 1) {
-            const uint32_t c2 = up1 ? s.probe2_hi : s.probe2_lo;
-            p = (mul24(sh, c2) <= s.off) ? p + kStep2 * kRow : p;
-        }
+        // only overshoot
+        if constexpr (FEW) {
+            constexpr int kHeld = FewSearch<LOG2, SKIP>::kHeld;
+            uint32_t left[kHeld];
 #pragma unroll
-        for (int step = kStep2 >> 1; step >= 1; step >>= 1)
-            p = (mul24(sh, lds_entry(p, step * kRow)) <= s.off) ? p + step * kRow : p;
-        // both bounds and the quotient in one round trip (entry lp - 1 exists, so the upper
-        // bound of the last symbol can be read and then replaced)
-        if (OUT != OUT_SYMBOLS) q = *(lds_f32 *)(p + s.lutoff);
-        lds_entries_high<kRow>(p, s.bound_lo, s.bound_hi);
+            for (int k = 1; k < kHeld; ++k) left[k] = s.held[k];
+#pragma unroll
+            for (int half = kHeld >> 1; half >= 1; half >>= 1) {
+                const bool up = mul24(sh, left[half]) <= s.off;
+                p = up ? p + half * 4 * kRow : p;
+#pragma unroll
+                for (int k = 1; k < half; ++k) {
+                    // both values first: a choice between two places becomes an indexed access
+                    const uint32_t below = left[k], above = left[half + k];
+                    left[k] = up ? above : below;
+                }
+            }
+            // entry p + 4 exists: the table has 2^LOG2 + 1 entries
+            uint32_t c0, c1, c2, c3, c4;
+            lds_five_entries<kRow>(p, c0, c1, c2, c3, c4);
+            const bool up1 = mul24(sh, c1) <= s.off, up2 = mul24(sh, c2) <= s.off, up3 = mul24(sh, c3) <= s.off;
+            p += up2 ? (up3 ? 3 * kRow : 2 * kRow) : (up1 ? kRow : 0);
+            s.bound_lo = (up2 ? (up3 ? c3 : c2) : (up1 ? c1 : c0)) << 16;
+            s.bound_hi = (up2 ? (up3 ? c4 : c3) : (up1 ? c2 : c1)) << 16;
+            // volatile: issued here, not joined with the rare path's load behind the update
+            if (OUT != OUT_SYMBOLS) q = *(volatile lds_f32 *)(p + s.lutoff);
+        } else {
+            // the first two probes compare entries held in registers
+            const bool up1 = mul24(sh, s.probe1) <= s.off;
+            p = up1 ? p + kStep1 * kRow : p;
+            if (kStep2 >= 1) {
+                const uint32_t c2 = up1 ? s.probe2_hi : s.probe2_lo;
+                p = (mul24(sh, c2) <= s.off) ? p + kStep2 * kRow : p;
+            }
+#pragma unroll
+            for (int step = kStep2 >> 1; step >= 1; step >>= 1)
+                p = (mul24(sh, lds_entry(p, step * kRow)) <= s.off) ? p + step * kRow : p;
+            // both bounds and the quotient in one round trip (entry lp - 1 exists, so the upper
+            // bound of the last symbol can be read and then replaced)
+            if (OUT != OUT_SYMBOLS) q = *(lds_f32 *)(p + s.lutoff);
+            lds_entries_high<kRow>(p, s.bound_lo, s.bound_hi);
+        }
         // T(c) = (span * c) >> 16 = high word of span * (c << 16) for c < 2^16; the one entry
         // that is 2^16, the upper bound of the last symbol (dec_new.cu:278), gives the span
         t_lo = __umulhi(s.span, s.bound_lo);
@@ -282,24 +325,27 @@ __device__ __forceinline__ void decode_symbol(const DecodeArgs &a, DecodeLane &s
         }
         rel = s.off - t_lo;
     }
-    if (OUT == OUT_SYMBOLS) {
-        s.osym[(int64_t)i * a.o1] = (uint8_t)((uint32_t)(p - s.colp) / (uint32_t)kRow);
-    } else {
-        float v = __fmul_rn(q, rm);
-        // the product is rounded to float32 before it is rounded to 16 bits (decoder.py:28-34
-        // works in float32): keep the compiler from merging the two into one mixed-precision
-        // multiply, which rounds once and turns -0 into +0
-        asm volatile("" : "+v"(v));
-        if (SAFE && a.delta_group > 0) {             // uniform over the block
-            if (s.phase == 0) s.anchor = v;
-            else v = __fadd_rn(v, s.anchor);
-            s.phase = s.phase + 1 == a.delta_group ? 0 : s.phase + 1;
+    auto put_out = [&]() {
+        if (OUT == OUT_SYMBOLS) {
+            s.osym[(int64_t)i * a.o1] = (uint8_t)((uint32_t)(p - s.colp) / (uint32_t)kRow);
+        } else {
+            float v = __fmul_rn(q, rm);
+            // the product is rounded to float32 before it is rounded to 16 bits (decoder.py:28-34
+            // works in float32): keep the compiler from merging the two into one mixed-precision
+            // multiply, which rounds once and turns -0 into +0
+            asm volatile("" : "+v"(v));
+            if (SAFE && a.delta_group > 0) {             // uniform over the block
+                if (s.phase == 0) s.anchor = v;
+                else v = __fadd_rn(v, s.anchor);
+                s.phase = s.phase + 1 == a.delta_group ? 0 : s.phase + 1;
+            }
+            uint32_t bits;
+            if (OUT == OUT_BF16) bits = float_to_bf16_bits_hw(v);
+            else bits = float_to_f16_bits(v);
+            __builtin_amdgcn_raw_buffer_store_b16((short)bits, s.orsrc, (int)s.ovoff, (int)((uint32_t)i * (uint32_t)a.ot * 2u), 0);
         }
-        uint32_t bits;
-        if (OUT == OUT_BF16) bits = float_to_bf16_bits_hw(v);
-        else bits = float_to_f16_bits(v);
-        __builtin_amdgcn_raw_buffer_store_b16((short)bits, s.orsrc, (int)s.ovoff, (int)((uint32_t)i * (uint32_t)a.ot * 2u), 0);
-    }
+    };
+    if (!FEW) put_out();
     s.low += t_lo;
     s.off = rel;
     const uint32_t d = width - 1u;
@@ -313,6 +359,10 @@ __device__ __forceinline__ void decode_symbol(const DecodeArgs &a, DecodeLane &s
     s.low = (uint32_t)(interval >> 32);
     s.span = (uint32_t)interval;
     s.off = s.rd.shift_in(s.off, n);
+    if (FEW) {
+        asm volatile("" : "+v"(q) : "v"(s.off), "v"(s.span));       // not before the update
+        put_out();
+    }
 }
 
 // last_round: the block is one of the launch's last, after which nothing takes the place of a
@@ -323,7 +373,7 @@ __device__ __forceinline__ void decode_symbol(const DecodeArgs &a, DecodeLane &s
 // the most advanced wavefronts first and leaves the least advanced for the end; these blocks
 // raise their wavefronts' priority by the work they have left instead, so that the wavefronts of
 // a SIMD finish closer together.
-template <int BS, int LOG2, int OUT, int SKIP, bool SAFE>
+template <int BS, int LOG2, int OUT, int SKIP, bool SAFE, bool FEW>
 __device__ __forceinline__ void decode_lane(const DecodeArgs &a, DecodeLane &s, int lp, int n, lds_f32 *rmp, bool last_round)
 {
     int nsteps = 0;
@@ -337,6 +387,10 @@ __device__ __forceinline__ void decode_lane(const DecodeArgs &a, DecodeLane &s, 
         s.probe2_hi = lds_entry(s.colp, (kStep1 + kStep2) * kRow);
         s.bound_lo = 0;
         s.bound_hi = 0;
+        if constexpr (FEW) {
+#pragma unroll
+            for (int k = 1; k < FewSearch<LOG2, SKIP>::kHeld; ++k) s.held[k] = lds_entry(s.colp, 4 * k * kRow);
+        }
     }
     // the window is topped up at the head of every group of kGroup symbols and, inside a
     // group, only when a symbol has left it short of bits
@@ -358,23 +412,22 @@ __device__ __forceinline__ void decode_lane(const DecodeArgs &a, DecodeLane &s, 
         for (int j = 0; j < kGroup; ++j) {
             if (j == 0) s.rd.top_up();
             else if (__builtin_expect(s.rd.short_of_bits, 0)) s.rd.top_up();
-            decode_symbol<BS, LOG2, OUT, SKIP, SAFE>(a, s, lp, nsteps, rm[j], i0 + j);
+            decode_symbol<BS, LOG2, OUT, SKIP, SAFE, FEW>(a, s, lp, nsteps, rm[j], i0 + j);
         }
     }
     // what is left of a sub-chunk whose tokens are no multiple of the group
 #pragma unroll 1
     for (; i0 < n; ++i0, ++rmp) {
         s.rd.top_up();
-        decode_symbol<BS, LOG2, OUT, SKIP, SAFE>(a, s, lp, nsteps, OUT != OUT_SYMBOLS ? *rmp : 0.0f, i0);
+        decode_symbol<BS, LOG2, OUT, SKIP, SAFE, FEW>(a, s, lp, nsteps, OUT != OUT_SYMBOLS ? *rmp : 0.0f, i0);
     }
 }
 
 // LOG2 >= 0: the table has exactly 2^LOG2 symbols (lp = 2^LOG2 + 1) and the search is
 // unrolled with immediate LDS offsets; LOG2 < 0: any lp.
-template <int BS, int LOG2, int SRC, int OUT>
-__global__ __launch_bounds__(BS) void decode_streams_kernel(DecodeArgs a)
+template <int BS, int LOG2, int SRC, int OUT, bool FEW>
+__device__ __forceinline__ void decode_streams(const DecodeArgs &a, uint32_t *smem)
 {
-    extern __shared__ uint32_t smem[];
     constexpr int kRow = DecodeLayout<BS, OUT>::kRow;
     const int tid = threadIdx.x;
     StreamId id;
@@ -513,9 +566,24 @@ __global__ __launch_bounds__(BS) void decode_streams_kernel(DecodeArgs a)
     // all three conditions are uniform over the block
     const bool safe = OUT == OUT_SYMBOLS || LOG2 < 0 || special || a.delta_group > 0 || nsym > lp - 2;
     const bool last_round = linear_block() >= a.last_round_first;
-    if (safe) decode_lane<BS, LOG2, OUT, 0, true>(a, s, lp, id.n, rmp, last_round);
-    else if (LOG2 > 1 && nsym <= (1 << (LOG2 > 1 ? LOG2 - 1 : 0))) decode_lane<BS, LOG2, OUT, 1, false>(a, s, lp, id.n, rmp, last_round);
-    else decode_lane<BS, LOG2, OUT, 0, false>(a, s, lp, id.n, rmp, last_round);
+    if (safe) decode_lane<BS, LOG2, OUT, 0, true, FEW>(a, s, lp, id.n, rmp, last_round);
+    else if (LOG2 > 1 && nsym <= (1 << (LOG2 > 1 ? LOG2 - 1 : 0))) decode_lane<BS, LOG2, OUT, 1, false, FEW>(a, s, lp, id.n, rmp, last_round);
+    else decode_lane<BS, LOG2, OUT, 0, false, FEW>(a, s, lp, id.n, rmp, last_round);
+}
+
+template <int BS, int LOG2, int SRC, int OUT>
+__global__ __launch_bounds__(BS) void decode_streams_kernel(DecodeArgs a)
+{
+    extern __shared__ uint32_t smem[];
+    decode_streams<BS, LOG2, SRC, OUT, false>(a, smem);
+}
+
+// One wavefront a block, so that few wavefronts spread over the compute units (see FewSearch).
+template <int LOG2, int SRC, int OUT>
+__global__ __launch_bounds__(64) void decode_few_kernel(DecodeArgs a)
+{
+    extern __shared__ uint32_t smem[];
+    decode_streams<64, LOG2, SRC, OUT, true>(a, smem);
 }
 
 }  // namespace

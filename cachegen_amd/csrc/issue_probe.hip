@@ -18,9 +18,9 @@ extern "C" {
 
 // kind: 0 = cheap class (v_add_u32, v_xor_b32, v_lshrrev_b32, v_and_b32 in turn)
 //       1 = full-rate class (v_mul_u32_u24, v_cndmask_b32, v_lshlrev_b32, v_add3_u32 in turn)
-//       2 = one decoded symbol of decode_streams_kernel (rows of at most 16 levels): 27 instructions
+//       2 = one decoded symbol of decode_streams_kernel (rows of at most 16 levels): 24 instructions
 //           of the full class and 11 of the cheap class in the order the compiler emits them
-// iters: loop trips of 64 (kinds 0, 1) or 76 (kind 2: two symbols of 38) instructions per wavefront
+// iters: loop trips of 64 (kinds 0, 1) or 70 (kind 2: two symbols of 35) instructions per wavefront
 // ns_per_instruction: time one SIMD takes per wave64 instruction, 8 wavefronts resident
 // clock_mhz: engine clock while the probe ran
 // Returns 0, or the hipError_t that stopped it.
@@ -90,17 +90,15 @@ __global__ __launch_bounds__(256) void issue_rate_kernel(uint32_t *sink, ClockSa
             "v_sub_u32 " q ", " q ", " p "\n\tv_sub_u32 " y ", " y ", " p "\n\t"                \
             "v_cmp_ge_u32 vcc, " y ", " q "\n\t"                                                \
             "v_mul_f32 " p ", " p ", " q "\n\tv_cvt_f16_f32 " p ", " p "\n\t"                   \
-            "v_add_u32 " p ", " p ", " x "\n\tv_add3_u32 " q ", " q ", " p ", -1\n\t"           \
-            "v_xor_b32 " y ", " q ", " p "\n\tv_bitop3_b32 " q ", " q ", " p ", " q " bitop3:0xf3\n\t" \
-            "v_ffbh_u32 " y ", " y "\n\tv_add_lshl_u32 " q ", " q ", " q ", " y "\n\t"          \
-            "v_ffbh_u32 " q ", " q "\n\tv_add_u32 " q ", " q ", " y "\n\t"                      \
-            "v_sub_co_u32 " p ", vcc, " p ", " q "\n\tv_lshlrev_b32 " x ", " q ", " x "\n\t"    \
-            "v_mov_b32 " y ", " p "\n\tv_lshlrev_b32 " p ", " q ", " p "\n\t"
+            "v_add_u32 " p ", " p ", " x "\n\tv_add_u32 " q ", -1, " q "\n\t"                   \
+            "v_add_u32 " y ", " p ", " q "\n\tv_bitop3_b32 " y ", " q ", " p ", " y " bitop3:0x90\n\t" \
+            "v_lshl_or_b32 " q ", " y ", 1, " q "\n\tv_ffbh_u32 " q ", " q "\n\t"               \
+            "v_sub_co_u32 " p ", vcc, " p ", " q "\n\tv_mov_b32 " y ", " p "\n\t"
             uint32_t t0 = a, t1 = c, t2 = b, t3 = d;
             asm volatile(CG_PROBE_SYMBOL("%0", "%1", "%4", "%5")
-                         "v_lshlrev_b64 %2, %5, %2\n\tv_lshlrev_b64 %3, %5, %3\n\t"
+                         "v_lshlrev_b64 %2, %5, %2\n\tv_lshlrev_b64 %3, %5, %3\n\tv_lshlrev_b64 %2, %5, %2\n\t"
                          CG_PROBE_SYMBOL("%1", "%0", "%6", "%7")
-                         "v_lshlrev_b64 %2, %7, %2\n\tv_lshlrev_b64 %3, %7, %3"
+                         "v_lshlrev_b64 %2, %7, %2\n\tv_lshlrev_b64 %3, %7, %3\n\tv_lshlrev_b64 %2, %7, %2"
                          : "+v"(a), "+v"(c), "+v"(w), "+v"(w2), "+v"(t0), "+v"(t1), "+v"(t2), "+v"(t3)
                          : "v"(b), "v"(d)
                          : "vcc");
@@ -174,7 +172,7 @@ extern "C" int cg_probe_issue_rate(int kind, int iters, double *ns_per_instructi
     CG_PROBE_CHECK(hipFree(sample));
     CG_PROBE_CHECK(hipEventDestroy(e0));
     CG_PROBE_CHECK(hipEventDestroy(e1));
-    const double per_trip = kind == 2 ? 76.0 : 64.0;     // instructions per loop trip and wavefront
+    const double per_trip = kind == 2 ? 70.0 : 64.0;     // instructions per loop trip and wavefront
     const double per_simd = (double)blocks * 4.0 * iters * per_trip / (cus * 4.0);
     *ns_per_instruction = (double)ms * 1e6 / per_simd;
     const double ticks = (double)(host.ticks1 - host.ticks0);

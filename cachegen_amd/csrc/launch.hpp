@@ -428,18 +428,44 @@ void launch_decode_log2(const DecodeArgs &a, dim3 grid, size_t shmem, hipStream_
     }
 }
 
+// Whether a decode of these wavefronts is bound by one stream's dependent chain (decode_few_kernel,
+// blocks of 64): up to kFewWavefronts a SIMD, tables of 16, 32 or 64 symbols.  Measured with 32
+// layers x 1024 channels, decode_streams_kernel / decode_few_kernel: three wavefronts a SIMD (768
+// tokens) 97 / 92 us for tables of 32 symbols, 86 / 83 for 16, 114 / 108 for 64; four (1024 tokens)
+// 101 / 105, 90 / 94, 122 / 127.  Tables of 8 symbols have one LDS search step to save and no
+// instantiation; other lengths search by bisection.
+constexpr int64_t kFewWavefronts = 3;
+bool few_wavefronts(int64_t rows, int64_t nc, int64_t nsub, int lp)
+{
+    if (lp != 17 && lp != 33 && lp != 65) return false;
+    const int64_t most = (int64_t)compute_units() * 4 * kFewWavefronts;
+    const int64_t tiles = ceil_div(nc, 64);
+    return rows <= most && tiles <= most && nsub <= most && rows * tiles <= most && rows * tiles * nsub <= most;
+}
+
+template <int SRC, int OUT>
+void launch_decode_few(const DecodeArgs &a, dim3 grid, size_t shmem, hipStream_t stream)
+{
+    switch (a.lp) {
+    case 17: decode_few_kernel<4, SRC, OUT><<<grid, 64, shmem, stream>>>(a); break;
+    case 33: decode_few_kernel<5, SRC, OUT><<<grid, 64, shmem, stream>>>(a); break;
+    default: decode_few_kernel<6, SRC, OUT><<<grid, 64, shmem, stream>>>(a); break;
+    }
+}
+
 template <int SRC>
-int launch_decode_symbols(const DecodeArgs &a, int64_t nblocks, int block, hipStream_t stream)
+int launch_decode_symbols(const DecodeArgs &a, int64_t nblocks, int block, bool few, hipStream_t stream)
 {
     const dim3 grid = stream_grid(a.sg, nblocks);
     const size_t shmem = decode_shmem(a.lp, block);
-    CG_DISPATCH_BS(block, (launch_decode_log2<BS, SRC, OUT_SYMBOLS>(a, grid, shmem, stream)));
+    if (few) launch_decode_few<SRC, OUT_SYMBOLS>(a, grid, shmem, stream);
+    else CG_DISPATCH_BS(block, (launch_decode_log2<BS, SRC, OUT_SYMBOLS>(a, grid, shmem, stream)));
     return check_launch("decode");
 }
 
 // Dequantised output (SRC_OFFSETS, SRC_LISTED): blocks of at most 128 lanes.
 template <int SRC>
-int launch_decode_kv(DecodeArgs &a, int64_t nblocks, int block, int out_dt, hipStream_t stream)
+int launch_decode_kv(DecodeArgs &a, int64_t nblocks, int block, bool few, int out_dt, hipStream_t stream)
 {
     const size_t shmem = decode_shmem(a.lp, block);
     const dim3 grid = stream_grid(a.sg, nblocks);
@@ -447,7 +473,10 @@ int launch_decode_kv(DecodeArgs &a, int64_t nblocks, int block, int out_dt, hipS
     // where registers and LDS allow it, which they do for tables of up to 33 entries)
     const int64_t resident = (int64_t)compute_units() * (2048 / block);
     a.last_round_first = (uint32_t)(nblocks > resident ? nblocks - resident : 0);
-    if (block == 128) {
+    if (few) {
+        if (out_dt == CG_DT_BF16) launch_decode_few<SRC, OUT_BF16>(a, grid, shmem, stream);
+        else launch_decode_few<SRC, OUT_F16>(a, grid, shmem, stream);
+    } else if (block == 128) {
         if (out_dt == CG_DT_BF16) launch_decode_log2<128, SRC, OUT_BF16>(a, grid, shmem, stream);
         else launch_decode_log2<128, SRC, OUT_F16>(a, grid, shmem, stream);
     } else {
