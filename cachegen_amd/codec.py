@@ -268,12 +268,19 @@ def decode_kv(cdf, maxima, offsets, payload, key_bins, value_bins, num_layers, n
     return out
 
 
+def check_output(out, num_layers, num_heads, head_size, fmt):
+    """Refuses an output tensor that `decode_listed` cannot write for this geometry; returns its tokens."""
+    (L, T, H, D), _ = _kv_strides(out, fmt)
+    if (L, H, D) != (num_layers, num_heads, head_size) or out.dtype not in _DT:
+        raise RuntimeError("output tensor does not match the encoded geometry")
+    return T
+
+
 def decode_listed(subs_ptr, nsub, max_bins, num_layers, num_heads, head_size, delta_group, out, fmt):
     """cg_decode_listed: nsub sub-chunks described by entries in device memory (serde/incoming.py
     writes them), all with tables of max_bins + 1 entries, into token ranges of `out`."""
+    check_output(out, num_layers, num_heads, head_size, fmt)
     (L, _, H, D), (ol, okv, ot, oh) = _kv_strides(out, fmt)
-    if (L, H, D) != (num_layers, num_heads, head_size) or out.dtype not in _DT:
-        raise RuntimeError("output tensor does not match the encoded geometry")
     with torch.cuda.device(out.device):
         _lib.check(_lib.lib().cg_decode_listed(subs_ptr, nsub, max_bins, L, H, D, int(delta_group), out.data_ptr(),
                                                _DT[out.dtype], ol, okv, ot, oh, _stream(out.device)))

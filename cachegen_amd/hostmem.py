@@ -57,3 +57,33 @@ def new_bytes(n: int):
             _libc.madvise(first, last - first, _MADV_HUGEPAGE)
             t.fill_(0)
     return b, t
+
+
+class StoredWords:
+    """Pinned words, zero at first, that kernels on the current stream store to; to be used in a
+    `with` block that holds the launches.
+
+    torch's pool of pinned memory hands a block to the next caller as soon as its tensor is gone,
+    unless one of torch's own copies still uses it: of a kernel's stores it knows nothing.  So the
+    words are held until the launches are through, also when the `with` block ends in an exception."""
+
+    def __init__(self, n: int, dtype: torch.dtype):
+        self.words = torch.zeros(n, dtype=dtype, pin_memory=True)
+        self._stream = torch.cuda.current_stream()
+        self._stored = None
+
+    def __enter__(self):
+        return self
+
+    def stored(self):
+        """Everything that stores to the words has been launched: `read` waits for that, and not for
+        what is launched afterwards."""
+        self._stored = self._stream.record_event()
+
+    def read(self):
+        """The words as a list, once the launches before `stored` are through."""
+        self._stored.synchronize()
+        return self.words.tolist()
+
+    def __exit__(self, *exc):
+        (self._stored or self._stream).synchronize()

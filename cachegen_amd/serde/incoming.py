@@ -7,6 +7,7 @@ sub-chunk where its tables, maxima, lengths, payload and output tokens are, and 
 the stream lengths, which the host has to add up anyway to check them against the payload's size.
 One launch then decodes every sub-chunk of every blob (`cg_decode_listed`): no per-blob launches,
 no scan of the lengths on the device, no conversion of 16-bit lengths."""
+import contextlib
 import ctypes
 import struct
 
@@ -133,6 +134,8 @@ def decode(items, out, fmt):
     L, H, D = first.num_layers, first.num_heads, first.head_size
     C, rows, device = H * D, 2 * first.num_layers, out.device
     lib = _lib.lib()
+    # everything that can be refused is, before anything is queued
+    T = codec.check_output(out, L, H, D, fmt)
     # launches: containers that share a table length (and the delta grouping), side by side
     launches = {}
     for item in items:
@@ -141,6 +144,8 @@ def decode(items, out, fmt):
             raise ValueError("containers of different caches in one call")
         if c.payload_bytes <= 0:
             raise RuntimeError("payload must be a contiguous, non-empty uint8 tensor")
+        if item[3] < 0 or item[3] + c.num_tokens > T:
+            raise RuntimeError("output tensor does not match the encoded geometry")
         launches.setdefault((c.max_bins, c.delta_group), []).append(item)
     # areas: containers, then the index: running sums, the sub-chunks' entries, what the count
     # tables are rebuilt from, levels that are still on the host
@@ -214,23 +219,19 @@ def decode(items, out, fmt):
         buf = _upload(pieces, total, index_at, write_index)
         base = buf.data_ptr() + index_at
         stream = codec._stream(buf.device)
-        verdict = None
-        if counted:
-            # zero unless a kernel stores to it, straight into host memory
-            verdict = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+        # a word that stays zero unless a kernel finds counts that make no table
+        with hostmem.StoredWords(1, torch.int32) if counted else contextlib.nullcontext() as verdict:
             for key, (tables, groups) in counted.items():
                 at = base + groups_at[key]
                 _lib.check(lib.cg_rebuild_tables(buf.data_ptr(), index_at, key[0], groups, C, at + 8 * groups, at + 12 * groups, at,
-                                                 tables.data_ptr(), verdict.data_ptr(), stream))
-            tables_done = torch.cuda.Event()
-            tables_done.record()
-        at = base + subs_at
-        for key, members in launches.items():
-            n = sum(k for c, _, _, _ in members for _, k in c.length_arrays)
-            codec.decode_listed(at, n, key[0], L, H, D, key[1], out, fmt)
-            at += n * _SUB_BYTES
-        if verdict is not None:
-            tables_done.synchronize()                # the tables, not the decode behind them
-            if int(verdict[0]):
+                                                 tables.data_ptr(), verdict.words.data_ptr(), stream))
+            if counted:
+                verdict.stored()
+            at = base + subs_at
+            for key, members in launches.items():
+                n = sum(k for c, _, _, _ in members for _, k in c.length_arrays)
+                codec.decode_listed(at, n, key[0], L, H, D, key[1], out, fmt)
+                at += n * _SUB_BYTES
+            if counted and verdict.read()[0]:        # the tables are waited for, not the decode behind them
                 raise ValueError("wire container: histogram counts do not add up to the chunk's tokens")
     return out

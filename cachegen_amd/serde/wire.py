@@ -366,7 +366,7 @@ def bring_to_host(enc, first_chunk, num_chunks, per_chunk=True, compact=False):
     counts, stored into pinned memory by one kernel) while the tables, whose size it knows, are
     already on the bus, and then for each piece of about _PIECE_BYTES."""
     import torch
-    from .. import _lib, codec
+    from .. import _lib, codec, hostmem
     L, H, D, S, T = enc.num_layers, enc.num_heads, enc.head_size, enc.chunk_tokens, enc.num_tokens
     C = H * D
     rows = 2 * L
@@ -422,29 +422,28 @@ def bring_to_host(enc, first_chunk, num_chunks, per_chunk=True, compact=False):
             if S <= MAX_STREAM_BYTES:
                 dense, nsym, inexact = _device_counts_launch(cdf, tokens)
         nbounds, ngroups = g_last - g_first + 1, 0 if nsym is None else nsym.numel()
-        meta = torch.empty(3 + nbounds + ngroups, dtype=torch.int64, pin_memory=True)
 
         def ptr(t):
             return None if t is None else t.data_ptr()
-        _lib.check(lib.cg_wire_meta(enc.status.data_ptr(), enc.offsets[g_first * rows * C:].data_ptr(), rows * C, nbounds,
-                                    ptr(wide), ptr(inexact), ptr(nsym), ngroups, meta.data_ptr(), stream))
-        sizes_known = mark()
-        chunk_bytes = max(1, cdf[0].numel() * cdf.element_size() + min(spc, lengths.shape[0]) * rows * C * 4)
-        step = max(1, _PIECE_BYTES // chunk_bytes) if per_chunk else 1
-        pieces = [(i, min(i + step, len(groups))) for i in range(0, len(groups), step)]
-        tables_src, lengths_src = cdf, lengths
-        if dense is not None:
-            # ragged count bytes; their places follow from nsym, which is on the device
-            tables_src = torch.empty(dense.numel(), dtype=torch.uint8, device=dev)
-            _lib.check(lib.cg_pack_counts(dense.data_ptr(), dense.shape[2], ngroups, C, nsym.data_ptr(), None,
-                                          tables_src.data_ptr(), stream))
-        elif not compact:
-            a, b = groups[0][0], groups[pieces[0][1] - 1][1]
-            early = {"tables": fetch_tables(cdf[a - c_first:b - c_first]), "lengths": fetch(lengths[subs(a):subs(b)])}
-        maxima = fetch(enc.maxima)
+        with hostmem.StoredWords(3 + nbounds + ngroups, torch.int64) as words:
+            _lib.check(lib.cg_wire_meta(enc.status.data_ptr(), enc.offsets[g_first * rows * C:].data_ptr(), rows * C, nbounds,
+                                        ptr(wide), ptr(inexact), ptr(nsym), ngroups, words.words.data_ptr(), stream))
+            words.stored()
+            chunk_bytes = max(1, cdf[0].numel() * cdf.element_size() + min(spc, lengths.shape[0]) * rows * C * 4)
+            step = max(1, _PIECE_BYTES // chunk_bytes) if per_chunk else 1
+            pieces = [(i, min(i + step, len(groups))) for i in range(0, len(groups), step)]
+            tables_src, lengths_src = cdf, lengths
+            if dense is not None:
+                # ragged count bytes; their places follow from nsym, which is on the device
+                tables_src = torch.empty(dense.numel(), dtype=torch.uint8, device=dev)
+                _lib.check(lib.cg_pack_counts(dense.data_ptr(), dense.shape[2], ngroups, C, nsym.data_ptr(), None,
+                                              tables_src.data_ptr(), stream))
+            elif not compact:
+                a, b = groups[0][0], groups[pieces[0][1] - 1][1]
+                early = {"tables": fetch_tables(cdf[a - c_first:b - c_first]), "lengths": fetch(lengths[subs(a):subs(b)])}
+            maxima = fetch(enc.maxima)
+            meta = words.read()
 
-    sizes_known.synchronize()
-    meta = meta.tolist()
     enc.raise_for_status(meta[0])
     bounds = meta[3:3 + nbounds]
     symbols = starts = None                              # starts: byte offset of every chunk's counts in tables_src

@@ -1,0 +1,70 @@
+"""What the containers' readers and writers do with the calls they were not tuned for: outputs they
+cannot write, levels of any type and stride, levels that a program changes, and errors between a launch
+and the host's look at what it stored."""
+import types
+
+import pytest
+import torch
+
+from cachegen_amd import hostmem
+from cachegen_amd.serde import incoming
+
+DEV = "cuda:0"
+
+
+@pytest.fixture
+def order(monkeypatch):
+    """Stands in for the stream and for pinned memory where there is no GPU; lists what happens."""
+    seen = []
+    event = types.SimpleNamespace(synchronize=lambda: seen.append("event waited for"))
+    stream = types.SimpleNamespace(synchronize=lambda: seen.append("stream waited for"), record_event=lambda: event)
+    zeros = torch.zeros
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: stream)
+    monkeypatch.setattr(torch, "zeros", lambda *a, pin_memory=False, **kw: zeros(*a, **kw))
+    return seen
+
+
+@pytest.mark.parametrize("launched", [False, True])
+def test_words_that_kernels_store_to_are_held_until_the_launches_are_through(order, launched):
+    with pytest.raises(KeyError):
+        with hostmem.StoredWords(2, torch.int64) as words:
+            if launched:
+                words.stored()
+            raise KeyError
+    assert order == ["event waited for" if launched else "stream waited for"]
+    with hostmem.StoredWords(2, torch.int64) as words:
+        words.stored()
+        assert words.read() == [0, 0]
+
+
+@pytest.mark.parametrize("out,tokens", [(torch.zeros(2, 2, 300, 2, 8), 0), (torch.zeros(2, 2, 300, 2, 9).half(), 0),
+                                        (torch.zeros(3, 2, 300, 2, 8).half(), 0), (torch.zeros(2, 2, 299, 2, 8).half(), 0),
+                                        (torch.zeros(2, 2, 300, 2, 8).half(), 1), (torch.zeros(2, 2, 300, 2, 8).half(), -1),
+                                        (torch.zeros(2, 2, 300, 2, 16).half()[..., ::2], 0)])
+def test_outputs_that_cannot_be_written_are_refused_before_anything_is_queued(out, tokens, monkeypatch):
+    monkeypatch.setattr(incoming, "_upload", lambda *a: pytest.fail("something was queued"))
+    container = incoming.Container(2, 300, 2, 8, 256, 32, 0, False, False)
+    container.payload_bytes = 1
+    bins = torch.full((2,), 32.0)
+    with pytest.raises(RuntimeError, match="output tensor does not match|must be contiguous"):
+        incoming.decode([(container, bins, bins, tokens)], out, "vllm")
+
+
+@pytest.mark.gpu
+def test_counts_that_make_no_table_are_refused_and_leave_the_reader_usable():
+    from cachegen_amd.kvgen import make_kv
+    from cachegen_amd.config import LMCacheEngineConfig, LMCacheEngineMetadata
+    from cachegen_amd.serde import CreateSerde, wire
+    s, d = CreateSerde("cachegen-compact", LMCacheEngineConfig.from_defaults(chunk_size=256),
+                       LMCacheEngineMetadata("lmsys/longchat-7b-16k", 1, 0, "vllm"))
+    blob = s.to_bytes(make_kv(32, 256, 2, 64, seed=3, device=DEV))
+    want = d.from_bytes(blob)
+    at = wire.read_header(blob)["geometry"]["cdf"][0] + 64 + 7          # a count: 64 rows' symbol counts come first
+    bad = bytearray(blob)
+    bad[at] = (bad[at] + 1) % 200
+    with pytest.raises(ValueError, match="add up"):
+        d.from_bytes(bytes(bad))
+    assert torch.equal(d.from_bytes(blob), want)
+    with pytest.raises(RuntimeError, match="output tensor does not match"):
+        d.from_bytes_into(blob, torch.empty(want.shape, device=DEV))
+    assert torch.equal(d.from_bytes(blob), want)
