@@ -38,6 +38,7 @@ SIGNATURES = {
     "cg_encode_kv_levels": (_INT, [_P, _INT, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _INT, _P, _P, _P, _I64,
                                    _P, _P, _P, _P, _P, _P, _P, _P, _SZ, _P]),
     "cg_collect_bytes": (_INT, [_P, _I64, _I64, _I64, _P, _I64, _I64, _P, _I64, _P]),
+    "cg_collect_sizes": (_INT, [_P, _I64, _I64, _I64, _P, _P]),
     "cg_scan_workspace": (_SZ, [_I64]),
     "cg_scan_lengths": (_INT, [_P, _I64, _P, _P, _SZ, _P]),
     "cg_scan_lengths_static": (_INT, [_P, _I64, _P, _P]),

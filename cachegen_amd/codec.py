@@ -13,7 +13,7 @@ from typing import Optional
 
 import torch
 
-from . import _lib
+from . import _lib, hostmem
 
 MAX_TOKENS_PER_STREAM = 256
 _DT = {torch.float16: _lib.DT_F16, torch.bfloat16: _lib.DT_BF16}
@@ -190,6 +190,8 @@ def encode_kv(kv, key_bins, value_bins, chunk_tokens=None, fmt="vllm", max_bins=
 
 def scan_lengths(lengths):
     """int32 lengths (any shape) -> int64 [n+1] exclusive running sum on the GPU."""
+    if lengths.dtype != torch.int32 or not lengths.is_cuda:
+        raise RuntimeError("stream lengths should be int32 on a GPU, got %s on %s" % (lengths.dtype, lengths.device))
     flat = lengths.contiguous().view(-1)
     n = flat.numel()
     lib = _lib.lib()
@@ -202,17 +204,40 @@ def scan_lengths(lengths):
 
 
 def collect_streams(padded, offsets):
-    """uint8 streams of a padded buffer [nl, nc, cap], back to back; offsets: scan_lengths of their
-    lengths."""
-    nl, nc, cap = padded.shape
-    total = int(offsets[-1].item())
-    out = torch.empty(total, dtype=torch.uint8, device=padded.device)
-    if total:
-        if padded.stride(2) != 1:
-            padded = padded.contiguous()
-        with torch.cuda.device(padded.device):
-            _lib.check(_lib.lib().cg_collect_bytes(padded.data_ptr(), cap, padded.stride(0), padded.stride(1), offsets.data_ptr(),
-                                                   nl, nc, out.data_ptr(), total, _stream(padded.device)))
+    """The streams of a padded buffer [..., cap] (3-dimensional ones are read in place), back to back;
+    offsets: scan_lengths of their lengths, in the order of the buffer's slots.  Lengths of fewer
+    streams than the buffer has slots are those of its first ones.  A stream that does not fit its
+    slot, or has none, is a RuntimeError."""
+    dev, cap = padded.device, padded.shape[-1]
+    if offsets.dtype != torch.int64 or offsets.dim() != 1 or offsets.numel() < 2 or not offsets.is_contiguous():
+        raise RuntimeError("offsets must be a contiguous int64 vector of one entry more than there are streams")
+    if not padded.is_cuda or offsets.device != dev:
+        raise RuntimeError("padded streams and offsets should be on the same GPU, got %s and %s" % (dev, offsets.device))
+    if padded.numel() == 0:
+        raise RuntimeError("padded streams: the buffer has no slots")
+    if padded.dim() != 3:
+        padded = padded.reshape(1, -1, cap)
+    nl, nc, _ = padded.shape
+    n, nslots = offsets.numel() - 1, nl * nc
+    with torch.cuda.device(dev):
+        lib, stream = _lib.lib(), _stream(dev)
+        with hostmem.StoredWords(2, torch.int64) as words:
+            _lib.check(lib.cg_collect_sizes(offsets.data_ptr(), n, nslots, cap, words.words.data_ptr(), stream))
+            words.stored()
+            total, unfit = words.read()
+        if unfit:
+            raise RuntimeError("padded streams: %d lengths do not fit %d slots of %d values" % (n, nslots, cap))
+        out = torch.empty(total, dtype=padded.dtype, device=dev)
+        if total:
+            if n < nslots:
+                offsets = torch.cat([offsets, offsets[-1:].expand(nslots - n)])
+            if padded.stride(2) != 1:
+                padded = padded.contiguous()
+            size = padded.element_size()
+            if size > 1:                                 # the kernel moves bytes
+                offsets = offsets * size
+            _lib.check(lib.cg_collect_bytes(padded.data_ptr(), cap * size, padded.stride(0) * size, padded.stride(1) * size,
+                                            offsets.data_ptr(), nl, nc, out.data_ptr(), total * size, stream))
     return out
 
 

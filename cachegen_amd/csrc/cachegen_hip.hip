@@ -227,6 +227,15 @@ int cg_collect_bytes(const uint8_t *padded, int64_t cap, int64_t p0, int64_t p1,
     return check_launch("collect_bytes");
 }
 
+int cg_collect_sizes(const int64_t *offsets, int64_t n, int64_t nslots, int64_t cap, int64_t *out, void *stream)
+{
+    if (!offsets || !out) return fail(CG_ERR_ARG, "collect_sizes: null pointer");
+    const int64_t nblocks = ceil_div(n, 256);
+    if (n <= 0 || nslots <= 0 || cap <= 0 || nblocks > INT_MAX) return fail(CG_ERR_ARG, "collect_sizes: bad count");
+    collect_sizes_kernel<<<dim3((unsigned)nblocks), dim3(256), 0, static_cast<hipStream_t>(stream)>>>(offsets, n, nslots, cap, out);
+    return check_launch("collect_sizes");
+}
+
 size_t cg_scan_workspace(int64_t n) { return align_up((size_t)(ceil_div(n > 0 ? n : 1, kScanTile) + 1) * sizeof(int64_t), 256); }
 
 int cg_scan_lengths(const int32_t *lengths, int64_t n, int64_t *offsets, void *scratch,

@@ -336,6 +336,22 @@ __global__ __launch_bounds__(256) void collect_bytes_kernel(
     }
 }
 
+// What the host has to know before it makes room for those streams, stored straight into pinned
+// memory (no copy, no second launch that reduces): out[0] = their bytes; out[1], zero before the
+// launch, is set where the offsets do not begin at 0, a stream is longer than its slot, or a stream
+// that is not empty has no slot among the buffer's nslots.  One load a thread, bound by its launch and
+// the host's wait, which takes the place of reading the total back: with the check the four functions
+// on one sub-chunk (2 layers, 512 channels) take 168 us, without it 166.
+__global__ __launch_bounds__(256) void collect_sizes_kernel(
+    const int64_t *__restrict__ offsets, int64_t n, int64_t nslots, int64_t cap, int64_t *out)
+{
+    const int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (g >= n) return;
+    const int64_t at = offsets[g], size = offsets[g + 1] - at;
+    if (g == n - 1) out[0] = at + size;
+    if ((g == 0 && at != 0) || size < 0 || size > (g < nslots ? cap : 0)) out[1] = 1;      // everybody who writes writes the same
+}
+
 __global__ void clear_status_kernel(int32_t *status) { *status = 0; }
 
 }  // namespace

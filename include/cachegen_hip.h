@@ -209,9 +209,17 @@ int cg_encode_kv_levels(const void *kv, int kv_dt, int64_t L, int64_t T, int64_t
 /* collect_bytes (encoder.py:209-222): the streams of a padded buffer, back to back.
  * padded   device uint8 [nl, nc, cap], strides (p0, p1, 1)
  * offsets  device int64 [nl*nc + 1]: exclusive running sum of the lengths (cg_scan_lengths)
- * out      device uint8 [out_bytes], written; nothing is written past it */
+ * out      device uint8 [out_bytes], written; nothing is written past it
+ * The lengths have to fit the slots: cg_collect_sizes says whether they do. */
 int cg_collect_bytes(const uint8_t *padded, int64_t cap, int64_t p0, int64_t p1, const int64_t *offsets,
                      int64_t nl, int64_t nc, uint8_t *out, int64_t out_bytes, void *stream);
+
+/* Looks n streams over before cg_collect_bytes: offsets device int64 [n + 1], nslots and cap the
+ * padded buffer's slots and their size.
+ * out  int64 [2] that the GPU can write, pinned host memory as a rule; out[0] is written: offsets[n];
+ *      out[1] (zero it first) is set to 1 if offsets[0] is not 0, a stream does not fit its slot, or
+ *      one behind the last slot is not empty */
+int cg_collect_sizes(const int64_t *offsets, int64_t n, int64_t nslots, int64_t cap, int64_t *out, void *stream);
 
 /* Exclusive running sum of stream lengths: offsets[0] = 0, offsets[i+1] =
  * offsets[i] + lengths[i] (the inclusive sums of decoder.py:70 are offsets[1:]).

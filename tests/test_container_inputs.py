@@ -68,3 +68,14 @@ def test_counts_that_make_no_table_are_refused_and_leave_the_reader_usable():
     with pytest.raises(RuntimeError, match="output tensor does not match"):
         d.from_bytes_into(blob, torch.empty(want.shape, device=DEV))
     assert torch.equal(d.from_bytes(blob), want)
+
+
+@pytest.mark.parametrize("offsets,match", [(torch.zeros(5, dtype=torch.int32), "offsets must be"), (torch.zeros((5, 1), dtype=torch.int64), "offsets must be"),
+                                           (torch.zeros(10, dtype=torch.int64)[::2], "offsets must be"), (torch.zeros(1, dtype=torch.int64), "offsets must be"),
+                                           (torch.zeros(5, dtype=torch.int64), "on the same GPU")])
+def test_offsets_that_the_packing_kernel_would_misread_are_refused(offsets, match):
+    from cachegen_amd import codec
+    with pytest.raises(RuntimeError, match=match):
+        codec.collect_streams(torch.zeros((2, 2, 8), dtype=torch.uint8), offsets)
+    with pytest.raises(RuntimeError, match="lengths should be int32"):
+        codec.scan_lengths(offsets)

@@ -47,3 +47,31 @@ def test_payload_places_from_all_tile_counts(nsub, chunk):
     n = a.total_bytes()
     assert n == b.total_bytes() == int(a.lengths.sum())
     assert torch.equal(a.offsets, b.offsets) and torch.equal(a.payload[:n], b.payload[:n]) and torch.equal(a.cdf, b.cdf)
+
+
+@pytest.mark.parametrize("dtype", [torch.uint8, torch.int8, torch.int32])
+@pytest.mark.parametrize("shape", [(40,), (5, 40), (3, 4, 40), (2, 3, 2, 40)])
+def test_padded_buffers_of_any_rank_and_type_are_packed(dtype, shape):
+    """As gathering the streams one by one does it, also with fewer lengths than slots and with empty
+    streams behind the last slot."""
+    from cachegen_amd.serde.cachegen_encoder import collect_bytes
+    rng = np.random.default_rng(len(shape))
+    padded = rng.integers(-100, 100, size=shape).astype(np.int32)
+    slots = padded.reshape(-1, 40)
+    device = torch.from_numpy(padded).to(dtype).to(DEV)
+    for n in {1, len(slots) - 1 or 1, len(slots), len(slots) + 3}:
+        lengths = rng.integers(0, 41, size=n).astype(np.int32)
+        lengths[len(slots):] = 0
+        want = torch.from_numpy(np.concatenate([slots[g, :lengths[g]] for g in range(min(n, len(slots)))])).to(dtype)
+        got = collect_bytes(device, torch.from_numpy(lengths).to(DEV))
+        assert got.dtype == dtype and torch.equal(got.cpu(), want)
+
+
+@pytest.mark.parametrize("lengths", [[8, 9, 8, 8], [8, 8, 8, 300], [0, 0, 0, 0, 1], [8, 8, 8, 8, 0, 2]])
+def test_lengths_that_do_not_fit_the_padded_buffer_are_refused(lengths):
+    from cachegen_amd.serde.cachegen_encoder import collect_bytes
+    padded = torch.zeros((2, 2, 8), dtype=torch.uint8, device=DEV)
+    with pytest.raises(RuntimeError, match="do not fit 4 slots of 8"):
+        collect_bytes(padded, torch.tensor(lengths, dtype=torch.int32, device=DEV))
+    with pytest.raises(RuntimeError, match="do not fit 4 slots of 8"):
+        codec.collect_streams(padded, torch.tensor([1, 2, 3, 4, 5], device=DEV))         # does not begin at 0
