@@ -71,8 +71,14 @@ class LMCacheEngine:
     @staticmethod
     def _tuple_kv_as_view(kv_tensors: KVCache) -> Optional[torch.Tensor]:
         """The same tensor without a copy where the tuple's tensors lie at even distances in one
-        storage (a cache that was allocated, or retrieved, in one piece); None where they do not."""
+        storage (a cache that was allocated, or retrieved, in one piece); None where they do not, and
+        where a compressing backend would refuse the view (a head dimension that is not contiguous)
+        or read it value by value and code it from plain bytes, while the stacked copy's rows of whole
+        16-byte units take the vector path."""
         first = kv_tensors[0][0]
+        size, head = first.element_size(), first.shape[-1]
+        if head > 1 and first.stride(-1) != 1:
+            return None
         storage = first.untyped_storage().data_ptr()
         offsets = []
         for pair in kv_tensors:
@@ -85,6 +91,8 @@ class LMCacheEngine:
         to_layer = offsets[2] - offsets[0] if len(kv_tensors) > 1 else 2 * to_value
         if to_value < 0 or to_layer < 0 or any(offsets[2 * l + j] != offsets[0] + l * to_layer + j * to_value
                                                for l in range(len(kv_tensors)) for j in (0, 1)):
+            return None
+        if head * size % 16 == 0 and (first.data_ptr() % 16 or any(s * size % 16 for s in (to_value, to_layer, *first.stride()[:-1]))):
             return None
         return first.as_strided((len(kv_tensors), 2, *first.shape), (to_layer, to_value, *first.stride()))
 

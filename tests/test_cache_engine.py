@@ -356,3 +356,50 @@ def test_store_reads_caches_of_any_layout():
             again, _ = engine.retrive(tokens, device="cpu")
             check_kv_cache_equal(want, again, T, "vllm")
             whole.copy_(torch.stack([torch.stack(p) for p in want]))
+
+
+def odd_layouts(whole):
+    """name -> (cache, whether a store reads it in place) for whole [L, 2, T, H, D], 16-bit, D a multiple of 8:
+    the same values, where a compressing backend cannot or should not take the view."""
+    L, _, T, H, D = whole.shape
+
+    def tuples(x):
+        return tuple((layer[0], layer[1]) for layer in x)
+    wide = torch.zeros((L, 2, T, H, D + 3), dtype=whole.dtype, device=whole.device)
+    wide[..., :D] = whole
+    late = torch.zeros(whole.numel() + 1, dtype=whole.dtype, device=whole.device)
+    late[1:] = whole.reshape(-1)
+    gapped = torch.zeros((L, 2, T * H * D + 4), dtype=whole.dtype, device=whole.device)
+    gapped[..., :T * H * D] = whole.reshape(L, 2, -1)
+    return {"in one piece": (tuples(whole), True),
+            "layers inside a token": (tuples(whole.permute(2, 0, 1, 3, 4).contiguous().permute(1, 2, 0, 3, 4)), True),
+            "padded heads of whole units": (tuples(torch.cat([whole, whole[..., :8]], dim=-1)[..., :D]), True),
+            "keys transposed": (tuples(whole.transpose(3, 4).contiguous().transpose(3, 4)), False),
+            "padded heads": (tuples(wide[..., :D]), False),
+            "begins at an odd element": (tuples(late[1:].view(whole.shape)), False),
+            "odd distances of layers": (tuples(gapped[..., :T * H * D].view(L, 2, T, H, D)), False)}
+
+
+def test_views_that_a_compressing_store_cannot_take_whole_are_stacked():
+    layouts = odd_layouts(torch.randn(3, 2, 5, 2, 16).half())
+    seen = {name: LMCacheEngine._tuple_kv_as_view(kv) is not None for name, (kv, _) in layouts.items()}
+    assert seen == {name: in_place for name, (_, in_place) in layouts.items()}
+    # heads that no vector load fits are read in place from wherever they lie
+    late = torch.zeros(3 * 2 * 5 * 2 * 7 + 1).half()[1:].view(3, 2, 5, 2, 7)
+    assert LMCacheEngine._tuple_kv_as_view(tuple((layer[0], layer[1]) for layer in late)) is not None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("serde", ["cachegen", "cachegen-compact"])
+def test_gpu_compressing_store_of_caches_of_any_layout(serde):
+    from cachegen_amd.kvgen import make_kv
+    T = 300
+    whole = make_kv(32, T, 2, 64, seed=21, device="cuda:0")
+    tokens, blobs = generate_tokens(T, "cuda"), {}
+    for name, (kv, _) in odd_layouts(whole).items():
+        engine = LMCacheEngine(backend_config("mem", 256, serde), LMCacheEngineMetadata("lmsys/longchat-7b-16k", 1, 0, "vllm"))
+        engine.store(tokens, kv)
+        blobs[name] = [engine.engine_.get_bytes(engine._make_key(h, "vllm")) for h in engine._prefix_hashes(tokens)]
+        assert engine.retrive(tokens, "cuda")[1] == T
+        engine.close()
+    assert all(b == blobs["in one piece"] for b in blobs.values())
