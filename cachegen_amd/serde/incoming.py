@@ -125,9 +125,17 @@ def _transfer(pieces, total, index_at, write_index, device):
     return buf
 
 
+def _levels(bins, num_layers, device):
+    """A bins vector as the kernels and the index take it: float32, dense, on `device`, or on the host
+    if it is there."""
+    if bins.numel() != num_layers:
+        raise RuntimeError("bins vectors must have one entry per layer (%d), got %d" % (num_layers, bins.numel()))
+    return bins.detach().to(device=device if bins.is_cuda else bins.device, dtype=torch.float32).reshape(-1).contiguous()
+
+
 def decode(items, out, fmt):
     """Decodes containers into one tensor.  items: [(Container, key_bins, value_bins, t0)]: levels
-    (float32 [L] tensors on the output's device, or on the CPU: these travel with the index) and
+    (tensors of L values, as `codec.decode_kv` takes them; those on the CPU travel with the index) and
     first output token of each; all containers have the same layers, heads and head size.  out: KV
     tensor in layout `fmt` on the GPU."""
     first = items[0][0]
@@ -147,6 +155,9 @@ def decode(items, out, fmt):
         if item[3] < 0 or item[3] + c.num_tokens > T:
             raise RuntimeError("output tensor does not match the encoded geometry")
         launches.setdefault((c.max_bins, c.delta_group), []).append(item)
+    # levels by their tensors (`items` holds these): one conversion and one place in the index for each
+    levels = {id(t): t for _, kb, vb, _ in items for t in (kb, vb)}
+    levels = {k: _levels(t, L, device) for k, t in levels.items()}
     # areas: containers, then the index: running sums, the sub-chunks' entries, what the count
     # tables are rebuilt from, levels that are still on the host
     pieces, pos, nsubs = [], 0, 0
@@ -171,23 +182,20 @@ def decode(items, out, fmt):
         groups_at[key] = size = _up(size, 64)
         size += groups * 8 + groups * 4 + groups     # starts, tokens, symbols
     levels_at = {}                                   # levels that are still on the host -> offset in the index
-    for _, kb, vb, _ in items:
-        for t in (kb, vb):
-            if t.numel() != L or t.dtype != torch.float32:
-                raise RuntimeError("bins vectors must be float32 with one entry per layer (%d)" % L)
-            if not t.is_cuda and id(t) not in levels_at:
-                levels_at[id(t)] = (_up(size, 64), t)
-                size = _up(size, 64) + 4 * L
+    for k, t in levels.items():
+        if not t.is_cuda:
+            levels_at[k] = size = _up(size, 64)
+            size += 4 * L
     total = index_at + size
 
     def write_index(base, host):
         raw = host.numpy()
         index = base + index_at
-        for at, t in levels_at.values():
-            raw[at:at + 4 * L].view(np.float32)[:] = t.numpy()
+        for k, at in levels_at.items():
+            raw[at:at + 4 * L].view(np.float32)[:] = levels[k].numpy()
 
-        def levels(t):
-            return t.data_ptr() if t.is_cuda else index + levels_at[id(t)][0]
+        def address(t):
+            return index + levels_at[id(t)] if id(t) in levels_at else levels[id(t)].data_ptr()
         described = bytearray(len(plan) * _ITEM.size)
         arrays, array_subs = [], []
         for i, (key, c, kb, vb, t_out, place, group) in enumerate(plan):
@@ -203,16 +211,16 @@ def decode(items, out, fmt):
                     tokens[0] if len(tokens) == 1 else np.repeat(np.asarray(tokens, dtype=np.int32), rows)
                 raw[at + 12 * groups + group:at + 12 * groups + group + n] = c.symbols
             _ITEM.pack_into(described, i * _ITEM.size, tables, place + base + c.maxima, place + base + c.lengths,
-                            place + base + c.payload, c.payload_bytes, levels(kb), levels(vb), t_out, c.num_tokens, c.chunk_tokens,
+                            place + base + c.payload, c.payload_bytes, address(kb), address(vb), t_out, c.num_tokens, c.chunk_tokens,
                             c.max_bins, _lib.DT_BF16 if c.bf16_maxima else _lib.DT_F16, int(c.lengths_u16), len(c.length_arrays))
             for lengths, n in c.length_arrays:
                 arrays.append(lengths.data_ptr())
                 array_subs.append(n)
         n = len(arrays)
         bad = ctypes.c_int(0)
-        address = host.data_ptr()
+        start = host.data_ptr()
         if lib.cg_host_list((ctypes.c_char * len(described)).from_buffer(described), len(plan), (ctypes.c_void_p * n)(*arrays),
-                            (ctypes.c_int64 * n)(*array_subs), L, C, address, index, address + subs_at, ctypes.byref(bad)) != _lib.CG_OK:
+                            (ctypes.c_int64 * n)(*array_subs), L, C, start, index, start + subs_at, ctypes.byref(bad)) != _lib.CG_OK:
             raise LengthsError("wire container: payload size is not the sum of the stream lengths")
 
     with torch.cuda.device(device):

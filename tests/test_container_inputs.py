@@ -79,3 +79,34 @@ def test_offsets_that_the_packing_kernel_would_misread_are_refused(offsets, matc
         codec.collect_streams(torch.zeros((2, 2, 8), dtype=torch.uint8), offsets)
     with pytest.raises(RuntimeError, match="lengths should be int32"):
         codec.scan_lengths(offsets)
+
+
+FORMS = {"strided": lambda b: torch.stack([b, b + 99], dim=1)[:, 0], "float64": lambda b: b.double(), "int64": lambda b: b.long(),
+         "float16": lambda b: b.half(), "column": lambda b: b[:, None], "grad": lambda b: b.clone().requires_grad_()}
+
+
+@pytest.mark.parametrize("form", sorted(FORMS))
+def test_levels_are_dense_float32_whatever_they_were(form):
+    bins = torch.tensor([32.0, 16.0, 12.0])
+    got = incoming._levels(FORMS[form](bins), 3, torch.device(DEV))
+    assert got.dtype == torch.float32 and got.is_contiguous() and not got.requires_grad and torch.equal(got, bins)
+    assert got.numpy().shape == (3,)
+    with pytest.raises(RuntimeError, match="one entry per layer"):
+        incoming._levels(FORMS[form](bins), 4, torch.device(DEV))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("device", ["cpu", DEV])
+@pytest.mark.parametrize("form", sorted(FORMS))
+def test_containers_take_levels_of_any_type_and_stride(form, device):
+    from cachegen_amd import codec
+    from cachegen_amd.kvgen import make_kv
+    from cachegen_amd.serde import wire
+    kb, vb = torch.tensor([32.0, 16.0, 12.0], device=device), torch.tensor([16.0, 8.0, 32.0], device=device)
+    enc = codec.encode_kv(make_kv(3, 300, 2, 64, seed=5, device=DEV), kb.to(DEV), vb.to(DEV), chunk_tokens=256)
+    want = codec.decode_encoded(enc, FORMS[form](kb), FORMS[form](vb), out_dtype=torch.float16)
+    items, out = [], torch.zeros_like(want)
+    for i, blob in enumerate(wire.pack_chunks(enc, compact=True)):
+        items.append((incoming.Container.flat(blob), FORMS[form](kb), FORMS[form](vb), 256 * i))
+    incoming.decode(items, out, "vllm")
+    assert torch.equal(out.view(torch.int16), want.view(torch.int16))
