@@ -67,8 +67,7 @@ class CacheGenSerializer(Serializer):
         self.fmt = metadata.fmt
         self.key_bins = self.make_key_bins(self.cachegen_config)
         self.value_bins = self.make_value_bins(self.cachegen_config)
-        # table size: known from the configuration, so that no call has to ask the device for it
-        self.max_bins = int(max(CGBasics.make_key_bins(self.cachegen_config).max(), CGBasics.make_value_bins(self.cachegen_config).max()))
+        self._sized = None
 
     def make_key_bins(self, config: CacheGenConfig) -> torch.Tensor:
         return CGBasics.make_key_bins(config).cuda()
@@ -76,17 +75,32 @@ class CacheGenSerializer(Serializer):
     def make_value_bins(self, config: CacheGenConfig) -> torch.Tensor:
         return CGBasics.make_value_bins(config).cuda()
 
+    def _levels(self):
+        """(key bins, value bins, table size) of a call.  The table size is the largest bins value:
+        a read of the device, which waits for everything queued before it, so it is kept together
+        with the two tensors and their write counters, and read again once a program has replaced
+        either tensor or written to it.  (A write that torch does not count, through `.data`, takes
+        effect when the attribute is assigned a new tensor.)"""
+        kb, vb, sized = self.key_bins, self.value_bins, self._sized
+        counted = not (kb.is_inference() or vb.is_inference())       # these have no write counter
+        if not counted or sized is None or sized[0] is not kb or sized[1] is not vb or sized[2] != (kb._version, vb._version):
+            versions = (kb._version, vb._version) if counted else None
+            sized = self._sized = (kb, vb, versions, codec._largest(kb, vb))
+        return kb, vb, sized[3]
+
+    def _encode(self, tensor, chunk_tokens):
+        kb, vb, max_bins = self._levels()
+        return codec.encode_kv(tensor.cuda(), kb, vb, chunk_tokens=chunk_tokens, max_bins=max_bins)
+
     def to_bytes(self, tensor: torch.Tensor) -> bytes:
         """tensor: [num_layers, 2, num_tokens, num_heads, head_size] for fmt "vllm",
         [num_layers, 2, num_heads, num_tokens, head_size] for "huggingface"; any device.
         The huggingface layout is read in place through strides (no permuted copy)."""
         if self.fmt == "huggingface":
             tensor = tensor.permute(0, 1, 3, 2, 4)
-        ntokens = tensor.shape[2]
+        enc = self._encode(tensor, tensor.shape[2])
         if self.wire_format != "pickle":
-            enc = codec.encode_kv(tensor.cuda(), self.key_bins, self.value_bins, chunk_tokens=ntokens, max_bins=self.max_bins)
             return wire.pack_chunks(enc, per_chunk=False, compact=self.wire_format == "compact")[0]
-        enc = codec.encode_kv(tensor.cuda(), self.key_bins, self.value_bins, chunk_tokens=ntokens, max_bins=self.max_bins)
         return self._pickled(enc)[0]
 
     def _pickled(self, enc):
@@ -102,7 +116,7 @@ class CacheGenSerializer(Serializer):
         tensor (not in the reference, whose callers loop over `to_bytes`)."""
         if self.fmt == "huggingface":
             tensor = tensor.permute(0, 1, 3, 2, 4)
-        enc = codec.encode_kv(tensor.cuda(), self.key_bins, self.value_bins, chunk_tokens=chunk_size, max_bins=self.max_bins)
+        enc = self._encode(tensor, chunk_size)
         if self.wire_format != "pickle":
             return wire.pack_chunks(enc, compact=self.wire_format == "compact")
         return self._pickled(enc)

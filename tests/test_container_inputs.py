@@ -110,3 +110,46 @@ def test_containers_take_levels_of_any_type_and_stride(form, device):
         items.append((incoming.Container.flat(blob), FORMS[form](kb), FORMS[form](vb), 256 * i))
     incoming.decode(items, out, "vllm")
     assert torch.equal(out.view(torch.int16), want.view(torch.int16))
+
+
+def test_the_serializers_tables_follow_its_bins(monkeypatch):
+    """The table size is that of the tensors a call codes with: what the hooks returned, what a program
+    put in their place, and what it wrote into them."""
+    from cachegen_amd import codec
+    from cachegen_amd.config import LMCacheEngineConfig, LMCacheEngineMetadata
+    from cachegen_amd.serde import cachegen_basics as basics
+    from cachegen_amd.serde.cachegen_encoder import CacheGenSerializer
+    taken = []
+
+    def encode(kv, key_bins, value_bins, chunk_tokens=None, max_bins=None, **kw):
+        taken.append(max_bins if max_bins is not None else codec._largest(key_bins, value_bins))
+        raise KeyError
+    monkeypatch.setattr(codec, "encode_kv", encode)
+    monkeypatch.setattr(torch.Tensor, "cuda", lambda self: self)
+
+    class Finer(CacheGenSerializer):
+        def make_key_bins(self, config):
+            return basics.make_key_bins(config) * 2
+
+    def size(s):
+        for call in (s.to_bytes, lambda kv: s.to_bytes_chunks(kv, 4)):
+            with pytest.raises(KeyError):
+                call(torch.zeros(32, 2, 8, 1, 8).half())
+        assert taken[-1] == taken[-2]
+        return taken[-1]
+    for wire_format in ("pickle", "flat", "compact"):
+        args = LMCacheEngineConfig.from_defaults(), LMCacheEngineMetadata("lmsys/longchat-7b-16k", 1, 0, "vllm"), wire_format
+        assert size(CacheGenSerializer(*args)) == 32
+        s = Finer(*args)
+        assert size(s) == 64
+        s.value_bins = torch.full((32,), 100.0)
+        assert size(s) == 100
+        s.value_bins[3] = 120
+        assert size(s) == 120
+        s.value_bins.fill_(8)
+        assert size(s) == 64
+        with torch.inference_mode():
+            s.key_bins = torch.full((32,), 16.0)
+            assert size(s) == 16
+            s.key_bins[0] = 20
+        assert size(s) == 20
