@@ -40,6 +40,7 @@
 #include "decoder.hpp"
 #include "scan_compact.hpp"
 #include "launch.hpp"
+#include "host_lengths.hpp"
 #include "tables_wire.hpp"
 
 // ======================================================================================
@@ -641,8 +642,8 @@ int cg_host_tile_starts(const void *lengths, int itemsize, int64_t nsub, int64_t
     if (!lengths || !tile_starts || !sub_bytes) return fail(CG_ERR_ARG, "host_tile_starts: null pointer");
     if (nsub <= 0 || rows <= 0 || C <= 0 || rows > (1 << 24) / C || (itemsize != 2 && itemsize != 4))
         return fail(CG_ERR_ARG, "host_tile_starts: bad shape");
-    const bool fine = itemsize == 2 ? host_tile_starts(static_cast<const uint16_t *>(lengths), nsub, rows, C, tile_starts, sub_bytes)
-                                    : host_tile_starts(static_cast<const int32_t *>(lengths), nsub, rows, C, tile_starts, sub_bytes);
+    const bool fine = itemsize == 2 ? host_tile_starts<uint16_t>(lengths, nsub, rows, C, kStreamCap, tile_starts, sub_bytes)
+                                    : host_tile_starts<int32_t>(lengths, nsub, rows, C, kStreamCap, tile_starts, sub_bytes);
     return fine ? CG_OK : fail(CG_ERR_ARG, "host_tile_starts: negative length");
 }
 

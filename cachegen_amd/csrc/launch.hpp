@@ -514,40 +514,4 @@ int decode_kv_block(int64_t C, int lp)
     return block > 128 ? 128 : block;
 }
 
-// Bytes that streams occupy before every 64th stream of a row, from their lengths in host memory:
-// lengths are min'ed with a stream's capacity; false if one is negative.
-template <typename T>
-bool host_tile_starts(const T *lengths, int64_t nsub, int64_t rows, int64_t C, uint32_t *starts, int64_t *sub_bytes)
-{
-    const int64_t tiles = ceil_div(C, 64);
-    int32_t lowest = 0;
-    for (int64_t s = 0; s < nsub; ++s) {
-        uint32_t run = 0;                       // at most 256 bytes of at most 2^24 streams: checked by the caller
-        for (int64_t r = 0; r < rows; ++r, lengths += C)
-            for (int64_t t = 0; t < tiles; ++t) {
-                *starts++ = run;
-                const int64_t n = C - t * 64 < 64 ? C - t * 64 : 64;
-                const T *p = lengths + t * 64;
-                int32_t sum = 0, low = 0;
-                if (n == 64) {
-                    for (int i = 0; i < 64; ++i) {          // a fixed count: vector instructions
-                        const int32_t v = p[i];
-                        sum += v < kStreamCap ? v : kStreamCap;
-                        low = v < low ? v : low;
-                    }
-                } else {
-                    for (int i = 0; i < n; ++i) {
-                        const int32_t v = p[i];
-                        sum += v < kStreamCap ? v : kStreamCap;
-                        low = v < low ? v : low;
-                    }
-                }
-                run += (uint32_t)sum;
-                lowest = low < lowest ? low : lowest;
-            }
-        sub_bytes[s] = run;
-    }
-    return lowest >= 0;
-}
-
 }  // namespace

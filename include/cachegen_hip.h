@@ -308,7 +308,7 @@ int cg_host_list(const CgHostContainer *items, int n, const void *const *lengths
                  int64_t L, int64_t C, uint32_t *tile_starts, int64_t starts_at, CgListedSub *subs, int *bad);
 
 /* HOST memory, no GPU work: the running sums of stream lengths that cg_decode_listed starts from.
- * lengths      [nsub, rows, C] int32, or uint16 (itemsize 2)
+ * lengths      [nsub, rows, C] int32, or uint16 (itemsize 2), at any byte address
  * tile_starts  uint32 [nsub, rows, ceil(C/64)], written: bytes of the sub-chunk's streams before
  *              stream (row, 64*i), a stream counting min(length, 256) bytes
  * sub_bytes    int64 [nsub], written: bytes of every sub-chunk
