@@ -61,6 +61,25 @@ dim3 stream_grid(const StreamGrid &sg, int64_t nblocks)
         else { constexpr int BS = 64; __VA_ARGS__; }    \
     } while (0)
 
+// Lanes (channels of all rows and chunks, up to a block's width) up to which the tables are counted by
+// four slices of a block (calculate_cdf_kernel).  The slices wait for their loads side by side, which is
+// what a call of few blocks or long chunks is made of; a block of four times the lanes costs more to
+// start and, from 640 blocks of 256 lanes on, leaves a second round of blocks.  Unsliced / sliced, 512 to
+// 4096 channels, 4 to 512 rows, tables of 33 entries, us:
+//   symbols as bytes, chunks of   32 tokens    64 k lanes 10.0 /  9.9   128 k 10.8 / 11.2   160 k 12.2 / 17.3
+//                                 64                      11.4 / 10.4         12.1 / 12.0         13.6 / 18.7
+//                                256                      19.5 / 13.1         22.1 / 17.9         26.6 / 26.9   250 k 29.9 / 32.2
+//                                512                      31.1 / 17.6         39.5 / 26.6         42.4 / 36.8         47.1 / 46.0
+//                               1024                      67.5 / 28.0         69.5 / 42.0         74.2 / 57.0         101.8 / 79.0
+//   packed (whole encode call)   512                       118 /  111          151 /  154          190 /  201
+//                               1500                       219 /  195          366 /  362          440 /  444
+//                               4096                       549 /  473          902 /  878         1099 / 1138
+int64_t sliced_lanes(bool packed, int64_t chunk_tokens)
+{
+    if (packed) return (chunk_tokens >= 1024 ? 128 : 64) << 10;
+    return (chunk_tokens >= 512 ? 256 : chunk_tokens >= 64 ? 128 : 64) << 10;
+}
+
 // key_bins, value_bins (packed symbols only, may be null): the rows of at most 15 symbols hold
 // four bits a symbol.
 int launch_cdf(const uint8_t *sym, const uint32_t *sym4, int64_t nsub, int64_t rows, int64_t T,
@@ -92,9 +111,7 @@ int launch_cdf(const uint8_t *sym, const uint32_t *sym4, int64_t nsub, int64_t r
     if (nblocks <= 0 || nblocks > INT_MAX) return fail(CG_ERR_ARG, "calculate_cdf: grid out of range");
     const size_t shmem = sym4 ? (size_t)(max_bins + 1) * (block + 2) * sizeof(uint16_t)
                               : (size_t)(max_bins + 1) * (block + 1) * sizeof(uint32_t);     // TableStride
-    // four blocks of 256 lanes per compute unit hide the loads of one another; below that the
-    // block's own slices do (see the kernel)
-    const bool sliced = nblocks * block < 1024 * 256;
+    const bool sliced = nblocks * block <= sliced_lanes(sym4 != nullptr, S < T ? S : T);
     const dim3 grid((unsigned)nblocks), blk(sliced ? block * 4 : block);
     if (sliced) {
         if (sym4) CG_DISPATCH_BS(block, (calculate_cdf_kernel<BS, true, 4><<<grid, blk, shmem, stream>>>(a)));
@@ -431,8 +448,12 @@ void launch_decode_log2(const DecodeArgs &a, dim3 grid, size_t shmem, hipStream_
 // Whether a decode of these wavefronts is bound by one stream's dependent chain (decode_few_kernel,
 // blocks of 64): up to kFewWavefronts a SIMD, tables of 16, 32 or 64 symbols.  Measured with 32
 // layers x 1024 channels, decode_streams_kernel / decode_few_kernel: three wavefronts a SIMD (768
-// tokens) 97 / 92 us for tables of 32 symbols, 86 / 83 for 16, 114 / 108 for 64; four (1024 tokens)
-// 101 / 105, 90 / 94, 122 / 127.  Tables of 8 symbols have one LDS search step to save and no
+// tokens) 98 / 91 us for tables of 32 symbols, 86 / 83 for 16, 115 / 109 for 64; four (1024 tokens)
+// 101 / 104, 88 / 94, 123 / 128.  The line is the same at 512, 1536 and 4096 channels and 2, 8 and 80
+// layers: up to three wavefronts the first takes 0.99 to 1.24 times the second's time, from three and
+// a half on 0.89 to 1.02 (tables of 64 from four and a half on 1.00 to 1.05).  With 400 channels, whose
+// last wavefront of a row is a quarter full, the second is still up to 1.1 times as fast at four and
+// five: its blocks are of one wavefront.  Tables of 8 symbols have one LDS search step to save and no
 // instantiation; other lengths search by bisection.
 constexpr int64_t kFewWavefronts = 3;
 bool few_wavefronts(int64_t rows, int64_t nc, int64_t nsub, int lp)

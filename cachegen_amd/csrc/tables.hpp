@@ -235,7 +235,7 @@ struct CdfArgs {
 // tokens into the same columns (the counters are added to atomically anyway).  A call of few blocks is
 // bound by the latency of its loads, one batch after the other down the chunk: four slices wait for a
 // quarter of the batches (512 tokens x 512 channels, two layers: 25.1 -> 15.0 us; 1333 tokens x 1024
-// channels, 32 layers: 62.4 -> 35.4 us).
+// channels, 32 layers: 62.4 -> 35.4 us); where that stops paying: sliced_lanes in launch.hpp.
 template <int BS, bool PACKED, int SLICES>
 __global__ __launch_bounds__(BS * SLICES) void calculate_cdf_kernel(CdfArgs a)
 {

@@ -75,3 +75,21 @@ def test_lengths_that_do_not_fit_the_padded_buffer_are_refused(lengths):
         collect_bytes(padded, torch.tensor(lengths, dtype=torch.int32, device=DEV))
     with pytest.raises(RuntimeError, match="do not fit 4 slots of 8"):
         codec.collect_streams(padded, torch.tensor([1, 2, 3, 4, 5], device=DEV))         # does not begin at 0
+
+
+# both sides of the lines of sliced_lanes (launch.hpp): rows of 1024 channels, tokens of a chunk
+@pytest.mark.parametrize("nt,rows", [(63, 64), (63, 65), (64, 128), (64, 129), (511, 128), (511, 129), (512, 256), (512, 257)])
+def test_tables_of_bytes_on_both_sides_of_the_slices_line(oracle, nt, rows):
+    sym = np.random.default_rng(nt).integers(0, 20, size=(rows, nt, 1024), dtype=np.uint8)
+    got = torchac_hip.calculate_cdf(torch.from_numpy(sym.view(np.int8)).to(DEV), 32)
+    assert np.array_equal(got.cpu().numpy().view(np.uint16), oracle.calculate_cdf(sym, 32))
+
+
+@pytest.mark.parametrize("chunk,tokens", [(1023, 2046), (1023, 2047), (1024, 4096), (1024, 4097), (5000, 4097)])
+def test_packed_tables_on_both_sides_of_the_slices_line(chunk, tokens):
+    """16 layers of 1024 channels: two and four chunks are the lines' 64 k and 128 k lanes."""
+    kv = torch.randn(16, 2, tokens, 8, 128, device=DEV, generator=torch.Generator(DEV).manual_seed(tokens)).half()
+    bins = torch.full((16,), 32.0, device=DEV)
+    a, b = (codec.encode_kv(kv, bins, bins, chunk_tokens=chunk, _test_flags=f) for f in (4, 2))      # a pass of their own, the quantizer
+    n = a.total_bytes()
+    assert torch.equal(a.cdf, b.cdf) and n == b.total_bytes() and torch.equal(a.payload[:n], b.payload[:n])
