@@ -215,15 +215,19 @@ def collect_streams(padded, offsets):
         raise RuntimeError("padded streams and offsets should be on the same GPU, got %s and %s" % (dev, offsets.device))
     if padded.numel() == 0:
         raise RuntimeError("padded streams: the buffer has no slots")
-    if padded.dim() != 3:
-        padded = padded.reshape(1, -1, cap)
-    nl, nc, _ = padded.shape
-    n, nslots = offsets.numel() - 1, nl * nc
+    n, nslots = offsets.numel() - 1, padded.numel() // cap
     with torch.cuda.device(dev):
         lib, stream = _lib.lib(), _stream(dev)
         with hostmem.StoredWords(2, torch.int64) as words:
             _lib.check(lib.cg_collect_sizes(offsets.data_ptr(), n, nslots, cap, words.words.data_ptr(), stream))
             words.stored()
+            if padded.dim() != 3:
+                padded = padded.reshape(1, -1, cap)
+            if padded.stride(2) != 1:
+                padded = padded.contiguous()
+            nl, nc, _ = padded.shape
+            p0, p1, _ = padded.stride()
+            size = padded.element_size()                 # the kernel moves bytes
             total, unfit = words.read()
         if unfit:
             raise RuntimeError("padded streams: %d lengths do not fit %d slots of %d values" % (n, nslots, cap))
@@ -231,13 +235,10 @@ def collect_streams(padded, offsets):
         if total:
             if n < nslots:
                 offsets = torch.cat([offsets, offsets[-1:].expand(nslots - n)])
-            if padded.stride(2) != 1:
-                padded = padded.contiguous()
-            size = padded.element_size()
-            if size > 1:                                 # the kernel moves bytes
+            if size > 1:
                 offsets = offsets * size
-            _lib.check(lib.cg_collect_bytes(padded.data_ptr(), cap * size, padded.stride(0) * size, padded.stride(1) * size,
-                                            offsets.data_ptr(), nl, nc, out.data_ptr(), total * size, stream))
+            _lib.check(lib.cg_collect_bytes(padded.data_ptr(), cap * size, p0 * size, p1 * size, offsets.data_ptr(), nl, nc,
+                                            out.data_ptr(), total * size, stream))
     return out
 
 

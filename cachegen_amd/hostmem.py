@@ -70,20 +70,26 @@ class StoredWords:
     def __init__(self, n: int, dtype: torch.dtype):
         self.words = torch.zeros(n, dtype=dtype, pin_memory=True)
         self._stream = torch.cuda.current_stream()
-        self._stored = None
+        self._stored, self._through = None, False
 
     def __enter__(self):
         return self
 
     def stored(self):
         """Everything that stores to the words has been launched: `read` waits for that, and not for
-        what is launched afterwards."""
+        what is launched afterwards.  (To be left out where nothing is: the event costs a few
+        microseconds.)"""
         self._stored = self._stream.record_event()
 
+    def _wait(self):
+        (self._stored or self._stream).synchronize()
+        self._through = True
+
     def read(self):
-        """The words as a list, once the launches before `stored` are through."""
-        self._stored.synchronize()
+        """The words as a list, once the launches that store to them are through."""
+        self._wait()
         return self.words.tolist()
 
     def __exit__(self, *exc):
-        (self._stored or self._stream).synchronize()
+        if not self._through:
+            self._wait()
