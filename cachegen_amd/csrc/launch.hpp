@@ -71,12 +71,13 @@ dim3 stream_grid(const StreamGrid &sg, int64_t nblocks)
 //                                256                      19.5 / 13.1         22.1 / 17.9         26.6 / 26.9   250 k 29.9 / 32.2
 //                                512                      31.1 / 17.6         39.5 / 26.6         42.4 / 36.8         47.1 / 46.0
 //                               1024                      67.5 / 28.0         69.5 / 42.0         74.2 / 57.0         101.8 / 79.0
-//   packed (whole encode call)   512                       118 /  111          151 /  154          190 /  201
-//                               1500                       219 /  195          366 /  362          440 /  444
-//                               4096                       549 /  473          902 /  878         1099 / 1138
+// Packed symbols, whole encode call, tables of 17 / 33 / 65 entries: with slices a chunk of 300 tokens takes
+// 1.02 / 1.03 / 1.05 times as long at 72 k to 128 k lanes and 1.08 / 1.08 / 1.1 at 160 k, one of 512 tokens
+// 1.00 / 1.01 / 1.02 and 1.06, one of 700 tokens 0.985 / 0.985 / 1.02 and 1.05, one of 1000 to 1500 0.98 /
+// 0.98 / 1.02 and 1.04; at 64 k lanes and below less time throughout (1500 tokens 0.89, 512 tokens 0.94).
 int64_t sliced_lanes(bool packed, int64_t chunk_tokens)
 {
-    if (packed) return (chunk_tokens >= 1024 ? 128 : 64) << 10;
+    if (packed) return (chunk_tokens >= 640 ? 128 : 64) << 10;
     return (chunk_tokens >= 512 ? 256 : chunk_tokens >= 64 ? 128 : 64) << 10;
 }
 
