@@ -3,10 +3,11 @@
 The reference ships a chunk as a pickle of `CacheGenGPUEncoderOutput` holding GPU tensors
 (LMCache/lmcache/storage_backend/serde/cachegen_basics.py:110-122): one device-to-host copy
 per tensor when it is written, code execution from the blob when it is read.  This container
-carries the same fields in one flat, versioned, little-endian buffer, so that a chunk is one
-device-to-host copy out of a staging buffer and one host-to-device copy back, and reading it
-executes nothing.  `CacheGenDeserializer.from_bytes` accepts both forms (it looks at the
-first four bytes); the pickle form stays the default for drop-in use.
+carries the same fields in one flat, versioned, little-endian buffer.  To write it, the encoder's
+tensors go to pinned memory as they are, and the blob is put together on the host; to read it, the
+blob goes to the GPU whole and is decoded from there (`incoming`), and reading it executes nothing.
+`CacheGenDeserializer.from_bytes` accepts both forms (it looks at the first four bytes); the pickle
+form stays the default for drop-in use.
 
 Layout (every section starts on a 64-byte boundary; the gaps are zero):
 
@@ -16,8 +17,9 @@ Layout (every section starts on a 64-byte boundary; the gaps are zero):
     lengths  int32  [nsub, 2L, C]       bytes of every stream, in stream order
     payload  uint8  [payload_bytes]     all streams back to back
 
-Stream offsets are not stored: they are the running sum of `lengths`, which the decoder
-recomputes on the GPU exactly as cachegen_decoder.py:70 does.  A stream longer than 256
+Stream offsets are not stored: they are the running sum of `lengths` (cachegen_decoder.py:70 adds
+it up on the GPU; the reader here does so on the host, where it checks it against the payload's
+size, and sends every 64th along with the blob).  A stream longer than 256
 bytes is stored cut to 256 (its length field keeps the full value), as in the device format.
 
 Version 2 ("compact") stores the same information in fewer bytes, for chunks of at most 256
@@ -279,7 +281,7 @@ def unpack_host(blob):
 
 
 # --------------------------------------------------------------------------- #
-# device form: one staging buffer, one copy over PCIe per direction
+# device form: out of the encoder's tensors
 # --------------------------------------------------------------------------- #
 def _device_counts_launch(cdf, tokens):
     """Device form of tables_to_counts for cdf int16 [nchunks, 2L, C, Lp]: launches the conversion
@@ -551,8 +553,8 @@ def unpack_to_device(blob, device):
     """-> (header dict, cdf, maxima, lengths, payload) on the device, which the blob reached in a
     single copy from pinned host memory: views of that buffer where the stored form is the
     tensor itself, rebuilt tensors where it is not (version 2).  The stream lengths are checked
-    against the payload size on the host.  (The deserializer and the engine decode blobs without
-    these tensors: incoming.py.)"""
+    against the payload size on the host.  For programs that want the sections themselves: the
+    deserializer and the engine decode blobs without these tensors (incoming.py)."""
     import torch
     h = read_header(blob)
     geo = h["geometry"]
