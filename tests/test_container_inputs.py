@@ -153,3 +153,26 @@ def test_the_serializers_tables_follow_its_bins(monkeypatch):
             assert size(s) == 16
             s.key_bins[0] = 20
         assert size(s) == 20
+
+
+@pytest.mark.gpu
+def test_an_error_behind_a_launch_that_stores_to_the_host_is_waited_out(monkeypatch):
+    """Writer and reader of compact containers, with something failing between the launch and the read."""
+    import dataclasses
+    from cachegen_amd import codec
+    from cachegen_amd.kvgen import make_kv
+    from cachegen_amd.serde import wire
+    waited = []
+    wait = hostmem.StoredWords._wait
+    monkeypatch.setattr(hostmem.StoredWords, "_wait", lambda self: (waited.append(self.words.numel()), wait(self)))
+    bins = torch.tensor([32.0, 16.0])
+    enc = codec.encode_kv(make_kv(2, 256, 2, 64, seed=3, device=DEV), bins, bins)
+    blob = wire.pack_chunks(enc, compact=True)[0]
+    assert waited == [3 + 2 + 4]                             # status, wide, inexact, two boundaries, four rows' symbols
+    with pytest.raises(AttributeError):
+        wire.pack_chunks(dataclasses.replace(enc, maxima=types.SimpleNamespace(dtype=torch.float16)))
+    assert waited == [9, 3 + 2]
+    monkeypatch.setattr(codec, "decode_listed", lambda *a: {}["launch failed"])
+    with pytest.raises(KeyError):
+        incoming.decode([(incoming.Container.flat(blob), bins, bins, 0)], torch.empty((2, 2, 256, 2, 64), dtype=torch.float16, device=DEV), "vllm")
+    assert waited == [9, 5, 1]
