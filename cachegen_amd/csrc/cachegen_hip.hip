@@ -24,6 +24,7 @@
 #include <cstring>
 #include <atomic>
 #include <mutex>
+#include <type_traits>
 
 #include "cachegen_hip.h"
 

@@ -140,6 +140,7 @@ constexpr int kBufferWord3 = 0x00020000;
 
 // Pointers into LDS, for loads with immediate offsets.
 typedef __attribute__((address_space(3))) const uint16_t lds_u16;
+typedef __attribute__((address_space(3))) const uint32_t lds_u32;
 typedef __attribute__((address_space(3))) const float lds_f32;
 typedef __attribute__((address_space(3))) const char lds_char;
 
@@ -153,17 +154,6 @@ __device__ __forceinline__ void lds_entries_high(lds_char *p, uint32_t &lo, uint
     asm volatile("ds_read_u16_d16_hi %0, %2\n\tds_read_u16_d16_hi %1, %2 offset:%3\n\ts_waitcnt lgkmcnt(0)"
                  : "+v"(lo), "+v"(hi)
                  : "v"(p), "n"(ROW));
-}
-
-// The five entries from p on, one row apart, in one round trip (the compiler sinks a load that it
-// needs last behind the wait for the others).
-template <int ROW>
-__device__ __forceinline__ void lds_five_entries(lds_char *p, uint32_t &e0, uint32_t &e1, uint32_t &e2, uint32_t &e3, uint32_t &e4)
-{
-    asm volatile("ds_read_u16 %0, %5\n\tds_read_u16 %1, %5 offset:%6\n\tds_read_u16 %2, %5 offset:%7\n\t"
-                 "ds_read_u16 %3, %5 offset:%8\n\tds_read_u16 %4, %5 offset:%9\n\ts_waitcnt lgkmcnt(0)"
-                 : "=&v"(e0), "=&v"(e1), "=&v"(e2), "=&v"(e3), "=&v"(e4)
-                 : "v"(p), "n"(ROW), "n"(2 * ROW), "n"(3 * ROW), "n"(4 * ROW));
 }
 
 }  // namespace

@@ -114,6 +114,20 @@ struct BitReader {
             nextw = raw();
         }
     }
+
+    // The same without a branch (a lane whose window is full enough loads its next word again).
+    __device__ __forceinline__ void top_up_flat()
+    {
+        const uint32_t step = (int32_t)spare <= 32 - (int)kSymbolBits ? 32u : 0u;
+        const uint32_t w = step ? __builtin_bswap32(nextw) : 0u;
+        win |= ((uint64_t)w << 32) >> ((spare + kSymbolBits) & 63u);
+        spare += step;
+        pos += step >> 3;
+        nextw = __builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)(pos - 4u), 0, 0);
+    }
+
+    // Bits left in the window; negative where shift_in() has moved more out of it than it held.
+    __device__ __forceinline__ int bits_left() const { return (int)(spare + kSymbolBits); }
 };
 
 enum { SRC_OFFSETS = 0, SRC_PREFIX = 1, SRC_PADDED = 2, SRC_LISTED = 3 };
@@ -176,7 +190,6 @@ struct DecodeLane {
     // the entries the first two probes of the unrolled search look at (one for the first, one
     // of two for the second), read once per stream: two LDS round trips less per symbol
     uint32_t probe1, probe2_lo, probe2_hi;
-    uint32_t held[16];         // FEW: every fourth entry of the part of the table that is searched (entry 0 unused)
     // the decoded symbol's two table entries, each shifted left by 16: only ever written by
     // loads into the upper half, so that the lower halves stay zero
     uint32_t bound_lo, bound_hi;
@@ -193,24 +206,10 @@ struct DecodeLane {
 // Distance of the unrolled search's first probe from entry 0, in entries.
 __host__ __device__ constexpr int first_probe(int log2, int skip) { return log2 >= 2 ? ((1 << log2) >> 1) >> skip : 0; }
 
-// A launch of few wavefronts (FEW) is as long as one stream's dependent chain: a SIMD with one to
-// three wavefronts has issue slots to spare, and an LDS round trip costs a lane some 120 cycles per
-// search step.  There the search holds every fourth entry in registers, halving them by selects
-// until four candidates are left, reads those and the next one in ONE round trip and picks both
-// bounds from them; a symbol's quotient and output follow after the interval's update, off the chain.
-// More instructions (about 50 instead of 35 to 39), so from four wavefronts a SIMD on the plain search
-// is faster (few_wavefronts in launch.hpp).  One chunk of 256 tokens x 1024 channels x 32 layers, one
-// wavefront a SIMD: tables of 32 symbols 93 -> 72 us, of 16 82 -> 68, of 64 107 -> 83 (the shorter step
-// count included).
-template <int LOG2, int SKIP>
-struct FewSearch {
-    static constexpr int kHeld = LOG2 - SKIP >= 3 ? (1 << (LOG2 - SKIP - 2)) : 0;   // four candidates per held entry
-};
-
 // One symbol.  SKIP: how many of the search's first probes are left out because the row's
 // alphabet fits the lower 2^(LOG2-SKIP) entries.  SAFE: the last table entry may be decoded
 // (its upper bound 2^16 is substituted, dec_new.cu:278) and values may be NaN.
-template <int BS, int LOG2, int OUT, int SKIP, bool SAFE, bool FEW>
+template <int BS, int LOG2, int OUT, int SKIP, bool SAFE>
 __device__ __forceinline__ void decode_symbol(const DecodeArgs &a, DecodeLane &s, int lp, int nsteps,
                                               float rm, int i)
 {
@@ -225,47 +224,20 @@ __device__ __forceinline__ void decode_symbol(const DecodeArgs &a, DecodeLane &s
     if (LOG2 >= 2) {
         // largest m with T(m) <= off, probed with the lower bound sh * c <= T(c), which can
         // only overshoot
-        if constexpr (FEW) {
-            constexpr int kHeld = FewSearch<LOG2, SKIP>::kHeld;
-            uint32_t left[kHeld];
-#pragma unroll
-            for (int k = 1; k < kHeld; ++k) left[k] = s.held[k];
-#pragma unroll
-            for (int half = kHeld >> 1; half >= 1; half >>= 1) {
-                const bool up = mul24(sh, left[half]) <= s.off;
-                p = up ? p + half * 4 * kRow : p;
-#pragma unroll
-                for (int k = 1; k < half; ++k) {
-                    // both values first: a choice between two places becomes an indexed access
-                    const uint32_t below = left[k], above = left[half + k];
-                    left[k] = up ? above : below;
-                }
-            }
-            // entry p + 4 exists: the table has 2^LOG2 + 1 entries
-            uint32_t c0, c1, c2, c3, c4;
-            lds_five_entries<kRow>(p, c0, c1, c2, c3, c4);
-            const bool up1 = mul24(sh, c1) <= s.off, up2 = mul24(sh, c2) <= s.off, up3 = mul24(sh, c3) <= s.off;
-            p += up2 ? (up3 ? 3 * kRow : 2 * kRow) : (up1 ? kRow : 0);
-            s.bound_lo = (up2 ? (up3 ? c3 : c2) : (up1 ? c1 : c0)) << 16;
-            s.bound_hi = (up2 ? (up3 ? c4 : c3) : (up1 ? c2 : c1)) << 16;
-            // volatile: issued here, not joined with the rare path's load behind the update
-            if (OUT != OUT_SYMBOLS) q = *(volatile lds_f32 *)(p + s.lutoff);
-        } else {
-            // the first two probes compare entries held in registers
-            const bool up1 = mul24(sh, s.probe1) <= s.off;
-            p = up1 ? p + kStep1 * kRow : p;
-            if (kStep2 >= 1) {
-                const uint32_t c2 = up1 ? s.probe2_hi : s.probe2_lo;
-                p = (mul24(sh, c2) <= s.off) ? p + kStep2 * kRow : p;
-            }
-#pragma unroll
-            for (int step = kStep2 >> 1; step >= 1; step >>= 1)
-                p = (mul24(sh, lds_entry(p, step * kRow)) <= s.off) ? p + step * kRow : p;
-            // both bounds and the quotient in one round trip (entry lp - 1 exists, so the upper
-            // bound of the last symbol can be read and then replaced)
-            if (OUT != OUT_SYMBOLS) q = *(lds_f32 *)(p + s.lutoff);
-            lds_entries_high<kRow>(p, s.bound_lo, s.bound_hi);
+        // the first two probes compare entries held in registers
+        const bool up1 = mul24(sh, s.probe1) <= s.off;
+        p = up1 ? p + kStep1 * kRow : p;
+        if (kStep2 >= 1) {
+            const uint32_t c2 = up1 ? s.probe2_hi : s.probe2_lo;
+            p = (mul24(sh, c2) <= s.off) ? p + kStep2 * kRow : p;
         }
+#pragma unroll
+        for (int step = kStep2 >> 1; step >= 1; step >>= 1)
+            p = (mul24(sh, lds_entry(p, step * kRow)) <= s.off) ? p + step * kRow : p;
+        // both bounds and the quotient in one round trip (entry lp - 1 exists, so the upper
+        // bound of the last symbol can be read and then replaced)
+        if (OUT != OUT_SYMBOLS) q = *(lds_f32 *)(p + s.lutoff);
+        lds_entries_high<kRow>(p, s.bound_lo, s.bound_hi);
         // T(c) = (span * c) >> 16 = high word of span * (c << 16) for c < 2^16; the one entry
         // that is 2^16, the upper bound of the last symbol (dec_new.cu:278), gives the span
         t_lo = __umulhi(s.span, s.bound_lo);
@@ -345,7 +317,7 @@ __device__ __forceinline__ void decode_symbol(const DecodeArgs &a, DecodeLane &s
             __builtin_amdgcn_raw_buffer_store_b16((short)bits, s.orsrc, (int)s.ovoff, (int)((uint32_t)i * (uint32_t)a.ot * 2u), 0);
         }
     };
-    if (!FEW) put_out();
+    put_out();
     s.low += t_lo;
     s.off = rel;
     const uint32_t d = width - 1u;
@@ -359,10 +331,6 @@ __device__ __forceinline__ void decode_symbol(const DecodeArgs &a, DecodeLane &s
     s.low = (uint32_t)(interval >> 32);
     s.span = (uint32_t)interval;
     s.off = s.rd.shift_in(s.off, n);
-    if (FEW) {
-        asm volatile("" : "+v"(q) : "v"(s.off), "v"(s.span));       // not before the update
-        put_out();
-    }
 }
 
 // last_round: the block is one of the launch's last, after which nothing takes the place of a
@@ -373,7 +341,7 @@ __device__ __forceinline__ void decode_symbol(const DecodeArgs &a, DecodeLane &s
 // the most advanced wavefronts first and leaves the least advanced for the end; these blocks
 // raise their wavefronts' priority by the work they have left instead, so that the wavefronts of
 // a SIMD finish closer together.
-template <int BS, int LOG2, int OUT, int SKIP, bool SAFE, bool FEW>
+template <int BS, int LOG2, int OUT, int SKIP, bool SAFE>
 __device__ __forceinline__ void decode_lane(const DecodeArgs &a, DecodeLane &s, int lp, int n, lds_f32 *rmp, bool last_round)
 {
     int nsteps = 0;
@@ -387,10 +355,6 @@ __device__ __forceinline__ void decode_lane(const DecodeArgs &a, DecodeLane &s, 
         s.probe2_hi = lds_entry(s.colp, (kStep1 + kStep2) * kRow);
         s.bound_lo = 0;
         s.bound_hi = 0;
-        if constexpr (FEW) {
-#pragma unroll
-            for (int k = 1; k < FewSearch<LOG2, SKIP>::kHeld; ++k) s.held[k] = lds_entry(s.colp, 4 * k * kRow);
-        }
     }
     // the window is topped up at the head of every group of kGroup symbols and, inside a
     // group, only when a symbol has left it short of bits
@@ -412,23 +376,179 @@ __device__ __forceinline__ void decode_lane(const DecodeArgs &a, DecodeLane &s, 
         for (int j = 0; j < kGroup; ++j) {
             if (j == 0) s.rd.top_up();
             else if (__builtin_expect(s.rd.short_of_bits, 0)) s.rd.top_up();
-            decode_symbol<BS, LOG2, OUT, SKIP, SAFE, FEW>(a, s, lp, nsteps, rm[j], i0 + j);
+            decode_symbol<BS, LOG2, OUT, SKIP, SAFE>(a, s, lp, nsteps, rm[j], i0 + j);
         }
     }
     // what is left of a sub-chunk whose tokens are no multiple of the group
 #pragma unroll 1
     for (; i0 < n; ++i0, ++rmp) {
         s.rd.top_up();
-        decode_symbol<BS, LOG2, OUT, SKIP, SAFE, FEW>(a, s, lp, nsteps, OUT != OUT_SYMBOLS ? *rmp : 0.0f, i0);
+        decode_symbol<BS, LOG2, OUT, SKIP, SAFE>(a, s, lp, nsteps, OUT != OUT_SYMBOLS ? *rmp : 0.0f, i0);
+    }
+}
+
+// ---- calls of few wavefronts ---------------------------------------------------------
+// Such a call lasts as long as one stream's chain of symbols.  A wavefront alone on its SIMD issues an
+// instruction every 5 cycles and waits 54 for an LDS round trip, but 35 to 45 at every branch on a mask
+// that a vector instruction made (all measured).  decode_lane takes two such branches a symbol (its one
+// test, bits that run out) and four or five round trips; here
+//   - the search compares exact products, so nothing is tested: it holds every fourth entry of the
+//     table's part that the row uses, halves them by selects until four candidates are left, and
+//     reads those and the next one, from a table of 32-bit entries, in one round trip;
+//   - four symbols are decoded between two looks at what can go wrong: a lane that ran out of bits
+//     (33 for four symbols) or met the full range makes the wavefront decode the four again, one
+//     by one, with a top-up before each;
+//   - the window is topped up without a branch.
+// 256 tokens x 1024 channels x 32 layers, one wavefront a SIMD, the whole call, against a form that kept
+// those branches (and decode_streams_kernel): tables of 32 symbols 74 -> 49 us (93), of 16 69 -> 45 (82),
+// of 64 84 -> 55 (107).  Where it stops paying: few_wavefronts in launch.hpp.
+template <int LOG2, int SKIP>
+struct FewSearch {
+    static constexpr int kSteps = LOG2 - SKIP - 2;           // search steps on held entries, every fourth of the part
+    static constexpr int kHeld = 1 << kSteps;
+};
+
+struct FewLane {
+    BitReader rd;
+    uint32_t off, low, span;
+    lds_char *col;             // this lane's entry 0: entry e << 16 in the word at e * 256 bytes
+    lds_char *quots;           // (symbol - C) / C
+    uint32_t held[16];
+    uint8_t *osym;
+    __amdgpu_buffer_rsrc_t orsrc;       // as in DecodeLane
+    uint32_t ovoff;
+    float anchor;
+    int phase;
+};
+
+// 2 * m + bit in one instruction
+__device__ __forceinline__ uint32_t twice_plus(uint32_t m, bool bit)
+{
+    const uint64_t carry = __builtin_amdgcn_ballot_w64(bit);
+    uint64_t unused;
+    uint32_t r;
+    asm("v_addc_co_u32 %0, %1, %2, %2, %3" : "=v"(r), "=&s"(unused) : "v"(m), "s"(carry));
+    return r;
+}
+
+// One symbol.  EXACT: the interval may be the full range, whose T(c) is c << 16.  row_offset: of the
+// token's row in the output (dequantised output only).
+template <int LOG2, int OUT, int SKIP, bool SAFE, bool EXACT>
+__device__ __forceinline__ void decode_few_symbol(const DecodeArgs &a, FewLane &s, float rm, int i, uint32_t row_offset)
+{
+    typedef FewSearch<LOG2, SKIP> Search;
+    auto scaled = [&](uint32_t e) { return EXACT && s.span == 0 ? e : __umulhi(s.span, e); };
+    uint32_t left[Search::kHeld], m = 0;
+#pragma unroll
+    for (int k = 1; k < Search::kHeld; ++k) left[k] = s.held[k];
+#pragma unroll
+    for (int h = Search::kHeld >> 1; h >= 1; h >>= 1) {
+        const bool up = scaled(left[h]) <= s.off;
+        m = h == Search::kHeld >> 1 ? (up ? 1u : 0u) : twice_plus(m, up);
+#pragma unroll
+        for (int k = 1; k < h; ++k) {
+            // both values first: a choice between two places becomes an indexed access
+            const uint32_t below = left[k], above = left[h + k];
+            left[k] = up ? above : below;
+        }
+    }
+    // entry p + 4 exists: the table has 2^LOG2 + 1 entries
+    const lds_u32 *p = (lds_u32 *)(s.col + (m << 10));
+    const uint32_t c0 = p[0], c1 = p[64], c2 = p[128], c3 = p[192], c4 = p[256];
+    const uint32_t t0 = scaled(c0), t2 = scaled(c2), t4 = scaled(c4);
+    const bool up2 = t2 <= s.off;
+    const uint32_t t = scaled(up2 ? c3 : c1);
+    const bool up = t <= s.off;
+    const uint32_t outer_lo = up2 ? t2 : t0, outer_hi = up2 ? t4 : t2;
+    const uint32_t t_lo = up ? t : outer_lo;
+    uint32_t t_hi = up ? outer_hi : t;
+    m = twice_plus(twice_plus(m, up2), up);
+    // the last symbol's upper bound is 2^16 (dec_new.cu:278)
+    if (SAFE && m == (1u << LOG2) - 1u) t_hi = s.span;
+    float q = 0.0f;
+    if (OUT != OUT_SYMBOLS) q = *(lds_f32 *)(s.quots + 4 * m);
+    s.low += t_lo;
+    s.off -= t_lo;
+    const uint32_t width = t_hi - t_lo, d = width - 1u;
+    const int n = step_count(s.low, s.low + d, d);
+    const uint64_t interval = (((uint64_t)s.low << 32) | width) << n;       // as in decode_symbol
+    s.low = (uint32_t)(interval >> 32);
+    s.span = (uint32_t)interval;
+    const uint64_t pair = (((uint64_t)s.off << 32) | (uint32_t)(s.rd.win >> 32)) << n;
+    s.off = (uint32_t)(pair >> 32);
+    asm("" : "+v"(s.off));             // or it is compared as the 64-bit value it was shifted in
+    s.rd.win <<= n;
+    s.rd.spare -= (uint32_t)n;
+    if (OUT == OUT_SYMBOLS) {
+        s.osym[(int64_t)i * a.o1] = (uint8_t)m;
+    } else {
+        float v = __fmul_rn(q, rm);
+        asm volatile("" : "+v"(v));                      // two roundings, as in decode_symbol
+        if (SAFE && a.delta_group > 0) {                 // uniform over the block
+            if (s.phase == 0) s.anchor = v;
+            else v = __fadd_rn(v, s.anchor);
+            s.phase = s.phase + 1 == a.delta_group ? 0 : s.phase + 1;
+        }
+        uint32_t bits;
+        if (OUT == OUT_BF16) bits = float_to_bf16_bits_hw(v);
+        else bits = float_to_f16_bits(v);
+        __builtin_amdgcn_raw_buffer_store_b16((short)bits, s.orsrc, (int)s.ovoff, (int)row_offset, 0);
+    }
+}
+
+template <int LOG2, int OUT, int SKIP, bool SAFE>
+__device__ __forceinline__ void decode_few_lane(const DecodeArgs &a, FewLane &s, int n, lds_f32 *rmp)
+{
+#pragma unroll
+    for (int k = 1; k < FewSearch<LOG2, SKIP>::kHeld; ++k) s.held[k] = ((lds_u32 *)s.col)[4 * k * 64];
+    const uint32_t row = (uint32_t)a.ot * 2u;
+    int i = 0;
+#pragma unroll 1
+    for (; i + 4 <= n; i += 4) {
+        const uint32_t at = (uint32_t)i * row;
+        s.rd.top_up_flat();
+        const uint32_t off = s.off, low = s.low, span = s.span, spare = s.rd.spare;
+        const uint64_t win = s.rd.win;
+        const float anchor = s.anchor;
+        const int phase = s.phase;
+        float rm[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) rm[j] = OUT != OUT_SYMBOLS ? rmp[i + j] : 0.0f;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) decode_few_symbol<LOG2, OUT, SKIP, SAFE, false>(a, s, rm[j], i + j, at + (uint32_t)j * row);
+        // the full range (span 0) stays it in these steps: both bounds of every symbol are 0
+        const int good = s.span ? s.rd.bits_left() : -1;
+        if (__builtin_expect(__ballot(good < 0) != 0, 0)) {
+            s.off = off;
+            s.low = low;
+            s.span = span;
+            s.rd.spare = spare;
+            s.rd.win = win;
+            s.anchor = anchor;
+            s.phase = phase;
+#pragma unroll 1
+            for (int j = i; j < i + 4; ++j) {
+                s.rd.top_up_flat();
+                if (s.span == 0) s.low = 0;
+                decode_few_symbol<LOG2, OUT, SKIP, SAFE, true>(a, s, OUT != OUT_SYMBOLS ? rmp[j] : 0.0f, j, (uint32_t)j * row);
+            }
+        }
+    }
+#pragma unroll 1
+    for (; i < n; ++i) {
+        s.rd.top_up_flat();
+        if (s.span == 0) s.low = 0;
+        decode_few_symbol<LOG2, OUT, SKIP, SAFE, true>(a, s, OUT != OUT_SYMBOLS ? rmp[i] : 0.0f, i, (uint32_t)i * row);
     }
 }
 
 // LOG2 >= 0: the table has exactly 2^LOG2 symbols (lp = 2^LOG2 + 1) and the search is
 // unrolled with immediate LDS offsets; LOG2 < 0: any lp.
+// FEW: decode_few_kernel's tables, 32-bit entries in rows of one word a lane, and the quotients behind the row maxima.
 template <int BS, int LOG2, int SRC, int OUT, bool FEW>
 __device__ __forceinline__ void decode_streams(const DecodeArgs &a, uint32_t *smem)
 {
-    constexpr int kRow = DecodeLayout<BS, OUT>::kRow;
+    constexpr int kRow = FEW ? 4 * BS : DecodeLayout<BS, OUT>::kRow;
     const int tid = threadIdx.x;
     StreamId id;
     // SRC_LISTED: the sub-chunks of a launch come from several containers, each with its own tables,
@@ -449,6 +569,7 @@ __device__ __forceinline__ void decode_streams(const DecodeArgs &a, uint32_t *sm
     const int lp = LOG2 >= 0 ? (1 << LOG2) + 1 : a.lp;
     char *rows = reinterpret_cast<char *>(smem);
     float *rowmax = reinterpret_cast<float *>(rows + lp * kRow);     // one per token of the sub-chunk
+    float *few_quots = rowmax + kSub;                                // FEW: one per table entry
     {
         // Every lane copies its own table (lp consecutive 16-bit entries) into its LDS column:
         // loads and LDS writes with immediate offsets, no address arithmetic per entry; the
@@ -457,9 +578,13 @@ __device__ __forceinline__ void decode_streams(const DecodeArgs &a, uint32_t *sm
         // it is stored as 0 whatever the input holds so that the walk back always ends.
         const uint16_t *tables = SRC == SRC_LISTED ? reinterpret_cast<const uint16_t *>(d.cdf) : a.cdf;
         const uint16_t *mine = tables + ((id.chunk * a.sg.rows + id.row) * a.sg.nc + id.ch) * lp;
-        char *column = rows + 2 * tid;
+        char *column = rows + (FEW ? 4 : 2) * tid;
+        auto put = [&](int e, uint16_t v) {
+            if (FEW) *reinterpret_cast<uint32_t *>(column + e * kRow) = (uint32_t)v << 16;
+            else *reinterpret_cast<uint16_t *>(column + e * kRow) = v;
+        };
         if (id.active) {
-            *reinterpret_cast<uint16_t *>(column) = 0;
+            put(0, 0);
             constexpr int kBatch = 16;      // loads in flight per lane
             if (LOG2 >= 0) {
 #pragma unroll
@@ -470,7 +595,7 @@ __device__ __forceinline__ void decode_streams(const DecodeArgs &a, uint32_t *sm
                         if (e0 + j < lp) v[j] = mine[e0 + j];
 #pragma unroll
                     for (int j = 0; j < kBatch; ++j)
-                        if (e0 + j < lp) *reinterpret_cast<uint16_t *>(column + (e0 + j) * kRow) = v[j];
+                        if (e0 + j < lp) put(e0 + j, v[j]);
                 }
             } else {
                 for (int e0 = 1; e0 < lp; e0 += kBatch) {
@@ -479,7 +604,7 @@ __device__ __forceinline__ void decode_streams(const DecodeArgs &a, uint32_t *sm
                     for (int j = 0; j < kBatch; ++j) v[j] = e0 + j < lp ? mine[e0 + j] : (uint16_t)0;
 #pragma unroll
                     for (int j = 0; j < kBatch; ++j)
-                        if (e0 + j < lp) *reinterpret_cast<uint16_t *>(column + (e0 + j) * kRow) = v[j];
+                        if (e0 + j < lp) put(e0 + j, v[j]);
                 }
             }
         }
@@ -495,7 +620,7 @@ __device__ __forceinline__ void decode_streams(const DecodeArgs &a, uint32_t *sm
         const float cq = floorf(bins * 0.5f) - 1.0f;
         nsym = (cq >= 0.0f && cq < 32768.0f) ? 2 * (int)cq + 1 : lp;
         for (int i = tid; i < lp; i += BS)
-            *reinterpret_cast<float *>(rows + i * kRow + DecodeLayout<BS, OUT>::kQuot) =
+            *(FEW ? few_quots + i : reinterpret_cast<float *>(rows + i * kRow + DecodeLayout<BS, OUT>::kQuot)) =
                 __fdiv_rn(__fsub_rn((float)i, cq), cq);
         const uint16_t *mx = SRC == SRC_LISTED ? static_cast<const uint16_t *>(d.maxima) + id.row * d.maxima_pitch
                                                : a.maxima + id.row * a.sg.g.T + id.t0;
@@ -539,13 +664,18 @@ __device__ __forceinline__ void decode_streams(const DecodeArgs &a, uint32_t *sm
     }
     if (!id.active) return;
 
-    DecodeLane s;
+    typename std::conditional<FEW, FewLane, DecodeLane>::type s;
     if (SRC == SRC_LISTED) s.off = s.rd.start(d.bytes, d.last_word, begin, lowest);
     else s.off = s.rd.start(a.bytes, a.last_word, begin + a.bytes_skew, lowest + a.bytes_skew);
     s.low = 0;
     s.span = 0;                        // span modulo 2^32: 0 is the full range (see RangeEncoder)
-    s.colp = (lds_char *)(rows + 2 * tid);
-    s.lutoff = DecodeLayout<BS, OUT>::kQuot - 2 * tid;
+    if constexpr (FEW) {
+        s.col = (lds_char *)(rows + 4 * tid);
+        s.quots = (lds_char *)few_quots;
+    } else {
+        s.colp = (lds_char *)(rows + 2 * tid);
+        s.lutoff = DecodeLayout<BS, OUT>::kQuot - 2 * tid;
+    }
     s.osym = nullptr;
     s.ovoff = 0;
     s.anchor = 0.0f;
@@ -565,10 +695,17 @@ __device__ __forceinline__ void decode_streams(const DecodeArgs &a, uint32_t *sm
 
     // all three conditions are uniform over the block
     const bool safe = OUT == OUT_SYMBOLS || LOG2 < 0 || special || a.delta_group > 0 || nsym > lp - 2;
-    const bool last_round = linear_block() >= a.last_round_first;
-    if (safe) decode_lane<BS, LOG2, OUT, 0, true, FEW>(a, s, lp, id.n, rmp, last_round);
-    else if (LOG2 > 1 && nsym <= (1 << (LOG2 > 1 ? LOG2 - 1 : 0))) decode_lane<BS, LOG2, OUT, 1, false, FEW>(a, s, lp, id.n, rmp, last_round);
-    else decode_lane<BS, LOG2, OUT, 0, false, FEW>(a, s, lp, id.n, rmp, last_round);
+    const bool half = LOG2 > 1 && nsym <= (1 << (LOG2 > 1 ? LOG2 - 1 : 0));
+    if constexpr (FEW) {
+        if (safe) decode_few_lane<LOG2, OUT, 0, true>(a, s, id.n, rmp);
+        else if (half) decode_few_lane<LOG2, OUT, 1, false>(a, s, id.n, rmp);
+        else decode_few_lane<LOG2, OUT, 0, false>(a, s, id.n, rmp);
+    } else {
+        const bool last_round = linear_block() >= a.last_round_first;
+        if (safe) decode_lane<BS, LOG2, OUT, 0, true>(a, s, lp, id.n, rmp, last_round);
+        else if (half) decode_lane<BS, LOG2, OUT, 1, false>(a, s, lp, id.n, rmp, last_round);
+        else decode_lane<BS, LOG2, OUT, 0, false>(a, s, lp, id.n, rmp, last_round);
+    }
 }
 
 template <int BS, int LOG2, int SRC, int OUT>
@@ -578,7 +715,7 @@ __global__ __launch_bounds__(BS) void decode_streams_kernel(DecodeArgs a)
     decode_streams<BS, LOG2, SRC, OUT, false>(a, smem);
 }
 
-// One wavefront a block, so that few wavefronts spread over the compute units (see FewSearch).
+// One wavefront a block, so that few wavefronts spread over the compute units (see decode_few_symbol).
 template <int LOG2, int SRC, int OUT>
 __global__ __launch_bounds__(64) void decode_few_kernel(DecodeArgs a)
 {

@@ -430,6 +430,8 @@ int set_byte_window(DecodeArgs &a, const uint8_t *bytes, int64_t nbytes, const c
     return CG_OK;
 }
 
+size_t decode_few_shmem(int lp) { return (size_t)lp * 64 * sizeof(uint32_t) + (size_t)(kSub + lp) * sizeof(float); }
+
 size_t decode_shmem(int lp, int block) { return align_up((size_t)lp * block * sizeof(uint16_t), 4) + (size_t)(lp + kSub) * sizeof(float); }
 
 // Tables of 2^k symbols (lp = 2^k + 1) take the kernel with the unrolled search.
@@ -446,21 +448,19 @@ void launch_decode_log2(const DecodeArgs &a, dim3 grid, size_t shmem, hipStream_
     }
 }
 
-// Whether a decode of these wavefronts is bound by one stream's dependent chain (decode_few_kernel,
-// blocks of 64): up to kFewWavefronts a SIMD, tables of 16, 32 or 64 symbols.  Measured with 32
-// layers x 1024 channels, decode_streams_kernel / decode_few_kernel: three wavefronts a SIMD (768
-// tokens) 98 / 91 us for tables of 32 symbols, 86 / 83 for 16, 115 / 109 for 64; four (1024 tokens)
-// 101 / 104, 88 / 94, 123 / 128.  The line is the same at 512, 1536 and 4096 channels and 2, 8 and 80
-// layers: up to three wavefronts the first takes 0.99 to 1.24 times the second's time, from three and
-// a half on 0.89 to 1.02 (tables of 64 from four and a half on 1.00 to 1.05).  With 400 channels, whose
-// last wavefront of a row is a quarter full, the second is still up to 1.1 times as fast at four and
-// five: its blocks are of one wavefront.  Tables of 8 symbols have one LDS search step to save and no
-// instantiation; other lengths search by bisection.
-constexpr int64_t kFewWavefronts = 3;
+// Whether a decode of these wavefronts is bound by one stream's chain of symbols (decode_few_kernel,
+// blocks of 64): tables of 16 and 32 symbols up to three wavefronts a SIMD, of 64 up to two (its tables
+// of 32-bit entries take 18 KB of LDS a block, so a third round of blocks would wait for the first).  Measured
+// with 32 layers x 1024 channels, decode_streams_kernel / decode_few_kernel, us, one wavefront a SIMD (256
+// tokens), two, three, four, five:
+//   tables of 32 symbols   93 / 49    - / 62    92 / 78   100 / 99   115 / 139
+//   of 16                  82 / 45               84 / 71    89 / 88   102 / 101
+//   of 64                 107 / 55    - / 75   110 / 129  122 / 163
+// Tables of 8 symbols have no instantiation; other lengths search by bisection.
+int64_t few_wavefronts_a_simd(int lp) { return lp == 17 || lp == 33 ? 3 : lp == 65 ? 2 : 0; }
 bool few_wavefronts(int64_t rows, int64_t nc, int64_t nsub, int lp)
 {
-    if (lp != 17 && lp != 33 && lp != 65) return false;
-    const int64_t most = (int64_t)compute_units() * 4 * kFewWavefronts;
+    const int64_t most = (int64_t)compute_units() * 4 * few_wavefronts_a_simd(lp);
     const int64_t tiles = ceil_div(nc, 64);
     return rows <= most && tiles <= most && nsub <= most && rows * tiles <= most && rows * tiles * nsub <= most;
 }
@@ -479,7 +479,7 @@ template <int SRC>
 int launch_decode_symbols(const DecodeArgs &a, int64_t nblocks, int block, bool few, hipStream_t stream)
 {
     const dim3 grid = stream_grid(a.sg, nblocks);
-    const size_t shmem = decode_shmem(a.lp, block);
+    const size_t shmem = few ? decode_few_shmem(a.lp) : decode_shmem(a.lp, block);
     if (few) launch_decode_few<SRC, OUT_SYMBOLS>(a, grid, shmem, stream);
     else CG_DISPATCH_BS(block, (launch_decode_log2<BS, SRC, OUT_SYMBOLS>(a, grid, shmem, stream)));
     return check_launch("decode");
@@ -489,7 +489,7 @@ int launch_decode_symbols(const DecodeArgs &a, int64_t nblocks, int block, bool 
 template <int SRC>
 int launch_decode_kv(DecodeArgs &a, int64_t nblocks, int block, bool few, int out_dt, hipStream_t stream)
 {
-    const size_t shmem = decode_shmem(a.lp, block);
+    const size_t shmem = few ? decode_few_shmem(a.lp) : decode_shmem(a.lp, block);
     const dim3 grid = stream_grid(a.sg, nblocks);
     // the blocks that are resident together at the launch's end (32 wavefronts per compute unit
     // where registers and LDS allow it, which they do for tables of up to 33 entries)
