@@ -38,6 +38,7 @@
 #include "tables.hpp"
 #include "quantize_tables.hpp"
 #include "encoder.hpp"
+#include "encoder_few.hpp"
 #include "decoder.hpp"
 #include "scan_compact.hpp"
 #include "launch.hpp"
@@ -143,12 +144,15 @@ int cg_encode_fast_new(const int16_t *cdf, int lp, const int8_t *sym, int64_t nl
     // nt == 0 still writes the two closing bits of every stream
     if (int rc = make_grid(nl, nc, nt ? nt : 1, nt ? nt : 1, 1, block, a.sg, nblocks)) return rc;
     if (nt == 0) a.sg.g.T = 0;
-    const size_t shmem = (size_t)lp * (block + 2) * sizeof(uint16_t);      // TableStride<BS>::k16 per entry
     const bool aligned = aligned_to(out, 4) && o0 % 4 == 0 && o1 % 4 == 0;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    const dim3 grid = stream_grid(a.sg, nblocks), blk(block);
-    if (aligned) CG_DISPATCH_BS(block, (encode_streams_kernel<BS, true, false, false, false><<<grid, blk, shmem, st>>>(a)));
-    else CG_DISPATCH_BS(block, (encode_streams_kernel<BS, false, false, false, false><<<grid, blk, shmem, st>>>(a)));
+    const dim3 grid = stream_grid(a.sg, nblocks);
+    if (aligned) {
+        const bool few = few_encode(nblocks, block, kFewEncodeBytes);
+        CG_DISPATCH_BS(block, return (launch_encode<BS, true, false, false, false>(a, grid, few, st)));
+    }
+    const size_t shmem = (size_t)lp * (block + 2) * sizeof(uint16_t);      // TableStride<BS>::k16 per entry
+    CG_DISPATCH_BS(block, (encode_streams_kernel<BS, false, false, false, false><<<grid, dim3(block), shmem, st>>>(a)));
     return check_launch("encode");
 }
 
@@ -341,10 +345,10 @@ struct LevelOut {
 // maxima, max_dt: the row maxima (packed symbols only); nibbles: the quantizer packed the rows
 // of at most 15 symbols four bits a symbol (see narrow_alphabet).
 // tables_ready: the tables were written by an earlier launch of the call (quantize_tables_kernel),
-// which also set the workspace's group sums to zero.
+// which also set the workspace's group sums to zero.  may_be_few: false keeps encode_few_kernel out.
 int code_and_compact(const LevelOut &o, const uint32_t *sym4, const uint8_t *sym_bytes, const EncodeWorkspace &w,
                      int64_t L, int64_t T, int64_t C, int64_t chunk_tokens, hipStream_t s,
-                     const void *maxima = nullptr, int max_dt = 0, bool nibbles = false, bool tables_ready = false)
+                     const void *maxima = nullptr, int max_dt = 0, bool nibbles = false, bool tables_ready = false, bool may_be_few = true)
 {
     const int64_t rows = 2 * L;
     const int lp = o.max_bins + 1;
@@ -365,8 +369,7 @@ int code_and_compact(const LevelOut &o, const uint32_t *sym4, const uint8_t *sym
     a.L = L;
     int64_t nblocks;
     if (int rc = make_grid(rows, C, T, chunk_tokens, w.nsub, block, a.sg, nblocks)) return rc;
-    const size_t shmem = (size_t)lp * (block + 2) * sizeof(uint16_t);      // TableStride<BS>::k16 per entry
-    const dim3 grid = stream_grid(a.sg, nblocks), blk(block);
+    const dim3 grid = stream_grid(a.sg, nblocks);
     // when every encoder block is exactly one tile of the scratch, the blocks leave their byte
     // counts behind and the compaction computes the stream offsets itself
     const bool fused_scan = block == kSlotTile && C % kSlotTile == 0;
@@ -383,19 +386,21 @@ int code_and_compact(const LevelOut &o, const uint32_t *sym4, const uint8_t *sym
         a.nibbles = nibbles ? 1 : 0;
         a.maxima = static_cast<const uint16_t *>(maxima);
         a.max_dt = max_dt;
-        if (tables_ready) {
-            if (fused_scan) encode_streams_kernel<kSlotTile, true, true, false, true, true><<<grid, blk, shmem, s>>>(a);
-            else CG_DISPATCH_BS(block, (encode_streams_kernel<BS, true, true, false, true><<<grid, blk, shmem, s>>>(a)));
-        } else if (chunk_tokens <= kSub) {
+        const bool few = may_be_few && few_encode(nblocks, block, kFewEncodePacked);
+        int rc = CG_OK;
+        if (!tables_ready && chunk_tokens <= kSub) {
             // one sub-chunk per chunk: the encoder builds the tables itself
-            if (fused_scan) encode_streams_kernel<kSlotTile, true, true, true, true, true><<<grid, blk, shmem, s>>>(a);
-            else CG_DISPATCH_BS(block, (encode_streams_kernel<BS, true, true, true, true><<<grid, blk, shmem, s>>>(a)));
+            if (fused_scan) rc = launch_encode<kSlotTile, true, true, true, true, true>(a, grid, few, s);
+            else CG_DISPATCH_BS(block, rc = (launch_encode<BS, true, true, true, true>(a, grid, few, s)));
         } else {
-            if (int rc = launch_cdf(nullptr, sym4, w.nsub, rows, T, C, 0, 0, 0, o.max_bins, chunk_tokens, tables, s,
-                                    nibbles ? o.key_bins : nullptr, nibbles ? o.value_bins : nullptr)) return rc;
-            if (fused_scan) encode_streams_kernel<kSlotTile, true, true, false, true, true><<<grid, blk, shmem, s>>>(a);
-            else CG_DISPATCH_BS(block, (encode_streams_kernel<BS, true, true, false, true><<<grid, blk, shmem, s>>>(a)));
+            if (!tables_ready)
+                rc = launch_cdf(nullptr, sym4, w.nsub, rows, T, C, 0, 0, 0, o.max_bins, chunk_tokens, tables, s,
+                                nibbles ? o.key_bins : nullptr, nibbles ? o.value_bins : nullptr);
+            if (rc) return rc;
+            if (fused_scan) rc = launch_encode<kSlotTile, true, true, false, true, true>(a, grid, few, s);
+            else CG_DISPATCH_BS(block, rc = (launch_encode<BS, true, true, false, true>(a, grid, few, s)));
         }
+        if (rc) return rc;
     } else {
         // any shape or alignment: byte symbols [2L, T, C]
         if (int rc = launch_cdf(sym_bytes, nullptr, 0, rows, T, C, T * C, C, 1, o.max_bins, chunk_tokens, tables, s)) return rc;
@@ -403,9 +408,10 @@ int code_and_compact(const LevelOut &o, const uint32_t *sym4, const uint8_t *sym
         a.s0 = T * C;
         a.s1 = C;
         a.s2 = 1;
-        CG_DISPATCH_BS(block, (encode_streams_kernel<BS, true, false, false, true><<<grid, blk, shmem, s>>>(a)));
+        const size_t shmem = (size_t)lp * (block + 2) * sizeof(uint16_t);      // TableStride<BS>::k16 per entry
+        CG_DISPATCH_BS(block, (encode_streams_kernel<BS, true, false, false, true><<<grid, dim3(block), shmem, s>>>(a)));
+        if (int rc = check_launch("encode_kv")) return rc;
     }
-    if (int rc = check_launch("encode_kv")) return rc;
 
     const int64_t cblocks = ceil_div(w.nstreams, kCompactStreams);
     if (cblocks > INT_MAX) return fail(CG_ERR_ARG, "encode_kv: too many streams");
@@ -448,7 +454,7 @@ int encode_kv(const void *kv, int kv_dt, int64_t L, int64_t T, int64_t H, int64_
               int32_t *lengths, int64_t *offsets, uint8_t *payload, int64_t payload_cap,
               int32_t *status, void *workspace, size_t workspace_bytes, void *stream, int flags)
 {
-    const bool four_bit_words = !(flags & CG_TEST_BYTE_SYMBOLS);
+    const bool four_bit_words = !(flags & CG_TEST_BYTE_SYMBOLS), may_be_few = !(flags & CG_TEST_MANY_WAVEFRONTS);
     if (!kv || !key_bins || !value_bins || !cdf || !maxima || !lengths || !offsets || !payload || !status || !workspace)
         return fail(CG_ERR_ARG, "encode_kv: null pointer");
     if (int rc = check_kv_geometry("encode_kv", kv_dt, L, T, H, D, chunk_tokens)) return rc;
@@ -494,12 +500,12 @@ int encode_kv(const void *kv, int kv_dt, int64_t L, int64_t T, int64_t H, int64_
                                                 reinterpret_cast<uint16_t *>(cdf), w.nsub, chunk_tokens, nibbles, status, shape, s,
                                                 nparts > 1 ? part_tokens : 0, nparts > 1 && part_tokens ? w.scratch : nullptr, slots_bytes,
                                                 w.group_sums)) return rc;
-            return code_and_compact(o, sym4, nullptr, w, L, T, C, chunk_tokens, s, maxima, kv_dt, nibbles, true);
+            return code_and_compact(o, sym4, nullptr, w, L, T, C, chunk_tokens, s, maxima, kv_dt, nibbles, true, may_be_few);
         }
         if (int rc = launch_quantize_pack(kv, kv_dt, L, T, H, D, sl, skv, st, sh, key_bins, value_bins, sym4,
                                           maxima, w.nsub, chunk_tokens, delta_group, s, status, 0, nullptr, nullptr, 0,
                                           nibbles, nullptr, max_bins + 1)) return rc;
-        return code_and_compact(o, sym4, nullptr, w, L, T, C, chunk_tokens, s, maxima, kv_dt, nibbles);
+        return code_and_compact(o, sym4, nullptr, w, L, T, C, chunk_tokens, s, maxima, kv_dt, nibbles, false, may_be_few);
     }
     clear_status_kernel<<<1, 1, 0, s>>>(status);
     if (int rc = launch_quantize(kv, kv_dt, L, T, H, D, sl, skv, st, sh, key_bins, value_bins, w.symbols, maxima, s)) return rc;

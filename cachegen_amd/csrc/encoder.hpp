@@ -343,6 +343,26 @@ __device__ __forceinline__ uint32_t packed_symbol(uint32_t v, int j, uint32_t sm
     return s;
 }
 
+// The bytes that the block's streams occupy in the payload, for the compaction.  Every lane of the block
+// is active where this is called (the host asks for tile sums only when a block is exactly one tile).
+template <int BS>
+__device__ __forceinline__ void leave_tile_sum(const EncodeArgs &a, int tid, int len)
+{
+    __shared__ int32_t wave_sums[BS / 64];
+    int32_t v = len < a.cap ? len : a.cap;
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
+    if ((tid & 63) == 0) wave_sums[tid >> 6] = v;
+    __syncthreads();
+    if (tid == 0) {
+        int32_t total = 0;
+        for (int w = 0; w < BS / 64; ++w) total += wave_sums[w];
+        const uint32_t tile = linear_block();
+        a.tile_sums[tile] = total;                            // at most 256 streams of 256 bytes
+        if (a.group_sums) __hip_atomic_fetch_add(a.group_sums + tile / kTileGroup, total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+}
+
 // PACKED: symbols come from sym4.  FUSE_CDF (PACKED only, one sub-chunk per chunk): the
 // block first builds its own tables from the same words and writes them out.
 // SLOTS: stream g of the launch is written to out[g * cap ...] (the fused path's scratch).
@@ -556,23 +576,7 @@ __global__ __launch_bounds__(BS) void encode_streams_kernel(EncodeArgs a)
     const int len = enc.finish();
     a.lengths[stream] = len;
     if (len > a.cap && a.status) atomicOr(a.status, 1);
-    if (SLOTS && a.tile_sums) {
-        // every lane of the block is active here (the host asks for tile sums only when a block
-        // is exactly one tile): bytes the block's streams occupy in the payload
-        __shared__ int32_t wave_sums[BS / 64];
-        int32_t v = len < a.cap ? len : a.cap;
-#pragma unroll
-        for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
-        if ((tid & 63) == 0) wave_sums[tid >> 6] = v;
-        __syncthreads();
-        if (tid == 0) {
-            int32_t total = 0;
-            for (int w = 0; w < BS / 64; ++w) total += wave_sums[w];
-            const uint32_t tile = linear_block();
-            a.tile_sums[tile] = total;                            // at most 256 streams of 256 bytes
-            if (a.group_sums) __hip_atomic_fetch_add(a.group_sums + tile / kTileGroup, total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-    }
+    if (SLOTS && a.tile_sums) leave_tile_sum<BS>(a, tid, len);
 }
 
 }  // namespace

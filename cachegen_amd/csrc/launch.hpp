@@ -301,10 +301,10 @@ int allow_dynamic_lds(const void *kernel, int bytes, std::atomic<uint64_t> &aske
 {
     if (bytes <= 64 * 1024) return CG_OK;
     int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return fail(CG_ERR_LAUNCH, "quantize_tables: hipGetDevice");
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return fail(CG_ERR_LAUNCH, "dynamic LDS: hipGetDevice");
     if (asked.load(std::memory_order_relaxed) >> dev & 1) return CG_OK;
     const hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-    if (e != hipSuccess) return fail(CG_ERR_LAUNCH, "quantize_tables: hipFuncSetAttribute: %s", hipGetErrorString(e));
+    if (e != hipSuccess) return fail(CG_ERR_LAUNCH, "dynamic LDS: hipFuncSetAttribute: %s", hipGetErrorString(e));
     asked.fetch_or(1ull << dev, std::memory_order_relaxed);
     return CG_OK;
 }
@@ -416,6 +416,39 @@ int compute_units()
         known[dev].store(n, std::memory_order_relaxed);
     }
     return n;
+}
+
+// Whether an encode of these wavefronts is bound by one stream's chain of symbols (encode_few_kernel):
+// up to two a SIMD, which is what the registers for a sub-chunk's symbols leave room for, three where
+// the symbols are bytes (fewer registers).  Measured with 32 layers x 1024 channels, encode_streams_kernel /
+// encode_few_kernel, the whole call, us, one wavefront a SIMD (256 tokens), two, three, four:
+//   tables in the coder or the quantizer      71.5 / 60.8   82.0 / 75.3    98.6 / 105.9  116.3 / 127.0
+//   tables of 65 entries                       86 / 77      103.1 / 101.4
+//   one table, counted by a pass of its own         -        88.1 / 88.4   109.3 / 119.6
+// byte symbols, the reference's four functions on 256 tokens x 1024 channels: 32 layers (one a SIMD) 182 / 166,
+// 50 layers (1.6) 204 / 188, 80 (2.5) 228 / 222.
+bool few_encode(int64_t nblocks, int block, int most)
+{
+    return nblocks <= (int64_t)compute_units() * 4 * most / (block / 64);
+}
+
+constexpr int kFewEncodePacked = 2, kFewEncodeBytes = 3;
+
+template <int BS, bool ALIGNED, bool PACKED, bool FUSE_CDF, bool SLOTS, bool TILE = false>
+int launch_encode(const EncodeArgs &a, dim3 grid, bool few, hipStream_t stream)
+{
+    if (few) {
+        static std::atomic<uint64_t> asked{0};          // per form of the kernel: these are templates
+        const size_t lds = (size_t)a.lp * BS * sizeof(uint32_t);
+        if (lds > 64 * 1024)
+            if (int rc = allow_dynamic_lds(reinterpret_cast<const void *>(&encode_few_kernel<BS, ALIGNED, PACKED, FUSE_CDF, SLOTS, TILE>),
+                                           CG_MAX_LP * BS * (int)sizeof(uint32_t), asked)) return rc;
+        encode_few_kernel<BS, ALIGNED, PACKED, FUSE_CDF, SLOTS, TILE><<<grid, dim3(BS), lds, stream>>>(a);
+    } else {
+        const size_t lds = (size_t)a.lp * TableStride<BS>::k16 * sizeof(uint16_t);
+        encode_streams_kernel<BS, ALIGNED, PACKED, FUSE_CDF, SLOTS, TILE><<<grid, dim3(BS), lds, stream>>>(a);
+    }
+    return check_launch("encode");
 }
 
 // Describe the readable byte window [bytes, bytes + nbytes) to the bit reader, which
