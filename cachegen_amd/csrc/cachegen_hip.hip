@@ -416,22 +416,22 @@ int code_and_compact(const LevelOut &o, const uint32_t *sym4, const uint8_t *sym
     const int64_t cblocks = ceil_div(w.nstreams, kCompactStreams);
     if (cblocks > INT_MAX) return fail(CG_ERR_ARG, "encode_kv: too many streams");
     const int32_t skew = (int32_t)(reinterpret_cast<uintptr_t>(o.payload) & 3u);
-    if (grouped) {
-        compact_streams_kernel<true><<<dim3((unsigned)cblocks), dim3(256), 0, s>>>(
-            w.scratch, kStreamCap, o.offsets, o.lengths, nullptr, w.nstreams, o.payload, o.payload_cap, skew, o.status,
-            w.group_sums, w.tile_sums);
-    } else if (fused_scan && w.ntiles <= kDirectTiles) {
-        compact_streams_kernel<true><<<dim3((unsigned)cblocks), dim3(256), 0, s>>>(
-            w.scratch, kStreamCap, o.offsets, o.lengths, nullptr, w.nstreams, o.payload, o.payload_cap, skew, o.status,
-            nullptr, w.tile_sums);
-    } else if (fused_scan) {
+    const int64_t *tile_base = nullptr;
+    if (fused_scan && !grouped && w.ntiles > kDirectTiles) {
         if (int rc = launch_scan(w.tile_sums, cblocks, INT_MAX, w.tile_base, w.tile_scan_scratch, s)) return rc;
-        compact_streams_kernel<true><<<dim3((unsigned)cblocks), dim3(256), 0, s>>>(
-            w.scratch, kStreamCap, o.offsets, o.lengths, w.tile_base, w.nstreams, o.payload, o.payload_cap, skew, o.status);
-    } else {
+        tile_base = w.tile_base;
+    } else if (!fused_scan) {
         if (int rc = launch_scan(o.lengths, w.nstreams, kStreamCap, o.offsets, w.scan_scratch, s)) return rc;
-        compact_streams_kernel<false><<<dim3((unsigned)cblocks), dim3(256), 0, s>>>(
-            w.scratch, kStreamCap, o.offsets, nullptr, nullptr, w.nstreams, o.payload, o.payload_cap, skew, o.status);
+    }
+    const CompactArgs c = {w.scratch, kStreamCap, o.offsets, fused_scan ? o.lengths : nullptr, tile_base, w.nstreams, o.payload,
+                           o.payload_cap, skew, o.status, grouped ? w.group_sums : nullptr, fused_scan ? w.tile_sums : nullptr};
+    const dim3 cgrid((unsigned)cblocks);
+    if (cblocks <= sliced_compact_blocks()) {
+        if (fused_scan) compact_few_kernel<true><<<cgrid, dim3(1024), 0, s>>>(c);
+        else compact_few_kernel<false><<<cgrid, dim3(1024), 0, s>>>(c);
+    } else {
+        if (fused_scan) compact_streams_kernel<true><<<cgrid, dim3(256), 0, s>>>(c);
+        else compact_streams_kernel<false><<<cgrid, dim3(256), 0, s>>>(c);
     }
     return check_launch("compact");
 }

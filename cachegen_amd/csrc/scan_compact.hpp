@@ -20,41 +20,26 @@ constexpr int kScanThreads = 256;
 constexpr int kScanPerThread = 8;
 constexpr int kScanTile = kScanThreads * kScanPerThread;
 
-__device__ __forceinline__ int64_t block_exclusive_scan(int64_t v, int64_t *lds, int64_t &total)
-{
-    const int tid = threadIdx.x;
-    lds[tid] = v;
-    __syncthreads();
-    for (int o = 1; o < kScanThreads; o <<= 1) {
-        const int64_t add = tid >= o ? lds[tid - o] : 0;
-        __syncthreads();
-        lds[tid] += add;
-        __syncthreads();
-    }
-    total = lds[kScanThreads - 1];
-    const int64_t incl = lds[tid];
-    __syncthreads();
-    return incl - v;
-}
-
-// The same for a block of 256 threads and 32-bit values, with wavefront shuffles and one
-// exchange of the four wavefront totals through `lds` (at least 4 words).
-__device__ __forceinline__ int32_t block_exclusive_scan_256(int32_t v, int32_t *lds, int32_t &total)
+// The block's exclusive running sum: wavefront shuffles and one exchange of the four wavefronts' totals
+// through `lds` (at least 4 values).  A sum in LDS, halving the distance eight times with two barriers
+// each, kept a launch of one block 1 us longer.
+template <typename T>
+__device__ __forceinline__ T block_exclusive_scan_256(T v, T *lds, T &total)
 {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    int32_t incl = v;
+    T incl = v;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
-        const int32_t up = __shfl_up(incl, o, 64);
+        const T up = __shfl_up(incl, o, 64);
         if (lane >= o) incl += up;
     }
     if (lane == 63) lds[wave] = incl;
     __syncthreads();
-    int32_t before = incl - v;
+    T before = incl - v;
     total = 0;
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
-        const int32_t t = lds[w];
+        const T t = lds[w];
         if (w < wave) before += t;
         total += t;
     }
@@ -75,7 +60,7 @@ __global__ __launch_bounds__(kScanThreads) void scan_tile_sums_kernel(
             s += v;
         }
     int64_t total;
-    block_exclusive_scan(s, lds, total);
+    block_exclusive_scan_256(s, lds, total);
     if (threadIdx.x == 0) sums[blockIdx.x] = total;
 }
 
@@ -98,7 +83,7 @@ __global__ __launch_bounds__(kScanThreads) void scan_sums_kernel(int64_t *sums, 
         for (int j = 0; j < kBatch; ++j) mine += v[j];
     }
     int64_t total;
-    int64_t run = block_exclusive_scan(mine, lds, total);
+    int64_t run = block_exclusive_scan_256(mine, lds, total);
     for (int64_t i0 = lo; i0 < hi; i0 += kBatch) {
         int64_t v[kBatch];
 #pragma unroll
@@ -127,7 +112,7 @@ __global__ __launch_bounds__(kScanThreads) void scan_apply_kernel(
     }
     int64_t total;
     // sums == nullptr: the input is a single tile and this kernel is the whole scan
-    int64_t run = (sums ? sums[blockIdx.x] : 0) + block_exclusive_scan(s, lds, total);
+    int64_t run = (sums ? sums[blockIdx.x] : 0) + block_exclusive_scan_256(s, lds, total);
     for (int j = 0; j < kScanPerThread; ++j) {
         if (base + j < n) offsets[base + j] = run;
         run += v[j];
@@ -200,22 +185,41 @@ constexpr int kCompactTile = 16384;
 // tiles before this one (neither: calls of at most kDirectTiles tiles, where that is a few loads per
 // thread and saves the scan launch, 5 us and its gap).
 constexpr int kDirectTiles = 1024;
-template <bool SCAN>
-__global__ __launch_bounds__(256) void compact_streams_kernel(
-    const uint8_t *__restrict__ slots, int32_t cap, int64_t *__restrict__ offsets,
-    const int32_t *__restrict__ lengths, const int64_t *__restrict__ tile_base,
-    int64_t nstreams, uint8_t *__restrict__ payload, int64_t payload_cap, int32_t skew, int32_t *status,
-    const int32_t *__restrict__ group_sums = nullptr, const int32_t *__restrict__ tile_sums = nullptr)
+// SLICES > 1: the block has SLICES x 256 threads, and a stream's words are dealt to SLICES threads, eight in
+// turn.
+struct CompactArgs {
+    const uint8_t *slots;
+    int32_t cap;
+    int64_t *offsets;
+    const int32_t *lengths;
+    const int64_t *tile_base;
+    int64_t nstreams;
+    uint8_t *payload;
+    int64_t payload_cap;
+    int32_t skew;
+    int32_t *status;
+    const int32_t *group_sums, *tile_sums;
+};
+
+template <bool SCAN, int SLICES>
+__device__ __forceinline__ void compact_streams(const CompactArgs &a, int32_t *rel, uint32_t *buf)
 {
-    __shared__ int32_t rel[kCompactStreams + 1];       // stream offsets relative to the block's first byte
-    __shared__ __align__(16) uint32_t buf[kCompactTile / 4];
-    const int tid = threadIdx.x;
+    const uint8_t *__restrict__ const slots = a.slots;
+    const int32_t *__restrict__ const lengths = a.lengths, *__restrict__ const group_sums = a.group_sums, *__restrict__ const tile_sums = a.tile_sums;
+    const int64_t *__restrict__ const tile_base = a.tile_base;
+    int64_t *__restrict__ const offsets = a.offsets;
+    uint8_t *__restrict__ const payload = a.payload;
+    int32_t *const status = a.status;
+    const int64_t nstreams = a.nstreams, payload_cap = a.payload_cap;
+    const int32_t cap = a.cap, skew = a.skew;
+    const int tid = threadIdx.x % 256, slice = SLICES > 1 ? threadIdx.x / 256 : 0;
+    const bool lead_slice = slice == 0;                // the threads that stand for the streams
     const int64_t sbase = (int64_t)blockIdx.x * kCompactStreams;
     const int count = (nstreams - sbase < kCompactStreams) ? (int)(nstreams - sbase) : kCompactStreams;
     int64_t o0;
     if (SCAN) {
         int32_t mine = 0;
-        if (tid < count) {
+        if (lead_slice && tid < count) {
             mine = lengths[sbase + tid];
             mine = mine < 0 ? 0 : (mine > cap ? cap : mine);
         }
@@ -225,15 +229,15 @@ __global__ __launch_bounds__(256) void compact_streams_kernel(
 #pragma unroll
             for (int i = 0; i < kDirectTiles / 256; ++i) {
                 const int t = tid + i * 256;
-                if (t < (int)blockIdx.x) part += tile_sums[t];
+                if (lead_slice && t < (int)blockIdx.x) part += tile_sums[t];
             }
             int32_t sum;
             block_exclusive_scan_256(part, reinterpret_cast<int32_t *>(buf), sum);
             o0 = sum;
         } else if (group_sums) {
             const int g = (int)(blockIdx.x / kTileGroup), r = (int)(blockIdx.x % kTileGroup);
-            int32_t part = tid < g ? group_sums[tid] : 0;
-            if (tid < r) part += tile_sums[(int64_t)g * kTileGroup + tid];
+            int32_t part = lead_slice && tid < g ? group_sums[tid] : 0;
+            if (lead_slice && tid < r) part += tile_sums[(int64_t)g * kTileGroup + tid];
             int32_t sum;
             block_exclusive_scan_256(part, reinterpret_cast<int32_t *>(buf), sum);     // at most 16384 tiles of 64 KiB: fits
             o0 = sum;
@@ -242,21 +246,21 @@ __global__ __launch_bounds__(256) void compact_streams_kernel(
         }
         const int32_t before = block_exclusive_scan_256(mine, reinterpret_cast<int32_t *>(buf), total32);    // buf is free until the copy
         const int64_t total64 = total32;                       // at most 256 streams of `cap` <= 256 bytes
-        rel[tid] = before;
-        if (tid == 0) rel[kCompactStreams] = total32;
-        if (tid < count) offsets[sbase + tid] = o0 + before;
-        if (sbase + count == nstreams && tid == 0) offsets[nstreams] = o0 + total64;
+        if (lead_slice) rel[tid] = before;
+        if (lead_slice && tid == 0) rel[kCompactStreams] = total32;
+        if (lead_slice && tid < count) offsets[sbase + tid] = o0 + before;
+        if (sbase + count == nstreams && lead_slice && tid == 0) offsets[nstreams] = o0 + total64;
         __syncthreads();
         // threads past the last stream carry the total, like the padding of the other form
     } else {
         o0 = offsets[sbase];
-        for (int i = tid; i <= kCompactStreams; i += 256)
+        for (int i = threadIdx.x; i <= kCompactStreams; i += 256 * SLICES)
             rel[i] = (int32_t)(offsets[sbase + (i < count ? i : count)] - o0);
         __syncthreads();
     }
     const int total = rel[count];
     if (o0 + total > payload_cap) {                    // never write past the caller's buffer
-        if (tid == 0 && status) atomicOr(status, 2);
+        if (threadIdx.x == 0 && status) atomicOr(status, 2);
         return;
     }
     // x = position in the range + lead: aligned words of the payload are at multiples of 4
@@ -275,7 +279,7 @@ __global__ __launch_bounds__(256) void compact_streams_kernel(
         const int xe = my1 < t1 ? my1 : t1;
         // aligned words j of the range that hold bytes [xs, xe) of this stream, eight at a time:
         // word j is stream bytes 4j - my0 .. +3, i.e. two stream words through a funnel shift
-        for (int j = xs >> 2; 4 * j < xe; j += 8) {
+        for (int j = (xs >> 2) + 8 * slice; 4 * j < xe; j += 8 * SLICES) {
             const int q = 4 * j - my0;                 // may be negative for the stream's first word
             const int k = q >> 2;
             const uint32_t sh = (uint32_t)(q & 3) * 8u;
@@ -298,7 +302,7 @@ __global__ __launch_bounds__(256) void compact_streams_kernel(
             }
         }
         __syncthreads();
-        for (int w = (t0 >> 2) + tid; 4 * w < t1; w += 256) {
+        for (int w = (t0 >> 2) + (int)threadIdx.x; 4 * w < t1; w += 256 * SLICES) {
             const int x0 = 4 * w;
             const uint32_t v = buf[w - (t0 >> 2)];
             if (x0 >= lead && x0 + 4 <= end) {
@@ -310,6 +314,24 @@ __global__ __launch_bounds__(256) void compact_streams_kernel(
         }
         __syncthreads();
     }
+}
+
+template <bool SCAN>
+__global__ __launch_bounds__(256) void compact_streams_kernel(CompactArgs a)
+{
+    __shared__ int32_t rel[kCompactStreams + 1];       // stream offsets relative to the block's first byte
+    __shared__ __align__(16) uint32_t buf[kCompactTile / 4];
+    compact_streams<SCAN, 1>(a, rel, buf);
+}
+
+// A launch of few blocks lasts as long as its longest stream: 160 bytes are five rounds of loads for one
+// thread, each as long as a trip to memory.
+template <bool SCAN>
+__global__ __launch_bounds__(1024) void compact_few_kernel(CompactArgs a)
+{
+    __shared__ int32_t rel[kCompactStreams + 1];
+    __shared__ __align__(16) uint32_t buf[kCompactTile / 4];
+    compact_streams<SCAN, 4>(a, rel, buf);
 }
 
 // collect_bytes for streams in a padded buffer (encoder.py:209-222): stream g = row * nc + channel
