@@ -148,7 +148,8 @@ int cg_encode_fast_new(const int16_t *cdf, int lp, const int8_t *sym, int64_t nl
     hipStream_t st = static_cast<hipStream_t>(stream);
     const dim3 grid = stream_grid(a.sg, nblocks);
     if (aligned) {
-        const bool few = few_encode(nblocks, block, kFewEncodeBytes);
+        // that form reaches a channel from its token row with a 32-bit offset
+        const bool few = few_encode(nblocks, block, kFewEncodeBytes) && s2 >= 0 && s2 <= 0x7FFFFFFFll / nc;
         CG_DISPATCH_BS(block, return (launch_encode<BS, true, false, false, false>(a, grid, few, st)));
     }
     const size_t shmem = (size_t)lp * (block + 2) * sizeof(uint16_t);      // TableStride<BS>::k16 per entry

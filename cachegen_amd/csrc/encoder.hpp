@@ -45,6 +45,7 @@ struct WordWriter {
     uint8_t *wptr;          // where the next word goes
     int wstride;            // bytes from one word of the stream to the next (4: contiguous)
     int cap;
+    uint32_t whole;         // places a whole word can start at: cap - 3, or none
     int nbytes;             // bytes written so far; -4 before the held-back word's first, empty turn
     __amdgpu_buffer_rsrc_t tile;    // TILE: the block's tile
     uint32_t voff, voff0;           // TILE: byte offset in the tile of the next word, and of the first
@@ -56,6 +57,7 @@ struct WordWriter {
         wptr = dst - stride;
         wstride = stride;
         cap = capacity;
+        whole = capacity >= 4 ? (uint32_t)capacity - 3u : 0u;
         nbytes = -4;
         voff = voff0 = 0;
     }
@@ -73,21 +75,20 @@ struct WordWriter {
             voff += kSlotTile * 4;
             return;
         }
-        if (nbytes >= 0) {
-            if (__builtin_expect(nbytes + 4 <= cap, 1)) {
-                if (ALIGNED) {
-                    *reinterpret_cast<uint32_t *>(wptr) = __builtin_bswap32(word);
-                } else {
-                    wptr[0] = (uint8_t)(word >> 24);
-                    wptr[1] = (uint8_t)(word >> 16);
-                    wptr[2] = (uint8_t)(word >> 8);
-                    wptr[3] = (uint8_t)word;
-                }
+        // one test on the common path: nbytes in [0, cap - 4]
+        if (__builtin_expect((uint32_t)nbytes < whole, 1)) {
+            if (ALIGNED) {
+                *reinterpret_cast<uint32_t *>(wptr) = __builtin_bswap32(word);
             } else {
-                // the last words of a stream that does not fit its slot: keep what fits
-                for (int j = 0; j < 4; ++j)
-                    if (nbytes + j < cap) wptr[j] = (uint8_t)(word >> (24 - 8 * j));
+                wptr[0] = (uint8_t)(word >> 24);
+                wptr[1] = (uint8_t)(word >> 16);
+                wptr[2] = (uint8_t)(word >> 8);
+                wptr[3] = (uint8_t)word;
             }
+        } else if (nbytes >= 0) {
+            // the last words of a stream that does not fit its slot: keep what fits
+            for (int j = 0; j < 4; ++j)
+                if (nbytes + j < cap) wptr[j] = (uint8_t)(word >> (24 - 8 * j));
         }
         wptr += wstride;
         nbytes += 4;

@@ -21,7 +21,7 @@ namespace {
 //   - a sub-chunk's symbols are in registers before the first is coded;
 //   - the store code runs once per eight symbols.
 // 256 symbols of 4096 streams (one wavefront a SIMD) 33 -> 27 us, with the tables counted here 47 -> 36,
-// from byte symbols 49 -> 37; of those 27, 17 are the 256 symbols (160 cycles each, about 20 instructions), 3
+// from byte symbols 49 -> 35; of those 27, 17 are the 256 symbols (160 cycles each, about 20 instructions), 3
 // the loads and the tables, the rest the launch and the last wavefront.
 // The stream is the same number, written the same way (see encoder.hpp): the interval's lower end with
 // its carries.
@@ -236,33 +236,8 @@ __global__ __launch_bounds__(BS) void encode_few_kernel(EncodeArgs a)
             if (mode == kNibbles) count(CodeTag<false, kNibbles>());
             else if (mode == kNibblesEscaped) count(CodeTag<false, kNibblesEscaped>());
             else count(CodeTag<false, kBytes>());
-            // running sum and normalisation (cal_cdf.cu:11-49), as normalize_column16_stride() does it
-            const uint32_t total = (uint32_t)id.n, scale = 0xFFFFu - (uint32_t)(lp - 1);
-            const bool pow2 = (total & (total - 1)) == 0;
-            const int sh = 31 - __builtin_clz(total);
-            const float inv = __fdiv_rn(1.0f, (float)total);
-            uint32_t running = 0;
-            auto normalize = [&](auto quotient) {
-                constexpr int kBatch = 8;                                // counters read in one round trip
-#pragma unroll 1
-                for (int e0 = 0; e0 < lp; e0 += kBatch) {
-                    uint32_t counts[kBatch];
-#pragma unroll
-                    for (int j = 0; j < kBatch; ++j) counts[j] = e0 + j < lp ? col[(e0 + j) * BS] : 0u;
-#pragma unroll
-                    for (int j = 0; j < kBatch; ++j) {
-                        running += counts[j];
-                        if (e0 + j < lp) col[(e0 + j) * BS] = (quotient(scale * running) + (uint32_t)(e0 + j)) << 16;
-                    }
-                }
-            };
-            // scale * running < 2^32, its quotient < 2^16
-            if (pow2) normalize([&](uint32_t x) { return x >> sh; });
-            else normalize([&](uint32_t x) {
-                uint32_t q = (uint32_t)((float)x * inv);
-                const int32_t rem = (int32_t)(x - q * total);
-                return rem < 0 ? q - 1u : rem >= (int32_t)total ? q + 1u : q;
-            });
+            normalize_counts(lp, 0xFFFFu - (uint32_t)(lp - 1), (uint32_t)id.n, [&](int i) { return col[i * BS]; },
+                             [&](int i, uint32_t c) { col[i * BS] = c << 16; });
             // to memory: two entries per 32-bit store, one where the table starts or ends off a word boundary
             const int first = (int)((reinterpret_cast<uintptr_t>(mine) >> 1) & 1u);
             if (first) mine[0] = (uint16_t)(col[0] >> 16);
@@ -342,28 +317,31 @@ __global__ __launch_bounds__(BS) void encode_few_kernel(EncodeArgs a)
 #pragma unroll 1
             for (int t = full * 4; t < id.n; ++t) enc.template put_one<SENTINEL>(enc.entry(symbol(tag, words[(t >> 2) & 31], t & 3)));
         } else {
-            // byte symbols: parts of 64 tokens, the next part's loads in flight while one is coded.  One
-            // copy of the code for all parts: straight-line code for 256 loads takes a lone wavefront 24 us to
-            // fetch.  A part's last loads may repeat the sub-chunk's last token.
-            typedef uint32_t words16 __attribute__((ext_vector_type(16)));
-            const uint8_t *sp = a.sym + id.row * a.s0 + id.t0 * a.s1 + id.ch * a.s2;
-            uint32_t bytes[64];
+            // byte symbols: parts of 64 tokens, the next part's loads in flight while one is coded, one copy of
+            // the code for all parts (straight-line code for 256 loads took a lone wavefront 24 us).  A
+            // part's last loads may repeat the sub-chunk's last token.
+            constexpr int kPart = 64;
+            typedef uint32_t part_words __attribute__((ext_vector_type(kPart / 4)));
+            const uint8_t *sp = a.sym + id.row * a.s0 + id.t0 * a.s1;             // uniform over the block
+            const uint32_t voff = (uint32_t)id.ch * (uint32_t)a.s2;               // the host checks that this fits
+            uint32_t bytes[kPart];
             auto fetch = [&](int t0) {
+                const uint8_t *row = sp + (int64_t)t0 * a.s1;
 #pragma unroll
-                for (int j = 0; j < 64; ++j) {
-                    const int t = t0 + j < id.n ? t0 + j : id.n - 1;
-                    bytes[j] = sp[(int64_t)t * a.s1];
+                for (int j = 0; j < kPart; ++j) {
+                    bytes[j] = row[voff];
+                    if (t0 + j + 1 < id.n) row += a.s1;
                 }
             };
             if (id.n > 0) fetch(0);
 #pragma unroll 1
-            for (int t0 = 0; t0 < id.n; t0 += 64) {
-                words16 part;
+            for (int t0 = 0; t0 < id.n; t0 += kPart) {
+                part_words part;
 #pragma unroll
-                for (int w = 0; w < 16; ++w)
+                for (int w = 0; w < kPart / 4; ++w)
                     part[w] = bytes[4 * w] | bytes[4 * w + 1] << 8 | bytes[4 * w + 2] << 16 | bytes[4 * w + 3] << 24;
-                if (t0 + 64 < id.n) fetch(t0 + 64);
-                const int left = id.n - t0 < 64 ? id.n - t0 : 64;
+                if (t0 + kPart < id.n) fetch(t0 + kPart);
+                const int left = id.n - t0 < kPart ? id.n - t0 : kPart;
                 const int wn = __builtin_amdgcn_readfirstlane((left >> 3) * 2);
 #pragma unroll 1
                 for (int w = 0; w < wn; w += 2) group(part[w], part[w + 1]);

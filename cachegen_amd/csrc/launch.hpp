@@ -122,8 +122,15 @@ int launch_cdf(const uint8_t *sym, const uint32_t *sym4, int64_t nsub, int64_t r
     a.g.T = T;
     a.g.S = S;
     a.g.nsc = (int32_t)ceil_div(S, kSub);
-    const int64_t nblocks = ceil_div(T, S) * rows * a.ctiles;
+    int64_t nblocks = ceil_div(T, S) * rows * a.ctiles;
     if (nblocks <= 0 || nblocks > INT_MAX) return fail(CG_ERR_ARG, "calculate_cdf: grid out of range");
+    // Narrower blocks where that is how more compute units get one: a block's lanes and slices all count
+    // through one unit's LDS.  512 channels x 4 rows: 512 tokens 13.1 -> 8.6 us, 256 tokens of byte symbols 11.1 -> 7.6.
+    while (block > 64 && nblocks * 2 <= compute_units()) {
+        block /= 2;
+        a.ctiles = (int32_t)ceil_div(nc, block);
+        nblocks = ceil_div(T, S) * rows * a.ctiles;
+    }
     const size_t shmem = sym4 ? (size_t)(max_bins + 1) * (block + 2) * sizeof(uint16_t)
                               : (size_t)(max_bins + 1) * (block + 1) * sizeof(uint32_t);     // TableStride
     const bool sliced = nblocks * block <= sliced_lanes(sym4 != nullptr, S < T ? S : T);

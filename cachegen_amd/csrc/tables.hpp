@@ -64,31 +64,82 @@ struct TableWalk {
     }
 };
 
-// Running sum and normalisation of one lane's column col[i * stride], i in [0, lp).
-template <int BS>
-__device__ __forceinline__ void normalize_column(uint32_t *col, int lp, int max_bins)
+// floor(x / total) for x < 2^32 with a quotient below 2^16, from inv = 1 / total in float32: the estimate is
+// off by one at most.
+__device__ __forceinline__ uint32_t divide16(uint32_t x, uint32_t total, float inv)
 {
-    constexpr int kS = TableStride<BS>::k32;
-    uint32_t running = 0;
-    for (int i = 1; i < lp; ++i) {
-        running = (running + col[i * kS]) & 0xFFFFu;
-        col[i * kS] = running;
-    }
-    const uint32_t scale = 0xFFFFu - (uint32_t)max_bins;
-    for (int i = 0; i < lp; ++i) {
-        const uint32_t q = running ? (scale * col[i * kS] / running) & 0xFFFFu : 0u;
-        col[i * kS] = (q + (uint32_t)i) & 0xFFFFu;
+    const uint32_t q = (uint32_t)((float)x * inv);
+    const int32_t rem = (int32_t)(x - q * total);
+    return rem < 0 ? q - 1u : rem >= (int32_t)total ? q + 1u : q;
+}
+
+// A lane's counts into its table's entries: entry i is floor(scale * (sum of the counts up to i) / total) + i
+// in 16 bits, scale * total < 2^32.  count(i) reads, entry(i, c) stores (which may be in the count's place).
+// Counts are read eight at a time: one by one, each behind the store of the one before, they took an
+// LDS round trip each.
+template <typename Count, typename Entry>
+__device__ __forceinline__ void normalize_counts(int lp, uint32_t scale, uint32_t total, Count count, Entry entry)
+{
+    auto walk = [&](auto quotient) {
+        constexpr int kBatch = 8;
+        uint32_t running = 0;
+        int e0 = 0;
+#pragma unroll 1
+        for (; e0 + kBatch <= lp; e0 += kBatch) {
+            uint32_t v[kBatch];
+#pragma unroll
+            for (int j = 0; j < kBatch; ++j) v[j] = count(e0 + j);
+#pragma unroll
+            for (int j = 0; j < kBatch; ++j) {
+                running += v[j];
+                entry(e0 + j, (quotient(scale * running) + (uint32_t)(e0 + j)) & 0xFFFFu);
+            }
+        }
+#pragma unroll 1
+        for (; e0 < lp; ++e0) {
+            running += count(e0);
+            entry(e0, (quotient(scale * running) + (uint32_t)e0) & 0xFFFFu);
+        }
+    };
+    if ((total & (total - 1)) == 0) {
+        const int sh = total ? 31 - __builtin_clz(total) : 0;
+        walk([&](uint32_t x) { return x >> sh; });
+    } else {
+        // the float estimate of the quotient, below 2^16, is off by one at most
+        const float inv = __fdiv_rn(1.0f, (float)total);
+        walk([&](uint32_t x) {
+            const uint32_t q = (uint32_t)((float)x * inv);
+            const int32_t rem = (int32_t)(x - q * total);
+            return rem < 0 ? q - 1u : rem >= (int32_t)total ? q + 1u : q;
+        });
     }
 }
 
-// Write the block's tables tab[entry * stride + lane] to cdf[lane][entry], coalesced.
+// Running sum and normalisation of one lane's column col[i * stride], i in [0, lp), whose first entry is 0.
 template <int BS>
+__device__ __forceinline__ void normalize_column(uint32_t *col, int lp, int max_bins)
+{
+    constexpr int kS = TableStride<BS>::k32, kBatch = 4;
+    uint32_t total = 0;                     // at most 65 535: cal_cdf.cu's 16-bit counters
+#pragma unroll 1
+    for (int e0 = 1; e0 < lp; e0 += kBatch) {
+        uint32_t v[kBatch];
+#pragma unroll
+        for (int j = 0; j < kBatch; ++j) v[j] = col[(e0 + j < lp ? e0 + j : 0) * kS];
+#pragma unroll
+        for (int j = 0; j < kBatch; ++j) total += v[j];
+    }
+    normalize_counts(lp, 0xFFFFu - (uint32_t)max_bins, total, [&](int i) { return col[i * kS]; }, [&](int i, uint32_t c) { col[i * kS] = c; });
+}
+
+// Write the block's tables tab[entry * stride + lane] to cdf[lane][entry], coalesced.
+template <int BS, int THREADS>
 __device__ __forceinline__ void write_tables(const uint32_t *tab, uint16_t *cdf, int lp, int64_t ch0, int64_t nc)
 {
     const int64_t nvalid = (nc - ch0 < BS) ? (nc - ch0) : BS;
     const int total = (int)nvalid * lp;
-    TableWalk w(threadIdx.x, BS, lp);
-    for (int i = threadIdx.x; i < total; i += BS, w.next(lp)) {
+    TableWalk w(threadIdx.x, THREADS, lp);
+    for (int i = threadIdx.x; i < total; i += THREADS, w.next(lp)) {
         cdf[i] = (uint16_t)tab[w.e * TableStride<BS>::k32 + w.c];
     }
 }
@@ -180,26 +231,8 @@ __device__ __forceinline__ void write_column16_stride(const uint16_t *col, uint1
 template <int kS>
 __device__ __forceinline__ void normalize_column16_stride(uint16_t *col, int lp, int max_bins, uint32_t total)
 {
-    const uint32_t scale = 0xFFFFu - (uint32_t)max_bins;
-    uint32_t running = 0;
-    if ((total & (total - 1)) == 0) {
-        const int sh = 31 - __builtin_clz(total);
-        for (int i = 0; i < lp; ++i) {
-            running += col[i * kS];
-            col[i * kS] = (uint16_t)(((scale * running) >> sh) + (uint32_t)i);
-        }
-    } else {
-        const float inv = __fdiv_rn(1.0f, (float)total);
-        for (int i = 0; i < lp; ++i) {
-            running += col[i * kS];
-            const uint32_t x = scale * running;                  // < 2^32, quotient < 2^16
-            uint32_t q = (uint32_t)((float)x * inv);
-            int32_t rem = (int32_t)(x - q * total);
-            if (rem < 0) { q--; rem += (int32_t)total; }
-            if (rem >= (int32_t)total) q++;
-            col[i * kS] = (uint16_t)(q + (uint32_t)i);
-        }
-    }
+    normalize_counts(lp, 0xFFFFu - (uint32_t)max_bins, total, [&](int i) { return (uint32_t)col[i * kS]; },
+                     [&](int i, uint32_t c) { col[i * kS] = (uint16_t)c; });
 }
 
 // The same two for a block's tables with the row stride of TableStride<BS>.
@@ -269,19 +302,17 @@ __global__ __launch_bounds__(BS * SLICES) void calculate_cdf_kernel(CdfArgs a)
     const uint32_t mb = (uint32_t)a.max_bins;
     if (ch < a.nc) {
         if (!PACKED) {
+            // a slice's tokens, kBatch loads in flight; behind the chunk's end the last token is read again and
+            // not counted
+            constexpr int kBatch = SLICES > 1 ? 32 : 8;
             const uint8_t *p = a.sym + row * a.s0 + ch * a.s2;
-            int64_t t = t0 + slice * 8;
-            for (; t + 8 <= t1; t += 8 * SLICES) {
-                uint32_t v[8];
+            for (int64_t t = t0 + slice * kBatch; t < t1; t += kBatch * SLICES) {
+                uint32_t v[kBatch];
 #pragma unroll
-                for (int j = 0; j < 8; ++j) v[j] = p[(t + j) * a.s1];
+                for (int j = 0; j < kBatch; ++j) v[j] = p[(t + j < t1 ? t + j : t1 - 1) * a.s1];
 #pragma unroll
-                for (int j = 0; j < 8; ++j)
-                    if (v[j] < mb) atomicAdd(col + (v[j] + 1) * kS32, 1u);      // no value returned: one LDS operation
-            }
-            for (; t < t1; ++t) {            // fewer than eight tokens are left: one slice's
-                const uint32_t v = p[t * a.s1];
-                if (v < mb) atomicAdd(col + (v + 1) * kS32, 1u);
+                for (int j = 0; j < kBatch; ++j)
+                    if (v[j] < mb && t + j < t1) atomicAdd(col + (v[j] + 1) * kS32, 1u);      // no value returned: one LDS operation
             }
         } else {
             uint32_t *const pair = smem + (tcol >> 1);
@@ -305,22 +336,27 @@ __global__ __launch_bounds__(BS * SLICES) void calculate_cdf_kernel(CdfArgs a)
                     uint32_t v[kBatch];
 #pragma unroll
                     for (int j = 0; j < kBatch; ++j) v[j] = (w0 + j < nwords) ? wp[(int64_t)(w0 + j) * a.nc] : 0u;
-                    if (narrow) {
-                        // the value 15 stands for a saturated byte: the table's last symbol
+                    // whole batches without a test per symbol
+                    auto count = [&](auto whole) {
+                        if (narrow) {
+                            // the value 15 stands for a saturated byte: the table's last symbol
 #pragma unroll
-                        for (int j = 0; j < 4 * kBatch; ++j) {
-                            uint32_t s = __builtin_amdgcn_ubfe(v[j >> 2] >> half_shift, (uint32_t)(4 * (j & 3)), 4u);
-                            s = s == 15u ? mb - 1u : s;
-                            if (w0 * 4 + j < n) atomicAdd(pair + (s + 1) * (kS16 / 2), one);
-                        }
-                    } else {
+                            for (int j = 0; j < 4 * kBatch; ++j) {
+                                uint32_t s = __builtin_amdgcn_ubfe(v[j >> 2] >> half_shift, (uint32_t)(4 * (j & 3)), 4u);
+                                s = s == 15u ? mb - 1u : s;
+                                if (decltype(whole)::value || w0 * 4 + j < n) atomicAdd(pair + (s + 1) * (kS16 / 2), one);
+                            }
+                        } else {
 #pragma unroll
-                        for (int j = 0; j < 4 * kBatch; ++j) {
-                            uint32_t s = (v[j >> 2] >> (8 * (j & 3))) & 0xFFu;
-                            s = s < mb - 1u ? s : mb - 1u;
-                            if (w0 * 4 + j < n) atomicAdd(pair + (s + 1) * (kS16 / 2), one);
+                            for (int j = 0; j < 4 * kBatch; ++j) {
+                                uint32_t s = (v[j >> 2] >> (8 * (j & 3))) & 0xFFu;
+                                s = s < mb - 1u ? s : mb - 1u;
+                                if (decltype(whole)::value || w0 * 4 + j < n) atomicAdd(pair + (s + 1) * (kS16 / 2), one);
+                            }
                         }
-                    }
+                    };
+                    if ((w0 + kBatch) * 4 <= n) count(BoolTag<true>());
+                    else count(BoolTag<false>());
                 }
             }
         }
@@ -339,9 +375,8 @@ __global__ __launch_bounds__(BS * SLICES) void calculate_cdf_kernel(CdfArgs a)
         if (SLICES > 1) {
             if (ch < a.nc && slice == 0) normalize_column<BS>(col, lp, a.max_bins);
             __syncthreads();
-            if (slice > 0) return;           // the write-out walks the tables BS entries at a time
         }
-        write_tables<BS>(smem, dst, lp, ch0, a.nc);
+        write_tables<BS, BS * SLICES>(smem, dst, lp, ch0, a.nc);
     }
 }
 
