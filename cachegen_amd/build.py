@@ -34,6 +34,7 @@ OCCUPANCY_BUDGETS = [
     (r"^encode_streams_kernel<", 7),         # the forms behind the four reference entry points and odd shapes
     (r"^encode_streams_kernel<256, true, true, (true|false), true, true>", 8),   # the fused path of cg_encode_kv
     (r"^decode_streams_kernel<", 8),
+    (r"^decode_float_kernel<", 8),
     (r"^compact_streams_kernel<", 8),
     (r"^quantize_pack_kernel<[01], (true|false), 2, false>", 8),                # up to 1024 channels, one level
     (r"^quantize_tables_kernel<[01], (true|false), [12], (9|17|33)>", 4),       # two blocks of eight wavefronts per compute unit
@@ -41,8 +42,9 @@ OCCUPANCY_BUDGETS = [
 
 
 # Kernels that address their dynamically allocated LDS from byte 0 (the counters of the table
-# builder: the address comes out of a byte permute): a statically allocated array would sit there.
-NO_STATIC_LDS = r"^(quantize_tables_kernel|tables_from_partial_kernel)<"
+# builder: the address comes out of a byte permute; the float search, which sets an entry's address
+# bit by bit): a statically allocated array would sit there.
+NO_STATIC_LDS = r"^(quantize_tables_kernel|tables_from_partial_kernel|decode_float_kernel)<"
 
 
 def parse_kernel_resources(report):

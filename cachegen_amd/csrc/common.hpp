@@ -156,4 +156,13 @@ __device__ __forceinline__ void lds_entries_high(lds_char *p, uint32_t &lo, uint
                  : "v"(p), "n"(ROW));
 }
 
+// The same from LDS byte p, and the float FLOATS bytes from byte f, in one round trip.
+template <int ROW, int FLOATS>
+__device__ __forceinline__ void lds_entries_high_and_float(uint32_t p, uint32_t f, uint32_t &lo, uint32_t &hi, float &value)
+{
+    asm volatile("ds_read_u16_d16_hi %0, %3\n\tds_read_u16_d16_hi %1, %3 offset:%5\n\tds_read_b32 %2, %4 offset:%6\n\ts_waitcnt lgkmcnt(0)"
+                 : "+v"(lo), "+v"(hi), "=&v"(value)
+                 : "v"(p), "v"(f), "n"(ROW), "n"(FLOATS));
+}
+
 }  // namespace

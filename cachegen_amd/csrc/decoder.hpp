@@ -163,10 +163,14 @@ struct DecodeArgs {
 // Tables in LDS for the decoder: entry e of lane c's column is the 16-bit word at byte
 // e * kRow + 2 * c.  When the kernel dequantises, every row carries one float behind the
 // lanes' entries: (e - C) / C, the quotient of symbol e (decoder.py:28-31).
-template <int BS, int OUT>
+// FLOAT (see below_off): a row is a power of two and the column, 2 * table_column(c), lies below it, from
+// LDS byte 0 (these kernels have no statically allocated LDS; the build checks it), so the bits of an
+// entry's address above the column are the symbol; the quotients follow the row maxima.
+template <int BS, int OUT, bool FLOAT = false>
 struct DecodeLayout {
-    static constexpr int kRow = OUT == OUT_SYMBOLS ? 2 * BS : 2 * BS + 4;
-    static constexpr int kQuot = 2 * BS;          // byte offset of the quotient inside a row
+    static constexpr int kRow = OUT == OUT_SYMBOLS || FLOAT ? 2 * BS : 2 * BS + 4;
+    static constexpr int kQuot = 2 * BS;          // byte offset of the quotient inside a row (not FLOAT)
+    static constexpr int kRowBits = BS == 256 ? 9 : BS == 128 ? 8 : 7;
 };
 
 
@@ -174,6 +178,10 @@ __device__ __forceinline__ uint32_t lds_entry(lds_char *p, int byte_offset)
 {
     return *(lds_u16 *)(p + byte_offset);
 }
+
+// (b & c) | a and b ? c : a bit by bit, one instruction each
+__device__ __forceinline__ uint32_t or_masked(uint32_t a, uint32_t mask, uint32_t bits) { return __builtin_amdgcn_bitop3_b32(a, mask, bits, 0xF8); }
+__device__ __forceinline__ uint32_t pick(uint32_t mask, uint32_t set, uint32_t clear) { return __builtin_amdgcn_bitop3_b32(mask, set, clear, 0xCA); }
 
 // float32 -> bfloat16 bits by the hardware's conversion (round to nearest even, a NaN stays
 // a NaN): one instruction on this GPU
@@ -190,6 +198,8 @@ struct DecodeLane {
     // the entries the first two probes of the unrolled search look at (one for the first, one
     // of two for the second), read once per stream: two LDS round trips less per symbol
     uint32_t probe1, probe2_lo, probe2_hi;
+    uint32_t held[8];          // FLOAT: the entries the first steps look at, evenly spaced (entry 0 unused)
+    uint32_t step[6];          // FLOAT: step[k] is 2^k rows, in a vector register (a scalar operand halves the issue rate)
     // the decoded symbol's two table entries, each shifted left by 16: only ever written by
     // loads into the upper half, so that the lower halves stay zero
     uint32_t bound_lo, bound_hi;
@@ -206,38 +216,100 @@ struct DecodeLane {
 // Distance of the unrolled search's first probe from entry 0, in entries.
 __host__ __device__ constexpr int first_probe(int log2, int skip) { return log2 >= 2 ? ((1 << log2) >> 1) >> skip : 0; }
 
+// The float search: how many of its steps look at entries held in registers, and how far those are apart.
+template <int LOG2, int SKIP>
+struct FloatSearch {
+    static constexpr int kSteps = LOG2 - SKIP;           // at least 2
+    static constexpr int kHeldSteps = kSteps >= 5 ? 3 : kSteps >= 2 ? kSteps - 2 : 0;
+    static constexpr int kApart = kSteps >= 2 ? 1 << (kSteps - kHeldSteps) : 1;
+};
+
 // One symbol.  SKIP: how many of the search's first probes are left out because the row's
 // alphabet fits the lower 2^(LOG2-SKIP) entries.  SAFE: the last table entry may be decoded
 // (its upper bound 2^16 is substituted, dec_new.cu:278) and values may be NaN.
-template <int BS, int LOG2, int OUT, int SKIP, bool SAFE>
+template <int BS, int LOG2, int OUT, int SKIP, bool SAFE, bool FLOAT>
 __device__ __forceinline__ void decode_symbol(const DecodeArgs &a, DecodeLane &s, int lp, int nsteps,
                                               float rm, int i)
 {
-    constexpr int kRow = DecodeLayout<BS, OUT>::kRow;
+    constexpr int kRow = DecodeLayout<BS, OUT, FLOAT>::kRow;
     constexpr int kStep1 = first_probe(LOG2, SKIP), kStep2 = kStep1 >> 1;
     lds_char *p = s.colp;              // entry of the decoded symbol
     lds_char *const plast = s.colp + (lp - 2) * kRow;
     uint32_t t_lo, width, rel;         // rel = off - t_lo
     float q = 0.0f;                    // (symbol - C) / C
+    // FLOAT: where the symbol's quotient is among the quotients: the address bits that are the symbol, moved
+    // down to whole floats
+    auto quotient_place = [&](lds_char *entry) {
+        uint32_t place = (uint32_t)(uintptr_t)entry >> (DecodeLayout<BS, OUT, FLOAT>::kRowBits - 2);
+        asm("" : "+v"(place));         // two instructions of the cheap class instead of a bit field's one
+        return place & 0x3FCu;
+    };
+    auto quotient = [&](lds_char *entry) {
+        if (FLOAT) return *(lds_f32 *)((lds_char *)quotient_place(entry) + lp * kRow + kSub * 4);
+        return *(lds_f32 *)(entry + s.lutoff);
+    };
     const bool full_range = s.span == 0;
     const uint32_t sh = s.span >> 16, sl = s.span & 0xFFFFu;
     if (LOG2 >= 2) {
         // largest m with T(m) <= off, probed with the lower bound sh * c <= T(c), which can
         // only overshoot
-        // the first two probes compare entries held in registers
-        const bool up1 = mul24(sh, s.probe1) <= s.off;
-        p = up1 ? p + kStep1 * kRow : p;
-        if (kStep2 >= 1) {
-            const uint32_t c2 = up1 ? s.probe2_hi : s.probe2_lo;
-            p = (mul24(sh, c2) <= s.off) ? p + kStep2 * kRow : p;
-        }
+        if constexpr (FLOAT) {
+            // span * c / 2^16 against off in float32: an entry as it was loaded is the denormal c * 2^-149, so
+            // the scales 2^95 and 2^-38 make both sides ordinary numbers.  The sign of the difference,
+            // spread over a register, sets one bit of the entry's address.  Wrong by one entry where off
+            // lies within a few parts in 2^23 of a bound, which the one test below sees.
+            uint32_t off = s.off;
+            asm("" : "+v"(off));       // or it is converted from the 64-bit pair it was shifted in
+            const float fs = (float)s.span * 0x1p95f, fo = (float)off * 0x1p-38f;
+            auto below_off = [&](uint32_t c) {
+                return (uint32_t)((int32_t)__float_as_uint(__builtin_fmaf(__uint_as_float(c), fs, -fo)) >> 31);
+            };
+            uint32_t at = (uint32_t)(uintptr_t)p;
+            // the first steps take their entries from registers, halving what is left of them
+            typedef FloatSearch<LOG2, SKIP> Search;
+            uint32_t left[1 << Search::kHeldSteps];
 #pragma unroll
-        for (int step = kStep2 >> 1; step >= 1; step >>= 1)
-            p = (mul24(sh, lds_entry(p, step * kRow)) <= s.off) ? p + step * kRow : p;
-        // both bounds and the quotient in one round trip (entry lp - 1 exists, so the upper
-        // bound of the last symbol can be read and then replaced)
-        if (OUT != OUT_SYMBOLS) q = *(lds_f32 *)(p + s.lutoff);
-        lds_entries_high<kRow>(p, s.bound_lo, s.bound_hi);
+            for (int k = 1; k < 1 << Search::kHeldSteps; ++k) left[k] = s.held[k];
+#pragma unroll
+            for (int h = Search::kHeldSteps - 1; h >= 0; --h) {
+                const uint32_t up = below_off(left[1 << h]);
+                at = or_masked(at, up, s.step[Search::kSteps - Search::kHeldSteps + h]);
+#pragma unroll
+                for (int k = 1; k < 1 << h; ++k) left[k] = pick(up, left[(1 << h) + k], left[k]);
+            }
+            // the others two at a time, three entries in a round trip
+            int k = Search::kSteps - Search::kHeldSteps - 1;
+            if (k % 2 == 0) {
+                at = or_masked(at, below_off(lds_entry((lds_char *)at, kRow << k)), s.step[k]);
+                --k;
+            }
+#pragma unroll
+            for (; k >= 1; k -= 2) {
+                lds_char *const q1 = (lds_char *)at;
+                const uint32_t c1 = lds_entry(q1, kRow << (k - 1)), c2 = lds_entry(q1, kRow << k), c3 = lds_entry(q1, 3 * (kRow << (k - 1)));
+                const uint32_t up = below_off(c2);
+                at = or_masked(at, up, s.step[k]);
+                at = or_masked(at, below_off(pick(up, c3, c1)), s.step[k - 1]);
+            }
+            p = (lds_char *)at;
+            // both bounds and the quotient in one round trip
+            lds_entries_high_and_float<kRow, ((1 << LOG2) + 1) * kRow + kSub * 4>(at, quotient_place(p), s.bound_lo, s.bound_hi, q);
+        } else {
+            // the first two probes compare entries held in registers
+            const bool up1 = mul24(sh, s.probe1) <= s.off;
+            p = up1 ? p + kStep1 * kRow : p;
+            if (kStep2 >= 1) {
+                const uint32_t c2 = up1 ? s.probe2_hi : s.probe2_lo;
+                p = (mul24(sh, c2) <= s.off) ? p + kStep2 * kRow : p;
+            }
+#pragma unroll
+            for (int step = kStep2 >> 1; step >= 1; step >>= 1)
+                p = (mul24(sh, lds_entry(p, step * kRow)) <= s.off) ? p + step * kRow : p;
+            // both bounds and the quotient in one round trip (entry lp - 1 exists, so the upper
+            // bound of the last symbol can be read and then replaced)
+            if (OUT != OUT_SYMBOLS) q = *(lds_f32 *)(p + s.lutoff);
+            lds_entries_high<kRow>(p, s.bound_lo, s.bound_hi);
+        }
         // T(c) = (span * c) >> 16 = high word of span * (c << 16) for c < 2^16; the one entry
         // that is 2^16, the upper bound of the last symbol (dec_new.cu:278), gives the span
         t_lo = __umulhi(s.span, s.bound_lo);
@@ -270,8 +342,17 @@ __device__ __forceinline__ void decode_symbol(const DecodeArgs &a, DecodeLane &s
                     t_lo = __umulhi(s.span, b_lo);
                 }
                 width = (top ? s.span : __umulhi(s.span, b_hi)) - t_lo;
+                if (FLOAT) {
+                    // and the search can have fallen short: forward, to the last entry that is searched at the furthest
+                    lds_char *const end = s.colp + ((1 << (LOG2 - SKIP)) - 1) * kRow;
+                    while (s.off - t_lo >= width && p < end) {
+                        p += kRow;
+                        t_lo = __umulhi(s.span, lds_entry(p, 0) << 16);
+                        width = ((SAFE && p == plast) ? s.span : __umulhi(s.span, lds_entry(p, kRow) << 16)) - t_lo;
+                    }
+                }
             }
-            if (OUT != OUT_SYMBOLS) q = *(lds_f32 *)(p + s.lutoff);
+            if (OUT != OUT_SYMBOLS) q = quotient(p);
             rel = s.off - t_lo;
         }
     } else {
@@ -286,7 +367,7 @@ __device__ __forceinline__ void decode_symbol(const DecodeArgs &a, DecodeLane &s
         p = s.colp + lo_i * kRow;
         const uint32_t c_lo = lds_entry(p, 0);
         const uint32_t c_hi = (SAFE && p == plast) ? 0x10000u : lds_entry(p, kRow);
-        if (OUT != OUT_SYMBOLS) q = *(lds_f32 *)(p + s.lutoff);
+        if (OUT != OUT_SYMBOLS) q = quotient(p);
         if (full_range) {
             t_lo = c_lo << 16;
             width = (c_hi - c_lo) << 16;
@@ -341,18 +422,26 @@ __device__ __forceinline__ void decode_symbol(const DecodeArgs &a, DecodeLane &s
 // the most advanced wavefronts first and leaves the least advanced for the end; these blocks
 // raise their wavefronts' priority by the work they have left instead, so that the wavefronts of
 // a SIMD finish closer together.
-template <int BS, int LOG2, int OUT, int SKIP, bool SAFE>
+template <int BS, int LOG2, int OUT, int SKIP, bool SAFE, bool FLOAT>
 __device__ __forceinline__ void decode_lane(const DecodeArgs &a, DecodeLane &s, int lp, int n, lds_f32 *rmp, bool last_round)
 {
     int nsteps = 0;
     if (LOG2 < 0)
         while ((1 << nsteps) < lp - 1) ++nsteps;
     if (LOG2 >= 2) {
-        constexpr int kRow = DecodeLayout<BS, OUT>::kRow;
+        constexpr int kRow = DecodeLayout<BS, OUT, FLOAT>::kRow;
         constexpr int kStep1 = first_probe(LOG2, SKIP), kStep2 = kStep1 >> 1;
-        s.probe1 = lds_entry(s.colp, kStep1 * kRow);
-        s.probe2_lo = lds_entry(s.colp, kStep2 * kRow);
-        s.probe2_hi = lds_entry(s.colp, (kStep1 + kStep2) * kRow);
+        if constexpr (FLOAT) {
+            typedef FloatSearch<LOG2, SKIP> Search;
+#pragma unroll
+            for (int k = 1; k < 1 << Search::kHeldSteps; ++k) s.held[k] = lds_entry(s.colp, k * Search::kApart * kRow);
+#pragma unroll
+            for (int k = 0; k < Search::kSteps; ++k) asm volatile("v_mov_b32 %0, %1" : "=v"(s.step[k]) : "n"(kRow << k));
+        } else {
+            s.probe1 = lds_entry(s.colp, kStep1 * kRow);
+            s.probe2_lo = lds_entry(s.colp, kStep2 * kRow);
+            s.probe2_hi = lds_entry(s.colp, (kStep1 + kStep2) * kRow);
+        }
         s.bound_lo = 0;
         s.bound_hi = 0;
     }
@@ -376,14 +465,14 @@ __device__ __forceinline__ void decode_lane(const DecodeArgs &a, DecodeLane &s, 
         for (int j = 0; j < kGroup; ++j) {
             if (j == 0) s.rd.top_up();
             else if (__builtin_expect(s.rd.short_of_bits, 0)) s.rd.top_up();
-            decode_symbol<BS, LOG2, OUT, SKIP, SAFE>(a, s, lp, nsteps, rm[j], i0 + j);
+            decode_symbol<BS, LOG2, OUT, SKIP, SAFE, FLOAT>(a, s, lp, nsteps, rm[j], i0 + j);
         }
     }
     // what is left of a sub-chunk whose tokens are no multiple of the group
 #pragma unroll 1
     for (; i0 < n; ++i0, ++rmp) {
         s.rd.top_up();
-        decode_symbol<BS, LOG2, OUT, SKIP, SAFE>(a, s, lp, nsteps, OUT != OUT_SYMBOLS ? *rmp : 0.0f, i0);
+        decode_symbol<BS, LOG2, OUT, SKIP, SAFE, FLOAT>(a, s, lp, nsteps, OUT != OUT_SYMBOLS ? *rmp : 0.0f, i0);
     }
 }
 
@@ -545,10 +634,10 @@ __device__ __forceinline__ void decode_few_lane(const DecodeArgs &a, FewLane &s,
 // LOG2 >= 0: the table has exactly 2^LOG2 symbols (lp = 2^LOG2 + 1) and the search is
 // unrolled with immediate LDS offsets; LOG2 < 0: any lp.
 // FEW: decode_few_kernel's tables, 32-bit entries in rows of one word a lane, and the quotients behind the row maxima.
-template <int BS, int LOG2, int SRC, int OUT, bool FEW>
+template <int BS, int LOG2, int SRC, int OUT, bool FEW, bool FLOAT = false>
 __device__ __forceinline__ void decode_streams(const DecodeArgs &a, uint32_t *smem)
 {
-    constexpr int kRow = FEW ? 4 * BS : DecodeLayout<BS, OUT>::kRow;
+    constexpr int kRow = FEW ? 4 * BS : DecodeLayout<BS, OUT, FLOAT>::kRow;
     const int tid = threadIdx.x;
     StreamId id;
     // SRC_LISTED: the sub-chunks of a launch come from several containers, each with its own tables,
@@ -569,7 +658,8 @@ __device__ __forceinline__ void decode_streams(const DecodeArgs &a, uint32_t *sm
     const int lp = LOG2 >= 0 ? (1 << LOG2) + 1 : a.lp;
     char *rows = reinterpret_cast<char *>(smem);
     float *rowmax = reinterpret_cast<float *>(rows + lp * kRow);     // one per token of the sub-chunk
-    float *few_quots = rowmax + kSub;                                // FEW: one per table entry
+    float *quots = rowmax + kSub;                                    // FEW, FLOAT: one per table entry
+    int *votes = reinterpret_cast<int *>(quots + lp);                // FLOAT: one per wavefront
     {
         // Every lane copies its own table (lp consecutive 16-bit entries) into its LDS column:
         // loads and LDS writes with immediate offsets, no address arithmetic per entry; the
@@ -578,7 +668,7 @@ __device__ __forceinline__ void decode_streams(const DecodeArgs &a, uint32_t *sm
         // it is stored as 0 whatever the input holds so that the walk back always ends.
         const uint16_t *tables = SRC == SRC_LISTED ? reinterpret_cast<const uint16_t *>(d.cdf) : a.cdf;
         const uint16_t *mine = tables + ((id.chunk * a.sg.rows + id.row) * a.sg.nc + id.ch) * lp;
-        char *column = rows + (FEW ? 4 : 2) * tid;
+        char *column = rows + (FEW ? 4 * tid : 2 * (FLOAT ? table_column<BS>(tid) : tid));
         auto put = [&](int e, uint16_t v) {
             if (FEW) *reinterpret_cast<uint32_t *>(column + e * kRow) = (uint32_t)v << 16;
             else *reinterpret_cast<uint16_t *>(column + e * kRow) = v;
@@ -620,7 +710,7 @@ __device__ __forceinline__ void decode_streams(const DecodeArgs &a, uint32_t *sm
         const float cq = floorf(bins * 0.5f) - 1.0f;
         nsym = (cq >= 0.0f && cq < 32768.0f) ? 2 * (int)cq + 1 : lp;
         for (int i = tid; i < lp; i += BS)
-            *(FEW ? few_quots + i : reinterpret_cast<float *>(rows + i * kRow + DecodeLayout<BS, OUT>::kQuot)) =
+            *(FEW || FLOAT ? quots + i : reinterpret_cast<float *>(rows + i * kRow + DecodeLayout<BS, OUT>::kQuot)) =
                 __fdiv_rn(__fsub_rn((float)i, cq), cq);
         const uint16_t *mx = SRC == SRC_LISTED ? static_cast<const uint16_t *>(d.maxima) + id.row * d.maxima_pitch
                                                : a.maxima + id.row * a.sg.g.T + id.t0;
@@ -632,7 +722,17 @@ __device__ __forceinline__ void decode_streams(const DecodeArgs &a, uint32_t *sm
             rowmax[i] = m;
         }
     }
-    special = __syncthreads_or(special);
+    if (FLOAT) {
+        // __syncthreads_or() takes LDS of its own, which would sit in front of the tables
+        const uint64_t voted = __ballot(special);
+        if ((tid & 63) == 0) votes[tid >> 6] = voted != 0;
+        __syncthreads();
+#pragma unroll
+        for (int w = 0; w < BS / 64; ++w) special |= votes[w];
+        special = __builtin_amdgcn_readfirstlane(special);
+    } else {
+        special = __syncthreads_or(special);
+    }
 
     const int64_t stream = (id.sub * a.sg.rows + id.row) * a.sg.nc + id.ch;
     int64_t begin = INT64_MAX;
@@ -671,9 +771,9 @@ __device__ __forceinline__ void decode_streams(const DecodeArgs &a, uint32_t *sm
     s.span = 0;                        // span modulo 2^32: 0 is the full range (see RangeEncoder)
     if constexpr (FEW) {
         s.col = (lds_char *)(rows + 4 * tid);
-        s.quots = (lds_char *)few_quots;
+        s.quots = (lds_char *)quots;
     } else {
-        s.colp = (lds_char *)(rows + 2 * tid);
+        s.colp = FLOAT ? (lds_char *)(2u * (uint32_t)table_column<BS>(tid)) : (lds_char *)(rows + 2 * tid);
         s.lutoff = DecodeLayout<BS, OUT>::kQuot - 2 * tid;
     }
     s.osym = nullptr;
@@ -702,9 +802,9 @@ __device__ __forceinline__ void decode_streams(const DecodeArgs &a, uint32_t *sm
         else decode_few_lane<LOG2, OUT, 0, false>(a, s, id.n, rmp);
     } else {
         const bool last_round = linear_block() >= a.last_round_first;
-        if (safe) decode_lane<BS, LOG2, OUT, 0, true>(a, s, lp, id.n, rmp, last_round);
-        else if (half) decode_lane<BS, LOG2, OUT, 1, false>(a, s, lp, id.n, rmp, last_round);
-        else decode_lane<BS, LOG2, OUT, 0, false>(a, s, lp, id.n, rmp, last_round);
+        if (safe) decode_lane<BS, LOG2, OUT, 0, true, FLOAT>(a, s, lp, id.n, rmp, last_round);
+        else if (half) decode_lane<BS, LOG2, OUT, 1, false, FLOAT>(a, s, lp, id.n, rmp, last_round);
+        else decode_lane<BS, LOG2, OUT, 0, false, FLOAT>(a, s, lp, id.n, rmp, last_round);
     }
 }
 
@@ -713,6 +813,14 @@ __global__ __launch_bounds__(BS) void decode_streams_kernel(DecodeArgs a)
 {
     extern __shared__ uint32_t smem[];
     decode_streams<BS, LOG2, SRC, OUT, false>(a, smem);
+}
+
+// The float search.
+template <int BS, int LOG2, int SRC, int OUT>
+__global__ __launch_bounds__(BS) void decode_float_kernel(DecodeArgs a)
+{
+    extern __shared__ uint32_t smem[];
+    decode_streams<BS, LOG2, SRC, OUT, false, true>(a, smem);
 }
 
 // One wavefront a block, so that few wavefronts spread over the compute units (see decode_few_symbol).

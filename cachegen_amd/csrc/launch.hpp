@@ -479,11 +479,43 @@ size_t decode_few_shmem(int lp) { return (size_t)lp * 64 * sizeof(uint32_t) + (s
 
 size_t decode_shmem(int lp, int block) { return align_up((size_t)lp * block * sizeof(uint16_t), 4) + (size_t)(lp + kSub) * sizeof(float); }
 
+size_t decode_float_shmem(int lp, int block) { return (size_t)lp * block * sizeof(uint16_t) + (size_t)(lp + kSub + block / 64) * sizeof(float); }
+
+// Whether a decode takes the float search (decode_float_kernel): tables of 64 symbols always, of 8, 16 and 32
+// up to sixteen wavefronts a SIMD.  It takes fewer cycles a symbol, but more energy, and a decode of more
+// than some 300 us runs at this GPU's power limit (1400 W), where the energy is what counts: 32 layers x
+// 8192 tokens x 1024 channels at 2.1 instead of 2.3 GHz.  Measured with 32 layers x 1024 channels,
+// decode_streams_kernel / decode_float_kernel, us:
+//   wavefronts a SIMD          4            6            8           12           16           24           32
+//   tables of  8 symbols   73 /  67     86 /  82    107 / 105    175 / 172    224 / 220    320 / 322    416 / 423
+//             16           88 /  72    104 /  92    128 / 121    204 / 194    263 / 252    368 / 368    479 / 483
+//             32          100 /  83    119 / 105    146 / 138    218 / 212    280 / 270    394 / 396    511 / 522
+//             64          122 / 101    199 / 171    231 / 212    343 / 319    452 / 407    656 / 590    861 / 773
+// (the 64-symbol tables leave room for half the wavefronts, which stay below that limit); the same for both
+// layouts of the output.  32 layers x 16384 tokens x 4096 channels, 32 symbols: 3669 / 3846.
+constexpr int64_t kFloatWavefronts = 16;
+bool float_search(int64_t rows, int64_t nc, int64_t nsub, int lp)
+{
+    if (lp == 65) return true;
+    return (lp == 9 || lp == 17 || lp == 33) && rows * ceil_div(nc, 64) * nsub <= (int64_t)compute_units() * 4 * kFloatWavefronts;
+}
+
 // Tables of 2^k symbols (lp = 2^k + 1) take the kernel with the unrolled search.
 template <int BS, int SRC, int OUT>
-void launch_decode_log2(const DecodeArgs &a, dim3 grid, size_t shmem, hipStream_t stream)
+void launch_decode_log2(const DecodeArgs &a, dim3 grid, size_t shmem, hipStream_t stream, bool flt = false)
 {
     const dim3 blk(BS);
+    if constexpr (OUT != OUT_SYMBOLS) {
+        if (flt) {
+            const size_t lds = decode_float_shmem(a.lp, BS);
+            switch (a.lp) {
+            case 9: decode_float_kernel<BS, 3, SRC, OUT><<<grid, blk, lds, stream>>>(a); return;
+            case 17: decode_float_kernel<BS, 4, SRC, OUT><<<grid, blk, lds, stream>>>(a); return;
+            case 33: decode_float_kernel<BS, 5, SRC, OUT><<<grid, blk, lds, stream>>>(a); return;
+            case 65: decode_float_kernel<BS, 6, SRC, OUT><<<grid, blk, lds, stream>>>(a); return;
+            }
+        }
+    }
     switch (a.lp) {
     case 9: decode_streams_kernel<BS, 3, SRC, OUT><<<grid, blk, shmem, stream>>>(a); break;
     case 17: decode_streams_kernel<BS, 4, SRC, OUT><<<grid, blk, shmem, stream>>>(a); break;
@@ -496,11 +528,11 @@ void launch_decode_log2(const DecodeArgs &a, dim3 grid, size_t shmem, hipStream_
 // Whether a decode of these wavefronts is bound by one stream's chain of symbols (decode_few_kernel,
 // blocks of 64): tables of 16 and 32 symbols up to three wavefronts a SIMD, of 64 up to two (its tables
 // of 32-bit entries take 18 KB of LDS a block, so a third round of blocks would wait for the first).  Measured
-// with 32 layers x 1024 channels, decode_streams_kernel / decode_few_kernel, us, one wavefront a SIMD (256
-// tokens), two, three, four, five:
-//   tables of 32 symbols   93 / 49    - / 62    92 / 78   100 / 99   115 / 139
-//   of 16                  82 / 45               84 / 71    89 / 88   102 / 101
-//   of 64                 107 / 55    - / 75   110 / 129  122 / 163
+// with 32 layers x 1024 channels, the form for more wavefronts (decode_float_kernel; below, decode_streams_kernel
+// for one wavefront) / decode_few_kernel, us, one wavefront a SIMD (256 tokens), two, three, four:
+//   tables of 32 symbols   93 / 49    67 / 62    81 / 79    82 / 99
+//   of 16                  82 / 45    59 / 54    71 / 69    71 / 88
+//   of 64                 107 / 55    80 / 74    97 / 129
 // Tables of 8 symbols have no instantiation; other lengths search by bisection.
 int64_t few_wavefronts_a_simd(int lp) { return lp == 17 || lp == 33 ? 3 : lp == 65 ? 2 : 0; }
 bool few_wavefronts(int64_t rows, int64_t nc, int64_t nsub, int lp)
@@ -540,15 +572,16 @@ int launch_decode_kv(DecodeArgs &a, int64_t nblocks, int block, bool few, int ou
     // where registers and LDS allow it, which they do for tables of up to 33 entries)
     const int64_t resident = (int64_t)compute_units() * (2048 / block);
     a.last_round_first = (uint32_t)(nblocks > resident ? nblocks - resident : 0);
+    const bool flt = !few && float_search(a.sg.rows, a.sg.nc, nblocks / (a.sg.rows * a.sg.ctiles), a.lp);
     if (few) {
         if (out_dt == CG_DT_BF16) launch_decode_few<SRC, OUT_BF16>(a, grid, shmem, stream);
         else launch_decode_few<SRC, OUT_F16>(a, grid, shmem, stream);
     } else if (block == 128) {
-        if (out_dt == CG_DT_BF16) launch_decode_log2<128, SRC, OUT_BF16>(a, grid, shmem, stream);
-        else launch_decode_log2<128, SRC, OUT_F16>(a, grid, shmem, stream);
+        if (out_dt == CG_DT_BF16) launch_decode_log2<128, SRC, OUT_BF16>(a, grid, shmem, stream, flt);
+        else launch_decode_log2<128, SRC, OUT_F16>(a, grid, shmem, stream, flt);
     } else {
-        if (out_dt == CG_DT_BF16) launch_decode_log2<64, SRC, OUT_BF16>(a, grid, shmem, stream);
-        else launch_decode_log2<64, SRC, OUT_F16>(a, grid, shmem, stream);
+        if (out_dt == CG_DT_BF16) launch_decode_log2<64, SRC, OUT_BF16>(a, grid, shmem, stream, flt);
+        else launch_decode_log2<64, SRC, OUT_F16>(a, grid, shmem, stream, flt);
     }
     return check_launch("decode_kv");
 }
