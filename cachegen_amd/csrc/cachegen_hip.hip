@@ -345,11 +345,12 @@ struct LevelOut {
 // The level's status word has been set to zero by an earlier launch of the same call.
 // maxima, max_dt: the row maxima (packed symbols only); nibbles: the quantizer packed the rows
 // of at most 15 symbols four bits a symbol (see narrow_alphabet).
-// tables_ready: the tables were written by an earlier launch of the call (quantize_tables_kernel),
-// which also set the workspace's group sums to zero.  may_be_few: false keeps encode_few_kernel out.
+// tables_ready: the tables were written by an earlier launch of the call (quantize_tables_kernel).
+// group_sums: kMaxTileGroups words that an earlier launch of the call set to zero, or null.  may_be_few: false keeps encode_few_kernel out.
 int code_and_compact(const LevelOut &o, const uint32_t *sym4, const uint8_t *sym_bytes, const EncodeWorkspace &w,
                      int64_t L, int64_t T, int64_t C, int64_t chunk_tokens, hipStream_t s,
-                     const void *maxima = nullptr, int max_dt = 0, bool nibbles = false, bool tables_ready = false, bool may_be_few = true)
+                     const void *maxima = nullptr, int max_dt = 0, bool nibbles = false, bool tables_ready = false,
+                     int32_t *group_sums = nullptr, bool may_be_few = true)
 {
     const int64_t rows = 2 * L;
     const int lp = o.max_bins + 1;
@@ -376,10 +377,11 @@ int code_and_compact(const LevelOut &o, const uint32_t *sym4, const uint8_t *sym
     const bool fused_scan = block == kSlotTile && C % kSlotTile == 0;
     a.tile_sums = fused_scan ? w.tile_sums : nullptr;
     // few enough tiles: no scan launch either, the coder's blocks add the counts up by groups of
-    // tiles (the sums were cleared by the quantizer that made the tables) and the compaction adds
-    // up what lies before each tile
-    const bool grouped = fused_scan && tables_ready && ceil_div(w.ntiles, kTileGroup) <= kMaxTileGroups;
-    a.group_sums = grouped ? w.group_sums : nullptr;
+    // tiles (the sums were cleared by the call's quantizer) and the compaction adds up what lies before
+    // each tile: four levels of 32 layers x 4096 tokens x 1024 channels 1164 -> 1153 us, 32 layers x 4096
+    // tokens x 4096 channels 1292 -> 1280 (both through quantize_pack_kernel)
+    const bool grouped = fused_scan && group_sums && ceil_div(w.ntiles, kTileGroup) <= kMaxTileGroups;
+    a.group_sums = grouped ? group_sums : nullptr;
 
     if (sym4) {
         // four tokens per word, read by one lane per channel
@@ -425,7 +427,7 @@ int code_and_compact(const LevelOut &o, const uint32_t *sym4, const uint8_t *sym
         if (int rc = launch_scan(o.lengths, w.nstreams, kStreamCap, o.offsets, w.scan_scratch, s)) return rc;
     }
     const CompactArgs c = {w.scratch, kStreamCap, o.offsets, fused_scan ? o.lengths : nullptr, tile_base, w.nstreams, o.payload,
-                           o.payload_cap, skew, o.status, grouped ? w.group_sums : nullptr, fused_scan ? w.tile_sums : nullptr};
+                           o.payload_cap, skew, o.status, grouped ? group_sums : nullptr, fused_scan ? w.tile_sums : nullptr};
     const dim3 cgrid((unsigned)cblocks);
     if (cblocks <= sliced_compact_blocks()) {
         if (fused_scan) compact_few_kernel<true><<<cgrid, dim3(1024), 0, s>>>(c);
@@ -501,12 +503,13 @@ int encode_kv(const void *kv, int kv_dt, int64_t L, int64_t T, int64_t H, int64_
                                                 reinterpret_cast<uint16_t *>(cdf), w.nsub, chunk_tokens, nibbles, status, shape, s,
                                                 nparts > 1 ? part_tokens : 0, nparts > 1 && part_tokens ? w.scratch : nullptr, slots_bytes,
                                                 w.group_sums)) return rc;
-            return code_and_compact(o, sym4, nullptr, w, L, T, C, chunk_tokens, s, maxima, kv_dt, nibbles, true, may_be_few);
+            return code_and_compact(o, sym4, nullptr, w, L, T, C, chunk_tokens, s, maxima, kv_dt, nibbles, true, w.group_sums, may_be_few);
         }
+        int32_t *const group_sums = w.ntiles > kDirectTiles ? w.group_sums : nullptr;
         if (int rc = launch_quantize_pack(kv, kv_dt, L, T, H, D, sl, skv, st, sh, key_bins, value_bins, sym4,
                                           maxima, w.nsub, chunk_tokens, delta_group, s, status, 0, nullptr, nullptr, 0,
-                                          nibbles, nullptr, max_bins + 1)) return rc;
-        return code_and_compact(o, sym4, nullptr, w, L, T, C, chunk_tokens, s, maxima, kv_dt, nibbles, false, may_be_few);
+                                          nibbles, nullptr, max_bins + 1, group_sums)) return rc;
+        return code_and_compact(o, sym4, nullptr, w, L, T, C, chunk_tokens, s, maxima, kv_dt, nibbles, false, group_sums, may_be_few);
     }
     clear_status_kernel<<<1, 1, 0, s>>>(status);
     if (int rc = launch_quantize(kv, kv_dt, L, T, H, D, sl, skv, st, sh, key_bins, value_bins, w.symbols, maxima, s)) return rc;
@@ -564,20 +567,25 @@ int cg_encode_kv_levels(const void *kv, int kv_dt, int64_t L, int64_t T, int64_t
     hipStream_t s = static_cast<hipStream_t>(stream);
 
     const bool packed = kv_vectorizable(kv, D, C, sl, skv, st, sh) && C % 8 == 0;
+    // the levels' group sums lie where the tiles' running sums would, which such calls do not make
+    static_assert((kDirectTiles + 1) * sizeof(int64_t) >= (size_t)CG_MAX_LEVELS * kMaxTileGroups * sizeof(int32_t), "the levels' group sums fit");
+    int32_t *const group_sums = packed && w.ntiles > kDirectTiles && ceil_div(w.ntiles, kTileGroup) <= kMaxTileGroups
+                                    ? reinterpret_cast<int32_t *>(w.tile_base) : nullptr;
     if (packed) {
         // one pass over the tensor: every row is loaded once, its maximum found once, and its
         // symbols written once per level
         uint32_t *sym4 = reinterpret_cast<uint32_t *>(w.symbols);
         if (int rc = launch_quantize_pack(kv, kv_dt, L, T, H, D, sl, skv, st, sh, nullptr, nullptr, sym4, maxima,
                                           w.nsub, chunk_tokens, 0, s, status, nlevels, key_bins, value_bins,
-                                          (int64_t)(w.symbols_bytes / 4), true, lp_lv)) return rc;
+                                          (int64_t)(w.symbols_bytes / 4), true, lp_lv, 0, group_sums)) return rc;
     }
     for (int v = 0; v < nlevels; ++v) {
         const LevelOut o = {key_bins[v], value_bins[v], max_bins[v], cdf[v], lengths[v], offsets[v],
                             payload[v], payload_cap[v], status + v};
         uint8_t *symbols = w.symbols + (size_t)v * w.symbols_bytes;
         if (packed) {
-            if (int rc = code_and_compact(o, reinterpret_cast<uint32_t *>(symbols), nullptr, w, L, T, C, chunk_tokens, s, maxima, kv_dt, true)) return rc;
+            if (int rc = code_and_compact(o, reinterpret_cast<uint32_t *>(symbols), nullptr, w, L, T, C, chunk_tokens, s, maxima, kv_dt, true, false,
+                                          group_sums ? group_sums + v * kMaxTileGroups : nullptr)) return rc;
         } else {
             // shapes the vector loads cannot take: one plain quantization pass per level
             clear_status_kernel<<<1, 1, 0, s>>>(status + v);

@@ -243,13 +243,16 @@ int launch_quantize_pack(const void *kv, int kv_dt, int64_t L, int64_t T, int64_
                          const float *value_bins, uint32_t *sym4, void *maxima, int64_t nsub,
                          int64_t S, int delta_group, hipStream_t stream, int32_t *status, int nlevels = 0,
                          const float *const *key_bins_lv = nullptr, const float *const *value_bins_lv = nullptr,
-                         int64_t level_words = 0, bool nibbles = false, const int *lp_lv = nullptr, int lp = 0)
+                         int64_t level_words = 0, bool nibbles = false, const int *lp_lv = nullptr, int lp = 0,
+                         int32_t *group_sums = nullptr)
 {
     PackedQuantArgs a;
     memset(&a, 0, sizeof(a));
     // status: one word per level (one word when nlevels == 0), consecutive
     a.nstatus = nlevels > 0 ? nlevels : 1;
     for (int v = 0; v < a.nstatus; ++v) a.status[v] = status + v;
+    a.group_sums = group_sums;          // kMaxTileGroups words per level
+    a.ngroup_sums = group_sums ? kMaxTileGroups * a.nstatus : 0;
     a.nlevels = nlevels;
     for (int v = 0; v < nlevels; ++v) {
         a.key_bins_lv[v] = key_bins_lv[v];

@@ -167,6 +167,9 @@ struct PackedQuantArgs {
     // sets to zero
     int32_t nstatus;
     int32_t *status[kMaxLevels];
+    // and sums that the coder's blocks add to, likewise (may be null)
+    int32_t *group_sums;
+    int32_t ngroup_sums;
     uint32_t *sym4;
     uint16_t *maxima;       // [2L, T]
     int32_t nunits;         // C / 8
@@ -185,7 +188,9 @@ struct PackedQuantArgs {
 // at QUANT_LEVEL 1..3); the maxima do not depend on the level.
 __device__ __forceinline__ void clear_statuses(const PackedQuantArgs &a)
 {
-    if (blockIdx.x == 0 && threadIdx.x < a.nstatus) *a.status[threadIdx.x] = 0;
+    if (blockIdx.x != 0) return;
+    if (threadIdx.x < a.nstatus) *a.status[threadIdx.x] = 0;
+    for (int i = threadIdx.x; i < a.ngroup_sums; i += 256) a.group_sums[i] = 0;
 }
 
 // A row quantized to `maxq` levels either side of zero has the symbols 0 .. 2 maxq: at most
