@@ -344,7 +344,8 @@ class HostPart:
     worth: uint8 tensors `tables`, `lengths`, `payload` as they lie on the device, `maxima` (uint16
     numpy view [2L, tokens]), `sub_bytes` (payload bytes per sub-chunk), tokens [t0, t1).  `symbols`:
     stored symbols per (chunk, row) where `tables` holds histogram counts, else None;
-    `lengths_itemsize` 2 or 4.  Sizes are known from the start; bytes are there after `arrive`."""
+    `lengths_itemsize` 2 or 4.  Sizes are known and the maxima are there from the start; the other
+    bytes are there after `arrive`."""
 
     def table_slices(self):
         """(start, end) slices of `tables`, each there when it is yielded."""
@@ -365,8 +366,8 @@ def bring_to_host(enc, first_chunk, num_chunks, per_chunk=True, compact=False):
     The sections leave the encoder's own tensors for pinned memory as they are; blobs are put
     together on the host, where they have to be written anyway: no second copy of them on the
     device.  The host waits for the device once for the sizes (status, payload offsets, symbol
-    counts, stored into pinned memory by one kernel) while the tables, whose size it knows, are
-    already on the bus, and then for each piece of about _PIECE_BYTES."""
+    counts, stored into pinned memory by one kernel) and the maxima while the tables, whose size it
+    knows, are already on the bus, and then for each piece of about _PIECE_BYTES."""
     import torch
     from .. import _lib, codec, hostmem
     L, H, D, S, T = enc.num_layers, enc.num_heads, enc.head_size, enc.chunk_tokens, enc.num_tokens
@@ -430,7 +431,8 @@ def bring_to_host(enc, first_chunk, num_chunks, per_chunk=True, compact=False):
         with hostmem.StoredWords(3 + nbounds + ngroups, torch.int64) as words:
             _lib.check(lib.cg_wire_meta(enc.status.data_ptr(), enc.offsets[g_first * rows * C:].data_ptr(), rows * C, nbounds,
                                         ptr(wide), ptr(inexact), ptr(nsym), ngroups, words.words.data_ptr(), stream))
-            words.stored()
+            maxima = fetch(enc.maxima)
+            words.stored()                               # one wait for the words and the maxima
             chunk_bytes = max(1, cdf[0].numel() * cdf.element_size() + min(spc, lengths.shape[0]) * rows * C * 4)
             step = max(1, _PIECE_BYTES // chunk_bytes) if per_chunk else 1
             pieces = [(i, min(i + step, len(groups))) for i in range(0, len(groups), step)]
@@ -443,7 +445,6 @@ def bring_to_host(enc, first_chunk, num_chunks, per_chunk=True, compact=False):
             elif not compact:
                 a, b = groups[0][0], groups[pieces[0][1] - 1][1]
                 early = {"tables": fetch_tables(cdf[a - c_first:b - c_first]), "lengths": fetch(lengths[subs(a):subs(b)])}
-            maxima = fetch(enc.maxima)
             meta = words.read()
 
     enc.raise_for_status(meta[0])
