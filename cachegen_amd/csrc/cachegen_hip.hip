@@ -382,6 +382,7 @@ int code_and_compact(const LevelOut &o, const uint32_t *sym4, const uint8_t *sym
     // tokens x 4096 channels 1292 -> 1280 (both through quantize_pack_kernel)
     const bool grouped = fused_scan && group_sums && ceil_div(w.ntiles, kTileGroup) <= kMaxTileGroups;
     a.group_sums = grouped ? group_sums : nullptr;
+    a.last_first = code_last_first(w.ntiles);
 
     if (sym4) {
         // four tokens per word, read by one lane per channel

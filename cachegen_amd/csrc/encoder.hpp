@@ -321,8 +321,10 @@ struct EncodeArgs {
     const float *key_bins, *value_bins;     // float32 [L] each, or null when the levels are not known
     int64_t L;
     StreamGrid sg;
+    int32_t last_first;     // encode_streams_kernel: the last sub-chunk's blocks are the launch's first (code_last_first)
 };
 
+__device__ __forceinline__ uint32_t coder_sub(const EncodeArgs &a) { return a.last_first ? gridDim.z - 1 - blockIdx.z : blockIdx.z; }
 
 // How a packed word holds its four symbols: kBytes, a byte each (any value; kept inside the
 // table where it is used); kNibbles, four bits each, every one a table symbol; kNibblesEscaped,
@@ -347,7 +349,7 @@ __device__ __forceinline__ uint32_t packed_symbol(uint32_t v, int j, uint32_t sm
 // The bytes that the block's streams occupy in the payload, for the compaction.  Every lane of the block
 // is active where this is called (the host asks for tile sums only when a block is exactly one tile).
 template <int BS>
-__device__ __forceinline__ void leave_tile_sum(const EncodeArgs &a, int tid, int len)
+__device__ __forceinline__ void leave_tile_sum(const EncodeArgs &a, uint32_t tile, int tid, int len)
 {
     __shared__ int32_t wave_sums[BS / 64];
     int32_t v = len < a.cap ? len : a.cap;
@@ -358,7 +360,6 @@ __device__ __forceinline__ void leave_tile_sum(const EncodeArgs &a, int tid, int
     if (tid == 0) {
         int32_t total = 0;
         for (int w = 0; w < BS / 64; ++w) total += wave_sums[w];
-        const uint32_t tile = linear_block();
         a.tile_sums[tile] = total;                            // at most 256 streams of 256 bytes
         if (a.group_sums) __hip_atomic_fetch_add(a.group_sums + tile / kTileGroup, total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
@@ -372,7 +373,7 @@ __global__ __launch_bounds__(BS) void encode_streams_kernel(EncodeArgs a)
 {
     extern __shared__ uint16_t tab[];
     const int tid = threadIdx.x;
-    const StreamId id = locate<BS>(a.sg);
+    const StreamId id = locate<BS>(a.sg, coder_sub(a));
     const int lp = a.lp;
     const int64_t ch0 = id.ch - tid;
     uint16_t *col = tab + table_column<BS>(tid);
@@ -498,7 +499,7 @@ __global__ __launch_bounds__(BS) void encode_streams_kernel(EncodeArgs a)
         // the tile, tid the stream's place in it
         enc.init(col, lp);
         enc.w.init(nullptr, 0, a.cap);
-        enc.w.init_tile(__builtin_amdgcn_make_buffer_rsrc((void *)(a.out + (int64_t)linear_block() * ((int64_t)kSlotTile * a.cap)), 0,
+        enc.w.init_tile(__builtin_amdgcn_make_buffer_rsrc((void *)(a.out + (int64_t)linear_block(coder_sub(a)) * ((int64_t)kSlotTile * a.cap)), 0,
                                                           kSlotTile * a.cap, kBufferWord3),
                         (uint32_t)tid * 4u);
     } else if (SLOTS) {
@@ -577,7 +578,7 @@ __global__ __launch_bounds__(BS) void encode_streams_kernel(EncodeArgs a)
     const int len = enc.finish();
     a.lengths[stream] = len;
     if (len > a.cap && a.status) atomicOr(a.status, 1);
-    if (SLOTS && a.tile_sums) leave_tile_sum<BS>(a, tid, len);
+    if (SLOTS && a.tile_sums) leave_tile_sum<BS>(a, linear_block(coder_sub(a)), tid, len);
 }
 
 }  // namespace

@@ -357,7 +357,7 @@ __global__ __launch_bounds__(BS) void encode_few_kernel(EncodeArgs a)
     const int len = enc.finish();
     a.lengths[stream] = len;
     if (len > a.cap && a.status) atomicOr(a.status, 1);
-    if (SLOTS && a.tile_sums) leave_tile_sum<BS>(a, tid, len);
+    if (SLOTS && a.tile_sums) leave_tile_sum<BS>(a, linear_block(), tid, len);
 }
 
 }  // namespace

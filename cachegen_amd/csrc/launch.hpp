@@ -461,6 +461,16 @@ int launch_encode(const EncodeArgs &a, dim3 grid, bool few, hipStream_t stream)
     return check_launch("encode");
 }
 
+// Whether the coder begins with the last sub-chunk: the compaction behind it begins with the first, and so
+// finds what the coder wrote last in the last-level cache (256 MB; the scratch of 8192 tiles is 0.22 GB of
+// partial lines) instead of pushing it out before it gets there.  Forward / last first, 32 layers x 1024
+// channels, us: 4096 tokens (4096 tiles), tables of 65 entries 904 / 896, four levels 1157 / 1153; 8192 tokens
+// 659 / 652, under one table 676 / 654; 12288 tokens 948 / 939, 16384 tokens 1286 / 1286; 8192 tokens x 4096
+// channels (32768 tiles) 2551-2573 / 2535-2546; up to 2048 tokens, whose scratch the cache holds anyway, no
+// difference.  80 layers x 32768 tokens (83840 tiles, of which it holds a tenth) 6220-6250 / 6240-6350.  Rows
+// outermost as well (the quantizer's order, mirrored) is slower: four levels 1186.
+bool code_last_first(int64_t ntiles) { return ntiles <= 32768; }
+
 // Tiles up to which the compaction deals a stream's words to four threads (compact_few_kernel): four a
 // compute unit.  16 tiles 16.9 -> 8.6 us, 256 tiles 12.2 -> 7.4; at 1024 tiles (32 layers x 1024 channels x
 // 1024 tokens) the encode takes 116.3 / 116.0 us, at 768 99.3 / 98.1.

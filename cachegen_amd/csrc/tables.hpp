@@ -398,11 +398,11 @@ struct StreamId {
 
 // The grid is (channel tile, row, sub-chunk): a block reads its place from its index.
 template <int BS>
-__device__ __forceinline__ StreamId locate(const StreamGrid &sg)
+__device__ __forceinline__ StreamId locate(const StreamGrid &sg, uint32_t sub = blockIdx.z)
 {
     StreamId s;
     s.row = blockIdx.y;
-    s.sub = blockIdx.z;
+    s.sub = sub;
     sub_range(sg.g, s.sub, s.chunk, s.t0, s.n);
     s.ch = (int64_t)blockIdx.x * BS + threadIdx.x;
     s.active = s.ch < sg.nc;
@@ -411,9 +411,9 @@ __device__ __forceinline__ StreamId locate(const StreamGrid &sg)
 
 // The block's number in the order (sub-chunk, row, channel tile), in which tiles of the encoder's
 // scratch and their byte counts are laid out.
-__device__ __forceinline__ uint32_t linear_block()
+__device__ __forceinline__ uint32_t linear_block(uint32_t sub = blockIdx.z)
 {
-    return (blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
+    return (sub * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
 }
 
 }  // namespace
