@@ -495,7 +495,7 @@ size_t decode_shmem(int lp, int block) { return align_up((size_t)lp * block * si
 size_t decode_float_shmem(int lp, int block) { return (size_t)lp * block * sizeof(uint16_t) + (size_t)(lp + kSub + block / 64) * sizeof(float); }
 
 // Whether a decode takes the float search (decode_float_kernel): tables of 64 symbols always, of 8, 16 and 32
-// up to sixteen wavefronts a SIMD.  It takes fewer cycles a symbol, but more energy, and a decode of more
+// up to twelve wavefronts a SIMD.  It takes fewer cycles a symbol, but more energy, and a decode of more
 // than some 300 us runs at this GPU's power limit (1400 W), where the energy is what counts: 32 layers x
 // 8192 tokens x 1024 channels at 2.1 instead of 2.3 GHz.  Measured with 32 layers x 1024 channels,
 // decode_streams_kernel / decode_float_kernel, us:
@@ -504,9 +504,11 @@ size_t decode_float_shmem(int lp, int block) { return (size_t)lp * block * sizeo
 //             16           88 /  72    104 /  92    128 / 121    204 / 194    263 / 252    368 / 368    479 / 483
 //             32          100 /  83    119 / 105    146 / 138    218 / 212    280 / 270    394 / 396    511 / 522
 //             64          122 / 101    199 / 171    231 / 212    343 / 319    452 / 407    656 / 590    861 / 773
+// On other data (bench.py's four levels of 4096 tokens, sixteen wavefronts) 8, 16, 32 symbols 247 / 252, 271 / 274,
+// 285 / 288, 64 symbols 450 / 406: the line is below sixteen.
 // (the 64-symbol tables leave room for half the wavefronts, which stay below that limit); the same for both
 // layouts of the output.  32 layers x 16384 tokens x 4096 channels, 32 symbols: 3669 / 3846.
-constexpr int64_t kFloatWavefronts = 16;
+constexpr int64_t kFloatWavefronts = 12;
 bool float_search(int64_t rows, int64_t nc, int64_t nsub, int lp)
 {
     if (lp == 65) return true;

@@ -1,6 +1,6 @@
-"""Decodes on both sides of the line between decode_float_kernel and decode_streams_kernel (sixteen
+"""Decodes on both sides of the line between decode_float_kernel and decode_streams_kernel (twelve
 wavefronts a SIMD, tables of 64 symbols never the latter): the same streams decoded in one large call
-and in calls of a few to sixteen wavefronts a SIMD give the same bits."""
+and in calls of a few to twelve wavefronts a SIMD give the same bits."""
 import pytest
 import torch
 
@@ -20,7 +20,7 @@ def wavefronts(per_simd):
 def test_large_and_smaller_decodes_agree(bins, H, D, fmt):
     L = 24 if H > 1 else 120
     per_sub = 2 * L * -(-H * D // 64)
-    nsub = wavefronts(16) // per_sub + 1                       # the least sub-chunks of the large side
+    nsub = wavefronts(12) // per_sub + 1                       # the least sub-chunks of the large side
     T = (nsub - 1) * 256 + 77
     gen = torch.Generator(DEV).manual_seed(4)
     spread = torch.rand(L, 2, 1, H, D, device=DEV, generator=gen) ** 4 + 0.01     # quiet channels and loud ones
