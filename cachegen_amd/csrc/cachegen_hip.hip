@@ -149,7 +149,7 @@ int cg_encode_fast_new(const int16_t *cdf, int lp, const int8_t *sym, int64_t nl
     const dim3 grid = stream_grid(a.sg, nblocks);
     if (aligned) {
         // that form reaches a channel from its token row with a 32-bit offset
-        const bool few = few_encode(nblocks, block, kFewEncodeBytes) && s2 >= 0 && s2 <= 0x7FFFFFFFll / nc;
+        const bool few = few_encode(nblocks, ENC_BYTES, lp, block, false) && s2 >= 0 && s2 <= 0x7FFFFFFFll / nc;
         CG_DISPATCH_BS(block, return (launch_encode<BS, true, false, false, false>(a, grid, few, st)));
     }
     const size_t shmem = (size_t)lp * (block + 2) * sizeof(uint16_t);      // TableStride<BS>::k16 per entry
@@ -390,9 +390,10 @@ int code_and_compact(const LevelOut &o, const uint32_t *sym4, const uint8_t *sym
         a.nibbles = nibbles ? 1 : 0;
         a.maxima = static_cast<const uint16_t *>(maxima);
         a.max_dt = max_dt;
-        const bool few = may_be_few && few_encode(nblocks, block, kFewEncodePacked);
+        const EncodeSource source = tables_ready ? ENC_QUANTIZER_TABLES : chunk_tokens <= kSub ? ENC_COUNTED : ENC_TABLES;
+        const bool few = may_be_few && few_encode(nblocks, source, lp, block, fused_scan);
         int rc = CG_OK;
-        if (!tables_ready && chunk_tokens <= kSub) {
+        if (source == ENC_COUNTED) {
             // one sub-chunk per chunk: the encoder builds the tables itself
             if (fused_scan) rc = launch_encode<kSlotTile, true, true, true, true, true>(a, grid, few, s);
             else CG_DISPATCH_BS(block, rc = (launch_encode<BS, true, true, true, true>(a, grid, few, s)));
@@ -539,6 +540,12 @@ int cg_test_encode_kv(const void *kv, int kv_dt, int64_t L, int64_t T, int64_t H
 {
     return encode_kv(kv, kv_dt, L, T, H, D, sl, skv, st, sh, key_bins, value_bins, max_bins, chunk_tokens, delta_group,
                      cdf, maxima, lengths, offsets, payload, payload_cap, status, workspace, workspace_bytes, stream, flags);
+}
+
+int cg_test_few_encode_blocks(int source, int lp, int block, int tile)
+{
+    if (source < ENC_BYTES || source > ENC_QUANTIZER_TABLES || lp < 2 || lp > CG_MAX_LP || (block != 64 && block != 128 && block != 256)) return -1;
+    return (int)few_encode_blocks(static_cast<EncodeSource>(source), lp, block, tile != 0);
 }
 
 int cg_encode_kv_levels(const void *kv, int kv_dt, int64_t L, int64_t T, int64_t H, int64_t D, int64_t sl,

@@ -428,21 +428,66 @@ int launch_quantize_tables(const void *kv, int kv_dt, int64_t L, int64_t T, int6
     return launch_quantize_tables_shape<CG_DT_BF16, false>(a, shape, grid, stream);
 }
 
-// Whether an encode of these wavefronts is bound by one stream's chain of symbols (encode_few_kernel):
-// up to two a SIMD, which is what the registers for a sub-chunk's symbols leave room for, three where
-// the symbols are bytes (fewer registers).  Measured with 32 layers x 1024 channels, encode_streams_kernel /
-// encode_few_kernel, the whole call, us, one wavefront a SIMD (256 tokens), two, three, four:
-//   tables in the coder or the quantizer      71.5 / 60.8   82.0 / 75.3    98.6 / 105.9  116.3 / 127.0
-//   tables of 65 entries                       86 / 77      103.1 / 101.4
-//   one table, counted by a pass of its own         -        88.1 / 88.4   109.3 / 119.6
-// byte symbols, the reference's four functions on 256 tokens x 1024 channels: 32 layers (one a SIMD) 182 / 166,
-// 50 layers (1.6) 204 / 188, 80 (2.5) 228 / 222.
-bool few_encode(int64_t nblocks, int block, int most)
+// Where the symbols and tables of an encode come from.
+enum EncodeSource {
+    ENC_BYTES,              // byte symbols, tables in memory (the reference's entry point)
+    ENC_COUNTED,            // packed symbols, tables made by the coder
+    ENC_TABLES,             // packed symbols, tables made by a pass of their own
+    ENC_QUANTIZER_TABLES,   // packed symbols, tables made by the quantizer
+};
+
+// Wavefronts a compute unit up to which an encode is bound by one stream's chain of symbols
+// (encode_few_kernel).  tile: every block is a whole tile of the scratch (TILE).  Measured on make_kv's caches,
+// encode_streams_kernel / encode_few_kernel, the whole call in a graph, us, by wavefronts a SIMD (a quarter of a unit's):
+//   1024 channels, tables of      17           33           41           65           97          129 entries
+//   byte symbols        1      51 /  29     52 /  38     53 /  42     58 /  49     67 /  60     70 /  61
+//   (256 tokens)        1.5    54 /  38     57 /  46     57 /  52     62 /  60     67 /  63     70 / 104
+//                       2      55 /  39     58 /  48     58 /  54     63 /  61     69 / 105     72 / 115
+//                       2.5    61 /  48     64 /  59     64 /  66     71 /  94     76 / 120    132 / 150
+//                       3      62 /  49     65 /  60     67 /  67     73 / 102     86 / 126    139 / 168
+//   tables by the       0.5    56 /  42     64 /  52     68 /  58     72 /  63     82 /  81     86 /  84
+//   coder (256 tokens)  1      63 /  48     71 /  57     74 /  63     78 /  68     93 /  94     97 /  98
+//                       1.5    69 /  59     76 /  67     79 /  73     86 /  82     99 / 103    105 / 144
+//                       2      76 /  65     85 /  77     87 /  82     94 /  91    109 / 149    114 / 165
+//   by a pass of their  1      63 /  54     70 /  66     74 /  70     79 /  76     96 / 102    103 / 110
+//   own (512 tokens)    1.5    71 /  65     78 /  79     81 /  85     92 /  96    105 / 113    113 / 159
+//                       2      76 /  71     87 /  88     92 /  96    101 / 105    114 / 158    123 / 176
+//   by the quantizer    1      75 /  65     81 /  75                  90 /  88
+//                       2      80 /  74     87 /  87                 101 / 105
+//   400, 128, 64 channels (blocks of 256, 128, 64 lanes), packed symbols, at the line taken and above it:
+//   by the coder        25 entries: 400  89 / 82 at 2;  128  97 / 94 at 1, 108 / 110 at 1.25;  64  93 / 90 at 0.5, 120 / 121 at 1
+//                       65 entries: 400  87 / 81 at 1, 92 / 92 at 1.25
+//   by a pass           17 entries: 400  85 / 82 at 2;  128  94 / 93 at 1, 109 / 109 at 1.5;  64  79 / 80 at 0.25
+//                       29 entries: 400  80 / 79 at 1, 85 / 88 at 1.25;  33 entries: 400  70 / 71 at 0.25, 80 / 81 at 1
+//   by the quantizer    17 entries: 400  79 / 74 at 2;  128  85 / 80 at 1, 110 / 111 at 2;  64  81 / 80 at 0.5, 106 / 107 at 1
+//                       33 entries: 400  82 / 81 at 1, 82 / 86 at 1.25;  128  82 / 85 at 0.25
+//   byte symbols of 64 channels and 25 to 29 entries, the worst of that form: 65 / 69 at 2.25, 71 / 73 at 2.5, 74 / 74 at 3
+// (the last column of byte symbols is 128 entries).  Longer tables cost encode_few_kernel more: it copies
+// those that are in memory entry by entry, at twice the width.
+int few_encode_wavefronts(EncodeSource source, int lp, int block, bool tile)
 {
-    return nblocks <= (int64_t)compute_units() * 4 * most / (block / 64);
+    if (source == ENC_BYTES) return lp <= 33 ? 12 : 8;
+    if (source == ENC_COUNTED) return lp > 80 || block == 64 ? 2 : block == 128 || (lp > 33 && !tile) ? 4 : 8;
+    if (tile) return lp <= (source == ENC_TABLES ? 17 : 33) ? 8 : 4;
+    if (block == 256) return lp <= 17 ? 8 : lp <= (source == ENC_TABLES ? 29 : 33) ? 4 : 0;
+    return block == 128 && lp <= 17 ? 4 : 0;
 }
 
-constexpr int kFewEncodePacked = 2, kFewEncodeBytes = 3;
+// Blocks a compute unit up to which it is taken: those wavefronts, and no more than its LDS holds at once,
+// or a second round of blocks waits for the first (65 entries from byte symbols, blocks of 65 KB, two a
+// unit: 61 us for two wavefronts a SIMD, 91 for 2.25).  LDS is given out by 1280 bytes (of blocks of 53 x 1024
+// bytes a unit holds two, not three); a block of packed symbols has 272 besides its tables.
+int64_t few_encode_blocks(EncodeSource source, int lp, int block, bool tile)
+{
+    const size_t lds = align_up((size_t)lp * block * sizeof(uint32_t) + (source == ENC_BYTES ? 0 : 272), 1280);
+    const int64_t fit = (int64_t)(kMaxLdsPerBlock / lds), chain = (int64_t)few_encode_wavefronts(source, lp, block, tile) * 64 / block;
+    return fit < chain ? fit : chain;
+}
+
+bool few_encode(int64_t nblocks, EncodeSource source, int lp, int block, bool tile)
+{
+    return nblocks <= (int64_t)compute_units() * few_encode_blocks(source, lp, block, tile);
+}
 
 template <int BS, bool ALIGNED, bool PACKED, bool FUSE_CDF, bool SLOTS, bool TILE = false>
 int launch_encode(const EncodeArgs &a, dim3 grid, bool few, hipStream_t stream)

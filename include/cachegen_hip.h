@@ -183,6 +183,12 @@ int cg_test_encode_kv(const void *kv, int kv_dt, int64_t L, int64_t T, int64_t H
                       uint8_t *payload, int64_t payload_cap, int32_t *status,
                       void *workspace, size_t workspace_bytes, void *stream, int flags);
 
+/* Test hook, no GPU work: blocks of `block` (64, 128 or 256) lanes a compute unit up to which an encode with
+ * tables of lp entries takes the coder's form for few wavefronts; -1 for arguments out of range.
+ * source: 0 byte symbols, 1 packed symbols with tables made by the coder, 2 by a pass of their own, 3 by
+ * the quantizer.  tile: the channels are a multiple of 256 and a block is 256 lanes. */
+int cg_test_few_encode_blocks(int source, int lp, int block, int tile);
+
 /* The same KV cache encoded at `nlevels` quantization levels from ONE read of the tensor: the
  * adaptive-streaming use of the reference, which pre-encodes every chunk at QUANT_LEVEL 1..3
  * by calling the serializer once per level (run_adaptation.py:63-72, src/utils.py:357-377).
