@@ -150,7 +150,7 @@ int cg_encode_fast_new(const int16_t *cdf, int lp, const int8_t *sym, int64_t nl
     if (aligned) {
         // that form reaches a channel from its token row with a 32-bit offset
         const bool few = few_encode(nblocks, ENC_BYTES, lp, block, false) && s2 >= 0 && s2 <= 0x7FFFFFFFll / nc;
-        CG_DISPATCH_BS(block, return (launch_encode<BS, true, false, false, false>(a, grid, few, st)));
+        CG_DISPATCH_BS(block, return (launch_encode<BS, false, false, false>(a, grid, few, st)));
     }
     const size_t shmem = (size_t)lp * (block + 2) * sizeof(uint16_t);      // TableStride<BS>::k16 per entry
     CG_DISPATCH_BS(block, (encode_streams_kernel<BS, false, false, false, false><<<grid, dim3(block), shmem, st>>>(a)));
@@ -395,15 +395,15 @@ int code_and_compact(const LevelOut &o, const uint32_t *sym4, const uint8_t *sym
         int rc = CG_OK;
         if (source == ENC_COUNTED) {
             // one sub-chunk per chunk: the encoder builds the tables itself
-            if (fused_scan) rc = launch_encode<kSlotTile, true, true, true, true, true>(a, grid, few, s);
-            else CG_DISPATCH_BS(block, rc = (launch_encode<BS, true, true, true, true>(a, grid, few, s)));
+            if (fused_scan) rc = launch_encode<kSlotTile, true, true, true, true>(a, grid, few, s);
+            else CG_DISPATCH_BS(block, rc = (launch_encode<BS, true, true, true>(a, grid, few, s)));
         } else {
             if (!tables_ready)
                 rc = launch_cdf(nullptr, sym4, w.nsub, rows, T, C, 0, 0, 0, o.max_bins, chunk_tokens, tables, s,
                                 nibbles ? o.key_bins : nullptr, nibbles ? o.value_bins : nullptr);
             if (rc) return rc;
-            if (fused_scan) rc = launch_encode<kSlotTile, true, true, false, true, true>(a, grid, few, s);
-            else CG_DISPATCH_BS(block, rc = (launch_encode<BS, true, true, false, true>(a, grid, few, s)));
+            if (fused_scan) rc = launch_encode<kSlotTile, true, false, true, true>(a, grid, few, s);
+            else CG_DISPATCH_BS(block, rc = (launch_encode<BS, true, false, true>(a, grid, few, s)));
         }
         if (rc) return rc;
     } else {

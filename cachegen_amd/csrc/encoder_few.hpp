@@ -25,7 +25,7 @@ namespace {
 // the loads and the tables, the rest the launch and the last wavefront.
 // The stream is the same number, written the same way (see encoder.hpp): the interval's lower end with
 // its carries.
-template <int BS, bool ALIGNED, bool TILE>
+template <int BS, bool TILE>
 struct FewEncoder {
     static constexpr int kRow = 4 * BS;     // bytes of a row of the tables: entry e << 16 of lane c at word e * BS + c
     lds_char *col;          // this lane's entry 0
@@ -36,7 +36,7 @@ struct FewEncoder {
     uint32_t waiting;       // at most 31 after take_words()
     uint32_t cache;         // the last complete word, not yet written: a carry may still reach it
     uint32_t ones;          // words of all ones that follow it
-    WordWriter<ALIGNED, TILE> w;
+    WordWriter<true, TILE> w;
 
     __device__ __forceinline__ void init(const uint32_t *column, int lp)
     {
@@ -151,8 +151,8 @@ struct FewEncoder {
     }
 };
 
-// The forms and arguments of encode_streams_kernel.
-template <int BS, bool ALIGNED, bool PACKED, bool FUSE_CDF, bool SLOTS, bool TILE = false>
+// The forms and arguments of encode_streams_kernel; streams begin at multiples of four bytes.
+template <int BS, bool PACKED, bool FUSE_CDF, bool SLOTS, bool TILE = false>
 __global__ __launch_bounds__(BS) void encode_few_kernel(EncodeArgs a)
 {
     extern __shared__ uint32_t entries[];
@@ -273,7 +273,7 @@ __global__ __launch_bounds__(BS) void encode_few_kernel(EncodeArgs a)
     asm volatile("" ::: "memory");          // LDS serves a wavefront's accesses in order
     if (!id.active) return;
 
-    FewEncoder<BS, ALIGNED, TILE> enc;
+    FewEncoder<BS, TILE> enc;
     const int64_t stream = (id.sub * a.sg.rows + id.row) * a.sg.nc + id.ch;
     enc.init(col, lp);
     if (TILE) {

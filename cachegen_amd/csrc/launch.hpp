@@ -489,19 +489,20 @@ bool few_encode(int64_t nblocks, EncodeSource source, int lp, int block, bool ti
     return nblocks <= (int64_t)compute_units() * few_encode_blocks(source, lp, block, tile);
 }
 
-template <int BS, bool ALIGNED, bool PACKED, bool FUSE_CDF, bool SLOTS, bool TILE = false>
+// Output buffers whose streams begin at multiples of four bytes.
+template <int BS, bool PACKED, bool FUSE_CDF, bool SLOTS, bool TILE = false>
 int launch_encode(const EncodeArgs &a, dim3 grid, bool few, hipStream_t stream)
 {
     if (few) {
         static std::atomic<uint64_t> asked{0};          // per form of the kernel: these are templates
         const size_t lds = (size_t)a.lp * BS * sizeof(uint32_t);
         if (lds > 64 * 1024)
-            if (int rc = allow_dynamic_lds(reinterpret_cast<const void *>(&encode_few_kernel<BS, ALIGNED, PACKED, FUSE_CDF, SLOTS, TILE>),
+            if (int rc = allow_dynamic_lds(reinterpret_cast<const void *>(&encode_few_kernel<BS, PACKED, FUSE_CDF, SLOTS, TILE>),
                                            CG_MAX_LP * BS * (int)sizeof(uint32_t), asked)) return rc;
-        encode_few_kernel<BS, ALIGNED, PACKED, FUSE_CDF, SLOTS, TILE><<<grid, dim3(BS), lds, stream>>>(a);
+        encode_few_kernel<BS, PACKED, FUSE_CDF, SLOTS, TILE><<<grid, dim3(BS), lds, stream>>>(a);
     } else {
         const size_t lds = (size_t)a.lp * TableStride<BS>::k16 * sizeof(uint16_t);
-        encode_streams_kernel<BS, ALIGNED, PACKED, FUSE_CDF, SLOTS, TILE><<<grid, dim3(BS), lds, stream>>>(a);
+        encode_streams_kernel<BS, true, PACKED, FUSE_CDF, SLOTS, TILE><<<grid, dim3(BS), lds, stream>>>(a);
     }
     return check_launch("encode");
 }
@@ -576,11 +577,16 @@ void launch_decode_log2(const DecodeArgs &a, dim3 grid, size_t shmem, hipStream_
             }
         }
     }
+    if constexpr (OUT == OUT_SYMBOLS) {
+        if (a.lp == 65) {
+            decode_streams_kernel<BS, 6, SRC, OUT><<<grid, blk, shmem, stream>>>(a);
+            return;
+        }
+    }
     switch (a.lp) {
     case 9: decode_streams_kernel<BS, 3, SRC, OUT><<<grid, blk, shmem, stream>>>(a); break;
     case 17: decode_streams_kernel<BS, 4, SRC, OUT><<<grid, blk, shmem, stream>>>(a); break;
     case 33: decode_streams_kernel<BS, 5, SRC, OUT><<<grid, blk, shmem, stream>>>(a); break;
-    case 65: decode_streams_kernel<BS, 6, SRC, OUT><<<grid, blk, shmem, stream>>>(a); break;
     default: decode_streams_kernel<BS, -1, SRC, OUT><<<grid, blk, shmem, stream>>>(a); break;
     }
 }

@@ -105,13 +105,8 @@ __device__ __forceinline__ void normalize_counts(int lp, uint32_t scale, uint32_
         const int sh = total ? 31 - __builtin_clz(total) : 0;
         walk([&](uint32_t x) { return x >> sh; });
     } else {
-        // the float estimate of the quotient, below 2^16, is off by one at most
         const float inv = __fdiv_rn(1.0f, (float)total);
-        walk([&](uint32_t x) {
-            const uint32_t q = (uint32_t)((float)x * inv);
-            const int32_t rem = (int32_t)(x - q * total);
-            return rem < 0 ? q - 1u : rem >= (int32_t)total ? q + 1u : q;
-        });
+        walk([&](uint32_t x) { return divide16(x, total, inv); });
     }
 }
 
