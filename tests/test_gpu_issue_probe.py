@@ -27,3 +27,15 @@ def test_clock_window_ends_and_reports():
     torch.cuda.synchronize()
     mhz, us = issue_probe.clock_window_result()
     assert 1900.0 <= us < 200000.0 and 500.0 < mhz < 3000.0
+
+
+def test_pairs_and_chains():
+    from cachegen_amd import issue_probe
+    torch.zeros(1, device="cuda:0")
+    ops = issue_probe.ops()
+    add, fma, mul_hi = (ops.index(name) for name in ("v_add_u32", "v_fma_f32", "v_mul_hi_u32"))
+    issue_probe.pair(add, add)
+    together, apart = issue_probe.pair(fma, add), issue_probe.pair(mul_hi, add)
+    assert 3.5 < together < 6.5 < apart < 10.0 and abs(issue_probe.pair(add, mul_hi) - apart) < 1.0
+    chains = issue_probe.chains()
+    assert len(chains) == 7 and all(2.0 < cycles < 200.0 for cycles in chains.values())
