@@ -68,12 +68,11 @@ def test_byte_symbols_on_both_sides(lp):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("top", [16, 32, 64, 79, 96, 128])
-@pytest.mark.parametrize("source,T,S,flags", [(COUNTED, 90, 256, 0), (TABLES, 300, 300, 4), (QUANTIZER_TABLES, 90, 256, 2)])
+@pytest.mark.parametrize("source,T,S,flags,top", [(COUNTED, 90, 256, 0, t) for t in (16, 32, 64, 79, 96, 128)] +
+                         [(TABLES, 300, 300, 4, t) for t in (16, 32, 64, 79, 96, 128)] +
+                         [(QUANTIZER_TABLES, 90, 256, 2, t) for t in (16, 32, 64)])
 @pytest.mark.parametrize("H,D", [(4, 64), (5, 80), (1, 128), (1, 64)])       # a whole tile, blocks of 256, 128 and 64 lanes
-def test_packed_symbols_on_both_sides(top, source, T, S, flags, H, D):
-    if source == QUANTIZER_TABLES and top not in (16, 32, 64):
-        pytest.skip("the quantizer makes tables of up to 65 entries")
+def test_packed_symbols_on_both_sides(source, T, S, flags, top, H, D):
     C = H * D
     block = 64 if C == 64 else 128 if C == 128 or top >= 80 else 256
     per_layer = 2 * -(-C // block) * -(-T // 256)
