@@ -477,9 +477,9 @@ __device__ __forceinline__ void decode_lane(const DecodeArgs &a, DecodeLane &s, 
 }
 
 // ---- calls of few wavefronts ---------------------------------------------------------
-// Such a call lasts as long as one stream's chain of symbols.  A wavefront alone on its SIMD issues an
-// instruction every 5 cycles and waits 54 for an LDS round trip, but 35 to 45 at every branch on a mask
-// that a vector instruction made (all measured).  decode_lane takes two such branches a symbol (its one
+// Such a call lasts as long as one stream's chain of symbols.  A wavefront alone on its SIMD issues a
+// dependent instruction every 4.5 to 7 cycles and waits 49 for an LDS round trip, but 36 at every branch on a mask
+// that a vector instruction made (issue_probe.hip).  decode_lane takes two such branches a symbol (its one
 // test, bits that run out) and four or five round trips; here
 //   - the search compares exact products, so nothing is tested: it holds every fourth entry of the
 //     table's part that the row uses, halves them by selects until four candidates are left, and

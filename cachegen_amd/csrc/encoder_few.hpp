@@ -9,8 +9,8 @@
 namespace {
 
 // A call of few wavefronts lasts as long as one stream's chain of symbols.  One wavefront alone on its
-// SIMD issues an instruction every 5 cycles and waits 54 for an LDS round trip, but 35 to 45 at every branch on
-// a mask that a vector instruction made (all measured): encode_streams_kernel, which takes two or
+// SIMD issues a dependent instruction every 4.5 to 7 cycles and waits 49 for an LDS round trip, but 36 at every branch
+// on a mask that a vector instruction made (issue_probe.hip): encode_streams_kernel, which takes two or
 // three such branches a symbol (bits that do not fit, a carry that runs far, the store code) and
 // reads a symbol's table entries when it comes to code it, takes 330 cycles a symbol alone.  Here
 //   - four symbols are coded without a branch: their bits are counted, and if a lane has more than

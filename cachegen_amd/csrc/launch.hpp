@@ -540,20 +540,20 @@ size_t decode_shmem(int lp, int block) { return align_up((size_t)lp * block * si
 
 size_t decode_float_shmem(int lp, int block) { return (size_t)lp * block * sizeof(uint16_t) + (size_t)(lp + kSub + block / 64) * sizeof(float); }
 
-// Whether a decode takes the float search (decode_float_kernel): tables of 64 symbols always, of 8, 16 and 32
-// up to twelve wavefronts a SIMD.  It takes fewer cycles a symbol, but more energy, and a decode of more
-// than some 300 us runs at this GPU's power limit (1400 W), where the energy is what counts: 32 layers x
-// 8192 tokens x 1024 channels at 2.1 instead of 2.3 GHz.  Measured with 32 layers x 1024 channels,
-// decode_streams_kernel / decode_float_kernel, us:
+// Whether a dequantising decode takes the float search (decode_float_kernel): tables of 64 symbols always, of
+// 8, 16 and 32 up to twelve wavefronts a SIMD.  It takes fewer cycles a symbol, but more energy, and a large
+// decode runs within some 10 to 40 W of this GPU's power limit (1400 W), where the energy is what counts:
+// 32 layers x 8192 tokens x 1024 channels 519 us at 2.34 GHz / 546 at 2.19, x 16384 tokens x 4096 channels
+// 3822 at 2.26 / 4051 at 2.04.  (Tables of 64 symbols leave room for half the wavefronts, which stay below
+// that limit: 1332 W at 2.39 GHz.)  The same for both layouts of the output.  Measured with 32 layers x 1024
+// channels, decode_streams_kernel / decode_float_kernel, us:
 //   wavefronts a SIMD          4            6            8           12           16           24           32
 //   tables of  8 symbols   73 /  67     86 /  82    107 / 105    175 / 172    224 / 220    320 / 322    416 / 423
 //             16           88 /  72    104 /  92    128 / 121    204 / 194    263 / 252    368 / 368    479 / 483
 //             32          100 /  83    119 / 105    146 / 138    218 / 212    280 / 270    394 / 396    511 / 522
 //             64          122 / 101    199 / 171    231 / 212    343 / 319    452 / 407    656 / 590    861 / 773
 // On other data (bench.py's four levels of 4096 tokens, sixteen wavefronts) 8, 16, 32 symbols 247 / 252, 271 / 274,
-// 285 / 288, 64 symbols 450 / 406: the line is below sixteen.
-// (the 64-symbol tables leave room for half the wavefronts, which stay below that limit); the same for both
-// layouts of the output.  32 layers x 16384 tokens x 4096 channels, 32 symbols: 3669 / 3846.
+// 285 / 288, 64 symbols 450 / 406: the line is below sixteen.  Calls with symbol output have no such form.
 constexpr int64_t kFloatWavefronts = 12;
 bool float_search(int64_t rows, int64_t nc, int64_t nsub, int lp)
 {
@@ -599,6 +599,13 @@ void launch_decode_log2(const DecodeArgs &a, dim3 grid, size_t shmem, hipStream_
 //   tables of 32 symbols   93 / 49    67 / 62    81 / 79    82 / 99
 //   of 16                  82 / 45    59 / 54    71 / 69    71 / 88
 //   of 64                 107 / 55    80 / 74    97 / 129
+// Symbol output (rows of 1024 channels, 256 tokens; decode_streams_kernel / decode_few_kernel), where there is no
+// float search, by wavefronts a SIMD:
+//                          1          2          2.125       2.5         3          3.5         4
+//   tables of 16 symbols   77 / 43    81 / 55    90 / 68     89 / 71     90 / 72    99 / 90    101 / 93
+//   of 32                  86 / 48    88 / 61    96 / 76     97 / 80     98 / 80   108 / 102   110 / 103
+//   of 64                  97 / 53   103 / 73   113 / 115   113 / 131   114 / 141  126 / 174   128 / 179
+// The same lines do for both: symbols spread evenly over the alphabet take 89.6 / 86.3 at 3.25 and 90.8 / 96.3 at four for 16.
 // Tables of 8 symbols have no instantiation; other lengths search by bisection.
 int64_t few_wavefronts_a_simd(int lp) { return lp == 17 || lp == 33 ? 3 : lp == 65 ? 2 : 0; }
 bool few_wavefronts(int64_t rows, int64_t nc, int64_t nsub, int lp)
