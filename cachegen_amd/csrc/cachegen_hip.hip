@@ -273,9 +273,11 @@ int cg_scan_lengths_static(const int32_t *lengths, int64_t n, int64_t *offsets, 
 namespace {
 
 // Workspace of the fused encoder, carved in this order: `nlevels` symbol areas (a 256-token
-// slot per stream each), the coder's scratch tiles, and the small arrays of the two running sums.
+// slot per stream each); per level the coder's scratch tiles and the small arrays of the two running
+// sums; the group sums of all levels.  The pointers are level 0's; level(v) has those of level v.
 struct EncodeWorkspace {
     size_t symbols_bytes;       // one level's symbols
+    size_t level_bytes;         // one level's scratch and sums
     uint8_t *symbols, *scratch;
     void *scan_scratch, *tile_scan_scratch;
     int32_t *tile_sums, *group_sums;
@@ -302,9 +304,25 @@ struct EncodeWorkspace {
         ws += align_up((size_t)(ntiles + 1) * sizeof(int64_t), 256);
         tile_scan_scratch = ws;
         ws += cg_scan_workspace(ntiles);
+        level_bytes = align_up((size_t)(ws - scratch), 256);
+        ws = scratch + level_bytes * (size_t)nlevels;
         group_sums = reinterpret_cast<int32_t *>(ws);          // bytes per group of kTileGroup tiles
-        ws += align_up((size_t)kMaxTileGroups * sizeof(int32_t), 256);
+        ws += align_up((size_t)nlevels * kMaxTileGroups * sizeof(int32_t), 256);
         total = (size_t)(ws - static_cast<uint8_t *>(base));
+    }
+
+    EncodeWorkspace level(int v) const
+    {
+        EncodeWorkspace w = *this;
+        const size_t by = level_bytes * (size_t)v;
+        w.symbols += symbols_bytes * (size_t)v;
+        w.scratch += by;
+        w.scan_scratch = static_cast<uint8_t *>(scan_scratch) + by;
+        w.tile_scan_scratch = static_cast<uint8_t *>(tile_scan_scratch) + by;
+        w.tile_sums += by / sizeof(int32_t);
+        w.tile_base += by / sizeof(int64_t);
+        w.group_sums += (size_t)v * kMaxTileGroups;
+        return w;
     }
 };
 
@@ -338,6 +356,23 @@ struct LevelOut {
     int64_t payload_cap;
     int32_t *status;
 };
+
+// The compaction's arguments, after the scan launches that it needs.  fused_scan: the coder left its tiles' byte
+// counts; grouped: and their sums by groups of tiles.
+int scan_for_compaction(const LevelOut &o, const EncodeWorkspace &w, bool fused_scan, bool grouped, const int32_t *group_sums, CompactArgs &c, hipStream_t s)
+{
+    const int32_t skew = (int32_t)(reinterpret_cast<uintptr_t>(o.payload) & 3u);
+    const int64_t *tile_base = nullptr;
+    if (fused_scan && !grouped && w.ntiles > kDirectTiles) {
+        if (int rc = launch_scan(w.tile_sums, w.ntiles, INT_MAX, w.tile_base, w.tile_scan_scratch, s)) return rc;
+        tile_base = w.tile_base;
+    } else if (!fused_scan) {
+        if (int rc = launch_scan(o.lengths, w.nstreams, kStreamCap, o.offsets, w.scan_scratch, s)) return rc;
+    }
+    c = {w.scratch, kStreamCap, o.offsets, fused_scan ? o.lengths : nullptr, tile_base, w.nstreams, o.payload,
+         o.payload_cap, skew, o.status, grouped ? group_sums : nullptr, fused_scan ? w.tile_sums : nullptr};
+    return CG_OK;
+}
 
 // Tables, streams and payload of one level from its symbols (packed words `sym4`, or byte
 // symbols [2L, T, C]): calculate_cdf + encode_fast_new + collect_bytes for every chunk
@@ -420,16 +455,8 @@ int code_and_compact(const LevelOut &o, const uint32_t *sym4, const uint8_t *sym
 
     const int64_t cblocks = ceil_div(w.nstreams, kCompactStreams);
     if (cblocks > INT_MAX) return fail(CG_ERR_ARG, "encode_kv: too many streams");
-    const int32_t skew = (int32_t)(reinterpret_cast<uintptr_t>(o.payload) & 3u);
-    const int64_t *tile_base = nullptr;
-    if (fused_scan && !grouped && w.ntiles > kDirectTiles) {
-        if (int rc = launch_scan(w.tile_sums, cblocks, INT_MAX, w.tile_base, w.tile_scan_scratch, s)) return rc;
-        tile_base = w.tile_base;
-    } else if (!fused_scan) {
-        if (int rc = launch_scan(o.lengths, w.nstreams, kStreamCap, o.offsets, w.scan_scratch, s)) return rc;
-    }
-    const CompactArgs c = {w.scratch, kStreamCap, o.offsets, fused_scan ? o.lengths : nullptr, tile_base, w.nstreams, o.payload,
-                           o.payload_cap, skew, o.status, grouped ? group_sums : nullptr, fused_scan ? w.tile_sums : nullptr};
+    CompactArgs c;
+    if (int rc = scan_for_compaction(o, w, fused_scan, grouped, group_sums, c, s)) return rc;
     const dim3 cgrid((unsigned)cblocks);
     if (cblocks <= sliced_compact_blocks()) {
         if (fused_scan) compact_few_kernel<true><<<cgrid, dim3(1024), 0, s>>>(c);
@@ -439,6 +466,112 @@ int code_and_compact(const LevelOut &o, const uint32_t *sym4, const uint8_t *sym
         else compact_streams_kernel<false><<<cgrid, dim3(256), 0, s>>>(c);
     }
     return check_launch("compact");
+}
+
+// Several levels of one tensor from their packed symbols (level v's in w.level(v)): as code_and_compact for each,
+// with a launch for all of them where they can share one.  A launch of one level ends with its slowest streams
+// while the next waits, and a small one does not fill the GPU: it lasts as long as one stream's chain of symbols,
+// as often as there are levels.  Tables of 9, 17, 33 and 65 entries, a launch per level / shared, the whole call, us:
+//                     chunks of 256 tokens    300 tokens      one chunk
+//   1024 channels  32 layers x 4096 tokens  1153 / 1070   1504 / 1436   1255 / 1144
+//                  32 x 1024                 382 /  328    493 /  434    416 /  345
+//                  32 x  256                 178 /  102
+//                   4 x  256                 155 /   59
+//    512 channels  32 x 4096                 695 /  618    918 /  830    785 /  668
+//                   4 x 2048                 169 /   71    199 /  101    244 /   89
+//   4096 channels  32 x 1024                1348 / 1250   1877 / 1806   1467 / 1385
+int code_and_compact_levels(const LevelOut *o, int n, const EncodeWorkspace &w, int64_t L, int64_t T, int64_t C,
+                            int64_t chunk_tokens, hipStream_t s, const void *maxima, int max_dt, bool sums_cleared)
+{
+    const int64_t rows = 2 * L;
+    int max_lp = 0;
+    bool alike = w.nsub * n <= 65535;                       // sub-chunks of all levels are one grid dimension
+    for (int v = 0; v < n; ++v) {
+        if (o[v].max_bins + 1 > max_lp) max_lp = o[v].max_bins + 1;
+        alike = alike && pick_block(C, o[v].max_bins + 1) == kSlotTile;
+    }
+    if (!alike || n == 1) {
+        for (int v = 0; v < n; ++v) {
+            const EncodeWorkspace wv = w.level(v);
+            if (int rc = code_and_compact(o[v], reinterpret_cast<uint32_t *>(wv.symbols), nullptr, wv, L, T, C, chunk_tokens, s, maxima, max_dt,
+                                          true, false, sums_cleared ? wv.group_sums : nullptr)) return rc;
+        }
+        return CG_OK;
+    }
+    EncodeLevelsArgs p;
+    memset(&p, 0, sizeof(p));
+    EncodeArgs &a = p.all;
+    a.nsub = w.nsub;
+    a.cap = kStreamCap;
+    a.L = L;
+    a.nibbles = 1;
+    a.maxima = static_cast<const uint16_t *>(maxima);
+    a.max_dt = max_dt;
+    a.last_first = code_last_first(w.ntiles);
+    int64_t nblocks;
+    if (int rc = make_grid(rows, C, T, chunk_tokens, w.nsub, kSlotTile, a.sg, nblocks)) return rc;
+    if (nblocks > INT_MAX / kMaxLevels) return fail(CG_ERR_ARG, "encode_kv_levels: too many streams");
+    const bool fused_scan = C % kSlotTile == 0;             // as in code_and_compact
+    const bool grouped = fused_scan && sums_cleared && ceil_div(w.ntiles, kTileGroup) <= kMaxTileGroups;
+    const bool counted = chunk_tokens <= kSub;              // the coder makes the tables
+    if (!counted) {
+        CdfLevelsArgs t;
+        memset(&t, 0, sizeof(t));
+        t.all.nsub = w.nsub;
+        t.all.nibbles = 1;
+        t.all.L = L;
+        t.all.rows = rows;
+        t.all.nc = C;
+        t.all.g = a.sg.g;
+        for (int v = 0; v < n; ++v)
+            t.level[v] = {reinterpret_cast<const uint32_t *>(w.level(v).symbols), o[v].key_bins, o[v].value_bins,
+                          reinterpret_cast<uint16_t *>(o[v].cdf), o[v].max_bins};
+        CdfGrid g;
+        if (int rc = make_cdf_grid(t.all, true, n, max_lp, g)) return rc;
+        if (g.sliced) CG_DISPATCH_BS(g.block, (calculate_cdf_levels_kernel<BS, 4><<<g.grid, dim3(BS * 4), g.shmem, s>>>(t)));
+        else CG_DISPATCH_BS(g.block, (calculate_cdf_levels_kernel<BS, 1><<<g.grid, dim3(BS), g.shmem, s>>>(t)));
+        if (int rc = check_launch("calculate_cdf levels")) return rc;
+    }
+    // The coder's launches: all levels together where that is a call of few wavefronts, or where even
+    // blocks with the longest table's LDS are all resident at once; else those levels together of whose tables a
+    // compute unit holds equally many blocks (with the LDS of a 65-entry table the shorter ones would run at half
+    // the wavefronts).
+    const dim3 grid = stream_grid(a.sg, nblocks);
+    const EncodeSource source = counted ? ENC_COUNTED : ENC_TABLES;
+    const bool few = few_encode(nblocks * n, source, max_lp, kSlotTile, fused_scan);
+    const bool together = few || nblocks * n <= (int64_t)compute_units() * resident_encode_blocks(max_lp);
+    for (int64_t resident = 8; resident >= 1; --resident) {
+        int count = 0, lp = 0;
+        for (int v = n - 1; v >= 0; --v) {
+            if (!together && resident_encode_blocks(o[v].max_bins + 1) != resident) continue;
+            const EncodeWorkspace wv = w.level(v);
+            p.level[count++] = {reinterpret_cast<uint16_t *>(o[v].cdf), reinterpret_cast<const uint32_t *>(wv.symbols), wv.scratch,
+                                o[v].lengths, o[v].status, fused_scan ? wv.tile_sums : nullptr, grouped ? wv.group_sums : nullptr,
+                                o[v].key_bins, o[v].value_bins, o[v].max_bins + 1};
+            if (o[v].max_bins + 1 > lp) lp = o[v].max_bins + 1;
+        }
+        if (!count) continue;
+        int rc;
+        if (counted) rc = fused_scan ? launch_encode_levels<true, true>(p, count, lp, grid, few, s) : launch_encode_levels<true, false>(p, count, lp, grid, few, s);
+        else rc = fused_scan ? launch_encode_levels<false, true>(p, count, lp, grid, few, s) : launch_encode_levels<false, false>(p, count, lp, grid, few, s);
+        if (rc) return rc;
+        if (together) break;
+    }
+    CompactLevelsArgs c;
+    for (int v = 0; v < n; ++v) {
+        const EncodeWorkspace wv = w.level(v);
+        if (int rc = scan_for_compaction(o[v], wv, fused_scan, grouped, wv.group_sums, c.level[v], s)) return rc;
+    }
+    const int64_t cblocks = ceil_div(w.nstreams, kCompactStreams);
+    const dim3 cgrid((unsigned)cblocks, (unsigned)n);
+    if (cblocks * n <= sliced_compact_blocks()) {
+        if (fused_scan) compact_levels_kernel<true, 4><<<cgrid, dim3(1024), 0, s>>>(c);
+        else compact_levels_kernel<false, 4><<<cgrid, dim3(1024), 0, s>>>(c);
+    } else {
+        if (fused_scan) compact_levels_kernel<true, 1><<<cgrid, dim3(256), 0, s>>>(c);
+        else compact_levels_kernel<false, 1><<<cgrid, dim3(256), 0, s>>>(c);
+    }
+    return check_launch("compact levels");
 }
 
 int check_kv_geometry(const char *what, int kv_dt, int64_t L, int64_t T, int64_t H, int64_t D, int64_t chunk_tokens)
@@ -562,11 +695,13 @@ int cg_encode_kv_levels(const void *kv, int kv_dt, int64_t L, int64_t T, int64_t
         return fail(CG_ERR_ARG, "encode_kv_levels: between 1 and %d levels, got %d", CG_MAX_LEVELS, nlevels);
     if (int rc = check_kv_geometry("encode_kv_levels", kv_dt, L, T, H, D, chunk_tokens)) return rc;
     int lp_lv[CG_MAX_LEVELS];
+    LevelOut outs[CG_MAX_LEVELS];
     for (int v = 0; v < nlevels; ++v) {
         if (!key_bins[v] || !value_bins[v] || !cdf[v] || !lengths[v] || !offsets[v] || !payload[v])
             return fail(CG_ERR_ARG, "encode_kv_levels: null pointer for level %d", v);
         if (int rc = check_lp(max_bins[v] + 1, "encode_kv_levels")) return rc;
         lp_lv[v] = max_bins[v] + 1;
+        outs[v] = {key_bins[v], value_bins[v], max_bins[v], cdf[v], lengths[v], offsets[v], payload[v], payload_cap[v], status + v};
     }
     const int64_t C = H * D;
     const EncodeWorkspace w(workspace, L, T, C, chunk_tokens, nlevels);
@@ -575,31 +710,21 @@ int cg_encode_kv_levels(const void *kv, int kv_dt, int64_t L, int64_t T, int64_t
     hipStream_t s = static_cast<hipStream_t>(stream);
 
     const bool packed = kv_vectorizable(kv, D, C, sl, skv, st, sh) && C % 8 == 0;
-    // the levels' group sums lie where the tiles' running sums would, which such calls do not make
-    static_assert((kDirectTiles + 1) * sizeof(int64_t) >= (size_t)CG_MAX_LEVELS * kMaxTileGroups * sizeof(int32_t), "the levels' group sums fit");
-    int32_t *const group_sums = packed && w.ntiles > kDirectTiles && ceil_div(w.ntiles, kTileGroup) <= kMaxTileGroups
-                                    ? reinterpret_cast<int32_t *>(w.tile_base) : nullptr;
     if (packed) {
         // one pass over the tensor: every row is loaded once, its maximum found once, and its
         // symbols written once per level
-        uint32_t *sym4 = reinterpret_cast<uint32_t *>(w.symbols);
-        if (int rc = launch_quantize_pack(kv, kv_dt, L, T, H, D, sl, skv, st, sh, nullptr, nullptr, sym4, maxima,
-                                          w.nsub, chunk_tokens, 0, s, status, nlevels, key_bins, value_bins,
+        int32_t *const group_sums = w.ntiles > kDirectTiles ? w.group_sums : nullptr;
+        if (int rc = launch_quantize_pack(kv, kv_dt, L, T, H, D, sl, skv, st, sh, nullptr, nullptr, reinterpret_cast<uint32_t *>(w.symbols),
+                                          maxima, w.nsub, chunk_tokens, 0, s, status, nlevels, key_bins, value_bins,
                                           (int64_t)(w.symbols_bytes / 4), true, lp_lv, 0, group_sums)) return rc;
+        return code_and_compact_levels(outs, nlevels, w, L, T, C, chunk_tokens, s, maxima, kv_dt, group_sums != nullptr);
     }
+    // shapes the vector loads cannot take: one plain quantization pass per level
     for (int v = 0; v < nlevels; ++v) {
-        const LevelOut o = {key_bins[v], value_bins[v], max_bins[v], cdf[v], lengths[v], offsets[v],
-                            payload[v], payload_cap[v], status + v};
-        uint8_t *symbols = w.symbols + (size_t)v * w.symbols_bytes;
-        if (packed) {
-            if (int rc = code_and_compact(o, reinterpret_cast<uint32_t *>(symbols), nullptr, w, L, T, C, chunk_tokens, s, maxima, kv_dt, true, false,
-                                          group_sums ? group_sums + v * kMaxTileGroups : nullptr)) return rc;
-        } else {
-            // shapes the vector loads cannot take: one plain quantization pass per level
-            clear_status_kernel<<<1, 1, 0, s>>>(status + v);
-            if (int rc = launch_quantize(kv, kv_dt, L, T, H, D, sl, skv, st, sh, key_bins[v], value_bins[v], symbols, maxima, s)) return rc;
-            if (int rc = code_and_compact(o, nullptr, symbols, w, L, T, C, chunk_tokens, s)) return rc;
-        }
+        const EncodeWorkspace wv = w.level(v);
+        clear_status_kernel<<<1, 1, 0, s>>>(status + v);
+        if (int rc = launch_quantize(kv, kv_dt, L, T, H, D, sl, skv, st, sh, key_bins[v], value_bins[v], wv.symbols, maxima, s)) return rc;
+        if (int rc = code_and_compact(outs[v], nullptr, wv.symbols, wv, L, T, C, chunk_tokens, s)) return rc;
     }
     return CG_OK;
 }

@@ -324,7 +324,44 @@ struct EncodeArgs {
     int32_t last_first;     // encode_streams_kernel: the last sub-chunk's blocks are the launch's first (code_last_first)
 };
 
-__device__ __forceinline__ uint32_t coder_sub(const EncodeArgs &a) { return a.last_first ? gridDim.z - 1 - blockIdx.z : blockIdx.z; }
+// Several quantization levels of one tensor in one launch: what they share, and what differs.  Level v has the
+// launch's blocks of z index v * nsub and up.
+struct EncodeLevel {
+    uint16_t *cdf;
+    const uint32_t *sym4;
+    uint8_t *out;
+    int32_t *lengths, *status, *tile_sums, *group_sums;
+    const float *key_bins, *value_bins;
+    int32_t lp;
+};
+struct EncodeLevelsArgs {
+    EncodeArgs all;
+    EncodeLevel level[kMaxLevels];
+};
+
+// The arguments of the level that this block belongs to; z becomes the block's sub-chunk (uniform: at most seven
+// subtractions on the scalar unit, once per block).
+__device__ __forceinline__ EncodeArgs level_args(const EncodeLevelsArgs &p, uint32_t &z)
+{
+    int v = 0;
+    while (z >= (uint32_t)p.all.nsub) {
+        z -= (uint32_t)p.all.nsub;
+        ++v;
+    }
+    const EncodeLevel &o = p.level[v];
+    EncodeArgs a = p.all;
+    a.cdf = o.cdf;
+    a.sym4 = o.sym4;
+    a.out = o.out;
+    a.lengths = o.lengths;
+    a.status = o.status;
+    a.tile_sums = o.tile_sums;
+    a.group_sums = o.group_sums;
+    a.key_bins = o.key_bins;
+    a.value_bins = o.value_bins;
+    a.lp = o.lp;
+    return a;
+}
 
 // How a packed word holds its four symbols: kBytes, a byte each (any value; kept inside the
 // table where it is used); kNibbles, four bits each, every one a table symbol; kNibblesEscaped,
@@ -368,12 +405,13 @@ __device__ __forceinline__ void leave_tile_sum(const EncodeArgs &a, uint32_t til
 // PACKED: symbols come from sym4.  FUSE_CDF (PACKED only, one sub-chunk per chunk): the
 // block first builds its own tables from the same words and writes them out.
 // SLOTS: stream g of the launch is written to out[g * cap ...] (the fused path's scratch).
-template <int BS, bool ALIGNED, bool PACKED, bool FUSE_CDF, bool SLOTS, bool TILE = false>
-__global__ __launch_bounds__(BS) void encode_streams_kernel(EncodeArgs a)
+// z: the block's sub-chunk, counted in the launch's order.
+template <int BS, bool ALIGNED, bool PACKED, bool FUSE_CDF, bool SLOTS, bool TILE>
+__device__ __forceinline__ void encode_streams(const EncodeArgs &a, uint16_t *tab, uint32_t z)
 {
-    extern __shared__ uint16_t tab[];
     const int tid = threadIdx.x;
-    const StreamId id = locate<BS>(a.sg, coder_sub(a));
+    const uint32_t coder_sub = a.last_first ? (uint32_t)a.nsub - 1 - z : z;
+    const StreamId id = locate<BS>(a.sg, coder_sub);
     const int lp = a.lp;
     const int64_t ch0 = id.ch - tid;
     uint16_t *col = tab + table_column<BS>(tid);
@@ -499,7 +537,7 @@ __global__ __launch_bounds__(BS) void encode_streams_kernel(EncodeArgs a)
         // the tile, tid the stream's place in it
         enc.init(col, lp);
         enc.w.init(nullptr, 0, a.cap);
-        enc.w.init_tile(__builtin_amdgcn_make_buffer_rsrc((void *)(a.out + (int64_t)linear_block(coder_sub(a)) * ((int64_t)kSlotTile * a.cap)), 0,
+        enc.w.init_tile(__builtin_amdgcn_make_buffer_rsrc((void *)(a.out + (int64_t)linear_block(coder_sub) * ((int64_t)kSlotTile * a.cap)), 0,
                                                           kSlotTile * a.cap, kBufferWord3),
                         (uint32_t)tid * 4u);
     } else if (SLOTS) {
@@ -578,7 +616,24 @@ __global__ __launch_bounds__(BS) void encode_streams_kernel(EncodeArgs a)
     const int len = enc.finish();
     a.lengths[stream] = len;
     if (len > a.cap && a.status) atomicOr(a.status, 1);
-    if (SLOTS && a.tile_sums) leave_tile_sum<BS>(a, linear_block(coder_sub(a)), tid, len);
+    if (SLOTS && a.tile_sums) leave_tile_sum<BS>(a, linear_block(coder_sub), tid, len);
+}
+
+template <int BS, bool ALIGNED, bool PACKED, bool FUSE_CDF, bool SLOTS, bool TILE = false>
+__global__ __launch_bounds__(BS) void encode_streams_kernel(EncodeArgs a)
+{
+    extern __shared__ uint16_t tab[];
+    encode_streams<BS, ALIGNED, PACKED, FUSE_CDF, SLOTS, TILE>(a, tab, blockIdx.z);
+}
+
+// Packed symbols of several levels, into the scratch.
+template <int BS, bool FUSE_CDF, bool TILE>
+__global__ __launch_bounds__(BS) void encode_streams_levels_kernel(EncodeLevelsArgs p)
+{
+    extern __shared__ uint16_t tab[];
+    uint32_t z = blockIdx.z;
+    const EncodeArgs a = level_args(p, z);
+    encode_streams<BS, true, true, FUSE_CDF, true, TILE>(a, tab, z);
 }
 
 }  // namespace

@@ -152,12 +152,11 @@ struct FewEncoder {
 };
 
 // The forms and arguments of encode_streams_kernel; streams begin at multiples of four bytes.
-template <int BS, bool PACKED, bool FUSE_CDF, bool SLOTS, bool TILE = false>
-__global__ __launch_bounds__(BS) void encode_few_kernel(EncodeArgs a)
+template <int BS, bool PACKED, bool FUSE_CDF, bool SLOTS, bool TILE>
+__device__ __forceinline__ void encode_few(const EncodeArgs &a, uint32_t *entries, uint32_t z)
 {
-    extern __shared__ uint32_t entries[];
     const int tid = threadIdx.x;
-    const StreamId id = locate<BS>(a.sg);
+    const StreamId id = locate<BS>(a.sg, z);
     const int lp = a.lp;
     uint32_t *col = entries + tid;
     uint16_t *mine = a.cdf + ((id.chunk * a.sg.rows + id.row) * a.sg.nc + id.ch) * lp;      // this lane's table in memory
@@ -278,7 +277,7 @@ __global__ __launch_bounds__(BS) void encode_few_kernel(EncodeArgs a)
     enc.init(col, lp);
     if (TILE) {
         enc.w.init(nullptr, 0, a.cap);
-        enc.w.init_tile(__builtin_amdgcn_make_buffer_rsrc((void *)(a.out + (int64_t)linear_block() * ((int64_t)kSlotTile * a.cap)), 0,
+        enc.w.init_tile(__builtin_amdgcn_make_buffer_rsrc((void *)(a.out + (int64_t)linear_block(z) * ((int64_t)kSlotTile * a.cap)), 0,
                                                           kSlotTile * a.cap, kBufferWord3),
                         (uint32_t)tid * 4u);
     } else if (SLOTS) {
@@ -357,7 +356,23 @@ __global__ __launch_bounds__(BS) void encode_few_kernel(EncodeArgs a)
     const int len = enc.finish();
     a.lengths[stream] = len;
     if (len > a.cap && a.status) atomicOr(a.status, 1);
-    if (SLOTS && a.tile_sums) leave_tile_sum<BS>(a, linear_block(), tid, len);
+    if (SLOTS && a.tile_sums) leave_tile_sum<BS>(a, linear_block(z), tid, len);
+}
+
+template <int BS, bool PACKED, bool FUSE_CDF, bool SLOTS, bool TILE = false>
+__global__ __launch_bounds__(BS) void encode_few_kernel(EncodeArgs a)
+{
+    extern __shared__ uint32_t entries[];
+    encode_few<BS, PACKED, FUSE_CDF, SLOTS, TILE>(a, entries, blockIdx.z);
+}
+
+template <int BS, bool FUSE_CDF, bool TILE>
+__global__ __launch_bounds__(BS) void encode_few_levels_kernel(EncodeLevelsArgs p)
+{
+    extern __shared__ uint32_t entries[];
+    uint32_t z = blockIdx.z;
+    const EncodeArgs a = level_args(p, z);
+    encode_few<BS, true, FUSE_CDF, true, TILE>(a, entries, z);
 }
 
 }  // namespace

@@ -95,14 +95,43 @@ int64_t sliced_lanes(bool packed, int64_t chunk_tokens)
     return (chunk_tokens >= 512 ? 256 : chunk_tokens >= 64 ? 128 : 64) << 10;
 }
 
+// The blocks of a table pass over `nlevels` levels (1 for byte symbols) and their LDS, the longest table's.
+struct CdfGrid {
+    int block;
+    bool sliced;
+    dim3 grid;
+    size_t shmem;
+};
+
+int make_cdf_grid(CdfArgs &a, bool packed, int nlevels, int max_lp, CdfGrid &g)
+{
+    const int64_t S = a.g.S, T = a.g.T;
+    int block = pick_block(a.nc, max_lp);
+    while (!packed && block > 64 && (size_t)max_lp * (block + 1) * sizeof(uint32_t) > 64 * 1024) block /= 2;
+    a.ctiles = (int32_t)ceil_div(a.nc, block);
+    int64_t nblocks = ceil_div(T, S) * a.rows * a.ctiles;
+    if (nblocks <= 0 || nblocks > INT_MAX) return fail(CG_ERR_ARG, "calculate_cdf: grid out of range");
+    // Narrower blocks where that is how more compute units get one: a block's lanes and slices all count
+    // through one unit's LDS.  512 channels x 4 rows: 512 tokens 13.1 -> 8.6 us, 256 tokens of byte symbols 11.1 -> 7.6.
+    while (block > 64 && nblocks * nlevels * 2 <= compute_units()) {
+        block /= 2;
+        a.ctiles = (int32_t)ceil_div(a.nc, block);
+        nblocks = ceil_div(T, S) * a.rows * a.ctiles;
+    }
+    g.block = block;
+    g.shmem = packed ? (size_t)max_lp * (block + 2) * sizeof(uint16_t)
+                     : (size_t)max_lp * (block + 1) * sizeof(uint32_t);     // TableStride
+    g.sliced = nblocks * nlevels * block <= sliced_lanes(packed, S < T ? S : T);
+    g.grid = dim3((unsigned)nblocks, (unsigned)nlevels);
+    return CG_OK;
+}
+
 // key_bins, value_bins (packed symbols only, may be null): the rows of at most 15 symbols hold
 // four bits a symbol.
 int launch_cdf(const uint8_t *sym, const uint32_t *sym4, int64_t nsub, int64_t rows, int64_t T,
                int64_t nc, int64_t s0, int64_t s1, int64_t s2, int max_bins, int64_t S,
                uint16_t *cdf, hipStream_t stream, const float *key_bins = nullptr, const float *value_bins = nullptr)
 {
-    int block = pick_block(nc, max_bins + 1);
-    while (!sym4 && block > 64 && (size_t)(max_bins + 1) * (block + 1) * sizeof(uint32_t) > 64 * 1024) block /= 2;
     CdfArgs a;
     a.sym = sym;
     a.s0 = s0;
@@ -117,30 +146,20 @@ int launch_cdf(const uint8_t *sym, const uint32_t *sym4, int64_t nsub, int64_t r
     a.cdf = cdf;
     a.rows = rows;
     a.nc = nc;
-    a.ctiles = (int32_t)ceil_div(nc, block);
     a.max_bins = max_bins;
     a.g.T = T;
     a.g.S = S;
     a.g.nsc = (int32_t)ceil_div(S, kSub);
-    int64_t nblocks = ceil_div(T, S) * rows * a.ctiles;
-    if (nblocks <= 0 || nblocks > INT_MAX) return fail(CG_ERR_ARG, "calculate_cdf: grid out of range");
-    // Narrower blocks where that is how more compute units get one: a block's lanes and slices all count
-    // through one unit's LDS.  512 channels x 4 rows: 512 tokens 13.1 -> 8.6 us, 256 tokens of byte symbols 11.1 -> 7.6.
-    while (block > 64 && nblocks * 2 <= compute_units()) {
-        block /= 2;
-        a.ctiles = (int32_t)ceil_div(nc, block);
-        nblocks = ceil_div(T, S) * rows * a.ctiles;
-    }
-    const size_t shmem = sym4 ? (size_t)(max_bins + 1) * (block + 2) * sizeof(uint16_t)
-                              : (size_t)(max_bins + 1) * (block + 1) * sizeof(uint32_t);     // TableStride
-    const bool sliced = nblocks * block <= sliced_lanes(sym4 != nullptr, S < T ? S : T);
-    const dim3 grid((unsigned)nblocks), blk(sliced ? block * 4 : block);
-    if (sliced) {
-        if (sym4) CG_DISPATCH_BS(block, (calculate_cdf_kernel<BS, true, 4><<<grid, blk, shmem, stream>>>(a)));
-        else CG_DISPATCH_BS(block, (calculate_cdf_kernel<BS, false, 4><<<grid, blk, shmem, stream>>>(a)));
+    CdfGrid g;
+    if (int rc = make_cdf_grid(a, sym4 != nullptr, 1, max_bins + 1, g)) return rc;
+    const dim3 grid = g.grid, blk(g.sliced ? g.block * 4 : g.block);
+    const size_t shmem = g.shmem;
+    if (g.sliced) {
+        if (sym4) CG_DISPATCH_BS(g.block, (calculate_cdf_kernel<BS, true, 4><<<grid, blk, shmem, stream>>>(a)));
+        else CG_DISPATCH_BS(g.block, (calculate_cdf_kernel<BS, false, 4><<<grid, blk, shmem, stream>>>(a)));
     } else {
-        if (sym4) CG_DISPATCH_BS(block, (calculate_cdf_kernel<BS, true, 1><<<grid, blk, shmem, stream>>>(a)));
-        else CG_DISPATCH_BS(block, (calculate_cdf_kernel<BS, false, 1><<<grid, blk, shmem, stream>>>(a)));
+        if (sym4) CG_DISPATCH_BS(g.block, (calculate_cdf_kernel<BS, true, 1><<<grid, blk, shmem, stream>>>(a)));
+        else CG_DISPATCH_BS(g.block, (calculate_cdf_kernel<BS, false, 1><<<grid, blk, shmem, stream>>>(a)));
     }
     return check_launch("calculate_cdf");
 }
@@ -505,6 +524,32 @@ int launch_encode(const EncodeArgs &a, dim3 grid, bool few, hipStream_t stream)
         encode_streams_kernel<BS, true, PACKED, FUSE_CDF, SLOTS, TILE><<<grid, dim3(BS), lds, stream>>>(a);
     }
     return check_launch("encode");
+}
+
+// Blocks of tables of `lp` entries that a compute unit holds at once (eight of 256 lanes are all its wavefronts).
+int64_t resident_encode_blocks(int lp)
+{
+    const int64_t fit = (int64_t)(kMaxLdsPerBlock / align_up((size_t)lp * TableStride<kSlotTile>::k16 * sizeof(uint16_t) + 32, 1280));
+    return fit < 8 ? fit : 8;
+}
+
+// `count` levels in one launch of blocks of 256 lanes; their tables' LDS is the longest's.
+template <bool FUSE_CDF, bool TILE>
+int launch_encode_levels(const EncodeLevelsArgs &p, int count, int max_lp, dim3 grid, bool few, hipStream_t stream)
+{
+    constexpr int BS = kSlotTile;
+    grid.z *= (unsigned)count;
+    if (few) {
+        static std::atomic<uint64_t> asked{0};          // per form of the kernel: these are templates
+        const size_t lds = (size_t)max_lp * BS * sizeof(uint32_t);
+        if (lds > 64 * 1024)
+            if (int rc = allow_dynamic_lds(reinterpret_cast<const void *>(&encode_few_levels_kernel<BS, FUSE_CDF, TILE>),
+                                           CG_MAX_LP * BS * (int)sizeof(uint32_t), asked)) return rc;
+        encode_few_levels_kernel<BS, FUSE_CDF, TILE><<<grid, dim3(BS), lds, stream>>>(p);
+    } else {
+        encode_streams_levels_kernel<BS, FUSE_CDF, TILE><<<grid, dim3(BS), (size_t)max_lp * TableStride<BS>::k16 * sizeof(uint16_t), stream>>>(p);
+    }
+    return check_launch("encode levels");
 }
 
 // Whether the coder begins with the last sub-chunk: the compaction behind it begins with the first, and so

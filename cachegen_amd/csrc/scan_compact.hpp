@@ -334,6 +334,19 @@ __global__ __launch_bounds__(1024) void compact_few_kernel(CompactArgs a)
     compact_streams<SCAN, 4>(a, rel, buf);
 }
 
+// The streams of several quantization levels of one tensor: level v has the blocks of y index v.
+struct CompactLevelsArgs {
+    CompactArgs level[kMaxLevels];
+};
+
+template <bool SCAN, int SLICES>
+__global__ __launch_bounds__(256 * SLICES) void compact_levels_kernel(CompactLevelsArgs p)
+{
+    __shared__ int32_t rel[kCompactStreams + 1];
+    __shared__ __align__(16) uint32_t buf[kCompactTile / 4];
+    compact_streams<SCAN, SLICES>(p.level[blockIdx.y], rel, buf);
+}
+
 // collect_bytes for streams in a padded buffer (encoder.py:209-222): stream g = row * nc + channel
 // goes to out[offsets[g] ...].  A wavefront copies four streams, a byte per lane: the streams are
 // some tens of bytes long and begin anywhere.

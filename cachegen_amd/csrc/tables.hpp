@@ -265,9 +265,8 @@ struct CdfArgs {
 // quarter of the batches (512 tokens x 512 channels, two layers: 25.1 -> 15.0 us; 1333 tokens x 1024
 // channels, 32 layers: 62.4 -> 35.4 us); where that stops paying: sliced_lanes in launch.hpp.
 template <int BS, bool PACKED, int SLICES>
-__global__ __launch_bounds__(BS * SLICES) void calculate_cdf_kernel(CdfArgs a)
+__device__ __forceinline__ void calculate_cdf(const CdfArgs &a, uint32_t *smem)
 {
-    extern __shared__ uint32_t smem[];
     const int tid = SLICES > 1 ? threadIdx.x % BS : threadIdx.x;
     const int slice = SLICES > 1 ? threadIdx.x / BS : 0;
     const int lp = a.max_bins + 1;
@@ -373,6 +372,40 @@ __global__ __launch_bounds__(BS * SLICES) void calculate_cdf_kernel(CdfArgs a)
         }
         write_tables<BS, BS * SLICES>(smem, dst, lp, ch0, a.nc);
     }
+}
+
+template <int BS, bool PACKED, int SLICES>
+__global__ __launch_bounds__(BS * SLICES) void calculate_cdf_kernel(CdfArgs a)
+{
+    extern __shared__ uint32_t smem[];
+    calculate_cdf<BS, PACKED, SLICES>(a, smem);
+}
+
+// Packed symbols of several quantization levels of one tensor in one launch: what they share, and what
+// differs.  Level v has the blocks of y index v.
+struct CdfLevel {
+    const uint32_t *sym4;
+    const float *key_bins, *value_bins;
+    uint16_t *cdf;
+    int32_t max_bins;
+};
+struct CdfLevelsArgs {
+    CdfArgs all;
+    CdfLevel level[kMaxLevels];
+};
+
+template <int BS, int SLICES>
+__global__ __launch_bounds__(BS * SLICES) void calculate_cdf_levels_kernel(CdfLevelsArgs p)
+{
+    extern __shared__ uint32_t smem[];
+    const CdfLevel &o = p.level[blockIdx.y];
+    CdfArgs a = p.all;
+    a.sym4 = o.sym4;
+    a.key_bins = o.key_bins;
+    a.value_bins = o.value_bins;
+    a.cdf = o.cdf;
+    a.max_bins = o.max_bins;
+    calculate_cdf<BS, true, SLICES>(a, smem);
 }
 
 // ------------------------------------------------------------------------------------

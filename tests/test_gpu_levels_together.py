@@ -1,0 +1,46 @@
+"""Levels of one cache coded by shared launches (cg_encode_kv_levels): every way the levels are dealt to
+launches gives the bytes of a separate encode at each level."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _bins(top, L):
+    """Two tiers: `top` bins in the first third of the layers, half of that in the others."""
+    b = torch.full((L,), max(4.0, top / 2))
+    b[:(L + 2) // 3] = top
+    return b
+
+
+# (layers, tokens, heads, head size), chunk, largest bins of each level
+CASES = [
+    ((1, 1, 1, 8), 16, (8, 16)),                  # one stream tile, mostly empty
+    ((2, 33, 8, 64), 16, (64, 8, 32)),            # few wavefronts, three chunks, the last one token
+    ((3, 257, 5, 80), 256, (16, 32, 64)),         # channels that fill no tile: offsets from a scan
+    ((4, 520, 8, 128), 260, (8, 16, 32, 64)),     # tables of two sub-chunks, all levels resident at once
+    ((6, 2048, 8, 128), 256, (8, 64, 32, 60)),    # more blocks than are resident: launches by table length
+    ((6, 2048, 8, 128), 700, (64, 8)),            # the same with tables made by a pass of their own
+    ((2, 300, 8, 128), 256, (16, 96)),            # a table too long for blocks of 256 lanes: one launch each
+    ((4, 256, 8, 128), 256, (8, 16, 24, 32, 40, 48, 56, 64)),
+]
+
+
+@pytest.mark.parametrize("shape,chunk,tops", CASES)
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_levels_in_shared_launches(shape, chunk, tops, dtype):
+    from cachegen_amd import codec
+    from cachegen_amd.kvgen import make_kv
+    L, T, H, D = shape
+    kv = make_kv(L, T, H, D, seed=5 + T, device=DEV, dtype=dtype)
+    levels = [(_bins(float(t), L), _bins(float(t), L)) for t in tops]
+    print(dict(shape=shape, chunk=chunk, tops=tops, dtype=str(dtype)), flush=True)
+    got = codec.encode_kv_levels(kv, levels, chunk_tokens=chunk)
+    for (kb, vb), e in zip(levels, got):
+        want = codec.encode_kv(kv, kb, vb, chunk_tokens=chunk)
+        n = want.total_bytes()
+        assert e.total_bytes() == n and int(e.status) == int(want.status) == 0
+        for name in ("cdf", "maxima", "lengths", "offsets"):
+            assert torch.equal(getattr(e, name), getattr(want, name)), name
+        assert torch.equal(e.payload[:n], want.payload[:n])
