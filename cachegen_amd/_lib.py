@@ -50,6 +50,9 @@ SIGNATURES = {
     "cg_tables_to_counts": (_INT, [_P, _INT, _I64, _I64, _P, _P, _P, _P, _P]),
     "cg_pack_counts": (_INT, [_P, _INT, _I64, _I64, _P, _P, _P, _P]),
     "cg_wire_meta": (_INT, [_P, _P, _I64, _I64, _P, _P, _P, _I64, _P, _P]),
+    "cg_move_bytes": (_INT, [_P, _P, _I64, _INT, _P, _INT, _P]),
+    "cg_mark": (_INT, [_P, _INT, _P]),
+    "cg_wait_mark": (_INT, [_P, _INT, _P]),
     "cg_lengths_to_u16": (_INT, [_P, _I64, _P, _P, _P]),
     "cg_counts_to_tables": (_INT, [_P, _I64, _INT, _I64, _I64, _P, _P, _P, _P, _P, _P]),
     "cg_decode_kv": (_INT, [_P, _INT, _P, _INT, _P, _P, _I64, _P, _P, _I64, _I64, _I64, _I64, _I64, _INT,

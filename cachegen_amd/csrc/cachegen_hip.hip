@@ -23,6 +23,7 @@
 #include <cstdio>
 #include <cstring>
 #include <atomic>
+#include <chrono>
 #include <mutex>
 #include <type_traits>
 
@@ -43,6 +44,7 @@
 #include "scan_compact.hpp"
 #include "launch.hpp"
 #include "host_lengths.hpp"
+#include "move_bytes.hpp"
 #include "tables_wire.hpp"
 
 // ======================================================================================
@@ -840,6 +842,26 @@ int cg_host_list(const CgHostContainer *items, int n, const void *const *lengths
             return fail(CG_ERR_ARG, "host_list: lengths do not add up to the payload");
     }
     return CG_OK;
+}
+
+int cg_move_bytes(const void *src, void *dst, int64_t n, int to_host, int32_t *mark, int32_t value, void *stream)
+{
+    if (!src || !dst || n <= 0) return fail(CG_ERR_ARG, "move_bytes: null pointer or nothing to move");
+    if (mark && !aligned_to(mark, 4)) return fail(CG_ERR_ARG, "move_bytes: the mark must be 4-byte aligned");
+    return launch_move_bytes(static_cast<const uint8_t *>(src), static_cast<uint8_t *>(dst), n, to_host != 0, mark, value, static_cast<hipStream_t>(stream));
+}
+
+int cg_mark(int32_t *mark, int32_t value, void *stream)
+{
+    if (!mark || !aligned_to(mark, 4)) return fail(CG_ERR_ARG, "mark: null or misaligned pointer");
+    mark_kernel<<<1, 1, 0, static_cast<hipStream_t>(stream)>>>(mark, value);
+    return check_launch("mark");
+}
+
+int cg_wait_mark(const int32_t *mark, int32_t value, void *stream)
+{
+    if (!mark || !aligned_to(mark, 4)) return fail(CG_ERR_ARG, "wait_mark: null or misaligned pointer");
+    return wait_for_mark(mark, value, static_cast<hipStream_t>(stream));
 }
 
 int cg_tables_to_counts(const int16_t *cdf, int max_bins, int64_t ngroups, int64_t C, const int32_t *tokens,

@@ -5,10 +5,14 @@ A blob that goes into or comes out of a store is a Python bytes object of severa
 is copied from and to pinned memory by torch's own copy, which runs on its thread pool and without
 the interpreter lock: 6 MB in 16 us warm and 45 us out of memory the GPU has just written, where
 one thread (numpy, bytes()) takes 80 and 200."""
+import collections
 import ctypes
+import threading
 import warnings
 
 import torch
+
+from . import _lib
 
 _new = ctypes.pythonapi.PyBytes_FromStringAndSize
 _new.restype = ctypes.py_object
@@ -75,11 +79,11 @@ class StoredWords:
     def __enter__(self):
         return self
 
-    def stored(self):
+    def stored(self, by=None):
         """Everything that stores to the words has been launched: `read` waits for that, and not for
         what is launched afterwards.  (To be left out where nothing is: the event costs a few
-        microseconds.)"""
-        self._stored = self._stream.record_event()
+        microseconds.)  by: an `Arrival` that comes no earlier, in the place of an event."""
+        self._stored = by or self._stream.record_event()
 
     def _wait(self):
         (self._stored or self._stream).synchronize()
@@ -93,3 +97,114 @@ class StoredWords:
     def __exit__(self, *exc):
         if not self._through:
             self._wait()
+
+
+class Arrival:
+    """What was queued up to one place of a stream."""
+
+    def __init__(self, moves, number):
+        self._moves, self._number = moves, number
+
+    def synchronize(self):
+        self._moves.wait(self._number)
+
+
+class Moves:
+    """Bytes between pinned host memory and device memory, moved by a kernel on one stream, and how far they
+    have got: every move sets a pinned word to the number of moves (and other launches that the caller
+    counts) before it, which the host reads without a call to the runtime.
+
+    torch's pool of pinned memory knows nothing of a kernel's accesses.  What comes down is waited for, at the
+    latest when the `with` block ends; what goes up is handed to `hold`."""
+
+    def __init__(self, device, stream):
+        self.device, self.stream = device, stream        # the stream's raw handle; the caller has made the device current
+        self._word = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+        self._at = self._word.data_ptr()
+        self._value = ctypes.c_int32.from_address(self._at)
+        self._count = self._marked = self._reached = 0
+        self._going_up, self._coming_down = [], []       # (number, pinned tensor)
+
+    def __enter__(self):
+        return self
+
+    def __exit__(self, *exc):
+        if self._reached < self._count:
+            self.wait(self._count)
+
+    def queued(self):
+        """What has been launched on the stream so far."""
+        self._count += 1
+        return Arrival(self, self._count)
+
+    def _move(self, src, dst, n, to_host):
+        _lib.check(_lib.lib().cg_move_bytes(src, dst, n, to_host, self._at, self._count, self.stream))
+        self._marked = self._count
+        return self.queued()
+
+    def down(self, src):
+        """(pinned uint8 tensor that receives the bytes of a device tensor, their arrival)."""
+        src = src.contiguous()
+        n, at = src.numel() * src.element_size(), src.data_ptr()
+        skew = at % 16                                   # the same place inside a 16-byte unit on both sides
+        host = torch.empty(n + skew, dtype=torch.uint8, pin_memory=True)[skew:]
+        return host, self.down_to(at, host) if n else self.queued()
+
+    def down_to(self, src, host):
+        """The same into a slice of pinned memory, from a device address."""
+        arrival = self._move(src, host.data_ptr(), host.numel(), 1)
+        self._coming_down.append((self._count, host))
+        return arrival
+
+    def up(self, host, dst):
+        """Pinned memory to a device address; `host` is kept until it has been read."""
+        arrival = self._move(host.data_ptr(), dst, host.numel(), 0)
+        self._going_up.append((self._count, host))
+        reached = self._value.value
+        while self._going_up[0][0] <= reached:
+            del self._going_up[0]
+        return arrival
+
+    def wait(self, number):
+        if self._reached < number:
+            with torch.cuda.device(self.device):
+                if self._marked < number:
+                    _lib.check(_lib.lib().cg_mark(self._at, self._count, self.stream))
+                    self._marked = self._count
+                _lib.check(_lib.lib().cg_wait_mark(self._at, number, self.stream))
+            self._reached = number
+            while self._coming_down and self._coming_down[0][0] <= number:
+                del self._coming_down[0]
+
+    def hold(self, event):
+        """Keeps what is still going up, and the word, until `event`, recorded behind all moves."""
+        _hold(event, [self._word] + [t for _, t in self._going_up])
+        self._reached = self._count
+
+
+_HELD_BYTES = 256 << 20                  # of pinned memory on its way up that is kept without waiting
+_held = collections.deque()              # (event, pinned tensors)
+_held_lock = threading.Lock()
+
+
+def _hold(event, tensors):
+    with _held_lock:
+        _held.append((event, tensors))
+        _let_go(_HELD_BYTES)
+
+
+def _let_go(most):
+    """Gives back what has been read; waits only for as much as is above `most` bytes."""
+    while _held and _held[0][0].query():
+        _held.popleft()
+    total = sum(t.numel() for _, tensors in _held for t in tensors)
+    while _held and total > most:
+        event, tensors = _held.popleft()
+        event.synchronize()
+        total -= sum(t.numel() for t in tensors)
+
+
+def let_go():
+    """Gives back the pinned memory of earlier calls that has been read by now."""
+    with _held_lock:
+        _let_go(_HELD_BYTES)

@@ -88,15 +88,13 @@ def _upload(pieces, total, index_at, write_index):
     For a single piece the events and the change of stream cost more than they hide (+25 us)."""
     device = torch.device("cuda", torch.cuda.current_device())          # the caller made it current
     if index_at <= _WHOLE_BYTES:
-        return _transfer(pieces, total, index_at, write_index, device)
+        return _transfer(pieces, total, index_at, write_index, device)[0]
     side = _upload_streams.get(device.index)
     if side is None:
         side = _upload_streams.setdefault(device.index, torch.cuda.Stream(device))
     current = torch.cuda.current_stream()
     with torch.cuda.stream(side):
-        buf = _transfer(pieces, total, index_at, write_index, device)
-        arrived = torch.cuda.Event()
-        arrived.record()
+        buf, arrived = _transfer(pieces, total, index_at, write_index, device)
     current.wait_event(arrived)
     buf.record_stream(current)
     return buf
@@ -104,25 +102,31 @@ def _upload(pieces, total, index_at, write_index):
 
 def _transfer(pieces, total, index_at, write_index, device):
     buf = torch.empty(total, dtype=torch.uint8, device=device)
+    base = buf.data_ptr()
     step = index_at if index_at <= _WHOLE_BYTES else _PIECE_BYTES
     k = 0
-    for p0 in range(0, index_at, step):
-        p1 = min(p0 + step, index_at)
-        # pinned blocks come from and go back to torch's pool, which reuses one only when the copy
-        # out of it is through
-        host = torch.empty(p1 - p0, dtype=torch.uint8, pin_memory=True)
-        while k < len(pieces) and pieces[k][0] < p1:
-            off, src = pieces[k]
-            a, b = max(off, p0), min(off + src.numel(), p1)
-            host[a - p0:b - p0].copy_(src[a - off:b - off])
-            if off + src.numel() > p1:
-                break
-            k += 1
-        buf[p0:p1].copy_(host, non_blocking=True)
-    host = torch.empty(total - index_at, dtype=torch.uint8, pin_memory=True)
-    write_index(buf.data_ptr(), host)
-    buf[index_at:].copy_(host, non_blocking=True)
-    return buf
+    hostmem.let_go()
+    moves = hostmem.Moves(device, codec._stream(device))
+    try:
+        for p0 in range(0, index_at, step):
+            p1 = min(p0 + step, index_at)
+            host = torch.empty(p1 - p0, dtype=torch.uint8, pin_memory=True)
+            while k < len(pieces) and pieces[k][0] < p1:
+                off, src = pieces[k]
+                a, b = max(off, p0), min(off + src.numel(), p1)
+                host[a - p0:b - p0].copy_(src[a - off:b - off])
+                if off + src.numel() > p1:
+                    break
+                k += 1
+            moves.up(host, base + p0)
+        host = torch.empty(total - index_at, dtype=torch.uint8, pin_memory=True)
+        write_index(base, host)
+        moves.up(host, base + index_at)
+    finally:
+        through = torch.cuda.Event()
+        through.record()
+        moves.hold(through)
+    return buf, through
 
 
 def _levels(bins, num_layers, device):

@@ -350,8 +350,8 @@ class HostPart:
     def table_slices(self):
         """(start, end) slices of `tables`, each there when it is yielded."""
         at = 0
-        for end, event in self.slices:
-            event.synchronize()
+        for end, arrival in self.slices:
+            arrival.synchronize()
             yield at, end
             at = end
 
@@ -369,7 +369,17 @@ def bring_to_host(enc, first_chunk, num_chunks, per_chunk=True, compact=False):
     counts, stored into pinned memory by one kernel) and the maxima while the tables, whose size it
     knows, are already on the bus, and then for each piece of about _PIECE_BYTES."""
     import torch
-    from .. import _lib, codec, hostmem
+    from .. import codec, hostmem
+    dev = enc.payload.device
+    with torch.cuda.device(dev):
+        moves = hostmem.Moves(dev, codec._stream(dev))
+    with moves:
+        yield from _bring_to_host(enc, first_chunk, num_chunks, per_chunk, compact, moves)
+
+
+def _bring_to_host(enc, first_chunk, num_chunks, per_chunk, compact, moves):
+    import torch
+    from .. import _lib, hostmem
     L, H, D, S, T = enc.num_layers, enc.num_heads, enc.head_size, enc.chunk_tokens, enc.num_tokens
     C = H * D
     rows = 2 * L
@@ -380,31 +390,17 @@ def bring_to_host(enc, first_chunk, num_chunks, per_chunk=True, compact=False):
     dev = enc.payload.device
     lib = _lib.lib()
 
-    def fetch(src):
-        """The bytes of a contiguous device tensor on their way into pinned memory."""
-        flat = src.reshape(-1).view(torch.uint8)
-        host = torch.empty(flat.numel(), dtype=torch.uint8, pin_memory=True)
-        host.copy_(flat, non_blocking=True)
-        return host
-
-    def mark():
-        event = torch.cuda.Event()
-        event.record()
-        return event
-
     def fetch_tables(src):
-        """(pinned tables, [(end, event)]): in slices where nothing else would overlap with them."""
-        flat = src.reshape(-1).view(torch.uint8)
-        n = flat.numel()
+        """(pinned tables, [(end, arrival)]): in slices where nothing else would overlap with them."""
+        n = src.numel() * src.element_size()
         if len(pieces) > 1 or n < 2 * _SLICE_BYTES:
-            return fetch(src), [(n, mark())]
+            host, arrival = moves.down(src)
+            return host, [(n, arrival)]
         host = torch.empty(n, dtype=torch.uint8, pin_memory=True)
-        ends = [n * (i + 1) // (n // _SLICE_BYTES) for i in range(n // _SLICE_BYTES)]
+        ends = [n * (i + 1) // (n // _SLICE_BYTES) // 64 * 64 for i in range(n // _SLICE_BYTES - 1)] + [n]
         slices = []
-        for i, end in enumerate(ends):
-            at = ends[i - 1] if i else 0
-            host[at:end].copy_(flat[at:end], non_blocking=True)
-            slices.append((end, mark()))
+        for at, end in zip([0] + ends, ends):
+            slices.append((end, moves.down_to(src.data_ptr() + at, host[at:end])))
         return host, slices
 
     def subs(c):
@@ -413,8 +409,8 @@ def bring_to_host(enc, first_chunk, num_chunks, per_chunk=True, compact=False):
     # blobs by pieces: (first blob, last blob) covering about _PIECE_BYTES of tables and lengths
     groups = [(c, c + 1) for c in range(c_first, c_last)] if per_chunk else [(c_first, c_last)]
     early = {}                                           # the first piece's tables and lengths: sizes not needed
+    stream = moves.stream
     with torch.cuda.device(dev):
-        stream = codec._stream(dev)
         cdf = enc.cdf[c_first:c_last]
         lengths = enc.lengths[g_first:g_last]
         wide = inexact = nsym = dense = None
@@ -431,8 +427,8 @@ def bring_to_host(enc, first_chunk, num_chunks, per_chunk=True, compact=False):
         with hostmem.StoredWords(3 + nbounds + ngroups, torch.int64) as words:
             _lib.check(lib.cg_wire_meta(enc.status.data_ptr(), enc.offsets[g_first * rows * C:].data_ptr(), rows * C, nbounds,
                                         ptr(wide), ptr(inexact), ptr(nsym), ngroups, words.words.data_ptr(), stream))
-            maxima = fetch(enc.maxima)
-            words.stored()                               # one wait for the words and the maxima
+            maxima, arrival = moves.down(enc.maxima)
+            words.stored(by=arrival)                     # one wait for the words and the maxima
             chunk_bytes = max(1, cdf[0].numel() * cdf.element_size() + min(spc, lengths.shape[0]) * rows * C * 4)
             step = max(1, _PIECE_BYTES // chunk_bytes) if per_chunk else 1
             pieces = [(i, min(i + step, len(groups))) for i in range(0, len(groups), step)]
@@ -444,7 +440,7 @@ def bring_to_host(enc, first_chunk, num_chunks, per_chunk=True, compact=False):
                                               tables_src.data_ptr(), stream))
             elif not compact:
                 a, b = groups[0][0], groups[pieces[0][1] - 1][1]
-                early = {"tables": fetch_tables(cdf[a - c_first:b - c_first]), "lengths": fetch(lengths[subs(a):subs(b)])}
+                early = {"tables": fetch_tables(cdf[a - c_first:b - c_first]), "lengths": moves.down(lengths[subs(a):subs(b)])}
             meta = words.read()
 
     enc.raise_for_status(meta[0])
@@ -472,13 +468,12 @@ def bring_to_host(enc, first_chunk, num_chunks, per_chunk=True, compact=False):
             tables = early.pop("tables", None)
             lens = early.pop("lengths", None)
             return (fetch_tables(table_range(a, b)) if tables is None else tables,
-                    fetch(lengths_src[subs(a):subs(b)]) if lens is None else lens,
-                    fetch(enc.payload[p0:p1])), mark()
+                    moves.down(lengths_src[subs(a):subs(b)]) if lens is None else lens, moves.down(enc.payload[p0:p1]))
 
     itemsize = lengths_src.element_size()
     queued = queue(pieces[0])
     for k, piece in enumerate(pieces):
-        (((tables, slices), lens, payload), arrived), queued = queued, queue(pieces[k + 1]) if k + 1 < len(pieces) else None
+        ((tables, slices), (lens, _), (payload, arrived)), queued = queued, queue(pieces[k + 1]) if k + 1 < len(pieces) else None
         at = [0, 0, 0]
         for a, b in groups[piece[0]:piece[1]]:
             part = HostPart()

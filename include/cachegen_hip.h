@@ -372,6 +372,24 @@ int cg_wire_meta(const int32_t *status, const int64_t *offsets, int64_t per_sub,
 /* out[i] = lengths[i] as 16 bits; *wide (device int32, written) = 1 if some length does not fit. */
 int cg_lengths_to_u16(const int32_t *lengths, int64_t n, uint16_t *out, int32_t *wide, void *stream);
 
+/* ---------------------------------------------------------------------------
+ * Between pinned host memory and device memory (no counterpart in the reference, which copies
+ * tensor by tensor and waits).
+ * ------------------------------------------------------------------------- */
+
+/* n > 0 bytes from src to dst, one of them in pinned host memory (to_host: dst) and the other in device
+ * memory, queued on the stream; fastest where the two addresses are equal modulo 16.  Both stay valid until
+ * the launch is through.
+ * mark   pinned host int32, or null: set to `value` when everything queued on the stream before this
+ *        call is through, together with what that stored to host memory */
+int cg_move_bytes(const void *src, void *dst, int64_t n, int to_host, int32_t *mark, int32_t value, void *stream);
+
+/* The mark alone. */
+int cg_mark(int32_t *mark, int32_t value, void *stream);
+
+/* HOST: returns when *mark >= value; CG_ERR_ARG if the stream is through and it is not. */
+int cg_wait_mark(const int32_t *mark, int32_t value, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1,0 +1,74 @@
+"""Bytes between pinned and device memory by kernel, and the marks that say how far a stream is."""
+import pytest
+import torch
+
+from cachegen_amd import _lib, codec, hostmem
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda:0")
+GUARD = 64
+
+
+def _bytes(n, seed):
+    return torch.randint(0, 256, (n,), generator=torch.Generator().manual_seed(seed), dtype=torch.uint8)
+
+
+# one byte, either side of a 16-byte unit, of a block's 4 KB, of the launch's 256 KB, several of its rounds
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 4095, 4097, (256 << 10) - 1, (256 << 10) + 33, (3 << 20) + 5])
+@pytest.mark.parametrize("at_host,at_dev", [(0, 0), (5, 5), (0, 1), (13, 2)])
+def test_bytes_arrive_and_no_others_change(n, at_host, at_dev):
+    print(n, at_host, at_dev, flush=True)
+    want = _bytes(n, n)
+    host = torch.full((n + at_host + GUARD,), 7, dtype=torch.uint8).pin_memory()
+    back = torch.full((n + at_host + GUARD,), 9, dtype=torch.uint8).pin_memory()
+    dev = torch.full((n + at_dev + GUARD,), 8, dtype=torch.uint8, device=DEV)
+    host[at_host:at_host + n] = want
+    with torch.cuda.device(DEV), hostmem.Moves(DEV, codec._stream(DEV)) as moves:
+        moves.up(host[at_host:at_host + n], dev.data_ptr() + at_dev)
+        arrival = moves.down_to(dev.data_ptr() + at_dev, back[at_host:at_host + n])
+        arrival.synchronize()
+        assert torch.equal(back[at_host:at_host + n], want)
+    got = dev.cpu()
+    assert torch.equal(got[at_dev:at_dev + n], want)
+    assert (got[:at_dev] == 8).all() and (got[at_dev + n:] == 8).all()
+    assert (back[:at_host] == 9).all() and (back[at_host + n:] == 9).all()
+
+
+def test_arrivals_come_in_order_and_memory_is_kept():
+    src = torch.arange(1 << 20, dtype=torch.int32, device=DEV)
+    with torch.cuda.device(DEV), hostmem.Moves(DEV, codec._stream(DEV)) as moves:
+        parts = [moves.down(src[i << 18:(i + 1) << 18]) for i in range(4)]
+        for i in (2, 0, 3, 1):
+            parts[i][1].synchronize()
+            assert torch.equal(parts[i][0].view(torch.int32), torch.arange(i << 18, (i + 1) << 18, dtype=torch.int32))
+        lost = moves.down(src)[1]                        # its memory is dropped here and kept by `moves`
+    lost.synchronize()
+    empty, arrival = hostmem.Moves(DEV, codec._stream(DEV)).down(src[:0])
+    assert empty.numel() == 0
+
+
+def test_memory_that_has_been_read_is_given_back(monkeypatch):
+    monkeypatch.setattr(hostmem, "_HELD_BYTES", 1 << 20)
+    dst = torch.empty(1 << 20, dtype=torch.uint8, device=DEV)
+    for i in range(8):
+        moves = hostmem.Moves(DEV, codec._stream(DEV))
+        moves.up(_bytes(1 << 20, i).pin_memory(), dst.data_ptr())
+        event = torch.cuda.Event()
+        event.record()
+        moves.hold(event)
+        assert sum(t.numel() for _, tensors in hostmem._held for t in tensors) <= 1 << 20
+    torch.cuda.synchronize()
+    hostmem.let_go()
+    assert not hostmem._held
+    assert torch.equal(dst.cpu(), _bytes(1 << 20, 7))
+
+
+def test_marks_are_refused_where_they_cannot_be_set():
+    lib = _lib.lib()
+    word = torch.zeros(2, dtype=torch.int32).pin_memory()
+    with pytest.raises(RuntimeError, match="misaligned"):
+        _lib.check(lib.cg_mark(word.data_ptr() + 2, 1, None))
+    with pytest.raises(RuntimeError, match="nothing on this stream sets the mark"):
+        _lib.check(lib.cg_wait_mark(word.data_ptr(), 1, codec._stream(DEV)))
+    with pytest.raises(RuntimeError, match="nothing to move"):
+        _lib.check(lib.cg_move_bytes(word.data_ptr(), word.data_ptr(), 0, 1, None, 0, None))
