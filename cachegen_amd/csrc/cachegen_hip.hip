@@ -44,6 +44,7 @@
 #include "scan_compact.hpp"
 #include "launch.hpp"
 #include "host_lengths.hpp"
+#include "host_copy.hpp"
 #include "move_bytes.hpp"
 #include "tables_wire.hpp"
 
@@ -862,6 +863,113 @@ int cg_wait_mark(const int32_t *mark, int32_t value, void *stream)
 {
     if (!mark || !aligned_to(mark, 4)) return fail(CG_ERR_ARG, "wait_mark: null or misaligned pointer");
     return wait_for_mark(mark, value, static_cast<hipStream_t>(stream));
+}
+
+int cg_host_fill(const CgHostPart *parts, int n, const int32_t *mark, const CgHostTeam *team, void *stream)
+{
+    if (!parts || n <= 0 || !mark) return fail(CG_ERR_ARG, "host_fill: null pointer or nothing to copy");
+    try {
+        HostJob job;
+        job.mark = mark;
+        job.nthreads = host_threads(team);
+        for (int i = 0; i < n; ++i) {
+            const CgHostPart &p = parts[i];
+            if (p.bytes < 0 || (p.bytes && (!p.dst || !p.src))) return fail(CG_ERR_ARG, "host_fill: bad part");
+            add_blocks(job, reinterpret_cast<uint8_t *>(p.dst), reinterpret_cast<const uint8_t *>(p.src), p.bytes, (uintptr_t)p.dst, p.value, 0);
+        }
+        seal(job, 1);
+        int32_t last = INT_MIN;
+        for (const HostBlock &b : job.blocks) last = b.value > last ? b.value : last;
+        int rc = CG_OK;
+        MarkWatch watch(mark, static_cast<hipStream_t>(stream));
+        const std::function<void()> idle = [&] {
+            if (rc || job.known.load(std::memory_order_relaxed) >= last || !watch.overdue(last)) return;
+            // everything was queued before the call: once the stream is through, all is there
+            if ((rc = watch.settle())) job.stop.store(true);
+            else job.known.store(last, std::memory_order_release);
+        };
+        run_job(job, team, &idle);
+        return rc;
+    } catch (const std::exception &e) {
+        return fail(CG_ERR_ARG, "host_fill: %s", e.what());
+    }
+}
+
+int cg_host_present(void *at, int64_t n, int64_t page, const CgHostTeam *team)
+{
+    if (!at || n <= 0 || page < 4096 || page % 4096 || page > INT_MAX || reinterpret_cast<uintptr_t>(at) % 4096)
+        return fail(CG_ERR_ARG, "host_present: whole pages of memory are wanted");
+    try {
+        HostJob job;
+        const int32_t always = 0;
+        job.mark = &always;
+        job.nthreads = host_threads(team);
+        uint8_t *p = static_cast<uint8_t *>(at);
+        for (int64_t i = 0; i * page < n; ++i)
+            job.blocks.push_back({p + i * page, nullptr, (int32_t)std::min(page, n - i * page), (int32_t)(i % job.nthreads), 0, 0});
+        seal(job, 1);
+        run_job(job, team, nullptr);
+        return CG_OK;
+    } catch (const std::exception &e) {
+        return fail(CG_ERR_ARG, "host_present: %s", e.what());
+    }
+}
+
+int cg_host_stage(const CgHostPart *parts, int n, void *const *slots, int nslots, int64_t step, void *area, int64_t bytes, int32_t *mark,
+                  int32_t value, const CgHostTeam *team, int *moves, void *stream)
+{
+    if (!parts || n < 0 || !slots || !area || !mark || !moves || bytes <= 0) return fail(CG_ERR_ARG, "host_stage: null pointer or nothing to move");
+    *moves = 0;
+    if (step < 64 || step % 64) return fail(CG_ERR_ARG, "host_stage: steps are multiples of 64 bytes");
+    const int64_t ring_bytes = nslots * step;
+    if (nslots < 2 && ring_bytes < bytes) return fail(CG_ERR_ARG, "host_stage: pinned memory too small");
+    for (int64_t i = 0; i < nslots && i * step < bytes; ++i)
+        if (!slots[i]) return fail(CG_ERR_ARG, "host_stage: null slot");
+    const HostSteps at_step = {step};
+    try {
+        hipStream_t s = static_cast<hipStream_t>(stream);
+        auto pinned = [&](int64_t at) { return static_cast<uint8_t *>(slots[at / step % nslots]) + at % step; };
+        const int32_t steps = (int32_t)at_step.of(bytes - 1) + 1;
+        HostJob job;
+        job.mark = mark;
+        job.known.store(value);
+        job.nthreads = host_threads(team);
+        for (int i = 0; i < n; ++i) {
+            const CgHostPart &p = parts[i];
+            if (p.bytes < 0 || (p.bytes && !p.src) || p.dst < 0 || p.dst + p.bytes > bytes) return fail(CG_ERR_ARG, "host_stage: bad part");
+            for (int64_t at = p.dst, end = p.dst + p.bytes; at < end;) {
+                const int64_t k = at_step.of(at), stop = std::min(end, at_step.start(k + 1));
+                // the slot is free once the move that was there is through, which the launch behind that one says
+                const int32_t need = at < ring_bytes ? value : value + (int32_t)at_step.of(stop - 1 - ring_bytes) + 1;
+                add_blocks(job, pinned(at), reinterpret_cast<const uint8_t *>(p.src) + (at - p.dst), stop - at,
+                           (uintptr_t)p.src + (uintptr_t)(at - p.dst), need, (int32_t)k);
+                at = stop;
+            }
+        }
+        seal(job, steps);
+        int rc = CG_OK;
+        int32_t launched = 0;
+        MarkWatch watch(mark, s);
+        const std::function<void()> idle = [&] {
+            while (!rc && launched < steps && job.left[(size_t)launched].load(std::memory_order_acquire) <= 0) {
+                const int64_t at = at_step.start(launched), end = std::min(bytes, at_step.start(launched + 1));
+                rc = launch_move_bytes(pinned(at), static_cast<uint8_t *>(area) + at, end - at, false, mark, value + launched, s);
+                if (!rc) ++launched;
+            }
+            if (!rc && launched < steps && launched > 0 && job.known.load(std::memory_order_relaxed) < value + launched &&
+                watch.overdue(value + launched)) {
+                // the launches so far are through once the stream is
+                if (!(rc = watch.settle())) job.known.store(value + launched, std::memory_order_release);
+            }
+            if (rc) job.stop.store(true);
+        };
+        run_job(job, team, &idle);
+        while (!rc && launched < steps) idle();
+        *moves = launched;
+        return rc;
+    } catch (const std::exception &e) {
+        return fail(CG_ERR_ARG, "host_stage: %s", e.what());
+    }
 }
 
 int cg_tables_to_counts(const int16_t *cdf, int max_bins, int64_t ngroups, int64_t C, const int32_t *tokens,

@@ -1,0 +1,160 @@
+// Part of the CacheGen KV codec library for MI355X (gfx950); included by cachegen_hip.hip.  Copies between ordinary
+// and pinned host memory by several threads, in step with what crosses the bus; plain C++, without HIP.
+#pragma once
+
+#include <algorithm>
+#include <atomic>
+#include <climits>
+#include <cstdint>
+#include <cstring>
+#include <functional>
+#include <sys/mman.h>
+#include <vector>
+
+#include "cachegen_hip.h"
+
+namespace {
+
+// A container is copied once on the host each way, out of the pinned memory that its sections reach or into the one they
+// leave from.  Done with one library call a section, each a fork and join of its own, a chunk's five copies took 190 us
+// of which the bytes are 60, and the bus waited meanwhile.  Here a call's copies are one job, cut into blocks; the blocks of
+// what has arrived are copied while the rest is on the bus, and what is staged leaves while the rest is staged.
+//
+// The threads are the caller's team: the OpenMP runtime that torch's own copies run on.  Threads of this library's
+// own, beside sixteen of that runtime that still look for work after a torch operation, are more than the cores that a
+// process has here, and a job then waits for a thread that waits for a core (53 MB: 3 to 10 ms instead of 1.2).
+// A block has an owner among the threads, by its address in ordinary memory: a blob that is read back soon lies in the
+// caches of the threads that wrote it.  Every thread takes its own blocks in order and then what nobody has begun, so a
+// job also ends on its caller alone.
+//
+// Staged and moved to the GPU, one thread / eight: 1 MB 57 / 52 us, 2.7 MB 96 / 86, 6 MB 168 / 152, 14 MB 343 / 326, 53 MB 1532 / 1152;
+// copied out of pinned memory just written: 1.4 MB 40 / 20, 6 MB 157 / 61, 14 MB 364 / 130.  Sixteen: the same.
+constexpr int64_t kHostBlock = 64 << 10;
+constexpr int kHostThreads = 8;
+
+struct HostBlock {
+    uint8_t *dst;
+    const uint8_t *src;                     // null: dst's pages are made present, its bytes are undefined
+    int32_t bytes;
+    int32_t owner;
+    int32_t value;                          // to be copied when the job's mark is this far
+    int32_t step;                           // counts towards this step's completion
+};
+
+struct HostJob {
+    std::vector<HostBlock> blocks;
+    std::vector<std::atomic<uint8_t>> taken;
+    std::vector<std::atomic<int32_t>> left; // blocks to come, per step
+    std::atomic<int32_t> done{0};           // blocks that are through
+    std::atomic<bool> stop{false};
+    const int32_t *mark = nullptr;
+    std::atomic<int32_t> known{INT_MIN};    // how far the mark is known to be by other means
+    int nthreads = 1;
+
+    bool reached(int32_t value) const { return __atomic_load_n(mark, __ATOMIC_ACQUIRE) >= value || known.load(std::memory_order_acquire) >= value; }
+};
+
+inline void host_pause()
+{
+#if defined(__x86_64__) && !defined(__HIP_DEVICE_COMPILE__)
+    __builtin_ia32_pause();
+#endif
+}
+
+inline void make_present(uint8_t *at, int64_t n)
+{
+#ifdef MADV_POPULATE_WRITE
+    if (madvise(at, (size_t)n, MADV_POPULATE_WRITE) == 0) return;
+#endif
+    for (int64_t i = 0; i < n; i += 4096) *static_cast<volatile uint8_t *>(at + i) = 0;
+}
+
+// Block i, if it is still to be had.  `idle` runs while the mark is waited for.
+inline void take_block(HostJob &job, size_t i, const std::function<void()> *idle)
+{
+    if (job.taken[i].load(std::memory_order_relaxed) || job.taken[i].exchange(1, std::memory_order_acq_rel)) return;
+    const HostBlock &b = job.blocks[i];
+    while (!job.reached(b.value) && !job.stop.load(std::memory_order_relaxed)) {
+        if (idle) (*idle)();
+        host_pause();
+    }
+    if (!b.src) make_present(b.dst, b.bytes);
+    else if (!job.stop.load(std::memory_order_relaxed)) memcpy(b.dst, b.src, (size_t)b.bytes);
+    job.left[(size_t)b.step].fetch_sub(1, std::memory_order_acq_rel);
+    job.done.fetch_add(1, std::memory_order_acq_rel);
+}
+
+inline void work_on(HostJob &job, int me, const std::function<void()> *idle)
+{
+    for (int mine = 1; mine >= 0; --mine)
+        for (size_t i = 0; i < job.blocks.size(); ++i) {
+            if (mine && job.blocks[i].owner != me) continue;
+            take_block(job, i, idle);
+            if (idle) (*idle)();
+        }
+}
+
+// The job on the team's threads; `idle` (may be null) is run by the caller now and then.
+struct HostRun {
+    HostJob *job;
+    const std::function<void()> *idle;
+    int (*thread_num)();
+};
+
+inline void host_member(void *run)
+{
+    const HostRun &r = *static_cast<HostRun *>(run);
+    const int me = r.thread_num();
+    const std::function<void()> *const idle = me == 0 ? r.idle : nullptr;       // the caller is thread 0
+    work_on(*r.job, me, idle);
+    // another thread's block may wait for what only the caller's idle() brings about: it stays until all are through
+    while (idle && r.job->done.load(std::memory_order_acquire) < (int32_t)r.job->blocks.size()) {
+        (*idle)();
+        host_pause();
+    }
+}
+
+inline int host_threads(const CgHostTeam *team)
+{
+    if (!team || !team->parallel || !team->thread_num || team->threads < 1) return 1;
+    return std::min(team->threads, kHostThreads);
+}
+
+inline void run_job(HostJob &job, const CgHostTeam *team, const std::function<void()> *idle)
+{
+    if (job.nthreads > 1 && job.blocks.size() > 1) {
+        HostRun r = {&job, idle, team->thread_num};
+        team->parallel(&host_member, &r, (unsigned)job.nthreads, 0u);
+    } else {
+        work_on(job, 0, idle);
+    }
+}
+
+// Blocks of one copy; `home`: the address by which they are dealt to the threads, which moves with the copy.
+inline void add_blocks(HostJob &job, uint8_t *dst, const uint8_t *src, int64_t n, uintptr_t home, int32_t value, int32_t step)
+{
+    while (n > 0) {
+        const int64_t m = std::min<int64_t>(n, kHostBlock - (int64_t)(home % kHostBlock));
+        job.blocks.push_back({dst, src, (int32_t)m, (int32_t)(home / kHostBlock % (uintptr_t)job.nthreads), value, step});
+        dst += m;
+        src += m;
+        home += (uintptr_t)m;
+        n -= m;
+    }
+}
+
+inline void seal(HostJob &job, int steps)
+{
+    job.taken = std::vector<std::atomic<uint8_t>>(job.blocks.size());
+    job.left = std::vector<std::atomic<int32_t>>((size_t)steps);
+    for (const HostBlock &b : job.blocks) job.left[(size_t)b.step].fetch_add(1, std::memory_order_relaxed);
+}
+
+// Where the steps of an upload begin: the first is a quarter of one so that the bus has something to do soon.
+struct HostSteps {
+    int64_t step;
+    int64_t start(int64_t k) const { return k == 0 ? 0 : k == 1 ? step / 4 : (k - 1) * step; }
+    int64_t of(int64_t at) const { return at < step / 4 ? 0 : at < step ? 1 : at / step + 1; }
+};
+
+}  // namespace

@@ -70,8 +70,10 @@ int launch_move_bytes(const uint8_t *src, uint8_t *dst, int64_t n, bool to_host,
     return check_launch("move_bytes");
 }
 
-// Until *mark >= value: the word is read for a while (20 ms are two hundred MB on the bus), then the stream is
-// waited for, which also finds out about a launch that failed.
+// The word is read for so long, then the stream is waited for, which also finds out about a launch that failed.
+constexpr std::chrono::milliseconds kMarkPatience{200};
+
+// Until *mark >= value.
 int wait_for_mark(const int32_t *mark, int32_t value, hipStream_t stream)
 {
     const auto start = std::chrono::steady_clock::now();
@@ -80,12 +82,43 @@ int wait_for_mark(const int32_t *mark, int32_t value, hipStream_t stream)
             if (__atomic_load_n(mark, __ATOMIC_ACQUIRE) >= value) return CG_OK;
             __builtin_ia32_pause();
         }
-        if (std::chrono::steady_clock::now() - start > std::chrono::milliseconds(20)) break;
+        if (std::chrono::steady_clock::now() - start > kMarkPatience) break;
     }
     const hipError_t e = hipStreamSynchronize(stream);
     if (e != hipSuccess) return fail(CG_ERR_LAUNCH, "wait_mark: %s", hipGetErrorString(e));
     if (__atomic_load_n(mark, __ATOMIC_ACQUIRE) >= value) return CG_OK;
     return fail(CG_ERR_ARG, "wait_mark: nothing on this stream sets the mark");
 }
+
+// The same for a caller that does something else meanwhile.
+class MarkWatch {
+public:
+    MarkWatch(const int32_t *mark, hipStream_t stream) : mark_(mark), stream_(stream), last_(__atomic_load_n(mark, __ATOMIC_RELAXED)) {}
+
+    // Whether the mark is short of `value` and has not moved for that long.
+    bool overdue(int32_t value)
+    {
+        const int32_t now = __atomic_load_n(mark_, __ATOMIC_ACQUIRE);
+        if (++looks_ % 64 && now == last_) return false;
+        const auto t = std::chrono::steady_clock::now();
+        if (now != last_) since_ = t;
+        last_ = now;
+        return now < value && t - since_ > kMarkPatience;
+    }
+
+    int settle()
+    {
+        since_ = std::chrono::steady_clock::now();
+        const hipError_t e = hipStreamSynchronize(stream_);
+        return e == hipSuccess ? CG_OK : fail(CG_ERR_LAUNCH, "moves: %s", hipGetErrorString(e));
+    }
+
+private:
+    const int32_t *mark_;
+    hipStream_t stream_;
+    int32_t last_;
+    uint32_t looks_ = 0;
+    std::chrono::steady_clock::time_point since_ = std::chrono::steady_clock::now();
+};
 
 }  // namespace

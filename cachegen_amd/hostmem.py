@@ -7,6 +7,9 @@ the interpreter lock: 6 MB in 16 us warm and 45 us out of memory the GPU has jus
 one thread (numpy, bytes()) takes 80 and 200."""
 import collections
 import ctypes
+import os
+import re
+import struct
 import threading
 import warnings
 
@@ -25,12 +28,39 @@ with warnings.catch_warnings():
     torch.frombuffer(b"\0", dtype=torch.uint8)
 
 
+_TEAM = struct.Struct("<2Q2i")           # CgHostTeam
 _libc = ctypes.CDLL(None)
 _libc.madvise.argtypes = [ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int]
 _libc.mincore.argtypes = [ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]
 _MADV_HUGEPAGE = 14
 _PAGE = 4096
 _HUGE_PAGE = 2 << 20
+
+
+def _openmp():
+    """(GOMP_parallel, omp_get_thread_num) of the OpenMP runtime that torch has loaded, as addresses; (0, 0) where there
+    is none."""
+    try:
+        with open("/proc/self/maps") as f:
+            paths = {line.split(None, 5)[-1].strip() for line in f if re.search(r"/lib(g|i|)omp[^/]*$", line)}
+        for path in sorted(paths, key=lambda p: not p.startswith(os.path.dirname(torch.__file__))):
+            runtime = ctypes.CDLL(path)
+            if hasattr(runtime, "GOMP_parallel") and hasattr(runtime, "omp_get_thread_num"):
+                return tuple(ctypes.cast(fn, ctypes.c_void_p).value for fn in (runtime.GOMP_parallel, runtime.omp_get_thread_num))
+    except OSError:
+        pass
+    return 0, 0
+
+
+_runtime = None
+
+
+def team() -> bytes:
+    """CgHostTeam: torch's threads, as many as torch uses."""
+    global _runtime
+    if _runtime is None:
+        _runtime = _openmp()
+    return _TEAM.pack(*_runtime, torch.get_num_threads(), 0)
 
 
 def view(buffer) -> torch.Tensor:
@@ -44,9 +74,8 @@ def new_bytes(n: int):
     through the tensor before anybody else sees the object.
 
     Memory that the allocator has just got from the system is made present here: asked for in huge
-    pages (a page fault per 4 KB costs more than the copy that causes it) and written once by all
-    threads at the same time (a blob is filled section by section, and the threads of one section's
-    copy wait for the zeroing of the same page).  A 15 MB pickle blob made and dropped: 0.95 ms
+    pages (a page fault per 4 KB costs more than the copy that causes it), each by one of a few
+    threads (the threads of a copy wait for the zeroing of the same page).  A 15 MB pickle blob made and dropped: 0.95 ms
     without, 0.55 with; a blob that gets memory used before is not written twice (54 MB in nine blobs
     of a store: 0.5 ms more if it were)."""
     b = _new(None, n)
@@ -59,7 +88,7 @@ def new_bytes(n: int):
             fresh += _libc.mincore(page + _HUGE_PAGE - _PAGE, _PAGE, ctypes.byref(present)) == 0 and not present.value & 1
         if 2 * fresh * _HUGE_PAGE > last - first:
             _libc.madvise(first, last - first, _MADV_HUGEPAGE)
-            t.fill_(0)
+            _lib.check(_lib.lib().cg_host_present(first, last - first, _HUGE_PAGE, team()))
     return b, t
 
 
@@ -97,6 +126,9 @@ class StoredWords:
     def __exit__(self, *exc):
         if not self._through:
             self._wait()
+
+
+_PART = struct.Struct("<3q2i")           # CgHostPart
 
 
 class Arrival:
@@ -156,6 +188,39 @@ class Moves:
         self._coming_down.append((self._count, host))
         return arrival
 
+    def fill(self, parts):
+        """parts: [(uint8 tensor in ordinary memory, uint8 tensor of the same size in pinned memory, its arrival
+        or None)]: copies each as it arrives."""
+        last = max((a._number for _, _, a in parts if a is not None), default=0)
+        with torch.cuda.device(self.device):
+            if self._marked < last:
+                self._mark()
+            described = b"".join(_PART.pack(dst.data_ptr(), src.data_ptr(), dst.numel(), 0 if a is None else a._number, 0)
+                                 for dst, src, a in parts)
+            _lib.check(_lib.lib().cg_host_fill(described, len(parts), self._at, team(), self.stream))
+        self._have(last)
+
+    def stage(self, pieces, base, size, step, slots=0):
+        """`size` bytes at the device address `base` from pieces of ordinary memory ((offset, uint8 tensor), in order): copied
+        to pinned memory and moved by steps as they are there.  slots: pinned steps that are used in turn (0: as
+        many as it takes)."""
+        nsteps = -(-size // step)
+        if slots and slots < nsteps:
+            pinned = [torch.empty(step, dtype=torch.uint8, pin_memory=True) for _ in range(slots)]
+            places = [t.data_ptr() for t in pinned]
+        else:
+            pinned = [torch.empty(size, dtype=torch.uint8, pin_memory=True)]
+            places = [pinned[0].data_ptr() + i * step for i in range(nsteps)]
+        described = b"".join(_PART.pack(at, t.data_ptr(), t.numel(), 0, 0) for at, t in pieces)
+        launched = ctypes.c_int(0)
+        rc = _lib.lib().cg_host_stage(described, len(pieces), (ctypes.c_void_p * len(places))(*places), len(places), step, base, size, self._at, self._count,
+                                      team(), ctypes.byref(launched), self.stream)
+        if launched.value:
+            self._count += launched.value
+            self._marked = self._count - 1
+            self._going_up += [(self._count, t) for t in pinned]
+        _lib.check(rc)
+
     def up(self, host, dst):
         """Pinned memory to a device address; `host` is kept until it has been read."""
         arrival = self._move(host.data_ptr(), dst, host.numel(), 0)
@@ -169,12 +234,18 @@ class Moves:
         if self._reached < number:
             with torch.cuda.device(self.device):
                 if self._marked < number:
-                    _lib.check(_lib.lib().cg_mark(self._at, self._count, self.stream))
-                    self._marked = self._count
+                    self._mark()
                 _lib.check(_lib.lib().cg_wait_mark(self._at, number, self.stream))
-            self._reached = number
-            while self._coming_down and self._coming_down[0][0] <= number:
-                del self._coming_down[0]
+            self._have(number)
+
+    def _mark(self):
+        _lib.check(_lib.lib().cg_mark(self._at, self._count, self.stream))
+        self._marked = self._count
+
+    def _have(self, number):
+        self._reached = max(self._reached, number)
+        while self._coming_down and self._coming_down[0][0] <= number:
+            del self._coming_down[0]
 
     def hold(self, event):
         """Keeps what is still going up, and the word, until `event`, recorded behind all moves."""

@@ -18,11 +18,10 @@ from .. import _lib, codec, hostmem
 from . import wire
 
 _ALIGN = 256
-# Uploads of more than _WHOLE_BYTES are cut into pieces of _PIECE_BYTES: below it, one host copy
-# and one transfer are faster than several of each (6 MB: 135 us whole, 151 in pieces of 4 MB),
-# above it the overlap pays (54 MB: 1.51 ms whole, 1.25 in pieces).
+# Uploads of more than _WHOLE_BYTES have a stream of their own (_upload) and pass through a few pinned pieces.  Pieces
+# are moved by a launch each, which costs the bus 2 us (53 MB by 2 MB: 1.1 ms, by 4 MB 1.04).
 _WHOLE_BYTES = 16 << 20
-_PIECE_BYTES = 4 << 20
+_PIECE_BYTES, _PIECES = 4 << 20, 4
 
 _ITEM = struct.Struct("<10q4i")      # CgHostContainer
 _SUB_BYTES = 96                      # sizeof(CgListedSub)
@@ -81,11 +80,11 @@ def _upload(pieces, total, index_at, write_index):
     index_at on, what write_index(device address, uint8 tensor in pinned memory) puts there;
     write_index runs while the pieces before it are on the bus.
 
-    A transfer in pieces has a stream of its own, which the current stream waits for: the blobs of a
+    A large transfer has a stream of its own, which the current stream waits for: the blobs of a
     call are on the bus while what the caller queued before (as a rule the decode of the blobs before
     them) still runs (32 blobs of 54 MB in all, one call behind the other: 1.46 -> 1.28 ms).  The
     buffer comes from that stream's memory and goes back when the current stream is through with it.
-    For a single piece the events and the change of stream cost more than they hide (+25 us)."""
+    For a small one the events and the change of stream cost more than they hide (+25 us)."""
     device = torch.device("cuda", torch.cuda.current_device())          # the caller made it current
     if index_at <= _WHOLE_BYTES:
         return _transfer(pieces, total, index_at, write_index, device)[0]
@@ -103,22 +102,13 @@ def _upload(pieces, total, index_at, write_index):
 def _transfer(pieces, total, index_at, write_index, device):
     buf = torch.empty(total, dtype=torch.uint8, device=device)
     base = buf.data_ptr()
-    step = index_at if index_at <= _WHOLE_BYTES else _PIECE_BYTES
-    k = 0
     hostmem.let_go()
     moves = hostmem.Moves(device, codec._stream(device))
     try:
-        for p0 in range(0, index_at, step):
-            p1 = min(p0 + step, index_at)
-            host = torch.empty(p1 - p0, dtype=torch.uint8, pin_memory=True)
-            while k < len(pieces) and pieces[k][0] < p1:
-                off, src = pieces[k]
-                a, b = max(off, p0), min(off + src.numel(), p1)
-                host[a - p0:b - p0].copy_(src[a - off:b - off])
-                if off + src.numel() > p1:
-                    break
-                k += 1
-            moves.up(host, base + p0)
+        if index_at <= _WHOLE_BYTES:
+            moves.stage(pieces, base, index_at, _PIECE_BYTES // 128 * 64)
+        else:
+            moves.stage(pieces, base, index_at, _PIECE_BYTES, _PIECES)
         host = torch.empty(total - index_at, dtype=torch.uint8, pin_memory=True)
         write_index(base, host)
         moves.up(host, base + index_at)

@@ -96,8 +96,9 @@ class _Writer:
     and back 2.06-2.17 ms one after the other, 1.80-1.93 so, in turn on one machine; on another the
     two were within their runs' spread, 2.09 and 2.13)."""
 
-    def __init__(self, location: str, arrive):
-        self.location, self.arrive = location.encode(), arrive
+    def __init__(self, location: str, arrive, fill=None):
+        """fill: copies [(bytes of the blob, host memory that `arrive` waits for)], waiting for it."""
+        self.location, self.arrive, self.fill = location.encode(), arrive, fill or self._fill
         self.large = {}              # id of a stand-in bytes object of _LARGE bytes -> (object, prefix, host tensor)
         self.count = 0
 
@@ -143,16 +144,21 @@ class _Writer:
         if seen != len(self.large):
             raise RuntimeError("pickle: a stand-in was copied instead of passed through")
         blob, into = hostmem.new_bytes(sum(len(p) if type(p) is bytes else p.numel() for p in parts))
-        raw, at = into.numpy(), 0
-        self.arrive()
+        raw, at, large = into.numpy(), 0, []
         for p in parts:
             if type(p) is bytes:
                 raw[at:at + len(p)] = np.frombuffer(p, dtype=np.uint8)
                 at += len(p)
             else:
-                into[at:at + p.numel()].copy_(p)
+                large.append((into[at:at + p.numel()], p))
                 at += p.numel()
+        self.fill(large)
         return blob
+
+    def _fill(self, large):
+        self.arrive()
+        for into, host in large:
+            into.copy_(host)
 
 
 def can_write(enc) -> bool:
@@ -166,7 +172,7 @@ def pack_chunks(enc):
     rows, C = 2 * L, H * D
     blobs = []
     for part in wire.bring_to_host(enc, 0, enc.num_chunks):
-        w = _Writer(str(enc.payload.device), part.arrive)
+        w = _Writer(str(enc.payload.device), part.arrive, lambda large: part.fill([(into, host, part.arrived) for into, host in large]))
         T = part.t1 - part.t0
         maxima = torch.from_numpy(np.ascontiguousarray(part.maxima).view(np.uint8).reshape(-1))
         half = maxima.numel() // 2

@@ -347,17 +347,14 @@ class HostPart:
     `lengths_itemsize` 2 or 4.  Sizes are known and the maxima are there from the start; the other
     bytes are there after `arrive`."""
 
-    def table_slices(self):
-        """(start, end) slices of `tables`, each there when it is yielded."""
-        at = 0
-        for end, arrival in self.slices:
-            arrival.synchronize()
-            yield at, end
-            at = end
-
     def arrive(self):
         """Waits for everything."""
         self.arrived.synchronize()
+
+    def fill(self, parts):
+        """[(uint8 tensor in ordinary memory, slice of `tables`, `lengths` or `payload`, its arrival)]: copied as they
+        arrive."""
+        self.moves.fill(parts)
 
 
 def bring_to_host(enc, first_chunk, num_chunks, per_chunk=True, compact=False):
@@ -473,7 +470,7 @@ def _bring_to_host(enc, first_chunk, num_chunks, per_chunk, compact, moves):
     itemsize = lengths_src.element_size()
     queued = queue(pieces[0])
     for k, piece in enumerate(pieces):
-        ((tables, slices), (lens, _), (payload, arrived)), queued = queued, queue(pieces[k + 1]) if k + 1 < len(pieces) else None
+        ((tables, slices), (lens, lens_arrived), (payload, arrived)), queued = queued, queue(pieces[k + 1]) if k + 1 < len(pieces) else None
         at = [0, 0, 0]
         for a, b in groups[piece[0]:piece[1]]:
             part = HostPart()
@@ -487,7 +484,7 @@ def _bring_to_host(enc, first_chunk, num_chunks, per_chunk, compact, moves):
             part.maxima = maxima.numpy().view(np.uint16).reshape(rows, T)[:, part.t0:part.t1]
             part.symbols = None if symbols is None else symbols[(a - c_first) * rows:(b - c_first) * rows]
             part.lengths_itemsize = itemsize
-            part.arrived = arrived
+            part.moves, part.lengths_arrived, part.arrived = moves, lens_arrived, arrived
             # several blobs in a piece: all of the piece's tables, there with its last slice
             part.slices = slices if piece[1] - piece[0] == 1 else [(n[0], slices[-1][1])]
             yield part
@@ -524,7 +521,7 @@ def pack_chunks(enc, first_chunk: int = 0, num_chunks: Optional[int] = None, per
         if part.symbols is not None:
             head += part.symbols.tobytes()
         blob, into = hostmem.new_bytes(geo["total"][0])
-        raw = into.numpy()
+        raw, parts = into.numpy(), []
         end = len(head)
         raw[:end] = np.frombuffer(head, dtype=np.uint8)
         for section, src in (("cdf", part.tables), ("maxima", part.maxima), ("lengths", part.lengths), ("payload", part.payload)):
@@ -533,14 +530,16 @@ def pack_chunks(enc, first_chunk: int = 0, num_chunks: Optional[int] = None, per
             raw[end:start] = 0                           # the gap before the section
             end = off + size
             if section == "cdf":
-                for a, b in part.table_slices():
-                    into[start + a:start + b].copy_(src[a:b])
-                part.arrive()
+                at = 0
+                for e, arrival in part.slices:
+                    parts.append((into[start + at:start + e], src[at:e], arrival))
+                    at = e
             elif section == "maxima":
                 np.copyto(raw[start:end].view(np.uint16).reshape(2 * L, T), src)
             else:
-                into[start:end].copy_(src)
+                parts.append((into[start:end], src, part.lengths_arrived if section == "lengths" else part.arrived))
         raw[end:] = 0
+        part.fill(parts)
         blobs.append(blob)
     return blobs
 

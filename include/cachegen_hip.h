@@ -390,6 +390,41 @@ int cg_mark(int32_t *mark, int32_t value, void *stream);
 /* HOST: returns when *mark >= value; CG_ERR_ARG if the stream is through and it is not. */
 int cg_wait_mark(const int32_t *mark, int32_t value, void *stream);
 
+/* The threads of a host function: those of an OpenMP runtime, through its documented entry points, at most `threads`
+ * of them.  Null, or null pointers: the caller alone. */
+typedef struct CgHostTeam {
+    void (*parallel)(void (*fn)(void *), void *data, unsigned num_threads, unsigned flags);      /* GOMP_parallel */
+    int (*thread_num)(void);                                                                     /* omp_get_thread_num */
+    int32_t threads;
+    int32_t reserved;
+} CgHostTeam;
+
+/* One copy on the host. */
+typedef struct CgHostPart {
+    int64_t dst, src;               /* addresses; cg_host_stage: dst is an offset in the area */
+    int64_t bytes;
+    int32_t value;                  /* cg_host_fill: src is there when the mark is this far */
+    int32_t reserved;
+} CgHostPart;
+
+/* HOST: the copies, by the team, each part as soon as *mark says that it has arrived; returns when all
+ * are done.  The launches that set the mark have been queued on the stream. */
+int cg_host_fill(const CgHostPart *parts, int n, const int32_t *mark, const CgHostTeam *team, void *stream);
+
+/* HOST: n bytes of memory that is new to the process made present by the team, `page` bytes (a multiple of 4096: the
+ * size of its large pages) at a time; `at` is a multiple of 4096, and the bytes are undefined afterwards. */
+int cg_host_present(void *at, int64_t n, int64_t page, const CgHostTeam *team);
+
+/* HOST and the stream: `bytes` bytes of device memory at `area` from the parts (ascending, not overlapping; what lies
+ * between them is undefined), staged in pinned memory by the team and moved in steps, each as soon as it is staged.
+ * step   bytes of a step, a multiple of 64 (the first is a quarter of one)
+ * slots  HOST array of nslots addresses of pinned memory, a step each, used in turn: two at least, or as many as
+ *        there are steps (the last of them then no larger than what is left); stays valid until the moves are through
+ * mark, value  as in cg_move_bytes, `value` for the first move and one more for each
+ * moves  written: the moves launched (all of them, or those before an error) */
+int cg_host_stage(const CgHostPart *parts, int n, void *const *slots, int nslots, int64_t step, void *area, int64_t bytes,
+                  int32_t *mark, int32_t value, const CgHostTeam *team, int *moves, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

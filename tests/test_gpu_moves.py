@@ -72,3 +72,38 @@ def test_marks_are_refused_where_they_cannot_be_set():
         _lib.check(lib.cg_wait_mark(word.data_ptr(), 1, codec._stream(DEV)))
     with pytest.raises(RuntimeError, match="nothing to move"):
         _lib.check(lib.cg_move_bytes(word.data_ptr(), word.data_ptr(), 0, 1, None, 0, None))
+
+
+# slots for everything, two and eight in turn; steps of 64 bytes and up; pieces with gaps between them
+@pytest.mark.parametrize("slots", [0, 2, 8])
+@pytest.mark.parametrize("step,size", [(64, 1000), (4352, 8 * 4352), (4352, 8 * 4352 + 1), (4352, 300001), (2 << 20, (20 << 20) + 77)])
+def test_staged_pieces_arrive(step, size, slots):
+    print(step, size, slots, flush=True)
+    g = torch.Generator().manual_seed(size)
+    cuts = sorted({0, size, *(int(x) for x in torch.randint(0, size, (9,), generator=g))})
+    pieces = [(a, _bytes(b - a - (1 if b - a > 5 and i % 2 else 0), i)) for i, (a, b) in enumerate(zip(cuts, cuts[1:]))]
+    dev = torch.full((size + GUARD,), 8, dtype=torch.uint8, device=DEV)
+    with torch.cuda.device(DEV):
+        for _ in range(3):
+            hostmem.let_go()
+            moves = hostmem.Moves(DEV, codec._stream(DEV))
+            moves.stage(pieces, dev.data_ptr(), size, step, slots)
+            event = torch.cuda.Event()
+            event.record()
+            moves.hold(event)
+    got = dev.cpu()
+    for at, want in pieces:
+        assert torch.equal(got[at:at + want.numel()], want)
+    assert (got[size:] == 8).all()
+
+
+def test_parts_are_filled_as_they_come():
+    src = torch.arange(3 << 20, dtype=torch.int32, device=DEV).view(torch.uint8)
+    n = src.numel()
+    with torch.cuda.device(DEV), hostmem.Moves(DEV, codec._stream(DEV)) as moves:
+        a, b = moves.down(src[:n // 3]), moves.down(src[n // 3 + 1:])
+        whole = torch.zeros(n, dtype=torch.uint8)
+        moves.fill([(whole[:n // 3], *a), (whole[n // 3 + 1:], *b)])
+    want = src.cpu()
+    want[n // 3] = 0
+    assert torch.equal(whole, want)

@@ -1,0 +1,133 @@
+"""Copies between ordinary and pinned memory by several threads (cg_host_fill), on the CPU: the mark is an ordinary
+word that the test sets."""
+import concurrent.futures
+import ctypes
+import struct
+import threading
+import time
+
+import pytest
+import torch
+
+from cachegen_amd import _lib, hostmem
+
+PART = struct.Struct("<3q2i")
+
+
+def team(threads):
+    """CgHostTeam of so many threads; 0: none."""
+    return struct.pack("<2Q2i", *hostmem._openmp(), threads, 0) if threads else None
+
+
+def fill(parts, mark, threads):
+    raw = b"".join(PART.pack(d.data_ptr(), s.data_ptr(), d.numel(), v, 0) for d, s, v in parts)
+    _lib.check(_lib.lib().cg_host_fill(raw, len(parts), mark.data_ptr(), team(threads), None))
+
+
+def test_torchs_threads_are_found():
+    parallel, number, threads, _ = struct.unpack("<2Q2i", hostmem.team())
+    assert parallel and number and threads == torch.get_num_threads()
+
+
+def data(n, seed):
+    return torch.randint(0, 256, (n,), generator=torch.Generator().manual_seed(seed), dtype=torch.uint8)
+
+
+# nothing, a byte, either side of a block, blocks dealt to more threads than there are
+@pytest.mark.parametrize("threads", [0, 1, 3, 64])
+@pytest.mark.parametrize("sizes", [(0, 1), ((64 << 10) - 1, 64 << 10, (64 << 10) + 1), (5, (3 << 20) + 17, 0, 300001)])
+def test_parts_are_copied(threads, sizes):
+    src = [data(n + 3, n)[3:] for n in sizes]
+    room = torch.full((sum(sizes) + 7 * len(sizes) + 1,), 9, dtype=torch.uint8)
+    dst, at = [], 1
+    for n in sizes:
+        dst.append(room[at:at + n])
+        at += n + 7
+    mark = torch.zeros(1, dtype=torch.int32)
+    fill([(d, s, 0) for d, s in zip(dst, src)], mark, threads)
+    assert all(torch.equal(d, s) for d, s in zip(dst, src))
+    assert int((room == 9).sum()) >= 7 * len(sizes) + 1                     # nothing between the parts was written
+    keep = torch.ones_like(room, dtype=torch.bool)
+    at = 1
+    for n in sizes:
+        keep[at:at + n] = False
+        at += n + 7
+    assert (room[keep] == 9).all()
+
+
+@pytest.mark.parametrize("threads", [1, 6])
+def test_a_part_is_read_only_when_it_has_arrived(threads):
+    n = 400000
+    want = [data(n, i) for i in range(4)]
+    src = [torch.zeros(n, dtype=torch.uint8) for _ in want]
+    dst = [torch.zeros(n, dtype=torch.uint8) for _ in want]
+    mark = torch.zeros(1, dtype=torch.int32)
+    word = ctypes.c_int32.from_address(mark.data_ptr())
+
+    def arrive():
+        for i, w in enumerate(want):
+            time.sleep(0.002)
+            src[i].copy_(w)
+            word.value = i + 1
+    t = threading.Thread(target=arrive)
+    t.start()
+    fill([(d, s, i + 1) for i, (d, s) in enumerate(zip(dst, src))], mark, threads)
+    t.join()
+    assert all(torch.equal(d, w) for d, w in zip(dst, want))
+
+
+def test_callers_side_by_side():
+    """Several jobs at once, some of them waiting for their marks."""
+    wrong = []
+
+    def caller(i):
+        mark = torch.zeros(1, dtype=torch.int32)
+        word = ctypes.c_int32.from_address(mark.data_ptr())
+        for k in range(10):
+            s, d = data(200000 + 977 * i, 31 * i + k), torch.zeros(200000 + 977 * i, dtype=torch.uint8)
+            late = threading.Timer(0.001, lambda v=k + 1: setattr(word, "value", v))
+            late.start()
+            try:
+                fill([(d[:100000], s[:100000], k), (d[100000:], s[100000:], k + 1)], mark, 4)
+            except RuntimeError as e:
+                wrong.append((i, k, e))
+            late.join()
+            if not torch.equal(d, s):
+                wrong.append((i, k))
+    callers = [threading.Thread(target=caller, args=(i,)) for i in range(6)]
+    for c in callers:
+        c.start()
+    for c in callers:
+        c.join()
+    assert not wrong
+
+
+@pytest.mark.parametrize("threads", [1, 4])
+@pytest.mark.parametrize("at,n", [(0, 1), (0, 512), (3, 509), (1, 1600), (511, 2)])          # in pages of 4 KB, 512 to a large one
+def test_memory_is_made_present(at, n, threads):
+    import mmap
+    libc = ctypes.CDLL(None)
+    region = mmap.mmap(-1, 8 << 20)
+    start = ctypes.addressof(ctypes.c_char.from_buffer(region))
+    first = -(-start // (2 << 20)) * (2 << 20) + at * 4096
+    _lib.check(_lib.lib().cg_host_present(first, n * 4096, 2 << 20, team(threads)))
+    there = (ctypes.c_ubyte * n)()
+    assert libc.mincore(ctypes.c_void_p(first), ctypes.c_size_t(n * 4096), there) == 0
+    assert all(b & 1 for b in there)
+
+
+def _refuse_bad_parts():
+    with pytest.raises(RuntimeError, match="whole pages"):
+        _lib.check(_lib.lib().cg_host_present(4096 + 8, 4096, 4096, None))
+    mark = torch.zeros(1, dtype=torch.int32)
+    with pytest.raises(RuntimeError, match="bad part"):
+        _lib.check(_lib.lib().cg_host_fill(PART.pack(0, 0, 5, 0, 0), 1, mark.data_ptr(), None, None))
+    with pytest.raises(RuntimeError, match="nothing to copy"):
+        _lib.check(_lib.lib().cg_host_fill(PART.pack(0, 0, 0, 0, 0), 0, mark.data_ptr(), None, None))
+    with pytest.raises(RuntimeError, match="too small"):
+        _lib.check(_lib.lib().cg_host_stage(PART.pack(0, 0, 0, 0, 0), 0, (ctypes.c_void_p * 1)(64), 1, 64, 64, 1000, mark.data_ptr(), 0, None, ctypes.byref(ctypes.c_int()), None))
+
+
+def test_bad_parts_are_refused():
+    with concurrent.futures.ThreadPoolExecutor(1) as other:                 # the last error's text belongs to a thread
+        other.submit(_refuse_bad_parts).result()
