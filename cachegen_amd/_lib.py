@@ -54,6 +54,10 @@ SIGNATURES = {
     "cg_host_fill": (_INT, [_P, _INT, _P, _P, _P]),
     "cg_host_present": (_INT, [_P, _I64, _I64, _P]),
     "cg_host_stage": (_INT, [_P, _INT, _P, _INT, _I64, _P, _I64, _P, _INT, _P, _P, _P]),
+    "cg_read_words": (_INT, [_P, _P, _INT, _P, _INT, _P]),
+    "cg_largest": (_INT, [_P, _P, _I64, _P, _INT, _P]),
+    "cg_scan_collect": (_INT, [_P, _I64, _P, _P, _SZ, _I64, _I64, _P, _INT, _P]),
+    "cg_decode_fast_lengths": (_INT, [_P, _INT, _P, _I64, _P, _I64, _I64, _I64, _P, _I64, _I64, _I64, _P, _P, _SZ, _P]),
     "cg_mark": (_INT, [_P, _INT, _P]),
     "cg_wait_mark": (_INT, [_P, _INT, _P]),
     "cg_lengths_to_u16": (_INT, [_P, _I64, _P, _P, _P]),

@@ -26,6 +26,14 @@ def _stream(device):
 
 def _largest(key_bins, value_bins):
     """The larger of two bins vectors' largest values: one read of the device for both."""
+    if key_bins.is_cuda and key_bins.device == value_bins.device and key_bins.dtype == value_bins.dtype == torch.float32 \
+            and key_bins.shape == value_bins.shape and key_bins.numel() and key_bins.is_contiguous() and value_bins.is_contiguous() \
+            and not torch.cuda.is_current_stream_capturing():
+        with torch.cuda.device(key_bins.device), hostmem.Words() as words:
+            _lib.check(_lib.lib().cg_largest(key_bins.data_ptr(), value_bins.data_ptr(), key_bins.numel(), words.at, words.value,
+                                             _stream(key_bins.device)))
+            largest = words.number()
+        return int(largest)
     if key_bins.device == value_bins.device:
         return int(float(torch.maximum(key_bins, value_bins).max()))
     return int(max(float(key_bins.max()), float(value_bins.max())))
@@ -80,10 +88,11 @@ class EncodedKV:
         return self.offsets[idx].tolist()
 
     def total_bytes(self):
-        return int(self.offsets[-1].item())
+        return int(hostmem.read_number(self.offsets, -1))
 
     def check(self):
-        self.raise_for_status(int(self.status.item()))
+        self.raise_for_status(int(hostmem.read_number(self.status, 0) if self.status.dim() == 1 and self.status.numel() == 1
+                                  else self.status.item()))
 
     @staticmethod
     def raise_for_status(st):
@@ -216,11 +225,40 @@ def collect_streams(padded, offsets):
     if padded.numel() == 0:
         raise RuntimeError("padded streams: the buffer has no slots")
     n, nslots = offsets.numel() - 1, padded.numel() // cap
+
+    def queue(words, stream):
+        words.clear()
+        _lib.check(_lib.lib().cg_collect_sizes(offsets.data_ptr(), n, nslots, cap, words.at, stream))
+        _lib.check(_lib.lib().cg_mark(words.mark, words.value, stream))
+    return _collect(padded, offsets, n, nslots, queue)
+
+
+def collect_lengths(padded, lengths):
+    """collect_streams from the streams' lengths (int32, any shape, in the order of the buffer's slots)."""
+    if lengths.dtype != torch.int32 or not lengths.is_cuda:
+        raise RuntimeError("stream lengths should be int32 on a GPU, got %s on %s" % (lengths.dtype, lengths.device))
+    dev, cap, n = lengths.device, padded.shape[-1], lengths.numel()
+    if n == 0:
+        return collect_streams(padded, scan_lengths(lengths))
+    if not padded.is_cuda or padded.device != dev:
+        raise RuntimeError("padded streams and offsets should be on the same GPU, got %s and %s" % (padded.device, dev))
+    if padded.numel() == 0:
+        raise RuntimeError("padded streams: the buffer has no slots")
+    nslots = padded.numel() // cap
+    flat = lengths.contiguous().view(-1)
+    offsets = torch.empty(n + 1, dtype=torch.int64, device=dev)
+    scratch = torch.empty(int(_lib.lib().cg_scan_workspace(n)), dtype=torch.uint8, device=dev)
+    return _collect(padded, offsets, n, nslots, lambda words, stream: _lib.check(_lib.lib().cg_scan_collect(
+        flat.data_ptr(), n, offsets.data_ptr(), scratch.data_ptr(), scratch.numel(), nslots, cap, words.at, words.value, stream)))
+
+
+def _collect(padded, offsets, n, nslots, queue):
+    """queue(words, stream) launches what stores the streams' total size, and whether they do not fit their slots, in `words`."""
+    dev, cap = padded.device, padded.shape[-1]
     with torch.cuda.device(dev):
         lib, stream = _lib.lib(), _stream(dev)
-        with hostmem.StoredWords(2, torch.int64) as words:
-            _lib.check(lib.cg_collect_sizes(offsets.data_ptr(), n, nslots, cap, words.words.data_ptr(), stream))
-            words.stored()
+        with hostmem.Words() as words:
+            queue(words, stream)
             if padded.dim() != 3:
                 padded = padded.reshape(1, -1, cap)
             if padded.stride(2) != 1:
@@ -228,7 +266,8 @@ def collect_streams(padded, offsets):
             nl, nc, _ = padded.shape
             p0, p1, _ = padded.stride()
             size = padded.element_size()                 # the kernel moves bytes
-            total, unfit = words.read()
+            words.wait(stream)
+            total, unfit = words.numbers(2)
         if unfit:
             raise RuntimeError("padded streams: %d lengths do not fit %d slots of %d values" % (n, nslots, cap))
         out = torch.empty(total, dtype=padded.dtype, device=dev)

@@ -35,6 +35,7 @@
 
 
 #include "common.hpp"
+#include "marks.hpp"
 #include "quantize.hpp"
 #include "tables.hpp"
 #include "quantize_tables.hpp"
@@ -863,6 +864,61 @@ int cg_wait_mark(const int32_t *mark, int32_t value, void *stream)
 {
     if (!mark || !aligned_to(mark, 4)) return fail(CG_ERR_ARG, "wait_mark: null or misaligned pointer");
     return wait_for_mark(mark, value, static_cast<hipStream_t>(stream));
+}
+
+// Pinned words of one reader at a time: eight 64-bit numbers, of which the last holds the mark.
+static int32_t *words_mark(void *words) { return reinterpret_cast<int32_t *>(static_cast<int64_t *>(words) + 7); }
+
+int cg_read_words(const void *const *at, const int32_t *bytes, int n, void *words, int32_t value, void *stream)
+{
+    if (!at || !bytes || !words || n < 1 || n > 4) return fail(CG_ERR_ARG, "read_words: between 1 and 4 words");
+    WordsArgs a;
+    memset(&a, 0, sizeof(a));
+    for (int i = 0; i < n; ++i) {
+        if (!at[i] || (bytes[i] != 4 && bytes[i] != 8) || !aligned_to(at[i], (size_t)bytes[i])) return fail(CG_ERR_ARG, "read_words: bad word");
+        a.at[i] = at[i];
+        a.bytes[i] = bytes[i];
+    }
+    a.n = n;
+    a.out = static_cast<int64_t *>(words);
+    a.mark = words_mark(words);
+    a.value = value;
+    read_words_kernel<<<1, 1, 0, static_cast<hipStream_t>(stream)>>>(a);
+    if (int rc = check_launch("read_words")) return rc;
+    return wait_for_mark(a.mark, value, static_cast<hipStream_t>(stream));
+}
+
+int cg_largest(const float *a, const float *b, int64_t n, void *words, int32_t value, void *stream)
+{
+    if (!a || !b || !words || n < 1) return fail(CG_ERR_ARG, "largest: null pointer or no values");
+    largest_kernel<<<1, 64, 0, static_cast<hipStream_t>(stream)>>>(a, b, n, static_cast<float *>(words), words_mark(words), value);
+    if (int rc = check_launch("largest")) return rc;
+    return wait_for_mark(words_mark(words), value, static_cast<hipStream_t>(stream));
+}
+
+int cg_scan_collect(const int32_t *lengths, int64_t n, int64_t *offsets, void *scratch, size_t scratch_bytes, int64_t nslots, int64_t cap,
+                    void *words, int32_t value, void *stream)
+{
+    if (!words) return fail(CG_ERR_ARG, "scan_collect: null pointer");
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    int64_t *const out = static_cast<int64_t *>(words);
+    if (lengths && offsets && n > 0 && n <= kScanSmallMax && nslots > 0 && cap > 0) {
+        scan_collect_kernel<<<1, kScanSmallThreads, 0, s>>>(lengths, (int32_t)n, offsets, nslots, cap, out, words_mark(words), value);
+        return check_launch("scan_collect");
+    }
+    out[0] = out[1] = 0;
+    if (int rc = cg_scan_lengths(lengths, n, offsets, scratch, scratch_bytes, stream)) return rc;
+    if (int rc = cg_collect_sizes(offsets, n, nslots, cap, out, stream)) return rc;
+    return cg_mark(words_mark(words), value, stream);
+}
+
+int cg_decode_fast_lengths(const int16_t *cdf, int lp, const uint8_t *bytes, int64_t nbytes, const int32_t *lengths, int64_t nl, int64_t nt,
+                           int64_t nc, uint8_t *out, int64_t o0, int64_t o1, int64_t o2, int64_t *offsets, void *scratch, size_t scratch_bytes,
+                           void *stream)
+{
+    if (nl <= 0 || nc <= 0) return fail(CG_ERR_ARG, "decode: empty input");
+    if (int rc = cg_scan_lengths(lengths, nl * nc, offsets, scratch, scratch_bytes, stream)) return rc;
+    return cg_decode_fast_prefsum(cdf, lp, bytes, nbytes, offsets + 1, nl, nt, nc, out, o0, o1, o2, stream);
 }
 
 int cg_host_fill(const CgHostPart *parts, int n, const int32_t *mark, const CgHostTeam *team, void *stream)

@@ -21,13 +21,6 @@ constexpr int64_t kMovePart = 1 << 30;      // bytes a launch: offsets from a bu
 // left in the GPU's caches, a store to it goes through to it.
 constexpr int kSystemScope = 1 | 16;
 
-// Sets *mark (pinned host memory) to `value`.  A stream runs its launches one behind the other, so the host that
-// reads the value knows that all launches before this one are through, with what they stored.
-__device__ __forceinline__ void set_mark(int32_t *mark, int32_t value)
-{
-    __hip_atomic_store(mark, value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-}
-
 __global__ void mark_kernel(int32_t *mark, int32_t value) { set_mark(mark, value); }
 
 // n bytes, n <= kMovePart.  mark (may be null): set first, for what was queued before.

@@ -128,6 +128,62 @@ class StoredWords:
             self._wait()
 
 
+_free = threading.local()                # words of this thread that nobody uses
+
+
+class Words:
+    """64 pinned bytes that kernels of one call store to, for a host that looks at their mark instead of waiting for an event
+    (cg_read_words and its like); to be used in a `with` block that holds the launches and the reads.  They are
+    kept for the thread's next call; where a `with` block ends in an exception, until the process ends: something may
+    still store to them."""
+    _lost = []
+
+    def __enter__(self):
+        kept = _free.__dict__.setdefault("words", [])
+        if kept:
+            self._memory, self.value = kept.pop()
+        else:
+            self._memory, self.value = torch.zeros(8, dtype=torch.int64, pin_memory=True), 0
+        self.at = self._memory.data_ptr()
+        self.mark = self.at + 56
+        self.value = self.value % (1 << 30) + 1
+        if self.value == 1:
+            self._memory[7] = 0
+        return self
+
+    def wait(self, stream):
+        _lib.check(_lib.lib().cg_wait_mark(self.mark, self.value, stream))
+
+    def clear(self):
+        self._memory[:2] = 0
+
+    def numbers(self, n):
+        return self._memory[:n].tolist()
+
+    def number(self):
+        return ctypes.c_float.from_address(self.at).value
+
+    def __exit__(self, kind, *exc):
+        if kind is None:
+            _free.words.append((self._memory, self.value))
+        else:
+            self._lost.append(self._memory)
+
+
+def read_number(tensor, index):
+    """Entry `index` of a vector of int32 or int64, once what the current stream holds is through: tensor[index].item()."""
+    if not tensor.is_cuda or tensor.dim() != 1 or tensor.dtype not in (torch.int32, torch.int64) or torch.cuda.is_current_stream_capturing():
+        return tensor[index].item()
+    n, size = tensor.shape[0], tensor.element_size()
+    if not -n <= index < n:
+        return tensor[index].item()                      # raises
+    at = tensor.data_ptr() + index % n * tensor.stride(0) * size
+    with torch.cuda.device(tensor.device), Words() as words:
+        _lib.check(_lib.lib().cg_read_words(ctypes.byref(ctypes.c_void_p(at)), ctypes.byref(ctypes.c_int32(size)), 1, words.at, words.value,
+                                            torch._C._cuda_getCurrentRawStream(tensor.device.index)))
+        return words.numbers(1)[0]
+
+
 _PART = struct.Struct("<3q2i")           # CgHostPart
 
 

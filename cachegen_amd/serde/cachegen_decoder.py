@@ -15,8 +15,7 @@ from .serde import Deserializer
 def decode_chunk(cdf: torch.Tensor, data_chunk: CacheGenGPUBytestream, target_buffer: torch.Tensor):
     """cachegen_decoder.py:52-75: decode one sub-chunk's streams into
     target_buffer [2L, ntokens, nchannels] (a strided view is fine)."""
-    prefsum = codec.scan_lengths(data_chunk.bytestream_lengths)[1:].view(data_chunk.bytestream_lengths.shape)
-    torchac_hip.decode_fast_prefsum(cdf, data_chunk.bytestream, prefsum, target_buffer)
+    torchac_hip.decode_fast_lengths(cdf, data_chunk.bytestream, data_chunk.bytestream_lengths, target_buffer)
 
 
 def decode_function_gpu(cdf: torch.Tensor, data_chunks: List[CacheGenGPUBytestream],

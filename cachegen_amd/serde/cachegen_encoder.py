@@ -21,8 +21,7 @@ def torch_quant_vectorized(bins: torch.Tensor, input_groups: torch.Tensor):
 
 def collect_bytes(output_buffer: torch.Tensor, output_lengths: torch.Tensor) -> torch.Tensor:
     """cachegen_encoder.py:209-222: the streams of a padded buffer, back to back."""
-    offsets = codec.scan_lengths(output_lengths)
-    return codec.collect_streams(output_buffer, offsets)
+    return codec.collect_lengths(output_buffer, output_lengths)
 
 
 def encode_ntokens(cdf_int, encode_input, output_buffer, output_lengths) -> torch.Tensor:

@@ -128,3 +128,28 @@ def decode_fast_prefsum(cdf, bytestreams, lengths_prefsum, output):
         _lib.check(_lib.lib().cg_decode_fast_prefsum(
             cdf.data_ptr(), cdf.shape[2], bytestreams.data_ptr(), bytestreams.numel(),
             lengths_prefsum.data_ptr(), nl, nt, nc, output.data_ptr(), o[0], o[1], o[2], _stream(cdf.device)))
+
+
+def decode_fast_lengths(cdf, bytestreams, lengths, output):
+    """decode_fast_prefsum from the stream lengths themselves, int32 [nl, nc], whose running sum is made in the same call
+    (cachegen_decoder.py:70)."""
+    _require(lengths.dtype == torch.int32 and lengths.is_cuda,
+             "stream lengths should be int32 on a GPU, got %s on %s" % (lengths.dtype, lengths.device))
+    _require(bytestreams.is_cuda, "Bytestreams should be on GPU")
+    _check_decode(cdf, lengths, output)
+    _require(bytestreams.dtype == torch.uint8 and bytestreams.dim() == 1, "expected a 1-D uint8 bytestream")
+    cdf = cdf.contiguous()
+    bytestreams = bytestreams.contiguous()
+    lengths = lengths.contiguous()
+    nl, nt, nc = output.shape
+    if nt == 0:
+        return
+    _require(lengths.numel() == nl * nc, "one length per layer and channel")
+    lib = _lib.lib()
+    offsets = torch.empty(nl * nc + 1, dtype=torch.int64, device=cdf.device)
+    scratch = torch.empty(int(lib.cg_scan_workspace(nl * nc)), dtype=torch.uint8, device=cdf.device)
+    o = output.stride()
+    with torch.cuda.device(cdf.device):
+        _lib.check(lib.cg_decode_fast_lengths(
+            cdf.data_ptr(), cdf.shape[2], bytestreams.data_ptr(), bytestreams.numel(), lengths.data_ptr(), nl, nt, nc,
+            output.data_ptr(), o[0], o[1], o[2], offsets.data_ptr(), scratch.data_ptr(), scratch.numel(), _stream(cdf.device)))

@@ -390,6 +390,26 @@ int cg_mark(int32_t *mark, int32_t value, void *stream);
 /* HOST: returns when *mark >= value; CG_ERR_ARG if the stream is through and it is not. */
 int cg_wait_mark(const int32_t *mark, int32_t value, void *stream);
 
+/* The functions below store to `words`: 64 bytes of pinned memory, 8-byte aligned, one reader's at a time, whose last
+ * int64 begins with the mark; the mark is set to `value`, which differs from call to call, behind everything else. */
+
+/* HOST, returns when they are there: words[i] = the 4-byte (signed) or 8-byte number at at[i], device memory; n <= 4. */
+int cg_read_words(const void *const *at, const int32_t *bytes, int n, void *words, int32_t value, void *stream);
+
+/* HOST, returns when it is there: the first float of words = the largest value of the device vectors a and b, n each; NaN
+ * if there is one. */
+int cg_largest(const float *a, const float *b, int64_t n, void *words, int32_t value, void *stream);
+
+/* cg_scan_lengths and cg_collect_sizes, with its numbers in words[0] and words[1]; does not wait. */
+int cg_scan_collect(const int32_t *lengths, int64_t n, int64_t *offsets, void *scratch, size_t scratch_bytes,
+                    int64_t nslots, int64_t cap, void *words, int32_t value, void *stream);
+
+/* cg_decode_fast_prefsum from the stream lengths (device int32 [nl, nc]): offsets (device int64 [nl*nc + 1]) is written
+ * by cg_scan_lengths, whose scratch is scratch. */
+int cg_decode_fast_lengths(const int16_t *cdf, int lp, const uint8_t *bytes, int64_t nbytes, const int32_t *lengths,
+                           int64_t nl, int64_t nt, int64_t nc, uint8_t *out, int64_t o0, int64_t o1, int64_t o2,
+                           int64_t *offsets, void *scratch, size_t scratch_bytes, void *stream);
+
 /* The threads of a host function: those of an OpenMP runtime, through its documented entry points, at most `threads`
  * of them.  Null, or null pointers: the caller alone. */
 typedef struct CgHostTeam {
