@@ -52,7 +52,6 @@ SIGNATURES = {
     "cg_wire_meta": (_INT, [_P, _P, _I64, _I64, _P, _P, _P, _I64, _P, _P]),
     "cg_move_bytes": (_INT, [_P, _P, _I64, _INT, _P, _INT, _P]),
     "cg_host_fill": (_INT, [_P, _INT, _P, _P, _P]),
-    "cg_host_present": (_INT, [_P, _I64, _I64, _P]),
     "cg_host_stage": (_INT, [_P, _INT, _P, _INT, _I64, _P, _I64, _P, _INT, _P, _P, _P]),
     "cg_read_words": (_INT, [_P, _P, _INT, _P, _INT, _P]),
     "cg_largest": (_INT, [_P, _P, _I64, _P, _INT, _P]),

@@ -951,26 +951,6 @@ int cg_host_fill(const CgHostPart *parts, int n, const int32_t *mark, const CgHo
     }
 }
 
-int cg_host_present(void *at, int64_t n, int64_t page, const CgHostTeam *team)
-{
-    if (!at || n <= 0 || page < 4096 || page % 4096 || page > INT_MAX || reinterpret_cast<uintptr_t>(at) % 4096)
-        return fail(CG_ERR_ARG, "host_present: whole pages of memory are wanted");
-    try {
-        HostJob job;
-        const int32_t always = 0;
-        job.mark = &always;
-        job.nthreads = host_threads(team);
-        uint8_t *p = static_cast<uint8_t *>(at);
-        for (int64_t i = 0; i * page < n; ++i)
-            job.blocks.push_back({p + i * page, nullptr, (int32_t)std::min(page, n - i * page), (int32_t)(i % job.nthreads), 0, 0});
-        seal(job, 1);
-        run_job(job, team, nullptr);
-        return CG_OK;
-    } catch (const std::exception &e) {
-        return fail(CG_ERR_ARG, "host_present: %s", e.what());
-    }
-}
-
 int cg_host_stage(const CgHostPart *parts, int n, void *const *slots, int nslots, int64_t step, void *area, int64_t bytes, int32_t *mark,
                   int32_t value, const CgHostTeam *team, int *moves, void *stream)
 {

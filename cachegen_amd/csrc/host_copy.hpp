@@ -8,7 +8,6 @@
 #include <cstdint>
 #include <cstring>
 #include <functional>
-#include <sys/mman.h>
 #include <vector>
 
 #include "cachegen_hip.h"
@@ -28,13 +27,15 @@ namespace {
 // job also ends on its caller alone.
 //
 // Staged and moved to the GPU, one thread / eight: 1 MB 57 / 52 us, 2.7 MB 96 / 86, 6 MB 168 / 152, 14 MB 343 / 326, 53 MB 1532 / 1152;
-// copied out of pinned memory just written: 1.4 MB 40 / 20, 6 MB 157 / 61, 14 MB 364 / 130.  Sixteen: the same.
+// copied out of pinned memory just written: 1.4 MB 40 / 20, 6 MB 157 / 61, 14 MB 364 / 130.  Sixteen are as fast; a team of
+// all of torch's threads is asked for, since the runtime ends the threads that a smaller one leaves out and has to start them
+// again for torch's next operation.
 constexpr int64_t kHostBlock = 64 << 10;
-constexpr int kHostThreads = 8;
+constexpr int kHostThreads = 1024;
 
 struct HostBlock {
     uint8_t *dst;
-    const uint8_t *src;                     // null: dst's pages are made present, its bytes are undefined
+    const uint8_t *src;
     int32_t bytes;
     int32_t owner;
     int32_t value;                          // to be copied when the job's mark is this far
@@ -61,14 +62,6 @@ inline void host_pause()
 #endif
 }
 
-inline void make_present(uint8_t *at, int64_t n)
-{
-#ifdef MADV_POPULATE_WRITE
-    if (madvise(at, (size_t)n, MADV_POPULATE_WRITE) == 0) return;
-#endif
-    for (int64_t i = 0; i < n; i += 4096) *static_cast<volatile uint8_t *>(at + i) = 0;
-}
-
 // Block i, if it is still to be had.  `idle` runs while the mark is waited for.
 inline void take_block(HostJob &job, size_t i, const std::function<void()> *idle)
 {
@@ -78,8 +71,7 @@ inline void take_block(HostJob &job, size_t i, const std::function<void()> *idle
         if (idle) (*idle)();
         host_pause();
     }
-    if (!b.src) make_present(b.dst, b.bytes);
-    else if (!job.stop.load(std::memory_order_relaxed)) memcpy(b.dst, b.src, (size_t)b.bytes);
+    if (!job.stop.load(std::memory_order_relaxed)) memcpy(b.dst, b.src, (size_t)b.bytes);
     job.left[(size_t)b.step].fetch_sub(1, std::memory_order_acq_rel);
     job.done.fetch_add(1, std::memory_order_acq_rel);
 }
@@ -122,7 +114,7 @@ inline int host_threads(const CgHostTeam *team)
 
 inline void run_job(HostJob &job, const CgHostTeam *team, const std::function<void()> *idle)
 {
-    if (job.nthreads > 1 && job.blocks.size() > 1) {
+    if (job.nthreads > 1 && job.blocks.size() > 2) {
         HostRun r = {&job, idle, team->thread_num};
         team->parallel(&host_member, &r, (unsigned)job.nthreads, 0u);
     } else {

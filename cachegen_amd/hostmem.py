@@ -74,21 +74,24 @@ def new_bytes(n: int):
     through the tensor before anybody else sees the object.
 
     Memory that the allocator has just got from the system is made present here: asked for in huge
-    pages (a page fault per 4 KB costs more than the copy that causes it), each by one of a few
-    threads (the threads of a copy wait for the zeroing of the same page).  A 15 MB pickle blob made and dropped: 0.95 ms
+    pages (a page fault per 4 KB costs more than the copy that causes it) and written once by all
+    threads at the same time (a blob is filled section by section, and the threads of one section's
+    copy wait for the zeroing of the same page).  Made present and filled, 3.6, 4.5, 6 and 14 MB: 225, 244, 193 and
+    261 us, left to the copies 436, 495, 646 and 1353, the kernel asked to populate the large pages alone -, 423, 377 and
+    424; 2 MB, of which a large page is seldom whole, 260 and 269.  A 15 MB pickle blob made and dropped: 0.95 ms
     without, 0.55 with; a blob that gets memory used before is not written twice (54 MB in nine blobs
     of a store: 0.5 ms more if it were)."""
     b = _new(None, n)
     t = view(b)
-    if n >= 2 * _HUGE_PAGE:
+    if n >= 3 * _HUGE_PAGE // 2:
         at = t.data_ptr()
         first, last = -(-at // _HUGE_PAGE) * _HUGE_PAGE, (at + n) // _HUGE_PAGE * _HUGE_PAGE
         present, fresh = ctypes.c_ubyte(), 0
         for page in range(first, last, _HUGE_PAGE):
             fresh += _libc.mincore(page + _HUGE_PAGE - _PAGE, _PAGE, ctypes.byref(present)) == 0 and not present.value & 1
-        if 2 * fresh * _HUGE_PAGE > last - first:
+        if 2 * fresh * _HUGE_PAGE > max(0, last - first):
             _libc.madvise(first, last - first, _MADV_HUGEPAGE)
-            _lib.check(_lib.lib().cg_host_present(first, last - first, _HUGE_PAGE, team()))
+            t.fill_(0)
     return b, t
 
 
@@ -151,6 +154,15 @@ class Words:
             self._memory[7] = 0
         return self
 
+    def set(self, stream):
+        """The mark alone, behind what the stream holds so far: for `StoredWords.stored`."""
+        _lib.check(_lib.lib().cg_mark(self.mark, self.value, stream))
+        self._stream = stream
+        return self
+
+    def synchronize(self):
+        self.wait(self._stream)
+
     def wait(self, stream):
         _lib.check(_lib.lib().cg_wait_mark(self.mark, self.value, stream))
 
@@ -185,6 +197,11 @@ def read_number(tensor, index):
 
 
 _PART = struct.Struct("<3q2i")           # CgHostPart
+
+
+# Up to so many bytes in one or two pieces are copied by torch and moved at once: 2.7 MB are in pinned memory after 11 us, and the
+# host is free after 17, where the steps take it 50 and the bytes are through no sooner.
+_FEW_BYTES = 4 << 20
 
 
 class Arrival:
@@ -260,6 +277,12 @@ class Moves:
         """`size` bytes at the device address `base` from pieces of ordinary memory ((offset, uint8 tensor), in order): copied
         to pinned memory and moved by steps as they are there.  slots: pinned steps that are used in turn (0: as
         many as it takes)."""
+        if size <= _FEW_BYTES and len(pieces) <= 2:
+            host = torch.empty(size, dtype=torch.uint8, pin_memory=True)
+            for at, t in pieces:
+                host[at:at + t.numel()].copy_(t)
+            self.up(host, base)
+            return
         nsteps = -(-size // step)
         if slots and slots < nsteps:
             pinned = [torch.empty(step, dtype=torch.uint8, pin_memory=True) for _ in range(slots)]
@@ -304,34 +327,33 @@ class Moves:
             del self._coming_down[0]
 
     def hold(self, event):
-        """Keeps what is still going up, and the word, until `event`, recorded behind all moves."""
-        _hold(event, [self._word] + [t for _, t in self._going_up])
+        """Keeps what is still going up, and the word, until `event`, recorded behind all moves; the event is `hold`'s
+        from here on."""
+        tensors = [self._word] + [t for _, t in self._going_up]
+        with _held_lock:
+            _held.append((event, self.device.index, tensors))
+            if sum(t.numel() for _, _, ts in _held for t in ts) > _HELD_BYTES:
+                _held[0][0].synchronize()
+                _let_go()
         self._reached = self._count
 
 
-_HELD_BYTES = 256 << 20                  # of pinned memory on its way up that is kept without waiting
-_held = collections.deque()              # (event, pinned tensors)
+_HELD_BYTES = 256 << 20                  # of pinned memory on its way up; what is above is waited for
+_held = collections.deque()              # (event, device index, pinned tensors)
 _held_lock = threading.Lock()
+_events = {}                             # device index -> events that are through, to be recorded again (a new one takes 9 us)
 
 
-def _hold(event, tensors):
-    with _held_lock:
-        _held.append((event, tensors))
-        _let_go(_HELD_BYTES)
-
-
-def _let_go(most):
-    """Gives back what has been read; waits only for as much as is above `most` bytes."""
+def _let_go():
     while _held and _held[0][0].query():
-        _held.popleft()
-    total = sum(t.numel() for _, tensors in _held for t in tensors)
-    while _held and total > most:
-        event, tensors = _held.popleft()
-        event.synchronize()
-        total -= sum(t.numel() for t in tensors)
+        event, device, _ = _held.popleft()
+        if len(_events.setdefault(device, [])) < 16:
+            _events[device].append(event)
 
 
-def let_go():
-    """Gives back the pinned memory of earlier calls that has been read by now."""
+def event(device):
+    """An event for `hold`; gives back the pinned memory of earlier calls that has been read by now."""
     with _held_lock:
-        _let_go(_HELD_BYTES)
+        _let_go()
+        kept = _events.get(device.index)
+        return kept.pop() if kept else torch.cuda.Event()

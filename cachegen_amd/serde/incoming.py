@@ -22,6 +22,10 @@ _ALIGN = 256
 # are moved by a launch each, which costs the bus 2 us (53 MB by 2 MB: 1.1 ms, by 4 MB 1.04).
 _WHOLE_BYTES = 16 << 20
 _PIECE_BYTES, _PIECES = 4 << 20, 4
+# Up to this, torch's own copies: the host, not the bus, is what such a call waits for, and what goes up by moves has to be
+# kept until it is through (chunks of 16 to 80 tokens x 512 channels x 32 layers as counts 110 us by copies, 117 by moves;
+# 150 tokens 116 and 116, 256 tokens 126 and 116).
+_SMALL_BYTES = 1 << 20
 
 _ITEM = struct.Struct("<10q4i")      # CgHostContainer
 _SUB_BYTES = 96                      # sizeof(CgListedSub)
@@ -102,7 +106,14 @@ def _upload(pieces, total, index_at, write_index):
 def _transfer(pieces, total, index_at, write_index, device):
     buf = torch.empty(total, dtype=torch.uint8, device=device)
     base = buf.data_ptr()
-    hostmem.let_go()
+    if total <= _SMALL_BYTES:
+        for at, end, write in ((0, index_at, lambda host: [host[a:a + t.numel()].copy_(t) for a, t in pieces]),
+                               (index_at, total, lambda host: write_index(base, host))):
+            host = torch.empty(end - at, dtype=torch.uint8, pin_memory=True)
+            write(host)
+            buf[at:end].copy_(host, non_blocking=True)
+        return buf, None
+    through = hostmem.event(device)
     moves = hostmem.Moves(device, codec._stream(device))
     try:
         if index_at <= _WHOLE_BYTES:
@@ -113,7 +124,6 @@ def _transfer(pieces, total, index_at, write_index, device):
         write_index(base, host)
         moves.up(host, base + index_at)
     finally:
-        through = torch.cuda.Event()
         through.record()
         moves.hold(through)
     return buf, through
@@ -222,13 +232,14 @@ def decode(items, out, fmt):
         base = buf.data_ptr() + index_at
         stream = codec._stream(buf.device)
         # a word that stays zero unless a kernel finds counts that make no table
-        with hostmem.StoredWords(1, torch.int32) if counted else contextlib.nullcontext() as verdict:
+        with hostmem.Words() if counted else contextlib.nullcontext() as there, \
+                hostmem.StoredWords(1, torch.int32) if counted else contextlib.nullcontext() as verdict:
             for key, (tables, groups) in counted.items():
                 at = base + groups_at[key]
                 _lib.check(lib.cg_rebuild_tables(buf.data_ptr(), index_at, key[0], groups, C, at + 8 * groups, at + 12 * groups, at,
                                                  tables.data_ptr(), verdict.words.data_ptr(), stream))
             if counted:
-                verdict.stored()
+                verdict.stored(by=there.set(stream))
             at = base + subs_at
             for key, members in launches.items():
                 n = sum(k for c, _, _, _ in members for _, k in c.length_arrays)

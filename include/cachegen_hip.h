@@ -431,10 +431,6 @@ typedef struct CgHostPart {
  * are done.  The launches that set the mark have been queued on the stream. */
 int cg_host_fill(const CgHostPart *parts, int n, const int32_t *mark, const CgHostTeam *team, void *stream);
 
-/* HOST: n bytes of memory that is new to the process made present by the team, `page` bytes (a multiple of 4096: the
- * size of its large pages) at a time; `at` is a multiple of 4096, and the bytes are undefined afterwards. */
-int cg_host_present(void *at, int64_t n, int64_t page, const CgHostTeam *team);
-
 /* HOST and the stream: `bytes` bytes of device memory at `area` from the parts (ascending, not overlapping; what lies
  * between them is undefined), staged in pinned memory by the team and moved in steps, each as soon as it is staged.
  * step   bytes of a step, a multiple of 64 (the first is a quarter of one)

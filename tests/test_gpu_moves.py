@@ -53,13 +53,13 @@ def test_memory_that_has_been_read_is_given_back(monkeypatch):
     for i in range(8):
         moves = hostmem.Moves(DEV, codec._stream(DEV))
         moves.up(_bytes(1 << 20, i).pin_memory(), dst.data_ptr())
-        event = torch.cuda.Event()
+        event = hostmem.event(DEV)
         event.record()
         moves.hold(event)
-        assert sum(t.numel() for _, tensors in hostmem._held for t in tensors) <= 1 << 20
+        assert sum(t.numel() for _, _, tensors in hostmem._held for t in tensors) <= 2 << 20       # the last one's, and the one it came on top of
     torch.cuda.synchronize()
-    hostmem.let_go()
-    assert not hostmem._held
+    hostmem.event(DEV)
+    assert not hostmem._held and len(hostmem._events[0]) <= 16
     assert torch.equal(dst.cpu(), _bytes(1 << 20, 7))
 
 
@@ -77,18 +77,21 @@ def test_marks_are_refused_where_they_cannot_be_set():
 # slots for everything, two and eight in turn; steps of 64 bytes and up; pieces with gaps between them
 @pytest.mark.parametrize("slots", [0, 2, 8])
 @pytest.mark.parametrize("step,size", [(64, 1000), (4352, 8 * 4352), (4352, 8 * 4352 + 1), (4352, 300001), (2 << 20, (20 << 20) + 77)])
-def test_staged_pieces_arrive(step, size, slots):
+@pytest.mark.parametrize("few", [0, 4 << 20])
+def test_staged_pieces_arrive(step, size, slots, few, monkeypatch):
+    monkeypatch.setattr(hostmem, "_FEW_BYTES", few)
     print(step, size, slots, flush=True)
     g = torch.Generator().manual_seed(size)
     cuts = sorted({0, size, *(int(x) for x in torch.randint(0, size, (9,), generator=g))})
+    if few:
+        cuts = cuts[:1] + cuts[-2:]
     pieces = [(a, _bytes(b - a - (1 if b - a > 5 and i % 2 else 0), i)) for i, (a, b) in enumerate(zip(cuts, cuts[1:]))]
     dev = torch.full((size + GUARD,), 8, dtype=torch.uint8, device=DEV)
     with torch.cuda.device(DEV):
         for _ in range(3):
-            hostmem.let_go()
+            event = hostmem.event(DEV)
             moves = hostmem.Moves(DEV, codec._stream(DEV))
             moves.stage(pieces, dev.data_ptr(), size, step, slots)
-            event = torch.cuda.Event()
             event.record()
             moves.hold(event)
     got = dev.cpu()

@@ -102,23 +102,7 @@ def test_callers_side_by_side():
     assert not wrong
 
 
-@pytest.mark.parametrize("threads", [1, 4])
-@pytest.mark.parametrize("at,n", [(0, 1), (0, 512), (3, 509), (1, 1600), (511, 2)])          # in pages of 4 KB, 512 to a large one
-def test_memory_is_made_present(at, n, threads):
-    import mmap
-    libc = ctypes.CDLL(None)
-    region = mmap.mmap(-1, 8 << 20)
-    start = ctypes.addressof(ctypes.c_char.from_buffer(region))
-    first = -(-start // (2 << 20)) * (2 << 20) + at * 4096
-    _lib.check(_lib.lib().cg_host_present(first, n * 4096, 2 << 20, team(threads)))
-    there = (ctypes.c_ubyte * n)()
-    assert libc.mincore(ctypes.c_void_p(first), ctypes.c_size_t(n * 4096), there) == 0
-    assert all(b & 1 for b in there)
-
-
 def _refuse_bad_parts():
-    with pytest.raises(RuntimeError, match="whole pages"):
-        _lib.check(_lib.lib().cg_host_present(4096 + 8, 4096, 4096, None))
     mark = torch.zeros(1, dtype=torch.int32)
     with pytest.raises(RuntimeError, match="bad part"):
         _lib.check(_lib.lib().cg_host_fill(PART.pack(0, 0, 5, 0, 0), 1, mark.data_ptr(), None, None))
