@@ -27,11 +27,11 @@ namespace {
 // job also ends on its caller alone.
 //
 // Staged and moved to the GPU, one thread / eight: 1 MB 57 / 52 us, 2.7 MB 96 / 86, 6 MB 168 / 152, 14 MB 343 / 326, 53 MB 1532 / 1152;
-// copied out of pinned memory just written: 1.4 MB 40 / 20, 6 MB 157 / 61, 14 MB 364 / 130.  Sixteen are as fast; a team of
-// all of torch's threads is asked for, since the runtime ends the threads that a smaller one leaves out and has to start them
-// again for torch's next operation.
+// copied out of pinned memory just written: 1.4 MB 40 / 20, 6 MB 157 / 61, 14 MB 364 / 130.  Sixteen are no faster (a chunk to
+// bytes and back 476 us, 458 with eight), but the team is of all of torch's threads, of which the others return at once: the
+// runtime ends the threads that a smaller one leaves out and has to start them again for torch's next operation.
 constexpr int64_t kHostBlock = 64 << 10;
-constexpr int kHostThreads = 1024;
+constexpr int kHostThreads = 8;
 
 struct HostBlock {
     uint8_t *dst;
@@ -97,6 +97,7 @@ inline void host_member(void *run)
 {
     const HostRun &r = *static_cast<HostRun *>(run);
     const int me = r.thread_num();
+    if (me >= r.job->nthreads) return;
     const std::function<void()> *const idle = me == 0 ? r.idle : nullptr;       // the caller is thread 0
     work_on(*r.job, me, idle);
     // another thread's block may wait for what only the caller's idle() brings about: it stays until all are through
@@ -116,7 +117,7 @@ inline void run_job(HostJob &job, const CgHostTeam *team, const std::function<vo
 {
     if (job.nthreads > 1 && job.blocks.size() > 2) {
         HostRun r = {&job, idle, team->thread_num};
-        team->parallel(&host_member, &r, (unsigned)job.nthreads, 0u);
+        team->parallel(&host_member, &r, (unsigned)team->threads, 0u);
     } else {
         work_on(job, 0, idle);
     }
