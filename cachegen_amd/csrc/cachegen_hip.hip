@@ -44,6 +44,7 @@
 #include "decoder.hpp"
 #include "scan_compact.hpp"
 #include "launch.hpp"
+#include "side_stream.hpp"
 #include "host_lengths.hpp"
 #include "host_copy.hpp"
 #include "move_bytes.hpp"
@@ -544,38 +545,69 @@ int code_and_compact_levels(const LevelOut *o, int n, const EncodeWorkspace &w, 
     const EncodeSource source = counted ? ENC_COUNTED : ENC_TABLES;
     const bool few = few_encode(nblocks * n, source, max_lp, kSlotTile, fused_scan);
     const bool together = few || nblocks * n <= (int64_t)compute_units() * resident_encode_blocks(max_lp);
-    for (int64_t resident = 8; resident >= 1; --resident) {
-        int count = 0, lp = 0;
-        for (int v = n - 1; v >= 0; --v) {
-            if (!together && resident_encode_blocks(o[v].max_bins + 1) != resident) continue;
-            const EncodeWorkspace wv = w.level(v);
-            p.level[count++] = {reinterpret_cast<uint16_t *>(o[v].cdf), reinterpret_cast<const uint32_t *>(wv.symbols), wv.scratch,
-                                o[v].lengths, o[v].status, fused_scan ? wv.tile_sums : nullptr, grouped ? wv.group_sums : nullptr,
-                                o[v].key_bins, o[v].value_bins, o[v].max_bins + 1};
-            if (o[v].max_bins + 1 > lp) lp = o[v].max_bins + 1;
-        }
+    // the levels by launches: members[i], longest tables first
+    int members[kMaxLevels][kMaxLevels], sizes[kMaxLevels], nlaunches = 0;
+    for (int64_t resident = 1; resident <= 8; ++resident) {
+        int count = 0;
+        for (int v = n - 1; v >= 0; --v)
+            if (together || resident_encode_blocks(o[v].max_bins + 1) == resident) members[nlaunches][count++] = v;
         if (!count) continue;
-        int rc;
-        if (counted) rc = fused_scan ? launch_encode_levels<true, true>(p, count, lp, grid, few, s) : launch_encode_levels<true, false>(p, count, lp, grid, few, s);
-        else rc = fused_scan ? launch_encode_levels<false, true>(p, count, lp, grid, few, s) : launch_encode_levels<false, false>(p, count, lp, grid, few, s);
-        if (rc) return rc;
+        sizes[nlaunches++] = count;
         if (together) break;
     }
-    CompactLevelsArgs c;
-    for (int v = 0; v < n; ++v) {
-        const EncodeWorkspace wv = w.level(v);
-        if (int rc = scan_for_compaction(o[v], wv, fused_scan, grouped, wv.group_sums, c.level[v], s)) return rc;
-    }
+    auto code = [&](int launch, hipStream_t on) {
+        int lp = 0;
+        for (int i = 0; i < sizes[launch]; ++i) {
+            const int v = members[launch][i];
+            const EncodeWorkspace wv = w.level(v);
+            p.level[i] = {reinterpret_cast<uint16_t *>(o[v].cdf), reinterpret_cast<const uint32_t *>(wv.symbols), wv.scratch,
+                          o[v].lengths, o[v].status, fused_scan ? wv.tile_sums : nullptr, grouped ? wv.group_sums : nullptr,
+                          o[v].key_bins, o[v].value_bins, o[v].max_bins + 1};
+            if (o[v].max_bins + 1 > lp) lp = o[v].max_bins + 1;
+        }
+        if (counted) return fused_scan ? launch_encode_levels<true, true>(p, sizes[launch], lp, grid, few, on)
+                                       : launch_encode_levels<true, false>(p, sizes[launch], lp, grid, few, on);
+        return fused_scan ? launch_encode_levels<false, true>(p, sizes[launch], lp, grid, few, on)
+                          : launch_encode_levels<false, false>(p, sizes[launch], lp, grid, few, on);
+    };
     const int64_t cblocks = ceil_div(w.nstreams, kCompactStreams);
-    const dim3 cgrid((unsigned)cblocks, (unsigned)n);
-    if (cblocks * n <= sliced_compact_blocks()) {
-        if (fused_scan) compact_levels_kernel<true, 4><<<cgrid, dim3(1024), 0, s>>>(c);
-        else compact_levels_kernel<false, 4><<<cgrid, dim3(1024), 0, s>>>(c);
-    } else {
-        if (fused_scan) compact_levels_kernel<true, 1><<<cgrid, dim3(256), 0, s>>>(c);
-        else compact_levels_kernel<false, 1><<<cgrid, dim3(256), 0, s>>>(c);
+    auto compact = [&](const int *levels, int count, hipStream_t on) {
+        CompactLevelsArgs c;
+        for (int i = 0; i < count; ++i) {
+            const EncodeWorkspace wv = w.level(levels[i]);
+            if (int rc = scan_for_compaction(o[levels[i]], wv, fused_scan, grouped, wv.group_sums, c.level[i], on)) return rc;
+        }
+        const dim3 cgrid((unsigned)cblocks, (unsigned)count);
+        if (cblocks * count <= sliced_compact_blocks()) {
+            if (fused_scan) compact_levels_kernel<true, 4><<<cgrid, dim3(1024), 0, on>>>(c);
+            else compact_levels_kernel<false, 4><<<cgrid, dim3(1024), 0, on>>>(c);
+        } else {
+            if (fused_scan) compact_levels_kernel<true, 1><<<cgrid, dim3(256), 0, on>>>(c);
+            else compact_levels_kernel<false, 1><<<cgrid, dim3(256), 0, on>>>(c);
+        }
+        return check_launch("compact levels");
+    };
+    if (nlaunches > 1) {
+        const SideStream side(s);
+        if (side.ok()) {
+            // the launch of the longest tables, whose LDS leaves half of a compute unit's wavefront slots empty, and its
+            // compaction beside the other levels' coder.  Four levels, one behind the other / beside, us: 32 layers x 4096 tokens
+            // x 1024 channels 1070 / 1049, x 1024 tokens 328 / 308, 512 channels 205 / 178, 400 channels 242 / 190; 4 layers x
+            // 2048 tokens in chunks of 1500 162 / 135
+            if (int rc = code(0, side.stream())) return rc;
+            if (int rc = compact(members[0], sizes[0], side.stream())) return rc;
+            for (int i = 1; i < nlaunches; ++i) {
+                if (int rc = code(i, s)) return rc;
+                if (int rc = compact(members[i], sizes[i], s)) return rc;
+            }
+            return CG_OK;
+        }
     }
-    return check_launch("compact levels");
+    for (int i = nlaunches - 1; i >= 0; --i)
+        if (int rc = code(i, s)) return rc;
+    int all[kMaxLevels];
+    for (int v = 0; v < n; ++v) all[v] = v;
+    return compact(all, n, s);
 }
 
 int check_kv_geometry(const char *what, int kv_dt, int64_t L, int64_t T, int64_t H, int64_t D, int64_t chunk_tokens)

@@ -44,3 +44,55 @@ def test_levels_in_shared_launches(shape, chunk, tops, dtype):
         for name in ("cdf", "maxima", "lengths", "offsets"):
             assert torch.equal(getattr(e, name), getattr(want, name)), name
         assert torch.equal(e.payload[:n], want.payload[:n])
+
+
+def _levels_and_cache(seed):
+    from cachegen_amd.kvgen import make_kv
+    kv = make_kv(6, 2048, 8, 128, seed=seed, device=DEV, dtype=torch.float16)      # two launches, one beside the other
+    return kv, [(_bins(float(t), 6).to(DEV), _bins(float(t), 6).to(DEV)) for t in (8, 64, 32)]
+
+
+def _bytes(encs):
+    return [t.clone() for e in encs for t in (e.cdf, e.lengths, e.offsets, e.payload[:e.total_bytes()])]
+
+
+def test_levels_in_a_graph():
+    from cachegen_amd import codec
+    kv, levels = _levels_and_cache(1)
+    tops = [8, 64, 32]
+    ws = torch.empty(codec.encode_levels_workspace_bytes(6, 2048, 1024, 256, 3), dtype=torch.uint8, device=DEV)
+    out = codec.encode_kv_levels(kv, levels, chunk_tokens=256, max_bins=tops, workspace=ws)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        codec.encode_kv_levels(kv, levels, chunk_tokens=256, max_bins=tops, workspace=ws, out=out)
+    for seed in (2, 3, 4):
+        other, _ = _levels_and_cache(seed)
+        want = _bytes(codec.encode_kv_levels(other, levels, chunk_tokens=256, max_bins=tops))
+        kv.copy_(other)
+        graph.replay()
+        assert all(torch.equal(a, b) for a, b in zip(_bytes(out), want))
+
+
+def test_levels_on_several_streams_at_once():
+    """More callers than there are side streams; each call's inputs are written just before it and dropped just behind."""
+    import threading
+    from cachegen_amd import codec
+    tops = [8, 64, 32]
+    want = {seed: _bytes(codec.encode_kv_levels(*_levels_and_cache(seed), chunk_tokens=256, max_bins=tops)) for seed in (1, 2, 3)}
+    torch.cuda.synchronize()
+    wrong = []
+
+    def caller(seed):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for _ in range(6):
+                kv, levels = _levels_and_cache(seed)
+                got = codec.encode_kv_levels(kv, levels, chunk_tokens=256, max_bins=tops)
+                del kv, levels
+                if not all(torch.equal(a, b) for a, b in zip(_bytes(got), want[seed])):
+                    wrong.append(seed)
+    callers = [threading.Thread(target=caller, args=(seed,)) for seed in want]
+    for c in callers:
+        c.start()
+    for c in callers:
+        c.join()
+    assert not wrong
