@@ -137,8 +137,8 @@ _free = threading.local()                # words of this thread that nobody uses
 class Words:
     """64 pinned bytes that kernels of one call store to, for a host that looks at their mark instead of waiting for an event
     (cg_read_words and its like); to be used in a `with` block that holds the launches and the reads.  They are
-    kept for the thread's next call; where a `with` block ends in an exception, until the process ends: something may
-    still store to them."""
+    kept for the thread's next call; where a `with` block ends in an exception and the mark is not there, until the
+    process ends: something may still store to them."""
     _lost = []
 
     def __enter__(self):
@@ -176,7 +176,7 @@ class Words:
         return ctypes.c_float.from_address(self.at).value
 
     def __exit__(self, kind, *exc):
-        if kind is None:
+        if kind is None or ctypes.c_int32.from_address(self.mark).value >= self.value:
             _free.words.append((self._memory, self.value))
         else:
             self._lost.append(self._memory)
@@ -264,6 +264,8 @@ class Moves:
     def fill(self, parts):
         """parts: [(uint8 tensor in ordinary memory, uint8 tensor of the same size in pinned memory, its arrival
         or None)]: copies each as it arrives."""
+        if not parts:
+            return
         last = max((a._number for _, _, a in parts if a is not None), default=0)
         with torch.cuda.device(self.device):
             if self._marked < last:

@@ -92,3 +92,27 @@ def test_decode_from_lengths(rows, cols, tokens):
     out = torch.zeros(sym.shape, dtype=torch.uint8, device=DEV)
     torchac_hip.decode_fast_lengths(cdf, stream, lengths, out)
     assert torch.equal(out, sym.view(torch.uint8))
+
+
+def test_words_are_used_again_after_an_error():
+    hostmem.read_number(torch.zeros(1, dtype=torch.int32, device=DEV), 0)
+    kept, lost = len(hostmem._free.words), len(hostmem.Words._lost)
+    with pytest.raises(KeyError):
+        with hostmem.Words() as words:
+            words.set(codec._stream(torch.device(DEV))).synchronize()
+            raise KeyError
+    assert (len(hostmem._free.words), len(hostmem.Words._lost)) == (kept, lost)
+    with pytest.raises(KeyError):
+        with hostmem.Words():
+            raise KeyError                              # nothing was launched, which nobody can know
+    assert (len(hostmem._free.words), len(hostmem.Words._lost)) == (kept - 1, lost + 1)
+
+
+def test_a_pickle_of_small_tensors():
+    from cachegen_amd.kvgen import make_kv
+    from cachegen_amd.serde import pickled
+    from cachegen_amd.serde.cachegen_basics import CacheGenGPUEncoderOutput
+    bins = torch.full((1,), 8.0)
+    enc = codec.encode_kv(make_kv(1, 9, 1, 8, seed=1, device=DEV), bins, bins)
+    out = CacheGenGPUEncoderOutput.from_bytes(pickled.pack_chunks(enc)[0])
+    assert torch.equal(out.cdf.to(DEV), enc.cdf[0]) and torch.equal(out.data_chunks[0].bytestream.to(DEV), enc.payload[:enc.total_bytes()])
