@@ -53,6 +53,7 @@ SIGNATURES = {
     "cg_move_bytes": (_INT, [_P, _P, _I64, _INT, _P, _INT, _P]),
     "cg_host_fill": (_INT, [_P, _INT, _P, _P, _P]),
     "cg_host_stage": (_INT, [_P, _INT, _P, _INT, _I64, _P, _I64, _P, _INT, _P, _P, _P]),
+    "cg_test_host_stage": (_INT, [_P, _INT, _P, _INT, _I64, _P, _I64, _P, _P]),
     "cg_read_words": (_INT, [_P, _P, _INT, _P, _INT, _P]),
     "cg_largest": (_INT, [_P, _P, _I64, _P, _INT, _P]),
     "cg_scan_collect": (_INT, [_P, _I64, _P, _P, _SZ, _I64, _I64, _P, _INT, _P]),

@@ -986,54 +986,43 @@ int cg_host_fill(const CgHostPart *parts, int n, const int32_t *mark, const CgHo
 int cg_host_stage(const CgHostPart *parts, int n, void *const *slots, int nslots, int64_t step, void *area, int64_t bytes, int32_t *mark,
                   int32_t value, const CgHostTeam *team, int *moves, void *stream)
 {
-    if (!parts || n < 0 || !slots || !area || !mark || !moves || bytes <= 0) return fail(CG_ERR_ARG, "host_stage: null pointer or nothing to move");
-    *moves = 0;
-    if (step < 64 || step % 64) return fail(CG_ERR_ARG, "host_stage: steps are multiples of 64 bytes");
-    const int64_t ring_bytes = nslots * step;
-    if (nslots < 2 && ring_bytes < bytes) return fail(CG_ERR_ARG, "host_stage: pinned memory too small");
-    for (int64_t i = 0; i < nslots && i * step < bytes; ++i)
-        if (!slots[i]) return fail(CG_ERR_ARG, "host_stage: null slot");
-    const HostSteps at_step = {step};
+    if (moves) *moves = 0;
+    if (const char *what = stage_fault(parts, n, slots, nslots, step, area, bytes, mark, moves)) return fail(CG_ERR_ARG, "host_stage: %s", what);
     try {
         hipStream_t s = static_cast<hipStream_t>(stream);
-        auto pinned = [&](int64_t at) { return static_cast<uint8_t *>(slots[at / step % nslots]) + at % step; };
-        const int32_t steps = (int32_t)at_step.of(bytes - 1) + 1;
-        HostJob job;
-        job.mark = mark;
-        job.known.store(value);
-        job.nthreads = host_threads(team);
-        for (int i = 0; i < n; ++i) {
-            const CgHostPart &p = parts[i];
-            if (p.bytes < 0 || (p.bytes && !p.src) || p.dst < 0 || p.dst + p.bytes > bytes) return fail(CG_ERR_ARG, "host_stage: bad part");
-            for (int64_t at = p.dst, end = p.dst + p.bytes; at < end;) {
-                const int64_t k = at_step.of(at), stop = std::min(end, at_step.start(k + 1));
-                // the slot is free once the move that was there is through, which the launch behind that one says
-                const int32_t need = at < ring_bytes ? value : value + (int32_t)at_step.of(stop - 1 - ring_bytes) + 1;
-                add_blocks(job, pinned(at), reinterpret_cast<const uint8_t *>(p.src) + (at - p.dst), stop - at,
-                           (uintptr_t)p.src + (uintptr_t)(at - p.dst), need, (int32_t)k);
-                at = stop;
-            }
-        }
-        seal(job, steps);
-        int rc = CG_OK;
-        int32_t launched = 0;
         MarkWatch watch(mark, s);
-        const std::function<void()> idle = [&] {
-            while (!rc && launched < steps && job.left[(size_t)launched].load(std::memory_order_acquire) <= 0) {
-                const int64_t at = at_step.start(launched), end = std::min(bytes, at_step.start(launched + 1));
-                rc = launch_move_bytes(pinned(at), static_cast<uint8_t *>(area) + at, end - at, false, mark, value + launched, s);
-                if (!rc) ++launched;
-            }
-            if (!rc && launched < steps && launched > 0 && job.known.load(std::memory_order_relaxed) < value + launched &&
-                watch.overdue(value + launched)) {
-                // the launches so far are through once the stream is
-                if (!(rc = watch.settle())) job.known.store(value + launched, std::memory_order_release);
-            }
-            if (rc) job.stop.store(true);
-        };
-        run_job(job, team, &idle);
-        while (!rc && launched < steps) idle();
-        *moves = launched;
+        return stage_job(parts, n, slots, nslots, step, bytes, mark, value, team, moves,
+                         [&](const uint8_t *from, int64_t at, int64_t size, int32_t mine) {
+                             return launch_move_bytes(from, static_cast<uint8_t *>(area) + at, size, false, mark, mine, s);
+                         },
+                         [&](int32_t upto) {
+                             if (!watch.overdue(upto)) return 0;
+                             const int rc = watch.settle();          // the launches so far are through once the stream is
+                             return rc ? rc : 1;
+                         });
+    } catch (const std::exception &e) {
+        return fail(CG_ERR_ARG, "host_stage: %s", e.what());
+    }
+}
+
+int cg_test_host_stage(const CgHostPart *parts, int n, void *const *slots, int nslots, int64_t step, void *area, int64_t bytes,
+                       const CgHostTeam *team, int *moves)
+{
+    int32_t mark = 0, value = 1;
+    if (moves) *moves = 0;
+    if (const char *what = stage_fault(parts, n, slots, nslots, step, area, bytes, &mark, moves)) return fail(CG_ERR_ARG, "host_stage: %s", what);
+    try {
+        // a move reads its slot as late as it may: when the one behind it is launched, which then sets the mark
+        struct { const uint8_t *from; uint8_t *to; int64_t size; } last = {nullptr, nullptr, 0};
+        const int rc = stage_job(parts, n, slots, nslots, step, bytes, &mark, value, team, moves,
+                                 [&](const uint8_t *from, int64_t at, int64_t size, int32_t mine) {
+                                     if (last.size) memcpy(last.to, last.from, (size_t)last.size);
+                                     last = {from, static_cast<uint8_t *>(area) + at, size};
+                                     __atomic_store_n(&mark, mine, __ATOMIC_RELEASE);
+                                     return 0;
+                                 },
+                                 [](int32_t) { return 0; });
+        if (last.size) memcpy(last.to, last.from, (size_t)last.size);
         return rc;
     } catch (const std::exception &e) {
         return fail(CG_ERR_ARG, "host_stage: %s", e.what());

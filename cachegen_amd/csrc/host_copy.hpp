@@ -23,8 +23,11 @@ namespace {
 // own, beside sixteen of that runtime that still look for work after a torch operation, are more than the cores that a
 // process has here, and a job then waits for a thread that waits for a core (53 MB: 3 to 10 ms instead of 1.2).
 // A block has an owner among the threads, by its address in ordinary memory: a blob that is read back soon lies in the
-// caches of the threads that wrote it.  Every thread takes its own blocks in order and then what nobody has begun, so a
-// job also ends on its caller alone.
+// caches of the threads that wrote it.  Owners are dealt before the team is there, and the runtime may give a smaller one
+// (a thread limit, dynamic teams, a caller inside a parallel region) or none.  So every thread goes through the job step
+// by step, its own blocks of a step first and then what nobody has begun of it: who waits for a pinned slot has seen
+// every block of the steps before taken, those are copied without waiting for this one, and the move that frees the slot
+// is launched.  A job ends with any team, on its caller alone too.
 //
 // Staged and moved to the GPU, one thread / eight: 1 MB 57 / 52 us, 2.7 MB 96 / 86, 6 MB 168 / 152, 14 MB 343 / 326, 53 MB 1532 / 1152;
 // copied out of pinned memory just written: 1.4 MB 40 / 20, 6 MB 157 / 61, 14 MB 364 / 130.  Sixteen are no faster (a chunk to
@@ -43,7 +46,8 @@ struct HostBlock {
 };
 
 struct HostJob {
-    std::vector<HostBlock> blocks;
+    std::vector<HostBlock> blocks;          // by steps
+    std::vector<size_t> ends;               // behind each step's blocks
     std::vector<std::atomic<uint8_t>> taken;
     std::vector<std::atomic<int32_t>> left; // blocks to come, per step
     std::atomic<int32_t> done{0};           // blocks that are through
@@ -78,12 +82,16 @@ inline void take_block(HostJob &job, size_t i, const std::function<void()> *idle
 
 inline void work_on(HostJob &job, int me, const std::function<void()> *idle)
 {
-    for (int mine = 1; mine >= 0; --mine)
-        for (size_t i = 0; i < job.blocks.size(); ++i) {
-            if (mine && job.blocks[i].owner != me) continue;
-            take_block(job, i, idle);
-            if (idle) (*idle)();
-        }
+    size_t first = 0;
+    for (const size_t end : job.ends) {
+        for (int mine = 1; mine >= 0; --mine)
+            for (size_t i = first; i < end; ++i) {
+                if (mine && job.blocks[i].owner != me) continue;
+                take_block(job, i, idle);
+                if (idle) (*idle)();
+            }
+        first = end;
+    }
 }
 
 // The job on the team's threads; `idle` (may be null) is run by the caller now and then.
@@ -140,7 +148,11 @@ inline void seal(HostJob &job, int steps)
 {
     job.taken = std::vector<std::atomic<uint8_t>>(job.blocks.size());
     job.left = std::vector<std::atomic<int32_t>>((size_t)steps);
+    const auto earlier = [](const HostBlock &a, const HostBlock &b) { return a.step < b.step; };
+    if (!std::is_sorted(job.blocks.begin(), job.blocks.end(), earlier)) std::stable_sort(job.blocks.begin(), job.blocks.end(), earlier);
     for (const HostBlock &b : job.blocks) job.left[(size_t)b.step].fetch_add(1, std::memory_order_relaxed);
+    size_t end = 0;
+    for (const auto &n : job.left) job.ends.push_back(end += (size_t)n.load(std::memory_order_relaxed));
 }
 
 // Where the steps of an upload begin: the first is a quarter of one so that the bus has something to do soon.
@@ -149,5 +161,66 @@ struct HostSteps {
     int64_t start(int64_t k) const { return k == 0 ? 0 : k == 1 ? step / 4 : (k - 1) * step; }
     int64_t of(int64_t at) const { return at < step / 4 ? 0 : at < step ? 1 : at / step + 1; }
 };
+
+// cg_host_stage's steps, launched by launch(from, offset in the area, bytes, value for the mark).  settle(value) returns 0
+// to go on looking, 1 when everything launched so far is through, or an error (negative).
+template <typename Launch, typename Settle>
+int stage_job(const CgHostPart *parts, int n, void *const *slots, int nslots, int64_t step, int64_t bytes, const int32_t *mark, int32_t value,
+              const CgHostTeam *team, int *moves, Launch launch, Settle settle)
+{
+    const HostSteps at_step = {step};
+    const int64_t ring_bytes = nslots * step;
+    auto pinned = [&](int64_t at) { return static_cast<uint8_t *>(slots[at / step % nslots]) + at % step; };
+    const int32_t steps = (int32_t)at_step.of(bytes - 1) + 1;
+    HostJob job;
+    job.mark = mark;
+    job.known.store(value);
+    job.nthreads = host_threads(team);
+    for (int i = 0; i < n; ++i) {
+        const CgHostPart &p = parts[i];
+        for (int64_t at = p.dst, end = p.dst + p.bytes; at < end;) {
+            const int64_t k = at_step.of(at), stop = std::min(end, at_step.start(k + 1));
+            // the slot is free once the move that was there is through, which the launch behind that one says
+            const int32_t need = at < ring_bytes ? value : value + (int32_t)at_step.of(stop - 1 - ring_bytes) + 1;
+            add_blocks(job, pinned(at), reinterpret_cast<const uint8_t *>(p.src) + (at - p.dst), stop - at,
+                       (uintptr_t)p.src + (uintptr_t)(at - p.dst), need, (int32_t)k);
+            at = stop;
+        }
+    }
+    seal(job, steps);
+    int rc = 0;
+    int32_t launched = 0;
+    const std::function<void()> idle = [&] {
+        while (!rc && launched < steps && job.left[(size_t)launched].load(std::memory_order_acquire) <= 0) {
+            const int64_t at = at_step.start(launched), end = std::min(bytes, at_step.start(launched + 1));
+            rc = launch(pinned(at), at, end - at, value + launched);
+            if (!rc) ++launched;
+        }
+        if (!rc && launched < steps && launched > 0 && job.known.load(std::memory_order_relaxed) < value + launched) {
+            const int through = settle(value + launched);
+            if (through > 0) job.known.store(value + launched, std::memory_order_release);
+            else rc = through;
+        }
+        if (rc) job.stop.store(true);
+    };
+    run_job(job, team, &idle);
+    while (!rc && launched < steps) idle();
+    *moves = launched;
+    return rc;
+}
+
+// Whether cg_host_stage's arguments describe something that it can do; null, or what is wrong.
+inline const char *stage_fault(const CgHostPart *parts, int n, void *const *slots, int nslots, int64_t step, const void *area, int64_t bytes,
+                               const int32_t *mark, const int *moves)
+{
+    if (!parts || n < 0 || !slots || !area || !mark || !moves || bytes <= 0) return "null pointer or nothing to move";
+    if (step < 64 || step % 64) return "steps are multiples of 64 bytes";
+    if (nslots < 2 && nslots * step < bytes) return "pinned memory too small";
+    for (int64_t i = 0; i < nslots && i * step < bytes; ++i)
+        if (!slots[i]) return "null slot";
+    for (int i = 0; i < n; ++i)
+        if (parts[i].bytes < 0 || (parts[i].bytes && !parts[i].src) || parts[i].dst < 0 || parts[i].dst + parts[i].bytes > bytes) return "bad part";
+    return nullptr;
+}
 
 }  // namespace

@@ -411,7 +411,7 @@ int cg_decode_fast_lengths(const int16_t *cdf, int lp, const uint8_t *bytes, int
                            int64_t *offsets, void *scratch, size_t scratch_bytes, void *stream);
 
 /* The threads of a host function: those of an OpenMP runtime, through its documented entry points, at most `threads`
- * of them.  Null, or null pointers: the caller alone. */
+ * of them (the runtime may give fewer).  Null, or null pointers: the caller alone. */
 typedef struct CgHostTeam {
     void (*parallel)(void (*fn)(void *), void *data, unsigned num_threads, unsigned flags);      /* GOMP_parallel */
     int (*thread_num)(void);                                                                     /* omp_get_thread_num */
@@ -440,6 +440,11 @@ int cg_host_fill(const CgHostPart *parts, int n, const int32_t *mark, const CgHo
  * moves  written: the moves launched (all of them, or those before an error) */
 int cg_host_stage(const CgHostPart *parts, int n, void *const *slots, int nslots, int64_t step, void *area, int64_t bytes,
                   int32_t *mark, int32_t value, const CgHostTeam *team, int *moves, void *stream);
+
+/* Test hook, no GPU work: cg_host_stage with a copy on the host in the place of each move, done as late as a move may be;
+ * `area` is host memory. */
+int cg_test_host_stage(const CgHostPart *parts, int n, void *const *slots, int nslots, int64_t step, void *area, int64_t bytes,
+                       const CgHostTeam *team, int *moves);
 
 #ifdef __cplusplus
 }

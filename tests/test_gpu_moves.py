@@ -100,6 +100,25 @@ def test_staged_pieces_arrive(step, size, slots, few, monkeypatch):
     assert (got[size:] == 8).all()
 
 
+@pytest.mark.parametrize("threads", [0, 1, 3])
+def test_staged_pieces_arrive_from_any_team(threads, monkeypatch):
+    own = hostmem.team()
+    monkeypatch.setattr(hostmem, "team", lambda: hostmem._TEAM.pack(*(hostmem._TEAM.unpack(own)[:2] if threads else (0, 0)), threads, 0))
+    monkeypatch.setattr(hostmem, "_FEW_BYTES", 0)
+    size = (5 << 20) + 77
+    want = _bytes(size, threads)
+    dev = torch.zeros(size, dtype=torch.uint8, device=DEV)
+    with torch.cuda.device(DEV):
+        for slots in (2, 4):
+            dev.zero_()
+            event = hostmem.event(DEV)
+            moves = hostmem.Moves(DEV, codec._stream(DEV))
+            moves.stage([(0, want[:1000001]), (1000001, want[1000001:])], dev.data_ptr(), size, 1 << 20, slots)
+            event.record()
+            moves.hold(event)
+            assert torch.equal(dev.cpu(), want)
+
+
 def test_parts_are_filled_as_they_come():
     src = torch.arange(3 << 20, dtype=torch.int32, device=DEV).view(torch.uint8)
     n = src.numel()

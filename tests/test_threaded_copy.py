@@ -2,7 +2,10 @@
 word that the test sets."""
 import concurrent.futures
 import ctypes
+import os
 import struct
+import subprocess
+import sys
 import threading
 import time
 
@@ -115,3 +118,60 @@ def _refuse_bad_parts():
 def test_bad_parts_are_refused():
     with concurrent.futures.ThreadPoolExecutor(1) as other:                 # the last error's text belongs to a thread
         other.submit(_refuse_bad_parts).result()
+
+
+class ShortTeam:
+    """A runtime that is asked for a team and gives `given` threads, the caller among them."""
+
+    def __init__(self, given):
+        self.given, self.numbers = given, {}
+        self.member = ctypes.CFUNCTYPE(None, ctypes.c_void_p)
+        self._parallel = ctypes.CFUNCTYPE(None, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_uint, ctypes.c_uint)(self.parallel)
+        self._number = ctypes.CFUNCTYPE(ctypes.c_int)(lambda: self.numbers[threading.get_ident()])
+
+    def parallel(self, fn, data, threads, flags):
+        def run(i):
+            self.numbers[threading.get_ident()] = i
+            self.member(fn)(data)
+        others = [threading.Thread(target=run, args=(i,)) for i in range(1, min(threads, self.given))]
+        for t in others:
+            t.start()
+        run(0)
+        for t in others:
+            t.join()
+
+    def packed(self, asked):
+        return struct.pack("<2Q2i", *(ctypes.cast(f, ctypes.c_void_p).value for f in (self._parallel, self._number)), asked, 0)
+
+
+def stage(lib, size, step, slots, asked, given, order=1):
+    """Whether all of `size` bytes arrive, staged by `given` threads where `asked` were dealt blocks."""
+    g = torch.Generator().manual_seed(size)
+    want = torch.randint(0, 256, (size,), generator=g, dtype=torch.uint8)
+    cuts = sorted({0, size, *(int(x) for x in torch.randint(0, size, (5,), generator=g))})
+    area = torch.zeros(size, dtype=torch.uint8)
+    pinned = [torch.empty(step, dtype=torch.uint8) for _ in range(slots)]
+    raw = b"".join([PART.pack(a, want[a:].data_ptr(), b - a, 0, 0) for a, b in zip(cuts, cuts[1:])][::order])
+    team, moves = ShortTeam(given), ctypes.c_int(0)
+    rc = lib.cg_test_host_stage(raw, len(cuts) - 1, (ctypes.c_void_p * slots)(*(t.data_ptr() for t in pinned)), slots, step,
+                                area.data_ptr(), size, team.packed(asked) if given else None, ctypes.byref(moves))
+    return rc == 0 and torch.equal(area, want) and moves.value == -(-size // step) + 1
+
+
+def stage_all():
+    """Pinned slots in turn, two and four of them, sizes in and above the ring; the caller alone, fewer threads than were asked
+    for, as many; parts that do not ascend."""
+    lib = _lib.lib()
+    for asked, given in ((8, 0), (1, 1), (8, 1), (8, 2), (8, 4), (16, 3), (8, 8)):
+        for slots in (2, 4):
+            for step, size in ((64, 1000), (256 << 10, (256 << 10) * slots), (256 << 10, (3 << 20) + 77), (1 << 20, (9 << 20) + 1)):
+                print(asked, given, slots, step, size, flush=True)
+                assert stage(lib, size, step, slots, asked, given)
+    assert stage(lib, (3 << 20) + 77, 256 << 10, 4, 8, 4, order=-1)
+
+
+def test_staged_uploads_end_with_any_team():
+    """In a process of its own, which a job that does not end would not leave."""
+    done = subprocess.run([sys.executable, "-c", "import test_threaded_copy as t; t.stage_all()"], timeout=100, capture_output=True, text=True,
+                          env={**os.environ, "PYTHONPATH": os.pathsep.join([os.path.dirname(__file__), os.path.dirname(os.path.dirname(__file__))])})
+    assert done.returncode == 0, done.stdout[-500:] + done.stderr[-2000:]
