@@ -5,11 +5,16 @@
 namespace {
 
 // Sets *mark (pinned host memory) to `value`.  A stream runs its launches one behind the other, so the host that
-// reads the value knows that all launches before this one are through, with what they stored.
+// reads the value knows that all launches before this one are through.  What they stored to device memory the launches behind
+// them see; what they stored to host memory the host sees only if the threads that stored it have released it to the
+// system (host_stores_done): the release here is of this thread's XCD, and theirs may be another.
 __device__ __forceinline__ void set_mark(int32_t *mark, int32_t value)
 {
     __hip_atomic_store(mark, value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
+
+// Ends a kernel's stores to host memory that a mark will stand for, in the threads that made them.
+__device__ __forceinline__ void host_stores_done() { __threadfence_system(); }
 
 // Up to four words of device memory, as 64-bit numbers, to pinned memory, and a mark behind them: 8 us until the host has
 // them, where a copy of one word and its wait are 14.

@@ -48,7 +48,7 @@ __global__ __launch_bounds__(kMoveThreads) void move_bytes_kernel(const uint8_t 
         const int at = (int)(i < head ? i : tail + (i - head));
         __builtin_amdgcn_raw_buffer_store_b8(__builtin_amdgcn_raw_buffer_load_b8(from, at, 0, kLoad), to, at, 0, kStore);
     }
-    if (TO_HOST) __threadfence_system();                 // there before the launch behind this one sets its mark
+    if (TO_HOST) host_stores_done();                     // there before the launch behind this one sets its mark
 }
 
 int launch_move_bytes(const uint8_t *src, uint8_t *dst, int64_t n, bool to_host, int32_t *mark, int32_t value, hipStream_t stream)

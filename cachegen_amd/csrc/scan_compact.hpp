@@ -165,7 +165,7 @@ __device__ __forceinline__ void scan_small(const int32_t *__restrict__ lengths, 
             if (lo + j == n - 1) offsets[n] = run;
             if (COLLECT && lo + j == n - 1) {
                 out[0] = run;
-                __threadfence_system();
+                host_stores_done();
             }
         }
     }
@@ -414,8 +414,10 @@ __global__ __launch_bounds__(256) void collect_sizes_kernel(
     const int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (g >= n) return;
     const int64_t at = offsets[g], size = offsets[g + 1] - at;
-    if (g == n - 1) out[0] = at + size;
-    if ((g == 0 && at != 0) || size < 0 || size > (g < nslots ? cap : 0)) out[1] = 1;      // everybody who writes writes the same
+    const bool last = g == n - 1, unfit = (g == 0 && at != 0) || size < 0 || size > (g < nslots ? cap : 0);
+    if (last) out[0] = at + size;
+    if (unfit) out[1] = 1;                               // everybody who writes writes the same
+    if (last || unfit) host_stores_done();
 }
 
 __global__ void clear_status_kernel(int32_t *status) { *status = 0; }

@@ -21,7 +21,7 @@ __global__ void clear_ints_kernel(int32_t *a, int64_t na, int32_t *b)
 }
 
 // What the host has to know of an encoded tensor before it can lay blobs out, stored straight into
-// host memory (pinned: the host reads it once the event behind this launch is through, without a
+// host memory (pinned: the host reads it once a mark behind this launch is there, without a
 // copy of its own): out = [status, wide, inexact, payload offset at each of nbounds sub-chunk
 // boundaries, nsym[0 .. ngroups)].  One block; a few hundred values.
 __global__ __launch_bounds__(kWireThreads) void wire_meta_kernel(
@@ -35,6 +35,7 @@ __global__ __launch_bounds__(kWireThreads) void wire_meta_kernel(
     }
     for (int64_t i = threadIdx.x; i < nbounds; i += kWireThreads) out[3 + i] = offsets[i * per_sub];
     for (int64_t i = threadIdx.x; i < ngroups; i += kWireThreads) out[3 + nbounds + i] = nsym[i];
+    host_stores_done();
 }
 
 // Stream lengths as 16-bit words; *wide (zero before the launch) is set where one does not fit.
@@ -191,7 +192,10 @@ __global__ __launch_bounds__(kTableChannels) void counts_to_tables_kernel(
             full += src[j] == 255u;
         }
         const uint32_t missing = n - sum;                           // wraps if the sum is too large
-        if (!inside || !(missing == 0u || (missing == 1u && full == 1u))) *invalid = 1;                                    // everybody who writes writes the same
+        if (!inside || !(missing == 0u || (missing == 1u && full == 1u))) {
+            *invalid = 1;                                           // everybody who writes writes the same; may be host memory
+            host_stores_done();
+        }
         uint32_t cum = 0;
         t[0] = 0;
         const int stored = inside ? k : 0;

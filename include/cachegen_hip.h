@@ -381,7 +381,8 @@ int cg_lengths_to_u16(const int32_t *lengths, int64_t n, uint16_t *out, int32_t 
  * memory, queued on the stream; fastest where the two addresses are equal modulo 16.  Both stay valid until
  * the launch is through.
  * mark   pinned host int32, or null: set to `value` when everything queued on the stream before this
- *        call is through, together with what that stored to host memory */
+ *        call is through, together with what this library's launches among it stored to host memory (others': what
+ *        they have themselves released to the system) */
 int cg_move_bytes(const void *src, void *dst, int64_t n, int to_host, int32_t *mark, int32_t value, void *stream);
 
 /* The mark alone. */
