@@ -331,26 +331,72 @@ class Moves:
     def hold(self, event):
         """Keeps what is still going up, and the word, until `event`, recorded behind all moves; the event is `hold`'s
         from here on."""
-        tensors = [self._word] + [t for _, t in self._going_up]
-        with _held_lock:
-            _held.append((event, self.device.index, tensors))
-            if sum(t.numel() for _, _, ts in _held for t in ts) > _HELD_BYTES:
-                _held[0][0].synchronize()
-                _let_go()
+        _hold(event, (self.device.index, self.stream), [self._word] + [t for _, t in self._going_up])
         self._reached = self._count
 
 
-_HELD_BYTES = 256 << 20                  # of pinned memory on its way up; what is above is waited for
-_held = collections.deque()              # (event, device index, pinned tensors)
+_HELD_BYTES = 256 << 20                  # of pinned memory on its way up, of all threads and streams
+_held = collections.deque()              # (event, (device index, stream), pinned tensors)
+_held_bytes = 0
 _held_lock = threading.Lock()
 _events = {}                             # device index -> events that are through, to be recorded again (a new one takes 9 us)
 
 
+def _hold(event, place, tensors):
+    """Where that makes more than _HELD_BYTES, the oldest of the caller's own stream are waited for, one after the other, until it
+    does not or they are all through: nobody waits for another stream's work, and as every caller does so, the bound holds
+    when a call has returned (calls in the middle of it come on top, with what they bring)."""
+    global _held_bytes
+    with _held_lock:
+        _held.append((event, place, tensors))
+        _held_bytes += _size(tensors)
+        if _held_bytes > _HELD_BYTES:
+            _let_all_go()
+    while True:
+        with _held_lock:
+            own = next((h for h in _held if h[1] == place), None)
+            if _held_bytes <= _HELD_BYTES or own is None:
+                return
+            _held.remove(own)            # nobody else records its event again while it is waited for
+        try:
+            own[0].synchronize()
+        except BaseException:
+            with _held_lock:
+                _held.appendleft(own)
+            raise
+        with _held_lock:
+            _gone(own)
+
+
+def _size(tensors):
+    return sum(t.numel() * t.element_size() for t in tensors)
+
+
+def _gone(held):
+    global _held_bytes
+    event, (device, _), tensors = held
+    _held_bytes -= _size(tensors)
+    if len(_events.setdefault(device, [])) < 16:
+        _events[device].append(event)
+
+
 def _let_go():
+    """What is through and has nothing older before it, which is what a program of one stream has."""
     while _held and _held[0][0].query():
-        event, device, _ = _held.popleft()
-        if len(_events.setdefault(device, [])) < 16:
-            _events[device].append(event)
+        _gone(_held.popleft())
+
+
+def _let_all_go():
+    """What is through of every stream: one that stands still keeps nobody else's."""
+    standing = set()
+    for h in list(_held):
+        if h[1] in standing:
+            continue
+        if h[0].query():
+            _held.remove(h)
+            _gone(h)
+        else:
+            standing.add(h[1])
 
 
 def event(device):
