@@ -91,19 +91,19 @@ def _upload(pieces, total, index_at, write_index):
     For a small one the events and the change of stream cost more than they hide (+25 us)."""
     device = torch.device("cuda", torch.cuda.current_device())          # the caller made it current
     if index_at <= _WHOLE_BYTES:
-        return _transfer(pieces, total, index_at, write_index, device)[0]
+        return _transfer(pieces, total, index_at, write_index, device)
     side = _upload_streams.get(device.index)
     if side is None:
         side = _upload_streams.setdefault(device.index, torch.cuda.Stream(device))
     current = torch.cuda.current_stream()
     with torch.cuda.stream(side):
-        buf, arrived = _transfer(pieces, total, index_at, write_index, device)
-    current.wait_event(arrived)
+        buf = _transfer(pieces, total, index_at, write_index, device, current)
     buf.record_stream(current)
     return buf
 
 
-def _transfer(pieces, total, index_at, write_index, device):
+def _transfer(pieces, total, index_at, write_index, device, waiting=None):
+    """waiting: a stream that waits for everything."""
     buf = torch.empty(total, dtype=torch.uint8, device=device)
     base = buf.data_ptr()
     if total <= _SMALL_BYTES:
@@ -112,7 +112,7 @@ def _transfer(pieces, total, index_at, write_index, device):
             host = torch.empty(end - at, dtype=torch.uint8, pin_memory=True)
             write(host)
             buf[at:end].copy_(host, non_blocking=True)
-        return buf, None
+        return buf
     through = hostmem.event(device)
     moves = hostmem.Moves(device, codec._stream(device))
     try:
@@ -125,8 +125,10 @@ def _transfer(pieces, total, index_at, write_index, device):
         moves.up(host, base + index_at)
     finally:
         through.record()
+        if waiting is not None:
+            waiting.wait_event(through)                  # before `hold`: from then on the next call may record it again
         moves.hold(through)
-    return buf, through
+    return buf
 
 
 def _levels(bins, num_layers, device):

@@ -119,6 +119,30 @@ def test_staged_pieces_arrive_from_any_team(threads, monkeypatch):
             assert torch.equal(dev.cpu(), want)
 
 
+def test_an_event_is_waited_for_before_it_may_be_recorded_again(monkeypatch):
+    """An upload with a stream of its own, whose event the next call gets at once and records behind long work."""
+    from cachegen_amd.serde import incoming
+    monkeypatch.setattr(incoming, "_WHOLE_BYTES", 1 << 20)
+    hold, other = hostmem.Moves.hold, torch.cuda.Stream()
+
+    def hold_and_lend(moves, event):
+        hold(moves, event)
+        event.synchronize()
+        with torch.cuda.stream(other):
+            torch.cuda._sleep(100_000_000)
+            event.record()
+    monkeypatch.setattr(hostmem.Moves, "hold", hold_and_lend)
+    want = _bytes(3 << 20, 1)
+    torch.cuda.synchronize()
+    with torch.cuda.device(DEV):
+        buf = incoming._upload([(0, want)], (3 << 20) + 64, 3 << 20, lambda base, host: host.zero_())
+        arrived = torch.cuda.current_stream().record_event()
+    arrived.synchronize()
+    assert not other.query(), "the upload was behind another stream's work"
+    other.synchronize()
+    assert torch.equal(buf[:3 << 20].cpu(), want)
+
+
 def test_parts_are_filled_as_they_come():
     src = torch.arange(3 << 20, dtype=torch.int32, device=DEV).view(torch.uint8)
     n = src.numel()
