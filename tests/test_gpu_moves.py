@@ -123,7 +123,7 @@ def test_an_event_is_waited_for_before_it_may_be_recorded_again(monkeypatch):
     """An upload with a stream of its own, whose event the next call gets at once and records behind long work."""
     from cachegen_amd.serde import incoming
     monkeypatch.setattr(incoming, "_WHOLE_BYTES", 1 << 20)
-    hold, other = hostmem.Moves.hold, torch.cuda.Stream()
+    hold, other, lent = hostmem.Moves.hold, torch.cuda.Stream(), []
 
     def hold_and_lend(moves, event):
         hold(moves, event)
@@ -131,6 +131,7 @@ def test_an_event_is_waited_for_before_it_may_be_recorded_again(monkeypatch):
         with torch.cuda.stream(other):
             torch.cuda._sleep(100_000_000)
             event.record()
+        lent.append(event)
     monkeypatch.setattr(hostmem.Moves, "hold", hold_and_lend)
     want = _bytes(3 << 20, 1)
     torch.cuda.synchronize()
@@ -138,8 +139,7 @@ def test_an_event_is_waited_for_before_it_may_be_recorded_again(monkeypatch):
         buf = incoming._upload([(0, want)], (3 << 20) + 64, 3 << 20, lambda base, host: host.zero_())
         arrived = torch.cuda.current_stream().record_event()
     arrived.synchronize()
-    assert not other.query(), "the upload was behind another stream's work"
-    other.synchronize()
+    assert not lent[0].query(), "the upload was behind another stream's work"
     assert torch.equal(buf[:3 << 20].cpu(), want)
 
 
