@@ -7,8 +7,9 @@ namespace {
 // Forks from the caller's stream when made and joins it when it goes out of scope, also after a failed launch: whatever was
 // queued on it is behind the caller's work before the call and before the caller's work after it, so the caller's memory
 // is used as on its own stream.  One stream and two events per device, kept, and lent to one call at a time: a call that
-// finds them lent (ok() false), or whose stream is being captured (a lent stream would belong to that capture until its
-// end), queues everything on its own stream.
+// finds them lent (ok() false), or with work of another stream still on them (it would wait for that: two calls on two
+// streams, the first behind 40 ms of other work, ended after 42 ms both), or whose stream is being captured (a lent
+// stream would belong to that capture until its end), queues everything on its own stream.
 class SideStream {
 public:
     explicit SideStream(hipStream_t caller) : caller_(caller)
@@ -22,7 +23,7 @@ public:
         if (capture != hipStreamCaptureStatusNone || hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kDevices) return;
         Kept &k = kept_[dev];
         if (k.lent.exchange(true, std::memory_order_acquire)) return;
-        if (!k.stream && !make(k)) {
+        if (!(k.stream || make(k)) || !free_for(k, caller)) {
             (void)hipGetLastError();
             k.lent.store(false, std::memory_order_release);
             return;
@@ -32,6 +33,7 @@ public:
             k.lent.store(false, std::memory_order_release);
             return;
         }
+        k.user = caller;
         kept = &k;
     }
 
@@ -54,7 +56,20 @@ private:
         std::atomic<bool> lent{false};
         hipStream_t stream = nullptr;
         hipEvent_t fork = nullptr, join = nullptr;
+        hipStream_t user = nullptr;         // the last caller's, whose work the stream and `join` stand for
     };
+
+    // Whether nothing is on the kept stream but what is before this call on the caller's anyway.  hipStreamPerThread is one
+    // handle for the streams of all threads.
+    static bool free_for(Kept &k, hipStream_t caller)
+    {
+        if (k.user == caller && caller != hipStreamPerThread) return true;
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;        // another thread's capture does not mind
+        const bool changed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+        const hipError_t e = hipEventQuery(k.join);                     // never recorded: through
+        if (changed) (void)hipThreadExchangeStreamCaptureMode(&mode);
+        return e == hipSuccess;
+    }
 
     static bool make(Kept &k)
     {

@@ -96,3 +96,24 @@ def test_levels_on_several_streams_at_once():
     for c in callers:
         c.join()
     assert not wrong
+
+
+def test_a_call_does_not_wait_for_another_streams_work():
+    from cachegen_amd import codec
+    tops = [8, 64, 32]
+    kv, levels = _levels_and_cache(1)
+    want = _bytes(codec.encode_kv_levels(kv, levels, chunk_tokens=256, max_bins=tops))
+    first, second = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(first):
+        torch.cuda._sleep(100_000_000)
+        late = codec.encode_kv_levels(kv, levels, chunk_tokens=256, max_bins=tops)
+        last = first.record_event()
+    with torch.cuda.stream(second):
+        got = codec.encode_kv_levels(kv, levels, chunk_tokens=256, max_bins=tops)
+        through = second.record_event()
+    through.synchronize()
+    assert not last.query(), "the second call was behind the first stream's work"
+    torch.cuda.synchronize()
+    for encs in (late, got):
+        assert all(torch.equal(a, b) for a, b in zip(_bytes(encs), want))
