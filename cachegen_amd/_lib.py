@@ -36,6 +36,8 @@ SIGNATURES = {
                                  _P, _P, _P, _P, _P, _I64, _P, _P, _SZ, _P, _INT]),
     "cg_test_few_encode_blocks": (_INT, [_INT, _INT, _INT, _INT]),
     "cg_encode_kv_levels_workspace": (_SZ, [_I64, _I64, _I64, _I64, _INT]),
+    "cg_encode_kv_levels_least_workspace": (_SZ, [_I64, _I64, _I64, _I64, _INT]),
+    "cg_encode_kv_levels_together": (_INT, [_P, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _INT, _P, _I64]),
     "cg_encode_kv_levels": (_INT, [_P, _INT, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _INT, _P, _P, _P, _I64,
                                    _P, _P, _P, _P, _P, _P, _P, _P, _SZ, _P]),
     "cg_collect_bytes": (_INT, [_P, _I64, _I64, _I64, _P, _I64, _I64, _P, _I64, _P]),

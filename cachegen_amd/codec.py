@@ -374,7 +374,23 @@ def quantize_kv(kv, key_bins, value_bins, fmt="vllm"):
 
 
 def encode_levels_workspace_bytes(num_layers, num_tokens, num_channels, chunk_tokens, num_levels):
+    """Bytes with which levels share launches where they can.  `encode_kv_levels` takes less, down to one level's scratch beside
+    all levels' symbols (`encode_levels_least_workspace_bytes`), and then codes the levels one behind the other."""
     return int(_lib.lib().cg_encode_kv_levels_workspace(num_layers, num_tokens, num_channels, chunk_tokens, num_levels))
+
+
+def encode_levels_least_workspace_bytes(num_layers, num_tokens, num_channels, chunk_tokens, num_levels):
+    return int(_lib.lib().cg_encode_kv_levels_least_workspace(num_layers, num_tokens, num_channels, chunk_tokens, num_levels))
+
+
+def _workspace(wanted, least, device):
+    """`wanted` bytes, or `least` where the GPU does not have that many."""
+    try:
+        return torch.empty(wanted, dtype=torch.uint8, device=device)
+    except torch.cuda.OutOfMemoryError:
+        if least == wanted:
+            raise
+    return torch.empty(least, dtype=torch.uint8, device=device)
 
 
 def encode_kv_levels(kv, levels, chunk_tokens=None, fmt="vllm", workspace=None, max_bins=None, out=None):
@@ -410,9 +426,6 @@ def encode_kv_levels(kv, levels, chunk_tokens=None, fmt="vllm", workspace=None, 
     nchunks = int(lib.cg_num_chunks(T, S))
     nsub = int(lib.cg_num_subchunks(T, S))
     nstreams = nsub * 2 * L * C
-    ws_bytes = int(lib.cg_encode_kv_levels_workspace(L, T, C, S, n))
-    if workspace is None or workspace.numel() < ws_bytes:
-        workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
     if out is None:
         maxima = torch.empty((2, L, T), dtype=kv.dtype, device=dev)
         status = torch.empty(n, dtype=torch.int32, device=dev)
@@ -439,6 +452,10 @@ def encode_kv_levels(kv, levels, chunk_tokens=None, fmt="vllm", workspace=None, 
     def ptrs(ctype, values):
         return (ctype * n)(*values)
 
+    least = int(lib.cg_encode_kv_levels_least_workspace(L, T, C, S, n))
+    if workspace is None or workspace.numel() < least:
+        together = lib.cg_encode_kv_levels_together(kv.data_ptr(), L, T, H, D, sl, skv, st, sh, n, ptrs(ctypes.c_int, max_bins), S)
+        workspace = _workspace(int(lib.cg_encode_kv_levels_workspace(L, T, C, S, n)) if together else least, least, dev)
     with torch.cuda.device(dev):
         _lib.check(lib.cg_encode_kv_levels(
             kv.data_ptr(), _DT[kv.dtype], L, T, H, D, sl, skv, st, sh, n,

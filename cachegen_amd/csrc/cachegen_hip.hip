@@ -278,11 +278,13 @@ int cg_scan_lengths_static(const int32_t *lengths, int64_t n, int64_t *offsets, 
 namespace {
 
 // Workspace of the fused encoder, carved in this order: `nlevels` symbol areas (a 256-token
-// slot per stream each); per level the coder's scratch tiles and the small arrays of the two running
+// slot per stream each); `areas` times the coder's scratch tiles and the small arrays of the two running
 // sums; the group sums of all levels.  The pointers are level 0's; level(v) has those of level v.
+// areas: one for each level, or one that levels coded one behind the other share.
 struct EncodeWorkspace {
     size_t symbols_bytes;       // one level's symbols
-    size_t level_bytes;         // one level's scratch and sums
+    size_t area_bytes;          // one area's scratch and sums
+    int areas;
     uint8_t *symbols, *scratch;
     void *scan_scratch, *tile_scan_scratch;
     int32_t *tile_sums, *group_sums;
@@ -290,7 +292,7 @@ struct EncodeWorkspace {
     int64_t nsub, nstreams, ntiles;
     size_t total;
 
-    EncodeWorkspace(void *base, int64_t L, int64_t T, int64_t C, int64_t chunk_tokens, int nlevels)
+    EncodeWorkspace(void *base, int64_t L, int64_t T, int64_t C, int64_t chunk_tokens, int nlevels, int nareas = 1) : areas(nareas)
     {
         nsub = cg_num_subchunks(T, chunk_tokens);
         nstreams = nsub * 2 * L * C;
@@ -309,8 +311,8 @@ struct EncodeWorkspace {
         ws += align_up((size_t)(ntiles + 1) * sizeof(int64_t), 256);
         tile_scan_scratch = ws;
         ws += cg_scan_workspace(ntiles);
-        level_bytes = align_up((size_t)(ws - scratch), 256);
-        ws = scratch + level_bytes * (size_t)nlevels;
+        area_bytes = align_up((size_t)(ws - scratch), 256);
+        ws = scratch + area_bytes * (size_t)areas;
         group_sums = reinterpret_cast<int32_t *>(ws);          // bytes per group of kTileGroup tiles
         ws += align_up((size_t)nlevels * kMaxTileGroups * sizeof(int32_t), 256);
         total = (size_t)(ws - static_cast<uint8_t *>(base));
@@ -319,7 +321,7 @@ struct EncodeWorkspace {
     EncodeWorkspace level(int v) const
     {
         EncodeWorkspace w = *this;
-        const size_t by = level_bytes * (size_t)v;
+        const size_t by = areas > 1 ? area_bytes * (size_t)v : 0;
         w.symbols += symbols_bytes * (size_t)v;
         w.scratch += by;
         w.scan_scratch = static_cast<uint8_t *>(scan_scratch) + by;
@@ -331,6 +333,19 @@ struct EncodeWorkspace {
     }
 };
 
+// Tiles of a level up to which several levels have an area of scratch each, so that they can share launches: that is
+// 1 GB of scratch for one level and 3 more for four.  Beyond, the launches' ends matter little and the memory much.  Four levels
+// of 1024 channels, one behind the other with one scratch / shared, us: 32 layers x 4096 tokens in chunks of 128 (8192 tiles)
+// 1381 / 1305, 8192 tokens in chunks of 256 2155 / 2060, 16384 tokens (16384 tiles) 4250 / 4100 and 4720 / 4407 with one
+// table over them; 2048 tokens in chunks of 16 (32768 tiles) 2958 / 2984, 4096 tokens (65536) 5957 / 5950, 80 layers x 32768
+// tokens in chunks of 256 (81920) 20480 / 20380 with 27 GB of workspace / 43.
+constexpr int64_t kApartTiles = 16384;
+
+int level_areas(int64_t L, int64_t T, int64_t C, int64_t chunk_tokens, int nlevels)
+{
+    return ceil_div(cg_num_subchunks(T, chunk_tokens) * 2 * L * C, kSlotTile) <= kApartTiles ? nlevels : 1;
+}
+
 }  // namespace
 
 extern "C" {
@@ -341,6 +356,12 @@ size_t cg_encode_kv_workspace(int64_t L, int64_t T, int64_t C, int64_t chunk_tok
 }
 
 size_t cg_encode_kv_levels_workspace(int64_t L, int64_t T, int64_t C, int64_t chunk_tokens, int nlevels)
+{
+    if (nlevels < 1 || nlevels > CG_MAX_LEVELS) return 0;
+    return EncodeWorkspace(nullptr, L, T, C, chunk_tokens, nlevels, level_areas(L, T, C, chunk_tokens, nlevels)).total;
+}
+
+size_t cg_encode_kv_levels_least_workspace(int64_t L, int64_t T, int64_t C, int64_t chunk_tokens, int nlevels)
 {
     if (nlevels < 1 || nlevels > CG_MAX_LEVELS) return 0;
     return EncodeWorkspace(nullptr, L, T, C, chunk_tokens, nlevels).total;
@@ -473,6 +494,15 @@ int code_and_compact(const LevelOut &o, const uint32_t *sym4, const uint8_t *sym
     return check_launch("compact");
 }
 
+// Whether levels of these table sizes can share launches: blocks of 256 lanes for all of them, and sub-chunks of
+// all levels are one grid dimension.
+bool levels_alike(const int *max_bins, int n, int64_t nsub, int64_t C)
+{
+    bool alike = n > 1 && nsub * n <= 65535;
+    for (int v = 0; v < n; ++v) alike = alike && pick_block(C, max_bins[v] + 1) == kSlotTile;
+    return alike;
+}
+
 // Several levels of one tensor from their packed symbols (level v's in w.level(v)): as code_and_compact for each,
 // with a launch for all of them where they can share one.  A launch of one level ends with its slowest streams
 // while the next waits, and a small one does not fill the GPU: it lasts as long as one stream's chain of symbols,
@@ -489,13 +519,12 @@ int code_and_compact_levels(const LevelOut *o, int n, const EncodeWorkspace &w, 
                             int64_t chunk_tokens, hipStream_t s, const void *maxima, int max_dt, bool sums_cleared)
 {
     const int64_t rows = 2 * L;
-    int max_lp = 0;
-    bool alike = w.nsub * n <= 65535;                       // sub-chunks of all levels are one grid dimension
+    int max_lp = 0, max_bins[kMaxLevels];
     for (int v = 0; v < n; ++v) {
-        if (o[v].max_bins + 1 > max_lp) max_lp = o[v].max_bins + 1;
-        alike = alike && pick_block(C, o[v].max_bins + 1) == kSlotTile;
+        max_bins[v] = o[v].max_bins;
+        if (max_bins[v] + 1 > max_lp) max_lp = max_bins[v] + 1;
     }
-    if (!alike || n == 1) {
+    if (w.areas != n || !levels_alike(max_bins, n, w.nsub, C)) {
         for (int v = 0; v < n; ++v) {
             const EncodeWorkspace wv = w.level(v);
             if (int rc = code_and_compact(o[v], reinterpret_cast<uint32_t *>(wv.symbols), nullptr, wv, L, T, C, chunk_tokens, s, maxima, max_dt,
@@ -717,6 +746,15 @@ int cg_test_few_encode_blocks(int source, int lp, int block, int tile)
     return (int)few_encode_blocks(static_cast<EncodeSource>(source), lp, block, tile != 0);
 }
 
+int cg_encode_kv_levels_together(const void *kv, int64_t L, int64_t T, int64_t H, int64_t D, int64_t sl, int64_t skv, int64_t st, int64_t sh,
+                                 int nlevels, const int *max_bins, int64_t chunk_tokens)
+{
+    if (!max_bins || nlevels < 1 || nlevels > CG_MAX_LEVELS || chunk_tokens <= 0) return 0;
+    const int64_t C = H * D;
+    return kv_vectorizable(kv, D, C, sl, skv, st, sh) && C % 8 == 0 && level_areas(L, T, C, chunk_tokens, nlevels) > 1 &&
+           levels_alike(max_bins, nlevels, cg_num_subchunks(T, chunk_tokens), C);
+}
+
 int cg_encode_kv_levels(const void *kv, int kv_dt, int64_t L, int64_t T, int64_t H, int64_t D, int64_t sl,
                         int64_t skv, int64_t st, int64_t sh, int nlevels, const float *const *key_bins,
                         const float *const *value_bins, const int *max_bins, int64_t chunk_tokens,
@@ -740,7 +778,9 @@ int cg_encode_kv_levels(const void *kv, int kv_dt, int64_t L, int64_t T, int64_t
         outs[v] = {key_bins[v], value_bins[v], max_bins[v], cdf[v], lengths[v], offsets[v], payload[v], payload_cap[v], status + v};
     }
     const int64_t C = H * D;
-    const EncodeWorkspace w(workspace, L, T, C, chunk_tokens, nlevels);
+    int areas = level_areas(L, T, C, chunk_tokens, nlevels);
+    if (workspace_bytes < EncodeWorkspace(nullptr, L, T, C, chunk_tokens, nlevels, areas).total) areas = 1;
+    const EncodeWorkspace w(workspace, L, T, C, chunk_tokens, nlevels, areas);
     if (workspace_bytes < w.total) return fail(CG_ERR_WORKSPACE, "encode_kv_levels: workspace too small");
     if (!aligned_to(workspace, 256)) return fail(CG_ERR_ARG, "encode_kv_levels: workspace must be 256-byte aligned");
     hipStream_t s = static_cast<hipStream_t>(stream);

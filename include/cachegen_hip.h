@@ -203,10 +203,20 @@ int cg_test_few_encode_blocks(int source, int lp, int block, int tile);
  *                        a HOST array of nlevels capacities
  * maxima                 device 16-bit [2, L, T]: the row maxima do not depend on the level
  * status                 device int32 [nlevels]
- * workspace              cg_encode_kv_levels_workspace(...) bytes, 256-aligned
+ * workspace              cg_encode_kv_levels_workspace(...) bytes, 256-aligned: symbols for every level and, up to
+ *                        16384 tiles of 256 streams a level, stream scratch for every level, so that levels can share
+ *                        launches; with less, down to cg_encode_kv_levels_least_workspace(...), whose levels share one
+ *                        scratch, they are coded one behind the other.  32 layers x 4096 tokens x 1024 channels, four
+ *                        levels: 2.15 GB and 1.35 GB
  * 1 <= nlevels <= CG_MAX_LEVELS.  Tensors whose head size or strides are not multiples of 8
  * are quantized once per level instead. */
 size_t cg_encode_kv_levels_workspace(int64_t L, int64_t T, int64_t C, int64_t chunk_tokens, int nlevels);
+size_t cg_encode_kv_levels_least_workspace(int64_t L, int64_t T, int64_t C, int64_t chunk_tokens, int nlevels);
+/* Whether the levels of a call with these arguments share launches where the workspace is the larger one (tensors that the
+ * vector loads take, tables of at most 80 entries, more than 128 channels): the least one is as good otherwise. */
+int cg_encode_kv_levels_together(const void *kv, int64_t L, int64_t T, int64_t H, int64_t D,
+                                 int64_t sl, int64_t skv, int64_t st, int64_t sh,
+                                 int nlevels, const int *max_bins, int64_t chunk_tokens);
 int cg_encode_kv_levels(const void *kv, int kv_dt, int64_t L, int64_t T, int64_t H, int64_t D,
                         int64_t sl, int64_t skv, int64_t st, int64_t sh,
                         int nlevels, const float *const *key_bins, const float *const *value_bins,

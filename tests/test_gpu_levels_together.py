@@ -117,3 +117,38 @@ def test_a_call_does_not_wait_for_another_streams_work():
     torch.cuda.synchronize()
     for encs in (late, got):
         assert all(torch.equal(a, b) for a, b in zip(_bytes(encs), want))
+
+
+@pytest.mark.parametrize("shape,chunk,tops", [c for c in CASES if len(c[2]) > 1])
+def test_levels_with_the_least_workspace(shape, chunk, tops):
+    """Levels that share one scratch, one behind the other; nothing behind the workspace is written."""
+    from cachegen_amd import codec
+    from cachegen_amd.kvgen import make_kv
+    L, T, H, D = shape
+    kv = make_kv(L, T, H, D, seed=3 + T, device=DEV, dtype=torch.float16)
+    levels = [(_bins(float(t), L), _bins(float(t), L)) for t in tops]
+    n = codec.encode_levels_least_workspace_bytes(L, T, H * D, chunk, len(tops))
+    assert n < codec.encode_levels_workspace_bytes(L, T, H * D, chunk, len(tops))
+    room = torch.full((n + 4096,), 7, dtype=torch.uint8, device=DEV)
+    print(dict(shape=shape, chunk=chunk, tops=tops), flush=True)
+    want = _bytes(codec.encode_kv_levels(kv, levels, chunk_tokens=chunk))
+    got = codec.encode_kv_levels(kv, levels, chunk_tokens=chunk, workspace=room[:n])
+    assert all(torch.equal(a, b) for a, b in zip(_bytes(got), want))
+    assert (room[n:] == 7).all()
+
+
+def test_a_gpu_without_room_for_the_larger_workspace(monkeypatch):
+    from cachegen_amd import codec
+    kv, levels = _levels_and_cache(1)
+    want = _bytes(codec.encode_kv_levels(kv, levels, chunk_tokens=256))
+    large = codec.encode_levels_workspace_bytes(6, 2048, 1024, 256, 3)
+    empty, asked = torch.empty, []
+
+    def little(*size, **kw):
+        if size == (large,):
+            asked.append(size)
+            raise torch.cuda.OutOfMemoryError
+        return empty(*size, **kw)
+    monkeypatch.setattr(torch, "empty", little)
+    got = codec.encode_kv_levels(kv, levels, chunk_tokens=256)
+    assert asked and all(torch.equal(a, b) for a, b in zip(_bytes(got), want))
