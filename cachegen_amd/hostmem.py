@@ -247,13 +247,17 @@ class Moves:
         self._marked = self._count
         return self.queued()
 
+    def room(self, src):
+        """(a tensor as a kernel can read it from its address on: dense, on the device; pinned uint8 tensor for its bytes, at the
+        same place inside a 16-byte unit)."""
+        src = src.to(self.device).contiguous()
+        n, skew = src.numel() * src.element_size(), src.data_ptr() % 16
+        return src, torch.empty(n + skew, dtype=torch.uint8, pin_memory=True)[skew:]
+
     def down(self, src):
-        """(pinned uint8 tensor that receives the bytes of a device tensor, their arrival)."""
-        src = src.contiguous()
-        n, at = src.numel() * src.element_size(), src.data_ptr()
-        skew = at % 16                                   # the same place inside a 16-byte unit on both sides
-        host = torch.empty(n + skew, dtype=torch.uint8, pin_memory=True)[skew:]
-        return host, self.down_to(at, host) if n else self.queued()
+        """(pinned uint8 tensor that receives the bytes of a tensor, their arrival)."""
+        src, host = self.room(src)
+        return host, self.down_to(src.data_ptr(), host) if host.numel() else self.queued()
 
     def down_to(self, src, host):
         """The same into a slice of pinned memory, from a device address."""

@@ -393,7 +393,7 @@ def _bring_to_host(enc, first_chunk, num_chunks, per_chunk, compact, moves):
         if len(pieces) > 1 or n < 2 * _SLICE_BYTES:
             host, arrival = moves.down(src)
             return host, [(n, arrival)]
-        host = torch.empty(n, dtype=torch.uint8, pin_memory=True)
+        src, host = moves.room(src)
         ends = [n * (i + 1) // (n // _SLICE_BYTES) // 64 * 64 for i in range(n // _SLICE_BYTES - 1)] + [n]
         slices = []
         for at, end in zip([0] + ends, ends):

@@ -153,3 +153,38 @@ def test_parts_are_filled_as_they_come():
     want = src.cpu()
     want[n // 3] = 0
     assert torch.equal(whole, want)
+
+
+# tables in one piece and in slices, dense or not, on the GPU or not
+@pytest.mark.parametrize("layers,tokens", [(2, 40), (36, 256)])
+@pytest.mark.parametrize("form", ["wide", "turned", "host"])
+def test_sections_of_any_layout(layers, tokens, form):
+    import dataclasses
+    from cachegen_amd.kvgen import make_kv
+    from cachegen_amd.serde import wire
+    bins = torch.full((layers,), 32.0, device=DEV)
+    enc = codec.encode_kv(make_kv(layers, tokens, 8, 128, seed=1, device=DEV), bins, bins)
+    want = wire.pack_chunks(enc)
+    if form == "wide":
+        room = torch.zeros((*enc.cdf.shape[:3], enc.cdf.shape[3] + 7), dtype=enc.cdf.dtype, device=DEV)
+        other = {"cdf": room[..., :enc.cdf.shape[3]]}
+        other["cdf"].copy_(enc.cdf)
+    elif form == "turned":
+        other = {"cdf": enc.cdf.transpose(1, 2).contiguous().transpose(1, 2), "lengths": enc.lengths.transpose(1, 2).contiguous().transpose(1, 2)}
+    else:
+        other = {"cdf": enc.cdf.cpu(), "lengths": enc.lengths.cpu(), "maxima": enc.maxima.cpu()}
+    assert wire.pack_chunks(dataclasses.replace(enc, **other)) == want
+
+
+def test_slices_keep_their_place_inside_a_unit():
+    """Tables that begin at no multiple of 16 bytes, in slices: the pinned memory begins at the same place."""
+    from cachegen_amd.kvgen import make_kv
+    from cachegen_amd.serde import wire
+    bins = torch.full((1,), 64.0, device=DEV)
+    enc = codec.encode_kv(make_kv(1, 16, 20001, 1, seed=1, device=DEV), bins, bins, chunk_tokens=8)
+    at = enc.cdf[1].data_ptr()
+    assert at % 16 and enc.cdf[1].numel() * 2 > 2 * wire._SLICE_BYTES
+    for part in wire.bring_to_host(enc, 1, 1):
+        part.arrive()
+        assert len(part.slices) > 1 and part.tables.data_ptr() % 16 == at % 16
+        assert torch.equal(part.tables.view(torch.int16), enc.cdf[1].cpu().view(-1))
