@@ -33,9 +33,12 @@ HIPCC_FLAGS = [
 OCCUPANCY_BUDGETS = [
     (r"^encode_streams_kernel<", 7),         # the forms behind the four reference entry points and odd shapes
     (r"^encode_streams_kernel<256, true, true, (true|false), true, true>", 8),   # the fused path of cg_encode_kv
+    (r"^encode_streams_levels_kernel<", 7),
+    (r"^encode_streams_levels_kernel<256, (true|false), true>", 8),              # of cg_encode_kv_levels
     (r"^decode_streams_kernel<", 8),
     (r"^decode_float_kernel<", 8),
     (r"^compact_streams_kernel<", 8),
+    (r"^compact_levels_kernel<", 8),
     (r"^quantize_pack_kernel<[01], (true|false), 2, false>", 8),                # up to 1024 channels, one level
     (r"^quantize_tables_kernel<[01], (true|false), [12], (9|17|33)>", 4),       # two blocks of eight wavefronts per compute unit
 ]

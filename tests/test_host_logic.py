@@ -253,6 +253,21 @@ def test_built_kernels_keep_their_register_budget():
         build.check_budgets(spilled)
 
 
+def test_budgets_cover_the_kernels_of_several_levels():
+    import json
+    from cachegen_amd import build
+    import pytest
+    with open(build.RESOURCES) as f:
+        resources = json.load(f)
+    build.check_budgets(resources)
+    for name, line in (("encode_streams_levels_kernel<256, true, true>", 8), ("encode_streams_levels_kernel<256, false, true>", 8),
+                       ("encode_streams_levels_kernel<256, false, false>", 7), ("compact_levels_kernel<true, 1>", 8)):
+        broken = dict(resources)
+        broken[name] = dict(resources[name], occupancy=line - 1)
+        with pytest.raises(RuntimeError, match="budget %d" % line):
+            build.check_budgets(broken)
+
+
 def test_probe_library_loads_and_exports_its_entry_points():
     from cachegen_amd import issue_probe
     h = issue_probe.lib()
