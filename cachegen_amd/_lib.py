@@ -52,6 +52,10 @@ SIGNATURES = {
     "cg_tables_to_counts": (_INT, [_P, _INT, _I64, _I64, _P, _P, _P, _P, _P]),
     "cg_pack_counts": (_INT, [_P, _INT, _I64, _I64, _P, _P, _P, _P]),
     "cg_wire_meta": (_INT, [_P, _P, _I64, _I64, _P, _P, _P, _I64, _P, _P]),
+    "cg_watch_new": (_P, [_P]),
+    "cg_watch_free": (None, [_P]),
+    "cg_watch_add": (_INT, [_P, _INT, _P]),
+    "cg_watch_wait": (_INT, [_P, _INT]),
     "cg_move_bytes": (_INT, [_P, _P, _I64, _INT, _P, _INT, _P]),
     "cg_host_fill": (_INT, [_P, _INT, _P, _P, _P]),
     "cg_host_stage": (_INT, [_P, _INT, _P, _INT, _I64, _P, _I64, _P, _INT, _P, _P, _P]),

@@ -229,7 +229,7 @@ def collect_streams(padded, offsets):
     def queue(words, stream):
         words.clear()
         _lib.check(_lib.lib().cg_collect_sizes(offsets.data_ptr(), n, nslots, cap, words.at, stream))
-        _lib.check(_lib.lib().cg_mark(words.mark, words.value, stream))
+        words.set(stream)
     return _collect(padded, offsets, n, nslots, queue)
 
 

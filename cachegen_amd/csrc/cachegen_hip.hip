@@ -47,7 +47,7 @@
 #include "side_stream.hpp"
 #include "host_lengths.hpp"
 #include "host_copy.hpp"
-#include "move_bytes.hpp"
+#include "moves.hpp"
 #include "tables_wire.hpp"
 
 // ======================================================================================
@@ -918,11 +918,33 @@ int cg_host_list(const CgHostContainer *items, int n, const void *const *lengths
     return CG_OK;
 }
 
-int cg_move_bytes(const void *src, void *dst, int64_t n, int to_host, int32_t *mark, int32_t value, void *stream)
+void *cg_watch_new(int32_t *mark)
+{
+    int device = 0;
+    if (!mark || hipGetDevice(&device) != hipSuccess) return nullptr;
+    return new (std::nothrow) Watch(mark, device);
+}
+
+void cg_watch_free(void *watch) { delete static_cast<Watch *>(watch); }
+
+int cg_watch_add(void *watch, int32_t value, void *stream)
+{
+    if (!watch) return fail(CG_ERR_ARG, "watch_add: null pointer");
+    return static_cast<Watch *>(watch)->add(value, static_cast<hipStream_t>(stream));
+}
+
+int cg_watch_wait(void *watch, int32_t value)
+{
+    if (!watch) return fail(CG_ERR_ARG, "watch_wait: null pointer");
+    return static_cast<Watch *>(watch)->wait(value);
+}
+
+int cg_move_bytes(const void *src, void *dst, int64_t n, int to_host, void *watch, int32_t value, void *stream)
 {
     if (!src || !dst || n <= 0) return fail(CG_ERR_ARG, "move_bytes: null pointer or nothing to move");
-    if (mark && !aligned_to(mark, 4)) return fail(CG_ERR_ARG, "move_bytes: the mark must be 4-byte aligned");
-    return launch_move_bytes(static_cast<const uint8_t *>(src), static_cast<uint8_t *>(dst), n, to_host != 0, mark, value, static_cast<hipStream_t>(stream));
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (int rc = move_bytes(src, dst, n, to_host != 0, s)) return rc;
+    return watch ? static_cast<Watch *>(watch)->add(value, s) : CG_OK;
 }
 
 int cg_mark(int32_t *mark, int32_t value, void *stream)
@@ -993,7 +1015,7 @@ int cg_decode_fast_lengths(const int16_t *cdf, int lp, const uint8_t *bytes, int
     return cg_decode_fast_prefsum(cdf, lp, bytes, nbytes, offsets + 1, nl, nt, nc, out, o0, o1, o2, stream);
 }
 
-int cg_host_fill(const CgHostPart *parts, int n, const int32_t *mark, const CgHostTeam *team, void *stream)
+int cg_host_fill(const CgHostPart *parts, int n, const int32_t *mark, const CgHostTeam *team, void *watch)
 {
     if (!parts || n <= 0 || !mark) return fail(CG_ERR_ARG, "host_fill: null pointer or nothing to copy");
     try {
@@ -1007,14 +1029,10 @@ int cg_host_fill(const CgHostPart *parts, int n, const int32_t *mark, const CgHo
         }
         seal(job, 1);
         int32_t last = INT_MIN;
-        for (const HostBlock &b : job.blocks) last = b.value > last ? b.value : last;
+        for (const HostBlock &b : job.blocks) last = std::max(last, b.value);
         int rc = CG_OK;
-        MarkWatch watch(mark, static_cast<hipStream_t>(stream));
         const std::function<void()> idle = [&] {
-            if (rc || job.known.load(std::memory_order_relaxed) >= last || !watch.overdue(last)) return;
-            // everything was queued before the call: once the stream is through, all is there
-            if ((rc = watch.settle())) job.stop.store(true);
-            else job.known.store(last, std::memory_order_release);
+            if (!rc && watch && (rc = static_cast<Watch *>(watch)->look(last))) job.stop.store(true);
         };
         run_job(job, team, &idle);
         return rc;
@@ -1023,23 +1041,33 @@ int cg_host_fill(const CgHostPart *parts, int n, const int32_t *mark, const CgHo
     }
 }
 
-int cg_host_stage(const CgHostPart *parts, int n, void *const *slots, int nslots, int64_t step, void *area, int64_t bytes, int32_t *mark,
+int cg_host_stage(const CgHostPart *parts, int n, void *const *slots, int nslots, int64_t step, void *area, int64_t bytes, void *watch,
                   int32_t value, const CgHostTeam *team, int *moves, void *stream)
 {
     if (moves) *moves = 0;
-    if (const char *what = stage_fault(parts, n, slots, nslots, step, area, bytes, mark, moves)) return fail(CG_ERR_ARG, "host_stage: %s", what);
+    if (const char *what = stage_fault(parts, n, slots, nslots, step, area, bytes, moves)) return fail(CG_ERR_ARG, "host_stage: %s", what);
     try {
         hipStream_t s = static_cast<hipStream_t>(stream);
-        MarkWatch watch(mark, s);
-        return stage_job(parts, n, slots, nslots, step, bytes, mark, value, team, moves,
-                         [&](const uint8_t *from, int64_t at, int64_t size, int32_t mine) {
-                             return launch_move_bytes(from, static_cast<uint8_t *>(area) + at, size, false, mark, mine, s);
-                         },
-                         [&](int32_t upto) {
-                             if (!watch.overdue(upto)) return 0;
-                             const int rc = watch.settle();          // the launches so far are through once the stream is
-                             return rc ? rc : 1;
-                         });
+        int device = 0;
+        if (hipGetDevice(&device) != hipSuccess) return fail(CG_ERR_LAUNCH, "host_stage: no device");
+        // a place behind each move whose slot is used again (the copy engine stops for 4 us at each)
+        int32_t through = 0;
+        Watch steps(&through, device);
+        int32_t launched = 0;
+        const int rc = stage_job(parts, n, slots, nslots, step, bytes, team, moves,
+                                 [&](const uint8_t *from, int64_t at, int64_t size) {
+                                     const int bad = move_bytes(from, static_cast<uint8_t *>(area) + at, size, false, s);
+                                     if (bad) return bad;
+                                     ++launched;
+                                     return at + nslots * step < bytes ? steps.add(launched, s) : CG_OK;
+                                 },
+                                 [&] {
+                                     const int bad = steps.look(through);
+                                     return bad ? bad : through;
+                                 });
+        *moves = launched;
+        if (rc || !watch) return rc;
+        return static_cast<Watch *>(watch)->add(value, s);
     } catch (const std::exception &e) {
         return fail(CG_ERR_ARG, "host_stage: %s", e.what());
     }
@@ -1048,20 +1076,22 @@ int cg_host_stage(const CgHostPart *parts, int n, void *const *slots, int nslots
 int cg_test_host_stage(const CgHostPart *parts, int n, void *const *slots, int nslots, int64_t step, void *area, int64_t bytes,
                        const CgHostTeam *team, int *moves)
 {
-    int32_t mark = 0, value = 1;
     if (moves) *moves = 0;
-    if (const char *what = stage_fault(parts, n, slots, nslots, step, area, bytes, &mark, moves)) return fail(CG_ERR_ARG, "host_stage: %s", what);
+    if (const char *what = stage_fault(parts, n, slots, nslots, step, area, bytes, moves)) return fail(CG_ERR_ARG, "host_stage: %s", what);
     try {
-        // a move reads its slot as late as it may: when the one behind it is launched, which then sets the mark
+        // a move reads its slot as late as it may: when the one behind it is launched
         struct { const uint8_t *from; uint8_t *to; int64_t size; } last = {nullptr, nullptr, 0};
-        const int rc = stage_job(parts, n, slots, nslots, step, bytes, &mark, value, team, moves,
-                                 [&](const uint8_t *from, int64_t at, int64_t size, int32_t mine) {
-                                     if (last.size) memcpy(last.to, last.from, (size_t)last.size);
+        int32_t through = 0;
+        const int rc = stage_job(parts, n, slots, nslots, step, bytes, team, moves,
+                                 [&](const uint8_t *from, int64_t at, int64_t size) {
+                                     if (last.size) {
+                                         memcpy(last.to, last.from, (size_t)last.size);
+                                         ++through;
+                                     }
                                      last = {from, static_cast<uint8_t *>(area) + at, size};
-                                     __atomic_store_n(&mark, mine, __ATOMIC_RELEASE);
                                      return 0;
                                  },
-                                 [](int32_t) { return 0; });
+                                 [&] { return through; });
         if (last.size) memcpy(last.to, last.from, (size_t)last.size);
         return rc;
     } catch (const std::exception &e) {

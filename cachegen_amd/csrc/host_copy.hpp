@@ -52,11 +52,10 @@ struct HostJob {
     std::vector<std::atomic<int32_t>> left; // blocks to come, per step
     std::atomic<int32_t> done{0};           // blocks that are through
     std::atomic<bool> stop{false};
-    const int32_t *mark = nullptr;
-    std::atomic<int32_t> known{INT_MIN};    // how far the mark is known to be by other means
+    const int32_t *mark = nullptr;          // how far what the blocks wait for has got
     int nthreads = 1;
 
-    bool reached(int32_t value) const { return __atomic_load_n(mark, __ATOMIC_ACQUIRE) >= value || known.load(std::memory_order_acquire) >= value; }
+    bool reached(int32_t value) const { return __atomic_load_n(mark, __ATOMIC_ACQUIRE) >= value; }
 };
 
 inline void host_pause()
@@ -162,44 +161,45 @@ struct HostSteps {
     int64_t of(int64_t at) const { return at < step / 4 ? 0 : at < step ? 1 : at / step + 1; }
 };
 
-// cg_host_stage's steps, launched by launch(from, offset in the area, bytes, value for the mark).  settle(value) returns 0
-// to go on looking, 1 when everything launched so far is through, or an error (negative).
-template <typename Launch, typename Settle>
-int stage_job(const CgHostPart *parts, int n, void *const *slots, int nslots, int64_t step, int64_t bytes, const int32_t *mark, int32_t value,
-              const CgHostTeam *team, int *moves, Launch launch, Settle settle)
+// cg_host_stage's steps, launched by launch(from, offset in the area, bytes); through() gives the number of them that are
+// through, or an error (negative).
+template <typename Launch, typename Through>
+int stage_job(const CgHostPart *parts, int n, void *const *slots, int nslots, int64_t step, int64_t bytes, const CgHostTeam *team, int *moves,
+              Launch launch, Through through)
 {
     const HostSteps at_step = {step};
     const int64_t ring_bytes = nslots * step;
     auto pinned = [&](int64_t at) { return static_cast<uint8_t *>(slots[at / step % nslots]) + at % step; };
     const int32_t steps = (int32_t)at_step.of(bytes - 1) + 1;
+    int32_t known = 0;                      // steps that are through, as the other threads read it
     HostJob job;
-    job.mark = mark;
-    job.known.store(value);
+    job.mark = &known;
     job.nthreads = host_threads(team);
     for (int i = 0; i < n; ++i) {
         const CgHostPart &p = parts[i];
         for (int64_t at = p.dst, end = p.dst + p.bytes; at < end;) {
             const int64_t k = at_step.of(at), stop = std::min(end, at_step.start(k + 1));
-            // the slot is free once the move that was there is through, which the launch behind that one says
-            const int32_t need = at < ring_bytes ? value : value + (int32_t)at_step.of(stop - 1 - ring_bytes) + 1;
+            // a slot is free once the step that it held is through
+            const int32_t need = at < ring_bytes ? 0 : (int32_t)at_step.of(stop - 1 - ring_bytes) + 1;
             add_blocks(job, pinned(at), reinterpret_cast<const uint8_t *>(p.src) + (at - p.dst), stop - at,
                        (uintptr_t)p.src + (uintptr_t)(at - p.dst), need, (int32_t)k);
             at = stop;
         }
     }
     seal(job, steps);
+    const bool in_turn = bytes > ring_bytes;
     int rc = 0;
     int32_t launched = 0;
     const std::function<void()> idle = [&] {
         while (!rc && launched < steps && job.left[(size_t)launched].load(std::memory_order_acquire) <= 0) {
             const int64_t at = at_step.start(launched), end = std::min(bytes, at_step.start(launched + 1));
-            rc = launch(pinned(at), at, end - at, value + launched);
+            rc = launch(pinned(at), at, end - at);
             if (!rc) ++launched;
         }
-        if (!rc && launched < steps && launched > 0 && job.known.load(std::memory_order_relaxed) < value + launched) {
-            const int through = settle(value + launched);
-            if (through > 0) job.known.store(value + launched, std::memory_order_release);
-            else rc = through;
+        if (!rc && in_turn && launched < steps && known < launched) {
+            const int32_t now = through();
+            if (now < 0) rc = now;
+            else if (now > known) __atomic_store_n(&known, now, __ATOMIC_RELEASE);
         }
         if (rc) job.stop.store(true);
     };
@@ -211,9 +211,9 @@ int stage_job(const CgHostPart *parts, int n, void *const *slots, int nslots, in
 
 // Whether cg_host_stage's arguments describe something that it can do; null, or what is wrong.
 inline const char *stage_fault(const CgHostPart *parts, int n, void *const *slots, int nslots, int64_t step, const void *area, int64_t bytes,
-                               const int32_t *mark, const int *moves)
+                               const int *moves)
 {
-    if (!parts || n < 0 || !slots || !area || !mark || !moves || bytes <= 0) return "null pointer or nothing to move";
+    if (!parts || n < 0 || !slots || !area || !moves || bytes <= 0) return "null pointer or nothing to move";
     if (step < 64 || step % 64) return "steps are multiples of 64 bytes";
     if (nslots < 2 && nslots * step < bytes) return "pinned memory too small";
     for (int64_t i = 0; i < nslots && i * step < bytes; ++i)

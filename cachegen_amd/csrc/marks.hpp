@@ -1,5 +1,6 @@
 // Part of the CacheGen KV codec library for MI355X (gfx950); included by cachegen_hip.hip, which
-// is the one translation unit.  Marks and words that kernels store to pinned memory for a host that looks at them.
+// is the one translation unit.  Marks and words that kernels store to pinned memory for a host that looks at them: only
+// where a kernel runs that can do it, since beside a busy GPU each launch waits its turn.
 #pragma once
 
 namespace {
@@ -12,6 +13,8 @@ __device__ __forceinline__ void set_mark(int32_t *mark, int32_t value)
 {
     __hip_atomic_store(mark, value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
+
+__global__ void mark_kernel(int32_t *mark, int32_t value) { set_mark(mark, value); }
 
 // Ends a kernel's stores to host memory that a mark will stand for, in the threads that made them.
 __device__ __forceinline__ void host_stores_done() { __threadfence_system(); }
@@ -51,6 +54,26 @@ __global__ __launch_bounds__(64) void largest_kernel(const float *a, const float
         *out = m;
         set_mark(mark, value);
     }
+}
+
+// The word is read for so long, then the stream is waited for, which also finds out about a launch that failed.
+constexpr std::chrono::milliseconds kMarkPatience{200};
+
+// Until *mark >= value.
+int wait_for_mark(const int32_t *mark, int32_t value, hipStream_t stream)
+{
+    const auto start = std::chrono::steady_clock::now();
+    for (;;) {
+        for (int i = 0; i < 64; ++i) {
+            if (__atomic_load_n(mark, __ATOMIC_ACQUIRE) >= value) return CG_OK;
+            __builtin_ia32_pause();
+        }
+        if (std::chrono::steady_clock::now() - start > kMarkPatience) break;
+    }
+    const hipError_t e = hipStreamSynchronize(stream);
+    if (e != hipSuccess) return fail(CG_ERR_LAUNCH, "wait_mark: %s", hipGetErrorString(e));
+    if (__atomic_load_n(mark, __ATOMIC_ACQUIRE) >= value) return CG_OK;
+    return fail(CG_ERR_ARG, "wait_mark: nothing on this stream sets the mark");
 }
 
 }  // namespace

@@ -215,20 +215,20 @@ class Arrival:
 
 
 class Moves:
-    """Bytes between pinned host memory and device memory, moved by a kernel on one stream, and how far they
-    have got: every move sets a pinned word to the number of moves (and other launches that the caller
-    counts) before it, which the host reads without a call to the runtime.
+    """Bytes between pinned host memory and device memory, moved by the copy engines on one stream, and how far they
+    have got: a place of the stream behind each move that is waited for, which the host looks at without waiting and, in
+    native code, in step with its own copies (cg_host_fill).
 
-    torch's pool of pinned memory knows nothing of a kernel's accesses.  What comes down is waited for, at the
+    torch's pool of pinned memory knows nothing of these moves.  What comes down is waited for, at the
     latest when the `with` block ends; what goes up is handed to `hold`."""
+    _watch = None
 
     def __init__(self, device, stream):
         self.device, self.stream = device, stream        # the stream's raw handle; the caller has made the device current
-        self._word = torch.zeros(1, dtype=torch.int32, pin_memory=True)
-        self._at = self._word.data_ptr()
-        self._value = ctypes.c_int32.from_address(self._at)
+        self._word = ctypes.c_int32(0)                   # the number of the last place that the stream is through with
+        self._at = ctypes.addressof(self._word)
         self._count = self._marked = self._reached = 0
-        self._going_up, self._coming_down = [], []       # (number, pinned tensor)
+        self._going_up, self._coming_down = [], []       # pinned tensors, (number, pinned tensor)
 
     def __enter__(self):
         return self
@@ -237,31 +237,45 @@ class Moves:
         if self._reached < self._count:
             self.wait(self._count)
 
+    def __del__(self):
+        if self._watch and _lib is not None:             # (None when the interpreter ends)
+            _lib.lib().cg_watch_free(self._watch)
+
+    def _places(self):
+        if self._watch is None:
+            self._watch = _lib.lib().cg_watch_new(self._at)
+        return self._watch
+
     def queued(self):
-        """What has been launched on the stream so far."""
+        """What has been queued on the stream so far."""
         self._count += 1
         return Arrival(self, self._count)
 
-    def _move(self, src, dst, n, to_host):
-        _lib.check(_lib.lib().cg_move_bytes(src, dst, n, to_host, self._at, self._count, self.stream))
-        self._marked = self._count
-        return self.queued()
+    def here(self):
+        """The same, and not what is queued until somebody waits."""
+        arrival = self.queued()
+        self._mark()
+        return arrival
 
     def room(self, src):
-        """(a tensor as a kernel can read it from its address on: dense, on the device; pinned uint8 tensor for its bytes, at the
+        """(a tensor as it can be moved from its address on: dense, on the device; pinned uint8 tensor for its bytes, at the
         same place inside a 16-byte unit)."""
         src = src.to(self.device).contiguous()
         n, skew = src.numel() * src.element_size(), src.data_ptr() % 16
         return src, torch.empty(n + skew, dtype=torch.uint8, pin_memory=True)[skew:]
 
-    def down(self, src):
-        """(pinned uint8 tensor that receives the bytes of a tensor, their arrival)."""
+    def down(self, src, place=True):
+        """(pinned uint8 tensor that receives the bytes of a tensor, their arrival).  place: False for what arrives just before
+        something else that is waited for (the copy engine stops for 4 us at a place)."""
         src, host = self.room(src)
-        return host, self.down_to(src.data_ptr(), host) if host.numel() else self.queued()
+        return host, self.down_to(src.data_ptr(), host, place) if host.numel() else self.queued()
 
-    def down_to(self, src, host):
+    def down_to(self, src, host, place=True):
         """The same into a slice of pinned memory, from a device address."""
-        arrival = self._move(src, host.data_ptr(), host.numel(), 1)
+        arrival = self.queued()
+        _lib.check(_lib.lib().cg_move_bytes(src, host.data_ptr(), host.numel(), 1, self._places() if place else None, self._count, self.stream))
+        if place:
+            self._marked = self._count
         self._coming_down.append((self._count, host))
         return arrival
 
@@ -276,7 +290,7 @@ class Moves:
                 self._mark()
             described = b"".join(_PART.pack(dst.data_ptr(), src.data_ptr(), dst.numel(), 0 if a is None else a._number, 0)
                                  for dst, src, a in parts)
-            _lib.check(_lib.lib().cg_host_fill(described, len(parts), self._at, team(), self.stream))
+            _lib.check(_lib.lib().cg_host_fill(described, len(parts), self._at, team(), self._places()))
         self._have(last)
 
     def stage(self, pieces, base, size, step, slots=0):
@@ -298,33 +312,29 @@ class Moves:
             places = [pinned[0].data_ptr() + i * step for i in range(nsteps)]
         described = b"".join(_PART.pack(at, t.data_ptr(), t.numel(), 0, 0) for at, t in pieces)
         launched = ctypes.c_int(0)
-        rc = _lib.lib().cg_host_stage(described, len(pieces), (ctypes.c_void_p * len(places))(*places), len(places), step, base, size, self._at, self._count,
+        rc = _lib.lib().cg_host_stage(described, len(pieces), (ctypes.c_void_p * len(places))(*places), len(places), step, base, size, None, 0,
                                       team(), ctypes.byref(launched), self.stream)
         if launched.value:
-            self._count += launched.value
-            self._marked = self._count - 1
-            self._going_up += [(self._count, t) for t in pinned]
+            self._count += 1
+            self._going_up += pinned
         _lib.check(rc)
 
     def up(self, host, dst):
         """Pinned memory to a device address; `host` is kept until it has been read."""
-        arrival = self._move(host.data_ptr(), dst, host.numel(), 0)
-        self._going_up.append((self._count, host))
-        reached = self._value.value
-        while self._going_up[0][0] <= reached:
-            del self._going_up[0]
-        return arrival
+        _lib.check(_lib.lib().cg_move_bytes(host.data_ptr(), dst, host.numel(), 0, None, 0, self.stream))
+        self._going_up.append(host)
+        return self.queued()
 
     def wait(self, number):
         if self._reached < number:
             with torch.cuda.device(self.device):
                 if self._marked < number:
                     self._mark()
-                _lib.check(_lib.lib().cg_wait_mark(self._at, number, self.stream))
+                _lib.check(_lib.lib().cg_watch_wait(self._places(), number))
             self._have(number)
 
     def _mark(self):
-        _lib.check(_lib.lib().cg_mark(self._at, self._count, self.stream))
+        _lib.check(_lib.lib().cg_watch_add(self._places(), self._count, self.stream))
         self._marked = self._count
 
     def _have(self, number):
@@ -333,9 +343,8 @@ class Moves:
             del self._coming_down[0]
 
     def hold(self, event):
-        """Keeps what is still going up, and the word, until `event`, recorded behind all moves; the event is `hold`'s
-        from here on."""
-        _hold(event, (self.device.index, self.stream), [self._word] + [t for _, t in self._going_up])
+        """Keeps what is going up until `event`, recorded behind all moves; the event is `hold`'s from here on."""
+        _hold(event, (self.device.index, self.stream), self._going_up)
         self._reached = self._count
 
 

@@ -19,12 +19,12 @@ from . import wire
 
 _ALIGN = 256
 # Uploads of more than _WHOLE_BYTES have a stream of their own (_upload) and pass through a few pinned pieces.  Pieces
-# are moved by a launch each, which costs the bus 2 us (53 MB by 2 MB: 1.1 ms, by 4 MB 1.04).
+# cost the bus some 15 us each besides their bytes (42 MB merged from pieces of 4 MB 1338 us, of 8 MB 1250, of 8 MB with pinned
+# memory for all of them 1225; a store of 59 MB is the same with either).
 _WHOLE_BYTES = 16 << 20
-_PIECE_BYTES, _PIECES = 4 << 20, 4
+_PIECE_BYTES, _PIECES = 8 << 20, 4
 # Up to this, torch's own copies: the host, not the bus, is what such a call waits for, and what goes up by moves has to be
-# kept until it is through (chunks of 16 to 80 tokens x 512 channels x 32 layers as counts 110 us by copies, 117 by moves;
-# 150 tokens 116 and 116, 256 tokens 126 and 116).
+# kept until it is through.
 _SMALL_BYTES = 1 << 20
 
 _ITEM = struct.Struct("<10q4i")      # CgHostContainer
@@ -234,14 +234,13 @@ def decode(items, out, fmt):
         base = buf.data_ptr() + index_at
         stream = codec._stream(buf.device)
         # a word that stays zero unless a kernel finds counts that make no table
-        with hostmem.Words() if counted else contextlib.nullcontext() as there, \
-                hostmem.StoredWords(1, torch.int32) if counted else contextlib.nullcontext() as verdict:
+        with hostmem.StoredWords(1, torch.int32) if counted else contextlib.nullcontext() as verdict:
             for key, (tables, groups) in counted.items():
                 at = base + groups_at[key]
                 _lib.check(lib.cg_rebuild_tables(buf.data_ptr(), index_at, key[0], groups, C, at + 8 * groups, at + 12 * groups, at,
                                                  tables.data_ptr(), verdict.words.data_ptr(), stream))
             if counted:
-                verdict.stored(by=there.set(stream))
+                verdict.stored(by=hostmem.Moves(device, stream).here())
             at = base + subs_at
             for key, members in launches.items():
                 n = sum(k for c, _, _, _ in members for _, k in c.length_arrays)

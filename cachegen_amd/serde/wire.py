@@ -333,10 +333,10 @@ def _device_tables(nsym_host, nsym_dev, data, C, lp, tokens):
 
 # Bytes of blobs that leave the GPU in one go: while the host copies one piece into its blobs, the
 # next is on the bus.  Blobs of one 256-token chunk (6 MB) are a piece each; where that is all
-# there is, the tables are cut in slices so that their copy overlaps with the rest's transfer (each
-# transfer costs about 10 us by itself).
+# there is, long tables are cut in slices so that their copy overlaps with the rest's transfer (each
+# transfer costs 6 to 15 us by itself: tables of 4.3 MB in two, one chunk to bytes and back 558 us, in one 544).
 _PIECE_BYTES = 4 << 20
-_SLICE_BYTES = 2 << 20
+_SLICE_BYTES = 4 << 20
 
 
 class HostPart:
@@ -424,8 +424,6 @@ def _bring_to_host(enc, first_chunk, num_chunks, per_chunk, compact, moves):
         with hostmem.StoredWords(3 + nbounds + ngroups, torch.int64) as words:
             _lib.check(lib.cg_wire_meta(enc.status.data_ptr(), enc.offsets[g_first * rows * C:].data_ptr(), rows * C, nbounds,
                                         ptr(wide), ptr(inexact), ptr(nsym), ngroups, words.words.data_ptr(), stream))
-            maxima, arrival = moves.down(enc.maxima)
-            words.stored(by=arrival)                     # one wait for the words and the maxima
             chunk_bytes = max(1, cdf[0].numel() * cdf.element_size() + min(spc, lengths.shape[0]) * rows * C * 4)
             step = max(1, _PIECE_BYTES // chunk_bytes) if per_chunk else 1
             pieces = [(i, min(i + step, len(groups))) for i in range(0, len(groups), step)]
@@ -435,9 +433,12 @@ def _bring_to_host(enc, first_chunk, num_chunks, per_chunk, compact, moves):
                 tables_src = torch.empty(dense.numel(), dtype=torch.uint8, device=dev)
                 _lib.check(lib.cg_pack_counts(dense.data_ptr(), dense.shape[2], ngroups, C, nsym.data_ptr(), None,
                                               tables_src.data_ptr(), stream))
-            elif not compact:
+            # behind the launches: a copy between two of them costs 20 us
+            maxima, arrival = moves.down(enc.maxima)
+            words.stored(by=arrival)                     # one wait for the words and the maxima
+            if dense is None and not compact:
                 a, b = groups[0][0], groups[pieces[0][1] - 1][1]
-                early = {"tables": fetch_tables(cdf[a - c_first:b - c_first]), "lengths": moves.down(lengths[subs(a):subs(b)])}
+                early = {"tables": fetch_tables(cdf[a - c_first:b - c_first]), "lengths": moves.down(lengths[subs(a):subs(b)], place=False)}
             meta = words.read()
 
     enc.raise_for_status(meta[0])
@@ -465,7 +466,7 @@ def _bring_to_host(enc, first_chunk, num_chunks, per_chunk, compact, moves):
             tables = early.pop("tables", None)
             lens = early.pop("lengths", None)
             return (fetch_tables(table_range(a, b)) if tables is None else tables,
-                    moves.down(lengths_src[subs(a):subs(b)]) if lens is None else lens, moves.down(enc.payload[p0:p1]))
+                    moves.down(lengths_src[subs(a):subs(b)], place=False) if lens is None else lens, moves.down(enc.payload[p0:p1]))
 
     itemsize = lengths_src.element_size()
     queued = queue(pieces[0])

@@ -387,15 +387,24 @@ int cg_lengths_to_u16(const int32_t *lengths, int64_t n, uint16_t *out, int32_t 
  * tensor by tensor and waits).
  * ------------------------------------------------------------------------- */
 
-/* n > 0 bytes from src to dst, one of them in pinned host memory (to_host: dst) and the other in device
- * memory, queued on the stream; fastest where the two addresses are equal modulo 16.  Both stay valid until
- * the launch is through.
- * mark   pinned host int32, or null: set to `value` when everything queued on the stream before this
- *        call is through, together with what this library's launches among it stored to host memory (others': what
- *        they have themselves released to the system) */
-int cg_move_bytes(const void *src, void *dst, int64_t n, int to_host, int32_t *mark, int32_t value, void *stream);
+/* A watch: places of a stream, in order, each with a number, that *mark shows (a word of ordinary host memory, ascending)
+ * once the stream is through with what was queued before the place; brought up to date by the functions that wait.  One
+ * thread at a time; made for the current device.  Null if there is no memory for it. */
+void *cg_watch_new(int32_t *mark);
+void cg_watch_free(void *watch);
+/* A place, here. */
+int cg_watch_add(void *watch, int32_t value, void *stream);
+/* HOST: returns when *mark >= value; CG_ERR_ARG if no place has such a number. */
+int cg_watch_wait(void *watch, int32_t value);
 
-/* The mark alone. */
+/* n > 0 bytes from src to dst, one of them in pinned host memory (to_host: dst) and the other in device
+ * memory, queued on the stream.  Both stay valid until it is through.
+ * watch  or null: a place behind it, with the number `value` */
+int cg_move_bytes(const void *src, void *dst, int64_t n, int to_host, void *watch, int32_t value, void *stream);
+
+/* Sets *mark (pinned host int32) to `value` when everything queued on the stream before this call is through, together with
+ * what this library's launches among it stored to host memory (others': what they have themselves released to
+ * the system). */
 int cg_mark(int32_t *mark, int32_t value, void *stream);
 
 /* HOST: returns when *mark >= value; CG_ERR_ARG if the stream is through and it is not. */
@@ -439,18 +448,18 @@ typedef struct CgHostPart {
 } CgHostPart;
 
 /* HOST: the copies, by the team, each part as soon as *mark says that it has arrived; returns when all
- * are done.  The launches that set the mark have been queued on the stream. */
-int cg_host_fill(const CgHostPart *parts, int n, const int32_t *mark, const CgHostTeam *team, void *stream);
+ * are done.  watch: the mark's, which has places up to the largest number; or null: somebody else sets the mark. */
+int cg_host_fill(const CgHostPart *parts, int n, const int32_t *mark, const CgHostTeam *team, void *watch);
 
 /* HOST and the stream: `bytes` bytes of device memory at `area` from the parts (ascending, not overlapping; what lies
  * between them is undefined), staged in pinned memory by the team and moved in steps, each as soon as it is staged.
  * step   bytes of a step, a multiple of 64 (the first is a quarter of one)
  * slots  HOST array of nslots addresses of pinned memory, a step each, used in turn: two at least, or as many as
  *        there are steps (the last of them then no larger than what is left); stays valid until the moves are through
- * mark, value  as in cg_move_bytes, `value` for the first move and one more for each
- * moves  written: the moves launched (all of them, or those before an error) */
+ * watch, value  as in cg_move_bytes, behind the last move
+ * moves  written: the moves queued (all of them, or those before an error) */
 int cg_host_stage(const CgHostPart *parts, int n, void *const *slots, int nslots, int64_t step, void *area, int64_t bytes,
-                  int32_t *mark, int32_t value, const CgHostTeam *team, int *moves, void *stream);
+                  void *watch, int32_t value, const CgHostTeam *team, int *moves, void *stream);
 
 /* Test hook, no GPU work: cg_host_stage with a copy on the host in the place of each move, done as late as a move may be;
  * `area` is host memory. */

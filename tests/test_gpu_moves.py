@@ -1,4 +1,4 @@
-"""Bytes between pinned and device memory by kernel, and the marks that say how far a stream is."""
+"""Bytes between pinned and device memory, and what says how far a stream is."""
 import pytest
 import torch
 
@@ -158,10 +158,11 @@ def test_parts_are_filled_as_they_come():
 # tables in one piece and in slices, dense or not, on the GPU or not
 @pytest.mark.parametrize("layers,tokens", [(2, 40), (36, 256)])
 @pytest.mark.parametrize("form", ["wide", "turned", "host"])
-def test_sections_of_any_layout(layers, tokens, form):
+def test_sections_of_any_layout(layers, tokens, form, monkeypatch):
     import dataclasses
     from cachegen_amd.kvgen import make_kv
     from cachegen_amd.serde import wire
+    monkeypatch.setattr(wire, "_SLICE_BYTES", 2 << 20)
     bins = torch.full((layers,), 32.0, device=DEV)
     enc = codec.encode_kv(make_kv(layers, tokens, 8, 128, seed=1, device=DEV), bins, bins)
     want = wire.pack_chunks(enc)
@@ -176,10 +177,11 @@ def test_sections_of_any_layout(layers, tokens, form):
     assert wire.pack_chunks(dataclasses.replace(enc, **other)) == want
 
 
-def test_slices_keep_their_place_inside_a_unit():
+def test_slices_keep_their_place_inside_a_unit(monkeypatch):
     """Tables that begin at no multiple of 16 bytes, in slices: the pinned memory begins at the same place."""
     from cachegen_amd.kvgen import make_kv
     from cachegen_amd.serde import wire
+    monkeypatch.setattr(wire, "_SLICE_BYTES", 2 << 20)
     bins = torch.full((1,), 64.0, device=DEV)
     enc = codec.encode_kv(make_kv(1, 16, 20001, 1, seed=1, device=DEV), bins, bins, chunk_tokens=8)
     at = enc.cdf[1].data_ptr()
@@ -188,3 +190,32 @@ def test_slices_keep_their_place_inside_a_unit():
         part.arrive()
         assert len(part.slices) > 1 and part.tables.data_ptr() % 16 == at % 16
         assert torch.equal(part.tables.view(torch.int16), enc.cdf[1].cpu().view(-1))
+
+
+def test_bytes_cross_beside_a_busy_gpu():
+    """Moves do not wait for the compute units: 16 MB up and down, in four steps each, while another stream's matrix products
+    (0.8 ms each) keep them busy: 0.7 ms, as on a quiet GPU; by launches, each of which waits for the product before it, 6,
+    but for one stream in four, which shares the products' hardware queue."""
+    a = torch.randn(8192, 8192, dtype=torch.bfloat16, device=DEV)
+    c = torch.empty_like(a)
+    want, dev = _bytes(16 << 20, 3), torch.empty(16 << 20, dtype=torch.uint8, device=DEV)
+    up, down = want.pin_memory(), torch.empty(16 << 20, dtype=torch.uint8, pin_memory=True)
+    busy, took = torch.cuda.Stream(), []
+    for _ in range(8):
+        mine = torch.cuda.Stream()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(busy):
+            for _ in range(30):
+                torch.mm(a, a, out=c)
+        begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        with torch.cuda.stream(mine), hostmem.Moves(DEV, codec._stream(DEV)) as moves:
+            begin.record()
+            for at in range(0, 16 << 20, 4 << 20):
+                moves.up(up[at:at + (4 << 20)], dev.data_ptr() + at)
+            for at in range(0, 16 << 20, 4 << 20):
+                moves.down_to(dev.data_ptr() + at, down[at:at + (4 << 20)])
+            end.record()
+        end.synchronize()
+        took.append(begin.elapsed_time(end))
+        assert torch.equal(down, want)
+    assert sorted(took)[4] < 2.5, took

@@ -36,8 +36,7 @@ def nothing_held(monkeypatch):
 def hold(size, event, stream=1):
     moves = object.__new__(hostmem.Moves)
     moves.device, moves.stream = torch.device("cuda", 0), stream
-    moves._word = torch.zeros(0, dtype=torch.int32)
-    moves._going_up, moves._count = [(1, torch.empty(size, dtype=torch.uint8))], 1
+    moves._going_up, moves._count = [torch.empty(size, dtype=torch.uint8)], 1
     moves.hold(event)
     return event
 

@@ -28,7 +28,7 @@ def code_object(tmp_path_factory):
 
 
 @pytest.mark.parametrize("kernel", ["mark_kernel", "read_words_kernel", "largest_kernel", "scan_collect_kernel", "collect_sizes_kernel",
-                                    "wire_meta_kernel", "counts_to_tables_kernel", "move_bytes_kernelILb1E"])
+                                    "wire_meta_kernel", "counts_to_tables_kernel"])
 def test_stores_are_released_to_the_system(code_object, kernel):
     at, name, symbols = code_object
     found = [s for s in symbols if re.search(r"\d%s" % kernel, s)]
