@@ -262,7 +262,7 @@ class Moves:
         same place inside a 16-byte unit)."""
         src = src.to(self.device).contiguous()
         n, skew = src.numel() * src.element_size(), src.data_ptr() % 16
-        return src, torch.empty(n + skew, dtype=torch.uint8, pin_memory=True)[skew:]
+        return src, pinned(n + skew)[skew:]
 
     def down(self, src, place=True):
         """(pinned uint8 tensor that receives the bytes of a tensor, their arrival).  place: False for what arrives just before
@@ -298,25 +298,25 @@ class Moves:
         to pinned memory and moved by steps as they are there.  slots: pinned steps that are used in turn (0: as
         many as it takes)."""
         if size <= _FEW_BYTES and len(pieces) <= 2:
-            host = torch.empty(size, dtype=torch.uint8, pin_memory=True)
+            host = pinned(size)
             for at, t in pieces:
                 host[at:at + t.numel()].copy_(t)
             self.up(host, base)
             return
         nsteps = -(-size // step)
         if slots and slots < nsteps:
-            pinned = [torch.empty(step, dtype=torch.uint8, pin_memory=True) for _ in range(slots)]
-            places = [t.data_ptr() for t in pinned]
+            memory = [pinned(step) for _ in range(slots)]
+            places = [t.data_ptr() for t in memory]
         else:
-            pinned = [torch.empty(size, dtype=torch.uint8, pin_memory=True)]
-            places = [pinned[0].data_ptr() + i * step for i in range(nsteps)]
+            memory = [pinned(size)]
+            places = [memory[0].data_ptr() + i * step for i in range(nsteps)]
         described = b"".join(_PART.pack(at, t.data_ptr(), t.numel(), 0, 0) for at, t in pieces)
         launched = ctypes.c_int(0)
         rc = _lib.lib().cg_host_stage(described, len(pieces), (ctypes.c_void_p * len(places))(*places), len(places), step, base, size, None, 0,
                                       team(), ctypes.byref(launched), self.stream)
         if launched.value:
             self._count += 1
-            self._going_up += pinned
+            self._going_up += memory
         _lib.check(rc)
 
     def up(self, host, dst):
@@ -410,6 +410,14 @@ def _let_all_go():
             _gone(h)
         else:
             standing.add(h[1])
+
+
+def pinned(n):
+    """uint8 tensor of pinned memory.  What earlier uploads have read by now is given back first: torch's pool would otherwise get
+    new memory from the system, which takes long and is not allowed while another thread captures a graph."""
+    with _held_lock:
+        _let_go()
+    return torch.empty(n, dtype=torch.uint8, pin_memory=True)
 
 
 def event(device):

@@ -109,7 +109,7 @@ def _transfer(pieces, total, index_at, write_index, device, waiting=None):
     if total <= _SMALL_BYTES:
         for at, end, write in ((0, index_at, lambda host: [host[a:a + t.numel()].copy_(t) for a, t in pieces]),
                                (index_at, total, lambda host: write_index(base, host))):
-            host = torch.empty(end - at, dtype=torch.uint8, pin_memory=True)
+            host = hostmem.pinned(end - at)
             write(host)
             buf[at:end].copy_(host, non_blocking=True)
         return buf
@@ -120,7 +120,7 @@ def _transfer(pieces, total, index_at, write_index, device, waiting=None):
             moves.stage(pieces, base, index_at, _PIECE_BYTES // 128 * 64)
         else:
             moves.stage(pieces, base, index_at, _PIECE_BYTES, _PIECES)
-        host = torch.empty(total - index_at, dtype=torch.uint8, pin_memory=True)
+        host = hostmem.pinned(total - index_at)
         write_index(base, host)
         moves.up(host, base + index_at)
     finally:

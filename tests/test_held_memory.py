@@ -91,3 +91,17 @@ def test_others_are_not_held_up_by_a_wait():
     go.set()
     t.join()
     assert held() == 0
+
+
+def test_memory_that_has_been_read_serves_the_next_allocation(monkeypatch):
+    """Not only the next upload: torch's pool would get new memory from the system for what comes down meanwhile."""
+    given = []
+    monkeypatch.setattr(torch, "empty", lambda *size, pin_memory=False, **kw: given.append(held()) or torch.zeros(*size, **kw))
+    first, second = hold(1000, Event()), hold(2000, Event())
+    given.clear()
+    first.through.set()
+    assert hostmem.pinned(64).shape == (64,) and given.pop() == 2000
+    second.through.set()
+    device = torch.device("cpu")
+    hostmem.Moves(device, 0).room(torch.zeros(8))
+    assert given.pop() == 0
