@@ -56,6 +56,17 @@ __global__ __launch_bounds__(64) void largest_kernel(const float *a, const float
     }
 }
 
+// hipEventQuery, also while another thread captures a graph: asked in that thread's way it counts among the calls that a
+// capture in the global mode refuses and is broken by.
+hipError_t query_event(hipEvent_t e)
+{
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    const bool changed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    const hipError_t rc = hipEventQuery(e);
+    if (changed) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    return rc;
+}
+
 // The word is read for so long, then the stream is waited for, which also finds out about a launch that failed.
 constexpr std::chrono::milliseconds kMarkPatience{200};
 

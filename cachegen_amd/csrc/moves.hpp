@@ -95,7 +95,7 @@ public:
     int look(int32_t value)
     {
         while (next_ < places_.size()) {
-            const hipError_t rc = hipEventQuery(places_[next_].event);
+            const hipError_t rc = query_event(places_[next_].event);
             if (rc == hipErrorNotReady) {
                 (void)hipGetLastError();
                 return CG_OK;

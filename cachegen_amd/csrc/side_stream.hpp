@@ -64,11 +64,7 @@ private:
     static bool free_for(Kept &k, hipStream_t caller)
     {
         if (k.user == caller && caller != hipStreamPerThread) return true;
-        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;        // another thread's capture does not mind
-        const bool changed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
-        const hipError_t e = hipEventQuery(k.join);                     // never recorded: through
-        if (changed) (void)hipThreadExchangeStreamCaptureMode(&mode);
-        return e == hipSuccess;
+        return query_event(k.join) == hipSuccess;                       // never recorded: through
     }
 
     static bool make(Kept &k)

@@ -1,4 +1,6 @@
 """Bytes between pinned and device memory, and what says how far a stream is."""
+import threading
+
 import pytest
 import torch
 
@@ -219,3 +221,59 @@ def test_bytes_cross_beside_a_busy_gpu():
         took.append(begin.elapsed_time(end))
         assert torch.equal(down, want)
     assert sorted(took)[4] < 2.5, took
+
+
+def _store_and_retrieve():
+    from cachegen_amd.kvgen import make_kv
+    from cachegen_amd.serde import incoming, wire
+    kv = make_kv(8, 600, 8, 128, seed=1, device=DEV)
+    bins = torch.full((8,), 32.0, device=DEV)
+    out = torch.empty_like(kv)
+
+    def store():
+        return wire.pack_chunks(codec.encode_kv(kv, bins, bins, 256, max_bins=32))
+
+    def retrieve(blobs):
+        incoming.decode([(incoming.Container.flat(b), bins, bins, 256 * i) for i, b in enumerate(blobs)], out, "vllm")
+        return out
+    return store, retrieve
+
+
+def test_stores_and_retrieves_in_turn_get_no_more_pinned_memory():
+    store, retrieve = _store_and_retrieve()
+    for i in range(10):
+        if i == 3:
+            before = torch.cuda.host_memory_stats()["num_host_alloc"]
+        retrieve(store())
+        torch.cuda.synchronize()
+    assert torch.cuda.host_memory_stats()["num_host_alloc"] == before
+
+
+def test_another_thread_may_capture_meanwhile():
+    """Neither new pinned memory nor an event's query gets in the way of a graph that another thread captures."""
+    store, retrieve = _store_and_retrieve()
+    want, x, got = store(), torch.zeros(1024, device=DEV), []
+    for _ in range(3):
+        retrieve(store())
+    first = retrieve(want).clone()
+
+    def other():
+        with torch.cuda.device(DEV):
+            got.append(store())
+            got.append(retrieve(got[0]).clone())
+            torch.cuda.current_stream().synchronize()
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    # (torch.cuda.graph would give the device memory that the calls use back to the system first)
+    with torch.cuda.stream(torch.cuda.Stream()):
+        graph.capture_begin(capture_error_mode="global")
+        x.add_(1)
+        t = threading.Thread(target=other)
+        t.start()
+        t.join()
+        x.add_(1)
+        graph.capture_end()
+    for _ in range(3):
+        graph.replay()
+    torch.cuda.synchronize()
+    assert got[0] == want and torch.equal(got[1], first) and (x == 6).all()
