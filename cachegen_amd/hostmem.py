@@ -2,9 +2,10 @@
 tensors.
 
 A blob that goes into or comes out of a store is a Python bytes object of several megabytes.  It
-is copied from and to pinned memory by torch's own copy, which runs on its thread pool and without
-the interpreter lock: 6 MB in 16 us warm and 45 us out of memory the GPU has just written, where
-one thread (numpy, bytes()) takes 80 and 200."""
+is copied from and to pinned memory by several threads and without the interpreter lock: a call's copies as one
+job in step with the bus (`Moves.fill`, `Moves.stage`; cg_host_fill, cg_host_stage), one or two small pieces by
+torch's own copy.  By eight threads 6 MB take 16 us warm and 45 us out of memory the GPU has just written, where
+one (numpy, bytes()) takes 80 and 200."""
 import collections
 import ctypes
 import os
@@ -155,13 +156,8 @@ class Words:
         return self
 
     def set(self, stream):
-        """The mark alone, behind what the stream holds so far: for `StoredWords.stored`."""
+        """The mark alone, behind what the stream holds so far."""
         _lib.check(_lib.lib().cg_mark(self.mark, self.value, stream))
-        self._stream = stream
-        return self
-
-    def synchronize(self):
-        self.wait(self._stream)
 
     def wait(self, stream):
         _lib.check(_lib.lib().cg_wait_mark(self.mark, self.value, stream))

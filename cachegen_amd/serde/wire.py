@@ -557,7 +557,7 @@ def unpack_to_device(blob, device):
     L, T, C = h["num_layers"], h["num_tokens"], h["num_heads"] * h["head_size"]
     lp, nchunks = h["max_bins"] + 1, geo["nchunks"][0]
     from .. import hostmem
-    host = torch.empty(len(blob), dtype=torch.uint8, pin_memory=True)
+    host = hostmem.pinned(len(blob))
     host.copy_(hostmem.view(blob))
     buf = host.to(device, non_blocking=False)      # waits: the pinned buffer is free for the next call at once
     # the lengths are in the blob: their sum is checked here, without asking the device
