@@ -58,6 +58,14 @@ def test_parts_are_copied(threads, sizes):
     assert (room[keep] == 9).all()
 
 
+# either side of the size from which stores go past the caches, with parts that begin and end at any place of a line
+@pytest.mark.parametrize("threads", [0, 3])
+@pytest.mark.parametrize("more", [-1, 0])
+def test_large_jobs_are_copied(threads, more):
+    small = list(range(1, 140))
+    test_parts_are_copied(threads, (*small, (8 << 20) + more - sum(small)))
+
+
 @pytest.mark.parametrize("threads", [1, 6])
 def test_a_part_is_read_only_when_it_has_arrived(threads):
     n = 400000
