@@ -158,6 +158,11 @@ class Words:
     def set(self, stream):
         """The mark alone, behind what the stream holds so far."""
         _lib.check(_lib.lib().cg_mark(self.mark, self.value, stream))
+        self._stream = stream
+        return self
+
+    def synchronize(self):
+        self.wait(self._stream)
 
     def wait(self, stream):
         _lib.check(_lib.lib().cg_wait_mark(self.mark, self.value, stream))
