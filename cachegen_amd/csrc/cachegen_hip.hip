@@ -515,6 +515,14 @@ bool levels_alike(const int *max_bins, int n, int64_t nsub, int64_t C)
 //    512 channels  32 x 4096                 695 /  618    918 /  830    785 /  668
 //                   4 x 2048                 169 /   71    199 /  101    244 /   89
 //   4096 channels  32 x 1024                1348 / 1250   1877 / 1806   1467 / 1385
+// Other tables, 1024 channels in chunks of 256 tokens, with every length that a compute unit holds another number of blocks of
+// in a launch of its own (below):
+//                         32 layers x 4096 tokens     32 x 1024     4 x 256
+//   41, 49, 57, 65                  1713 / 1600       555 / 519    213 /  69
+//   17, 41, 57, 65                  1574 / 1449       515 / 480    195 /  66
+//   13, 21, 33                       978 /  894       328 / 266    125 /  60
+//   65, 65                           965 /  907       276 / 263    109 /  60
+//   9 to 65, eight levels           2890 / 2667       977 / 823    372 /  76
 int code_and_compact_levels(const LevelOut *o, int n, const EncodeWorkspace &w, int64_t L, int64_t T, int64_t C,
                             int64_t chunk_tokens, hipStream_t s, const void *maxima, int max_dt, bool sums_cleared)
 {
@@ -619,8 +627,11 @@ int code_and_compact_levels(const LevelOut *o, int n, const EncodeWorkspace &w, 
     if (nlaunches > 1) {
         const SideStream side(s);
         if (side.ok()) {
-            // the launch of the longest tables, whose LDS leaves half of a compute unit's wavefront slots empty, and its
-            // compaction beside the other levels' coder.  Four levels, one behind the other / beside, us: 32 layers x 4096 tokens
+            // the launch of the longest tables beside the other levels' coder and their compaction.  Their LDS (four blocks of
+            // 65 entries are 135 of 160 KB) leaves half of a compute unit's wavefront slots empty, but room for one block
+            // more with the LDS of 33 entries: on large caches the coders take as long as one behind the other (796 us
+            // and 812), and what is won is the compaction of the shorter tables, which runs beside the longest
+            // tables' coder.  Four levels, one behind the other / beside, us: 32 layers x 4096 tokens
             // x 1024 channels 1070 / 1049, x 1024 tokens 328 / 308, 512 channels 205 / 178, 400 channels 242 / 190; 4 layers x
             // 2048 tokens in chunks of 1500 162 / 135
             if (int rc = code(0, side.stream())) return rc;

@@ -12,8 +12,8 @@ namespace {
 // one 11) and from the copy before it (5 to 15).  But beside a model that keeps the compute units busy every launch waits
 // until the model's kernel has no more workgroups to send.  By kernel / by copies, us: beside matrix products of
 // 0.8 ms each, one behind another, eight chunks (59 MB) decoded 12600 / 2000, one chunk 4500 / 1230, eight chunks
-// stored 15400 / 2920, one 4230 / 390; on a quiet GPU one chunk to bytes and back 449 / 497, a chunk of counts from bytes
-// 135 / 151, store and retrieve of 59 MB 3400 / 3560.
+// stored 15400 / 2920, one 4230 / 390; on a quiet GPU one chunk to bytes and back 442 / 493, a chunk of counts from bytes
+// 130 / 147, store and retrieve of 59 MB 3070 / 3340, merge of 44 MB 1011 / 907.
 //
 // How far they are the host sees by asking an event, which takes 0.1 us and needs no compute unit either; an event's record
 // is 1 us.  Events are kept, up to kKeptEvents a device: a new one takes 9 us.
