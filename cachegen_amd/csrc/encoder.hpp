@@ -417,21 +417,6 @@ __device__ __forceinline__ void encode_streams(const EncodeArgs &a, uint16_t *ta
     uint16_t *col = tab + table_column<BS>(tid);
     uint16_t *cdf_block = a.cdf + ((id.chunk * a.sg.rows + id.row) * a.sg.nc + ch0) * lp;
     const int nwords = (id.n + 3) >> 2;
-    // PACKED: the sub-chunk's words ([word][channel]) are read through a buffer descriptor that
-    // ends with its last word row: the lane's channel is the vector offset, the word row the
-    // scalar one, and a row past the end (or the offset of a lane without a channel) reads
-    // zero, so a load costs no address arithmetic, compare or branch.
-    __amdgpu_buffer_rsrc_t symbols_rsrc;
-    uint32_t symbols_voff = 0xFFFFFFFCu;
-    const uint32_t row_bytes = (uint32_t)a.sg.nc * 4u;
-    if (PACKED) {
-        const int64_t first = ((id.row * a.nsub + id.sub) * kWordsPerSub) * a.sg.nc;        // uniform over the block
-        const uint32_t lo32 = __builtin_amdgcn_readfirstlane((uint32_t)first);
-        const uint32_t hi32 = __builtin_amdgcn_readfirstlane((uint32_t)((uint64_t)first >> 32));
-        symbols_rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)(a.sym4 + (int64_t)(((uint64_t)hi32 << 32) | lo32)), 0,
-                                                         (int)((uint32_t)nwords * row_bytes), kBufferWord3);
-        if (id.active) symbols_voff = (uint32_t)id.ch * 4u;
-    }
     // The row's alphabet (2C + 1 symbols for `bins` levels, encoder.py:44-52): it may leave the
     // table's last symbol unused (then its special upper bound is never needed), and with at
     // most 15 symbols the quantizer may have packed it four bits a symbol, two channels to a
@@ -449,11 +434,25 @@ __device__ __forceinline__ void encode_streams(const EncodeArgs &a, uint16_t *ta
         sentinel = !(cq >= 0.0f && 2.0f * cq + 1.0f <= (float)(lp - 2));
         if (a.nibbles && narrow_alphabet(cq, lp)) {
             mode = kNibbles;
-            if (id.active) symbols_voff = (uint32_t)(id.ch >> 1) * 4u;
             half_shift = (uint32_t)(id.ch & 1) * 16u;
         }
     }
 
+    // PACKED: the sub-chunk's words ([word][channel]) are read through a buffer descriptor that
+    // ends with its last word row: the lane's channel is the vector offset, the word row the
+    // scalar one, and a row past the end (or the offset of a lane without a channel) reads
+    // zero, so a load costs no address arithmetic, compare or branch.
+    __amdgpu_buffer_rsrc_t symbols_rsrc;
+    uint32_t symbols_voff = 0xFFFFFFFCu;
+    const uint32_t row_bytes = (uint32_t)a.sg.nc * (mode == kNibbles ? 2u : 4u);
+    if (PACKED) {
+        const int64_t first = ((id.row * a.nsub + id.sub) * kWordsPerSub) * a.sg.nc;        // uniform over the block
+        const uint32_t lo32 = __builtin_amdgcn_readfirstlane((uint32_t)first);
+        const uint32_t hi32 = __builtin_amdgcn_readfirstlane((uint32_t)((uint64_t)first >> 32));
+        symbols_rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)(a.sym4 + (int64_t)(((uint64_t)hi32 << 32) | lo32)), 0,
+                                                         (int)((uint32_t)nwords * row_bytes), kBufferWord3);
+        if (id.active) symbols_voff = (uint32_t)(mode == kNibbles ? id.ch >> 1 : id.ch) * 4u;
+    }
     // Half a sub-chunk (32 words = 128 symbols) at a time is loaded into registers and indexed
     // by the (uniform) loop counter, so the coding loop has no loads to wait for and its stores
     // never hold it up.

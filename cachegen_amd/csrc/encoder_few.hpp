@@ -177,7 +177,7 @@ __device__ __forceinline__ void encode_few(const EncodeArgs &a, uint32_t *entrie
     words32 words, later;
     const int nwords = (id.n + 3) >> 2;
     if (PACKED) {
-        const uint32_t row_bytes = (uint32_t)a.sg.nc * 4u;
+        const uint32_t row_bytes = (uint32_t)a.sg.nc * (mode == kNibbles ? 2u : 4u);
         const int64_t first = ((id.row * a.nsub + id.sub) * kWordsPerSub) * a.sg.nc;        // uniform over the block
         const uint32_t lo32 = __builtin_amdgcn_readfirstlane((uint32_t)first);
         const uint32_t hi32 = __builtin_amdgcn_readfirstlane((uint32_t)((uint64_t)first >> 32));

@@ -198,7 +198,7 @@ __global__ __launch_bounds__(QuantTablesBlock<NU>::kThreads, 4) void quantize_ta
     // symbols that may lie past the table's last one are kept inside it before they are counted
     const bool fits = maxq >= 0.0f && 2.0f * maxq <= (float)(LP - 2);
     constexpr uint32_t smax = (uint32_t)(LP - 2);
-    const int64_t C = (int64_t)a.nunits * 8;
+    const int64_t C = (int64_t)a.nunits * 8, word_row = narrow ? C / 2 : C;
 
     for (int i = tid; i < Layout::kBytes / 16; i += kThreads)
         reinterpret_cast<uint4 *>(counts)[i] = make_uint4(0, 0, 0, 0);
@@ -269,7 +269,7 @@ __global__ __launch_bounds__(QuantTablesBlock<NU>::kThreads, 4) void quantize_ta
             plain = plain && !scale_overflows(maxq, mf);
         }
         const int64_t sub = sub0 + (tt0 >> 8);
-        uint32_t *out = a.sym4 + ((row * a.nsub + sub) * kWordsPerSub + ((tt0 & (kSub - 1)) >> 2)) * C;
+        uint32_t *out = a.sym4 + (row * a.nsub + sub) * kWordsPerSub * C + ((tt0 & (kSub - 1)) >> 2) * word_row;
 #pragma unroll
         for (int i = 0; i < NU; ++i) {
             const int u = lane + 64 * i;

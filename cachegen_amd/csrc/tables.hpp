@@ -317,7 +317,7 @@ __device__ __forceinline__ void calculate_cdf(const CdfArgs &a, uint32_t *smem)
                 const int64_t kvi = row / a.L, l = row - kvi * a.L;
                 narrow = narrow_alphabet(floorf((kvi ? a.value_bins : a.key_bins)[l] * 0.5f) - 1.0f, lp);
             }
-            const int64_t column = narrow ? (ch >> 1) : ch;
+            const int64_t column = narrow ? (ch >> 1) : ch, word_row = narrow ? a.nc / 2 : a.nc;
             const uint32_t half_shift = narrow ? (uint32_t)(ch & 1) * 16u : 0u;
             const int nsubs = (int)((t1 - t0 + kSub - 1) / kSub);
             for (int sidx = 0; sidx < nsubs; ++sidx) {
@@ -329,7 +329,7 @@ __device__ __forceinline__ void calculate_cdf(const CdfArgs &a, uint32_t *smem)
                 for (int w0 = slice * kBatch; w0 < nwords; w0 += kBatch * SLICES) {
                     uint32_t v[kBatch];
 #pragma unroll
-                    for (int j = 0; j < kBatch; ++j) v[j] = (w0 + j < nwords) ? wp[(int64_t)(w0 + j) * a.nc] : 0u;
+                    for (int j = 0; j < kBatch; ++j) v[j] = (w0 + j < nwords) ? wp[(w0 + j) * word_row] : 0u;
                     // whole batches without a test per symbol
                     auto count = [&](auto whole) {
                         if (narrow) {
