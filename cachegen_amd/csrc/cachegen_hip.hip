@@ -301,7 +301,7 @@ struct EncodeWorkspace {
         uint8_t *ws = static_cast<uint8_t *>(base);
         symbols = ws;
         ws += symbols_bytes * (size_t)nlevels;
-        scratch = ws;           // kStreamCap bytes per stream, in tiles of kSlotTile word-interleaved streams
+        scratch = ws;           // kStreamCap bytes per stream, in tiles of kSlotTile streams (kQuadRow)
         ws += (size_t)ntiles * kSlotTile * kStreamCap;
         scan_scratch = ws;
         ws += cg_scan_workspace(nstreams);

@@ -36,26 +36,30 @@ constexpr int kSlotTile = 256;      // streams per tile of the encoder's scratch
 constexpr int kTileGroup = 64;
 constexpr int kMaxTileGroups = 256;
 
-// TILE: the stream's words go to a tile of the scratch (word w of the tile's stream t at the
-// tile's word w * kSlotTile + t) through a buffer descriptor that covers exactly the tile: a
-// word or byte past the stream's capacity falls outside the descriptor and is dropped by the
+// Streams of a tile lie interleaved by quads of four words: word w of the tile's stream t is the tile's
+// word (w / 4 * kSlotTile + t) * 4 + w % 4.  The words that a wavefront writes at about the same time share
+// a few lines, and the many words of a long stream among short ones share theirs.
+constexpr int kQuadRow = kSlotTile * 16;        // bytes from one quad of a stream to the next
+
+// TILE: the stream's words go to a tile of the scratch through a buffer descriptor that covers exactly the
+// tile: a word or byte past the stream's capacity falls outside the descriptor and is dropped by the
 // hardware, so nothing is compared or counted per word.
 template <bool ALIGNED, bool TILE = false>
 struct WordWriter {
     uint8_t *wptr;          // where the next word goes
-    int wstride;            // bytes from one word of the stream to the next (4: contiguous)
+    int quad_step;          // bytes from the last word of a quad to the next quad's first (4: contiguous)
     int cap;
     uint32_t whole;         // places a whole word can start at: cap - 3, or none
     int nbytes;             // bytes written so far; -4 before the held-back word's first, empty turn
     __amdgpu_buffer_rsrc_t tile;    // TILE: the block's tile
-    uint32_t voff, voff0;           // TILE: byte offset in the tile of the next word, and of the first
+    uint32_t voff, voff0;           // TILE: byte offset in the tile of the next word, and of the first (of stream t: 16 t)
 
-    __device__ __forceinline__ void init(uint8_t *dst, int stride, int capacity)
+    __device__ __forceinline__ void init(uint8_t *dst, int step, int capacity)
     {
         // the first word stored is the empty held-back word: it goes one word before the
         // stream (TILE: the offset wraps and the hardware drops the store)
-        wptr = dst - stride;
-        wstride = stride;
+        wptr = dst - step;
+        quad_step = step;
         cap = capacity;
         whole = capacity >= 4 ? (uint32_t)capacity - 3u : 0u;
         nbytes = -4;
@@ -65,14 +69,15 @@ struct WordWriter {
     {
         tile = rsrc;
         voff0 = first;
-        voff = first - kSlotTile * 4;
+        voff = first - (kQuadRow - 12);
     }
 
     __device__ __forceinline__ void store_word(uint32_t word)
     {
         if (TILE) {
             __builtin_amdgcn_raw_buffer_store_b32((int)__builtin_bswap32(word), tile, (int)voff, 0, 0);
-            voff += kSlotTile * 4;
+            // the stream's place, bits 4 to 11, is all ones while 4 is added: the carry out of the quad passes over it
+            voff = (((voff | (kQuadRow - 16u)) + 4u) & ~(kQuadRow - 16u)) | voff0;
             return;
         }
         // one test on the common path: nbytes in [0, cap - 4]
@@ -90,7 +95,7 @@ struct WordWriter {
             for (int j = 0; j < 4; ++j)
                 if (nbytes + j < cap) wptr[j] = (uint8_t)(word >> (24 - 8 * j));
         }
-        wptr += wstride;
+        wptr += (nbytes & 12) == 12 ? quad_step : 4;
         nbytes += 4;
     }
 
@@ -98,7 +103,7 @@ struct WordWriter {
     // (enc_new.cu:42-55); returns the stream length
     __device__ __forceinline__ int finish(uint32_t word, int nbits)
     {
-        if (TILE) nbytes = (int)((voff - voff0) / kSlotTile);     // four bytes per word written
+        if (TILE) nbytes = (int)((voff / kQuadRow << 4) | (voff & 12u));
         for (int left = nbits, j = 0; left > 0; left -= 8, ++j) {
             if (TILE) __builtin_amdgcn_raw_buffer_store_b8((char)(word >> 24), tile, (int)(voff + j), 0, 0);
             else if (nbytes < cap) wptr[j] = (uint8_t)(word >> 24);
@@ -528,9 +533,7 @@ __device__ __forceinline__ void encode_streams(const EncodeArgs &a, uint16_t *ta
 
     RangeEncoder<BS, ALIGNED, TILE> enc;
     const int64_t stream = (id.sub * a.sg.rows + id.row) * a.sg.nc + id.ch;
-    // SLOTS: the scratch is cut into tiles of kSlotTile streams; word w of a tile's stream t is
-    // the tile's word w * kSlotTile + t, so that the words the lanes of a wavefront write, and
-    // the words the compaction reads, lie side by side
+    // SLOTS: the scratch is cut into tiles of kSlotTile streams
     if (TILE) {
         // the block is exactly one tile (the host launches this form only then): its number is
         // the tile, tid the stream's place in it
@@ -538,10 +541,10 @@ __device__ __forceinline__ void encode_streams(const EncodeArgs &a, uint16_t *ta
         enc.w.init(nullptr, 0, a.cap);
         enc.w.init_tile(__builtin_amdgcn_make_buffer_rsrc((void *)(a.out + (int64_t)linear_block(coder_sub) * ((int64_t)kSlotTile * a.cap)), 0,
                                                           kSlotTile * a.cap, kBufferWord3),
-                        (uint32_t)tid * 4u);
+                        (uint32_t)tid * 16u);
     } else if (SLOTS) {
         enc.init(col, lp);
-        enc.w.init(a.out + (stream / kSlotTile) * ((int64_t)kSlotTile * a.cap) + (stream % kSlotTile) * 4, kSlotTile * 4, a.cap);
+        enc.w.init(a.out + (stream / kSlotTile) * ((int64_t)kSlotTile * a.cap) + (stream % kSlotTile) * 16, kQuadRow - 12, a.cap);
     } else {
         enc.init(col, lp);
         enc.w.init(a.out + id.row * a.o0 + id.ch * a.o1, 4, a.cap);

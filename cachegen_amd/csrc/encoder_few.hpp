@@ -279,9 +279,9 @@ __device__ __forceinline__ void encode_few(const EncodeArgs &a, uint32_t *entrie
         enc.w.init(nullptr, 0, a.cap);
         enc.w.init_tile(__builtin_amdgcn_make_buffer_rsrc((void *)(a.out + (int64_t)linear_block(z) * ((int64_t)kSlotTile * a.cap)), 0,
                                                           kSlotTile * a.cap, kBufferWord3),
-                        (uint32_t)tid * 4u);
+                        (uint32_t)tid * 16u);
     } else if (SLOTS) {
-        enc.w.init(a.out + (stream / kSlotTile) * ((int64_t)kSlotTile * a.cap) + (stream % kSlotTile) * 4, kSlotTile * 4, a.cap);
+        enc.w.init(a.out + (stream / kSlotTile) * ((int64_t)kSlotTile * a.cap) + (stream % kSlotTile) * 16, kQuadRow - 12, a.cap);
     } else {
         enc.w.init(a.out + id.row * a.o0 + id.ch * a.o1, 4, a.cap);
     }

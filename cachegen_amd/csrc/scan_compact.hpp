@@ -198,9 +198,9 @@ __global__ __launch_bounds__(kScanSmallThreads) void scan_collect_kernel(
 // ------------------------------------------------------------------------------------
 // collect_bytes (encoder.py:209-222).  A block owns 256 consecutive streams, i.e. one
 // contiguous range of the payload, and assembles it in LDS, 16 KiB at a time: every thread
-// copies its own stream from its slot to the stream's place in the range (aligned words
-// through a funnel shift, single bytes at the two ends), then the block writes the tile out
-// as aligned 32-bit words.  Only the first and last word of a block's range are written
+// copies its own stream from its slot to the stream's place in the range (two quads of words in
+// flight, aligned words by a byte permute, single bytes at the two ends), then the block writes the
+// tile out as aligned 32-bit words.  Only the first and last word of a block's range are written
 // byte by byte, so neighbouring blocks never write the same byte.  All positions are
 // 32-bit offsets from the range's start.
 // ------------------------------------------------------------------------------------
@@ -215,6 +215,11 @@ constexpr int kCompactTile = 16384;
 // tiles before this one (neither: calls of at most kDirectTiles tiles, where that is a few loads per
 // thread and saves the scan launch, 5 us and its gap).
 constexpr int kDirectTiles = 1024;
+// Bound by the trips to memory of a wavefront's longest stream and by HBM: what the words of long streams
+// cost among short ones.  Word by word (word w of stream t at w * 256 + t) each of them was a line of its own, read and written
+// for four bytes; a quad of four words is loaded by one instruction, and its words share the line.  32
+// layers x 8192 tokens x 1024 channels 63.9 -> 45.6 us, and the coder 274.9 -> 271.5; the whole encode
+// 626 -> 607, 80 layers x 32768 tokens 6100 -> 5850, four levels of 4096 tokens 1043 -> 1008, 4096 channels 2540 -> 2470.
 // SLICES > 1: the block has SLICES x 256 threads, and a stream's words are dealt to SLICES threads, eight in
 // turn.
 struct CompactArgs {
@@ -298,38 +303,48 @@ __device__ __forceinline__ void compact_streams(const CompactArgs &a, int32_t *r
     uint8_t *const dst = payload + o0 - lead;
     const int end = lead + total;
     const int my0 = rel[tid] + lead, my1 = rel[tid + 1] + lead;     // rel[] is padded with the total
-    // word k of this thread's stream (see encode_streams_kernel: tiles of kSlotTile streams)
-    const uint32_t *const words = reinterpret_cast<const uint32_t *>(slots + sbase * (int64_t)cap) + tid;
-    const int kmax = (my1 - my0 - 1) >> 2;             // last word that holds bytes of the stream
+    // this thread's stream, quad by quad (kQuadRow in encoder.hpp)
+    const uint8_t *const mine_at = slots + sbase * (int64_t)cap + tid * 16;
+    const int nquads = (my1 - my0 + 15) >> 4;
     uint8_t *const bytes = reinterpret_cast<uint8_t *>(buf);
+    // Aligned word first + i of the range holds the end of the stream's word i - 1 and the beginning of word i:
+    // four of their eight bytes, the same four for every i.
+    const int first = my0 >> 2;
+    const uint32_t pick_bytes = 0x07060504u - (uint32_t)(my0 & 3) * 0x01010101u;
 
     for (int t0 = 0; t0 < end; t0 += kCompactTile) {
         const int t1 = t0 + kCompactTile < end ? t0 + kCompactTile : end;
         const int xs = my0 > t0 ? my0 : t0;
         const int xe = my1 < t1 ? my1 : t1;
-        // aligned words j of the range that hold bytes [xs, xe) of this stream, eight at a time:
-        // word j is stream bytes 4j - my0 .. +3, i.e. two stream words through a funnel shift
-        for (int j = (xs >> 2) + 8 * slice; 4 * j < xe; j += 8 * SLICES) {
-            const int q = 4 * j - my0;                 // may be negative for the stream's first word
-            const int k = q >> 2;
-            const uint32_t sh = (uint32_t)(q & 3) * 8u;
-            const int left = ((xe + 3) >> 2) - j;      // words still to produce
-            uint32_t wv[9];
+        if (xs < xe) {
+            const int whole0 = (xs + 3) >> 2, whole1 = xe >> 2;         // the range's words that are all this stream's
+            uint32_t head = 0, tail = 0, prev = 0;
+            bool ends_here = false;                                     // this thread has the word that the stream ends inside
+            const int i_first = ((xs >> 2) - first) & ~7;
+            for (int i0 = i_first + 8 * slice; 4 * (first + i0) < xe; i0 += 8 * SLICES) {
+                const int g = i0 >> 2;
+                uint4 q0 = make_uint4(0, 0, 0, 0), q1 = q0;
+                if (g < nquads) q0 = *reinterpret_cast<const uint4 *>(mine_at + g * kQuadRow);
+                if (g + 1 < nquads) q1 = *reinterpret_cast<const uint4 *>(mine_at + (g + 1) * kQuadRow);
+                if (i0 > 0 && (SLICES > 1 || i0 == i_first)) prev = *reinterpret_cast<const uint32_t *>(mine_at + (g - 1) * kQuadRow + 12);
+                const uint32_t w[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
 #pragma unroll
-            for (int u = 0; u < 9; ++u)
-                wv[u] = (k + u >= 0 && k + u <= kmax && u <= left) ? words[(k + u) * kSlotTile] : 0u;
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                if (u >= left) break;
-                const uint32_t v = __builtin_amdgcn_alignbit(wv[u + 1], wv[u], sh);
-                const int x0 = 4 * (j + u);
-                if (x0 >= xs && x0 + 4 <= xe) {
-                    buf[(x0 - t0) >> 2] = v;
-                } else {
-                    for (int c = 0; c < 4; ++c)
-                        if (x0 + c >= xs && x0 + c < xe) bytes[x0 + c - t0] = (uint8_t)(v >> (8 * c));
+                for (int u = 0; u < 8; ++u) {
+                    const uint32_t v = __builtin_amdgcn_perm(w[u], u ? w[u - 1] : prev, pick_bytes);
+                    const int j = first + i0 + u;
+                    if (u == 0 && i0 == 0) head = v;
+                    if (j == whole1) tail = v, ends_here = true;
+                    if (j >= whole0 && j < whole1) buf[j - (t0 >> 2)] = v;
                 }
+                prev = w[7];
             }
+            // the words that this stream shares with its neighbours, byte by byte
+            if (slice == 0 && xs == my0 && first < whole0)
+                for (int c = 0; c < 4; ++c)
+                    if (4 * first + c >= xs && 4 * first + c < xe) bytes[4 * first + c - t0] = (uint8_t)(head >> (8 * c));
+            if (ends_here && whole1 >= whole0)
+                for (int c = 0; c < 3; ++c)
+                    if (4 * whole1 + c < xe) bytes[4 * whole1 + c - t0] = (uint8_t)(tail >> (8 * c));
         }
         __syncthreads();
         for (int w = (t0 >> 2) + (int)threadIdx.x; 4 * w < t1; w += 256 * SLICES) {
