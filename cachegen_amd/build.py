@@ -47,7 +47,7 @@ OCCUPANCY_BUDGETS = [
 # Kernels that address their dynamically allocated LDS from byte 0 (the counters of the table
 # builder: the address comes out of a byte permute; the float search, which sets an entry's address
 # bit by bit): a statically allocated array would sit there.
-NO_STATIC_LDS = r"^(quantize_tables_kernel|tables_from_partial_kernel|decode_float_kernel)<"
+NO_STATIC_LDS = r"^(quantize_tables_kernel|tables_from_partial_kernel|decode_float_kernel|encode_streams_kernel|encode_streams_levels_kernel)<"
 
 
 def parse_kernel_resources(report):

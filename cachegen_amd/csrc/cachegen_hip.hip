@@ -157,8 +157,7 @@ int cg_encode_fast_new(const int16_t *cdf, int lp, const int8_t *sym, int64_t nl
         const bool few = few_encode(nblocks, ENC_BYTES, lp, block, false) && s2 >= 0 && s2 <= 0x7FFFFFFFll / nc;
         CG_DISPATCH_BS(block, return (launch_encode<BS, false, false, false>(a, grid, few, st)));
     }
-    const size_t shmem = (size_t)lp * (block + 2) * sizeof(uint16_t);      // TableStride<BS>::k16 per entry
-    CG_DISPATCH_BS(block, (encode_streams_kernel<BS, false, false, false, false><<<grid, dim3(block), shmem, st>>>(a)));
+    CG_DISPATCH_BS(block, (encode_streams_kernel<BS, false, false, false, false><<<grid, dim3(block), encode_lds<BS, false>(lp), st>>>(a)));
     return check_launch("encode");
 }
 
@@ -474,8 +473,7 @@ int code_and_compact(const LevelOut &o, const uint32_t *sym4, const uint8_t *sym
         a.s0 = T * C;
         a.s1 = C;
         a.s2 = 1;
-        const size_t shmem = (size_t)lp * (block + 2) * sizeof(uint16_t);      // TableStride<BS>::k16 per entry
-        CG_DISPATCH_BS(block, (encode_streams_kernel<BS, true, false, false, true><<<grid, dim3(block), shmem, s>>>(a)));
+        CG_DISPATCH_BS(block, (encode_streams_kernel<BS, true, false, false, true><<<grid, dim3(block), encode_lds<BS, false>(lp), s>>>(a)));
         if (int rc = check_launch("encode_kv")) return rc;
     }
 

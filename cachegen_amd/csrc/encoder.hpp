@@ -52,7 +52,7 @@ struct WordWriter {
     uint32_t whole;         // places a whole word can start at: cap - 3, or none
     int nbytes;             // bytes written so far; -4 before the held-back word's first, empty turn
     __amdgpu_buffer_rsrc_t tile;    // TILE: the block's tile
-    uint32_t voff, voff0;           // TILE: byte offset in the tile of the next word, and of the first (of stream t: 16 t)
+    uint32_t voff;                  // TILE: byte offset in the tile of the next word (of stream t's first: 16 t)
 
     __device__ __forceinline__ void init(uint8_t *dst, int step, int capacity)
     {
@@ -63,12 +63,11 @@ struct WordWriter {
         cap = capacity;
         whole = capacity >= 4 ? (uint32_t)capacity - 3u : 0u;
         nbytes = -4;
-        voff = voff0 = 0;
+        voff = 0;
     }
     __device__ __forceinline__ void init_tile(__amdgpu_buffer_rsrc_t rsrc, uint32_t first)
     {
         tile = rsrc;
-        voff0 = first;
         voff = first - (kQuadRow - 12);
     }
 
@@ -77,7 +76,8 @@ struct WordWriter {
         if (TILE) {
             __builtin_amdgcn_raw_buffer_store_b32((int)__builtin_bswap32(word), tile, (int)voff, 0, 0);
             // the stream's place, bits 4 to 11, is all ones while 4 is added: the carry out of the quad passes over it
-            voff = (((voff | (kQuadRow - 16u)) + 4u) & ~(kQuadRow - 16u)) | voff0;
+            const uint32_t next = (voff | (kQuadRow - 16u)) + 4u;
+            asm("v_bitop3_b32 %0, %1, %0, %2 bitop3:0xD8" : "+v"(voff) : "v"(next), "s"(kQuadRow - 16u));    // the place of voff, the rest of next
             return;
         }
         // one test on the common path: nbytes in [0, cap - 4]
@@ -119,12 +119,22 @@ struct WordWriter {
 // a binary fraction) is 2^32 - 1 there, and floor(span * c / 2^16) is the high word of
 // span_less_one * (c << 16) + (c << 16) for every span, one 64-bit multiply-add with nothing set
 // apart for the full range.  Renormalising by n bits maps span to span << n for E1/E2 and E3
-// steps alike.
-template <int BS, bool ALIGNED, bool TILE = false>
+// steps alike, span_less_one to itself with n ones moved in: the upper half of a 64-bit shift of
+// `width_ones`, which holds the width less one above 32 ones.
+//
+// What bounds the coding loop is the issue of its vector instructions, 3.5 cycles each.  The width less one comes by one
+// subtraction with a borrow that is always there, the next span by that shift, a symbol's table address by a shift and one
+// v_bitop3 (RowPlace below), what a symbol's bits and its carry ask for by one branch, and a power of two of lanes a
+// table row leaves no LDS bank conflicts (36.6 M cycles before): 169.2 -> 160.9 M instructions for 32 layers x
+// 8192 tokens x 1024 channels, coder 272 -> 263 us, encode 606 -> 600; 80 layers x 32768 tokens 5918 -> 5780, four levels of
+// 4096 tokens 1012 -> 980.
+template <int BS, bool ALIGNED, bool TILE, int kS>
 struct RangeEncoder {
-    lds_char *col;          // this lane's table column: entry e at byte e * 2 * TableStride<BS>::k16
+    static constexpr int kRow = 2 * kS;     // bytes from an entry to the next of the same table
+    uint32_t col;           // LDS byte of this lane's table column: entry e at col + e * kRow
     uint32_t smax;          // lp - 2: the largest symbol
-    uint32_t span_less_one;
+    uint64_t span;          // span_less_one in its upper half
+    uint64_t width_ones;    // the coded symbol's width less one, above 32 ones
     // the number's last 96 bits: `tail` holds the window (its lower half, called low in the
     // comments) and above it the first 32 of the bits waiting to be written, `out_hi` the rest
     // of them: 63 - room bits wait, and above them there may be a carry (0 or 1) that belongs
@@ -144,11 +154,12 @@ struct RangeEncoder {
 
     __device__ __forceinline__ void init(const uint16_t *column, int lp)
     {
-        col = (lds_char *)column;
+        col = (uint32_t)(uintptr_t)(lds_char *)column;
         bound_lo = 0;
         bound_hi = 0;
         smax = (uint32_t)(lp - 2);
-        span_less_one = 0xFFFFFFFFu;
+        span = ~0ull;
+        width_ones = 0xFFFFFFFFu;
         tail = 0;
         out_hi = 0;
         room = 63;
@@ -210,41 +221,51 @@ struct RangeEncoder {
             : "vcc");
     }
 
-    // the same, then the step count of the interval [low, low + width - 1], as step_count() has it
-    // (common.hpp), four instructions after the window's add
-    __device__ __forceinline__ int add_and_count(uint32_t add, uint32_t width)
+    // the same for the lower bound (lo_pair's upper half) of a symbol with upper bound `hi`, without the third add (a carry out
+    // of the 64 low bits needs 32 waiting ones: the lanes that have one are left in `carry`): leaves the width less
+    // one in width_ones and gives the step count of the interval [low, low + width - 1], as step_count() has
+    // it (common.hpp), four instructions after the window's add
+    __device__ __forceinline__ int add_and_count(uint64_t lo_pair, uint32_t hi, uint64_t &carry)
     {
         int n;
-        uint32_t t;
-        // a carry out of the 64 low bits needs 32 waiting ones: left to a branch that is next to
-        // never taken, instead of a third add in every symbol
-        uint64_t carry;
-        asm("v_add_co_u32 v56, vcc, v56, %4\n\t"
+        asm("s_mov_b64 vcc, -1\n\tv_subb_co_u32 v61, vcc, %5, v63, vcc\n\t"
+            "v_add_co_u32 v56, vcc, v56, v63\n\t"
             "v_addc_co_u32 v57, %2, 0, v57, vcc\n\t"
-            "v_add_u32 %0, -1, %5\n\t"
-            "v_add_u32 %1, %0, v56\n\t"
-            "v_bitop3_b32 %1, %1, v56, %0 bitop3:0x82\n\t"
-            "v_lshl_or_b32 %1, %1, 1, %0\n\t"
-            "v_ffbh_u32 %0, %1"
-            : "=&v"(n), "=&v"(t), "=&s"(carry), "+{v[56:57]}"(tail)
-            : "v"(add), "v"(width)
+            "v_add_u32 v62, v61, v56\n\t"
+            "v_bitop3_b32 v62, v62, v56, v61 bitop3:0x82\n\t"
+            "v_lshl_or_b32 v62, v62, 1, v61\n\t"
+            "v_ffbh_u32 %0, v62"
+            : "=&v"(n), "+{v[62:63]}"(lo_pair), "=&s"(carry), "+{v[56:57]}"(tail), "+{v[60:61]}"(width_ones)
+            : "v"(hi)
             : "vcc");
-        if (__builtin_expect(carry != 0, 0))
-            asm("v_addc_co_u32 v59, %0, 0, v59, %0" : "+s"(carry), "+{v59}"(out_hi));
         return n;
     }
-
-    // the number moves left by n <= 31 bits.  ROOM: the caller knows that the bits fit
-    template <bool ROOM = false>
-    __device__ __forceinline__ void shift(int n)
+    __device__ __forceinline__ void add_carry(uint64_t carry)
     {
-        uint32_t left;
-        if (__builtin_expect(__builtin_usub_overflow(room, (uint32_t)n, &left), 0) && !ROOM) {
-            asm volatile("");
-            flush_word();                               // more than 32 bits were waiting
-            left = room - (uint32_t)n;
+        asm("v_addc_co_u32 v59, %0, 0, v59, %0" : "+s"(carry), "+{v59}"(out_hi));
+    }
+
+    // n <= 31 bits more will wait; what is to happen for a carry out of the low bits and, unless ROOM (the
+    // caller knows that the bits fit), where more than 32 bits were waiting already is left to one branch on
+    // both, which is next to never taken
+    template <bool ROOM>
+    __device__ __forceinline__ void book(int n, uint64_t carry)
+    {
+        uint64_t full = 0;
+        if (ROOM) room -= (uint32_t)n;
+        else asm("v_sub_co_u32 %0, %1, %0, %2" : "+v"(room), "=s"(full) : "v"(n));
+        if (__builtin_expect((carry | full) != 0, 0)) {
+            add_carry(carry);
+            if (!ROOM && (int32_t)room < 0) {
+                room += (uint32_t)n;
+                flush_word();
+                room -= (uint32_t)n;
+            }
         }
-        room = left;
+    }
+    // the number moves left by n bits
+    __device__ __forceinline__ void move(int n)
+    {
         asm("v_mov_b32 v58, v57\n\t"
             "v_lshlrev_b64 v[58:59], %2, v[58:59]\n\t"
             "v_lshlrev_b64 v[56:57], %2, v[56:57]"
@@ -253,36 +274,42 @@ struct RangeEncoder {
             : "v58");
     }
 
-    // SENTINEL: symbol smax may occur, whose upper bound is 2^16 and not the table's last
-    // entry (enc_new.cu:270)
     // FIRST: the symbol directly follows a flush (the first of a group)
+    // at: the LDS byte of the symbol's lower bound; top: the symbol is smax, whose upper bound is 2^16 and not
+    // the table's last entry (enc_new.cu:270)
+    template <bool FIRST>
+    __device__ __forceinline__ void put_at(uint32_t at, bool top)
+    {
+        // both entries into the upper halves of the lower registers of two pairs whose upper
+        // registers stay 0: the pairs are the entries shifted left by 16, as 64-bit values
+        asm volatile("ds_read_u16_d16_hi v52, %2\n\tds_read_u16_d16_hi v54, %2 offset:%3\n\ts_waitcnt lgkmcnt(0)"
+                     : "+{v[52:53]}"(bound_lo), "+{v[54:55]}"(bound_hi)
+                     : "v"(at), "n"(kRow));
+        // T(c) = (span * c) >> 16 = high word of span * (c << 16) = high word of
+        // span_less_one * (c << 16) + (c << 16): one 64-bit multiply-add, right for the full range
+        // (span_less_one = 2^32 - 1) as for every other span, so no case is set apart
+        // (the second product takes the span's place)
+        const uint32_t all = top ? (uint32_t)(span >> 32) + 1u : 0u;            // T(2^16) is the span
+        uint64_t prod;
+        asm("v_mad_u64_u32 v[62:63], vcc, v51, v52, v[52:53]\n\tv_mad_u64_u32 v[50:51], vcc, v51, v54, v[54:55]"
+            : "=&{v[62:63]}"(prod), "+{v[50:51]}"(span)
+            : "{v[52:53]}"(bound_lo), "{v[54:55]}"(bound_hi)
+            : "vcc");
+        uint64_t carry;
+        const int n = add_and_count(prod, top ? all : (uint32_t)(span >> 32), carry);
+        book<FIRST>(n, carry);
+        move(n);
+        span = width_ones << n;
+    }
+
+    // SENTINEL: symbol smax may occur
     // CLAMP: the symbol may lie outside the table (it is kept inside; symbols that are known to
     // be table symbols skip the compare)
     template <bool SENTINEL, bool FIRST, bool CLAMP = true>
     __device__ __forceinline__ void put_symbol(uint32_t s)
     {
         if (CLAMP) s = s < smax ? s : smax;             // keep table reads inside the table
-        constexpr int kRow = 2 * TableStride<BS>::k16;
-        // both entries into the upper halves of the lower registers of two pairs whose upper
-        // registers stay 0: the pairs are the entries shifted left by 16, as 64-bit values
-        asm volatile("ds_read_u16_d16_hi v52, %2\n\tds_read_u16_d16_hi v54, %2 offset:%3\n\ts_waitcnt lgkmcnt(0)"
-                     : "+{v[52:53]}"(bound_lo), "+{v[54:55]}"(bound_hi)
-                     : "v"(col + s * kRow), "n"(kRow));
-        // T(c) = (span * c) >> 16 = high word of span * (c << 16) = high word of
-        // span_less_one * (c << 16) + (c << 16): one 64-bit multiply-add, right for the full range
-        // (span_less_one = 2^32 - 1) as for every other span, so no case is set apart
-        uint64_t prod_lo, prod_hi;
-        asm("v_mad_u64_u32 %0, vcc, %2, v52, v[52:53]\n\tv_mad_u64_u32 %1, vcc, %2, v54, v[54:55]"
-            : "=&v"(prod_lo), "=&v"(prod_hi)
-            : "v"(span_less_one), "{v[52:53]}"(bound_lo), "{v[54:55]}"(bound_hi)
-            : "vcc");
-        const uint32_t t_lo = (uint32_t)(prod_lo >> 32);
-        // the upper bound of symbol smax is 2^16 and not the table's last entry: T(2^16) is the span
-        const bool top = SENTINEL && s == smax;
-        const uint32_t width = (top ? span_less_one + 1u : (uint32_t)(prod_hi >> 32)) - t_lo;
-        const int n = add_and_count(t_lo, width);
-        shift<FIRST>(n);
-        span_less_one = (width << n) - 1u;
+        put_at<FIRST>(col + s * (uint32_t)kRow, SENTINEL && s == smax);
     }
 
     // one group of symbols is through: write a word if 32 bits are waiting
@@ -296,7 +323,8 @@ struct RangeEncoder {
         // the closing bits (enc_new.cu:309-317): the two bits below `out` of the number plus a
         // quarter of the window
         add_low(0x40000000u);
-        shift(2);
+        book<false>(2, 0);
+        move(2);
         end_group();
         const uint32_t nbits = 63u - room;              // fewer than 32 are left
         const uint32_t out_lo = (uint32_t)(tail >> 32);
@@ -390,10 +418,10 @@ __device__ __forceinline__ uint32_t packed_symbol(uint32_t v, int j, uint32_t sm
 
 // The bytes that the block's streams occupy in the payload, for the compaction.  Every lane of the block
 // is active where this is called (the host asks for tile sums only when a block is exactly one tile).
+// wave_sums: BS / 64 words of LDS.
 template <int BS>
-__device__ __forceinline__ void leave_tile_sum(const EncodeArgs &a, uint32_t tile, int tid, int len)
+__device__ __forceinline__ void leave_tile_sum(const EncodeArgs &a, int32_t *wave_sums, uint32_t tile, int tid, int len)
 {
-    __shared__ int32_t wave_sums[BS / 64];
     int32_t v = len < a.cap ? len : a.cap;
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
@@ -407,6 +435,44 @@ __device__ __forceinline__ void leave_tile_sum(const EncodeArgs &a, uint32_t til
     }
 }
 
+// Entries of the coder's tables in LDS from one entry of a lane to its next.  Packed symbols: every lane reads and
+// writes its own column only, so the row is the block's lanes and a power of two: a symbol's bits, moved to their place, and
+// the column's make an entry's address without an add.  Byte symbols, whose tables are staged transposed: TableStride.
+template <int BS, bool PACKED>
+struct EncodeTable {
+    static constexpr int kS = PACKED ? BS : TableStride<BS>::k16;
+};
+// Words of LDS behind the tables: one a wavefront for whether a row saturates, one a wavefront for the streams' bytes.
+constexpr int kEncodeLdsWords = 8;
+template <int BS, bool PACKED>
+constexpr size_t encode_lds(int lp)
+{
+    return (size_t)lp * EncodeTable<BS, PACKED>::kS * sizeof(uint16_t) + kEncodeLdsWords * sizeof(uint32_t);
+}
+
+// Where the four symbols of a word go in an entry's address.  The tables begin at LDS byte 0 (no static
+// LDS: the build checks it), a lane's column is below kRow and a symbol's entry a multiple of it, so
+// the address is one v_bitop3 of the moved word, the symbol's bits there and the column.
+template <int BS, int MODE>
+struct RowPlace {
+    static constexpr int kBit = BS == 256 ? 9 : BS == 128 ? 8 : 7;          // 2 BS bytes a row
+    static_assert(2 * BS == 1 << kBit, "");
+    static constexpr uint32_t kMask = (MODE == kBytes ? 0xFFu : 0xFu) << kBit;
+    // a word of four-bit symbols is turned first, so that the lane's half begins at bit kBit: half_shift + turn
+    static constexpr uint32_t kTurn = 32u - kBit;
+
+    static __device__ __forceinline__ uint32_t entry(uint32_t v, int j, uint32_t col)
+    {
+        // the mask from a vector register: with a scalar operand the instruction takes a turn of its own (605 -> 600 us an encode)
+        uint32_t x;
+        const int left = MODE == kBytes ? kBit - 8 * j : -4 * j;
+        if (left == 1) asm("v_add_u32 %0, %1, %1" : "=v"(x) : "v"(v));       // issues beside other wavefronts', a left shift does not
+        else x = left >= 0 ? v << left : v >> -left;
+        asm("v_bitop3_b32 %0, %1, %2, %3 bitop3:0xEA" : "=v"(x) : "v"(x), "v"(kMask), "v"(col));     // (x & mask) | col
+        return x;
+    }
+};
+
 // PACKED: symbols come from sym4.  FUSE_CDF (PACKED only, one sub-chunk per chunk): the
 // block first builds its own tables from the same words and writes them out.
 // SLOTS: stream g of the launch is written to out[g * cap ...] (the fused path's scratch).
@@ -418,8 +484,10 @@ __device__ __forceinline__ void encode_streams(const EncodeArgs &a, uint16_t *ta
     const uint32_t coder_sub = a.last_first ? (uint32_t)a.nsub - 1 - z : z;
     const StreamId id = locate<BS>(a.sg, coder_sub);
     const int lp = a.lp;
-    const int64_t ch0 = id.ch - tid;
+    const int64_t ch0 = (int64_t)blockIdx.x * BS;
+    constexpr int kS = EncodeTable<BS, PACKED>::kS;
     uint16_t *col = tab + table_column<BS>(tid);
+    int32_t *const lds_words = reinterpret_cast<int32_t *>(tab + lp * kS);          // kEncodeLdsWords
     uint16_t *cdf_block = a.cdf + ((id.chunk * a.sg.rows + id.row) * a.sg.nc + ch0) * lp;
     const int nwords = (id.n + 3) >> 2;
     // The row's alphabet (2C + 1 symbols for `bins` levels, encoder.py:44-52): it may leave the
@@ -478,12 +546,19 @@ __device__ __forceinline__ void encode_streams(const EncodeArgs &a, uint16_t *ta
             const float m = a.max_dt == CG_DT_BF16 ? load16f<CG_DT_BF16>(bits) : load16f<CG_DT_F16>(bits);
             saturates |= scale_overflows(cq, m);
         }
-        if (__syncthreads_or(saturates)) sentinel = true;       // the last symbol does occur
+        // by hand: __syncthreads_or() takes LDS of its own, which would sit in front of the tables
+        const bool wave_saturates = __any(saturates);
+        if ((tid & 63) == 0) lds_words[tid >> 6] = wave_saturates;
+        __syncthreads();
+        int any = 0;
+#pragma unroll
+        for (int w = 0; w < BS / 64; ++w) any |= lds_words[w];
+        if (__builtin_amdgcn_readfirstlane(any)) sentinel = true;       // the last symbol does occur
     }
     if (mode == kNibbles && sentinel) mode = kNibblesEscaped;
 
     if (FUSE_CDF) {
-        for (int i = 0; i < lp; ++i) col[i * TableStride<BS>::k16] = 0;
+        for (int i = 0; i < lp; ++i) col[i * kS] = 0;
         __syncthreads();                     // another lane, of another wavefront, shares this lane's words
         if (id.active) {
             const uint32_t smax = (uint32_t)(lp - 2);
@@ -504,7 +579,7 @@ __device__ __forceinline__ void encode_streams(const EncodeArgs &a, uint16_t *ta
                         for (int j = 0; j < 4; ++j) {
                             uint32_t s = packed_symbol<MODE>(v, j, smax);
                             if (MODE == kBytes) s = s < smax ? s : smax;
-                            if ((h * 32 + w) * 4 + j < id.n) atomicAdd(pair + (s + 1) * (TableStride<BS>::k16 / 2), one);
+                            if ((h * 32 + w) * 4 + j < id.n) atomicAdd(pair + (s + 1) * (kS / 2), one);
                         }
                     }
                 }
@@ -515,8 +590,8 @@ __device__ __forceinline__ void encode_streams(const EncodeArgs &a, uint16_t *ta
         }
         __syncthreads();                     // the other lane's counts are all in
         if (id.active) {
-            normalize_column16<BS>(col, lp, lp - 1, (uint32_t)id.n);
-            write_column16<BS>(col, cdf_block + (int64_t)tid * lp, lp);
+            normalize_column16_stride<kS>(col, lp, lp - 1, (uint32_t)id.n);
+            write_column16_stride<kS>(col, cdf_block + (int64_t)tid * lp, lp);
         }
     } else if (!PACKED) {
         stage_tables16<BS>(tab, cdf_block, lp, ch0, a.sg.nc);
@@ -526,12 +601,12 @@ __device__ __forceinline__ void encode_streams(const EncodeArgs &a, uint16_t *ta
         // dozen instructions an entry; this one costs the coder under one a symbol).  A lane reads
         // its own column only and LDS serves a wavefront's accesses in order: no barrier, but the
         // compiler must not move the coder's reads up.
-        stage_column16_stride<TableStride<BS>::k16>(col, cdf_block + (int64_t)tid * lp, lp);
+        stage_column16_stride<kS>(col, cdf_block + (int64_t)tid * lp, lp);
         asm volatile("" ::: "memory");
     }
     if (!id.active) return;
 
-    RangeEncoder<BS, ALIGNED, TILE> enc;
+    RangeEncoder<BS, ALIGNED, TILE, kS> enc;
     const int64_t stream = (id.sub * a.sg.rows + id.row) * a.sg.nc + id.ch;
     // SLOTS: the scratch is cut into tiles of kSlotTile streams
     if (TILE) {
@@ -558,6 +633,9 @@ __device__ __forceinline__ void encode_streams(const EncodeArgs &a, uint16_t *ta
         constexpr bool CLAMP = MODE == kBytes && SENTINEL;
         const uint32_t smax = (uint32_t)(lp - 2);
         if (PACKED) {
+            typedef RowPlace<BS, MODE> Place;
+            const uint32_t turn = half_shift + (SENTINEL ? 0u : Place::kTurn);          // modulo 32
+            auto word = [&](uint32_t x) { return MODE == kBytes ? x : __builtin_amdgcn_alignbit(x, x, turn); };
             const int full = (id.n >> 3) * 2;              // words of full groups
             for (int h = 0; h == 0 || h * 32 < full; ++h) {
                 load_half(h);
@@ -565,21 +643,26 @@ __device__ __forceinline__ void encode_streams(const EncodeArgs &a, uint16_t *ta
                 const int wn = __builtin_amdgcn_readfirstlane(full - h * 32 < 32 ? full - h * 32 : 32);
                 // two words = eight symbols between two visits of the store code, and no test per
                 // symbol of whether there is one
+                auto put = [&](auto first_tag, uint32_t v, int j) {
+                    constexpr bool FIRST = decltype(first_tag)::value;
+                    if (SENTINEL) enc.template put_symbol<SENTINEL, FIRST, CLAMP>(packed_symbol<MODE>(v, j, smax));
+                    else enc.template put_at<FIRST>(Place::entry(v, j, enc.col), false);
+                };
 #pragma unroll 1
                 for (int w = 0; w < wn; w += 2) {
-                    const uint32_t v = MODE == kBytes ? words[w] : words[w] >> half_shift;
-                    enc.template put_symbol<SENTINEL, true, CLAMP>(packed_symbol<MODE>(v, 0, smax));
-                    enc.template put_symbol<SENTINEL, false, CLAMP>(packed_symbol<MODE>(v, 1, smax));
-                    enc.template put_symbol<SENTINEL, false, CLAMP>(packed_symbol<MODE>(v, 2, smax));
-                    enc.template put_symbol<SENTINEL, false, CLAMP>(packed_symbol<MODE>(v, 3, smax));
+                    const uint32_t v = word(words[w]);
+                    put(BoolTag<true>(), v, 0);
+                    put(BoolTag<false>(), v, 1);
+                    put(BoolTag<false>(), v, 2);
+                    put(BoolTag<false>(), v, 3);
                     // fetched only here: there is no register to hold it earlier
                     int w1 = w + 1;
                     asm volatile("" : "+s"(w1));
-                    const uint32_t u = MODE == kBytes ? words[w1] : words[w1] >> half_shift;
-                    enc.template put_symbol<SENTINEL, false, CLAMP>(packed_symbol<MODE>(u, 0, smax));
-                    enc.template put_symbol<SENTINEL, false, CLAMP>(packed_symbol<MODE>(u, 1, smax));
-                    enc.template put_symbol<SENTINEL, false, CLAMP>(packed_symbol<MODE>(u, 2, smax));
-                    enc.template put_symbol<SENTINEL, false, CLAMP>(packed_symbol<MODE>(u, 3, smax));
+                    const uint32_t u = word(words[w1]);
+                    put(BoolTag<false>(), u, 0);
+                    put(BoolTag<false>(), u, 1);
+                    put(BoolTag<false>(), u, 2);
+                    put(BoolTag<false>(), u, 3);
                     enc.end_group();
                 }
             }
@@ -588,7 +671,8 @@ __device__ __forceinline__ void encode_streams(const EncodeArgs &a, uint16_t *ta
 #pragma unroll 1
             for (int t = full * 4; t < id.n; ++t) {
                 const uint32_t x = __builtin_amdgcn_raw_buffer_load_b32(symbols_rsrc, (int)symbols_voff, (int)((uint32_t)(t >> 2) * row_bytes), 0);
-                enc.template put_symbol<SENTINEL, false, CLAMP>(packed_symbol<MODE>(MODE == kBytes ? x : x >> half_shift, t & 3, smax));
+                const uint32_t v = word(x) >> (MODE == kBytes || SENTINEL ? 0 : Place::kBit);
+                enc.template put_symbol<SENTINEL, false, CLAMP>(packed_symbol<MODE>(v, t & 3, smax));
             }
             enc.end_group();
         } else {
@@ -616,9 +700,10 @@ __device__ __forceinline__ void encode_streams(const EncodeArgs &a, uint16_t *ta
     else if (PACKED && !sentinel) code(CodeTag<false, kBytes>());
     else code(CodeTag<true, kBytes>());
     const int len = enc.finish();
-    a.lengths[stream] = len;
+    // the lane's place by its index alone: nothing of the channel's number is kept in registers through the loop
+    a.lengths[(id.sub * a.sg.rows + id.row) * a.sg.nc + ch0 + (uint32_t)tid] = len;
     if (len > a.cap && a.status) atomicOr(a.status, 1);
-    if (SLOTS && a.tile_sums) leave_tile_sum<BS>(a, linear_block(coder_sub), tid, len);
+    if (SLOTS && a.tile_sums) leave_tile_sum<BS>(a, lds_words + BS / 64, linear_block(coder_sub), tid, len);
 }
 
 template <int BS, bool ALIGNED, bool PACKED, bool FUSE_CDF, bool SLOTS, bool TILE = false>

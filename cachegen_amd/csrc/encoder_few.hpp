@@ -356,7 +356,10 @@ __device__ __forceinline__ void encode_few(const EncodeArgs &a, uint32_t *entrie
     const int len = enc.finish();
     a.lengths[stream] = len;
     if (len > a.cap && a.status) atomicOr(a.status, 1);
-    if (SLOTS && a.tile_sums) leave_tile_sum<BS>(a, linear_block(z), tid, len);
+    if (SLOTS && a.tile_sums) {
+        __shared__ int32_t wave_sums[BS / 64];
+        leave_tile_sum<BS>(a, wave_sums, linear_block(z), tid, len);
+    }
 }
 
 template <int BS, bool PACKED, bool FUSE_CDF, bool SLOTS, bool TILE = false>

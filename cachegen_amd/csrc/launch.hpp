@@ -520,7 +520,7 @@ int launch_encode(const EncodeArgs &a, dim3 grid, bool few, hipStream_t stream)
                                            CG_MAX_LP * BS * (int)sizeof(uint32_t), asked)) return rc;
         encode_few_kernel<BS, PACKED, FUSE_CDF, SLOTS, TILE><<<grid, dim3(BS), lds, stream>>>(a);
     } else {
-        const size_t lds = (size_t)a.lp * TableStride<BS>::k16 * sizeof(uint16_t);
+        const size_t lds = encode_lds<BS, PACKED>(a.lp);
         encode_streams_kernel<BS, true, PACKED, FUSE_CDF, SLOTS, TILE><<<grid, dim3(BS), lds, stream>>>(a);
     }
     return check_launch("encode");
@@ -529,7 +529,7 @@ int launch_encode(const EncodeArgs &a, dim3 grid, bool few, hipStream_t stream)
 // Blocks of tables of `lp` entries that a compute unit holds at once (eight of 256 lanes are all its wavefronts).
 int64_t resident_encode_blocks(int lp)
 {
-    const int64_t fit = (int64_t)(kMaxLdsPerBlock / align_up((size_t)lp * TableStride<kSlotTile>::k16 * sizeof(uint16_t) + 32, 1280));
+    const int64_t fit = (int64_t)(kMaxLdsPerBlock / align_up(encode_lds<kSlotTile, true>(lp), 1280));
     return fit < 8 ? fit : 8;
 }
 
@@ -547,7 +547,7 @@ int launch_encode_levels(const EncodeLevelsArgs &p, int count, int max_lp, dim3 
                                            CG_MAX_LP * BS * (int)sizeof(uint32_t), asked)) return rc;
         encode_few_levels_kernel<BS, FUSE_CDF, TILE><<<grid, dim3(BS), lds, stream>>>(p);
     } else {
-        encode_streams_levels_kernel<BS, FUSE_CDF, TILE><<<grid, dim3(BS), (size_t)max_lp * TableStride<BS>::k16 * sizeof(uint16_t), stream>>>(p);
+        encode_streams_levels_kernel<BS, FUSE_CDF, TILE><<<grid, dim3(BS), encode_lds<BS, true>(max_lp), stream>>>(p);
     }
     return check_launch("encode levels");
 }
