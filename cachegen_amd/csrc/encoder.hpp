@@ -213,8 +213,8 @@ struct RangeEncoder {
     // the number grows by `add` (a carry may run into the waiting bits)
     __device__ __forceinline__ void add_low(uint32_t add)
     {
-        asm("v_add_co_u32 v56, vcc, v56, %2\n\t"
-            "v_addc_co_u32 v57, vcc, 0, v57, vcc\n\t"
+        asm("v_add_co_u32 v56, vcc, v56, %2\n\ts_nop 1\n\t"
+            "v_addc_co_u32 v57, vcc, 0, v57, vcc\n\ts_nop 1\n\t"
             "v_addc_co_u32 v59, vcc, 0, v59, vcc"
             : "+{v[56:57]}"(tail), "+{v59}"(out_hi)
             : "v"(add)
@@ -228,10 +228,11 @@ struct RangeEncoder {
     __device__ __forceinline__ int add_and_count(uint64_t lo_pair, uint32_t hi, uint64_t &carry)
     {
         int n;
+        // (a carry that a vector instruction wrote is read no sooner than two instructions later)
         asm("s_mov_b64 vcc, -1\n\tv_subb_co_u32 v61, vcc, %5, v63, vcc\n\t"
-            "v_add_co_u32 v56, vcc, v56, v63\n\t"
-            "v_addc_co_u32 v57, %2, 0, v57, vcc\n\t"
+            "v_add_co_u32 v56, vcc, v56, v63\n\ts_nop 0\n\t"
             "v_add_u32 v62, v61, v56\n\t"
+            "v_addc_co_u32 v57, %2, 0, v57, vcc\n\t"
             "v_bitop3_b32 v62, v62, v56, v61 bitop3:0x82\n\t"
             "v_lshl_or_b32 v62, v62, 1, v61\n\t"
             "v_ffbh_u32 %0, v62"
