@@ -517,15 +517,9 @@ struct FewLane {
     int phase;
 };
 
-// 2 * m + bit in one instruction
-__device__ __forceinline__ uint32_t twice_plus(uint32_t m, bool bit)
-{
-    const uint64_t carry = __builtin_amdgcn_ballot_w64(bit);
-    uint64_t unused;
-    uint32_t r;
-    asm("v_addc_co_u32 %0, %1, %2, %2, %3" : "=v"(r), "=&s"(unused) : "v"(m), "s"(carry));
-    return r;
-}
+// In C, so that the compiler sees the compare whose mask is read: an instruction that reads a mask stands no
+// closer than two behind the vector instruction that wrote it (see add_and_count in encoder.hpp).
+__device__ __forceinline__ uint32_t twice_plus(uint32_t m, bool bit) { return 2u * m + (bit ? 1u : 0u); }
 
 // One symbol.  EXACT: the interval may be the full range, whose T(c) is c << 16.  row_offset: of the
 // token's row in the output (dequantised output only).
