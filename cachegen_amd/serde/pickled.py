@@ -10,7 +10,6 @@ between the blob and pinned memory: the same pickle, with one copy of the bytes.
 What a torch-saved storage looks like is taken from torch itself once (`_storage_template`); a
 storage that looks different is left to the plain unpickler."""
 import collections
-import functools
 import io
 import pickle
 import re
@@ -279,12 +278,13 @@ class _Reader(_ContainerUnpickler):
     What `find_class` gives out must not lead back to the reader: it stays in the unpickler's memo, which the
     garbage collector does not look into, and the blob would stay with it for good (a context of 1333
     tokens to a blob of 13.8 MB and back 1640 us with methods of the reader here,
-    each time in memory new from the system, 1289 now)."""
+    each time in memory new from the system, 1289 now).  Nor is it a function of this module: a pickle may
+    set the attributes of what it is given (BUILD), and those of a module's function outlive the blob."""
 
     def __init__(self, condensed, large, whole):
         super().__init__(io.BytesIO(condensed))
-        self._given = {("torch._utils", "_rebuild_tensor_v2"): _tensor,
-                       ("torch.storage", "_load_from_bytes"): functools.partial(_storage, large, whole)}
+        self._given = {("torch._utils", "_rebuild_tensor_v2"): lambda *args: _tensor(*args),
+                       ("torch.storage", "_load_from_bytes"): lambda *args: _storage(large, whole, *args)}
 
     def find_class(self, module, name):
         return self._given.get((module, name)) or super().find_class(module, name)
