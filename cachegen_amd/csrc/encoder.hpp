@@ -43,23 +43,23 @@ constexpr int kQuadRow = kSlotTile * 16;        // bytes from one quad of a stre
 
 // TILE: the stream's words go to a tile of the scratch through a buffer descriptor that covers exactly the
 // tile: a word or byte past the stream's capacity falls outside the descriptor and is dropped by the
-// hardware, so nothing is compared or counted per word.
-template <bool ALIGNED, bool TILE = false>
+// hardware, so nothing is compared or counted per word.  QUADS without TILE: a tile through pointers, for blocks that
+// are not whole tiles.  Neither: the stream's words lie one behind the other.
+template <bool ALIGNED, bool QUADS, bool TILE>
 struct WordWriter {
+    static constexpr int kQuadStep = kQuadRow - 12;     // bytes from the last word of a quad to the next quad's first
     uint8_t *wptr;          // where the next word goes
-    int quad_step;          // bytes from the last word of a quad to the next quad's first (4: contiguous)
     int cap;
     uint32_t whole;         // places a whole word can start at: cap - 3, or none
     int nbytes;             // bytes written so far; -4 before the held-back word's first, empty turn
     __amdgpu_buffer_rsrc_t tile;    // TILE: the block's tile
     uint32_t voff;                  // TILE: byte offset in the tile of the next word (of stream t's first: 16 t)
 
-    __device__ __forceinline__ void init(uint8_t *dst, int step, int capacity)
+    __device__ __forceinline__ void init(uint8_t *dst, int capacity)
     {
         // the first word stored is the empty held-back word: it goes one word before the
         // stream (TILE: the offset wraps and the hardware drops the store)
-        wptr = dst - step;
-        quad_step = step;
+        wptr = dst - (QUADS ? kQuadStep : 4);
         cap = capacity;
         whole = capacity >= 4 ? (uint32_t)capacity - 3u : 0u;
         nbytes = -4;
@@ -68,7 +68,7 @@ struct WordWriter {
     __device__ __forceinline__ void init_tile(__amdgpu_buffer_rsrc_t rsrc, uint32_t first)
     {
         tile = rsrc;
-        voff = first - (kQuadRow - 12);
+        voff = first - kQuadStep;
     }
 
     __device__ __forceinline__ void store_word(uint32_t word)
@@ -95,7 +95,7 @@ struct WordWriter {
             for (int j = 0; j < 4; ++j)
                 if (nbytes + j < cap) wptr[j] = (uint8_t)(word >> (24 - 8 * j));
         }
-        wptr += (nbytes & 12) == 12 ? quad_step : 4;
+        wptr += QUADS && (nbytes & 12) == 12 ? kQuadStep : 4;
         nbytes += 4;
     }
 
@@ -128,7 +128,7 @@ struct WordWriter {
 // table row leaves no LDS bank conflicts (36.6 M cycles before): 169.2 -> 160.9 M instructions for 32 layers x
 // 8192 tokens x 1024 channels, coder 272 -> 263 us, encode 606 -> 600; 80 layers x 32768 tokens 5918 -> 5780, four levels of
 // 4096 tokens 1012 -> 980.
-template <int BS, bool ALIGNED, bool TILE, int kS>
+template <int BS, bool ALIGNED, bool QUADS, bool TILE, int kS>
 struct RangeEncoder {
     static constexpr int kRow = 2 * kS;     // bytes from an entry to the next of the same table
     uint32_t col;           // LDS byte of this lane's table column: entry e at col + e * kRow
@@ -150,7 +150,7 @@ struct RangeEncoder {
     // the coded symbol's two table entries, each shifted left by 16: only ever written by
     // loads into the upper half, so that the lower halves stay zero
     uint64_t bound_lo, bound_hi;
-    WordWriter<ALIGNED, TILE> w;
+    WordWriter<ALIGNED, QUADS, TILE> w;
 
     __device__ __forceinline__ void init(const uint16_t *column, int lp)
     {
@@ -607,23 +607,23 @@ __device__ __forceinline__ void encode_streams(const EncodeArgs &a, uint16_t *ta
     }
     if (!id.active) return;
 
-    RangeEncoder<BS, ALIGNED, TILE, kS> enc;
+    RangeEncoder<BS, ALIGNED, SLOTS, TILE, kS> enc;
     const int64_t stream = (id.sub * a.sg.rows + id.row) * a.sg.nc + id.ch;
     // SLOTS: the scratch is cut into tiles of kSlotTile streams
     if (TILE) {
         // the block is exactly one tile (the host launches this form only then): its number is
         // the tile, tid the stream's place in it
         enc.init(col, lp);
-        enc.w.init(nullptr, 0, a.cap);
+        enc.w.init(nullptr, a.cap);
         enc.w.init_tile(__builtin_amdgcn_make_buffer_rsrc((void *)(a.out + (int64_t)linear_block(coder_sub) * ((int64_t)kSlotTile * a.cap)), 0,
                                                           kSlotTile * a.cap, kBufferWord3),
                         (uint32_t)tid * 16u);
     } else if (SLOTS) {
         enc.init(col, lp);
-        enc.w.init(a.out + (stream / kSlotTile) * ((int64_t)kSlotTile * a.cap) + (stream % kSlotTile) * 16, kQuadRow - 12, a.cap);
+        enc.w.init(a.out + (stream / kSlotTile) * ((int64_t)kSlotTile * a.cap) + (stream % kSlotTile) * 16, a.cap);
     } else {
         enc.init(col, lp);
-        enc.w.init(a.out + id.row * a.o0 + id.ch * a.o1, 4, a.cap);
+        enc.w.init(a.out + id.row * a.o0 + id.ch * a.o1, a.cap);
     }
 
     auto code = [&](auto tag) {

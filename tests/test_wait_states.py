@@ -34,6 +34,9 @@ def early_readers(lines):
             kernel, written = m.group(1), {}
             continue
         name, _, rest = line.split("//")[0].strip().partition(" ")
+        if name in ("s_branch", "s_setpc_b64", "s_endpgm"):     # what is written below is not what comes next
+            written = {}
+            continue
         if not rest:
             t += 1
             continue
