@@ -178,12 +178,15 @@ __device__ __forceinline__ void stage_tables16(uint16_t *tab, const uint16_t *cd
 // col[e * kS]: loads and LDS writes on immediate offsets.  Whole batches carry no test per entry, so
 // that the compiler joins a batch's loads into two of 128 bits: the lanes of a wavefront read places
 // lp entries apart, and every load instruction costs the memory pipeline a visit to each of them (33
-// 16-bit loads a lane took it longer than the data takes to arrive).
+// 16-bit loads a lane took it longer than the data takes to arrive).  Two batches in flight: with four, which the
+// compiler takes for rows of 512 bytes if left to itself, tables of 65 entries come in more slowly (4096 tokens x 32 layers x 1024
+// channels in chunks of 16, the whole encode 1964 -> 1908 us; in chunks of 8, the coder 2042 -> 1905) and those of 33 wait twice.
 template <int kS>
 __device__ __forceinline__ void stage_column16_stride(uint16_t *col, const uint16_t *mine, int lp)
 {
     constexpr int kBatch = 16;
     int e0 = 0;
+#pragma unroll 2
     for (; e0 + kBatch <= lp; e0 += kBatch) {
         uint16_t v[kBatch];
 #pragma unroll
