@@ -87,6 +87,32 @@ def test_stream_longer_than_256_bytes_is_reported(oracle, flags):
     assert np.array_equal(lengths[last], len_l)
 
 
+@pytest.mark.parametrize("C", [64, 256, 512])
+@pytest.mark.parametrize("flags", [0, 16])          # 16: CG_TEST_MANY_WAVEFRONTS, the coder's form for many wavefronts
+def test_what_exceeds_256_bytes_lands_nowhere(oracle, C, flags):
+    """Blocks that are a whole tile of the scratch (256 and 512 channels) and that are not, both forms of the coder: a
+    tile's first and last stream are too long, and every stream beside them and of the next tile is what it should be."""
+    codec, _ = _mods()
+    T = 65280
+    kv = _overflowing_kv(T, C)
+    long_channels = sorted({0, min(C, 256) - 1, C - 1})
+    kv[..., long_channels] = kv[..., :1]
+    noise = torch.rand((1, 2, 1024, 1, C), generator=torch.Generator().manual_seed(C)) * 1.6 - 0.8       # the others: streams of many lengths
+    keep = torch.tensor([c not in (1, *long_channels) for c in range(C)])
+    kv[:, :, :1024] = torch.where(keep, (noise * torch.linspace(0, 1, C)).half(), kv[:, :, :1024])
+    bins = torch.tensor([32.0])
+    enc = codec.encode_kv(kv.to(DEV), bins, bins, chunk_tokens=T, _test_flags=flags)
+    with pytest.raises(RuntimeError, match="exceeded 256 bytes"):
+        enc.check()
+    want = oracle.encode_function(kv.reshape(1, 2, T, C).contiguous().view(torch.int16).numpy().view(np.uint16), bins.numpy(), bins.numpy())
+    lengths, offs = enc.lengths.cpu().numpy(), enc.offsets.cpu().numpy()
+    assert (want["data_chunks"][0][1][:, long_channels] > 256).all()
+    per_sub = 2 * C
+    for g, (data, length, _) in enumerate(want["data_chunks"]):
+        assert np.array_equal(lengths[g], length), g
+        assert np.array_equal(enc.payload[offs[g * per_sub]:offs[(g + 1) * per_sub]].cpu().numpy(), data), g
+
+
 def test_payload_buffer_too_small_is_reported():
     codec, _ = _mods()
     from cachegen_amd.kvgen import make_kv
