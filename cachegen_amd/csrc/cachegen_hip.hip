@@ -289,6 +289,7 @@ struct EncodeWorkspace {
     int32_t *tile_sums, *group_sums;
     int64_t *tile_base;
     int64_t nsub, nstreams, ntiles;
+    uint32_t place;             // how streams lie in their tile
     size_t total;
 
     EncodeWorkspace(void *base, int64_t L, int64_t T, int64_t C, int64_t chunk_tokens, int nlevels, int nareas = 1) : areas(nareas)
@@ -296,11 +297,12 @@ struct EncodeWorkspace {
         nsub = cg_num_subchunks(T, chunk_tokens);
         nstreams = nsub * 2 * L * C;
         ntiles = ceil_div(nstreams, kSlotTile);
+        place = chunk_tokens <= kShortStreams || T <= kShortStreams ? kWordPlace : kQuadPlace;
         symbols_bytes = align_up((size_t)nstreams * kSub, 256);
         uint8_t *ws = static_cast<uint8_t *>(base);
         symbols = ws;
         ws += symbols_bytes * (size_t)nlevels;
-        scratch = ws;           // kStreamCap bytes per stream, in tiles of kSlotTile streams (kQuadRow)
+        scratch = ws;           // kStreamCap bytes per stream, in tiles of kSlotTile streams (kQuadPlace, kWordPlace)
         ws += (size_t)ntiles * kSlotTile * kStreamCap;
         scan_scratch = ws;
         ws += cg_scan_workspace(nstreams);
@@ -395,7 +397,7 @@ int scan_for_compaction(const LevelOut &o, const EncodeWorkspace &w, bool fused_
         if (int rc = launch_scan(o.lengths, w.nstreams, kStreamCap, o.offsets, w.scan_scratch, s)) return rc;
     }
     c = {w.scratch, kStreamCap, o.offsets, fused_scan ? o.lengths : nullptr, tile_base, w.nstreams, o.payload,
-         o.payload_cap, skew, o.status, grouped ? group_sums : nullptr, fused_scan ? w.tile_sums : nullptr};
+         o.payload_cap, skew, o.status, grouped ? group_sums : nullptr, fused_scan ? w.tile_sums : nullptr, w.place};
     return CG_OK;
 }
 
@@ -443,6 +445,7 @@ int code_and_compact(const LevelOut &o, const uint32_t *sym4, const uint8_t *sym
     const bool grouped = fused_scan && group_sums && ceil_div(w.ntiles, kTileGroup) <= kMaxTileGroups;
     a.group_sums = grouped ? group_sums : nullptr;
     a.last_first = code_last_first(w.ntiles);
+    a.place = w.place;
 
     if (sym4) {
         // four tokens per word, read by one lane per channel
@@ -548,6 +551,7 @@ int code_and_compact_levels(const LevelOut *o, int n, const EncodeWorkspace &w, 
     a.maxima = static_cast<const uint16_t *>(maxima);
     a.max_dt = max_dt;
     a.last_first = code_last_first(w.ntiles);
+    a.place = w.place;
     int64_t nblocks;
     if (int rc = make_grid(rows, C, T, chunk_tokens, w.nsub, kSlotTile, a.sg, nblocks)) return rc;
     if (nblocks > INT_MAX / kMaxLevels) return fail(CG_ERR_ARG, "encode_kv_levels: too many streams");

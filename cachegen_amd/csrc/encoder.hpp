@@ -38,16 +38,29 @@ constexpr int kMaxTileGroups = 256;
 
 // Streams of a tile lie interleaved by quads of four words: word w of the tile's stream t is the tile's
 // word (w / 4 * kSlotTile + t) * 4 + w % 4.  The words that a wavefront writes at about the same time share
-// a few lines, and the many words of a long stream among short ones share theirs.
+// a few lines, and the many words of a long stream among short ones share theirs.  Streams that hardly fill a quad are
+// interleaved word by word (word w of stream t is word w * kSlotTile + t): quads are four times the lines for
+// a stream of one word.
 constexpr int kQuadRow = kSlotTile * 16;        // bytes from one quad of a stream to the next
+constexpr int kWordRow = kSlotTile * 4;         // bytes from one word of a stream to the next
+// Symbols of a call's longest sub-chunk up to which its streams are interleaved word by word.  By words / by quads, the whole
+// encode, us, 32 layers x 4096 tokens in chunks of   16         24         32         40         48         56         64         96
+//   1024 channels, tables of 17 entries               700/724    556/569    441/444    415/416    383/385    364/364    338/338    313/312
+//                            33                       897/941    731/759    546/556    526/533    469/473    448/449    402/401    359/357
+//                            65                     1908/1944  1500/1522  1068/1076  1022/1028   879/883    814/819    692/695    601/600
+//   400 channels, 33 entries                          490/505    377/384    288/291               244/244               198/198    187/186
+// one chunk of so many tokens, 74 layers x 1536 ch.  51.8/52.1  53.9/53.9  54.6/54.8             58.9/58.8             62.2/61.7  69.4/69.3
+constexpr int kShortStreams = 48;
+// The bits of a word's offset in its tile that are the stream's place there; the others count the stream's words.
+constexpr uint32_t kQuadPlace = kQuadRow - 16, kWordPlace = kWordRow - 4;
 
 // TILE: the stream's words go to a tile of the scratch through a buffer descriptor that covers exactly the
 // tile: a word or byte past the stream's capacity falls outside the descriptor and is dropped by the
-// hardware, so nothing is compared or counted per word.  QUADS without TILE: a tile through pointers, for blocks that
+// hardware, so nothing is compared or counted per word.  SLOTS without TILE: a tile through pointers, for blocks that
 // are not whole tiles.  Neither: the stream's words lie one behind the other.
-template <bool ALIGNED, bool QUADS, bool TILE>
+template <bool ALIGNED, bool SLOTS, bool TILE>
 struct WordWriter {
-    static constexpr int kQuadStep = kQuadRow - 12;     // bytes from the last word of a quad to the next quad's first
+    uint32_t place;         // SLOTS: kQuadPlace or kWordPlace (uniform)
     uint8_t *wptr;          // where the next word goes
     int cap;
     uint32_t whole;         // places a whole word can start at: cap - 3, or none
@@ -55,29 +68,31 @@ struct WordWriter {
     __amdgpu_buffer_rsrc_t tile;    // TILE: the block's tile
     uint32_t voff;                  // TILE: byte offset in the tile of the next word (of stream t's first: 16 t)
 
-    __device__ __forceinline__ void init(uint8_t *dst, int capacity)
+    // bytes from one word to the next inside a quad, and from its last word to the next quad's first
+    __device__ __forceinline__ int step() const { return SLOTS && place == kWordPlace ? kWordRow : 4; }
+    __device__ __forceinline__ int last_step() const { return !SLOTS ? 4 : place == kWordPlace ? kWordRow : kQuadRow - 12; }
+
+    // SLOTS: dst is the tile and t the stream's place in it
+    __device__ __forceinline__ void init(uint8_t *dst, int capacity, uint32_t tile_place = 0, uint32_t t = 0)
     {
+        place = tile_place;
         // the first word stored is the empty held-back word: it goes one word before the
         // stream (TILE: the offset wraps and the hardware drops the store)
-        wptr = dst - (QUADS ? kQuadStep : 4);
+        wptr = dst + first(t) - last_step();
         cap = capacity;
         whole = capacity >= 4 ? (uint32_t)capacity - 3u : 0u;
         nbytes = -4;
-        voff = 0;
+        voff = (first(t) | ~place) & ~3u;
     }
-    __device__ __forceinline__ void init_tile(__amdgpu_buffer_rsrc_t rsrc, uint32_t first)
-    {
-        tile = rsrc;
-        voff = first - kQuadStep;
-    }
+    __device__ __forceinline__ uint32_t first(uint32_t t) const { return !SLOTS ? 0u : place == kWordPlace ? t * 4u : t * 16u; }
 
     __device__ __forceinline__ void store_word(uint32_t word)
     {
         if (TILE) {
             __builtin_amdgcn_raw_buffer_store_b32((int)__builtin_bswap32(word), tile, (int)voff, 0, 0);
-            // the stream's place, bits 4 to 11, is all ones while 4 is added: the carry out of the quad passes over it
-            const uint32_t next = (voff | (kQuadRow - 16u)) + 4u;
-            asm("v_bitop3_b32 %0, %1, %0, %2 bitop3:0xD8" : "+v"(voff) : "v"(next), "s"(kQuadRow - 16u));    // the place of voff, the rest of next
+            // the stream's place is all ones while 4 is added: the carry out of the bits below passes over it
+            const uint32_t next = (voff | place) + 4u;
+            asm("v_bitop3_b32 %0, %1, %0, %2 bitop3:0xD8" : "+v"(voff) : "v"(next), "s"(place));    // the place of voff, the rest of next
             return;
         }
         // one test on the common path: nbytes in [0, cap - 4]
@@ -95,7 +110,7 @@ struct WordWriter {
             for (int j = 0; j < 4; ++j)
                 if (nbytes + j < cap) wptr[j] = (uint8_t)(word >> (24 - 8 * j));
         }
-        wptr += QUADS && (nbytes & 12) == 12 ? kQuadStep : 4;
+        wptr += SLOTS && (nbytes & 12) == 12 ? last_step() : step();
         nbytes += 4;
     }
 
@@ -103,7 +118,7 @@ struct WordWriter {
     // (enc_new.cu:42-55); returns the stream length
     __device__ __forceinline__ int finish(uint32_t word, int nbits)
     {
-        if (TILE) nbytes = (int)((voff / kQuadRow << 4) | (voff & 12u));
+        if (TILE) nbytes = place == kWordPlace ? (int)(voff / kWordRow * 4) : (int)((voff / kQuadRow << 4) | (voff & 12u));
         for (int left = nbits, j = 0; left > 0; left -= 8, ++j) {
             if (TILE) __builtin_amdgcn_raw_buffer_store_b8((char)(word >> 24), tile, (int)(voff + j), 0, 0);
             else if (nbytes < cap) wptr[j] = (uint8_t)(word >> 24);
@@ -128,7 +143,7 @@ struct WordWriter {
 // table row leaves no LDS bank conflicts (36.6 M cycles before): 169.2 -> 160.9 M instructions for 32 layers x
 // 8192 tokens x 1024 channels, coder 272 -> 263 us, encode 606 -> 600; 80 layers x 32768 tokens 5918 -> 5780, four levels of
 // 4096 tokens 1012 -> 980.
-template <int BS, bool ALIGNED, bool QUADS, bool TILE, int kS>
+template <int BS, bool ALIGNED, bool SLOTS, bool TILE, int kS>
 struct RangeEncoder {
     static constexpr int kRow = 2 * kS;     // bytes from an entry to the next of the same table
     uint32_t col;           // LDS byte of this lane's table column: entry e at col + e * kRow
@@ -150,7 +165,7 @@ struct RangeEncoder {
     // the coded symbol's two table entries, each shifted left by 16: only ever written by
     // loads into the upper half, so that the lower halves stay zero
     uint64_t bound_lo, bound_hi;
-    WordWriter<ALIGNED, QUADS, TILE> w;
+    WordWriter<ALIGNED, SLOTS, TILE> w;
 
     __device__ __forceinline__ void init(const uint16_t *column, int lp)
     {
@@ -356,6 +371,7 @@ struct EncodeArgs {
     int64_t L;
     StreamGrid sg;
     int32_t last_first;     // encode_streams_kernel: the last sub-chunk's blocks are the launch's first (code_last_first)
+    uint32_t place;         // SLOTS: kQuadPlace or kWordPlace
 };
 
 // Several quantization levels of one tensor in one launch: what they share, and what differs.  Level v has the
@@ -614,13 +630,12 @@ __device__ __forceinline__ void encode_streams(const EncodeArgs &a, uint16_t *ta
         // the block is exactly one tile (the host launches this form only then): its number is
         // the tile, tid the stream's place in it
         enc.init(col, lp);
-        enc.w.init(nullptr, a.cap);
-        enc.w.init_tile(__builtin_amdgcn_make_buffer_rsrc((void *)(a.out + (int64_t)linear_block(coder_sub) * ((int64_t)kSlotTile * a.cap)), 0,
-                                                          kSlotTile * a.cap, kBufferWord3),
-                        (uint32_t)tid * 16u);
+        enc.w.init(nullptr, a.cap, a.place, (uint32_t)tid);
+        enc.w.tile = __builtin_amdgcn_make_buffer_rsrc((void *)(a.out + (int64_t)linear_block(coder_sub) * ((int64_t)kSlotTile * a.cap)), 0,
+                                                       kSlotTile * a.cap, kBufferWord3);
     } else if (SLOTS) {
         enc.init(col, lp);
-        enc.w.init(a.out + (stream / kSlotTile) * ((int64_t)kSlotTile * a.cap) + (stream % kSlotTile) * 16, a.cap);
+        enc.w.init(a.out + (stream / kSlotTile) * ((int64_t)kSlotTile * a.cap), a.cap, a.place, (uint32_t)(stream % kSlotTile));
     } else {
         enc.init(col, lp);
         enc.w.init(a.out + id.row * a.o0 + id.ch * a.o1, a.cap);

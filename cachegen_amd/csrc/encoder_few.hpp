@@ -25,7 +25,7 @@ namespace {
 // the loads and the tables, the rest the launch and the last wavefront.
 // The stream is the same number, written the same way (see encoder.hpp): the interval's lower end with
 // its carries.
-template <int BS, bool QUADS, bool TILE>
+template <int BS, bool SLOTS, bool TILE>
 struct FewEncoder {
     static constexpr int kRow = 4 * BS;     // bytes of a row of the tables: entry e << 16 of lane c at word e * BS + c
     lds_char *col;          // this lane's entry 0
@@ -36,7 +36,7 @@ struct FewEncoder {
     uint32_t waiting;       // at most 31 after take_words()
     uint32_t cache;         // the last complete word, not yet written: a carry may still reach it
     uint32_t ones;          // words of all ones that follow it
-    WordWriter<true, QUADS, TILE> w;
+    WordWriter<true, SLOTS, TILE> w;
 
     __device__ __forceinline__ void init(const uint32_t *column, int lp)
     {
@@ -276,12 +276,11 @@ __device__ __forceinline__ void encode_few(const EncodeArgs &a, uint32_t *entrie
     const int64_t stream = (id.sub * a.sg.rows + id.row) * a.sg.nc + id.ch;
     enc.init(col, lp);
     if (TILE) {
-        enc.w.init(nullptr, a.cap);
-        enc.w.init_tile(__builtin_amdgcn_make_buffer_rsrc((void *)(a.out + (int64_t)linear_block(z) * ((int64_t)kSlotTile * a.cap)), 0,
-                                                          kSlotTile * a.cap, kBufferWord3),
-                        (uint32_t)tid * 16u);
+        enc.w.init(nullptr, a.cap, a.place, (uint32_t)tid);
+        enc.w.tile = __builtin_amdgcn_make_buffer_rsrc((void *)(a.out + (int64_t)linear_block(z) * ((int64_t)kSlotTile * a.cap)), 0,
+                                                       kSlotTile * a.cap, kBufferWord3);
     } else if (SLOTS) {
-        enc.w.init(a.out + (stream / kSlotTile) * ((int64_t)kSlotTile * a.cap) + (stream % kSlotTile) * 16, a.cap);
+        enc.w.init(a.out + (stream / kSlotTile) * ((int64_t)kSlotTile * a.cap), a.cap, a.place, (uint32_t)(stream % kSlotTile));
     } else {
         enc.w.init(a.out + id.row * a.o0 + id.ch * a.o1, a.cap);
     }

@@ -234,6 +234,7 @@ struct CompactArgs {
     int32_t skew;
     int32_t *status;
     const int32_t *group_sums, *tile_sums;
+    uint32_t place;         // kQuadPlace or kWordPlace
 };
 
 template <bool SCAN, int SLICES>
@@ -303,9 +304,10 @@ __device__ __forceinline__ void compact_streams(const CompactArgs &a, int32_t *r
     uint8_t *const dst = payload + o0 - lead;
     const int end = lead + total;
     const int my0 = rel[tid] + lead, my1 = rel[tid + 1] + lead;     // rel[] is padded with the total
-    // this thread's stream, quad by quad (kQuadRow in encoder.hpp)
-    const uint8_t *const mine_at = slots + sbase * (int64_t)cap + tid * 16;
-    const int nquads = (my1 - my0 + 15) >> 4;
+    // this thread's stream, quad by quad or word by word (kQuadRow in encoder.hpp)
+    const bool quads = a.place == kQuadPlace;
+    const uint8_t *const mine_at = slots + sbase * (int64_t)cap + tid * (quads ? 16 : 4);
+    const int nquads = (my1 - my0 + 15) >> 4, nwords = (my1 - my0 + 3) >> 2;
     uint8_t *const bytes = reinterpret_cast<uint8_t *>(buf);
     // Aligned word first + i of the range holds the end of the stream's word i - 1 and the beginning of word i:
     // four of their eight bytes, the same four for every i.
@@ -322,12 +324,21 @@ __device__ __forceinline__ void compact_streams(const CompactArgs &a, int32_t *r
             bool ends_here = false;                                     // this thread has the word that the stream ends inside
             const int i_first = ((xs >> 2) - first) & ~7;
             for (int i0 = i_first + 8 * slice; 4 * (first + i0) < xe; i0 += 8 * SLICES) {
-                const int g = i0 >> 2;
-                uint4 q0 = make_uint4(0, 0, 0, 0), q1 = q0;
-                if (g < nquads) q0 = *reinterpret_cast<const uint4 *>(mine_at + g * kQuadRow);
-                if (g + 1 < nquads) q1 = *reinterpret_cast<const uint4 *>(mine_at + (g + 1) * kQuadRow);
-                if (i0 > 0 && (SLICES > 1 || i0 == i_first)) prev = *reinterpret_cast<const uint32_t *>(mine_at + (g - 1) * kQuadRow + 12);
-                const uint32_t w[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
+                uint32_t w[8];
+                const bool want_prev = i0 > 0 && (SLICES > 1 || i0 == i_first);
+                if (quads) {
+                    const int g = i0 >> 2;
+                    uint4 q0 = make_uint4(0, 0, 0, 0), q1 = q0;
+                    if (g < nquads) q0 = *reinterpret_cast<const uint4 *>(mine_at + g * kQuadRow);
+                    if (g + 1 < nquads) q1 = *reinterpret_cast<const uint4 *>(mine_at + (g + 1) * kQuadRow);
+                    if (want_prev) prev = *reinterpret_cast<const uint32_t *>(mine_at + (g - 1) * kQuadRow + 12);
+                    w[0] = q0.x, w[1] = q0.y, w[2] = q0.z, w[3] = q0.w;
+                    w[4] = q1.x, w[5] = q1.y, w[6] = q1.z, w[7] = q1.w;
+                } else {
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) w[u] = i0 + u < nwords ? *reinterpret_cast<const uint32_t *>(mine_at + (i0 + u) * kWordRow) : 0u;
+                    if (want_prev) prev = *reinterpret_cast<const uint32_t *>(mine_at + (i0 - 1) * kWordRow);
+                }
 #pragma unroll
                 for (int u = 0; u < 8; ++u) {
                     const uint32_t v = __builtin_amdgcn_perm(w[u], u ? w[u - 1] : prev, pick_bytes);

@@ -21,6 +21,7 @@ CASES = [
     ((3, 257, 5, 80), 256, (16, 32, 64)),         # channels that fill no tile: offsets from a scan
     ((4, 520, 8, 128), 260, (8, 16, 32, 64)),     # tables of two sub-chunks, all levels resident at once
     ((6, 2048, 8, 128), 256, (8, 64, 32, 60)),    # more blocks than are resident: launches by table length
+    ((6, 2048, 8, 128), 40, (8, 64, 32)),         # the same with scratch laid word by word
     ((6, 2048, 8, 128), 700, (64, 8)),            # the same with tables made by a pass of their own
     ((2, 300, 8, 128), 256, (16, 96)),            # a table too long for blocks of 256 lanes: one launch each
     ((4, 256, 8, 128), 256, (8, 16, 24, 32, 40, 48, 56, 64)),

@@ -1,6 +1,6 @@
-"""The encoder's scratch holds streams in quads of four words, and the compaction takes two quads at a time:
-streams that end on either side of a quad, ranges of several LDS tiles, long streams among short ones, in
-launches of few and of many blocks."""
+"""The encoder's scratch holds streams in quads of four words, or word by word where sub-chunks have at most 48 tokens, and the
+compaction takes eight words at a time: streams that end on either side of a quad, ranges of several LDS tiles, long
+streams among short ones, in launches of few and of many blocks."""
 import numpy as np
 import pytest
 import torch
@@ -16,6 +16,12 @@ MANY_WAVEFRONTS = 16
     (1, 300, 4, 64, 300, (64.0,)),              # two tiles, streams of up to 200 bytes
     (1, 512, 3, 40, 64, (64.0,)),               # 120 channels: tiles that straddle rows
     (1, 21, 5, 40, 7, (128.0,)),                # tables of 129 entries, blocks of 128 lanes
+    (2, 197, 4, 64, 48, (64.0, 32.0)),          # word by word: the longest sub-chunks, of streams past eight words
+    (2, 197, 4, 64, 49, (64.0, 32.0)),          # the shortest in quads
+    (1, 144, 5, 40, 48, (64.0,)),               # tiles that straddle rows: both again
+    (1, 147, 5, 40, 49, (64.0,)),
+    (2, 48, 4, 64, 1500, (64.0, 16.0)),         # one chunk, short by its tokens
+    (1, 48, 1, 64, 48, (128.0,)),               # idle lanes, a tile of several rows
 ])
 def test_streams_of_any_length_beside_one_another(oracle, L, T, H, D, S, bins):
     from cachegen_amd import codec
