@@ -341,6 +341,7 @@ __device__ __forceinline__ void compact_streams(const CompactArgs &a, int32_t *r
                 }
 #pragma unroll
                 for (int u = 0; u < 8; ++u) {
+                    if (u == 4 && 4 * (first + i0 + u) >= xe) break;    // short streams (chunks of 8 tokens, 32 layers x 4096 x 1024 channels): 239 -> 231 us
                     const uint32_t v = __builtin_amdgcn_perm(w[u], u ? w[u - 1] : prev, pick_bytes);
                     const int j = first + i0 + u;
                     if (u == 0 && i0 == 0) head = v;
