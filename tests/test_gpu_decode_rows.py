@@ -1,6 +1,8 @@
-"""decode_streams_kernel reads tables whose rows are a power of two, in calls of more wavefronts than the forms for few and for
-some take: blocks of 64, 128 and 256 lanes, with idle lanes, tables of 9, 17, 33, 65 and other lengths, symbols and
-dequantised values, a row whose last symbol occurs."""
+"""decode_streams_kernel's unrolled search begins with a choice between two addresses that it holds in registers (tables of 9, 17
+and 33 entries; rows that use the lower half of their table, and rows that use all of it), in calls of more wavefronts than the
+forms for few take: blocks of 64 and 128 lanes, with idle lanes, symbols and dequantised values, a row whose last
+symbol occurs (bfloat16: a scale that overflows).  Tables of 65 entries (decode_float_kernel) and of other lengths (the search
+without those probes) go the same way through the same calls beside them."""
 import numpy as np
 import pytest
 import torch
@@ -19,13 +21,15 @@ def test_dequantised_values(oracle, H, D, nsub, S, bins, dtype, dt):
     kv = torch.rand((L, 2, T, H, D), generator=gen) * 2 - 1
     kv = kv.to(dtype)
     if dtype is torch.bfloat16:
-        kv[1, 1, 3 * S] *= 1e-38                             # the scale overflows: the table's last symbol
+        kv[1, 1, 3 * S] *= 1e-39                             # the scale overflows at any level: the table's last symbol
     kb, vb = torch.tensor(bins), torch.tensor(bins[::-1])
     max_bins = int(max(bins))
     dev = kv.to(DEV)
     enc = codec.encode_kv(dev, kb, vb, chunk_tokens=S)
     out = codec.decode_encoded(enc, kb, vb, fmt="vllm", out_dtype=dtype)
     sym, maxima = codec.quantize_kv(dev, kb.to(DEV), vb.to(DEV))
+    saturated = sym[L + 1, 3 * S] == 255
+    assert bool(saturated.any()) == (dtype is torch.bfloat16)
     sym = np.minimum(sym.cpu().numpy(), max_bins - 1)        # bytes outside the table are its last symbol
     mx = maxima.cpu().view(torch.int16).numpy().view(np.uint16)
     got = out.cpu().view(torch.int16).numpy().view(np.uint16).reshape(L, 2, T, H * D)

@@ -3,8 +3,8 @@ shift count taken from two count-leading-zero operations, write the encoder's ou
 interval's lower end with carries instead of counting pending bits, track the decoder's code
 value relative to the interval's low end, take the interval bounds from a high multiply and
 leave bit 31 of `low` as it falls.  This module restates exactly
-that arithmetic on Python integers (cachegen_amd/csrc/encoder.hpp: RangeEncoder::put_symbol,
-decoder.hpp: decode_symbol) and checks it, on the CPU, against the independent bit-serial coder
+that arithmetic on Python integers (cachegen_amd/csrc/encoder.hpp: RangeEncoder::put_at, RowPlace::entry and
+WordWriter::store_word, decoder.hpp: decode_symbol) and checks it, on the CPU, against the independent bit-serial coder
 of tests/pycoder.py: same bytes out of the encoder, same symbols out of the decoder, for tables
 that provoke long underflow runs, full-range intervals and the last symbol's special bound."""
 import random
@@ -114,10 +114,15 @@ def model_encode(cdf, symbols, group=8):
         t_lo, width = bound_less_one(cdf, s, span_less_one)
         assert (t_lo, width) == bound(cdf, s, (span_less_one + 1) & M32)
         add_low(t_lo)
-        high = (low + width - 1) & M32                     # bit 31 of low may differ from the reference's
+        t_hi = (t_lo + width) & M32
+        width_less_one = (t_hi - t_lo - 1) & M32           # one subtraction with a borrow that is always there
+        high = (low + width_less_one) & M32                # bit 31 of low may differ from the reference's
         n1, k = shift_count(low, high)
+        assert n1 + k == step_count(low, high, width_less_one)
         shift(n1 + k)
-        span_less_one = ((width << (n1 + k)) - 1) & M32
+        # the width less one above 32 ones, moved left: ones come in from below
+        span_less_one = (((width_less_one << 32 | M32) << (n1 + k)) >> 32) & M32
+        assert span_less_one == ((width << (n1 + k)) - 1) & M32
         if i % group == group - 1 and nout >= 32:
             flush_word()
     add_low(0x40000000)
@@ -301,3 +306,61 @@ def test_low_and_span_shifted_as_one_word():
             true = (low << n) & M32, (width << n) & M32
             assert state[1] == true[1] and (state[1] == 0 or (state[0] - true[0]) & (M32 >> 1) == 0)
     assert full > 20
+
+
+def bitop3(a, b, c, table):
+    """v_bitop3_b32: bit (a, b, c) of the table for every bit of the operands."""
+    out = 0
+    for i in range(8):
+        if table >> i & 1:
+            out |= (a if i & 4 else ~a) & (b if i & 2 else ~b) & (c if i & 1 else ~c)
+    return out & M32
+
+
+def rotate_right(x, n):
+    n &= 31
+    return (x >> n | x << (32 - n)) & M32
+
+
+@pytest.mark.parametrize("block,bit", [(256, 9), (128, 8), (64, 7)])
+@pytest.mark.parametrize("half", [None, 0, 16])            # a byte a symbol, or four bits in the lower or upper half of a word
+def test_a_symbols_place_in_its_table(block, bit, half):
+    """RowPlace::entry: entry s of the column at byte `col` of rows of 2 * block bytes."""
+    rng = random.Random(block + (half or 1))
+    row, mask = 2 * block, (0xFF if half is None else 0xF) << bit
+    assert row == 1 << bit
+    for _ in range(2000):
+        symbols = [rng.randrange(256 if half is None else 16) for _ in range(4)]
+        word = sum(s << 8 * j for j, s in enumerate(symbols)) if half is None else \
+            sum(s << half + 4 * j for j, s in enumerate(symbols)) | rng.getrandbits(16) << (16 - half)
+        col = 2 * rng.randrange(block)
+        moved = word if half is None else rotate_right(word, half + 32 - bit)
+        for j, s in enumerate(symbols):
+            left = bit - 8 * j if half is None else -4 * j
+            x = (moved << left & M32) if left >= 0 else moved >> -left
+            assert bitop3(x, mask, col, 0xEA) == col + s * row
+
+
+QUAD_PLACE, WORD_PLACE = 256 * 16 - 16, 256 * 4 - 4
+
+
+@pytest.mark.parametrize("place", [QUAD_PLACE, WORD_PLACE])
+def test_words_of_a_tile(place):
+    """WordWriter's offsets: the held-back word of the start and what exceeds 256 bytes lie outside the tile's 64 KB, every other
+    word where the compaction reads it, no two in the same place, and the count of words comes out of the offset."""
+    taken = set()
+    for t in range(256):
+        first = t * 16 if place == QUAD_PLACE else t * 4
+        at = (first | ~place) & M32 & ~3
+        assert at >= 1 << 16                               # stored before the stream's first word: dropped
+        for w in range(100):
+            at = bitop3(((at | place) + 4) & M32, at, place, 0xD8)
+            if place == QUAD_PLACE:
+                assert at == w // 4 * 4096 + t * 16 + w % 4 * 4
+                assert (at // 4096 << 4 | at & 12) == 4 * w
+            else:
+                assert at == w * 1024 + t * 4 and at // 1024 * 4 == 4 * w
+            assert (at < 1 << 16) == (w < 64)
+            if w < 64:
+                taken.add(at)
+    assert len(taken) == 1 << 14
