@@ -493,7 +493,7 @@ def main():
         from cachegen_amd import issue_probe
         cal = issue_probe.calibrate()
         insts = counters["valu_insts"]
-        cheap = counters.get("cheap_class_fraction", 11.0 / 35.0)
+        cheap = counters.get("cheap_class_fraction", 12.0 / 35.0)
         simds = torch.cuda.get_device_properties(0).multi_processor_count * 4
         mhz = (r.get("clock") or {}).get("engine_clock_mhz") or cal["decoder_symbol"]["clock_mhz"]
         per_simd = insts / simds

@@ -13,7 +13,8 @@
 //
 // The second half takes single instructions: two of them in turn on full SIMDs (whether they issue
 // beside each other, and, read beside the card's power, what each costs), and chains of dependent ones in a
-// wavefront that is alone on its compute unit (what a call of few wavefronts waits for).
+// wavefront that is alone on its compute unit (what a call of few wavefronts waits for).  What the instructions compute is of no
+// account there: a select may read a mask sooner than it may be relied on.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -22,8 +23,8 @@ extern "C" {
 
 // kind: 0 = cheap class (v_add_u32, v_xor_b32, v_lshrrev_b32, v_and_b32 in turn)
 //       1 = full-rate class (v_mul_u32_u24, v_cndmask_b32, v_lshlrev_b32, v_add3_u32 in turn)
-//       2 = one decoded symbol of decode_streams_kernel (rows of at most 16 levels): 24 instructions
-//           of the full class and 11 of the cheap class in the order the compiler emits them
+//       2 = one decoded symbol of decode_streams_kernel (rows of at most 16 levels): 23 instructions
+//           of the full class and 12 of the cheap class in the order the compiler emits them
 // iters: loop trips of 64 (kinds 0, 1) or 70 (kind 2: two symbols of 35) instructions per wavefront
 // ns_per_instruction: time one SIMD takes per wave64 instruction, 8 wavefronts resident
 // clock_mhz: engine clock while the probe ran
@@ -91,17 +92,17 @@ __global__ __launch_bounds__(256) void issue_rate_kernel(uint32_t *sink, ClockSa
         } else {
             // the symbol loop of decode_streams_kernel<128, 5, OFFSETS, F16>, rows of at most 16
             // levels, as compiled: search (two probes on registers, two on table entries), bounds
-            // and the one test, dequantisation, state update, bit window; LDS reads and the store
-            // left out (they are not vector-ALU instructions); twice, on two sets of registers
+            // and the one test, dequantisation, state update, bit window, and the wait states before a mask is read;
+            // LDS reads and the store left out (they are not vector-ALU instructions); twice, on two sets of registers
 #define CG_PROBE_SYMBOL(x, y, p, q)                                                         \
             "v_mul_u32_u24 " p ", " x ", %8\n\tv_cmp_gt_u32 vcc, " p ", " y "\n\t"              \
-            "v_cndmask_b32 " q ", %8, %9, vcc\n\tv_mul_u32_u24 " q ", " q ", " x "\n\t"         \
-            "v_cndmask_b32 " p ", %9, 0, vcc\n\tv_cmp_gt_u32 vcc, " q ", " y "\n\t"             \
-            "v_cndmask_b32 " q ", %8, 0, vcc\n\tv_add3_u32 " p ", %9, " p ", " q "\n\t"         \
+            "s_nop 1\n\tv_cndmask_b32 " q ", %8, %9, vcc\n\tv_cndmask_b32 " p ", %9, %8, vcc\n\t" \
+            "v_mul_u32_u24 " q ", " q ", " x "\n\tv_cmp_gt_u32 vcc, " q ", " y "\n\t"           \
+            "v_add_u32 " q ", 0x410, " p "\n\ts_nop 0\n\tv_cndmask_b32 " p ", " q ", " p ", vcc\n\t" \
             "v_add_u32 " q ", 0x208, " p "\n\tv_mul_u32_u24 " p ", " x ", " p "\n\t"            \
-            "v_cmp_gt_u32 vcc, " p ", " y "\n\tv_cndmask_b32 " p ", " q ", " p ", vcc\n\t"      \
+            "v_cmp_gt_u32 vcc, " p ", " y "\n\ts_nop 1\n\tv_cndmask_b32 " p ", " q ", " p ", vcc\n\t" \
             "v_add_u32 " q ", 0x104, " p "\n\tv_mul_u32_u24 " p ", " x ", " p "\n\t"            \
-            "v_cmp_gt_u32 vcc, " p ", " y "\n\tv_cndmask_b32 " p ", " q ", " p ", vcc\n\t"      \
+            "v_cmp_gt_u32 vcc, " p ", " y "\n\ts_nop 1\n\tv_cndmask_b32 " p ", " q ", " p ", vcc\n\t" \
             "v_add_u32 " q ", " p ", %9\n\t"                                                    \
             "v_mul_hi_u32 " p ", " p ", " x "\n\tv_mul_hi_u32 " q ", " q ", " x "\n\t"          \
             "v_sub_u32 " q ", " q ", " p "\n\tv_sub_u32 " y ", " y ", " p "\n\t"                \
