@@ -141,8 +141,9 @@ struct WordWriter {
 // subtraction with a borrow that is always there, the next span by that shift, a symbol's table address by a shift and one
 // v_bitop3 (RowPlace below), what a symbol's bits and its carry ask for by one branch, and a power of two of lanes a
 // table row leaves no LDS bank conflicts (36.6 M cycles before): 169.2 -> 160.9 M instructions for 32 layers x
-// 8192 tokens x 1024 channels, coder 272 -> 263 us, encode 606 -> 600; 80 layers x 32768 tokens 5918 -> 5780, four levels of
-// 4096 tokens 1012 -> 980.
+// 8192 tokens x 1024 channels, coder 272 -> 263 us, encode 606 -> 601; 80 layers x 32768 tokens 5918 -> 5839, four levels of
+// 4096 tokens 1013 -> 987 (all of it together, each pair on one machine).  Forms in which the last symbol may occur
+// (SENTINEL) compare the symbol and so extract it first.
 template <int BS, bool ALIGNED, bool SLOTS, bool TILE, int kS>
 struct RangeEncoder {
     static constexpr int kRow = 2 * kS;     // bytes from an entry to the next of the same table
@@ -243,7 +244,9 @@ struct RangeEncoder {
     __device__ __forceinline__ int add_and_count(uint64_t lo_pair, uint32_t hi, uint64_t &carry)
     {
         int n;
-        // (a carry that a vector instruction wrote is read no sooner than two instructions later)
+        // (a carry that a vector instruction wrote is read no sooner than two instructions later, the distance that the
+        // compiler keeps everywhere for this GPU; it sees nothing of what is written out here.  No change in time:
+        // 599 -> 598 us an encode)
         asm("s_mov_b64 vcc, -1\n\tv_subb_co_u32 v61, vcc, %5, v63, vcc\n\t"
             "v_add_co_u32 v56, vcc, v56, v63\n\ts_nop 0\n\t"
             "v_add_u32 v62, v61, v56\n\t"

@@ -10,9 +10,9 @@ namespace {
 
 // A call of few wavefronts lasts as long as one stream's chain of symbols.  One wavefront alone on its
 // SIMD issues a dependent instruction every 4.5 to 7 cycles and waits 49 for an LDS round trip, but 36 at every branch
-// on a mask that a vector instruction made (issue_probe.hip): encode_streams_kernel, which takes two or
-// three such branches a symbol (bits that do not fit, a carry that runs far, the store code) and
-// reads a symbol's table entries when it comes to code it, takes 330 cycles a symbol alone.  Here
+// on a mask that a vector instruction made (issue_probe.hip): encode_streams_kernel, which takes one such
+// branch a symbol (bits that do not fit, or a carry that runs far) and more with the store code, and
+// reads a symbol's table entries when it comes to code it, takes 114 ns a symbol alone where this takes 93.  Here
 //   - four symbols are coded without a branch: their bits are counted, and if a lane has more than
 //     its register holds, or meets the full range, the wavefront codes the four again one by one,
 //     exactly (tables of up to 64 symbols need 7.75 bits a symbol for that; a stream's first four
@@ -20,9 +20,8 @@ namespace {
 //   - the entries of eight symbols are read in one round trip, from tables of 32-bit entries;
 //   - a sub-chunk's symbols are in registers before the first is coded;
 //   - the store code runs once per eight symbols.
-// 256 symbols of 4096 streams (one wavefront a SIMD) 33 -> 27 us, with the tables counted here 47 -> 36,
-// from byte symbols 49 -> 35; of those 27, 17 are the 256 symbols (160 cycles each, about 20 instructions), 3
-// the loads and the tables, the rest the launch and the last wavefront.
+// 256 symbols of 65536 streams (one wavefront a SIMD; 32 layers x 1024 channels), encode_streams_kernel / here: 36 / 30 us, with
+// the tables counted in the kernel 44 / 34, from byte symbols 52 / 38; of 128 symbols 21 / 18, 26 / 21, 30 / 22.
 // The stream is the same number, written the same way (see encoder.hpp): the interval's lower end with
 // its carries.
 template <int BS, bool SLOTS, bool TILE>

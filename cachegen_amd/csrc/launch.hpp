@@ -459,27 +459,29 @@ enum EncodeSource {
 // (encode_few_kernel).  tile: every block is a whole tile of the scratch (TILE).  Measured on make_kv's caches,
 // encode_streams_kernel / encode_few_kernel, the whole call in a graph, us, by wavefronts a SIMD (a quarter of a unit's):
 //   1024 channels, tables of      17           33           41           65           97          129 entries
-//   byte symbols        1      51 /  29     52 /  38     53 /  42     58 /  49     67 /  60     70 /  61
-//   (256 tokens)        1.5    54 /  38     57 /  46     57 /  52     62 /  60     67 /  63     70 / 104
-//                       2      55 /  39     58 /  48     58 /  54     63 /  61     69 / 105     72 / 115
-//                       2.5    61 /  48     64 /  59     64 /  66     71 /  94     76 / 120    132 / 150
-//                       3      62 /  49     65 /  60     67 /  67     73 / 102     86 / 126    139 / 168
-//   tables by the       0.5    56 /  42     64 /  52     68 /  58     72 /  63     82 /  81     86 /  84
-//   coder (256 tokens)  1      63 /  48     71 /  57     74 /  63     78 /  68     93 /  94     97 /  98
-//                       1.5    69 /  59     76 /  67     79 /  73     86 /  82     99 / 103    105 / 144
-//                       2      76 /  65     85 /  77     87 /  82     94 /  91    109 / 149    114 / 165
-//   by a pass of their  1      63 /  54     70 /  66     74 /  70     79 /  76     96 / 102    103 / 110
-//   own (512 tokens)    1.5    71 /  65     78 /  79     81 /  85     92 /  96    105 / 113    113 / 159
-//                       2      76 /  71     87 /  88     92 /  96    101 / 105    114 / 158    123 / 176
-//   by the quantizer    1      75 /  65     81 /  75                  90 /  88
-//                       2      80 /  74     87 /  87                 101 / 105
+//   byte symbols        1      49 /  29     52 /  39     53 /  43     58 /  49     67 /  60     70 /  61
+//   (256 tokens)        1.5    53 /  37     55 /  47     56 /  52     62 /  61     67 /  62     70 / 102
+//                       2      53 /  38     56 /  48     57 /  52     62 /  61     68 / 104     71 / 113
+//                       2.5    58 /  48     61 /  61     62 /  64     69 /  93     74 / 119    133 / 148
+//                       3      58 /  48     61 /  61     63 /  66     70 / 104     82 / 124    139 / 165
+//   tables by the       0.5    53 /  39     62 /  51     64 /  55     69 /  60     81 /  80     84 /  83
+//   coder (256 tokens)  1      60 /  45     69 /  57     71 /  62     76 /  66     92 /  94     96 /  97
+//                       1.5    66 /  57     73 /  68     77 /  73     82 /  80     97 / 102    102 / 146
+//                       2      71 /  62     81 /  76     85 /  81     91 /  88    107 / 149    113 / 166
+//   by a pass of their  1      62 /  53     69 /  64     71 /  67     77 /  74     95 / 101    102 / 108
+//   own (512 tokens)    1.5    70 /  66     76 /  75     79 /  82     88 /  93    103 / 112    112 / 162
+//                       2      75 /  71     85 /  87     88 /  92     98 / 104    111 / 160    122 / 178
+//   by the quantizer    1      80 /  69     87 /  82                 102 / 100
+//   (512 tokens)        2      84 /  79     95 /  97                 114 / 119
+//   (256 tokens)        1      74 /  63     80 /  75                  89 /  87
+//                       2                   86 /  86
 //   400, 128, 64 channels (blocks of 256, 128, 64 lanes), packed symbols, at the line taken and above it:
-//   by the coder        25 entries: 400  89 / 82 at 2;  128  97 / 94 at 1, 108 / 110 at 1.25;  64  93 / 90 at 0.5, 120 / 121 at 1
-//                       65 entries: 400  87 / 81 at 1, 92 / 92 at 1.25
-//   by a pass           17 entries: 400  85 / 82 at 2;  128  94 / 93 at 1, 109 / 109 at 1.5;  64  79 / 80 at 0.25
-//                       29 entries: 400  80 / 79 at 1, 85 / 88 at 1.25;  33 entries: 400  70 / 71 at 0.25, 80 / 81 at 1
-//   by the quantizer    17 entries: 400  79 / 74 at 2;  128  85 / 80 at 1, 110 / 111 at 2;  64  81 / 80 at 0.5, 106 / 107 at 1
-//                       33 entries: 400  82 / 81 at 1, 82 / 86 at 1.25;  128  82 / 85 at 0.25
+//   by the coder        25 entries: 400  87 / 83 at 2;  128  97 / 95 at 1, 106 / 111 at 1.25;  64  91 / 91 at 0.5, 119 / 122 at 1
+//                       65 entries: 400  86 / 81 at 1, 90 / 92 at 1.25
+//   by a pass           17 entries: 400  84 / 82 at 2;  128  95 / 94 at 1, 110 / 111 at 1.5;  64  78 / 81 at 0.25
+//                       29 entries: 400  80 / 79 at 1, 85 / 87 at 1.25;  33 entries: 400  68 / 69 at 0.25, 80 / 80 at 1
+//   by the quantizer    17 entries: 400  85 / 83 at 2;  128  93 / 92 at 1, 115 / 118 at 2;  64  87 / 89 at 0.5, 115 / 121 at 1
+//                       33 entries: 400  89 / 89 at 1, 91 / 95 at 1.25;  128  88 / 93 at 0.25
 //   byte symbols of 64 channels and 25 to 29 entries, the worst of that form: 65 / 69 at 2.25, 71 / 73 at 2.5, 74 / 74 at 3
 // (the last column of byte symbols is 128 entries).  Longer tables cost encode_few_kernel more: it copies
 // those that are in memory entry by entry, at twice the width.

@@ -218,8 +218,9 @@ constexpr int kDirectTiles = 1024;
 // Bound by the trips to memory of a wavefront's longest stream and by HBM: what the words of long streams
 // cost among short ones.  Word by word (word w of stream t at w * 256 + t) each of them was a line of its own, read and written
 // for four bytes; a quad of four words is loaded by one instruction, and its words share the line.  32
-// layers x 8192 tokens x 1024 channels 63.9 -> 45.6 us, and the coder 274.9 -> 271.5; the whole encode
-// 626 -> 607, 80 layers x 32768 tokens 6100 -> 5850, four levels of 4096 tokens 1043 -> 1008, 4096 channels 2540 -> 2470.
+// layers x 8192 tokens x 1024 channels 63.9 -> 45.6 us (183 -> 137 MB read), and the coder 274.9 -> 271.5 (220 -> 151 MB written); the
+// whole encode 626 -> 607, 80 layers x 32768 tokens 6100 -> 5850, four levels of 4096 tokens 1043 -> 1008, 4096 channels 2540 ->
+// 2470 (each pair on one machine).  Sub-chunks of at most kShortStreams tokens lie word by word.
 // SLICES > 1: the block has SLICES x 256 threads, and a stream's words are dealt to SLICES threads, eight in
 // turn.
 struct CompactArgs {
